@@ -284,6 +284,23 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_tiled_k(const void* coo
   }
 }
 
+// The points of this wave in a sweep: `per` consecutive ones, fewer (perhaps none) at the end.  Every wave of a launch gets as many,
+// so that all take the same number of gather rounds per level and stay at the same level: with the points dealt to workgroups evenly
+// but to their waves in turn (64 points to the first, the next 64 to the second, ...) some waves had one round per level and
+// some two, the first ran ahead and the tables of more levels than an L2 holds were in use at once (304800 points: 169 against 120 us).
+struct SweepPart {
+  int64_t first;
+  int count;
+  __device__ __forceinline__ SweepPart(int64_t N, int per) {
+    first = ((int64_t)blockIdx.x * (TILE_THREADS / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * per;
+    const int64_t left = N - first;
+    count = left < per ? (left > 0 ? (int)left : 0) : per;
+    if (count == 0) first = N - 1;
+  }
+  // lanes past the end repeat the last point (their result is not stored)
+  __device__ __forceinline__ int64_t point(int k) const { return first + (k < count ? k : count > 0 ? count - 1 : 0); }
+};
+
 // Level sweep: the same work with (nearly) the whole grid resident at once.  A thread keeps the packed results of all
 // its PPT points' levels in registers and stores finished 64-byte rows at the end; nothing is staged in LDS, so three
 // or four workgroups fit a CU and a million points take little more than one round of workgroups.  Workgroups
@@ -295,17 +312,15 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_tiled_k(const void* coo
 template <typename TT, int PPT, int D, bool LDS0 = false>
 __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_sweep_k(const void* coords, int cdt, int64_t csn, int64_t csd,
                                                                  const uint32_t* table, uint16_t* out, int64_t out_stride,
-                                                                 int64_t N, DevGeom g, const int64_t* primes, float scale) {
-  constexpr int P = TILE_THREADS * PPT;
+                                                                 int64_t N, int per, DevGeom g, const int64_t* primes, float scale) {
   constexpr int LMAX = 16;
-  const int t = threadIdx.x;
-  const int64_t p0 = (int64_t)blockIdx.x * P;
+  const int t = threadIdx.x, lane = t & 63;
+  const SweepPart part(N, per);
   const int L = g.levels;
   float x[PPT][3];
 #pragma unroll
   for (int i = 0; i < PPT; ++i) {
-    int64_t n = p0 + t + TILE_THREADS * i;
-    if (n >= N) n = N - 1;
+    const int64_t n = part.point(lane + 64 * i);
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       float v = load_as_f32(coords, n * csn + d * csd, cdt);
@@ -332,10 +347,11 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_sweep_k(const void* coo
       const uint32_t* tab = table + g.row_offset[l];
 #pragma unroll
       for (int i0 = 0; i0 < PPT; i0 += 2) {
-        uint32_t v[2][8];
-        float w[2][8];
+        constexpr int AT_ONCE = PPT > 1 ? 2 : 1;
+        uint32_t v[AT_ONCE][8];
+        float w[AT_ONCE][8];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < AT_ONCE && i0 + i < PPT; ++i) {
           uint32_t c[3];
           float fr[3];
 #pragma unroll
@@ -346,13 +362,19 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_sweep_k(const void* coo
             fr[d] = pos - fl;
           }
           const Corner8 r = D == 3 ? rows_d3(c, hashed, res, mask, pi) : rows_d2(c, hashed, res, mask, pi);
+          // four points to a thread: each point's eight together are better than the pair's sixteen (327 and 334 us; three points: 119 and 116)
+          if constexpr (D == 3 && PPT == 4) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int j = 0; j < CN; ++j) v[i][j] = (LDS0 && l == 0) ? level0_rows[r.row[j]] : tab[r.row[j]];
+          if constexpr (D == 3 && PPT == 4) __builtin_amdgcn_sched_barrier(0);
           if (D == 3) weights_d3(fr, w[i]);
           else weights_d2(fr, w[i]);
         }
+        // the gathers leave together, ahead of the sums: left to itself the compiler puts the second point's between the
+        // first point's additions, and they leave one by one (2^20 points: 410 us)
+        if constexpr (D == 3 && PPT < 4) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < AT_ONCE && i0 + i < PPT; ++i) {
           float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
           for (int j = 0; j < CN; ++j) {
@@ -369,9 +391,8 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_sweep_k(const void* coo
   }
 #pragma unroll
   for (int i = 0; i < PPT; ++i) {
-    const int64_t n = p0 + t + TILE_THREADS * i;
-    if (n >= N) continue;
-    uint4* dst = reinterpret_cast<uint4*>(out + n * out_stride);
+    if (lane + 64 * i >= part.count) continue;
+    uint4* dst = reinterpret_cast<uint4*>(out + (part.first + lane + 64 * i) * out_stride);
 #pragma unroll
     for (int q = 0; q < LMAX / 4; ++q)
       if (4 * q < L) dst[q] = make_uint4(enc[i][4 * q], enc[i][4 * q + 1], enc[i][4 * q + 2], enc[i][4 * q + 3]);
@@ -383,23 +404,22 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_sweep_k(const void* coo
 template <int PPT>
 __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_sweep32_k(const void* coords, int cdt, int64_t csn, int64_t csd,
                                                                    const float2* table, float* out, int64_t out_stride,
-                                                                   int64_t N, DevGeom g, const int64_t* primes, float scale) {
-  constexpr int P = TILE_THREADS * PPT;
+                                                                   int64_t N, int per, DevGeom g, const int64_t* primes, float scale) {
   constexpr int LMAX = 16;
-  const int t = threadIdx.x;
-  const int64_t p0 = (int64_t)blockIdx.x * P;
+  const int lane = threadIdx.x & 63;
+  const SweepPart part(N, per);
   const int L = g.levels;
   float x[PPT][3];
 #pragma unroll
   for (int i = 0; i < PPT; ++i) {
-    int64_t n = p0 + t + TILE_THREADS * i;
-    if (n >= N) n = N - 1;
+    const int64_t n = part.point(lane + 64 * i);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       float v = load_as_f32(coords, n * csn + d * csd, cdt);
       x[i][d] = scale != 1.0f ? v / scale : v;
     }
   }
+  if (part.count == 0) return;
   const uint32_t pi[3] = {(uint32_t)primes[0], (uint32_t)primes[1], (uint32_t)primes[2]};
   float2 enc[PPT][LMAX];
 #pragma unroll
@@ -445,9 +465,8 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_sweep32_k(const void* c
   }
 #pragma unroll
   for (int i = 0; i < PPT; ++i) {
-    const int64_t n = p0 + t + TILE_THREADS * i;
-    if (n >= N) continue;
-    float4* dst = reinterpret_cast<float4*>(out + n * out_stride);
+    if (lane + 64 * i >= part.count) continue;
+    float4* dst = reinterpret_cast<float4*>(out + (part.first + lane + 64 * i) * out_stride);
 #pragma unroll
     for (int q = 0; q < LMAX / 2; ++q)
       if (2 * q < L) dst[q] = make_float4(enc[i][2 * q].x, enc[i][2 * q].y, enc[i][2 * q + 1].x, enc[i][2 * q + 1].y);
@@ -620,10 +639,39 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_bwd_level_k(const void* coo
 constexpr int64_t SCAN_MIN_POINTS = 32768;
 constexpr int64_t BIN_MIN_POINTS = 8192;  // below: the sort's fixed cost (about 100 us) exceeds the scattered atomics' 13 ns per point
 constexpr int SWEEP_PPT = 4;
-constexpr int64_t SWEEP_MIN_POINTS = (int64_t)256 * TILE_THREADS * SWEEP_PPT;
+// Batches from which the sweeps run.  In three dimensions with 16-bit tables the staged kernel's 512 points per workgroup are one
+// workgroup per unit up to 2^17 points (51 us, the sweep 56) and two beyond (150000 points: 97 us, the sweep 67); the other kinds have
+// the per-(point, level) kernels below them (two dimensions, 10^5 points: 36 us, the sweep 25; float32: 79 and 63 us).
+constexpr int64_t SWEEP_MIN_POINTS = ((int64_t)1 << 17) + 1;
+constexpr int64_t SWEEP_MIN_POINTS_D2 = (int64_t)1 << 16;
+constexpr int64_t SWEEP_MIN_POINTS_F32 = (int64_t)1 << 16;
 // the forward per (point, level) serves batches up to this where the staged kernel is the alternative (three
 // dimensions: 45 against 53 us at 2^16 points, 75 against 52 us at 2^17); in two dimensions up to the sweep's minimum
 constexpr int64_t LEVEL_MAX_POINTS = 65536;
+
+// How a sweep's points are dealt out.  A compute unit works its gathers off at a rate of its own (one workgroup on a unit runs
+// at the rate of three: 1024 points take 83 us either way, because the unit's L1 takes about three lanes in four clocks
+// whatever waits behind it), so the time is that of the unit with the most points.  A launch therefore takes whole multiples of
+// one workgroup per unit, all of the same number of points, instead of full workgroups and a remainder that a few units
+// run alone (304800 points, full workgroups of 1024: 298 workgroups, twice the time of 256).
+constexpr int64_t COMPUTE_UNITS = 256;
+
+// points per wave, at most `most`, four waves to a workgroup
+static int sweep_wave_points(int64_t n, int most) {
+  const int64_t waves = 4 * COMPUTE_UNITS * ((n + 4 * COMPUTE_UNITS * most - 1) / (4 * COMPUTE_UNITS * most));
+  return (int)((n + waves - 1) / waves);
+}
+
+// the sweep for waves of `per` points: as many per thread as that takes
+template <typename TT, int PPT = SWEEP_PPT>
+static const void* sweep_kernel(int per, int dims, bool lds0) {
+  if constexpr (PPT > 1)
+    if (per <= 64 * (PPT - 1)) return sweep_kernel<TT, PPT - 1>(per, dims, lds0);
+  if (dims == 2) return (const void*)hash_fwd_sweep_k<TT, PPT, 2>;
+  return lds0 ? (const void*)hash_fwd_sweep_k<TT, PPT, 3, true> : (const void*)hash_fwd_sweep_k<TT, PPT, 3>;
+}
+
+static unsigned sweep_groups(int64_t n, int per) { return (unsigned)((n + 4 * per - 1) / (4 * per)); }
 
 static bool tiled_ok(const nf_hash_geom* g, int table_dt, const void* rows_ptr, int64_t row_stride, int feat = 2, int dims = 3) {
   if (g->dims != dims || g->feat != feat || table_dt == NF_F32) return false;
@@ -766,60 +814,43 @@ extern "C" int nf_hash_encode_fwd(const void* coords, int coords_dtype, int64_t 
   }
 
   // float32 tables: the same sweep on 8-byte rows
-  if (!(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FWD_STAGED)) && n_points >= SWEEP_MIN_POINTS && table_dtype == NF_F32 &&
+  if (!(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FWD_STAGED)) && n_points >= SWEEP_MIN_POINTS_F32 && table_dtype == NF_F32 &&
       sweep32_ok(geom, table, out, out_stride_n)) {
     constexpr int PPT = 2;
-    constexpr int P = TILE_THREADS * PPT;
-    // launches of 1024 workgroups (2^19 points), for the reason given at the 16-bit sweep below
+    // launches of up to 1024 workgroups (2^19 points), for the reason given at the 16-bit sweep below
     // (2^20 points: 663 -> 613 us, 2^22 points: 3514 -> 2687 us)
-    constexpr int64_t CHUNK = (int64_t)1024 * P;
-    for (int64_t n0 = 0; n0 < n_points; n0 += CHUNK) {
-      const int64_t n = n_points - n0 < CHUNK ? n_points - n0 : CHUNK;
+    constexpr int64_t chunk = (int64_t)1 << 19;
+    for (int64_t n0 = 0; n0 < n_points; n0 += chunk) {
+      const int64_t n = n_points - n0 < chunk ? n_points - n0 : chunk;
+      const int per = sweep_wave_points(n, 64 * PPT);
       const void* c = (const char*)coords + n0 * csn * dtype_size(coords_dtype);
-      hipLaunchKernelGGL((hash_fwd_sweep32_k<PPT>), dim3((unsigned)((n + P - 1) / P)), dim3(TILE_THREADS), 0, s, c, coords_dtype, csn,
-                         csd, (const float2*)table, (float*)out + n0 * out_stride_n, out_stride_n, n, g, primes, scale);
+      hipLaunchKernelGGL((hash_fwd_sweep32_k<PPT>), dim3(sweep_groups(n, per)), dim3(TILE_THREADS), 0, s, c, coords_dtype, csn,
+                         csd, (const float2*)table, (float*)out + n0 * out_stride_n, out_stride_n, n, per, g, primes, scale);
     }
     return check_launch("hash_fwd_sweep32");
   }
-  // The level sweep wants at least one workgroup per compute unit; below that the staged kernel's smaller tiles
-  // spread the points over more of the chip.
-  if (!(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FWD_STAGED)) && n_points >= SWEEP_MIN_POINTS &&
-      tiled_ok(geom, table_dtype, out, out_stride_n)) {
-    constexpr int PPT = SWEEP_PPT;
-    constexpr int P = TILE_THREADS * PPT;
+  // 16-bit tables in three dimensions, and over four corners in two
+  if (!(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FWD_STAGED)) && n_points >= (g.dims == 2 ? SWEEP_MIN_POINTS_D2 : SWEEP_MIN_POINTS) &&
+      tiled_ok(geom, table_dtype, out, out_stride_n, 2, g.dims == 2 ? 2 : 3)) {
     // level 0 in LDS where it is dense and small (19.6 KB at resolution 16): worth about 1 % (its rows mostly hit L1 anyway)
-    const bool lds0 = geom->first_hash_level > 0 && geom->rows[0] * 4 <= 32 * 1024;
+    const bool lds0 = g.dims == 3 && geom->first_hash_level > 0 && geom->rows[0] * 4 <= 32 * 1024;
     const size_t lds = lds0 ? (size_t)geom->rows[0] * 4 : 0;
-    const void* kern = table_dtype == NF_F16 ? (lds0 ? (const void*)hash_fwd_sweep_k<F16, PPT, 3, true> : (const void*)hash_fwd_sweep_k<F16, PPT, 3>)
-                                             : (lds0 ? (const void*)hash_fwd_sweep_k<BF16, PPT, 3, true> : (const void*)hash_fwd_sweep_k<BF16, PPT, 3>);
     const uint32_t* tab = (const uint32_t*)table;
     // Launches of at most 2^20 points: the workgroups of one launch are (nearly) all resident and walk the levels
     // together; in one launch of 2^22 points later rounds of workgroups meet earlier ones at other levels and the
     // tables compete for L2 (1545 us against 1324 us in four launches; 677 against 661 us at 2^21).
-    constexpr int64_t CHUNK = (int64_t)1 << 20;
-    for (int64_t n0 = 0; n0 < n_points; n0 += CHUNK) {
-      const int64_t n = n_points - n0 < CHUNK ? n_points - n0 : CHUNK;
+    constexpr int64_t chunk = (int64_t)1 << 20;
+    for (int64_t n0 = 0; n0 < n_points; n0 += chunk) {
+      int64_t n = n_points - n0 < chunk ? n_points - n0 : chunk;
+      int per = sweep_wave_points(n, 64 * SWEEP_PPT);
+      const void* kern = table_dtype == NF_F16 ? sweep_kernel<F16>(per, g.dims, lds0) : sweep_kernel<BF16>(per, g.dims, lds0);
       const void* c = (const char*)coords + n0 * csn * dtype_size(coords_dtype);
       uint16_t* o = (uint16_t*)out + n0 * out_stride_n;
       void* args[] = {(void*)&c, (void*)&coords_dtype, (void*)&csn, (void*)&csd, (void*)&tab, (void*)&o, (void*)&out_stride_n,
-                      (void*)&n, (void*)&g, (void*)&primes, (void*)&scale};
-      const hipError_t e = hipLaunchKernel(kern, dim3((unsigned)((n + P - 1) / P)), dim3(TILE_THREADS), args, lds, s);
+                      (void*)&n, (void*)&per, (void*)&g, (void*)&primes, (void*)&scale};
+      const hipError_t e = hipLaunchKernel(kern, dim3(sweep_groups(n, per)), dim3(TILE_THREADS), args, lds, s);
       if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(hash_fwd_sweep): %s", hipGetErrorString(e));
     }
-    return check_launch("hash_fwd_sweep");
-  }
-  // two dimensions: the same sweep over four corners
-  if (!(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FWD_STAGED)) && n_points >= SWEEP_MIN_POINTS &&
-      tiled_ok(geom, table_dtype, out, out_stride_n, 2, 2)) {
-    constexpr int PPT = SWEEP_PPT;
-    constexpr int P = TILE_THREADS * PPT;
-    dim3 grid((unsigned)((n_points + P - 1) / P));
-    if (table_dtype == NF_F16)
-      hipLaunchKernelGGL((hash_fwd_sweep_k<F16, PPT, 2>), grid, dim3(TILE_THREADS), 0, s, coords, coords_dtype, csn, csd,
-                         (const uint32_t*)table, (uint16_t*)out, out_stride_n, n_points, g, primes, scale);
-    else
-      hipLaunchKernelGGL((hash_fwd_sweep_k<BF16, PPT, 2>), grid, dim3(TILE_THREADS), 0, s, coords, coords_dtype, csn, csd,
-                         (const uint32_t*)table, (uint16_t*)out, out_stride_n, n_points, g, primes, scale);
     return check_launch("hash_fwd_sweep");
   }
   // batches below the sweep's minimum: a thread per (point, level)

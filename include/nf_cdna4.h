@@ -213,6 +213,18 @@ int nf_mlp_bwd_rounded(const void* x, int64_t x_stride, const void* dy, int64_t 
                        int x_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 int64_t nf_mlp_bwd_rounded_workspace_bytes(int d_in, int d_hidden, int d_out);
 
+/* nf_mlp_bwd_rounded with the gradients in grad_dtype: `dtype`, or NF_F32 (the sums as they are, for float32 parameters whose
+ * float16 copies the network ran on). */
+int nf_mlp_bwd_summed(const void* x, int64_t x_stride, const void* dy, int64_t dy_stride, void* dx, int64_t dx_stride,
+                      const void* w_in, const void* b_in, const void* w_hid, const void* b_hid, const void* w_out,
+                      const void* b_out, void* dw_in, void* db_in, void* dw_hid, void* db_hid, void* dw_out,
+                      void* db_out, int64_t rows, int d_in, int d_hidden, int d_out, int depth, int act, int dtype,
+                      int x_dtype, int grad_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* n (<= 8) float32 arrays of count[k] values cast to float16 in one launch: piece k starts at dst plus the counts before it,
+ * each rounded up to a multiple of 8. src and count are host arrays. */
+int nf_cast_pieces_f16(const float* const* src, const int64_t* count, int n, void* dst, void* stream);
+
 /* Reversible MLP of `blocks` additive couplings over rows of width 2*half:
  *   y1 = x1 + F_k(x2),  y2 = x2 + G_k(y1),  F/G(u) = act(u W1^T + b1) W2^T + b2.
  * w1, w2 [blocks*2*half, half] (F_k then G_k per block), b1, b2 [blocks*2, half] or NULL. */

@@ -24,3 +24,80 @@ def test_forward_sweep_deals_out_every_point(N, dims, dtype, monkeypatch):
         monkeypatch.setattr(hk, "_FLAGS", flags)
         outs.append(hk.hash_encoding(x, table, None, None, T, lo, hi, L))
     assert torch.equal(outs[0], outs[1])
+
+
+def _grads(tensors):
+    return [None if t is None else t.grad for t in tensors]
+
+
+@pytest.mark.parametrize("depth,bias,dtype", [(1, True, torch.bfloat16), (2, False, torch.float16), (4, True, torch.float32)])
+def test_mlp_node_equals_the_python_function(depth, bias, dtype):
+    """The native node and the autograd Function of the same name come to the same launches: the same bits."""
+    from triton_helpers_amd.layers.fully_fused_mlp.kernel import _fully_fused_mlp, fully_fused_mlp
+
+    torch.manual_seed(4)
+    u = lambda *s: (torch.rand(*s, device=DEV) - 0.5).to(dtype)  # noqa: E731
+    H, n = 64, depth - 1
+    base = [u(3, 41, 32), u(H, 32), u(H) if bias else None, u(16, H), u(16) if bias else None, u(n * H, H) if n else None, u(n, H) if n and bias else None]
+    got = []
+    for fn in (fully_fused_mlp, _fully_fused_mlp.apply):
+        leaves = [None if t is None else t.clone().requires_grad_() for t in base]
+        y = fn(*leaves, "relu")
+        y.backward(torch.ones_like(y))
+        got.append([y.detach(), *_grads(leaves)])
+    for a, b in zip(*got):
+        assert (a is None and b is None) or (a.dtype == b.dtype and torch.allclose(a.float(), b.float(), rtol=1e-5, atol=1e-6))
+
+
+@pytest.mark.parametrize("depth,act", [(2, "relu"), (3, "relu"), (2, "silu")])
+def test_mlp_under_autocast(depth, act):
+    """float32 parameters under autocast: float16 operands, float32 gradients of the parameters, equal to those of float16
+    parameters up to the rounding that those end with."""
+    from triton_helpers_amd.layers.fully_fused_mlp import fully_fused_mlp
+
+    torch.manual_seed(5)
+    u = lambda *s: torch.rand(*s, device=DEV) - 0.5  # noqa: E731
+    H, n = 64, depth - 1
+    base = [u(1, 1000, 32), u(H, 32), u(H), u(16, H), u(16), u(n * H, H), u(n, H)]
+    got = []
+    for cast in (True, False):
+        leaves = [(t.clone() if cast else t.half()).requires_grad_() for t in base]
+        with torch.autocast("cuda", dtype=torch.float16, enabled=cast):
+            y = fully_fused_mlp(*leaves, activation=act)
+        assert y.dtype == torch.float16
+        y.backward(torch.full_like(y, 0.01))
+        got.append([y.detach(), *_grads(leaves)])
+    assert torch.equal(got[0][0], got[1][0])
+    for a, b in zip(got[0][1:], got[1][1:]):
+        assert a.dtype == torch.float32
+        torch.testing.assert_close(a, b.float(), rtol=2e-3, atol=2e-3 * float(b.abs().max()))
+
+
+@pytest.mark.parametrize("case", ["cpu table", "features", "coords grad", "float64", "small table", "strided"])
+def test_hash_node_hands_unusual_calls_to_the_python_function(case):
+    from triton_helpers_amd.layers.hash_encoding import hash_encoding
+
+    geo = dict(max_entries_per_level=2**10, min_res=4, max_res=32, levels=4)
+    E = O.level_row_offsets(4, 2**10, 3, 4, 32)[-1]
+    x, table = torch.rand(100, 3, device=DEV), torch.randn(E, 2, device=DEV)
+    want = hash_encoding(x, table, **geo)
+    if case == "cpu table":
+        with pytest.raises(AssertionError):
+            hash_encoding(x, table.cpu(), **geo)
+    elif case == "features":
+        out = hash_encoding(x, table, torch.ones(100, 3, device=DEV), **geo)
+        assert torch.equal(out[:, :8], want) and torch.equal(out[:, 8:], torch.ones(100, 3, device=DEV))
+    elif case == "coords grad":
+        with pytest.raises(AssertionError):
+            hash_encoding(x.clone().requires_grad_(), table, **geo)
+    elif case == "float64":
+        with pytest.raises(TypeError):
+            hash_encoding(x.double(), table, **geo)
+    elif case == "small table":
+        with pytest.raises(AssertionError):
+            hash_encoding(x, table[:-1], **geo)
+    else:
+        wide = torch.zeros(100, 5, device=DEV)
+        wide[:, ::2] = x
+        assert torch.equal(hash_encoding(wide[:, ::2], table, **geo), want)
+        assert torch.equal(hash_encoding(x.view(4, 25, 3), table, **geo).view(100, 8), want)

@@ -13,6 +13,7 @@ from typing import Optional
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "libnf_cdna4.so"
+NATIVE_PATH = LIB_PATH.with_name("_native.so")
 
 NF_ABI_VERSION = 9
 NF_F32, NF_F16, NF_BF16 = 0, 1, 2
@@ -46,6 +47,8 @@ EXPORTS = (
     "nf_mlp_workspace_bytes",
     "nf_mlp_bwd_rounded",
     "nf_mlp_bwd_rounded_workspace_bytes",
+    "nf_mlp_bwd_summed",
+    "nf_cast_pieces_f16",
     "nf_revmlp_fwd",
     "nf_revmlp_bwd",
 )
@@ -108,12 +111,16 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.nf_mlp_fwd.argtypes = [P, I64, P, I64, P, P, P, P, P, P, I64, I, I, I, I, I, I, I, P, I64, P]
     lib.nf_mlp_bwd_rounded.restype = c_int
     lib.nf_mlp_bwd_rounded.argtypes = [P, I64, P, I64, P, I64, P, P, P, P, P, P, P, P, P, P, P, P, I64, I, I, I, I, I, I, I, P, I64, P]
+    lib.nf_mlp_bwd_summed.restype = c_int
+    lib.nf_mlp_bwd_summed.argtypes = [P, I64, P, I64, P, I64, P, P, P, P, P, P, P, P, P, P, P, P, I64, I, I, I, I, I, I, I, I, P, I64, P]
     lib.nf_mlp_bwd_rounded_workspace_bytes.restype = I64
     lib.nf_mlp_bwd_rounded_workspace_bytes.argtypes = [I, I, I]
     lib.nf_mlp_workspace_bytes.restype = I64
     lib.nf_mlp_workspace_bytes.argtypes = [I64, I, I, I, I, I]
     lib.nf_mlp_bwd.restype = c_int
     lib.nf_mlp_bwd.argtypes = [P, I64, P, I64, P, I64, P, P, P, P, P, P, P, P, P, P, P, P, I64, I, I, I, I, I, I, I, P, I64, P]
+    lib.nf_cast_pieces_f16.restype = c_int
+    lib.nf_cast_pieces_f16.argtypes = [P, P, I, P, P]
     lib.nf_revmlp_fwd.restype = c_int
     lib.nf_revmlp_fwd.argtypes = [P, I64, P, I64, P, P, P, P, I64, I, I, I, I, P]
     lib.nf_revmlp_bwd.restype = c_int
@@ -144,6 +151,22 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_native = None
+
+
+def native():
+    """The operators' host side (``csrc/host_native.cpp``): imported once, raises ``NativeLibraryError`` if it is absent."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise NativeLibraryError(f"cannot load {NATIVE_PATH}: {e}: build it with `python -m triton_helpers_amd.build`") from e
+        _native = module
+    return _native
+
+
 def check(rc: int, what: str) -> None:
     """Turn a non-zero return code of the library into ``RuntimeError``."""
     if rc != 0:
@@ -166,30 +189,10 @@ def current_stream(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-class GradBuffers:
-    """float32 zero accumulators shaped like the given tensors (``None`` stays ``None``), carved out of one buffer
-    so that a single fill kernel clears them all and a single cast kernel rounds them all to the parameters' dtype.
-    The kernels only need addresses, so no view tensors are made for the accumulators (each tensor op costs the host
-    a few microseconds, which is what bounds a small step)."""
-
-    def __init__(self, *tensors):
-        self._like = tensors
-        self._offsets, off = [], 0
-        for t in tensors:
-            self._offsets.append(off)
-            if t is not None:
-                off += (t.numel() + 3) // 4 * 4  # 16-byte aligned pieces
-        self.flat = torch.zeros(off, dtype=torch.float32, device=next(t for t in tensors if t is not None).device) if off else None
-
-    def pointers(self):
-        """Device addresses of the accumulators (``None`` where the tensor is absent)."""
-        base = self.flat.data_ptr() if self.flat is not None else 0
-        return tuple(None if t is None else base + 4 * o for t, o in zip(self._like, self._offsets))
-
-    def rounded(self, dtype):
-        """The accumulators rounded once to ``dtype`` (what autograd would do tensor by tensor), as views."""
-        if self.flat is None:
-            return tuple(None for _ in self._like)
-        flat = self.flat if dtype == torch.float32 else self.flat.to(dtype)
-        return tuple(None if t is None else flat.as_strided(t.shape, t.stride(), o) if t.is_contiguous()
-                     else flat[o:o + t.numel()].view(t.shape) for t, o in zip(self._like, self._offsets))
+def rows2d(t: torch.Tensor, width: int) -> torch.Tensor:
+    """2-D view ``(N, width)`` with unit inner stride (copies only when the layout forces it)."""
+    t2 = t.reshape(-1, width)
+    # rows that overlap (an expanded / broadcast tensor has row stride 0) or a strided inner dimension: copy
+    if t2.stride(1) != 1 or (t2.shape[0] > 1 and t2.stride(0) < width):
+        t2 = t2.contiguous()
+    return t2

@@ -2,7 +2,8 @@
 
 ``python -m triton_helpers_amd.build`` cross-compiles every ``csrc/*.hip`` with
 ``hipcc --offload-arch=gfx950`` (no GPU needed) and links them into
-``triton_helpers_amd/libnf_cdna4.so`` next to this file.
+``triton_helpers_amd/libnf_cdna4.so`` next to this file, then compiles the host side of the
+operators (``csrc/host_native.cpp``) into ``triton_helpers_amd/_native.so``.
 """
 from __future__ import annotations
 
@@ -10,6 +11,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 from typing import List
@@ -19,6 +21,7 @@ CSRC = PKG_DIR / "csrc"
 INCLUDE = PKG_DIR.parent / "include"
 LIB_PATH = PKG_DIR / "libnf_cdna4.so"
 BUILD_DIR = PKG_DIR / "build"
+NATIVE_PATH = PKG_DIR / "_native.so"
 
 ARCH = "gfx950"
 COMMON_FLAGS = [
@@ -61,8 +64,24 @@ def sources() -> List[Path]:
     return sorted(CSRC.glob("*.hip"))
 
 
+def native_command(out: Path) -> List[str]:
+    """The operators' host side: a CPython module on torch's headers, linked to the kernel library beside it."""
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("a C++ compiler is required to build _native.so")
+    rocm = Path(_hipcc()).resolve().parent.parent
+    includes = [*include_paths(), str(rocm / "include"), sysconfig.get_paths()["include"]]
+    return [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}", *(f"-isystem{d}" for d in includes),
+            str(CSRC / "host_native.cpp"), "-o", str(out), f"-L{PKG_DIR}", f"-l:{LIB_PATH.name}", *(f"-L{d}" for d in library_paths()),
+            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+
+
 def build(verbose: bool = True, jobs: int = 8) -> Path:
-    """Compile all kernels and link the shared library; returns its path."""
+    """Compile all kernels, link the shared library and the native host module on it; returns the library's path."""
     hipcc = _hipcc()
     BUILD_DIR.mkdir(exist_ok=True)
     objs = []
@@ -81,6 +100,9 @@ def build(verbose: bool = True, jobs: int = 8) -> Path:
     tmp = LIB_PATH.with_suffix(".so.tmp")
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)], verbose)
     os.replace(tmp, LIB_PATH)
+    tmp = NATIVE_PATH.with_suffix(".so.tmp")
+    _run(native_command(tmp), verbose)
+    os.replace(tmp, NATIVE_PATH)
     return LIB_PATH
 
 

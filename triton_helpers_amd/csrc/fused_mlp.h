@@ -142,7 +142,7 @@ int launch_mlp_bwd2_w8(const MlpArgs& a, int dtype, hipStream_t s, bool* handled
 // (dw_in, db_in, dw_hid, db_hid, dw_out, db_out; NULL entries skipped); workspace: mlp_bwd2_w8_rounded_bytes().
 // Also covers the shapes of launch_mlp_bwd2_ws.
 size_t mlp_bwd2_w8_rounded_bytes(int d_in, int d_hidden, int d_out);
-int launch_mlp_bwd2_w8_rounded(const MlpArgs& a, int dtype, void* const out[6], void* workspace, hipStream_t s, bool* handled);
+int launch_mlp_bwd2_w8_rounded(const MlpArgs& a, int dtype, int grad_dtype, void* const out[6], void* workspace, hipStream_t s, bool* handled);
 
 
 // One hidden layer, width 64, ReLU, with d_in > 32 or d_out > 16 (aligned rows, extents below 2^31 bytes): chain and

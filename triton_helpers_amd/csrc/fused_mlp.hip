@@ -910,14 +910,15 @@ extern "C" int64_t nf_mlp_bwd_rounded_workspace_bytes(int d_in, int d_hidden, in
   return (int64_t)mlp_bwd2_w8_rounded_bytes(d_in, d_hidden, d_out);
 }
 
-extern "C" int nf_mlp_bwd_rounded(const void* x, int64_t x_stride, const void* dy, int64_t dy_stride, void* dx, int64_t dx_stride,
-                                  const void* w_in, const void* b_in, const void* w_hid, const void* b_hid, const void* w_out,
-                                  const void* b_out, void* dw_in, void* db_in, void* dw_hid, void* db_hid, void* dw_out,
-                                  void* db_out, int64_t rows, int d_in, int d_hidden, int d_out, int depth, int act, int dtype,
-                                  int x_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+extern "C" int nf_mlp_bwd_summed(const void* x, int64_t x_stride, const void* dy, int64_t dy_stride, void* dx, int64_t dx_stride,
+                                 const void* w_in, const void* b_in, const void* w_hid, const void* b_hid, const void* w_out,
+                                 const void* b_out, void* dw_in, void* db_in, void* dw_hid, void* db_hid, void* dw_out,
+                                 void* db_out, int64_t rows, int d_in, int d_hidden, int d_out, int depth, int act, int dtype,
+                                 int x_dtype, int grad_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
   if (int rc = validate(rows, d_in, d_hidden, d_out, depth, act, dtype)) return rc;
   NF_REQUIRE(dtype != NF_F32 && (x_dtype == NF_F16 || x_dtype == NF_BF16), NF_EUNSUPPORTED,
              "rounded weight gradients: 16-bit tensors only (dtype code %d, x_dtype code %d)", dtype, x_dtype);
+  NF_REQUIRE(grad_dtype == dtype || grad_dtype == NF_F32, NF_EINVAL, "grad_dtype code %d: the parameters' (%d) or float32", grad_dtype, dtype);
   NF_REQUIRE(rows > 0, NF_EUNSUPPORTED, "rounded weight gradients: no rows (the buffers would stay unwritten)");
   const bool identity = identity_layer_applies(d_hidden, depth, act, dtype);  // one hidden layer: see identity_layer()
   NF_REQUIRE(x && dy && w_in && w_out && dw_in && dw_out && (identity || (w_hid && dw_hid)), NF_EINVAL, "NULL pointer argument");
@@ -942,8 +943,17 @@ extern "C" int nf_mlp_bwd_rounded(const void* x, int64_t x_stride, const void* d
   }
   void* const out[6] = {dw_in, db_in, dw_hid, db_hid, dw_out, db_out};
   bool handled = false;
-  const int rc = launch_mlp_bwd2_w8_rounded(a, dtype, out, workspace, (hipStream_t)stream, &handled);
+  const int rc = launch_mlp_bwd2_w8_rounded(a, dtype, grad_dtype, out, workspace, (hipStream_t)stream, &handled);
   if (rc != 0 || handled) return rc;
   return fail(NF_EUNSUPPORTED, "rounded weight gradients: built for one hidden-to-hidden layer, d_hidden = 64, d_in <= 64, d_out <= 64, "
                                "ReLU, 8-byte aligned rows and (beyond d_in 32 / d_out 16) x stored like the weights (nothing was launched; use nf_mlp_bwd)");
+}
+
+extern "C" int nf_mlp_bwd_rounded(const void* x, int64_t x_stride, const void* dy, int64_t dy_stride, void* dx, int64_t dx_stride,
+                                  const void* w_in, const void* b_in, const void* w_hid, const void* b_hid, const void* w_out,
+                                  const void* b_out, void* dw_in, void* db_in, void* dw_hid, void* db_hid, void* dw_out,
+                                  void* db_out, int64_t rows, int d_in, int d_hidden, int d_out, int depth, int act, int dtype,
+                                  int x_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  return nf_mlp_bwd_summed(x, x_stride, dy, dy_stride, dx, dx_stride, w_in, b_in, w_hid, b_hid, w_out, b_out, dw_in, db_in, dw_hid, db_hid, dw_out,
+                           db_out, rows, d_in, d_hidden, d_out, depth, act, dtype, x_dtype, dtype, workspace, workspace_bytes, stream);
 }

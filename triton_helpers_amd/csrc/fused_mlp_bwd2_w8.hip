@@ -51,7 +51,7 @@ __global__ __launch_bounds__(1024) void mlp_sum_slots_k(const float* partials, i
   int k = 0;
 #pragma unroll
   for (int q = 1; q < 6; ++q) k += i >= pc.first[q];
-  if (pc.out[k] != nullptr) reinterpret_cast<uint16_t*>(pc.out[k])[i - pc.first[k]] = T::from_f32(total);
+  if (pc.out[k] != nullptr) reinterpret_cast<typename T::storage*>(pc.out[k])[i - pc.first[k]] = T::from_f32(total);
 }
 
 template <typename T>
@@ -110,7 +110,7 @@ int launch_mlp_bwd2_w8(const MlpArgs& a, int dtype, hipStream_t s, bool* handled
   return dtype == NF_BF16 ? launch2_w8<BF16>(a, s) : launch2_w8<F16>(a, s);
 }
 
-int launch_mlp_bwd2_w8_rounded(const MlpArgs& a0, int dtype, void* const out[6], void* workspace, hipStream_t s, bool* handled) {
+int launch_mlp_bwd2_w8_rounded(const MlpArgs& a0, int dtype, int grad_dtype, void* const out[6], void* workspace, hipStream_t s, bool* handled) {
   *handled = false;
   const bool decoder = w8_shape(a0, dtype);
   MlpArgs a = a0;
@@ -146,7 +146,9 @@ int launch_mlp_bwd2_w8_rounded(const MlpArgs& a0, int dtype, void* const out[6],
   const float* part = a.partials;
   const int64_t st = a.partial_stride;
   void* args[] = {(void*)&part, (void*)&blocks, (void*)&st, (void*)&pc};
-  const void* kern = dtype == NF_BF16 ? (const void*)mlp_sum_slots_k<BF16> : (const void*)mlp_sum_slots_k<F16>;
+  const void* kern = grad_dtype == NF_F32    ? (const void*)mlp_sum_slots_k<F32>
+                     : grad_dtype == NF_BF16 ? (const void*)mlp_sum_slots_k<BF16>
+                                             : (const void*)mlp_sum_slots_k<F16>;
   const hipError_t e = hipLaunchKernel(kern, dim3((unsigned)((at + 63) / 64)), dim3(1024), args, 0, s);
   if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(mlp_sum_slots): %s", hipGetErrorString(e));
   return check_launch("mlp_sum_slots");

@@ -120,37 +120,11 @@ def _check_storage(x: Tensor, w_in: Tensor, *others: Optional[Tensor]) -> None:
     assert x.device.type == "cuda", "All tensors must be on a GPU device"
 
 
-def _rows2d(t: Tensor, width: int) -> Tensor:
-    t2 = t.reshape(-1, width)
-    # rows that overlap (an expanded / broadcast tensor has row stride 0) or a strided inner dimension: copy
-    if t2.stride(1) != 1 or (t2.shape[0] > 1 and t2.stride(0) < width):
-        t2 = t2.contiguous()
-    return t2
+_rows2d = _lib.rows2d
 
 
 def _half(t: Optional[Tensor]) -> Optional[Tensor]:
     return None if t is None else t.to(torch.float16)
-
-
-def _c(t: Optional[Tensor]) -> Optional[Tensor]:
-    return None if t is None else (t if t.is_contiguous() else t.contiguous())
-
-
-_workspace_sizes: dict = {}
-
-
-def _workspace(lib, rows2d: Tensor, d_hidden: int, depth: int, activation: str, backward: bool, dtype: torch.dtype):
-    """Scratch for networks that run as several launches (none for the usual depths) and for the float32 backward."""
-    key = (rows2d.shape[0], d_hidden, depth, activation, backward, dtype)
-    n = _workspace_sizes.get(key)
-    if n is None:
-        n = lib.nf_mlp_workspace_bytes(rows2d.shape[0], d_hidden, depth, _lib.NF_ACT[activation], int(backward),
-                                       _lib.dtype_code(dtype))
-        if len(_workspace_sizes) < 4096:
-            _workspace_sizes[key] = n
-    if n == 0:
-        return None, 0
-    return torch.empty(n, dtype=torch.uint8, device=rows2d.device), n
 
 
 class _fully_fused_mlp(Function):
@@ -195,125 +169,22 @@ class _fully_fused_mlp(Function):
         ctx.save_for_backward(x, w_in, b_in, w_out, b_out, w_hid, b_hid)
         ctx.activation = activation
         ctx.fp16_acc = fp16_acc
-        ctx.depth = depth
         ctx.wide = wide = w_in.dtype == torch.float32 and _FLOAT32_OPERANDS == "float16"
         if wide:  # float16 operands, float32 accumulation and results
             x, w_in, b_in, w_out, b_out, w_hid, b_hid = (_half(t) for t in (x, w_in, b_in, w_out, b_out, w_hid, b_hid))
-        w_in, b_in, w_out, b_out, w_hid, b_hid = (_c(t) for t in (w_in, b_in, w_out, b_out, w_hid, b_hid))
-        x2 = _rows2d(x, D_in)
-        o = x.new_empty((B, L, D_out), dtype=w_in.dtype)
-        o2 = o.view(-1, D_out)
-        lib = _lib.load()
-        ws, ws_bytes = _workspace(lib, x2, D_hidden, depth, activation, False, w_in.dtype)
-        rc = lib.nf_mlp_fwd(
-            x2.data_ptr(), x2.stride(0), o2.data_ptr(), o2.stride(0),
-            w_in.data_ptr(), _lib.ptr(b_in), _lib.ptr(w_hid), _lib.ptr(b_hid), w_out.data_ptr(), _lib.ptr(b_out),
-            x2.shape[0], D_in, D_hidden, D_out, depth, _lib.NF_ACT[activation], _lib.dtype_code(w_in.dtype),
-            _lib.dtype_code(x.dtype), _lib.ptr(ws), ws_bytes, _lib.current_stream(x.device),
-        )
-        _lib.check(rc, "nf_mlp_fwd")
+        o = _lib.native().mlp_launch_forward(x, w_in, b_in, w_out, b_out, w_hid, b_hid, _lib.NF_ACT[activation])
         return o.float() if wide else o
 
     @staticmethod
     @torch.amp.custom_bwd(device_type="cuda")
     def backward(ctx, do: Tensor):
-        x, w_in, b_in, w_out, b_out, w_hid, b_hid = ctx.saved_tensors
-        B, L, D_in = x.shape
-        D_hidden = w_in.shape[0]
-        D_out = w_out.shape[0]
-        wide = ctx.wide
-        if wide:
-            x, w_in, b_in, w_out, b_out, w_hid, b_hid = (_half(t) for t in (x, w_in, b_in, w_out, b_out, w_hid, b_hid))
-        if do.dtype != w_in.dtype:
-            do = do.to(w_in.dtype)
-        converts = (ctx.depth == 2 and D_hidden > 32) or (ctx.depth == 1 and D_hidden == 64)
-        if x.dtype != w_in.dtype and not (w_in.dtype != torch.float32 and converts and ctx.activation == "relu"):
-            x = x.to(w_in.dtype)  # only the ReLU backward of one or two 64-wide hidden layers converts on the fly
-        do2 = _rows2d(do, D_out)
-        need_dx = ctx.needs_input_grad[0]
-        decoder = D_in <= 32 and D_out <= 16  # the wider shapes need x in the parameters' dtype
-        # (one hidden layer runs on the same kernels behind an identity layer that the library supplies)
-        if (not wide and w_in.dtype != torch.float32 and ctx.depth in (1, 2) and D_hidden == 64 and D_in <= 64 and D_out <= 64
-                and (decoder or x.dtype == w_in.dtype)
-                and D_in % 4 == 0 and D_out % 4 == 0 and ctx.activation == "relu" and do2.shape[0] > 0):
-            done = _backward_rounded(x, do2, w_in, b_in, w_out, b_out, w_hid, b_hid, need_dx, D_in, D_hidden, D_out, ctx.depth)
-            if done is not None:
-                return done
-        grads = _lib.GradBuffers(w_in, b_in, w_out, b_out, w_hid, b_hid)
-        p_dw_in, p_db_in, p_dw_out, p_db_out, p_dw_hid, p_db_hid = grads.pointers()
-        lib = _lib.load()
-        ws, ws_bytes = _workspace(lib, do2, D_hidden, ctx.depth, ctx.activation, True, w_in.dtype)
-        while True:
-            x2 = _rows2d(x, D_in)
-            dx = x.new_empty(x.shape) if need_dx else None
-            rc = lib.nf_mlp_bwd(
-                x2.data_ptr(), x2.stride(0), do2.data_ptr(), do2.stride(0),
-                _lib.ptr(dx), D_in,
-                w_in.data_ptr(), _lib.ptr(b_in), _lib.ptr(w_hid), _lib.ptr(b_hid), w_out.data_ptr(), _lib.ptr(b_out),
-                p_dw_in, p_db_in, p_dw_hid, p_db_hid, p_dw_out, p_db_out,
-                x2.shape[0], D_in, D_hidden, D_out, ctx.depth, _lib.NF_ACT[ctx.activation], _lib.dtype_code(w_in.dtype),
-                _lib.dtype_code(x.dtype), _lib.ptr(ws), ws_bytes, _lib.current_stream(x.device),
-            )
-            if rc == _lib.NF_EUNSUPPORTED and x.dtype != w_in.dtype:
-                x = x.to(w_in.dtype)  # a shape / alignment the converting backward does not cover: cast first
-                continue
-            break
-        _lib.check(rc, "nf_mlp_bwd")
-        # float32 accumulators, rounded once to the parameters' dtype (one kernel for all of them)
-        dw_in, db_in, dw_out, db_out, dw_hid, db_hid = grads.rounded(torch.float32 if wide else w_in.dtype)
-        if wide and dx is not None:
+        tensors = ctx.saved_tensors
+        if ctx.wide:
+            tensors = tuple(_half(t) for t in tensors)
+        dx, *grads = _lib.native().mlp_launch_backward(*tensors, _lib.NF_ACT[ctx.activation], do, ctx.needs_input_grad[0], ctx.wide)
+        if ctx.wide and dx is not None:
             dx = dx.float()
-        return dx, dw_in, db_in, dw_out, db_out, dw_hid, db_hid, None, None
-
-
-_rounded_plans: dict = {}
-
-
-def _rounded_plan(lib, like, D_in, D_hidden, D_out):
-    """Where each gradient sits in the flat buffer (16-byte aligned pieces), its length and the scratch size, per
-    combination of parameter shapes (a handful per process)."""
-    key = tuple(None if t is None else (tuple(t.shape), t.stride(), t.dtype) for t in like)
-    plan = _rounded_plans.get(key)
-    if plan is None:
-        offsets, off = [], 0
-        for t in like:
-            offsets.append(off)
-            if t is not None:
-                off += (t.numel() + 7) // 8 * 8
-        plan = (tuple(offsets), off, lib.nf_mlp_bwd_rounded_workspace_bytes(D_in, D_hidden, D_out))
-        if len(_rounded_plans) < 4096:
-            _rounded_plans[key] = plan
-    return plan
-
-
-def _backward_rounded(x, do2, w_in, b_in, w_out, b_out, w_hid, b_hid, need_dx, D_in, D_hidden, D_out, depth=2):
-    """Backward of the one-hidden-layer ReLU shapes through ``nf_mlp_bwd_rounded``: the weight gradients come back summed
-    in a fixed order and rounded to the parameters' dtype, into one uninitialised buffer (no clearing, no cast kernel).
-    ``None`` when the library declines (rows not 8-byte aligned): the caller takes the general path.  The buffer is
-    allocated per call: its pieces become the ``.grad`` tensors, which a later backward must not overwrite."""
-    lib = _lib.load()
-    like = (w_in, b_in, w_out, b_out, w_hid, b_hid)
-    offsets, total, ws_bytes = _rounded_plan(lib, like, D_in, D_hidden, D_out)
-    flat = torch.empty(total, dtype=w_in.dtype, device=w_in.device)
-    base, es = flat.data_ptr(), flat.element_size()
-    p = [None if t is None else base + es * o for t, o in zip(like, offsets)]
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=w_in.device)
-    x2 = _rows2d(x, D_in)
-    dx = x.new_empty(x.shape) if need_dx else None
-    rc = lib.nf_mlp_bwd_rounded(
-        x2.data_ptr(), x2.stride(0), do2.data_ptr(), do2.stride(0), _lib.ptr(dx), D_in,
-        w_in.data_ptr(), _lib.ptr(b_in), _lib.ptr(w_hid), _lib.ptr(b_hid), w_out.data_ptr(), _lib.ptr(b_out),
-        p[0], p[1], p[4], p[5], p[2], p[3],
-        x2.shape[0], D_in, D_hidden, D_out, depth, _lib.NF_ACT["relu"], _lib.dtype_code(w_in.dtype), _lib.dtype_code(x.dtype),
-        ws.data_ptr(), ws_bytes, _lib.current_stream(x.device),
-    )
-    if rc == _lib.NF_EUNSUPPORTED:
-        return None
-    _lib.check(rc, "nf_mlp_bwd_rounded")
-    g = [None if t is None else flat.as_strided(t.shape, t.stride(), o) if t.is_contiguous() else flat[o:o + t.numel()].view(t.shape)
-         for t, o in zip(like, offsets)]
-    dw_in, db_in, dw_out, db_out, dw_hid, db_hid = g
-    return dx, dw_in, db_in, dw_out, db_out, dw_hid, db_hid, None, None
+        return dx, *grads, None, None
 
 
 def fully_fused_mlp(
@@ -336,4 +207,9 @@ def fully_fused_mlp(
     ``activation`` is one of ``"relu"``, ``"relu2"``, ``"silu"``, ``"none"`` and is applied after every
     layer but the last.
     """
+    if _FLOAT32_OPERANDS == "float32":
+        y = _lib.native().mlp(x, w_in, b_in, w_out, b_out, w_hid, b_hid, activation)
+        if y is not None:
+            return y
+    # float16 operands for float32 tensors, or arguments to be refused
     return _fully_fused_mlp.apply(x, w_in, b_in, w_out, b_out, w_hid, b_hid, activation, fp16_acc)

@@ -18,6 +18,7 @@ Differences, all supersets or accuracy improvements:
 from __future__ import annotations
 
 import math
+from ctypes import addressof
 from typing import Any, Dict, Final, Optional, Tuple
 
 import torch
@@ -81,30 +82,7 @@ def _launch_forward(coords2d: Tensor, embeddings: Tensor, pi: Tensor, out2d: Ten
     _lib.check(rc, "nf_hash_encode_fwd")
 
 
-def _launch_backward(coords2d: Tensor, do2d: Tensor, de: Tensor, pi: Tensor, T: int, min_res: int, max_res: int,
-                     levels: int, scale: float) -> None:
-    N, D = coords2d.shape
-    F = de.shape[-1]
-    geom = level_geometry(T, levels, D, F, min_res, max_res)
-    lib = _lib.load()
-    # scratch for the LDS-tile backward; torch's caching allocator makes this free after the first call
-    ws_bytes = lib.nf_hash_encode_bwd_workspace_bytes(N, geom, _lib.dtype_code(do2d.dtype), _FLAGS)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=coords2d.device) if ws_bytes > 0 else None
-    rc = lib.nf_hash_encode_bwd(
-        coords2d.data_ptr(), _lib.dtype_code(coords2d.dtype), coords2d.stride(0), coords2d.stride(1),
-        do2d.data_ptr(), _lib.dtype_code(do2d.dtype), do2d.stride(0), de.data_ptr(), N,
-        geom, pi.data_ptr(), float(scale), _lib.ptr(ws), ws_bytes, _FLAGS, _lib.current_stream(coords2d.device),
-    )
-    _lib.check(rc, "nf_hash_encode_bwd")
-
-
-def _as_rows(t: Tensor, width: int) -> Tensor:
-    """2-D view ``(N, width)`` with unit inner stride (copies only when the layout forces it)."""
-    t2 = t.reshape(-1, width)
-    # rows that overlap (an expanded / broadcast tensor has row stride 0) or a strided inner dimension: copy
-    if t2.stride(1) != 1 or (t2.shape[0] > 1 and t2.stride(0) < width):
-        t2 = t2.contiguous()
-    return t2
+_as_rows = _lib.rows2d
 
 
 def hash_encoding_table_grad(
@@ -131,13 +109,10 @@ def hash_encoding_table_grad(
     assert pi.numel() >= coords.shape[-1], "Pi must have at least D_in elements"
     de = out if out is not None else torch.zeros(num_embeddings, d_embed, dtype=torch.float32, device=coords.device)
     assert de.dtype == torch.float32 and de.is_contiguous() and de.shape == (num_embeddings, d_embed)
-    coords2d = _flat_coords(coords)
-    do2d = _as_rows(do, do.shape[-1])
-    if do2d.shape[0] >= _REPACK_MIN_POINTS and ((do2d.stride(0) * do2d.element_size()) % 16 != 0 or do2d.data_ptr() % 16 != 0):
-        # gradient rows off 16-byte boundaries (the output carried appended features): the LDS-tile kernels read whole
-        # aligned rows, so the encoding's columns are packed first (one pass instead of scattered atomics per corner)
-        do2d = do2d[:, : levels * d_embed].contiguous()
-    _launch_backward(coords2d, do2d, de, pi, max_entries_per_level, min_res, max_res, levels, scale)
+    assert do.shape[:-1].numel() == coords.shape[:-1].numel() and do.device == coords.device == de.device == pi.device
+    geom = level_geometry(max_entries_per_level, levels, coords.shape[-1], d_embed, min_res, max_res)
+    # scratch for the LDS-tile backward is allocated per call: torch's caching allocator makes that free after the first
+    _lib.native().hash_table_grad(coords, do, de, pi, addressof(geom), float(scale), _FLAGS)
     return de
 
 
@@ -202,6 +177,8 @@ class HashEncoding(torch.autograd.Function):
         if pi.dtype != torch.int64:
             pi = pi.to(torch.int64)
 
+        geom = level_geometry(max_entries_per_level, levels, D_in, D_embed, min_res, max_res)
+        _lib.native().add_geometry(max_entries_per_level, levels, D_in, D_embed, min_res, max_res, addressof(geom), need)
         D_out = D_embed * levels + D_feature
         table = embeddings.detach()
         if not table.is_contiguous():
@@ -275,6 +252,12 @@ def hash_encoding(
     Returns:
         :math:`(..., L \times D_e + D_f)` tensor of the tables' dtype.
     """
+    out = _lib.native().hash_encoding(
+        coord, embeddings, features, pi, max_entries_per_level, min_res, max_res, levels, divider, bwd_divider, scale, _FLAGS
+    )
+    if out is not None:
+        return out
+    # appended features, autocast, a geometry seen for the first time, or arguments to be refused
     return HashEncoding.apply(
         coord, embeddings, pi, features, max_entries_per_level, min_res, max_res, levels, divider, bwd_divider, scale
     )

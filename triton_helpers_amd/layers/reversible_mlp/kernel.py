@@ -29,12 +29,7 @@ from ... import _lib
 _ACTIVATIONS = ("gelu", "relu", "relu2", "silu", "none")
 
 
-def _rows2d(t: Tensor, width: int) -> Tensor:
-    t2 = t.reshape(-1, width)
-    # rows that overlap (an expanded / broadcast tensor has row stride 0) or a strided inner dimension: copy
-    if t2.stride(1) != 1 or (t2.shape[0] > 1 and t2.stride(0) < width):
-        t2 = t2.contiguous()
-    return t2
+_rows2d = _lib.rows2d
 
 
 def _validate(x: Tensor, w1: Tensor, b1: Optional[Tensor], w2: Tensor, b2: Optional[Tensor], activation: str):
@@ -64,25 +59,14 @@ class _reversible_mlp(Function):
     @torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.float16)
     @torch.no_grad()
     def forward(ctx, x: Tensor, w1: Tensor, b1: Optional[Tensor], w2: Tensor, b2: Optional[Tensor], activation: str = "gelu") -> Tensor:
-        H, blocks = _validate(x, w1, b1, w2, b2, activation)
+        _validate(x, w1, b1, w2, b2, activation)
         # float32 tensors run with float16 operands (float32 accumulation) and come back as float32, like the fused MLP
         wide = x.dtype == torch.float32
         if wide:
             x, w1, b1, w2, b2 = (None if t is None else t.to(torch.float16) for t in (x, w1, b1, w2, b2))
-        w1, b1, w2, b2 = (_c(t) for t in (w1, b1, w2, b2))
-        x2 = _rows2d(x, 2 * H)
-        y = x.new_empty(x.shape)
-        y2 = y.view(-1, 2 * H)
-        lib = _lib.load()
-        rc = lib.nf_revmlp_fwd(
-            x2.data_ptr(), x2.stride(0), y2.data_ptr(), y2.stride(0), w1.data_ptr(), _lib.ptr(b1), w2.data_ptr(), _lib.ptr(b2),
-            x2.shape[0], H, blocks, _lib.NF_ACT[activation], _lib.dtype_code(x.dtype), _lib.current_stream(x.device),
-        )
-        _lib.check(rc, "nf_revmlp_fwd")
+        y = _lib.native().reversible_launch_forward(x, w1, b1, w2, b2, _lib.NF_ACT[activation])
         ctx.save_for_backward(y, w1, b1, w2, b2)  # the output, not the input
         ctx.activation = activation
-        ctx.half = H
-        ctx.blocks = blocks
         ctx.wide = wide
         return y.float() if wide else y
 
@@ -90,27 +74,8 @@ class _reversible_mlp(Function):
     @torch.amp.custom_bwd(device_type="cuda")
     @torch.no_grad()
     def backward(ctx, dy: Tensor):
-        y, w1, b1, w2, b2 = ctx.saved_tensors
-        H = ctx.half
-        if dy.dtype != y.dtype:
-            dy = dy.to(y.dtype)
-        y2 = _rows2d(y, 2 * H)
-        dy2 = _rows2d(dy, 2 * H)
-        dx = y.new_empty(y.shape)
-        x_rec = y.new_empty(y.shape)
-
-        grads = _lib.GradBuffers(w1, b1, w2, b2)
-        p_dw1, p_db1, p_dw2, p_db2 = grads.pointers()
-        lib = _lib.load()
-        rc = lib.nf_revmlp_bwd(
-            y2.data_ptr(), y2.stride(0), dy2.data_ptr(), dy2.stride(0), dx.data_ptr(), 2 * H, x_rec.data_ptr(), 2 * H,
-            w1.data_ptr(), _lib.ptr(b1), w2.data_ptr(), _lib.ptr(b2),
-            p_dw1, p_db1, p_dw2, p_db2,
-            y2.shape[0], H, ctx.blocks, _lib.NF_ACT[ctx.activation], _lib.dtype_code(y.dtype), _lib.current_stream(y.device),
-        )
-        _lib.check(rc, "nf_revmlp_bwd")
-        dw1, db1, dw2, db2 = grads.rounded(torch.float32 if ctx.wide else w1.dtype)
-        return (dx.float() if ctx.wide else dx), dw1, db1, dw2, db2, None
+        dx, *grads = _lib.native().reversible_launch_backward(*ctx.saved_tensors, _lib.NF_ACT[ctx.activation], dy, ctx.wide)
+        return (dx.float() if ctx.wide else dx), *grads, None
 
 
 def reversible_mlp(x: Tensor, w1: Tensor, b1: Optional[Tensor], w2: Tensor, b2: Optional[Tensor], activation: str = "gelu") -> Tensor:
@@ -121,6 +86,10 @@ def reversible_mlp(x: Tensor, w1: Tensor, b1: Optional[Tensor], w2: Tensor, b2: 
         - w1, w2: :math:`(\text{blocks} \cdot 2H, H)`; b1, b2: :math:`(\text{blocks} \cdot 2, H)` or ``None``
         - Output: same shape and dtype as ``x``
     """
+    y = _lib.native().reversible(x, w1, b1, w2, b2, activation)
+    if y is not None:
+        return y
+    # float32 tensors, autocast, or arguments to be refused
     return _reversible_mlp.apply(x, w1, b1, w2, b2, activation)
 
 

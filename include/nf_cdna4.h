@@ -96,6 +96,17 @@ int nf_hash_encode_bwd(const void* coords, int coords_dtype, int64_t coords_stri
                        const nf_hash_geom* geom, const int64_t* primes, float scale, void* workspace,
                        int64_t workspace_bytes, int flags, void* stream);
 
+/* The gradient of the whole table in one go: every row of the geometry's levels is WRITTEN, in table_dtype, with the sum over
+ * all points (rounded once from float32; rows that no point touches get zero) -- nothing to clear before the call and
+ * nothing to cast after it.  The sums are added in a fixed order: the same inputs give the same bits.  Runs on the sorted-record
+ * kernels only (D = 2 or 3, batches of 8192 to 2^21 points, rows that they take) and needs the workspace of
+ * nf_hash_encode_bwd_workspace_bytes(); NF_EUNSUPPORTED otherwise, before anything is launched.  (The reference clears and adds
+ * in the table's type, triton_helpers/layers/hash_encoding/kernel.py:636.) */
+int nf_hash_encode_bwd_write(const void* coords, int coords_dtype, int64_t coords_stride_n, int64_t coords_stride_d,
+                             const void* dout, int dout_dtype, int64_t dout_stride_n, void* dtable, int table_dtype,
+                             int64_t n_points, const nf_hash_geom* geom, const int64_t* primes, float scale, void* workspace,
+                             int64_t workspace_bytes, int flags, void* stream);
+
 /* Scratch bytes nf_hash_encode_bwd can use for this call shape and these flags (NF_HASH_FORCE_PLANES gives the
  * size of the smaller variant; tables of at most 2^14 rows per level take a walk without records and ask for
  * 4 bytes -- 8 with a float32 gradient -- per point, level and feature pair unless NF_HASH_BWD_RECORDS is set);

@@ -101,3 +101,52 @@ def test_hash_node_hands_unusual_calls_to_the_python_function(case):
         wide[:, ::2] = x
         assert torch.equal(hash_encoding(wide[:, ::2], table, **geo), want)
         assert torch.equal(hash_encoding(x.view(4, 25, 3), table, **geo).view(100, 8), want)
+
+
+@pytest.mark.parametrize("N,dims,F,T,L,hi,dtype,layout", [
+    (8193, 3, 2, 2**16, 8, 1024, torch.float16, "uniform"),         # one record block and one point
+    (16383, 3, 1, 2**15, 8, 512, torch.bfloat16, "uniform"),        # odd feature counts: one feature in the last pass
+    (16385, 2, 3, 2**16, 8, 2048, torch.float32, "uniform"),
+    (50000, 3, 4, 2**17, 8, 2048, torch.bfloat16, "uniform"),
+    (200001, 3, 2, 2**19, 16, 7006, torch.float16, "corner"),       # all points in one corner: bins of many tasks
+    (200001, 3, 2, 2**16, 16, 1024, torch.float32, "corner"),
+    (2**18 - 1, 3, 2, 2**21, 8, 7006, torch.float16, "uniform"),    # the largest batch of small blocks over a wide level
+    (2**18, 3, 2, 2**21, 8, 7006, torch.float16, "uniform"),        # wide blocks, ragged and not
+    (2**18 + 2049, 3, 2, 2**21, 8, 7006, torch.float32, "corner"),
+    (2**18 + 1, 2, 2, 2**21, 8, 7006, torch.bfloat16, "uniform"),
+    (2**18 + 1, 3, 2, 2**21, 16, 7006, torch.float16, "corner"),    # more bins than can be split
+])
+def test_sorted_backward_writes_the_table(N, dims, F, T, L, hi, dtype, layout):
+    """The backward of the sorted records, added to a float32 table and written in the table's own type: every row against
+    float64 sums over the corner rows, rows that no point touches are zeros, and a second run has the same bits."""
+    from triton_helpers_amd.layers.hash_encoding import kernel as hk
+
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.rand(N, dims, generator=g, device=DEV)
+    if layout == "corner":
+        x[: N // 2] *= 0.05
+    *first, E = O.level_row_offsets(L, T, dims, 16, hi)
+    first = torch.tensor(first, device=DEV).view(1, L, 1)
+    do = torch.randn(N, L * F, generator=g, device=DEV).to(dtype)
+    want = torch.zeros(E, F, device=DEV, dtype=torch.float64)
+    count = torch.zeros(E, device=DEV)
+    for part in range(0, N, 2**16):
+        rows, w = hk.hash_encoding_indices(x[part : part + 2**16], None, T, 16, hi, L, return_weights=True)
+        rows += first
+        d = do[part : part + 2**16].double().view(-1, L, 1, F) * w.double().unsqueeze(-1)
+        want.index_add_(0, rows.reshape(-1), d.reshape(-1, F))
+        count.index_add_(0, rows.reshape(-1), torch.ones(rows.numel(), device=DEV))
+    table = torch.zeros(E, F, device=DEV, dtype=dtype).requires_grad_()
+    grads = []
+    for _ in range(2):
+        table.grad = None
+        hk.hash_encoding(x, table, None, None, T, 16, hi, L).backward(do)
+        grads.append(table.grad)
+    assert grads[0].dtype == dtype and torch.equal(grads[0], grads[1])
+    added = torch.full((E, F), 0.5, device=DEV)
+    hk.hash_encoding_table_grad(x, do, E, F, None, T, 16, hi, L, out=added)
+    atol = 1e-4 + 2e-5 * float(want.abs().max())
+    torch.testing.assert_close(added.double() - 0.5, want, rtol=1e-3, atol=atol)
+    ulp = {torch.float16: 2**-10, torch.bfloat16: 2**-7, torch.float32: 1e-5}[dtype]
+    torch.testing.assert_close(grads[0].double(), want, rtol=ulp, atol=atol)
+    assert not grads[0][count == 0].any()

@@ -36,6 +36,7 @@ EXPORTS = (
     "nf_hash_encode_fwd",
     "nf_hash_encode_bwd",
     "nf_hash_encode_bwd_workspace_bytes",
+    "nf_hash_encode_bwd_write",
     "nf_hash_encode_bwd_static",
     "nf_hash_encode_bwd_static_bytes",
     "nf_hash_encode_indices",
@@ -93,6 +94,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.nf_hash_encode_fwd.argtypes = [P, I, I64, I64, P, I, P, I64, I64, POINTER(HashGeom), P, c_float, I, P]
     lib.nf_hash_encode_bwd.restype = c_int
     lib.nf_hash_encode_bwd.argtypes = [P, I, I64, I64, P, I, I64, P, I64, POINTER(HashGeom), P, c_float, P, I64, I, P]
+    lib.nf_hash_encode_bwd_write.restype = c_int
+    lib.nf_hash_encode_bwd_write.argtypes = [P, I, I64, I64, P, I, I64, P, I, I64, POINTER(HashGeom), P, c_float, P, I64, I, P]
     lib.nf_hash_encode_bwd_workspace_bytes.restype = c_int64
     lib.nf_hash_encode_bwd_workspace_bytes.argtypes = [I64, POINTER(HashGeom), I, I]
     lib.nf_hash_encode_bwd_static.restype = c_int

@@ -197,5 +197,10 @@ bool bwd_direct_applies(int64_t n_points, const nf_hash_geom* geom, int flags);
 int launch_bwd_bin(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
                    float* dtable, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
                    void* workspace, int flags, hipStream_t s);
+// the same with every row of the table's gradient written, in a type of its own, instead of added to float32
+bool bwd_write_applies(int64_t n_points, const nf_hash_geom* geom, int flags);
+int launch_bwd_write(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride, void* table,
+                     int table_dtype, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
+                     void* workspace, hipStream_t s);
 
 }  // namespace nf

@@ -977,6 +977,27 @@ extern "C" int nf_hash_encode_bwd(const void* coords, int coords_dtype, int64_t 
   return check_launch("hash_bwd_generic");
 }
 
+extern "C" int nf_hash_encode_bwd_write(const void* coords, int coords_dtype, int64_t csn, int64_t csd, const void* dout, int dout_dtype,
+                                        int64_t dout_stride_n, void* dtable, int table_dtype, int64_t n_points, const nf_hash_geom* geom,
+                                        const int64_t* primes, float scale, void* workspace, int64_t workspace_bytes, int flags,
+                                        void* stream) {
+  DevGeom g;
+  if (int rc = make_dev_geom(geom, &g)) return rc;
+  NF_REQUIRE(dtype_ok(coords_dtype) && dtype_ok(dout_dtype) && dtype_ok(table_dtype), NF_EINVAL, "unknown dtype code");
+  NF_REQUIRE(dout_stride_n >= (int64_t)g.levels * g.feat, NF_EINVAL, "dout_stride_n=%lld < levels*feat", (long long)dout_stride_n);
+  NF_REQUIRE(scale > 0.0f, NF_EINVAL, "scale must be positive");
+  NF_REQUIRE(n_points >= BIN_MIN_POINTS && bwd_write_applies(n_points, geom, flags) &&
+                 !(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FORCE_ATOMIC | NF_HASH_FORCE_PLANES)),
+             NF_EUNSUPPORTED, "no kernel that writes this gradient in one go (nothing was launched; use nf_hash_encode_bwd)");
+  NF_REQUIRE(coords && dout && dtable && primes && workspace, NF_EINVAL, "NULL pointer argument");
+  const int64_t need = bwd_bin_workspace_bytes(n_points, geom, dout_dtype, flags);
+  NF_REQUIRE(need > 0 && (uintptr_t)dout % (dout_dtype == NF_F32 ? 8 : 4) == 0 && dout_stride_n % 2 == 0, NF_EUNSUPPORTED,
+             "shape or alignment outside the sorted-record kernels (nothing was launched; use nf_hash_encode_bwd)");
+  NF_REQUIRE(workspace_bytes >= need && (uintptr_t)workspace % 16 == 0, NF_EINVAL, "a 16-byte aligned workspace of %lld bytes is needed", (long long)need);
+  return launch_bwd_write(coords, coords_dtype, csn, csd, dout, dout_dtype, dout_stride_n, dtable, table_dtype, n_points, geom, g, primes, scale,
+                          workspace, (hipStream_t)stream);
+}
+
 extern "C" int nf_hash_encode_indices_fast(const void* coords, int coords_dtype, int64_t csn, int64_t csd,
                                            int64_t* out_rows, float* out_w, int64_t n_points, const nf_hash_geom* geom,
                                            const int64_t* primes, float scale, void* stream) {

@@ -4,15 +4,20 @@
 // global atomics is bound by the chip's atomic request rate; accumulating them in LDS needs the contributions to
 // one stretch of the table together.  So the contributions are first sorted by table bin (BIN_ROWS rows):
 //
-//   count   : per (level, bin) the number of records, for the whole batch (histogram) and per workgroup
-//   offsets : exclusive scan of the histogram -> where each bin's records start; list of accumulation tasks
-//   fill    : every workgroup takes FILL_POINTS points and, level by level, sorts their records by bin in LDS
-//             and copies them out in runs, into room reserved with one atomic per (workgroup, bin)
-//   accum   : one workgroup per (bin, slice of its records): the bin's rows live in LDS as two 64-bit integers
+//   fill    : every workgroup takes some hundred consecutive points and, level by level, sorts their records by bin
+//             in LDS and writes them out as one contiguous block, with the place of every bin inside the block
+//   totals  : the number of records of every bin
+//   accum   : a workgroup per compute unit takes task after task, a task being a bin (or, where a bin holds many more records
+//             than others, a share of its blocks): the bin's rows live in LDS as two 64-bit integers
 //             each and every contribution is one integer LDS atomic per feature (float LDS atomics and
 //             compare-and-swap loops are an order of magnitude slower once a few thousand adds are in flight on
-//             a tile); the tile is then converted and added to the gradient table (plain read-modify-write when
-//             the bin has a single slice, atomics otherwise)
+//             a tile); the tile is then converted and written to, or added to, the gradient table -- or to a slot of its
+//             own where the bin has several tasks
+//   reduce  : the slots of every bin with several tasks, summed in a fixed order, into the gradient table
+//
+// A block is self-contained: no pass counts the records beforehand, nothing is reserved with atomics and the blocks leave as
+// whole lines.  (With records in one run per bin for the whole batch, a count pass over all points and two global atomics per
+// workgroup and bin cost 50 us at 2^20 points and the fill wrote scattered pieces.)
 //
 // A record is the pair of corners that differ in x only: 12 bytes {row0 | row1 << 13 inside the bin, w0 and w1 in
 // 19-bit fixed point (rounded to nearest: each contribution is off by at most 2^-20 |dout|), packed 16-bit gradient
@@ -20,7 +25,7 @@
 // a weight.  The two rows of a pair share the bin: on a dense level they are
 // neighbours, on a hashed level the x prime is 1 and  (x+1) ^ a  differs from  x ^ a  only below the lowest zero
 // bit of x.  When they do not (bin border, 13 trailing ones in x) the pair becomes two records with one zero weight
-// each.  The count and fill kernels apply the same rule, so their record counts agree.
+// each.
 //
 // Dense levels whose cells span less than a bin (3-D, 16-bit gradients) take ONE record per point and level instead
 // of four: {row of corner 0 relative to the bin, the three cell fractions in 18 / 16 / 16-bit fixed point, gradient
@@ -31,8 +36,12 @@
 // Integer accumulation: fill also finds max |dout| per level; with 2^e the power of two above it, a contribution
 // w * g is accumulated as round(w * g * 2^(30 - e)), below 2^30 in magnitude, so a task's records cannot
 // overflow 64 bits, the rounding is 2^-30 of the level's largest gradient per contribution, and a task's sum does
-// not depend on the order of its records (tasks of a split bin still meet in float atomics).  A level whose gradient holds an inf or a nan gets nan in every row
-// it touches.
+// not depend on the order of its records.  The tasks of a split bin are added in their order: a gradient has the same bits in
+// every run.  A level whose gradient holds an inf or a nan gets nan in every row it touches.
+//
+// One MI355X, 16 levels of 2^19 rows, fp16, uniform points, gradient of the table in its own type (before: count, offsets, fill
+// and accumulate passes over one run per bin, into a float32 table that was then converted): 8192 points 136 -> 92 us,
+// 2^18 184 -> 143, 2^20 506 -> 374, 2^21 947 -> 676; along rays 2^20 698 -> 431.
 //
 // Arithmetic (cell, corner rows, weights) is the forward's, see hash_encoding.hip.
 #include "hash_common.h"
@@ -44,29 +53,29 @@ constexpr int BIN_ROWS = 1 << BIN_ROWS_LOG2;  // rows per bin (two 64-bit sums e
 constexpr uint32_t BIN_MASK = BIN_ROWS - 1;
 constexpr int W_BITS = 19;
 constexpr uint32_t W_MAX = (1u << W_BITS) - 1u;
-constexpr int FILL_POINTS = 1024;              // points (= threads) per workgroup of count and fill
-constexpr int FILL_RECORDS = FILL_POINTS * 8; // most records a workgroup stages per level
+// A fill workgroup (a block of records per level): small ones leave four to a unit, each covering the others' barriers.  With
+// more than FILL_WIDE_BINS bins on a level the runs of a bin inside a block get short, and a wide workgroup makes them longer;
+// a batch of less than FILL_WIDE_POINTS would leave half of the chip without one.
+constexpr int FILL_THREADS = 512, FILL_WIDE_THREADS = 1024;
+constexpr int fill_points(bool wide) { return wide ? 2 * FILL_WIDE_THREADS : FILL_THREADS; }
+constexpr int FILL_WIDE_BINS = 128;
+constexpr int64_t FILL_WIDE_POINTS = (int64_t)1 << 18;
 constexpr int ACC_THREADS = 1024;
-constexpr int ACC_INFLIGHT = 8;               // records in flight per thread
-constexpr uint32_t SLICE_RECORDS = 98304;     // a bin with at most this many records is one accumulation task
-constexpr uint32_t SPLIT_RECORDS = 32768;     // a bigger bin is cut into tasks of about this many
-// A cell record stands for eight corners (sixteen LDS adds against an x-pair record's four).  In batches of up to
-// CELL_FINE_MAX_POINTS points a cell level's tasks are cut four times finer: with the x-pair limits a coarse level of one
-// or two bins was a single task of up to 98304 cell records, and from 2^16 to 2^17 points that one task (about 100 us)
-// outlasted the rest of the accumulate launch (2^16 points: 109 -> 49 us, 2^17: 128 -> 57, 2^18: 89 -> 76).  Larger
-// batches hide such a task behind the others, and four times as many flushes of the same few thousand rows cost them
-// 30 us at 2^20 points.
-constexpr uint32_t CELL_FINE = 4;
-constexpr int64_t CELL_FINE_MAX_POINTS = (int64_t)1 << 18;
-static uint32_t cell_task_div(int64_t n_points) { return n_points <= CELL_FINE_MAX_POINTS ? CELL_FINE : 1u; }
+constexpr int ACC_INFLIGHT = 2;               // records in flight per thread
+constexpr int GROUP = 16;                     // records named by one entry of a task's list
+constexpr int LIST = 6144;                    // entries of the list that LDS holds at a time
+constexpr int LIST_PAD = 2 * ACC_THREADS * ACC_INFLIGHT / GROUP;  // empty entries behind it
+constexpr int SPLIT_MAX_BINS = 1536;          // bins that can be split: those of the coarse levels, where points meet
+constexpr uint32_t SPLIT_MIN_COST = 32768;    // least cost (x-pair records) of a share of a split bin
+constexpr uint32_t CELL_COST = 4;             // a cell record is sixteen LDS adds against an x-pair record's four
 constexpr int MAX_BINS_PER_LEVEL = 2048;        // 2^24 rows
-constexpr int MAX_BINS_TOTAL = 2560;          // LDS of the count and fill kernels
-
 struct BinPlan {
   int n_levels;
   int nbins[NF_MAX_LEVELS];
   int binbase[NF_MAX_LEVELS + 1];  // first global bin of the level
   int cell[NF_MAX_LEVELS];         // the level's records are cells (one per point) instead of x-pairs
+  int64_t record_base[NF_MAX_LEVELS];  // first record of the level's blocks
+  int block_records[NF_MAX_LEVELS];    // room of one block
 };
 
 // cell record = {u | qx << 14,  qy | qz << 16,  packed gradient pair}: u = row of corner 0 minus the bin's first row,
@@ -77,17 +86,26 @@ __device__ __forceinline__ uint3 make_cell_record(int32_t rel_row, const float (
   return make_uint3((uint32_t)(rel_row + BIN_ROWS) | qx << 14, qy | qz << 16, packed);
 }
 
-// workspace (32-bit words): hist[NB] | gmax[32] | cursor[NB] | n_tasks, pad[3] | tasks[max_tasks][4] |
-// wg_counts[workgroups][NB] | records[R][3]      (hist and gmax are cleared together)
+struct BinHeader {  // cleared by the fill kernel's first workgroup for the kernels behind it
+  uint32_t next_task, n_splits, pad[2];
+  uint32_t gmax[NF_MAX_LEVELS];  // largest |dout| bit pattern of every level
+};
+
+// A bin cut into several tasks, each summing into a slot (of BIN_ROWS rows of two floats) of its own.
+struct BinSplit {
+  uint32_t bin, slot, n, pad;
+};
+
 struct BinWs {
-  uint32_t* hist;
-  uint32_t* gmax;  // per level: largest |dout| bit pattern (15 bits)
-  uint32_t* cursor;
-  uint32_t* n_tasks;
-  uint4* tasks;
-  uint32_t* wg_counts;
-  uint32_t* records;  // 3 words per record (16-bit gradient) or 4 (float32 gradient)
-  uint32_t max_tasks;
+  BinHeader* header;
+  uint32_t* totals;     // records of every bin (cleared with the header)
+  uint32_t* block_max;  // [levels][blocks] largest |dout| bit pattern
+  BinSplit* splits;
+  uint16_t* starts;     // [blocks][start_stride]: place of every bin inside the block, one more per level for its end
+  float* slots;
+  uint32_t* records;    // 3 words per record (16-bit gradient) or 4 (float32 gradient)
+  uint32_t max_slots, split_cost;
+  int start_stride, blocks;
 };
 
 // Workgroup barrier that orders LDS accesses only: global stores issued before it stay in flight (a plain
@@ -295,77 +313,317 @@ __global__ void hash_bwd_bin_zero_k(uint32_t* p, int n) {
 }
 
 // ---------------------------------------------------------------------------------------
-// count
+// fill
 // ---------------------------------------------------------------------------------------
+// A level goes through three barriers: ranks inside the bins (LDS adds on one counter per bin), an exclusive scan of the
+// counters by one wave, the records into the stage in sorted order, and the stage out to the block.  The copy-out of a level runs
+// beside the hashing of the next one, and two or three workgroups per unit cover each other's barriers.
+// 16-bit upstream gradient: 12-byte records {.., .., packed pair}; float32 (G32): 16-byte records {.., .., g0, g1}.
+// A stage holds a little more than the usual number of records; the rare ones behind it (pairs split over two bins) go
+// straight to their place.
 // DX: dimensions beyond the third (D == 3 then); hi: which corner of them this pass covers
-template <int D, int DX = 0>
-__global__ __launch_bounds__(FILL_POINTS) void hash_bwd_bin_count_k(const void* coords, int cdt, int64_t csn, int64_t csd,
-                                                                    int64_t N, DevGeom g, BinPlan bp, const int64_t* primes,
-                                                                    float scale, uint32_t* hist, uint32_t* wg_counts, int hi) {
-  extern __shared__ uint32_t lh[];  // all bins of all levels
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int NB = bp.binbase[bp.n_levels];
-  for (int i = tid; i < NB; i += FILL_POINTS) lh[i] = 0u;
-  lds_barrier();
-  const int64_t n = (int64_t)blockIdx.x * FILL_POINTS + tid;
-  const bool valid = n < N;
-  float v[3 + DX] = {};
+constexpr int stage_records(int D, bool wide) { return fill_points(wide) * (D == 3 ? 4 : 2) + 256; }
+
+typedef uint32_t Words4 __attribute__((ext_vector_type(4)));
+
+template <bool WIDE, bool G32, int D, int DX = 0>
+__global__ __launch_bounds__(WIDE ? FILL_WIDE_THREADS : FILL_THREADS, WIDE || G32 || DX ? 4 : 8) void hash_bwd_bin_fill_k(const void* coords, int cdt, int64_t csn, int64_t csd,
+                                                                    const void* dout_v, int64_t dout_stride, int64_t N, int points,
+                                                                    DevGeom g, BinPlan bp, const int64_t* primes, float scale,
+                                                                    BinWs ws, int max_nb, int feat, int f0, int hi) {
+  extern __shared__ __align__(16) uint32_t fill_smem[];
+  constexpr int RW = G32 ? 4 : 3;  // words of a record
+  constexpr int THREADS = WIDE ? FILL_WIDE_THREADS : FILL_THREADS, POINTS = fill_points(WIDE), PPT = POINTS / THREADS;
+  constexpr uint32_t ROOM = stage_records(D, WIDE);
   constexpr int PAIRS = 1 << (D - 1);
-  if (valid) load_point_d<D + DX>(coords, cdt, csn, csd, n, scale, v);
-  const uint32_t pi[3] = {(uint32_t)primes[0], (uint32_t)primes[1], D > 2 ? (uint32_t)primes[D > 2 ? 2 : 0] : 0u};
-  for (int l = 0; l < bp.n_levels; ++l) {
-    uint32_t* cnt = lh + bp.binbase[l];
-    const int nb = bp.nbins[l];
-    const bool cells = D == 3 && bp.cell[l];
-    if (nb == 1) {
-      if (valid) {
-        const unsigned long long m = __ballot(true);
-        if (lane == __ffsll((long long)m) - 1) atomicAdd(cnt, (cells ? 1u : (uint32_t)PAIRS) * (uint32_t)__popcll(m));
-      }
-      continue;
-    }
-    if constexpr (D == 3) {
-      if (cells) {
-        // one record in the bin of corner 0 and, when the cell reaches into the next bin, one there
-        const uint32_t res = (uint32_t)g.res[l];
-        const Located3 q = locate(v, (float)g.res[l]);
-        const uint32_t b = q.c[0] + q.c[1] * res + q.c[2] * res * res;
-        const uint32_t k0 = b >> BIN_ROWS_LOG2, k1 = (b + res * res + res + 1u) >> BIN_ROWS_LOG2;
-        if (valid) {
-          atomicAdd(cnt + k0, 1u);
-          if (k1 != k0) atomicAdd(cnt + k1, 1u);
-        }
-        continue;
-      }
-    }
-    uint32_t row[1 << D];
-    if constexpr (DX > 0) {
-      const ExtraDims ex = extra_dims<DX>(v, (float)g.res[l], (uint32_t)g.res[l], hi, primes);
-      cell_rows<D>(v, (float)g.res[l], l >= g.first_hash, (uint32_t)g.res[l], g.rows[l] - 1u, pi, primes, row, nullptr, &ex);
-    } else {
-      cell_rows<D>(v, (float)g.res[l], l >= g.first_hash, (uint32_t)g.res[l], g.rows[l] - 1u, pi, primes, row, nullptr);
-    }
+  uint32_t* stage = fill_smem;               // [ROOM][RW], sorted by bin
+  uint32_t* cnt0 = stage + ROOM * RW;        // [2][max_nb] records per bin of this level and of the next one
+  uint32_t* start = cnt0 + 2 * max_nb;       // [max_nb + 1] first record of every bin
+  uint32_t* lmax = start + max_nb + 1;       // [levels] largest |dout| pattern
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t n0 = (int64_t)blockIdx.x * points;
+  const int here = N - n0 < points ? (int)(N - n0) : points;
+  if (blockIdx.x == 0)  // the header and the totals behind it
+    for (int i = tid; i < (int)(sizeof(BinHeader) / 4) + bp.binbase[bp.n_levels]; i += THREADS) reinterpret_cast<uint32_t*>(ws.header)[i] = 0u;
+  for (int i = tid; i < 2 * max_nb; i += THREADS) cnt0[i] = 0u;
+  if (tid < NF_MAX_LEVELS) lmax[tid] = 0u;
+  float v[PPT][3 + DX] = {};
+  bool valid[PPT];
+  int64_t n[PPT];
 #pragma unroll
-    for (int c = 0; c < PAIRS; ++c) {
-      const uint32_t b0 = row[2 * c] >> BIN_ROWS_LOG2, b1 = row[2 * c + 1] >> BIN_ROWS_LOG2;
-      if (valid) {
-        atomicAdd(cnt + b0, 1u);
-        if (b1 != b0) atomicAdd(cnt + b1, 1u);
+  for (int i = 0; i < PPT; ++i) {
+    // neighbouring lanes take points sixteen apart: along a ray neighbours share a cell, and the accumulation's lanes, which follow
+    // the order of the records, would add to the same few rows (64 adds to one address one after the other)
+    const int k = lane * (POINTS / 64) + wave * PPT + i;
+    valid[i] = k < here;
+    n[i] = n0 + (valid[i] ? k : 0);
+    load_point_d<D + DX>(coords, cdt, csn, csd, n[i], scale, v[i]);
+  }
+  const uint32_t pi[3] = {(uint32_t)primes[0], (uint32_t)primes[1], D > 2 ? (uint32_t)primes[D > 2 ? 2 : 0] : 0u};
+  // The gradient pairs (features f0, f0 + 1) of four levels are read together: rows of 2, 4 or 8 features in 16-byte pieces where
+  // they are aligned, pair by pair otherwise.
+  const bool row_vec = !G32 && (feat == 2 || feat == 4 || feat == 8) && (bp.n_levels & 3) == 0 && ((uintptr_t)dout_v & 15u) == 0 && (dout_stride & 7) == 0;
+  const bool row_vec32 = G32 && feat == 2 && (bp.n_levels & 3) == 0 && ((uintptr_t)dout_v & 15u) == 0 && (dout_stride & 3) == 0;
+  const int pair_in_level = f0 >> 1;
+  auto word = [](const uint4& q, int c) { return c == 0 ? q.x : c == 1 ? q.y : c == 2 ? q.z : q.w; };
+  uint32_t quad[PPT][4][G32 ? 2 : 1];
+  auto load_quad = [&](int l0) {
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) {
+      if constexpr (G32) {
+        const float* row = reinterpret_cast<const float*>(dout_v) + n[i] * dout_stride;
+        if (row_vec32) {
+          const uint4 a = *reinterpret_cast<const uint4*>(row + 2 * l0), b = *reinterpret_cast<const uint4*>(row + 2 * l0 + 4);
+          quad[i][0][0] = a.x; quad[i][0][1] = a.y; quad[i][1][0] = a.z; quad[i][1][1] = a.w;
+          quad[i][2][0] = b.x; quad[i][2][1] = b.y; quad[i][3][0] = b.z; quad[i][3][1] = b.w;
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int e = (l0 + q) * feat + f0;
+            const bool in = l0 + q < bp.n_levels;
+            quad[i][q][0] = in ? __float_as_uint(row[e]) : 0u;
+            quad[i][q][1] = in && f0 + 1 < feat ? __float_as_uint(row[e + 1]) : 0u;  // an odd feature count: the last has no partner
+          }
+        }
+      } else {
+        const uint16_t* row = reinterpret_cast<const uint16_t*>(dout_v) + n[i] * dout_stride;
+        if (row_vec) {
+          const uint4* g4 = reinterpret_cast<const uint4*>(row);
+          uint4 t;
+          const int q0 = l0 >> 2;
+          if (feat == 2) {
+            t = g4[q0];
+          } else if (feat == 4) {
+            const uint4 a = g4[2 * q0], b = g4[2 * q0 + 1];
+            t = pair_in_level ? make_uint4(a.y, a.w, b.y, b.w) : make_uint4(a.x, a.z, b.x, b.z);
+          } else {
+            t = make_uint4(word(g4[4 * q0], pair_in_level), word(g4[4 * q0 + 1], pair_in_level), word(g4[4 * q0 + 2], pair_in_level),
+                           word(g4[4 * q0 + 3], pair_in_level));
+          }
+          quad[i][0][0] = t.x; quad[i][1][0] = t.y; quad[i][2][0] = t.z; quad[i][3][0] = t.w;
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int e = (l0 + q) * feat + f0;
+            uint32_t packed = 0u;
+            if (l0 + q < bp.n_levels) {
+              packed = row[e];
+              if (f0 + 1 < feat) packed |= (uint32_t)row[e + 1] << 16;
+            }
+            quad[i][q][0] = packed;
+          }
+        }
       }
     }
-  }
+  };
   lds_barrier();
-  uint32_t* mine = wg_counts + (int64_t)blockIdx.x * NB;  // the fill kernel's workgroup of the same index reads these
-  for (int i = tid; i < NB; i += FILL_POINTS) {
-    const uint32_t c = lh[i];
-    mine[i] = c;
-    if (c) atomicAdd(hist + i, c);
+
+  for (int l = 0; l < bp.n_levels; ++l) {
+    const int nb = bp.nbins[l];
+    uint32_t* cnt = cnt0 + (l & 1) * max_nb;
+    if ((l & 3) == 0) load_quad(l);
+    uint32_t gp[PPT][G32 ? 2 : 1], m = 0u;
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) {
+#pragma unroll
+      for (int e = 0; e < (G32 ? 2 : 1); ++e) {
+        const int q = l & 3;
+        gp[i][e] = q == 0 ? quad[i][0][e] : q == 1 ? quad[i][1][e] : q == 2 ? quad[i][2][e] : quad[i][3][e];
+      }
+      if (!valid[i]) continue;
+      // largest |g| of the level: positive float patterns order like integers
+      if constexpr (G32) {
+        m = max(m, max(gp[i][0] & 0x7fffffffu, gp[i][1] & 0x7fffffffu));
+      } else {
+        const uint32_t pk = gp[i][0] & 0x7fff7fffu;
+        m = max(m, max(pk & 0xffffu, pk >> 16));
+      }
+    }
+    m = wave_max_u32(m);
+    if (lane == 63 && m) atomicMax(lmax + l, m);
+
+    // the records, and their ranks inside the bins: {bin, rank << 12}; ~0 where a pair does not reach into a second bin
+    uint32_t rx[PPT][PAIRS], ry[PPT][PAIRS], at[PAIRS * PPT], at2[PAIRS * PPT];
+    bool cells = false;
+    if constexpr (D == 3 && !G32 && DX == 0) cells = bp.cell[l] != 0;
+    const int per_point = cells ? 1 : PAIRS;
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) {
+      if (cells) {
+        if constexpr (D == 3 && !G32 && DX == 0) {
+          const uint32_t res = (uint32_t)g.res[l];
+          const Located3 q = locate(v[i], (float)g.res[l]);
+          const uint32_t b = q.c[0] + q.c[1] * res + q.c[2] * res * res;
+          const uint32_t k0 = b >> BIN_ROWS_LOG2, k1 = (b + res * res + res + 1u) >> BIN_ROWS_LOG2;
+          const uint3 rec = make_cell_record((int32_t)(b - (k0 << BIN_ROWS_LOG2)), q.fr, 0u);
+          rx[i][0] = rec.x;
+          ry[i][0] = rec.y;
+          at[i * PAIRS] = k0;
+          at2[i * PAIRS] = valid[i] && k1 != k0 ? k1 : ~0u;
+        }
+      } else {
+        uint32_t row[1 << D];
+        float w[1 << D];
+        if constexpr (DX > 0) {
+          const ExtraDims ex = extra_dims<DX>(v[i], (float)g.res[l], (uint32_t)g.res[l], hi, primes);
+          cell_rows<D>(v[i], (float)g.res[l], l >= g.first_hash, (uint32_t)g.res[l], g.rows[l] - 1u, pi, primes, row, w, &ex);
+        } else {
+          cell_rows<D>(v[i], (float)g.res[l], l >= g.first_hash, (uint32_t)g.res[l], g.rows[l] - 1u, pi, primes, row, w);
+        }
+#pragma unroll
+        for (int c = 0; c < PAIRS; ++c) {
+          const uint32_t r0 = row[2 * c], r1 = row[2 * c + 1], k0 = r0 >> BIN_ROWS_LOG2, k1 = r1 >> BIN_ROWS_LOG2;
+          const uint3 rec = make_record(r0 & BIN_MASK, r1 & BIN_MASK, w[2 * c], w[2 * c + 1], 0u);
+          rx[i][c] = rec.x;
+          ry[i][c] = rec.y;
+          at[i * PAIRS + c] = k0;
+          at2[i * PAIRS + c] = valid[i] && k1 != k0 ? k1 : ~0u;
+        }
+      }
+    }
+    // all ranks of the thread asked for together: a wave waits for LDS once per level
+    if (nb > 1) {
+      uint32_t rank[PAIRS * PPT];
+#pragma unroll
+      for (int k = 0; k < PAIRS * PPT; ++k)
+        rank[k] = valid[k / PAIRS] && k % PAIRS < per_point ? atomicAdd(cnt + at[k], 1u) : 0u;
+#pragma unroll
+      for (int k = 0; k < PAIRS * PPT; ++k) at[k] |= rank[k] << 12;
+      bool more = false;
+#pragma unroll
+      for (int k = 0; k < PAIRS * PPT; ++k) more = more || (k % PAIRS < per_point && at2[k] != ~0u);
+      if (__any(more)) {
+#pragma unroll
+        for (int k = 0; k < PAIRS * PPT; ++k)
+          if (k % PAIRS < per_point && at2[k] != ~0u) at2[k] |= atomicAdd(cnt + at2[k], 1u) << 12;
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < PAIRS * PPT; ++k) {
+        const int i = k / PAIRS;  // a full block in the order of the threads, a ragged one in the order of its points
+        const int p = here == POINTS ? tid + THREADS * i : lane * (POINTS / 64) + wave * PPT + i;
+        at[k] = (uint32_t)(p * per_point + k % PAIRS) << 12;
+      }
+    }
+    lds_barrier();
+    // exclusive scan of the counters: into LDS for this workgroup, and out for the plan; the other waves clear the next
+    // level's counters
+    uint16_t* out_start = ws.starts + (int64_t)blockIdx.x * ws.start_stride + bp.binbase[l] + l;
+    if (wave == 0) {
+      if (nb == 1) {
+        if (lane == 0) {
+          start[0] = 0u;
+          start[1] = (uint32_t)(here * per_point);
+          out_start[0] = 0;
+          out_start[1] = (uint16_t)(here * per_point);
+        }
+      } else {
+        uint32_t run = 0;
+        for (int b0 = 0; b0 < nb; b0 += 64) {
+          const int b = b0 + lane;
+          const uint32_t c = b < nb ? cnt[b] : 0u;
+          uint32_t incl = c;
+#pragma unroll
+          for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)incl, d);
+            if (lane >= d) incl += y;
+          }
+          const uint32_t excl = run + incl - c;
+          if (b < nb) {
+            start[b] = excl;
+            out_start[b] = (uint16_t)excl;
+          }
+          run += (uint32_t)__shfl((int)incl, 63);
+        }
+        if (lane == 0) {
+          start[nb] = run;
+          out_start[nb] = (uint16_t)run;
+        }
+      }
+    } else {
+      uint32_t* other = cnt0 + ((l + 1) & 1) * max_nb;
+      for (int i = tid - 64; i < max_nb; i += THREADS - 64) other[i] = 0u;
+    }
+    lds_barrier();
+    const uint32_t room = (uint32_t)bp.block_records[l];
+    uint32_t* block = ws.records + (bp.record_base[l] + (int64_t)blockIdx.x * room) * RW;
+    auto put = [&](uint32_t pos, uint32_t x, uint32_t y, int i) {
+      if (pos < ROOM) {
+        stage[pos * RW] = x;
+        stage[pos * RW + 1] = y;
+        stage[pos * RW + 2] = gp[i][0];
+        if constexpr (G32) stage[pos * RW + 3] = gp[i][1];
+      } else {
+        block[pos * RW] = x;
+        block[pos * RW + 1] = y;
+        block[pos * RW + 2] = gp[i][0];
+        if constexpr (G32) block[pos * RW + 3] = gp[i][1];
+      }
+    };
+    bool more = false;
+#pragma unroll
+    for (int k = 0; k < PAIRS * PPT; ++k) {
+      const int i = k / PAIRS, c = k % PAIRS;
+      if (!valid[i] || c >= per_point) continue;
+      const bool split = at2[k] != ~0u;
+      more = more || split;
+      uint32_t x = rx[i][c], y = ry[i][c];
+      if (split && !cells) {  // the second corner leaves as a record of its own
+        x = (x & BIN_MASK) | (x & BIN_MASK) << BIN_ROWS_LOG2;
+        y &= W_MAX;
+      }
+      put(start[at[k] & 0xfffu] + (at[k] >> 12), x, y, i);
+    }
+    if (__any(more)) {
+#pragma unroll
+      for (int k = 0; k < PAIRS * PPT; ++k) {
+        const int i = k / PAIRS, c = k % PAIRS;
+        if (!valid[i] || c >= per_point || at2[k] == ~0u) continue;
+        const uint32_t x = rx[i][c], y = ry[i][c];
+        const uint32_t pos = start[at2[k] & 0xfffu] + (at2[k] >> 12);
+        if (cells) {
+          put(pos, x - (((at2[k] & 0xfffu) - (at[k] & 0xfffu)) << BIN_ROWS_LOG2), y, i);  // the same cell seen from the next bin
+        } else {
+          const uint32_t r1 = (x >> BIN_ROWS_LOG2) & BIN_MASK, w1 = (x >> 26) << 13 | y >> W_BITS;
+          put(pos, r1 | r1 << BIN_ROWS_LOG2, w1, i);
+        }
+      }
+    }
+    lds_barrier();
+    // The stage leaves as it is: whole 16-byte pieces, the last one perhaps with words of no meaning behind the end; past the caches,
+    // which the records of a batch overflow anyway (fill 199 -> 180 us and accum 212 -> 189 us at 2^20 points).
+    const uint32_t pieces = (min(start[nb], ROOM) * RW + 3u) / 4u;
+    for (uint32_t i = tid; i < pieces; i += THREADS) __builtin_nontemporal_store(reinterpret_cast<const Words4*>(stage)[i], reinterpret_cast<Words4*>(block) + i);
   }
+  if (tid < bp.n_levels) ws.block_max[(int64_t)tid * ws.blocks + blockIdx.x] = lmax[tid];
 }
 
 // ---------------------------------------------------------------------------------------
-// offsets: one workgroup
+// totals: a wave adds up 64 bins of 64 blocks (and takes the largest |dout| of the level)
 // ---------------------------------------------------------------------------------------
+constexpr int TOTALS_BLOCKS = 64;
+__global__ __launch_bounds__(64) void hash_bwd_bin_totals_k(BinWs ws, BinPlan bp) {
+  int first = blockIdx.x, l = 0;  // blockIdx.x counts pieces of 64 bins over all levels
+  for (;; ++l) {
+    const int pieces = (bp.nbins[l] + 63) / 64;
+    if (first < pieces) break;
+    first -= pieces;
+  }
+  const int w0 = blockIdx.y * TOTALS_BLOCKS, w1 = min(w0 + TOTALS_BLOCKS, ws.blocks);
+  if (first == 0) {
+    const int w = w0 + (int)threadIdx.x;
+    const uint32_t m = wave_max_u32(w < w1 ? ws.block_max[(int64_t)l * ws.blocks + w] : 0u);
+    if (threadIdx.x == 63 && m) atomicMax(ws.header->gmax + l, m);
+  }
+  const int b = first * 64 + (int)threadIdx.x;
+  if (b >= bp.nbins[l]) return;
+  const uint16_t* mine = ws.starts + (int64_t)w0 * ws.start_stride + bp.binbase[l] + l + b;
+  uint32_t sum = 0;
+#pragma unroll 8
+  for (int w = w0; w < w1; ++w, mine += ws.start_stride) sum += (uint32_t)mine[1] - (uint32_t)mine[0];
+  if (sum) atomicAdd(ws.totals + bp.binbase[l] + b, sum);
+}
+
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t x, uint32_t* wave_sums, uint32_t* total) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
   uint32_t incl = x;
@@ -385,296 +643,6 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t x, uint32_t* w
   }
   *total = all;
   return before + incl - x;
-}
-
-__global__ __launch_bounds__(1024) void hash_bwd_bin_offsets_k(const uint32_t* hist, uint32_t* cursor, uint32_t* n_tasks,
-                                                               uint4* tasks, int NB, uint32_t max_tasks, BinPlan bp,
-                                                               uint32_t cell_div) {
-  __shared__ uint32_t wave_sums[16];
-  __shared__ uint32_t first_task[1025], bin_start[1024], bin_count[1024];  // of the 1024 bins of a pass
-  uint32_t rec_run = 0, task_run = 0;
-  for (int b0 = 0; b0 < NB; b0 += 1024) {
-    const int b = b0 + (int)threadIdx.x;
-    const uint32_t c = b < NB ? hist[b] : 0u;
-    int lvl = 0;
-    while (lvl + 1 < bp.n_levels && b >= bp.binbase[lvl + 1]) ++lvl;
-    const bool cell = bp.cell[lvl] != 0;
-    const uint32_t one = cell ? SLICE_RECORDS / cell_div : SLICE_RECORDS, cut = cell ? SPLIT_RECORDS / cell_div : SPLIT_RECORDS;
-    const uint32_t slices = c <= one ? (c ? 1u : 0u) : (c + cut - 1u) / cut;
-    uint32_t rec_total, task_total;
-    const uint32_t start = rec_run + block_exclusive_scan(c, wave_sums, &rec_total);
-    const uint32_t t0 = block_exclusive_scan(slices, wave_sums, &task_total);
-    if (b < NB) cursor[b] = start;
-    first_task[threadIdx.x] = t0;
-    bin_start[threadIdx.x] = start;
-    bin_count[threadIdx.x] = c;
-    if (threadIdx.x == 0) first_task[1024] = task_total;
-    __syncthreads();
-    // every task of the pass by a thread of its own (a coarse dense level is one bin cut into a hundred slices): the
-    // task's bin is the last one whose first task is not behind it
-    for (uint32_t t = threadIdx.x; t < task_total; t += 1024) {
-      uint32_t lo_b = 0, hi_b = 1023;
-      while (lo_b < hi_b) {
-        const uint32_t mid = (lo_b + hi_b + 1) >> 1;
-        if (first_task[mid] <= t) lo_b = mid; else hi_b = mid - 1;
-      }
-      // bins without records share their first task with the bin behind them: the search lands on the last of the run
-      const uint32_t c_b = bin_count[lo_b], n_sl = first_task[lo_b + 1] - first_task[lo_b], sl = t - first_task[lo_b];
-      // equal slices, so that no workgroup gets a short tail
-      const uint32_t per = (c_b + n_sl - 1u) / n_sl;
-      uint32_t lo = bin_start[lo_b] + sl * per, hi = bin_start[lo_b] + (sl + 1u) * per;
-      if (hi > bin_start[lo_b] + c_b) hi = bin_start[lo_b] + c_b;
-      if (lo > hi) lo = hi;
-      if (task_run + t < max_tasks) tasks[task_run + t] = make_uint4((uint32_t)b0 + lo_b, lo, hi, n_sl > 1u ? 1u : 0u);
-    }
-    __syncthreads();
-    rec_run += rec_total;
-    task_run += task_total;
-  }
-  if (threadIdx.x == 0) *n_tasks = task_run < max_tasks ? task_run : max_tasks;
-}
-
-// ---------------------------------------------------------------------------------------
-// fill
-// ---------------------------------------------------------------------------------------
-// G32 = false: 16-bit upstream gradient, 12-byte records {.., .., packed pair}.  G32 = true: float32 upstream gradient,
-// 16-byte records {.., .., g0, g1}; a staged entry then names the point instead of carrying the pair, and the copy-out
-// takes the pair from the workgroup's per-level gradient table in LDS (the stage has no room for 20-byte entries).
-template <bool G32, int D, int DX = 0>
-__global__ __launch_bounds__(FILL_POINTS) void hash_bwd_bin_fill_k(const void* coords, int cdt, int64_t csn, int64_t csd,
-                                                                   const void* dout_v, int64_t dout_stride, int64_t N,
-                                                                   DevGeom g, BinPlan bp, const int64_t* primes, float scale,
-                                                                   const uint32_t* wg_counts, uint32_t* cursor, uint32_t* gmax,
-                                                                   uint32_t* records_v, int feat, int f0, int hi) {
-  extern __shared__ __align__(16) unsigned char fill_smem[];
-  const int NB = bp.binbase[bp.n_levels];
-  const uint16_t* dout = reinterpret_cast<const uint16_t*>(dout_v);
-  uint3* records = reinterpret_cast<uint3*>(records_v);
-  uint4* records4 = reinterpret_cast<uint4*>(records_v);
-  uint4* stage = reinterpret_cast<uint4*>(fill_smem);                     // [FILL_RECORDS] {record, its place in `records`}, sorted by bin
-  uint2* gtab = reinterpret_cast<uint2*>(stage + FILL_RECORDS);           // G32: [FILL_POINTS] this level's gradient pair of every point
-  uint32_t* cur = reinterpret_cast<uint32_t*>(gtab + (G32 ? FILL_POINTS : 0));  // [NB] next staged position of a bin
-  uint32_t* delta = cur + NB;                                             // [NB] global minus staged position
-  uint32_t* totals = delta + NB;                                          // [levels] records of this workgroup per level
-  uint32_t* lmax = totals + NF_MAX_LEVELS;                                // [levels] largest |dout| pattern
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t n0 = (int64_t)blockIdx.x * FILL_POINTS;
-  const int64_t n = n0 + tid;
-  const bool valid = n < N;
-  // This workgroup's share of every bin, counted by the count kernel: one reservation per non-empty bin, all in
-  // flight together.
-  for (int i = tid; i < NB; i += FILL_POINTS) {
-    const uint32_t c = wg_counts[(int64_t)blockIdx.x * NB + i];
-    cur[i] = c;
-    delta[i] = c ? atomicAdd(cursor + i, c) : 0u;
-  }
-  if (tid < NF_MAX_LEVELS) lmax[tid] = 0u;
-  float v[3 + DX] = {};
-  constexpr int PAIRS = 1 << (D - 1);
-  if (valid) load_point_d<D + DX>(coords, cdt, csn, csd, n, scale, v);
-  const uint32_t pi[3] = {(uint32_t)primes[0], (uint32_t)primes[1], D > 2 ? (uint32_t)primes[D > 2 ? 2 : 0] : 0u};
-  // this point's gradient row, read once (up to 16 levels live in registers); float32 rows are read level by level
-  const uint32_t* grow = reinterpret_cast<const uint32_t*>(dout + (valid ? n : 0) * dout_stride);
-  const float* grow32 = reinterpret_cast<const float*>(dout_v) + (valid ? n : 0) * dout_stride;
-  uint32_t gr[16];
-  // this pass covers features f0, f0 + 1 of every level: the pair of level l sits at element l * feat + f0 of the row
-  // (rows of 2, 4 or 8 features in 16-byte pieces: with 4 or 8 features a piece holds the pairs of two levels or of one,
-  // and the pass keeps its own; per-level 4-byte reads touch a point's 128 or 256 bytes sixteen times instead)
-  const bool row_vec = !G32 && (feat == 2 || feat == 4 || feat == 8) && bp.n_levels <= 16 && (bp.n_levels & 3) == 0 &&
-                       ((uintptr_t)dout & 15u) == 0 && (dout_stride & 7) == 0;
-  const bool row_vec32 = G32 && feat == 2 && (bp.n_levels & 3) == 0 && ((uintptr_t)dout_v & 15u) == 0 && (dout_stride & 3) == 0;
-  uint2 held[3] = {make_uint2(0u, 0u), make_uint2(0u, 0u), make_uint2(0u, 0u)};
-  const int pair_in_level = f0 >> 1;
-  auto word = [](const uint4& q, int c) { return c == 0 ? q.x : c == 1 ? q.y : c == 2 ? q.z : q.w; };
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint4 t = make_uint4(0u, 0u, 0u, 0u);
-    if (row_vec && valid && 4 * i < bp.n_levels) {
-      const uint4* g4 = reinterpret_cast<const uint4*>(grow);
-      if (feat == 2) {
-        t = g4[i];
-      } else if (feat == 4) {
-        const uint4 a = g4[2 * i], b = g4[2 * i + 1];
-        t = pair_in_level ? make_uint4(a.y, a.w, b.y, b.w) : make_uint4(a.x, a.z, b.x, b.z);
-      } else {
-        const uint4 q0 = g4[4 * i], q1 = g4[4 * i + 1], q2 = g4[4 * i + 2], q3 = g4[4 * i + 3];
-        t = make_uint4(word(q0, pair_in_level), word(q1, pair_in_level), word(q2, pair_in_level), word(q3, pair_in_level));
-      }
-    }
-    gr[4 * i] = t.x;
-    gr[4 * i + 1] = t.y;
-    gr[4 * i + 2] = t.z;
-    gr[4 * i + 3] = t.w;
-  }
-  lds_barrier();
-  // staged start of every bin inside its level (exclusive scan of the counts), one wave per level
-  for (int l = wave; l < bp.n_levels; l += FILL_POINTS / 64) {
-    const int nb = bp.nbins[l], gb0 = bp.binbase[l];
-    uint32_t run = 0;
-    for (int b0 = 0; b0 < nb; b0 += 64) {
-      const int b = b0 + lane;
-      const uint32_t c = b < nb ? cur[gb0 + b] : 0u;
-      uint32_t incl = c;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)incl, d);
-        if (lane >= d) incl += y;
-      }
-      const uint32_t excl = run + incl - c;
-      if (b < nb) {
-        cur[gb0 + b] = excl;
-        delta[gb0 + b] -= excl;
-      }
-      run += (uint32_t)__shfl((int)incl, 63);
-    }
-    if (lane == 0) totals[l] = run;
-  }
-  lds_barrier();
-
-  for (int l = 0; l < bp.n_levels; ++l) {
-    const int nb = bp.nbins[l];
-    uint32_t* lcur = cur + bp.binbase[l];
-    const uint32_t* ldelta = delta + bp.binbase[l];
-    uint32_t packed = 0u;  // 16-bit: the pair; float32: the point's index in the workgroup (its pair goes to gtab)
-    if (G32) {
-      uint2 pair = make_uint2(0u, 0u);
-      if (valid) {
-        if (feat & 1) {  // an odd row width: the pair is not 8-byte aligned, and the last feature has no partner
-          pair.x = __float_as_uint(grow32[l * feat + f0]);
-          if (f0 + 1 < feat) pair.y = __float_as_uint(grow32[l * feat + f0 + 1]);
-        } else if (row_vec32) {  // four levels' pairs in two 16-byte reads: a quarter of the passes over the point's 128 bytes
-          if ((l & 3) == 0) {
-            const uint4 q0 = *reinterpret_cast<const uint4*>(grow32 + 2 * l), q1 = *reinterpret_cast<const uint4*>(grow32 + 2 * l + 4);
-            pair = make_uint2(q0.x, q0.y);
-            held[0] = make_uint2(q0.z, q0.w);
-            held[1] = make_uint2(q1.x, q1.y);
-            held[2] = make_uint2(q1.z, q1.w);
-          } else {
-            pair = (l & 3) == 1 ? held[0] : (l & 3) == 2 ? held[1] : held[2];
-          }
-        } else {
-          pair = *reinterpret_cast<const uint2*>(grow32 + l * feat + f0);
-        }
-      }
-      gtab[tid] = pair;
-      packed = (uint32_t)tid;
-      // largest |g| of the level: positive float patterns order like integers
-      const uint32_t a0 = pair.x & 0x7fffffffu, a1 = pair.y & 0x7fffffffu;
-      const uint32_t m = wave_max_u32(a0 > a1 ? a0 : a1);
-      if (lane == 63 && m) atomicMax(lmax + l, m);
-    } else {
-      if (row_vec) {
-        packed = gr[0];
-#pragma unroll
-        for (int i = 1; i < 16; ++i) packed = (l == i) ? gr[i] : packed;
-      } else if (valid) {
-        if (feat & 1) {  // an odd row width: 16-bit loads, and the last feature has no partner
-          const uint16_t* g16 = reinterpret_cast<const uint16_t*>(grow);
-          packed = g16[l * feat + f0];
-          if (f0 + 1 < feat) packed |= (uint32_t)g16[l * feat + f0 + 1] << 16;
-        } else {
-          packed = grow[(l * feat + f0) >> 1];
-        }
-      }
-      // largest |g| of the level: positive 16-bit float patterns order like integers
-      const uint32_t pk = packed & 0x7fff7fffu;
-      const uint32_t m = wave_max_u32((pk & 0xffffu) > (pk >> 16) ? (pk & 0xffffu) : (pk >> 16));
-      if (lane == 63 && m) atomicMax(lmax + l, m);
-    }
-    bool cells = false;
-    if constexpr (D == 3 && !G32) cells = bp.cell[l] != 0;
-    if (cells) {
-      const uint32_t res = (uint32_t)g.res[l];
-      const Located3 q = locate(v, (float)g.res[l]);
-      const uint32_t b = q.c[0] + q.c[1] * res + q.c[2] * res * res;
-      const uint32_t k0 = b >> BIN_ROWS_LOG2, k1 = (b + res * res + res + 1u) >> BIN_ROWS_LOG2;
-      const bool two = k1 != k0;
-      uint32_t pos0;
-      if (nb == 1) pos0 = (uint32_t)tid;  // the valid points are the first of the workgroup
-      else pos0 = valid ? atomicAdd(lcur + k0, 1u) : 0u;
-      if (valid) {
-        const uint3 rec = make_cell_record((int32_t)(b - (k0 << BIN_ROWS_LOG2)), q.fr, packed);
-        stage[pos0] = make_uint4(rec.x, rec.y, rec.z, pos0 + ldelta[k0]);
-      }
-      if (nb > 1 && __any(valid && two)) {
-        const bool on = valid && two;
-        const uint32_t pos1 = on ? atomicAdd(lcur + k1, 1u) : 0u;
-        if (on) {
-          const uint3 rec = make_cell_record((int32_t)b - (int32_t)(k1 << BIN_ROWS_LOG2), q.fr, packed);
-          stage[pos1] = make_uint4(rec.x, rec.y, rec.z, pos1 + ldelta[k1]);
-        }
-      }
-    } else {
-      uint32_t row[1 << D];
-      float w[1 << D];
-      if constexpr (DX > 0) {
-        const ExtraDims ex = extra_dims<DX>(v, (float)g.res[l], (uint32_t)g.res[l], hi, primes);
-        cell_rows<D>(v, (float)g.res[l], l >= g.first_hash, (uint32_t)g.res[l], g.rows[l] - 1u, pi, primes, row, w, &ex);
-      } else {
-        cell_rows<D>(v, (float)g.res[l], l >= g.first_hash, (uint32_t)g.res[l], g.rows[l] - 1u, pi, primes, row, w);
-      }
-      // The x-pairs of the point (four in 3-D, two in 2-D): their ranks are asked for together, so that a wave waits
-      // for LDS once per level and not once per pair.
-      uint32_t b0[PAIRS], b1[PAIRS], pos[PAIRS], dlt[PAIRS];
-      bool split[PAIRS];
-      bool any_split = false;
-#pragma unroll
-      for (int c = 0; c < PAIRS; ++c) {
-        b0[c] = row[2 * c] >> BIN_ROWS_LOG2;
-        b1[c] = row[2 * c + 1] >> BIN_ROWS_LOG2;
-        split[c] = b1[c] != b0[c];
-        any_split = any_split || split[c];
-      }
-      if (nb == 1) {
-#pragma unroll
-        for (int c = 0; c < PAIRS; ++c) pos[c] = (uint32_t)tid * (uint32_t)PAIRS + (uint32_t)c;  // the valid points are the first of the workgroup
-      } else {
-#pragma unroll
-        for (int c = 0; c < PAIRS; ++c) pos[c] = valid ? atomicAdd(lcur + b0[c], 1u) : 0u;
-      }
-#pragma unroll
-      for (int c = 0; c < PAIRS; ++c) dlt[c] = ldelta[b0[c]];
-      if (valid) {
-#pragma unroll
-        for (int c = 0; c < PAIRS; ++c) {
-          const uint32_t r0 = row[2 * c], r1 = row[2 * c + 1];
-          const uint3 rec = make_record(r0 & BIN_MASK, (split[c] ? r0 : r1) & BIN_MASK, w[2 * c], split[c] ? 0.0f : w[2 * c + 1], packed);
-          stage[pos[c]] = G32 ? make_uint4(rec.x, rec.y, pos[c] + dlt[c], rec.z) : make_uint4(rec.x, rec.y, rec.z, pos[c] + dlt[c]);
-        }
-      }
-      // a pair that straddles two bins leaves its second corner as a record of its own (rare)
-      if (nb > 1 && __any(valid && any_split)) {
-#pragma unroll
-        for (int c = 0; c < PAIRS; ++c) {
-          const bool on = valid && split[c];
-          if (!__any(on)) continue;
-          const uint32_t pos1 = on ? atomicAdd(lcur + b1[c], 1u) : 0u;
-          if (on) {
-            const uint32_t r1 = row[2 * c + 1];
-            const uint3 rec = make_record(r1 & BIN_MASK, r1 & BIN_MASK, w[2 * c + 1], 0.0f, packed);
-            const uint32_t gp = pos1 + ldelta[b1[c]];
-            stage[pos1] = G32 ? make_uint4(rec.x, rec.y, gp, rec.z) : make_uint4(rec.x, rec.y, rec.z, gp);
-          }
-        }
-      }
-    }
-    lds_barrier();
-    const uint32_t total = totals[l];
-    for (uint32_t i = tid; i < total; i += FILL_POINTS) {
-      const uint4 e = stage[i];
-      if (G32) {
-        const uint2 pair = gtab[e.w];
-        records4[e.z] = make_uint4(e.x, e.y, pair.x, pair.y);
-      } else {
-        records[e.w] = make_uint3(e.x, e.y, e.z);
-      }
-    }
-    lds_barrier();  // the next level overwrites the stage
-  }
-  if (tid < bp.n_levels) {
-    const uint32_t m = lmax[tid];
-    if (m > *(volatile uint32_t*)(gmax + tid)) atomicMax(gmax + tid, m);
-  }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -698,167 +666,385 @@ struct BinRec<F32> {
   __device__ static __forceinline__ float level_max(uint32_t pattern) { return __uint_as_float(pattern); }
 };
 
-template <typename GT>
-__global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(const typename BinRec<GT>::type* records, const uint4* tasks,
-                                                                    const uint32_t* n_tasks, const uint32_t* gmax, float* dtable,
-                                                                    DevGeom g, BinPlan bp, int feat, int f0) {
+// Nearest integer (halves upwards) of |x| < 2^31, in one instruction; __float2int_rn() takes two.
+__device__ __forceinline__ int32_t round_to_int(float x) {
+  int32_t r;
+  asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+  return r;
+}
+
+// How a sum reaches the gradient table.
+enum TableMode { TABLE_ADD = 0, TABLE_F32 = 1, TABLE_F16 = 2, TABLE_BF16 = 3 };  // added to float32, or written in a type of its own
+template <int MODE>
+__device__ __forceinline__ void store_table(void* table, int64_t i, float x) {
+  if constexpr (MODE == TABLE_ADD || MODE == TABLE_F32) reinterpret_cast<float*>(table)[i] = x;
+  else if constexpr (MODE == TABLE_F16) reinterpret_cast<uint16_t*>(table)[i] = F16::from_f32(x);
+  else reinterpret_cast<uint16_t*>(table)[i] = BF16::from_f32(x);
+}
+
+// two features of a row (one if not `pair`); whole: the row is these two (one access)
+template <int MODE>
+__device__ __forceinline__ void store_pair(void* table, int64_t i, float x, float y, bool whole, bool pair) {
+  if (whole) {
+    if constexpr (MODE == TABLE_F32) *reinterpret_cast<float2*>(reinterpret_cast<float*>(table) + i) = make_float2(x, y);
+    else if constexpr (MODE == TABLE_F16) *reinterpret_cast<uint32_t*>(reinterpret_cast<uint16_t*>(table) + i) = F16::pack(x, y);
+    else *reinterpret_cast<uint32_t*>(reinterpret_cast<uint16_t*>(table) + i) = BF16::pack(x, y);
+  } else {
+    store_table<MODE>(table, i, x);
+    if (pair) store_table<MODE>(table, i + 1, y);
+  }
+}
+
+template <typename GT, int MODE>
+__global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, void* table, DevGeom g, BinPlan bp, int feat, int f0) {
   typedef typename BinRec<GT>::type Rec;
   // Fixed-point sums, one plane of BIN_ROWS 64-bit cells per feature: the 64 lanes of an add go to random rows of one
   // feature, and with 8-byte cells those spread over all 64 banks (interleaved features would leave them half).
   extern __shared__ unsigned long long acc_tile[];
-  if (blockIdx.x >= *n_tasks) return;
+  uint32_t* list = reinterpret_cast<uint32_t*>(acc_tile + 2 * BIN_ROWS);  // [LIST + LIST_PAD] first word of up to GROUP records in the level | their number << 27
+  uint32_t* first_task = list + LIST + LIST_PAD;                          // [SB + 1] first task of a bin | its first slot << 16
+  __shared__ uint32_t next_task[2], wave_sums[ACC_THREADS / 64];
+  __shared__ int level_base[NF_MAX_LEVELS];
   const int tid = threadIdx.x;
-  const uint4 task = tasks[blockIdx.x];
-  int l = 0;
-  while (l + 1 < bp.n_levels && (int)task.x >= bp.binbase[l + 1]) ++l;
-  const uint32_t row0 = (task.x - (uint32_t)bp.binbase[l]) << BIN_ROWS_LOG2;
-  const uint32_t left = g.rows[l] - row0;
-  const uint32_t nrows = left < (uint32_t)BIN_ROWS ? left : (uint32_t)BIN_ROWS;
-  // fixed-point scale 2^se of the level:  |w * g| * 2^se < 2^30
-  const float gm = BinRec<GT>::level_max(gmax[l]);
-  const bool nonfinite = !(gm <= 3.0e38f);
-  int se = 0;
-  if (!nonfinite && gm > 0.0f) {
-    int ex;
-    frexpf(gm, &ex);  // gm = f * 2^ex, f in [0.5, 1)
-    se = 30 - ex;
-    se = se > 120 ? 120 : se;
+  const int NB = bp.binbase[bp.n_levels];
+  int SB = 0;  // bins of the leading levels, which may be split
+  for (int l = 0; l < bp.n_levels && bp.binbase[l + 1] <= SPLIT_MAX_BINS; ++l) SB = bp.binbase[l + 1];
+  for (uint32_t i = tid; i < 2u * BIN_ROWS; i += ACC_THREADS) acc_tile[i] = 0ull;
+  if (tid < bp.n_levels) level_base[tid] = bp.binbase[tid];
+  __syncthreads();
+  // The tasks, worked out by every workgroup for itself: one per bin, several for a bin of more than one and a half shares.
+  uint32_t split_tasks = 0;
+  {
+    uint32_t slots = 0;
+    for (int b0 = 0; b0 < SB; b0 += ACC_THREADS) {
+      const int b = b0 + tid;
+      uint32_t n = 0, cost = 0;
+      if (b < SB) {
+        int l = 0;
+        while (l + 1 < bp.n_levels && b >= level_base[l + 1]) ++l;
+        cost = ws.totals[b] * (bp.cell[l] ? CELL_COST : 1u);
+        n = cost <= ws.split_cost + ws.split_cost / 2 ? 1u : min((cost + ws.split_cost - 1u) / ws.split_cost, (uint32_t)ws.blocks);
+        if (cost == 0u && MODE == TABLE_ADD) n = 0u;  // nothing to add (a table that is written gets its zeros)
+      }
+      uint32_t total;
+      const uint32_t slot = slots + block_exclusive_scan(n > 1u ? n : 0u, wave_sums, &total);
+      if (n > 1u && slot + n > ws.max_slots) n = 1u;  // out of slots: the bin stays one task
+      slots += total;
+      const uint32_t first = split_tasks + block_exclusive_scan(n, wave_sums, &total);
+      split_tasks += total;
+      if (b < SB) first_task[b] = first | slot << 16;
+      if (blockIdx.x == 0 && n > 1u) ws.splits[atomicAdd(&ws.header->n_splits, 1u)] = BinSplit{(uint32_t)b, slot, n, 0u};
+    }
+    if (tid == 0) first_task[SB] = split_tasks;
   }
-  // two steps stay inside float range; the weight decode rides on the second
-  const float s_lo = nonfinite ? 0.0f : ldexpf(1.0f, se / 2), s_hi = ldexpf(1.0f, se - se / 2) * (1.0f / (float)W_MAX);
-  for (uint32_t i = tid; i < 2u * nrows; i += ACC_THREADS) acc_tile[(i & 1u) * BIN_ROWS + (i >> 1)] = 0ull;
-  lds_barrier();
-  // The task's records behind a buffer descriptor that ends with them: reads past the end return zeros (zero weights),
-  // so the loop carries no bounds tests.
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<Rec*>(records + task.y), 0,
-                                                                      (int)((task.z - task.y) * (uint32_t)sizeof(Rec)), 0x00020000);
-  auto load_rec = [&](uint32_t at) {  // record `at` of the task
-    Rec r;
-    if constexpr (sizeof(Rec) == 12) {
-      typedef unsigned int v3u __attribute__((ext_vector_type(3)));
-      const v3u v = __builtin_amdgcn_raw_buffer_load_b96(rs, at * 12u, 0, 0);
-      r.x = v[0]; r.y = v[1]; r.z = v[2];
-    } else {
-      typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-      const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rs, at * 16u, 0, 0);
-      r.x = v[0]; r.y = v[1]; r.z = v[2]; r.w = v[3];
+  const uint32_t n_tasks = split_tasks + (uint32_t)(NB - SB);
+  // What a task needs, the same for all threads.
+  struct Task {
+    int bin, level, block0, block1;
+    uint32_t slot;
+  };
+  const int lane = tid & 63;
+  auto task_of = [&](uint32_t t) {
+    Task k = {SB + (int)(t - split_tasks), 0, 0, ws.blocks, ~0u};
+    if (t < split_tasks) {
+      // the bin whose first task is the last one not behind t (a bin without tasks shares it with the one behind it), found
+      // in two looks of 64 lanes each
+      const int step = (SB + 63) / 64;
+      auto not_behind = [&](int b) { return __builtin_popcountll(__ballot(b < SB && (first_task[b] & 0xffffu) <= t)); };
+      const int seg = (not_behind(lane * step) - 1) * step;
+      k.bin = seg + not_behind(lane < step ? seg + lane : SB) - 1;
+      const uint32_t at = first_task[k.bin], t0 = at & 0xffffu, n = (first_task[k.bin + 1] & 0xffffu) - t0;
+      if (n > 1u) {
+        k.slot = (at >> 16) + t - t0;
+        k.block0 = (int)((int64_t)ws.blocks * (t - t0) / n);
+        k.block1 = (int)((int64_t)ws.blocks * (t - t0 + 1u) / n);
+      }
+    }
+    k.level = __builtin_popcountll(__ballot(lane < bp.n_levels && level_base[lane] <= k.bin)) - 1;
+    k.bin = __builtin_amdgcn_readfirstlane(k.bin);
+    k.level = __builtin_amdgcn_readfirstlane(k.level);
+    k.block0 = __builtin_amdgcn_readfirstlane(k.block0);
+    k.block1 = __builtin_amdgcn_readfirstlane(k.block1);
+    k.slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)k.slot);
+    return k;
+  };
+  // where this thread's block of the task's first ACC_THREADS has the bin's records: {first, end}
+  auto block_part = [&](const Task& k, int w) {
+    uint2 r = make_uint2(0u, 0u);
+    if (w < k.block1) {
+      const uint16_t* s = ws.starts + (int64_t)w * ws.start_stride + k.bin + k.level;
+      r = make_uint2(s[0], s[1]);
     }
     return r;
   };
-  const uint32_t n_rec = task.z - task.y;
   // an odd feature count leaves the last pass with one feature: plane 1 then has no column in the table
   const bool has_pair = f0 + 1 < feat;
-  // the next round's records are loaded before this round's adds; a level with an inf or a nan in its gradient only
-  // marks the rows it touches (its own copy of the loop, so that the usual one has no test per record)
-  auto accumulate = [&](auto nonfinite_c) {
-    constexpr bool NONFINITE = decltype(nonfinite_c)::value;
-    Rec q[ACC_INFLIGHT];
-#pragma unroll
-    for (int k = 0; k < ACC_INFLIGHT; ++k) q[k] = load_rec(k * ACC_THREADS + tid);
-    for (uint32_t i0 = 0; i0 < n_rec; i0 += ACC_THREADS * ACC_INFLIGHT) {
-      uint32_t slot[ACC_INFLIGHT][2];
-      int32_t f[ACC_INFLIGHT][4];
-#pragma unroll
-      for (int k = 0; k < ACC_INFLIGHT; ++k) {
-        const float g0 = BinRec<GT>::g0(q[k]) * s_lo, g1 = BinRec<GT>::g1(q[k]) * s_lo;
-        const float w0 = (float)(q[k].y & W_MAX), w1 = (float)((q[k].x >> 26) << 13 | q[k].y >> W_BITS);
-        slot[k][0] = q[k].x & BIN_MASK;
-        slot[k][1] = (q[k].x >> BIN_ROWS_LOG2) & BIN_MASK;
-        if constexpr (NONFINITE) {
-          f[k][0] = w0 != 0.0f;
-          f[k][2] = w1 != 0.0f;
-          f[k][1] = has_pair && f[k][0];
-          f[k][3] = has_pair && f[k][2];
-        } else {
-          f[k][0] = __float2int_rn(w0 * g0 * s_hi);
-          f[k][1] = __float2int_rn(w0 * g1 * s_hi);
-          f[k][2] = __float2int_rn(w1 * g0 * s_hi);
-          f[k][3] = __float2int_rn(w1 * g1 * s_hi);
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < ACC_INFLIGHT; ++k) q[k] = load_rec(i0 + ACC_THREADS * ACC_INFLIGHT + k * ACC_THREADS + tid);
-#pragma unroll
-      for (int k = 0; k < ACC_INFLIGHT; ++k)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (f[k][j]) atomicAdd(acc_tile + (uint32_t)(j & 1) * BIN_ROWS + slot[k][j >> 1], (unsigned long long)(long long)f[k][j]);
+  // Task numbers come from a counter, fetched a task ahead, and so are the places of the next task's records: neither is waited
+  // for.  Every workgroup leaves as soon as the counter has passed the last task.
+  if (tid == 0) {
+    next_task[0] = atomicAdd(&ws.header->next_task, 1u);
+    next_task[1] = atomicAdd(&ws.header->next_task, 1u);
+  }
+  __syncthreads();
+  uint32_t t = next_task[0], t_next = next_task[1];
+  if (t >= n_tasks) return;
+  Task task = task_of(t);
+  uint2 part = block_part(task, task.block0 + tid);
+  for (;;) {
+    const int l = task.level;
+    const uint32_t row0 = (uint32_t)(task.bin - bp.binbase[l]) << BIN_ROWS_LOG2;
+    const uint32_t left = g.rows[l] - row0;
+    const uint32_t nrows = left < (uint32_t)BIN_ROWS ? left : (uint32_t)BIN_ROWS;
+    // fixed-point scale 2^se of the level:  |w * g| * 2^se < 2^30
+    const float gm = BinRec<GT>::level_max(ws.header->gmax[l]);
+    const bool nonfinite = !(gm <= 3.0e38f);
+    int se = 0;
+    if (!nonfinite && gm > 0.0f) {
+      int ex;
+      frexpf(gm, &ex);  // gm = f * 2^ex, f in [0.5, 1)
+      se = 30 - ex;
+      se = se > 120 ? 120 : se < -120 ? -120 : se;
     }
-  };
-  // cell records (dense levels): the eight corners' rows and weights are rebuilt from the record; a corner outside this
-  // bin belongs to the copy of the record in the neighbouring bin
-  auto accumulate_cells = [&](auto nonfinite_c) {
-    constexpr bool NONFINITE = decltype(nonfinite_c)::value;
-    const uint32_t res = (uint32_t)g.res[l], r2 = res * res;
-    const float s_cell = ldexpf(1.0f, se - se / 2);
-    Rec q[ACC_INFLIGHT];
+    const float scale = nonfinite ? 0.0f : ldexpf(1.0f, se);  // |g| * 2^se < 2^30, and |se| stays inside float's exponents
+    const float scale_w = scale * (1.0f / (float)W_MAX);      // with the decoding of the pair records' weights
+    // The level's records behind a buffer descriptor: a lane without a record asks for one past the end and gets zeros (zero
+    // weights), so the loop carries no bounds tests.
+    constexpr uint32_t RW = sizeof(Rec) / 4;
+    const uint32_t room = (uint32_t)bp.block_records[l];
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(ws.records + bp.record_base[l] * (int64_t)RW, 0,
+                                                                        (int)((uint32_t)ws.blocks * room * (uint32_t)sizeof(Rec)), 0x00020000);
+    const uint32_t in_group = (uint32_t)tid % GROUP;
+    auto load_rec = [&](uint32_t entry) {
+      const uint32_t at = in_group < entry >> 27 ? (entry & 0x7ffffffu) * 4u + in_group * (uint32_t)sizeof(Rec) : 0xf0000000u;
+      Rec r;
+      if constexpr (sizeof(Rec) == 12) {
+        typedef unsigned int v3u __attribute__((ext_vector_type(3)));
+        const v3u v = __builtin_amdgcn_raw_buffer_load_b96(rs, at, 0, 0);
+        r.x = v[0]; r.y = v[1]; r.z = v[2];
+      } else {
+        typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+        const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0);
+        r.x = v[0]; r.y = v[1]; r.z = v[2]; r.w = v[3];
+      }
+      return r;
+    };
+    // a lane without a record, and a record without a gradient, add nothing
+    auto live = [](const Rec& r) {
+      if constexpr (sizeof(Rec) == 12) return (r.z & 0x7fff7fffu) != 0u;
+      else return ((r.z | r.w) & 0x7fffffffu) != 0u;
+    };
+    auto add_to = [&](uint32_t at, int32_t v) { atomicAdd(acc_tile + at, (unsigned long long)(long long)v); };
+    constexpr uint32_t ROUND = ACC_THREADS * ACC_INFLIGHT;
+    // The next round's records are loaded before this round's adds; a level with an inf or a nan in its gradient only marks the
+    // rows it touches (its own copy of the loop, so that the usual one has no test per record).
+    auto rounds = [&](uint32_t entries, auto add) {
+      const uint32_t* mine = list + (uint32_t)tid / GROUP;  // (the list goes on with empty entries for two rounds)
+      Rec q[ACC_INFLIGHT];
 #pragma unroll
-    for (int k = 0; k < ACC_INFLIGHT; ++k) q[k] = load_rec(k * ACC_THREADS + tid);
-    for (uint32_t i0 = 0; i0 < n_rec; i0 += ACC_THREADS * ACC_INFLIGHT) {
-      Rec cur[ACC_INFLIGHT];
+      for (int k = 0; k < ACC_INFLIGHT; ++k) q[k] = load_rec(mine[k * (ACC_THREADS / GROUP)]);
+      for (uint32_t e = 0; e < entries; e += ROUND / GROUP) {
+        mine += ROUND / GROUP;
+        add(q, [&] {
 #pragma unroll
-      for (int k = 0; k < ACC_INFLIGHT; ++k) cur[k] = q[k];
+          for (int k = 0; k < ACC_INFLIGHT; ++k) q[k] = load_rec(mine[k * (ACC_THREADS / GROUP)]);
+        });
+      }
+    };
+    auto add_pairs = [&](auto nonfinite_c) {
+      constexpr bool NONFINITE = decltype(nonfinite_c)::value;
+      return [&](Rec (&q)[ACC_INFLIGHT], auto load_next) {
+        uint32_t slot[ACC_INFLIGHT][2];
+        int32_t f[ACC_INFLIGHT][4];
+        bool on[ACC_INFLIGHT];
 #pragma unroll
-      for (int k = 0; k < ACC_INFLIGHT; ++k) q[k] = load_rec(i0 + ACC_THREADS * ACC_INFLIGHT + k * ACC_THREADS + tid);
-#pragma unroll
-      for (int k = 0; k < ACC_INFLIGHT; ++k) {
-        const bool live = (cur[k].x & 0x3fffu) != 0u;  // reads past the task's end return zero words
-        const int32_t rel = (int32_t)(cur[k].x & 0x3fffu) - BIN_ROWS;
-        const float fx = (float)(cur[k].x >> 14) * (1.0f / CELL_QX), fy = (float)(cur[k].y & 0xffffu) * (1.0f / CELL_QYZ),
-                    fz = (float)(cur[k].y >> 16) * (1.0f / CELL_QYZ);
-        const float fr[3] = {fx, fy, fz};
-        float w[8];
-        weights_d3(fr, w);
-        const float g0 = BinRec<GT>::g0(cur[k]) * s_lo, g1 = BinRec<GT>::g1(cur[k]) * s_lo;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int32_t slot = rel + (j & 1) + ((j >> 1) & 1) * (int32_t)res + (j >> 2) * (int32_t)r2;
-          if (!live || slot < 0 || slot >= BIN_ROWS) continue;
-          int32_t f0v, f1v;
+        for (int k = 0; k < ACC_INFLIGHT; ++k) {
+          const float g0 = BinRec<GT>::g0(q[k]) * scale_w, g1 = BinRec<GT>::g1(q[k]) * scale_w;
+          const float w0 = (float)(q[k].y & W_MAX), w1 = (float)((q[k].x >> 26) << 13 | q[k].y >> W_BITS);
+          slot[k][0] = q[k].x & BIN_MASK;
+          slot[k][1] = (q[k].x >> BIN_ROWS_LOG2) & BIN_MASK;
+          on[k] = live(q[k]);
           if constexpr (NONFINITE) {
-            f0v = w[j] != 0.0f;
-            f1v = has_pair && f0v;
+            f[k][0] = w0 != 0.0f;
+            f[k][2] = w1 != 0.0f;
+            f[k][1] = has_pair && f[k][0];
+            f[k][3] = has_pair && f[k][2];
           } else {
-            f0v = __float2int_rn(w[j] * g0 * s_cell);
-            f1v = __float2int_rn(w[j] * g1 * s_cell);
+            f[k][0] = round_to_int(w0 * g0);
+            f[k][1] = round_to_int(w0 * g1);
+            f[k][2] = round_to_int(w1 * g0);
+            f[k][3] = round_to_int(w1 * g1);
           }
-          if (f0v) atomicAdd(acc_tile + (uint32_t)slot, (unsigned long long)(long long)f0v);
-          if (f1v) atomicAdd(acc_tile + (uint32_t)BIN_ROWS + (uint32_t)slot, (unsigned long long)(long long)f1v);
+        }
+        load_next();
+#pragma unroll
+        for (int k = 0; k < ACC_INFLIGHT; ++k)
+          if (on[k]) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) add_to((uint32_t)(j & 1) * BIN_ROWS + slot[k][j >> 1], f[k][j]);
+          }
+      };
+    };
+    // cell records (dense levels): the eight corners' rows and weights are rebuilt from the record; a corner outside this
+    // bin belongs to the copy of the record in the neighbouring bin
+    auto add_cells = [&](auto nonfinite_c) {
+      constexpr bool NONFINITE = decltype(nonfinite_c)::value;
+      return [&](Rec (&q)[ACC_INFLIGHT], auto load_next) {
+        const uint32_t res = (uint32_t)g.res[l], r2 = res * res;
+        Rec cur[ACC_INFLIGHT];
+#pragma unroll
+        for (int k = 0; k < ACC_INFLIGHT; ++k) cur[k] = q[k];
+        load_next();
+#pragma unroll
+        for (int k = 0; k < ACC_INFLIGHT; ++k) {
+          if (!live(cur[k])) continue;
+          const int32_t rel = (int32_t)(cur[k].x & 0x3fffu) - BIN_ROWS;
+          const float fx = (float)(cur[k].x >> 14) * (1.0f / CELL_QX), fy = (float)(cur[k].y & 0xffffu) * (1.0f / CELL_QYZ),
+                      fz = (float)(cur[k].y >> 16) * (1.0f / CELL_QYZ);
+          const float fr[3] = {fx, fy, fz};
+          float w[8];
+          weights_d3(fr, w);
+          const float g0 = BinRec<GT>::g0(cur[k]) * scale, g1 = BinRec<GT>::g1(cur[k]) * scale;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const uint32_t slot = (uint32_t)(rel + (j & 1) + ((j >> 1) & 1) * (int32_t)res + (j >> 2) * (int32_t)r2);
+            if (slot >= (uint32_t)BIN_ROWS) continue;
+            if constexpr (NONFINITE) {
+              if (w[j] == 0.0f) continue;
+              add_to(slot, 1);
+              if (has_pair) add_to((uint32_t)BIN_ROWS + slot, 1);
+            } else {
+              add_to(slot, round_to_int(w[j] * g0));
+              add_to((uint32_t)BIN_ROWS + slot, round_to_int(w[j] * g1));
+            }
+          }
+        }
+      };
+    };
+    bool cells = false;
+    if constexpr (sizeof(Rec) == 12) cells = bp.cell[l] != 0;
+    // the task's records, listed for up to ACC_THREADS blocks and LIST entries at a time
+    Task task_next = {};
+    uint2 part_next = make_uint2(0u, 0u);
+    uint32_t t_later = 0u;
+    bool ahead = false;
+    for (int w0 = task.block0; w0 < task.block1; w0 += ACC_THREADS) {
+      if (w0 != task.block0) part = block_part(task, w0 + tid);
+      const uint32_t at = ((uint32_t)(w0 + tid) * room + part.x) * RW, c = part.y - part.x, mine = (c + GROUP - 1u) / GROUP;
+      uint32_t entries;
+      const uint32_t before = block_exclusive_scan(mine, wave_sums, &entries);
+      for (uint32_t e0 = 0; e0 == 0 || e0 < entries; e0 += LIST) {
+        for (uint32_t e = before < e0 ? e0 : before; e < before + mine && e < e0 + LIST; ++e) {
+          const uint32_t k = (e - before) * GROUP;
+          list[e - e0] = (at + k * RW) | min(c - k, (uint32_t)GROUP) << 27;
+        }
+        const uint32_t now = min(entries - e0, (uint32_t)LIST);
+        for (uint32_t e = now + tid; e < now + LIST_PAD; e += ACC_THREADS) list[e] = 0u;
+        if (!ahead) {
+          ahead = true;
+          if (t_next < n_tasks) {
+            task_next = task_of(t_next);
+            part_next = block_part(task_next, task_next.block0 + tid);
+          }
+          if (tid == 0) t_later = atomicAdd(&ws.header->next_task, 1u);
+        }
+        lds_barrier();
+        if (cells) {
+          if (nonfinite) rounds(now, add_cells(std::true_type{}));
+          else rounds(now, add_cells(std::false_type{}));
+        } else if (nonfinite) rounds(now, add_pairs(std::true_type{}));
+        else rounds(now, add_pairs(std::false_type{}));
+        if (tid == 0) next_task[0] = t_later;
+        lds_barrier();
+      }
+    }
+    // the tile to the table (or the task's slot), and back to zero for the next task
+    const float qnan = __uint_as_float(0x7fc00000u);
+    const int64_t first = (g.row_offset[l] + (int64_t)row0) * feat + f0;  // features f0, f0 + 1 of the bin's rows
+    // |a| < 2^48 and its quotient by 2^se are exact in double: one rounding, to float, at the end
+    const double unscale = ldexp(1.0, -se), unscale_hi = ldexp(1.0, 32 - se);
+    auto value = [&](uint32_t i) {
+      const long long a = (long long)acc_tile[i];
+      acc_tile[i] = 0ull;
+      const float x = (float)((double)(int)(a >> 32) * unscale_hi + (double)(uint32_t)a * unscale);
+      return nonfinite && a != 0 ? qnan : x;
+    };
+    constexpr int U = 8;  // rows of a thread that are under way together
+    for (uint32_t r0 = tid; r0 < nrows; r0 += ACC_THREADS * U) {
+      float x[U], y[U];
+      float2 old[MODE == TABLE_ADD ? U : 1];
+      if constexpr (MODE == TABLE_ADD)
+        if (feat == 2 && task.slot == ~0u) {
+          const float2* src = reinterpret_cast<const float2*>(reinterpret_cast<const float*>(table) + first);
+#pragma unroll
+          for (int u = 0; u < U; ++u) old[u] = src[min(r0 + u * ACC_THREADS, nrows - 1u)];
+        }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t r = r0 + u * ACC_THREADS;
+        x[u] = r < nrows ? value(r) : 0.0f;
+        y[u] = r < nrows ? value(BIN_ROWS + r) : 0.0f;
+      }
+      if (task.slot != ~0u) {
+        float2* dst = reinterpret_cast<float2*>(ws.slots + (int64_t)task.slot * (2 * BIN_ROWS));
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (r0 + u * ACC_THREADS < nrows) dst[r0 + u * ACC_THREADS] = make_float2(x[u], y[u]);
+      } else {
+        if constexpr (MODE == TABLE_ADD) {
+          float* dst = reinterpret_cast<float*>(table) + first;
+          if (feat == 2) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (x[u] != 0.0f || y[u] != 0.0f) reinterpret_cast<float2*>(dst)[r0 + u * ACC_THREADS] = make_float2(old[u].x + x[u], old[u].y + y[u]);
+          } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              float* cell = dst + (int64_t)(r0 + u * ACC_THREADS) * feat;
+              if (x[u] != 0.0f) cell[0] += x[u];
+              if (has_pair && y[u] != 0.0f) cell[1] += y[u];
+            }
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const uint32_t r = r0 + u * ACC_THREADS;
+            if (r < nrows) store_pair<MODE>(table, first + (int64_t)r * feat, x[u], y[u], feat == 2, has_pair);
+          }
         }
       }
     }
-  };
-  bool cells = false;
-  if constexpr (sizeof(Rec) == 12) cells = bp.cell[l] != 0;
-  if (cells) {
-    if (nonfinite) accumulate_cells(std::true_type{});
-    else accumulate_cells(std::false_type{});
-  } else if (nonfinite) accumulate(std::true_type{});
-  else accumulate(std::false_type{});
-  lds_barrier();
-  float* dst = dtable + (g.row_offset[l] + (int64_t)row0) * feat + f0;  // features f0, f0 + 1 of the bin's rows
-  const float qnan = __uint_as_float(0x7fc00000u);
-  const uint32_t nvals = 2u * nrows;
-  constexpr int U = 16;  // values per thread whose table reads are in flight together (a full bin in one pass)
-  for (uint32_t i0 = 0; i0 < nvals; i0 += ACC_THREADS * U) {
-    float x[U], old[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint32_t i = i0 + u * ACC_THREADS + tid;
-      const long long a = (i < nvals && (has_pair || !(i & 1u))) ? (long long)acc_tile[(i & 1u) * BIN_ROWS + (i >> 1)] : 0ll;
-      // |a| < 2^48 is exact in double and so is the division by 2^se: one rounding, to float, at the end
-      x[u] = a == 0 ? 0.0f : (float)ldexp((double)a, -se);
-      if (nonfinite && a != 0) x[u] = qnan;
-      old[u] = (x[u] != 0.0f && !task.w) ? dst[(i >> 1) * feat + (i & 1u)] : 0.0f;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint32_t i = i0 + u * ACC_THREADS + tid;
-      if (x[u] != 0.0f) {
-        float* cell = dst + (i >> 1) * feat + (i & 1u);
-        if (task.w) unsafeAtomicAdd(cell, x[u]);
-        else *cell = old[u] + x[u];
-      }
+    if (t_next >= n_tasks) return;
+    t_next = next_task[0];
+    task = task_next;
+    part = part_next;
+    // (the scan of the next task's parts has barriers between this task's last use of the tile and the next adds)
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// reduce: the slots of a bin with several tasks, in the order of the tasks
+// ---------------------------------------------------------------------------------------
+constexpr int REDUCE_THREADS = 256, REDUCE_VALUES = 256;
+template <int MODE>
+__global__ __launch_bounds__(REDUCE_THREADS) void hash_bwd_bin_reduce_k(BinWs ws, void* table, DevGeom g, BinPlan bp, int feat, int f0) {
+  if (blockIdx.y >= ws.header->n_splits) return;
+  const BinSplit sp = ws.splits[blockIdx.y];
+  int l = 0;
+  while (l + 1 < bp.n_levels && (int)sp.bin >= bp.binbase[l + 1]) ++l;
+  const uint32_t row0 = (sp.bin - (uint32_t)bp.binbase[l]) << BIN_ROWS_LOG2;
+  const uint32_t left = g.rows[l] - row0, nvals = 2u * (left < (uint32_t)BIN_ROWS ? left : (uint32_t)BIN_ROWS);
+  const int64_t first = (g.row_offset[l] + (int64_t)row0) * feat + f0;
+  const float* src = ws.slots + (int64_t)sp.slot * (2 * BIN_ROWS);
+  for (uint32_t i = blockIdx.x * REDUCE_VALUES + threadIdx.x; i < min(nvals, (blockIdx.x + 1u) * REDUCE_VALUES); i += REDUCE_THREADS) {
+    float x = 0.0f;
+#pragma unroll 8
+    for (uint32_t k = 0; k < sp.n; ++k) x += src[(int64_t)k * (2 * BIN_ROWS) + i];
+    if ((i & 1u) && f0 + 1 >= feat) continue;
+    const int64_t to = first + (int64_t)(i >> 1) * feat + (i & 1u);
+    if constexpr (MODE == TABLE_ADD) {
+      if (x != 0.0f) reinterpret_cast<float*>(table)[to] += x;
+    } else {
+      store_table<MODE>(table, to, x);
     }
   }
 }
@@ -1058,86 +1244,66 @@ __global__ __launch_bounds__(DIRECT_THREADS) void hash_bwd_direct_k(const void* 
 // ---------------------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------------------
-// Plan for levels la .. lb-1 (the kernels see them as levels 0 .. lb-la-1 of a shifted geometry).
 // cells: dense 3-D levels whose eight corners span less than a bin take one record per point (16-bit gradients)
-static bool bin_plan(int64_t N, const nf_hash_geom* geom, int la, int lb, BinPlan* bp, int64_t* records, uint32_t* max_tasks,
-                     bool cells = false) {
-  bp->n_levels = lb - la;
+static bool bin_plan(int64_t N, int points, const nf_hash_geom* geom, BinPlan* bp, int64_t* records, bool cells) {
+  // features are taken two at a time (one pass of fill + accumulate per pair; the last feature of an odd count alone)
+  if (geom->dims < 2 || geom->dims > NF_MAX_DIMS || geom->feat < 1 || N <= 0) return false;
+  bp->n_levels = geom->levels;
+  const int64_t blocks = (N + points - 1) / points;
   int nb_total = 0;
-  int64_t R = 0, R_cell = 0;
-  for (int l = la; l < lb; ++l) {
+  int64_t R = 0;
+  for (int l = 0; l < geom->levels; ++l) {
     const int64_t r = geom->rows[l];
     const int64_t nb = (r + BIN_ROWS - 1) / BIN_ROWS;
     if (nb > MAX_BINS_PER_LEVEL) return false;
-    bp->nbins[l - la] = (int)nb;
-    bp->binbase[l - la] = nb_total;
+    bp->nbins[l] = (int)nb;
+    bp->binbase[l] = nb_total;
     const int64_t res = geom->res[l];
-    bp->cell[l - la] = cells && geom->dims == 3 && l < geom->first_hash_level && res * res + res + 1 < BIN_ROWS;
+    bp->cell[l] = cells && geom->dims == 3 && l < geom->first_hash_level && res * res + res + 1 < BIN_ROWS;
     // a cell level leaves at most two records per point; an x-pair level has room for every pair to be split in two
     // (normally half of it is used); more than three dimensions run as passes of the 3-D pipeline
-    R += N * (bp->cell[l - la] ? 2 : geom->dims >= 3 ? 8 : 4);
-    if (bp->cell[l - la]) R_cell += N * 2;
+    bp->block_records[l] = points * (bp->cell[l] ? 2 : geom->dims >= 3 ? 8 : 4);
+    bp->record_base[l] = R;
+    R += blocks * bp->block_records[l];
     nb_total += (int)nb;
   }
-  bp->binbase[lb - la] = nb_total;
-  if (nb_total > MAX_BINS_TOTAL) return false;
-  if (R >= ((int64_t)1 << 32) - 4 * ACC_THREADS * ACC_INFLIGHT) return false;  // 32-bit record positions
+  bp->binbase[geom->levels] = nb_total;
   *records = R;
-  *max_tasks = (uint32_t)(nb_total + (R - R_cell) / SPLIT_RECORDS + R_cell / (SPLIT_RECORDS / cell_task_div(N)) + 1);
   return true;
 }
 
-// The count and fill kernels keep per-bin counters of all their levels in LDS (MAX_BINS_TOTAL): tables with more bins
-// go through the pipeline in groups of consecutive levels.  first[k] .. first[k+1]-1 are the levels of group k.
-// (A fixed array, no heap: the entry points allocate nothing, on the host either.)
-struct LevelGroups {
-  int n;                             // groups
-  int first[NF_MAX_LEVELS + 2];      // first[k] .. first[k + 1] - 1
-  size_t size() const { return (size_t)n + 1; }
-  int operator[](size_t k) const { return first[k]; }
-};
-static bool bin_groups(int64_t N, const nf_hash_geom* geom, LevelGroups* groups) {
-  // features are taken two at a time (one pass of fill + accumulate per pair; the last feature of an odd count alone)
-  if (geom->dims < 2 || geom->dims > NF_MAX_DIMS || geom->feat < 1 || N <= 0) return false;
-  groups->n = 0;
-  groups->first[0] = 0;
-  int nb_total = 0;
-  for (int l = 0; l < geom->levels; ++l) {
-    const int64_t nb = (geom->rows[l] + BIN_ROWS - 1) / BIN_ROWS;
-    if (nb > MAX_BINS_PER_LEVEL) return false;
-    if (nb_total + nb > MAX_BINS_TOTAL) {
-      groups->first[++groups->n] = l;
-      nb_total = 0;
-    }
-    nb_total += (int)nb;
-  }
-  groups->first[++groups->n] = geom->levels;
-  for (int k = 0; k < groups->n; ++k) {
-    BinPlan bp;
-    int64_t R;
-    uint32_t mt;
-    if (!bin_plan(N, geom, groups->first[k], groups->first[k + 1], &bp, &R, &mt)) return false;
-  }
-  return true;
+// points of a block (a multiple of four keeps the blocks of records on 16-byte boundaries)
+static bool wide_blocks(int64_t n_points, const nf_hash_geom* geom) {
+  if (n_points < FILL_WIDE_POINTS) return false;
+  for (int l = 0; l < geom->levels; ++l)
+    if (geom->rows[l] > (int64_t)FILL_WIDE_BINS * BIN_ROWS) return true;
+  return false;
 }
 
-static int64_t wg_count_words(int64_t N, int NB) { return (((N + FILL_POINTS - 1) / FILL_POINTS) * NB + 3) & ~(int64_t)3; }
-
-static int64_t bin_ws(void* workspace, const BinPlan& bp, int64_t N, int64_t R, int rec_words, uint32_t max_tasks, BinWs* ws) {
-  uint32_t* p = (uint32_t*)workspace;
+static int64_t bin_ws(void* workspace, const BinPlan& bp, int64_t N, int points, int64_t R, int rec_words, BinWs* ws) {
+  char* p = (char*)workspace;
   const int NB = bp.binbase[bp.n_levels];
-  const int NBp = (NB + 3) & ~3;
+  const int64_t blocks = (N + points - 1) / points;
   int64_t o = 0;
-  ws->hist = p + o; o += NBp;
-  ws->gmax = p + o; o += 32;
-  ws->cursor = p + o; o += NBp;
-  ws->n_tasks = p + o; o += 4;
-  ws->tasks = reinterpret_cast<uint4*>(p + o); o += 4 * (int64_t)max_tasks;
-  ws->wg_counts = p + o; o += wg_count_words(N, NB);
-  o = (o + 3) & ~(int64_t)3;  // 16-byte records start on a 16-byte boundary
-  ws->records = p + o; o += (int64_t)rec_words * R;
-  ws->max_tasks = max_tasks;
-  return o * 4;
+  auto take = [&](int64_t bytes) {
+    char* at = p + o;
+    o += (bytes + 255) / 256 * 256;
+    return at;
+  };
+  ws->blocks = (int)blocks;
+  ws->start_stride = (NB + bp.n_levels + 1) & ~1;
+  // a share of a split bin: a third of what a compute unit gets of x-pair records on every level
+  const int64_t share = N * bp.n_levels / 192;
+  ws->split_cost = (uint32_t)(share > SPLIT_MIN_COST ? share : SPLIT_MIN_COST);
+  ws->max_slots = (uint32_t)(16 + N / 1024);
+  ws->header = (BinHeader*)take(sizeof(BinHeader) + NB * 4);
+  ws->totals = (uint32_t*)(ws->header + 1);
+  ws->block_max = (uint32_t*)take(blocks * NF_MAX_LEVELS * 4);
+  ws->splits = (BinSplit*)take((int64_t)ws->max_slots * sizeof(BinSplit));
+  ws->starts = (uint16_t*)take(blocks * ws->start_stride * 2);
+  ws->slots = (float*)take((int64_t)ws->max_slots * 2 * BIN_ROWS * 4);
+  ws->records = (uint32_t*)take((int64_t)rec_words * R * 4);
+  return o;
 }
 
 // Batches above this many points go through the pipeline in pieces of this size, one after the other on the stream:
@@ -1171,27 +1337,21 @@ static int64_t direct_workspace_bytes(int64_t n_points, const nf_hash_geom* geom
 int64_t bwd_bin_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags) {
   if (n_points > BIN_CHUNK_POINTS) n_points = BIN_CHUNK_POINTS;
   if (direct_ok(n_points, geom, flags)) return direct_workspace_bytes(n_points, geom, dout_dtype);
-  LevelGroups first;
-  if (!bin_groups(n_points, geom, &first)) return 0;
-  int64_t bytes = 0;
-  for (size_t k = 0; k + 1 < first.size(); ++k) {
+  auto bytes = [&](int64_t n, bool wide) -> int64_t {
     BinPlan bp;
-    int64_t R;
-    uint32_t max_tasks;
-    bin_plan(n_points, geom, first[k], first[k + 1], &bp, &R, &max_tasks, dout_dtype != NF_F32);
     BinWs ws;
-    const int64_t b = bin_ws(nullptr, bp, n_points, R, dout_dtype == NF_F32 ? 4 : 3, max_tasks, &ws);
-    if (b > bytes) bytes = b;
-  }
-  return bytes;
+    int64_t R;
+    const int points = fill_points(wide);
+    return bin_plan(n, points, geom, &bp, &R, dout_dtype != NF_F32) ? bin_ws(nullptr, bp, n, points, R, dout_dtype == NF_F32 ? 4 : 3, &ws) : 0;
+  };
+  if (!wide_blocks(n_points, geom)) return bytes(n_points, false);
+  // room for every smaller batch too: many small blocks have more starts than fewer wide ones
+  const int64_t wide = bytes(n_points, true), small = bytes(FILL_WIDE_POINTS - 1, false);
+  return wide > small ? wide : small;
 }
 
-static int launch_bwd_bin_group(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
-                                float* dtable, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const BinPlan& bp, int64_t R,
-                                uint32_t max_tasks, const int64_t* primes, float scale, void* workspace, hipStream_t s);
-
 static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
-                                float* dtable, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
+                                void* table, int mode, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
                                 void* workspace, hipStream_t s);
 
 static int launch_bwd_direct(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
@@ -1208,10 +1368,22 @@ int launch_bwd_bin(const void* coords, int cdt, int64_t csn, int64_t csd, const 
     const char* c = (const char*)coords + n0 * csn * dtype_size(cdt);
     const char* d = (const char*)dout + n0 * dout_stride * dtype_size(ddt);
     const int rc = direct ? launch_bwd_direct(c, cdt, csn, csd, d, ddt, dout_stride, dtable, n, geom, g, primes, scale, workspace, s)
-                          : launch_bwd_bin_piece(c, cdt, csn, csd, d, ddt, dout_stride, dtable, n, geom, g, primes, scale, workspace, s);
+                          : launch_bwd_bin_piece(c, cdt, csn, csd, d, ddt, dout_stride, dtable, TABLE_ADD, n, geom, g, primes, scale, workspace, s);
     if (rc) return rc;
   }
   return 0;
+}
+
+bool bwd_write_applies(int64_t n_points, const nf_hash_geom* geom, int flags) {
+  // one pass over the points that leaves every row's whole sum in one place
+  return n_points <= BIN_CHUNK_POINTS && (geom->dims == 2 || geom->dims == 3) && !direct_ok(n_points, geom, flags);
+}
+
+int launch_bwd_write(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride, void* table,
+                     int table_dtype, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
+                     void* workspace, hipStream_t s) {
+  const int mode = table_dtype == NF_F32 ? TABLE_F32 : table_dtype == NF_F16 ? TABLE_F16 : TABLE_BF16;
+  return launch_bwd_bin_piece(coords, cdt, csn, csd, dout, ddt, dout_stride, table, mode, N, geom, g, primes, scale, workspace, s);
 }
 
 static int direct_cus() {
@@ -1229,11 +1401,12 @@ static int launch_bwd_direct(const void* coords, int cdt, int64_t csn, int64_t c
                              float* dtable, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
                              void* workspace, hipStream_t s) {
   NF_REQUIRE(((uintptr_t)workspace & 15u) == 0, NF_EALIGN, "workspace must be 16-byte aligned");
-  BinPlan bp;
-  int64_t R;
-  uint32_t max_tasks;
-  NF_REQUIRE(bin_plan(N, geom, 0, geom->levels, &bp, &R, &max_tasks, false), NF_EUNSUPPORTED,
-             "backward without records does not cover this geometry");
+  BinPlan bp = {};
+  bp.n_levels = geom->levels;
+  for (int l = 0; l < geom->levels; ++l) {
+    bp.nbins[l] = (int)((geom->rows[l] + BIN_ROWS - 1) / BIN_ROWS);
+    bp.binbase[l + 1] = bp.binbase[l] + bp.nbins[l];
+  }
   const int NB = bp.binbase[bp.n_levels];
   uint32_t* gmax = reinterpret_cast<uint32_t*>(workspace);
   uint32_t* pairs = gmax + 64;
@@ -1282,114 +1455,76 @@ static int launch_bwd_direct(const void* coords, int cdt, int64_t csn, int64_t c
 }
 
 static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
-                                float* dtable, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
+                                void* table, int mode, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
                                 void* workspace, hipStream_t s) {
-  LevelGroups first;
-  NF_REQUIRE(bin_groups(N, geom, &first), NF_EUNSUPPORTED, "binned backward does not cover this geometry");
-  NF_REQUIRE(((uintptr_t)workspace & 15u) == 0, NF_EALIGN, "workspace must be 16-byte aligned");
-  for (size_t k = 0; k + 1 < first.size(); ++k) {
-    const int la = first[k], lb = first[k + 1];
-    BinPlan bp;
-    int64_t R;
-    uint32_t max_tasks;
-    bin_plan(N, geom, la, lb, &bp, &R, &max_tasks, ddt != NF_F32);
-    // the group's levels as levels 0 .. of a geometry of their own; their gradient columns start at la * feat
-    DevGeom gg = g;
-    gg.levels = lb - la;
-    gg.first_hash = g.first_hash - la;
-    for (int l = la; l < lb; ++l) {
-      gg.res[l - la] = g.res[l];
-      gg.rows[l - la] = g.rows[l];
-      gg.row_offset[l - la] = g.row_offset[l];
-    }
-    const char* dcol = (const char*)dout + (size_t)la * geom->feat * (ddt == NF_F32 ? 4 : 2);
-    if (int rc = launch_bwd_bin_group(coords, cdt, csn, csd, dcol, ddt, dout_stride, dtable, N, geom, gg, bp, R, max_tasks, primes,
-                                      scale, workspace, s))
-      return rc;
-  }
-  return 0;
-}
-
-static int launch_bwd_bin_group(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
-                                float* dtable, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const BinPlan& bp, int64_t R,
-                                uint32_t max_tasks, const int64_t* primes, float scale, void* workspace, hipStream_t s) {
   const bool g32 = ddt == NF_F32;
+  BinPlan bp;
+  int64_t R;
+  const bool wide = wide_blocks(N, geom);
+  int points = fill_points(wide);
+  NF_REQUIRE(bin_plan(N, points, geom, &bp, &R, !g32), NF_EUNSUPPORTED, "binned backward does not cover this geometry");
+  NF_REQUIRE(((uintptr_t)workspace & 15u) == 0, NF_EALIGN, "workspace must be 16-byte aligned");
   BinWs ws;
-  bin_ws(workspace, bp, N, R, g32 ? 4 : 3, max_tasks, &ws);
+  bin_ws(workspace, bp, N, points, R, g32 ? 4 : 3, &ws);
   const int NB = bp.binbase[bp.n_levels];
-  const int NBp = (NB + 3) & ~3;
-  const unsigned blocks = (unsigned)((N + FILL_POINTS - 1) / FILL_POINTS);
-
+  int max_nb = 1, bin_pieces = 0;
+  for (int l = 0; l < bp.n_levels; ++l) {
+    max_nb = bp.nbins[l] > max_nb ? bp.nbins[l] : max_nb;
+    bin_pieces += (bp.nbins[l] + 63) / 64;
+  }
+  const int feat = geom->feat, D = g.dims == 2 ? 2 : 3;
+  auto large_lds = [](const void* kern, size_t lds) -> int {
+    const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    return e == hipSuccess ? 0 : fail((int)e, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+  };
+  auto pick_fill = [&](auto wide_c, auto g32_c) -> const void* {
+    constexpr bool W = decltype(wide_c)::value, G = decltype(g32_c)::value;
+    return g.dims == 6   ? (const void*)hash_bwd_bin_fill_k<W, G, 3, 3>
+           : g.dims == 5 ? (const void*)hash_bwd_bin_fill_k<W, G, 3, 2>
+           : g.dims == 4 ? (const void*)hash_bwd_bin_fill_k<W, G, 3, 1>
+           : g.dims == 3 ? (const void*)hash_bwd_bin_fill_k<W, G, 3>
+                         : (const void*)hash_bwd_bin_fill_k<W, G, 2>;
+  };
+  auto pick_accum = [&](auto mode_c) -> const void* {
+    constexpr int M = decltype(mode_c)::value;
+    return ddt == NF_F16 ? (const void*)hash_bwd_bin_accum_k<F16, M> : ddt == NF_BF16 ? (const void*)hash_bwd_bin_accum_k<BF16, M> : (const void*)hash_bwd_bin_accum_k<F32, M>;
+  };
+  const void* fill = wide ? (g32 ? pick_fill(std::true_type{}, std::true_type{}) : pick_fill(std::true_type{}, std::false_type{}))
+                          : (g32 ? pick_fill(std::false_type{}, std::true_type{}) : pick_fill(std::false_type{}, std::false_type{}));
+  const void* accum = mode == TABLE_ADD   ? pick_accum(std::integral_constant<int, TABLE_ADD>{})
+                      : mode == TABLE_F32 ? pick_accum(std::integral_constant<int, TABLE_F32>{})
+                      : mode == TABLE_F16 ? pick_accum(std::integral_constant<int, TABLE_F16>{})
+                                          : pick_accum(std::integral_constant<int, TABLE_BF16>{});
+  const void* reduce = mode == TABLE_ADD   ? (const void*)hash_bwd_bin_reduce_k<TABLE_ADD>
+                       : mode == TABLE_F32 ? (const void*)hash_bwd_bin_reduce_k<TABLE_F32>
+                       : mode == TABLE_F16 ? (const void*)hash_bwd_bin_reduce_k<TABLE_F16>
+                                           : (const void*)hash_bwd_bin_reduce_k<TABLE_BF16>;
+  const size_t fill_lds = ((size_t)stage_records(D, wide) * (g32 ? 4 : 3) + 3 * (size_t)max_nb + 1 + NF_MAX_LEVELS) * 4;
+  const size_t acc_lds = (size_t)BIN_ROWS * 2 * sizeof(unsigned long long) + ((size_t)LIST + LIST_PAD + (NB < SPLIT_MAX_BINS ? NB : SPLIT_MAX_BINS) + 1) * 4;
+  if (int rc = large_lds(fill, fill_lds)) return rc;
+  if (int rc = large_lds(accum, acc_lds)) return rc;
+  auto launch = [&](const char* what, const void* kern, dim3 grid, int threads, void** args, size_t lds) -> int {
+    const hipError_t e = hipLaunchKernel(kern, grid, dim3((unsigned)threads), args, lds, s);
+    if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(%s): %s", what, hipGetErrorString(e));
+    return check_launch(what);
+  };
+  const unsigned units = (unsigned)direct_cus();
   // more than three dimensions: the whole pipeline once per corner of the extra coordinates (`hi`), see ExtraDims
   const int passes = g.dims > 3 ? 1 << (g.dims - 3) : 1;
-  for (int hi = 0; hi < passes; ++hi) {
-  hipLaunchKernelGGL(hash_bwd_bin_zero_k, dim3((unsigned)((NBp + 32 + 255) / 256)), dim3(256), 0, s, ws.hist, NBp + 32);
-  if (int rc = check_launch("hash_bwd_bin_zero")) return rc;
-  if (g.dims == 6)
-    hipLaunchKernelGGL((hash_bwd_bin_count_k<3, 3>), dim3(blocks), dim3(FILL_POINTS), (size_t)NB * 4, s, coords, cdt, csn, csd, N, g, bp,
-                       primes, scale, ws.hist, ws.wg_counts, hi);
-  else if (g.dims == 5)
-    hipLaunchKernelGGL((hash_bwd_bin_count_k<3, 2>), dim3(blocks), dim3(FILL_POINTS), (size_t)NB * 4, s, coords, cdt, csn, csd, N, g, bp,
-                       primes, scale, ws.hist, ws.wg_counts, hi);
-  else if (g.dims == 4)
-    hipLaunchKernelGGL((hash_bwd_bin_count_k<3, 1>), dim3(blocks), dim3(FILL_POINTS), (size_t)NB * 4, s, coords, cdt, csn, csd, N, g, bp,
-                       primes, scale, ws.hist, ws.wg_counts, hi);
-  else if (g.dims == 3)
-    hipLaunchKernelGGL(hash_bwd_bin_count_k<3>, dim3(blocks), dim3(FILL_POINTS), (size_t)NB * 4, s, coords, cdt, csn, csd, N, g, bp,
-                       primes, scale, ws.hist, ws.wg_counts, hi);
-  else
-    hipLaunchKernelGGL(hash_bwd_bin_count_k<2>, dim3(blocks), dim3(FILL_POINTS), (size_t)NB * 4, s, coords, cdt, csn, csd, N, g, bp,
-                       primes, scale, ws.hist, ws.wg_counts, hi);
-  if (int rc = check_launch("hash_bwd_bin_count")) return rc;
-  hipLaunchKernelGGL(hash_bwd_bin_offsets_k, dim3(1), dim3(1024), 0, s, (const uint32_t*)ws.hist, ws.cursor, ws.n_tasks,
-                     ws.tasks, NB, max_tasks, bp, cell_task_div(N));
-  if (int rc = check_launch("hash_bwd_bin_offsets")) return rc;
-  const int feat = geom->feat;
-  for (int f0 = 0; f0 < feat; f0 += 2) {
-    if (f0 > 0) {
-      // the next pair of features: same bins and tasks; fresh level maxima and bin cursors
-      hipLaunchKernelGGL(hash_bwd_bin_zero_k, dim3(1), dim3(256), 0, s, ws.gmax, 32);
-      if (int rc = check_launch("hash_bwd_bin_zero")) return rc;
-      hipLaunchKernelGGL(hash_bwd_bin_offsets_k, dim3(1), dim3(1024), 0, s, (const uint32_t*)ws.hist, ws.cursor, ws.n_tasks,
-                         ws.tasks, NB, max_tasks, bp, cell_task_div(N));
-      if (int rc = check_launch("hash_bwd_bin_offsets")) return rc;
+  for (int hi = 0; hi < passes; ++hi)
+    for (int f0 = 0; f0 < feat; f0 += 2) {
+      DevGeom gg = g;
+      void* fill_args[] = {(void*)&coords, (void*)&cdt, (void*)&csn, (void*)&csd, (void*)&dout, (void*)&dout_stride, (void*)&N, (void*)&points,
+                           (void*)&gg, (void*)&bp, (void*)&primes, (void*)&scale, (void*)&ws, (void*)&max_nb, (void*)&feat, (void*)&f0, (void*)&hi};
+      if (int rc = launch("hash_bwd_bin_fill", fill, dim3((unsigned)ws.blocks), wide ? FILL_WIDE_THREADS : FILL_THREADS, fill_args, fill_lds)) return rc;
+      void* totals_args[] = {(void*)&ws, (void*)&bp};
+      const unsigned pieces = (unsigned)((ws.blocks + TOTALS_BLOCKS - 1) / TOTALS_BLOCKS);
+      if (int rc = launch("hash_bwd_bin_totals", (const void*)hash_bwd_bin_totals_k, dim3((unsigned)bin_pieces, pieces), 64, totals_args, 0)) return rc;
+      void* acc_args[] = {(void*)&ws, (void*)&table, (void*)&gg, (void*)&bp, (void*)&feat, (void*)&f0};
+      if (int rc = launch("hash_bwd_bin_accum", accum, dim3(units), ACC_THREADS, acc_args, acc_lds)) return rc;
+      const unsigned max_splits = (unsigned)NB < ws.max_slots / 2 ? (unsigned)NB : ws.max_slots / 2;
+      if (int rc = launch("hash_bwd_bin_reduce", reduce, dim3(2 * BIN_ROWS / REDUCE_VALUES, max_splits), REDUCE_THREADS, acc_args, 0)) return rc;
     }
-  {
-    const size_t lds = (size_t)FILL_RECORDS * sizeof(uint4) + (g32 ? (size_t)FILL_POINTS * sizeof(uint2) : 0) +
-                       ((size_t)2 * NB + 2 * NF_MAX_LEVELS) * 4;
-    const void* kern = g.dims == 6   ? (g32 ? (const void*)hash_bwd_bin_fill_k<true, 3, 3> : (const void*)hash_bwd_bin_fill_k<false, 3, 3>)
-                       : g.dims == 5 ? (g32 ? (const void*)hash_bwd_bin_fill_k<true, 3, 2> : (const void*)hash_bwd_bin_fill_k<false, 3, 2>)
-                       : g.dims == 4 ? (g32 ? (const void*)hash_bwd_bin_fill_k<true, 3, 1> : (const void*)hash_bwd_bin_fill_k<false, 3, 1>)
-                       : g.dims == 3 ? (g32 ? (const void*)hash_bwd_bin_fill_k<true, 3> : (const void*)hash_bwd_bin_fill_k<false, 3>)
-                                     : (g32 ? (const void*)hash_bwd_bin_fill_k<true, 2> : (const void*)hash_bwd_bin_fill_k<false, 2>);
-    hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return fail((int)e, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-    const uint32_t* wc = ws.wg_counts;
-    void* args[] = {(void*)&coords, (void*)&cdt,   (void*)&csn,    (void*)&csd,   (void*)&dout, (void*)&dout_stride, (void*)&N, (void*)&g,
-                    (void*)&bp,     (void*)&primes, (void*)&scale, (void*)&wc,    (void*)&ws.cursor, (void*)&ws.gmax, (void*)&ws.records,
-                    (void*)&feat,   (void*)&f0,     (void*)&hi};
-    e = hipLaunchKernel(kern, dim3(blocks), dim3(FILL_POINTS), args, lds, s);
-    if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(hash_bwd_bin_fill): %s", hipGetErrorString(e));
-    if (int rc = check_launch("hash_bwd_bin_fill")) return rc;
-  }
-  {
-    const size_t lds = (size_t)BIN_ROWS * 2 * sizeof(unsigned long long);
-    const void* kern = ddt == NF_F16    ? (const void*)hash_bwd_bin_accum_k<F16>
-                       : ddt == NF_BF16 ? (const void*)hash_bwd_bin_accum_k<BF16>
-                                        : (const void*)hash_bwd_bin_accum_k<F32>;
-    hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return fail((int)e, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-    const uint32_t* rc_ = ws.records;
-    const uint4* tk = ws.tasks;
-    const uint32_t* nt = ws.n_tasks;
-    const uint32_t* gm = ws.gmax;
-    void* args[] = {(void*)&rc_, (void*)&tk, (void*)&nt, (void*)&gm, (void*)&dtable, (void*)&g, (void*)&bp, (void*)&feat, (void*)&f0};
-    e = hipLaunchKernel(kern, dim3(max_tasks), dim3(ACC_THREADS), args, lds, s);
-    if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(hash_bwd_bin_accum): %s", hipGetErrorString(e));
-    if (int rc = check_launch("hash_bwd_bin_accum")) return rc;
-  }
-  }
-  }
   return 0;
 }
 

@@ -138,27 +138,62 @@ Tensor encode_forward(const Tensor& coords, const Tensor& table, const Tensor& p
   return out;
 }
 
+// The upstream gradient as rows that the kernels take, the scratch, and the point coordinates of a backward.
+struct BackwardArgs {
+  Rows rows;
+  Tensor c, ws;
+  int64_t n, csn, csd, bytes;
+  int dt;
+  BackwardArgs(const Tensor& coords, const Tensor& grad, const nf_hash_geom& g, int64_t flags) : rows(grad, grad.size(-1)) {
+    const int64_t D = coords.size(-1);
+    n = coords.numel() / D;
+    if (rows.n >= REPACK_MIN_POINTS && (rows.stride * grad.element_size() % 16 != 0 || (uintptr_t)rows.p % 16 != 0)) {
+      // gradient rows off 16-byte boundaries (the output carried appended features): the LDS-tile kernels read whole aligned
+      // rows, so the encoding's columns are packed first (one pass instead of scattered atomics per corner)
+      const int64_t width = g.levels * g.feat;
+      rows.hold = rows.hold.reshape({-1, grad.size(-1)}).narrow(1, 0, width).clone(at::MemoryFormat::Contiguous);
+      rows.p = rows.hold.data_ptr();
+      rows.stride = width;
+    }
+    dt = code_of(grad.scalar_type());
+    const bool flat = coords.is_contiguous();
+    c = flat ? coords : coords.reshape({-1, D});
+    csn = flat ? D : c.stride(0);
+    csd = flat ? 1 : c.stride(1);
+    bytes = nf_hash_encode_bwd_workspace_bytes(n, &g, dt, (int)flags);
+    ws = scratch(bytes, coords);
+  }
+};
+
+void encode_backward_add(const BackwardArgs& a, const Tensor& de, const Tensor& pi, const nf_hash_geom& g, double scale, int64_t flags) {
+  check(nf_hash_encode_bwd(a.c.data_ptr(), code_of(a.c.scalar_type()), a.csn, a.csd, a.rows.p, a.dt, a.rows.stride, de.data_ptr<float>(), a.n, &g,
+                           pi.data_ptr<int64_t>(), (float)scale, ptr(a.ws), a.bytes, (int)flags, stream_of(a.c)),
+        "nf_hash_encode_bwd");
+}
+
 // adds into de
 void encode_backward(const Tensor& coords, const Tensor& grad, const Tensor& de, const Tensor& pi, const nf_hash_geom& g, double scale, int64_t flags) {
   const c10::DeviceGuard guard(coords.device());
-  const int64_t D = coords.size(-1), n = coords.numel() / D;
-  Rows rows(grad, grad.size(-1));
-  if (rows.n >= REPACK_MIN_POINTS && (rows.stride * grad.element_size() % 16 != 0 || (uintptr_t)rows.p % 16 != 0)) {
-    // gradient rows off 16-byte boundaries (the output carried appended features): the LDS-tile kernels read whole aligned
-    // rows, so the encoding's columns are packed first (one pass instead of scattered atomics per corner)
-    const int64_t width = g.levels * g.feat;
-    rows.hold = rows.hold.reshape({-1, grad.size(-1)}).narrow(1, 0, width).clone(at::MemoryFormat::Contiguous);
-    rows.p = rows.hold.data_ptr();
-    rows.stride = width;
+  encode_backward_add(BackwardArgs(coords, grad, g, flags), de, pi, g, scale, flags);
+}
+
+// the gradient of `table`: in its own type where the kernels write it whole, else float32 sums that autograd rounds to that type
+Tensor encode_table_grad(const Tensor& coords, const Tensor& grad, const Tensor& table, const Tensor& pi, const Geometry& geo, double scale, int64_t flags) {
+  const c10::DeviceGuard guard(coords.device());
+  const BackwardArgs a(coords, grad, geo.g, flags);
+  if (table.size(0) == geo.rows && a.bytes > 0) {
+    const Tensor de = at::empty(table.sizes(), table.options());
+    const int rc = nf_hash_encode_bwd_write(a.c.data_ptr(), code_of(a.c.scalar_type()), a.csn, a.csd, a.rows.p, a.dt, a.rows.stride, de.data_ptr(),
+                                            code_of(table.scalar_type()), a.n, &geo.g, pi.data_ptr<int64_t>(), (float)scale, ptr(a.ws), a.bytes,
+                                            (int)flags, stream_of(a.c));
+    if (rc != NF_EUNSUPPORTED) {
+      check(rc, "nf_hash_encode_bwd_write");
+      return de;
+    }
   }
-  const int dt = code_of(grad.scalar_type());
-  const bool flat = coords.is_contiguous();
-  const Tensor c = flat ? coords : coords.reshape({-1, D});
-  const int64_t bytes = nf_hash_encode_bwd_workspace_bytes(n, &g, dt, (int)flags);
-  const Tensor ws = scratch(bytes, coords);
-  check(nf_hash_encode_bwd(c.data_ptr(), code_of(c.scalar_type()), flat ? D : c.stride(0), flat ? 1 : c.stride(1), rows.p, dt, rows.stride,
-                           de.data_ptr<float>(), n, &g, pi.data_ptr<int64_t>(), (float)scale, ptr(ws), bytes, (int)flags, stream_of(coords)),
-        "nf_hash_encode_bwd");
+  const Tensor de = at::zeros(table.sizes(), table.options().dtype(at::kFloat));
+  encode_backward_add(a, de, pi, geo.g, scale, flags);
+  return de;
 }
 
 struct HashEncoding : torch::autograd::Function<HashEncoding> {
@@ -175,9 +210,7 @@ struct HashEncoding : torch::autograd::Function<HashEncoding> {
     const at::AutoDispatchBelowADInplaceOrView below;
     const variable_list saved = ctx->get_saved_variables();
     const auto* geo = (const Geometry*)(uintptr_t)ctx->saved_data["geometry"].toInt();
-    // float32 accumulators; autograd rounds them once to the table's dtype
-    const Tensor de = at::zeros(saved[1].sizes(), saved[1].options().dtype(at::kFloat));
-    encode_backward(saved[0], grads[0], de, saved[2], geo->g, ctx->saved_data["scale"].toDouble(), ctx->saved_data["flags"].toInt());
+    const Tensor de = encode_table_grad(saved[0], grads[0], saved[1], saved[2], *geo, ctx->saved_data["scale"].toDouble(), ctx->saved_data["flags"].toInt());
     return {Tensor(), de, Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };

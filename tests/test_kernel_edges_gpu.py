@@ -26,6 +26,29 @@ def test_forward_sweep_deals_out_every_point(N, dims, dtype, monkeypatch):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("N", [1, 4096, 16384, 16385, 8 * 1024 * 3 + 1, 2**18 - 1, 2**20 + 5])
+@pytest.mark.parametrize("dims,F,T,L,dtype", [
+    (3, 2, 2**14, 16, torch.float32), (3, 2, 2**14, 4, torch.float16), (3, 2, 2**15, 16, torch.bfloat16), (2, 2, 2**14, 2, torch.float16),
+    (3, 4, 2**14, 16, torch.float16), (2, 2, 2**14, 16, torch.float32), (2, 4, 2**13, 2, torch.bfloat16), (3, 2, 2**11, 16, torch.float16),
+])
+def test_forward_with_levels_in_lds(N, dims, F, T, L, dtype, monkeypatch):
+    """Levels of up to 128 KiB are gathered from LDS, one or two to a workgroup: the bits of the per-(point, level) kernel
+    (flag 1), on points of the upper edge too, and into rows of a wider output."""
+    from triton_helpers_amd.layers.hash_encoding import kernel as hk
+
+    torch.manual_seed(6)
+    x = torch.rand(N, dims, device=DEV)
+    x[: N // 8, 0] = 1.0
+    x[: N // 16] = 1.0
+    table = torch.randn(O.level_row_offsets(L, T, dims, 16, 512)[-1], F, device=DEV).to(dtype)
+    tail = torch.zeros(N, 4, device=DEV, dtype=dtype)
+    outs = []
+    for flags in (0, 1):
+        monkeypatch.setattr(hk, "_FLAGS", flags)
+        outs.append([hk.hash_encoding(x, table, f, None, T, 16, 512, L) for f in (None, tail)])
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
 def _grads(tensors):
     return [None if t is None else t.grad for t in tensors]
 

@@ -16,6 +16,14 @@ struct DevGeom {
 
 constexpr int TILE_THREADS = 256;
 
+// Workgroup barrier that orders LDS accesses only: global stores issued before it stay in flight (a plain
+// __syncthreads() would wait for them to complete).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 struct Corner8 {
   uint32_t row[8];
 };

@@ -288,11 +288,13 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_tiled_k(const void* coo
 // so that all take the same number of gather rounds per level and stay at the same level: with the points dealt to workgroups evenly
 // but to their waves in turn (64 points to the first, the next 64 to the second, ...) some waves had one round per level and
 // some two, the first ran ahead and the tables of more levels than an L2 holds were in use at once (304800 points: 169 against 120 us).
+constexpr int LEVELS_THREADS = 1024, LEVELS_LDS = 128 * 1024, LEVELS_XCDS = 8;  // of the kernel that copies whole levels to LDS
+template <int WAVES = TILE_THREADS / 64>
 struct SweepPart {
   int64_t first;
   int count;
   __device__ __forceinline__ SweepPart(int64_t N, int per) {
-    first = ((int64_t)blockIdx.x * (TILE_THREADS / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * per;
+    first = ((int64_t)blockIdx.x * WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * per;
     const int64_t left = N - first;
     count = left < per ? (left > 0 ? (int)left : 0) : per;
     if (count == 0) first = N - 1;
@@ -315,7 +317,7 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_sweep_k(const void* coo
                                                                  int64_t N, int per, DevGeom g, const int64_t* primes, float scale) {
   constexpr int LMAX = 16;
   const int t = threadIdx.x, lane = t & 63;
-  const SweepPart part(N, per);
+  const SweepPart<> part(N, per);
   const int L = g.levels;
   float x[PPT][3];
 #pragma unroll
@@ -407,7 +409,7 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_sweep32_k(const void* c
                                                                    int64_t N, int per, DevGeom g, const int64_t* primes, float scale) {
   constexpr int LMAX = 16;
   const int lane = threadIdx.x & 63;
-  const SweepPart part(N, per);
+  const SweepPart<> part(N, per);
   const int L = g.levels;
   float x[PPT][3];
 #pragma unroll
@@ -470,6 +472,127 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_sweep32_k(const void* c
 #pragma unroll
     for (int q = 0; q < LMAX / 2; ++q)
       if (2 * q < L) dst[q] = make_float4(enc[i][2 * q].x, enc[i][2 * q].y, enc[i][2 * q + 1].x, enc[i][2 * q + 1].y);
+  }
+}
+
+// Levels in LDS: where the largest level of the table fits (2^14 rows, the reference's default, are 64 KiB of 16-bit pairs and 128 KiB of
+// float32 ones), a workgroup copies one level, or two, into LDS and takes its share of the points through them.  A gather from
+// memory costs a unit's L1 about one and a half cycles per lane and the waves wait for it; one from LDS a fraction of
+// one, and what is left is the vector arithmetic of the cell and the weights (about 105 instructions per point and level; 2^20 points
+// of 16 levels are 50 us of it).  Nothing is kept over the levels, so a thread needs 32 to 47 registers.  A row of the output is
+// written in 4- or 8-byte pieces by the workgroups of its levels: they sit on one XCD and go through the same points at the same
+// time, so the pieces meet in that XCD's L2 and leave it as whole lines.
+// Before -> after (sweep and per-(point, level) kernels, us): float32 2^14 rows, 2^18 points 80 -> 33, 2^20 307 -> 105; fp16 2^14
+// rows 2^18 54 -> 22, 2^20 184 -> 71; fp16 2^15 rows 2^20 234 -> 101; two dimensions fp16 2^20 97 -> 47; bf16 rows of four
+// features 2^20 256 -> 108; float32 2^16 points 25 -> 12.
+template <typename TT, int D, int FEAT, int LW>
+__global__ __launch_bounds__(LEVELS_THREADS) void hash_fwd_levels_k(const void* coords, int cdt, int64_t csn, int64_t csd, const uint32_t* table,
+                                                                    typename TT::storage* out, int64_t out_stride, int64_t N, int sets, int64_t share,
+                                                                    DevGeom g, const int64_t* primes, float scale) {
+  typedef typename TT::storage S;
+  constexpr int RW = FEAT * (int)sizeof(S) / 4, CN = 1 << D;  // words of a row, corners of a cell
+  typedef uint32_t Piece __attribute__((ext_vector_type(4), aligned(4)));  // a level begins wherever the one before it ends
+  extern __shared__ __align__(16) uint32_t level_rows[];
+  const int tid = threadIdx.x;
+  const int set = (int)(blockIdx.x / LEVELS_XCDS) % sets, part = (int)(blockIdx.x / (LEVELS_XCDS * sets)) * LEVELS_XCDS + (int)(blockIdx.x % LEVELS_XCDS);
+  const int64_t n_begin = (int64_t)part * share, n_end = n_begin + share < N ? n_begin + share : N;
+  if (n_begin >= n_end) return;
+  const int l0 = set * LW;
+  uint32_t base[LW];  // first word of the level in LDS
+  uint32_t at = 0;
+#pragma unroll
+  for (int k = 0; k < LW; ++k) {
+    base[k] = at;
+    if (l0 + k < g.levels) {
+      const uint32_t* src = table + g.row_offset[l0 + k] * RW;
+      const uint32_t words = g.rows[l0 + k] * RW, whole = words & ~3u;
+#pragma unroll 4
+      for (uint32_t i = tid * 4; i < whole; i += LEVELS_THREADS * 4) {
+        const Piece v = *reinterpret_cast<const Piece*>(src + i);
+        *reinterpret_cast<uint4*>(level_rows + at + i) = make_uint4(v[0], v[1], v[2], v[3]);
+      }
+      if (whole + tid < words) level_rows[at + whole + tid] = src[whole + tid];
+      at += (words + 3u) & ~3u;
+    }
+  }
+  __syncthreads();
+  uint32_t pi[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) pi[d] = d < D ? (uint32_t)primes[d < D ? d : 0] * (RW * 4) : 0u;
+  auto load_point = [&](int64_t n, float (&x)[3]) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const float v = load_as_f32(coords, n * csn + d * csd, cdt);
+      x[d] = scale != 1.0f ? v / scale : v;
+    }
+  };
+  float x[3], ahead[3] = {0.0f, 0.0f, 0.0f};
+  load_point(n_begin + tid < n_end ? n_begin + tid : n_end - 1, ahead);
+  for (int64_t n = n_begin + tid; n - tid < n_end; n += LEVELS_THREADS) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) x[d] = ahead[d];
+    load_point(n + LEVELS_THREADS < n_end ? n + LEVELS_THREADS : n_end - 1, ahead);
+    uint32_t enc[LW * RW];
+#pragma unroll
+    for (int k = 0; k < LW; ++k) {
+      const int l = l0 + k < g.levels ? l0 + k : l0;
+      const uint32_t res = (uint32_t)g.res[l];
+      const float fres = (float)g.res[l];
+      uint32_t c[3];
+      float fr[3], w[8];
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const float pos = x[d] * fres;
+        const float fl = floorf(pos);
+        c[d] = cell_index(fl, fres);
+        fr[d] = pos - fl;
+      }
+      // rows as byte offsets in the level: a hashed level's primes and mask carry the size of a row
+      Corner8 r;
+      if (l >= g.first_hash) {
+        const uint32_t mask = (g.rows[l] - 1) * (RW * 4);
+        r = D == 3 ? rows_d3(c, true, res, mask, pi) : rows_d2(c, true, res, mask, pi);
+      } else {
+        r = D == 3 ? rows_d3(c, false, res, g.rows[l] - 1, pi) : rows_d2(c, false, res, g.rows[l] - 1, pi);
+#pragma unroll
+        for (int j = 0; j < CN; ++j) r.row[j] *= RW * 4;
+      }
+      if (D == 3) weights_d3(fr, w);
+      else weights_d2(fr, w);
+      uint32_t v[CN][RW];
+#pragma unroll
+      for (int j = 0; j < CN; ++j) {
+        const uint32_t* row = reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(level_rows + base[k]) + r.row[j]);
+        if constexpr (RW == 2) {
+          const uint2 q = *reinterpret_cast<const uint2*>(row);
+          v[j][0] = q.x;
+          v[j][1] = q.y;
+        } else {
+          v[j][0] = *row;
+        }
+      }
+      float a[FEAT];
+#pragma unroll
+      for (int f = 0; f < FEAT; ++f) a[f] = 0.0f;
+#pragma unroll
+      for (int j = 0; j < CN; ++j)
+#pragma unroll
+        for (int f = 0; f < FEAT; ++f) {
+          if constexpr (sizeof(S) == 4) a[f] = a[f] + w[j] * __uint_as_float(v[j][f]);
+          else a[f] = a[f] + w[j] * TT::to_f32((uint16_t)(f & 1 ? v[j][f / 2] >> 16 : v[j][f / 2] & 0xffffu));
+        }
+#pragma unroll
+      for (int q = 0; q < RW; ++q) {
+        if constexpr (sizeof(S) == 4) enc[k * RW + q] = __float_as_uint(a[q]);
+        else enc[k * RW + q] = TT::pack(a[2 * q], a[2 * q + 1]);
+      }
+    }
+    if (n < n_end) {
+      uint32_t* dst = reinterpret_cast<uint32_t*>(out + n * out_stride + l0 * FEAT);
+      if constexpr (LW * RW == 1) *dst = enc[0];
+      else if (LW == 1 || l0 + 1 < g.levels) *reinterpret_cast<uint2*>(dst) = make_uint2(enc[0], enc[1]);
+      else *dst = enc[0];
+    }
   }
 }
 
@@ -656,6 +779,11 @@ constexpr int64_t LEVEL_MAX_POINTS = 65536;
 // run alone (304800 points, full workgroups of 1024: 298 workgroups, twice the time of 256).
 constexpr int64_t COMPUTE_UNITS = 256;
 
+// Levels in LDS: batches from which the copying pays.  Under that the per-(point, level) kernels run (16-bit pairs: 5.3 and 5.8 us
+// at 8192 points, 8.5 and 6.3 at 2^14; float32: 5.1 and 5.0 us at 4096, 6.2 and 5.5 at 8192), and for rows of four features the staged
+// kernel, which takes 20 us and more for any batch.
+constexpr int64_t LEVELS_MIN_POINTS_16 = 16384, LEVELS_MIN_POINTS_F32 = 4096;
+
 // points per wave, at most `most`, four waves to a workgroup
 static int sweep_wave_points(int64_t n, int most) {
   const int64_t waves = 4 * COMPUTE_UNITS * ((n + 4 * COMPUTE_UNITS * most - 1) / (4 * COMPUTE_UNITS * most));
@@ -695,6 +823,54 @@ static bool level_ok(const nf_hash_geom* g, int table_dt, const void* rows_ptr, 
     if ((r & (r - 1)) != 0) return false;
   }
   return ((uintptr_t)rows_ptr & 3u) == 0 && row_stride % 2 == 0;
+}
+
+// whether every level fits LDS and the rows can be read and written in words; pair: two levels fit together
+static bool levels_ok(const nf_hash_geom* g, int table_dt, const void* table, const void* out, int64_t out_stride, bool* pair) {
+  const int es = table_dt == NF_F32 ? 4 : 2, row = g->feat * es;
+  if ((g->dims != 2 && g->dims != 3) || g->levels > 16 || !(g->feat == 2 || (g->feat == 4 && es == 2))) return false;
+  int64_t most = 0;
+  for (int l = 0; l < g->levels; ++l) {
+    if (g->rows[l] * row > LEVELS_LDS) return false;
+    if (l >= g->first_hash_level && (g->rows[l] & (g->rows[l] - 1)) != 0) return false;
+    most = g->rows[l] > most ? g->rows[l] : most;
+  }
+  *pair = row == 4 && most * row <= LEVELS_LDS / 2;
+  const int piece = row == 4 && !*pair ? 4 : 8;
+  return ((uintptr_t)table & 3u) == 0 && ((uintptr_t)out % piece) == 0 && (out_stride * es) % piece == 0;
+}
+
+static int launch_fwd_levels(const void* coords, int cdt, int64_t csn, int64_t csd, const void* table, int table_dt, void* out, int64_t out_stride,
+                             int64_t N, const DevGeom& g, const int64_t* primes, float scale, bool pair, hipStream_t s) {
+  auto pick = [&](auto tt) -> const void* {
+    typedef decltype(tt) TT;
+    if constexpr (sizeof(typename TT::storage) == 4) return g.dims == 3 ? (const void*)hash_fwd_levels_k<TT, 3, 2, 1> : (const void*)hash_fwd_levels_k<TT, 2, 2, 1>;
+    else if (g.feat == 4) return g.dims == 3 ? (const void*)hash_fwd_levels_k<TT, 3, 4, 1> : (const void*)hash_fwd_levels_k<TT, 2, 4, 1>;
+    else if (pair) return g.dims == 3 ? (const void*)hash_fwd_levels_k<TT, 3, 2, 2> : (const void*)hash_fwd_levels_k<TT, 2, 2, 2>;
+    else return g.dims == 3 ? (const void*)hash_fwd_levels_k<TT, 3, 2, 1> : (const void*)hash_fwd_levels_k<TT, 2, 2, 1>;
+  };
+  const void* kern = table_dt == NF_F32 ? pick(F32{}) : table_dt == NF_F16 ? pick(F16{}) : pick(BF16{});
+  const int lw = pair ? 2 : 1, row = g.feat * (table_dt == NF_F32 ? 4 : 2);
+  int sets = (g.levels + lw - 1) / lw;
+  size_t lds = 0;
+  for (int l = 0; l < g.levels; l += lw) {
+    size_t bytes = 0;
+    for (int k = l; k < l + lw && k < g.levels; ++k) bytes += ((size_t)g.rows[k] * row + 15) / 16 * 16;
+    lds = bytes > lds ? bytes : lds;
+  }
+  hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return fail((int)e, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+  // one workgroup per unit: the points in parts, a multiple of the XCDs of them, and of at least a turn of the workgroup
+  int64_t parts = COMPUTE_UNITS / (LEVELS_XCDS * sets);
+  const int64_t most = (N + LEVELS_XCDS * LEVELS_THREADS - 1) / (LEVELS_XCDS * LEVELS_THREADS);
+  parts = LEVELS_XCDS * (most < parts ? most : parts);
+  int64_t share = (N + parts - 1) / parts;
+  const uint32_t* tab = (const uint32_t*)table;
+  DevGeom gg = g;
+  void* args[] = {(void*)&coords, (void*)&cdt, (void*)&csn, (void*)&csd, (void*)&tab, (void*)&out, (void*)&out_stride, (void*)&N, (void*)&sets, (void*)&share, (void*)&gg, (void*)&primes, (void*)&scale};
+  e = hipLaunchKernel(kern, dim3((unsigned)(parts * sets)), dim3(LEVELS_THREADS), args, lds, s);
+  if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(hash_fwd_levels): %s", hipGetErrorString(e));
+  return check_launch("hash_fwd_levels");
 }
 
 static bool sweep32_ok(const nf_hash_geom* g, const void* table, const void* rows_ptr, int64_t row_stride) {
@@ -813,6 +989,11 @@ extern "C" int nf_hash_encode_fwd(const void* coords, int coords_dtype, int64_t 
     return 0;
   }
 
+  bool level_pairs;
+  if (!(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FWD_STAGED)) &&
+      n_points >= (table_dtype == NF_F32 ? LEVELS_MIN_POINTS_F32 : geom->feat == 2 ? LEVELS_MIN_POINTS_16 : 1) &&
+      levels_ok(geom, table_dtype, table, out, out_stride_n, &level_pairs))
+    return launch_fwd_levels(coords, coords_dtype, csn, csd, table, table_dtype, out, out_stride_n, n_points, g, primes, scale, level_pairs, s);
   // float32 tables: the same sweep on 8-byte rows
   if (!(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FWD_STAGED)) && n_points >= SWEEP_MIN_POINTS_F32 && table_dtype == NF_F32 &&
       sweep32_ok(geom, table, out, out_stride_n)) {

@@ -108,14 +108,6 @@ struct BinWs {
   int start_stride, blocks;
 };
 
-// Workgroup barrier that orders LDS accesses only: global stores issued before it stay in flight (a plain
-// __syncthreads() would wait for them to complete).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // record = {row0 | row1 << 13 | w1[18:13] << 26,  w0 | w1[12:0] << 19,  packed gradient pair}
 __device__ __forceinline__ uint3 make_record(uint32_t row0, uint32_t row1, float w0, float w1, uint32_t packed) {
   const uint32_t q0 = (uint32_t)(w0 * (float)W_MAX + 0.5f), q1 = (uint32_t)(w1 * (float)W_MAX + 0.5f);

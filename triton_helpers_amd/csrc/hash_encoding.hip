@@ -596,82 +596,6 @@ __global__ __launch_bounds__(LEVELS_THREADS) void hash_fwd_levels_k(const void* 
   }
 }
 
-template <typename GT, int PPT>
-__global__ __launch_bounds__(TILE_THREADS) void hash_bwd_tiled_k(const void* coords, int cdt, int64_t csn, int64_t csd,
-                                                                 const uint16_t* dout, int64_t dout_stride,
-                                                                 float* dtable, int64_t N, DevGeom g,
-                                                                 const int64_t* primes, float scale) {
-  constexpr int P = TILE_THREADS * PPT;
-  constexpr int LD = P + 2;
-  extern __shared__ uint32_t stage[];
-  const int t = threadIdx.x;
-  const int64_t p0 = (int64_t)blockIdx.x * P;
-  const int L = g.levels;
-
-  const int pieces = L >> 2;
-  const int total = P * pieces;
-  for (int c = t; c < total; c += TILE_THREADS) {
-    const int p = c / pieces, q = c - p * pieces;
-    const int64_t n = p0 + p;
-    uint4 val = make_uint4(0u, 0u, 0u, 0u);
-    if (n < N) val = *reinterpret_cast<const uint4*>(dout + n * dout_stride + 8 * q);
-    stage[(4 * q + 0) * LD + p] = val.x;
-    stage[(4 * q + 1) * LD + p] = val.y;
-    stage[(4 * q + 2) * LD + p] = val.z;
-    stage[(4 * q + 3) * LD + p] = val.w;
-  }
-
-  float x[PPT][3];
-  bool valid[PPT];
-#pragma unroll
-  for (int i = 0; i < PPT; ++i) {
-    int64_t n = p0 + t + TILE_THREADS * i;
-    valid[i] = n < N;
-    if (n >= N) n = N - 1;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      float v = load_as_f32(coords, n * csn + d * csd, cdt);
-      x[i][d] = scale != 1.0f ? v / scale : v;
-    }
-  }
-  const uint32_t pi[3] = {(uint32_t)primes[0], (uint32_t)primes[1], (uint32_t)primes[2]};
-  __syncthreads();
-
-  for (int l = 0; l < L; ++l) {
-    const uint32_t res = (uint32_t)g.res[l];
-    const float fres = (float)g.res[l];
-    const bool hashed = l >= g.first_hash;
-    const uint32_t mask = g.rows[l] - 1;
-    float* tab = dtable + g.row_offset[l] * 2;
-#pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-      const uint32_t packed = stage[l * LD + t + TILE_THREADS * i];
-      // a zero upstream gradient (both features) contributes nothing
-      if (!valid[i] || (packed & 0x7fff7fffu) == 0u) continue;
-      const float g0 = GT::to_f32((uint16_t)(packed & 0xffffu));
-      const float g1 = GT::to_f32((uint16_t)(packed >> 16));
-      uint32_t c[3];
-      float fr[3];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const float pos = x[i][d] * fres;
-        const float fl = floorf(pos);
-        c[d] = cell_index(fl, fres);
-        fr[d] = pos - fl;
-      }
-      const Corner8 r = rows_d3(c, hashed, res, mask, pi);
-      float w[8];
-      weights_d3(fr, w);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float* dst = tab + 2 * (size_t)r.row[j];
-        unsafeAtomicAdd(dst, w[j] * g0);
-        unsafeAtomicAdd(dst + 1, w[j] * g1);
-      }
-    }
-  }
-}
-
 // Small batches: one thread per (point, level), the levels of a point side by side in blockIdx.y.  A thread per point
 // walks its levels one after the other, and a batch of a few thousand points is then a handful of workgroups that wait
 // out sixteen rounds of memory latency (forward) or queue five hundred atomics per thread behind each other (backward)
@@ -715,44 +639,41 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_level_k(const void* coo
   *reinterpret_cast<uint32_t*>(out + n * out_stride + 2 * l) = TT::pack(a0, a1);
 }
 
-template <typename GT, int D>
+// Backward of small batches: one lane per (point, level, corner, feature).  What it costs are the atomics' requests, one per 64 bytes
+// that a wave's instruction touches: with the features of a row, and the mostly adjacent rows of an x-pair of corners, in neighbouring
+// lanes, an instruction of 64 adds is about twenty requests, where a lane that goes through the corners of its own point makes
+// 64.  The cell is worked out once per lane, which costs next to nothing in comparison.
+// 4096 points, 16 levels of 2^19 rows: 55 -> 19 us.
+template <typename GT, int D, int FEAT>
 __global__ __launch_bounds__(TILE_THREADS) void hash_bwd_level_k(const void* coords, int cdt, int64_t csn, int64_t csd,
-                                                                 const uint16_t* dout, int64_t dout_stride, float* dtable,
+                                                                 const typename GT::storage* dout, int64_t dout_stride, float* dtable,
                                                                  int64_t N, DevGeom g, const int64_t* primes, float scale) {
+  constexpr int LANES = FEAT << D;  // of a point: corner, then feature
   const int l = blockIdx.y;
-  const int64_t n = (int64_t)blockIdx.x * TILE_THREADS + threadIdx.x;
+  const int64_t n = ((int64_t)blockIdx.x * TILE_THREADS + threadIdx.x) / LANES;
   if (n >= N) return;
-  const uint32_t packed = *reinterpret_cast<const uint32_t*>(dout + n * dout_stride + 2 * l);
-  // a zero upstream gradient (both features) contributes nothing
-  if ((packed & 0x7fff7fffu) == 0u) return;
-  constexpr int CN = 1 << D;
-  const float g0 = GT::to_f32((uint16_t)(packed & 0xffffu));
-  const float g1 = GT::to_f32((uint16_t)(packed >> 16));
-  const uint32_t pi[3] = {(uint32_t)primes[0], (uint32_t)primes[1], D > 2 ? (uint32_t)primes[D > 2 ? 2 : 0] : 0u};
-  const uint32_t res = (uint32_t)g.res[l];
+  const int f = (int)(threadIdx.x % FEAT), j = (int)(threadIdx.x % LANES) / FEAT;
+  const float grad = GT::to_f32(dout[n * dout_stride + l * FEAT + f]);
+  if (grad == 0.0f) return;
+  const uint32_t mask = g.rows[l] - 1, res = (uint32_t)g.res[l];
   const float fres = (float)g.res[l];
-  float* tab = dtable + g.row_offset[l] * 2;
-  uint32_t c[3];
-  float fr[3];
+  const bool hashed = l >= g.first_hash;
+  uint32_t row = 0u, unit = 1u;
+  float w = 1.0f;
 #pragma unroll
   for (int d = 0; d < D; ++d) {
     float v = load_as_f32(coords, n * csn + d * csd, cdt);
     v = scale != 1.0f ? v / scale : v;
     const float pos = v * fres;
-    const float fl = floorf(pos);
-    c[d] = cell_index(fl, fres);
-    fr[d] = pos - fl;
+    const float fl = floorf(pos), fr = pos - fl;
+    const uint32_t side = (uint32_t)(j >> d) & 1u, c = cell_index(fl, fres) + side;
+    const float wd = side ? fr : 1.0f - fr;
+    w = d == 0 ? wd : w * wd;
+    row = hashed ? row ^ c * (uint32_t)primes[d] : row + c * unit;
+    unit *= res;
   }
-  const Corner8 r = D == 3 ? rows_d3(c, l >= g.first_hash, res, g.rows[l] - 1, pi) : rows_d2(c, l >= g.first_hash, res, g.rows[l] - 1, pi);
-  float w[8];
-  if (D == 3) weights_d3(fr, w);
-  else weights_d2(fr, w);
-#pragma unroll
-  for (int j = 0; j < CN; ++j) {
-    float* dst = tab + 2 * (size_t)r.row[j];
-    unsafeAtomicAdd(dst, w[j] * g0);
-    unsafeAtomicAdd(dst + 1, w[j] * g1);
-  }
+  row = hashed ? row & mask : row < mask ? row : mask;  // (x == scale in two dimensions, see rows_d2())
+  unsafeAtomicAdd(dtable + (g.row_offset[l] + (int64_t)row) * FEAT + f, w * grad);
 }
 
 // ---------------------------------------------------------------------------
@@ -760,7 +681,6 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_bwd_level_k(const void* coo
 // ---------------------------------------------------------------------------
 // below this many points the scattered-atomic kernels are faster than planning + scanning
 constexpr int64_t SCAN_MIN_POINTS = 32768;
-constexpr int64_t BIN_MIN_POINTS = 8192;  // below: the sort's fixed cost (about 100 us) exceeds the scattered atomics' 13 ns per point
 constexpr int SWEEP_PPT = 4;
 // Batches from which the sweeps run.  In three dimensions with 16-bit tables the staged kernel's 512 points per workgroup are one
 // workgroup per unit up to 2^17 points (51 us, the sweep 56) and two beyond (150000 points: 97 us, the sweep 67); the other kinds have
@@ -1080,7 +1000,7 @@ extern "C" int nf_hash_encode_fwd(const void* coords, int coords_dtype, int64_t 
 // whether a batch is large enough for one of the backward's LDS-tile variants
 static bool bwd_tiles_apply(int64_t n_points, const nf_hash_geom* geom, int flags) {
   if (flags & NF_HASH_FORCE_PLANES) return n_points >= SCAN_MIN_POINTS;
-  return n_points >= BIN_MIN_POINTS || bwd_direct_applies(n_points, geom, flags);
+  return n_points >= bwd_records_min(geom, flags) || bwd_walk_applies(n_points, geom, flags);
 }
 
 extern "C" int64_t nf_hash_encode_bwd_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags) {
@@ -1121,30 +1041,19 @@ extern "C" int nf_hash_encode_bwd(const void* coords, int coords_dtype, int64_t 
       return launch_bwd_scan(coords, coords_dtype, csn, csd, dout, dout_dtype, dout_stride_n, dtable, n_points, geom, g,
                              primes, scale, workspace, s);
   }
-  // small batches: a thread per (point, level)
-  if (!(flags & NF_HASH_FORCE_GENERIC) && level_ok(geom, dout_dtype, dout, dout_stride_n) &&
-      (n_points < BIN_MIN_POINTS || !tiled_ok(geom, dout_dtype, dout, dout_stride_n))) {
-    dim3 grid((unsigned)((n_points + TILE_THREADS - 1) / TILE_THREADS), (unsigned)g.levels);
-    const void* kern = dout_dtype == NF_F16 ? (g.dims == 3 ? (const void*)hash_bwd_level_k<F16, 3> : (const void*)hash_bwd_level_k<F16, 2>)
-                                            : (g.dims == 3 ? (const void*)hash_bwd_level_k<BF16, 3> : (const void*)hash_bwd_level_k<BF16, 2>);
-    const uint16_t* d = (const uint16_t*)dout;
-    void* args[] = {&coords, &coords_dtype, &csn, &csd, &d, &dout_stride_n, &dtable, &n_points, &g, &primes, &scale};
+  if (!(flags & NF_HASH_FORCE_GENERIC) && bwd_level_ok(geom)) {
+    auto pick = [&](auto gt) -> const void* {
+      typedef decltype(gt) GT;
+      return g.feat == 2 ? (g.dims == 3 ? (const void*)hash_bwd_level_k<GT, 3, 2> : (const void*)hash_bwd_level_k<GT, 2, 2>)
+                         : (g.dims == 3 ? (const void*)hash_bwd_level_k<GT, 3, 4> : (const void*)hash_bwd_level_k<GT, 2, 4>);
+    };
+    const void* kern = dout_dtype == NF_F32 ? pick(F32{}) : dout_dtype == NF_F16 ? pick(F16{}) : pick(BF16{});
+    const int64_t lanes = n_points * (g.feat << g.dims);
+    dim3 grid((unsigned)((lanes + TILE_THREADS - 1) / TILE_THREADS), (unsigned)g.levels);
+    void* args[] = {&coords, &coords_dtype, &csn, &csd, &dout, &dout_stride_n, &dtable, &n_points, &g, &primes, &scale};
     const hipError_t e = hipLaunchKernel(kern, grid, dim3(TILE_THREADS), args, 0, s);
     if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(hash_bwd_level): %s", hipGetErrorString(e));
     return check_launch("hash_bwd_level");
-  }
-  if (!(flags & NF_HASH_FORCE_GENERIC) && tiled_ok(geom, dout_dtype, dout, dout_stride_n)) {
-    constexpr int PPT = 2;
-    constexpr int P = TILE_THREADS * PPT;
-    const size_t lds = (size_t)g.levels * (P + 2) * sizeof(uint32_t);
-    dim3 grid((unsigned)((n_points + P - 1) / P));
-    if (dout_dtype == NF_F16)
-      hipLaunchKernelGGL((hash_bwd_tiled_k<F16, PPT>), grid, dim3(TILE_THREADS), lds, s, coords, coords_dtype, csn,
-                         csd, (const uint16_t*)dout, dout_stride_n, dtable, n_points, g, primes, scale);
-    else
-      hipLaunchKernelGGL((hash_bwd_tiled_k<BF16, PPT>), grid, dim3(TILE_THREADS), lds, s, coords, coords_dtype, csn,
-                         csd, (const uint16_t*)dout, dout_stride_n, dtable, n_points, g, primes, scale);
-    return check_launch("hash_bwd_tiled");
   }
   dim3 grid((unsigned)((n_points + 255) / 256), (unsigned)g.levels);
   switch (g.dims) {
@@ -1167,7 +1076,7 @@ extern "C" int nf_hash_encode_bwd_write(const void* coords, int coords_dtype, in
   NF_REQUIRE(dtype_ok(coords_dtype) && dtype_ok(dout_dtype) && dtype_ok(table_dtype), NF_EINVAL, "unknown dtype code");
   NF_REQUIRE(dout_stride_n >= (int64_t)g.levels * g.feat, NF_EINVAL, "dout_stride_n=%lld < levels*feat", (long long)dout_stride_n);
   NF_REQUIRE(scale > 0.0f, NF_EINVAL, "scale must be positive");
-  NF_REQUIRE(n_points >= BIN_MIN_POINTS && bwd_write_applies(n_points, geom, flags) &&
+  NF_REQUIRE(bwd_write_applies(n_points, geom, flags) &&
                  !(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FORCE_ATOMIC | NF_HASH_FORCE_PLANES)),
              NF_EUNSUPPORTED, "no kernel that writes this gradient in one go (nothing was launched; use nf_hash_encode_bwd)");
   NF_REQUIRE(coords && dout && dtable && primes && workspace, NF_EINVAL, "NULL pointer argument");
@@ -1176,7 +1085,7 @@ extern "C" int nf_hash_encode_bwd_write(const void* coords, int coords_dtype, in
              "shape or alignment outside the sorted-record kernels (nothing was launched; use nf_hash_encode_bwd)");
   NF_REQUIRE(workspace_bytes >= need && (uintptr_t)workspace % 16 == 0, NF_EINVAL, "a 16-byte aligned workspace of %lld bytes is needed", (long long)need);
   return launch_bwd_write(coords, coords_dtype, csn, csd, dout, dout_dtype, dout_stride_n, dtable, table_dtype, n_points, geom, g, primes, scale,
-                          workspace, (hipStream_t)stream);
+                          workspace, flags, (hipStream_t)stream);
 }
 
 extern "C" int nf_hash_encode_indices_fast(const void* coords, int coords_dtype, int64_t csn, int64_t csd,

@@ -299,11 +299,6 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t m) {
   return m;
 }
 
-__global__ void hash_bwd_bin_zero_k(uint32_t* p, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0u;
-}
-
 // ---------------------------------------------------------------------------------------
 // fill
 // ---------------------------------------------------------------------------------------
@@ -687,6 +682,28 @@ __device__ __forceinline__ void store_pair(void* table, int64_t i, float x, floa
   }
 }
 
+template <int MODE>
+__device__ __forceinline__ void add_or_store_pair(void* table, int64_t i, float x, float y, bool whole, bool pair) {
+  if constexpr (MODE == TABLE_ADD) {
+    float* cell = reinterpret_cast<float*>(table) + i;
+    if (x != 0.0f) cell[0] += x;
+    if (pair && y != 0.0f) cell[1] += y;
+  } else {
+    store_pair<MODE>(table, i, x, y, whole, pair);
+  }
+}
+
+// body(integral_constant) for the mode in use
+template <typename Body>
+__host__ __device__ __forceinline__ auto with_mode(int mode, Body&& body) {
+  switch (mode) {
+    case TABLE_ADD: return body(std::integral_constant<int, TABLE_ADD>{});
+    case TABLE_F32: return body(std::integral_constant<int, TABLE_F32>{});
+    case TABLE_F16: return body(std::integral_constant<int, TABLE_F16>{});
+    default: return body(std::integral_constant<int, TABLE_BF16>{});
+  }
+}
+
 template <typename GT, int MODE>
 __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, void* table, DevGeom g, BinPlan bp, int feat, int f0) {
   typedef typename BinRec<GT>::type Rec;
@@ -1042,195 +1059,296 @@ __global__ __launch_bounds__(REDUCE_THREADS) void hash_bwd_bin_reduce_k(BinWs ws
 }
 
 // ---------------------------------------------------------------------------------------
-// Levels of a few bins: no records
+// Small batches, and levels of a few bins: no records
 // ---------------------------------------------------------------------------------------
-// When a level's table is only a few bins (the reference's default of 2^14 rows per level is two), a sorted record per
-// corner pair costs more than hashing a point once per bin: a workgroup owns one bin and a slice of the points, walks
-// the slice, hashes each point's corners and adds those that fall into its bin to the same 64-bit fixed-point LDS tile
-// as the record kernels, then adds the tile to the table.  The upstream gradient is transposed first into level-major
-// pairs, so that a bin's walk reads 4 (float32: 8) contiguous bytes per point instead of touching a whole row; the same
-// pass takes the per-level maxima that set the fixed-point scales.
-constexpr int DIRECT_THREADS = 1024;
-constexpr int DIRECT_PREP_THREADS = 256;
+// Where points times bins are few, sorting costs more than hashing a point once per bin: a task is one bin of a level and a slice of
+// the points; its workgroup walks the slice, hashes each point's corners and adds those inside its bin to the same 64-bit
+// fixed-point LDS tile as the record kernels.  The upstream gradient is transposed first into level-major pairs, so that a
+// task's walk reads 4 (float32: 8) contiguous bytes per point instead of touching a whole row; the same pass takes the maxima that
+// set the fixed-point scales.  A bin of one slice goes from the tile to the table; slices leave their sums in slots, which a last
+// pass adds in their order: a gradient has the same bits in every run.
+// Before (two rounds of workgroups that waited for each point, scattered adds of the tiles, zeros and rounding of the table as passes of
+// their own) -> now: 2^14 rows float32, 2^18 points 145 -> 68 us, of which the walk 91 -> 42; fp16 2^16 rows, 8192 points 80 -> 35 (was: records).
+constexpr int WALK_THREADS = 1024;
+constexpr int WALK_PREP_THREADS = 256;
+constexpr int WALK_STRIDE = 16;  // points between neighbouring lanes of a walk
 
-// pairs[(level * np + p) * N + n] = features 2p, 2p + 1 of the level's gradient of point n (np = ceil(feat / 2); a missing
-// partner is zero); gmax[level] = largest |gradient| pattern of the level over all its features
-template <bool G32>
-__global__ __launch_bounds__(DIRECT_PREP_THREADS) void hash_bwd_direct_prep_k(const void* dout_v, int64_t dout_stride, int64_t N,
-                                                                               int levels, int feat, uint32_t* pairs, uint32_t* gmax) {
-  __shared__ uint32_t lmax[NF_MAX_LEVELS];
+struct WalkPlan {
+  int n_levels, n_tasks, prep_blocks;
+  int bins[NF_MAX_LEVELS], slices[NF_MAX_LEVELS];
+  int first[NF_MAX_LEVELS + 1];  // first task of a level; task first + which * slices + slice
+};
+// What a task's tile holds.  A level of one bin: both features of the pair.  A level of two bins: one of the features, of all the
+// level's rows; either way every corner of a point lands in the tile, so the walk has no test per corner and its LDS adds
+// run with all lanes.  A level of more bins: both features of one bin's rows.
+enum WalkKind { WALK_LEVEL = 0, WALK_FEATURE = 1, WALK_BIN = 2 };
+
+struct WalkWs {
+  uint32_t* block_max;  // [levels][ceil(feat / 2)][prep_blocks] largest |gradient| pattern of a block of points
+  float* points;        // [dims][N] coordinates, divided by the scale
+  uint32_t* pairs;      // [levels][ceil(feat / 2)][N] gradient pairs (a missing partner is zero)
+  float* slots;         // [n_tasks][2 * BIN_ROWS], where any level has more than one slice
+};
+
+// Gradient pairs level by level and coordinates dimension by dimension, both in the order of the walk: neighbouring lanes of a walk take
+// points WALK_STRIDE apart, because along a ray neighbouring points share cells and their adds to one row would wait for each other
+// (T = 2^14, 2^18 points along rays: 258 us without, 85 with).  The pass is bound by its loads, a row per lane: they are all
+// asked for before any is used (a loop over the levels that waited for each pair took 45 us for 2^18 rows of 16 float32 pairs, this 18).
+template <bool G32, int D>
+__global__ __launch_bounds__(WALK_PREP_THREADS) void hash_bwd_walk_prep_k(const void* coords, int cdt, int64_t csn, int64_t csd, float scale,
+                                                                          const void* dout_v, int64_t dout_stride, int64_t N, int levels, int feat,
+                                                                          WalkWs ws) {
+  extern __shared__ uint32_t plane_max[];
   const int tid = threadIdx.x, lane = tid & 63;
-  if (tid < NF_MAX_LEVELS) lmax[tid] = 0u;
+  const int np = (feat + 1) / 2, planes = levels * np;
+  for (int i = tid; i < planes; i += WALK_PREP_THREADS) plane_max[i] = 0u;
   __syncthreads();
-  const int64_t n = (int64_t)blockIdx.x * DIRECT_PREP_THREADS + tid;
-  const bool valid = n < N;
-  const int np = (feat + 1) / 2;
-  const uint16_t* row16 = reinterpret_cast<const uint16_t*>(dout_v) + (valid ? n : 0) * dout_stride;
-  const float* row32 = reinterpret_cast<const float*>(dout_v) + (valid ? n : 0) * dout_stride;
-  // an even row width with 4-byte aligned rows: a pair is one dword
-  const bool dword_pairs = !G32 && (feat & 1) == 0 && ((uintptr_t)dout_v & 3u) == 0 && (dout_stride & 1) == 0;
-  // rows of up to sixteen levels of one pair each, 16-byte aligned: the row in four loads, level l in dword l
-  const bool row_vec = !G32 && feat == 2 && levels <= 16 && (levels & 3) == 0 && ((uintptr_t)dout_v & 15u) == 0 && (dout_stride & 7) == 0;
+  const int64_t at = (int64_t)blockIdx.x * WALK_PREP_THREADS + tid;  // position in the walk's order
+  const bool valid = at < N;
+  constexpr int CHUNK = 64 * WALK_STRIDE;
+  const int64_t chunk = at / CHUNK * CHUNK;
+  const int in_chunk = (int)(at - chunk);
+  const int64_t n = !valid ? 0 : chunk + CHUNK <= N ? chunk + (in_chunk & 63) * WALK_STRIDE + (in_chunk >> 6) : at;
+  float v[D];
+  load_point_d<D>(coords, cdt, csn, csd, n, scale, v);
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (valid) ws.points[d * N + at] = v[d];
+  const uint16_t* row16 = reinterpret_cast<const uint16_t*>(dout_v) + n * dout_stride;
+  const float* row32 = reinterpret_cast<const float*>(dout_v) + n * dout_stride;
+  auto put = [&](int plane, uint32_t x, uint32_t y) {
+    if (valid) {
+      if (G32) reinterpret_cast<uint2*>(ws.pairs)[(int64_t)plane * N + at] = make_uint2(x, y);
+      else ws.pairs[(int64_t)plane * N + at] = x;
+    }
+    uint32_t m = G32 ? max(x & 0x7fffffffu, y & 0x7fffffffu) : max(x & 0x7fffu, (x >> 16) & 0x7fffu);
+    m = wave_max_u32(valid ? m : 0u);
+    if (lane == 63 && m) atomicMax(plane_max + plane, m);
+  };
+  // rows of whole 16-byte pieces, each four planes (float32: two); pieces of a row that ends between them read zeros
+  constexpr int PER = G32 ? 2 : 4;
+  const bool row_vec = (feat & 1) == 0 && planes % PER == 0 && ((uintptr_t)dout_v & 15u) == 0 && dout_stride % (G32 ? 4 : 8) == 0;
   if (row_vec) {
-    uint32_t gr[16];
+    constexpr int AT_ONCE = 8;
+    const uint4* row = G32 ? reinterpret_cast<const uint4*>(row32) : reinterpret_cast<const uint4*>(row16);
+    for (int q0 = 0; q0 < planes / PER; q0 += AT_ONCE) {
+      uint4 q[AT_ONCE];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      uint4 t = make_uint4(0u, 0u, 0u, 0u);
-      if (valid && 4 * i < levels) t = reinterpret_cast<const uint4*>(row16)[i];
-      gr[4 * i] = t.x;
-      gr[4 * i + 1] = t.y;
-      gr[4 * i + 2] = t.z;
-      gr[4 * i + 3] = t.w;
-    }
+      for (int i = 0; i < AT_ONCE; ++i)
+        if (q0 + i < planes / PER) q[i] = row[q0 + i];
 #pragma unroll
-    for (int l = 0; l < 16; ++l) {
-      if (l >= levels) break;
-      if (valid) pairs[(int64_t)l * N + n] = gr[l];
-      const uint32_t pk = gr[l] & 0x7fff7fffu;
-      const uint32_t m = wave_max_u32(max(pk & 0xffffu, pk >> 16));
-      if (lane == 63 && m) atomicMax(lmax + l, m);
-    }
-  } else
-  for (int l = 0; l < levels; ++l) {
-    uint32_t m = 0u;
-    for (int p = 0; p < np; ++p) {
-      const int e0 = l * feat + 2 * p;
-      const bool two = 2 * p + 1 < feat;
-      const int64_t at = ((int64_t)l * np + p) * N + n;
-      if (G32) {
-        uint2 pair = make_uint2(0u, 0u);
-        if (valid) {
-          pair.x = __float_as_uint(row32[e0]);
-          if (two) pair.y = __float_as_uint(row32[e0 + 1]);
-          reinterpret_cast<uint2*>(pairs)[at] = pair;
-        }
-        const uint32_t a0 = pair.x & 0x7fffffffu, a1 = pair.y & 0x7fffffffu;
-        m = max(m, max(a0, a1));
-      } else {
-        uint32_t packed = 0u;
-        if (valid) {
-          if (dword_pairs) {
-            packed = reinterpret_cast<const uint32_t*>(row16)[e0 >> 1];
+      for (int i = 0; i < AT_ONCE; ++i)
+        if (q0 + i < planes / PER) {
+          const int plane = (q0 + i) * PER;
+          if constexpr (G32) {
+            put(plane, q[i].x, q[i].y);
+            put(plane + 1, q[i].z, q[i].w);
           } else {
-            packed = row16[e0];
-            if (two) packed |= (uint32_t)row16[e0 + 1] << 16;
+            put(plane, q[i].x, 0u);
+            put(plane + 1, q[i].y, 0u);
+            put(plane + 2, q[i].z, 0u);
+            put(plane + 3, q[i].w, 0u);
           }
-          pairs[at] = packed;
         }
-        const uint32_t pk = packed & 0x7fff7fffu;
-        m = max(m, max(pk & 0xffffu, pk >> 16));
-      }
     }
-    m = wave_max_u32(m);
-    if (lane == 63 && m) atomicMax(lmax + l, m);
+  } else {
+    for (int plane = 0; plane < planes; ++plane) {
+      const int e0 = plane / np * feat + 2 * (plane % np);
+      const bool two = 2 * (plane % np) + 1 < feat;
+      if (G32) put(plane, __float_as_uint(row32[e0]), two ? __float_as_uint(row32[e0 + 1]) : 0u);
+      else put(plane, (uint32_t)row16[e0] | (two ? (uint32_t)row16[e0 + 1] << 16 : 0u), 0u);
+    }
   }
   __syncthreads();
-  if (tid < levels) {
-    const uint32_t m = lmax[tid];
-    if (m > *(volatile uint32_t*)(gmax + tid)) atomicMax(gmax + tid, m);
+  for (int i = tid; i < planes; i += WALK_PREP_THREADS) ws.block_max[(int64_t)i * gridDim.x + blockIdx.x] = plane_max[i];
+}
+
+template <typename GT, int D>
+__global__ __launch_bounds__(WALK_THREADS) void hash_bwd_walk_k(WalkWs ws, int64_t N, DevGeom g, WalkPlan wp, const int64_t* primes, void* table, int mode,
+                                                                int feat, int p) {
+  constexpr bool G32 = sizeof(typename BinRec<GT>::type) == 16;
+  constexpr int CN = 1 << D, VD = D > 3 ? D : 3;
+  extern __shared__ unsigned long long acc_tile[];  // 2 * BIN_ROWS sums
+  __shared__ uint32_t level_max, hit;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int np = (feat + 1) / 2, f0 = 2 * p;
+  const bool has_pair = f0 + 1 < feat;
+  const uint32_t pi[3] = {(uint32_t)primes[0], (uint32_t)primes[1], D > 2 ? (uint32_t)primes[D > 2 ? 2 : 0] : 0u};
+  for (uint32_t i = tid; i < 2u * BIN_ROWS; i += WALK_THREADS) acc_tile[i] = 0ull;
+  if (tid == 0) level_max = hit = 0u;
+  for (int t = (int)blockIdx.x; t < wp.n_tasks; t += (int)gridDim.x) {
+    int l = 0;
+    while (l + 1 < wp.n_levels && t >= wp.first[l + 1]) ++l;
+    const int slices = wp.slices[l], which = (t - wp.first[l]) / slices, slice = (t - wp.first[l]) % slices;
+    const WalkKind kind = wp.bins[l] == 1 ? WALK_LEVEL : wp.bins[l] == 2 ? WALK_FEATURE : WALK_BIN;
+    if (kind == WALK_FEATURE && which == 1 && !has_pair) continue;  // an odd feature count: the last pair has one feature
+    const uint32_t row0 = kind == WALK_BIN ? (uint32_t)which << BIN_ROWS_LOG2 : 0u;
+    const uint32_t left = g.rows[l] - row0, nrows = kind == WALK_BIN && left > (uint32_t)BIN_ROWS ? (uint32_t)BIN_ROWS : left;
+    // fixed-point scale 2^se of the pair on this level, as in the record kernels:  |w * g| * 2^se < 2^30
+    uint32_t m = 0u;
+    for (int i = tid; i < wp.prep_blocks; i += WALK_THREADS) m = max(m, ws.block_max[((int64_t)l * np + p) * wp.prep_blocks + i]);
+    m = wave_max_u32(m);
+    __syncthreads();  // the tile is clear, and nobody reads the maximum of the task before
+    if (lane == 63 && m) atomicMax(&level_max, m);
+    __syncthreads();
+    const float gm = BinRec<GT>::level_max(level_max);
+    const bool nonfinite = !(gm <= 3.0e38f);
+    int se = 0;
+    if (!nonfinite && gm > 0.0f) {
+      int ex;
+      frexpf(gm, &ex);
+      se = 30 - ex;
+      se = se > 120 ? 120 : se;
+    }
+    // |g| * 2^se < 2^30: the scaled gradient is a float (the two steps are exact powers of two inside float range)
+    const float s_lo = nonfinite ? 0.0f : ldexpf(1.0f, se / 2), s_hi = ldexpf(1.0f, se - se / 2);
+    const bool hashed = l >= g.first_hash;
+    const float fres = (float)g.res[l];
+    const uint32_t res = (uint32_t)g.res[l], mask = g.rows[l] - 1u;
+    const uint32_t* level_pairs = ws.pairs + (((int64_t)l * np + p) * N) * (G32 ? 2 : 1);
+    const int64_t n_begin = N * slice / slices, n_end = N * (slice + 1) / slices;
+    struct Point {
+      float v[VD];
+      typename BinRec<GT>::type rec;
+    };
+    auto load = [&](int64_t n) {
+      Point q = {{}, BinRec<GT>::zero()};
+#pragma unroll
+      for (int d = 0; d < D; ++d) q.v[d] = ws.points[d * N + n];
+      if constexpr (G32) {
+        const uint2 pair = reinterpret_cast<const uint2*>(level_pairs)[n];
+        q.rec.z = pair.x;
+        q.rec.w = pair.y;
+      } else {
+        q.rec.z = level_pairs[n];
+      }
+      return q;
+    };
+    // One point per thread and turn, the next one under way.  The loop exists in six copies, by the kind of tile and for levels with an
+    // inf or a nan in their gradient (which only mark the rows they touch), so that it carries no branch.
+    auto walk = [&](auto kind_c, auto nonfinite_c) {
+      constexpr WalkKind KIND = decltype(kind_c)::value;
+      constexpr bool NONFINITE = decltype(nonfinite_c)::value;
+      auto fixed = [&](float w, float gs) { return NONFINITE ? (int32_t)(w != 0.0f) : round_to_int(w * gs); };
+      auto add_to = [&](uint32_t at, int32_t f) { atomicAdd(acc_tile + at, (unsigned long long)(long long)f); };
+      if (n_begin + tid >= n_end) return;
+      Point next = load(n_begin + tid);
+      for (int64_t n = n_begin + tid; n < n_end; n += WALK_THREADS) {
+        const Point q = next;
+        next = load(n + WALK_THREADS < n_end ? n + WALK_THREADS : n);
+        uint32_t row[CN];
+        float w[CN];
+        cell_rows<D>(q.v, fres, hashed, res, mask, pi, primes, row, w);
+        const float g0 = BinRec<GT>::g0(q.rec) * s_lo * s_hi, g1 = BinRec<GT>::g1(q.rec) * s_lo * s_hi;
+        const float gs = which ? g1 : g0;
+        if constexpr (KIND == WALK_BIN) {
+#pragma unroll
+          for (int j = 0; j < CN; j += 2) {
+            const uint32_t a = row[j] - row0, b = row[j + 1] - row0;
+            if (a < (uint32_t)BIN_ROWS || b < (uint32_t)BIN_ROWS) {
+              hit = 1u;
+              if (a < (uint32_t)BIN_ROWS) {
+                add_to(a, fixed(w[j], g0));
+                if (has_pair) add_to((uint32_t)BIN_ROWS + a, fixed(w[j], g1));
+              }
+              if (b < (uint32_t)BIN_ROWS) {
+                add_to(b, fixed(w[j + 1], g0));
+                if (has_pair) add_to((uint32_t)BIN_ROWS + b, fixed(w[j + 1], g1));
+              }
+            }
+          }
+        } else {
+          // zero contributions are rare here: the adds carry no test
+#pragma unroll
+          for (int j = 0; j < CN; ++j) {
+            if constexpr (KIND == WALK_FEATURE) {
+              add_to(row[j], fixed(w[j], gs));
+            } else {
+              add_to(row[j], fixed(w[j], g0));
+              add_to((uint32_t)BIN_ROWS + row[j], has_pair ? fixed(w[j], g1) : 0);
+            }
+          }
+        }
+      }
+      if constexpr (KIND != WALK_BIN) hit = 1u;
+    };
+    auto walk_kind = [&](auto kind_c) {
+      if (nonfinite) walk(kind_c, std::true_type{});
+      else walk(kind_c, std::false_type{});
+    };
+    if (kind == WALK_LEVEL) walk_kind(std::integral_constant<WalkKind, WALK_LEVEL>{});
+    else if (kind == WALK_FEATURE) walk_kind(std::integral_constant<WalkKind, WALK_FEATURE>{});
+    else walk_kind(std::integral_constant<WalkKind, WALK_BIN>{});
+    lds_barrier();
+    // the tile to the slot or the table, and back to zero for the next task; a tile that nothing was added to is zeros already
+    const bool touched = hit != 0u;
+    const float qnan = __uint_as_float(0x7fc00000u);
+    const double unscale = ldexp(1.0, -se), unscale_hi = ldexp(1.0, 32 - se);
+    auto value = [&](uint32_t i) {
+      if (!touched) return 0.0f;
+      const long long a = (long long)acc_tile[i];
+      acc_tile[i] = 0ull;
+      const float x = (float)((double)(int)(a >> 32) * unscale_hi + (double)(uint32_t)a * unscale);
+      return nonfinite && a != 0 ? qnan : x;
+    };
+    const int64_t first = (g.row_offset[l] + (int64_t)row0) * feat + f0;
+    const bool pairs = kind != WALK_FEATURE;
+    if (ws.slots != nullptr) {
+      float* slot = ws.slots + (int64_t)t * (2 * BIN_ROWS);
+      for (uint32_t r = tid; r < nrows; r += WALK_THREADS) {
+        slot[r] = value(r);
+        if (pairs) slot[BIN_ROWS + r] = value(BIN_ROWS + r);
+      }
+    } else if (touched || mode != TABLE_ADD) {
+      auto flush = [&](auto mode_c) {
+        constexpr int MODE = decltype(mode_c)::value;
+#pragma unroll 4
+        for (uint32_t r = tid; r < nrows; r += WALK_THREADS) {
+          if (pairs) {
+            const float x = value(r), y = value(BIN_ROWS + r);
+            add_or_store_pair<MODE>(table, first + (int64_t)r * feat, x, y, feat == 2, has_pair);
+          } else {
+            const int64_t at = first + which + (int64_t)r * feat;
+            const float x = value(r);
+            if constexpr (MODE == TABLE_ADD) {
+              if (x != 0.0f) reinterpret_cast<float*>(table)[at] += x;
+            } else {
+              store_table<MODE>(table, at, x);
+            }
+          }
+        }
+      };
+      with_mode(mode, flush);
+    }
+    lds_barrier();
+    if (tid == 0) level_max = hit = 0u;
   }
 }
 
-// blockIdx.x: a task, numbered like the bins of BinPlan; blockIdx.y: the slice of the points.  Every level here is one or
-// two bins.  A level of one bin is one task whose tile holds both features of the pair; a level of two bins is two
-// tasks, one per feature of the pair, whose tile holds that feature of all the level's rows: either way every corner of a
-// point lands in the tile, so the walk has no test per corner and its LDS adds run with all lanes.
-template <typename GT, int D>
-__global__ __launch_bounds__(DIRECT_THREADS) void hash_bwd_direct_k(const void* coords, int cdt, int64_t csn, int64_t csd,
-                                                                     const uint32_t* pairs, int64_t N, DevGeom g, BinPlan bp,
-                                                                     const int64_t* primes, float scale, const uint32_t* gmax,
-                                                                     float* dtable, int feat, int p, int64_t slice_points) {
-  typedef typename BinRec<GT>::type Rec;
-  constexpr bool G32 = sizeof(Rec) == 16;
-  extern __shared__ unsigned long long acc_tile[];  // 2 * BIN_ROWS sums
-  const int tid = threadIdx.x;
-  int l = 0;
-  while (l + 1 < bp.n_levels && (int)blockIdx.x >= bp.binbase[l + 1]) ++l;
-  const uint32_t which = blockIdx.x - (uint32_t)bp.binbase[l];
-  const bool by_feature = bp.nbins[l] == 2;
-  const int np = (feat + 1) / 2, f0 = 2 * p;
-  const bool has_pair = f0 + 1 < feat;
-  if (by_feature && which == 1u && !has_pair) return;  // an odd feature count: the last pair has one feature
-  const uint32_t nrows = g.rows[l];                    // <= 2 * BIN_ROWS, and <= BIN_ROWS unless by_feature
-  // fixed-point scale 2^se of the level, as in the record kernels:  |w * g| * 2^se < 2^30
-  const float gm = BinRec<GT>::level_max(gmax[l]);
-  const bool nonfinite = !(gm <= 3.0e38f);
-  int se = 0;
-  if (!nonfinite && gm > 0.0f) {
-    int ex;
-    frexpf(gm, &ex);
-    se = 30 - ex;
-    se = se > 120 ? 120 : se;
-  }
-  // |g| * 2^se < 2^30: the scaled gradient is a float (the two steps are exact powers of two inside float range)
-  const float s_lo = nonfinite ? 0.0f : ldexpf(1.0f, se / 2), s_hi = ldexpf(1.0f, se - se / 2);
-  const uint32_t ncells = by_feature ? nrows : 2u * BIN_ROWS;
-  for (uint32_t i = tid; i < ncells; i += DIRECT_THREADS) acc_tile[i] = 0ull;
-  lds_barrier();
-  const bool hashed = l >= g.first_hash;
-  const float fres = (float)g.res[l];
-  const uint32_t res = (uint32_t)g.res[l], mask = g.rows[l] - 1u;
-  const uint32_t pi[3] = {(uint32_t)primes[0], (uint32_t)primes[1], D > 2 ? (uint32_t)primes[D > 2 ? 2 : 0] : 0u};
-  const uint32_t* level_pairs = pairs + (((int64_t)l * np + p) * N) * (G32 ? 2 : 1);
-  const int64_t n_begin = (int64_t)blockIdx.y * slice_points;
-  const int64_t n_end = n_begin + slice_points < N ? n_begin + slice_points : N;
-  // One point per thread and turn: the sixteen waves of the workgroup keep enough loads in flight, and more points per
-  // thread only cost registers (two: +4 %, eight: +70 %).  The loop exists in four copies, by the kind of tile and for
-  // levels with an inf or a nan in their gradient (which only mark the rows they touch), so that it carries no branch.
-  auto walk = [&](auto by_feature_c, auto nonfinite_c) {
-    constexpr bool BY_FEATURE = decltype(by_feature_c)::value, NONFINITE = decltype(nonfinite_c)::value;
-    for (int64_t n = n_begin + tid; n < n_end; n += DIRECT_THREADS) {
-      float v[D > 3 ? D : 3] = {};
-      Rec rec = BinRec<GT>::zero();
-      load_point_d<D>(coords, cdt, csn, csd, n, scale, v);
-      if constexpr (G32) {
-        const uint2 t = reinterpret_cast<const uint2*>(level_pairs)[n];
-        rec.z = t.x;
-        rec.w = t.y;
-      } else {
-        rec.z = level_pairs[n];
-      }
-      uint32_t row[1 << D];
-      float w[1 << D];
-      cell_rows<D>(v, fres, hashed, res, mask, pi, primes, row, w);
-      const float g0 = BinRec<GT>::g0(rec) * s_lo * s_hi, g1 = BinRec<GT>::g1(rec) * s_lo * s_hi;
-      const float gs = which ? g1 : g0;
-#pragma unroll
-      for (int j = 0; j < (1 << D); ++j) {
-        // zero contributions are rare here: the adds carry no test
-        if constexpr (BY_FEATURE) {
-          const int32_t fv = NONFINITE ? (int32_t)(w[j] != 0.0f) : __float2int_rn(w[j] * gs);
-          atomicAdd(acc_tile + row[j], (unsigned long long)(long long)fv);
-        } else {
-          const int32_t f0v = NONFINITE ? (int32_t)(w[j] != 0.0f) : __float2int_rn(w[j] * g0);
-          const int32_t f1v = NONFINITE ? (int32_t)(has_pair && w[j] != 0.0f) : __float2int_rn(w[j] * g1);
-          atomicAdd(acc_tile + row[j], (unsigned long long)(long long)f0v);
-          atomicAdd(acc_tile + (uint32_t)BIN_ROWS + row[j], (unsigned long long)(long long)f1v);
-        }
-      }
+// the slots of every bin, in the order of their slices: a thread takes four rows of a level
+template <int MODE>
+__global__ __launch_bounds__(REDUCE_THREADS) void hash_bwd_walk_reduce_k(WalkWs ws, void* table, DevGeom g, WalkPlan wp, int feat, int f0) {
+  const int l = (int)blockIdx.y;
+  const uint32_t r = (blockIdx.x * REDUCE_THREADS + threadIdx.x) * 4u;
+  if (r >= g.rows[l]) return;
+  const int slices = wp.slices[l];
+  const bool by_feature = wp.bins[l] == 2, has_pair = f0 + 1 < feat;
+  const int64_t task = wp.first[l] + (by_feature ? 0 : (int64_t)(r >> BIN_ROWS_LOG2) * slices);
+  const float* src0 = ws.slots + task * (2 * BIN_ROWS) + (by_feature ? r : r & BIN_MASK);
+  const float* src1 = src0 + (by_feature ? (int64_t)slices * (2 * BIN_ROWS) : (int64_t)BIN_ROWS);
+  float x[4] = {}, y[4] = {};
+#pragma unroll 4
+  for (int s = 0; s < slices; ++s) {
+    const float4 a = *reinterpret_cast<const float4*>(src0 + (int64_t)s * (2 * BIN_ROWS));
+    x[0] += a.x; x[1] += a.y; x[2] += a.z; x[3] += a.w;
+    if (has_pair) {
+      const float4 b = *reinterpret_cast<const float4*>(src1 + (int64_t)s * (2 * BIN_ROWS));
+      y[0] += b.x; y[1] += b.y; y[2] += b.z; y[3] += b.w;
     }
-  };
-  if (by_feature) {
-    if (nonfinite) walk(std::true_type{}, std::true_type{});
-    else walk(std::true_type{}, std::false_type{});
-  } else {
-    if (nonfinite) walk(std::false_type{}, std::true_type{});
-    else walk(std::false_type{}, std::false_type{});
   }
-  lds_barrier();
-  float* dst = dtable + g.row_offset[l] * feat + f0;
-  const float qnan = __uint_as_float(0x7fc00000u);
-  const uint32_t nvals = by_feature ? nrows : 2u * nrows;
-  for (uint32_t i = tid; i < nvals; i += DIRECT_THREADS) {
-    // by feature: value i is row i of feature `which`; else value i is feature i & 1 of row i >> 1
-    const uint32_t r = by_feature ? i : i >> 1, f = by_feature ? which : (i & 1u);
-    if (f && !has_pair) continue;
-    const long long a = (long long)acc_tile[by_feature ? r : f * (uint32_t)BIN_ROWS + r];
-    if (a == 0) continue;
-    // |a| < 2^53 is exact in double and so is the division by 2^se: one rounding, to float
-    const float x = nonfinite ? qnan : (float)ldexp((double)a, -se);
-    if (x != 0.0f) unsafeAtomicAdd(dst + (int64_t)r * feat + f, x);
-  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (r + e < g.rows[l]) add_or_store_pair<MODE>(table, (g.row_offset[l] + r + e) * feat + f0, x[e], y[e], feat == 2, has_pair);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1304,31 +1422,93 @@ static int64_t bin_ws(void* workspace, const BinPlan& bp, int64_t N, int points,
 // and cost 2.5 % of a 2^21-point training step: every piece pays the fixed part of the pipeline again.)
 constexpr int64_t BIN_CHUNK_POINTS = (int64_t)1 << 21;
 
-// The walk without records hashes every point once per task of a level (two for a level of two bins); the records pay a
-// count, a fill and an accumulate pass per level whatever its size.  With every level at most two bins (2^14 rows, the
-// reference's default table size) the walk is the faster one; four bins would already cost it more hashing than the
-// records' passes take.
-constexpr int DIRECT_MAX_BINS_PER_LEVEL = 2;
-constexpr int DIRECT_MAX_DIMS = 4;  // the walk is built for 1 to 4 dimensions (the sorted records for 2 and 3)
-constexpr int64_t DIRECT_MIN_POINTS = 4096;  // below: one launch of scattered atomics is as quick
-static bool direct_ok(int64_t n_points, const nf_hash_geom* geom, int flags) {
-  if ((flags & NF_HASH_BWD_RECORDS) || n_points < DIRECT_MIN_POINTS) return false;
-  if (geom->dims < 1 || geom->dims > DIRECT_MAX_DIMS) return false;
-  for (int l = 0; l < geom->levels; ++l)
-    if (geom->rows[l] > (int64_t)DIRECT_MAX_BINS_PER_LEVEL * BIN_ROWS) return false;
-  return true;
+// The walk without records hashes every point once per bin of a level; the records pay a fill and an accumulate pass per level
+// whatever its size.  So the walk takes tables whose levels are all at most two bins (2^14 rows, the reference's default), where it has no
+// test per corner, and of the others those with a bin or less per unit (a second round of tiles costs what the whole walk does), in
+// batches of few points times bins (three bins a level cost the walk what they cost the records).  16 levels of fp16, uniform points
+// and rays, walk and records: 2^15 rows 262144 points 106, 136 and 221, 238 us; 2^16 rows 131072 points 101, 130 and 121, 141; 2^17 rows
+// 32768 points 62, 95 and 98, 115, 65536 points 112, 172 and 100, 120.  Under WALK_MIN_POINTS the atomics of hash_bwd_level_k are
+// quicker, where they apply: 2^16 rows 4096 points 19 and 31, 8192 points 38 and 35, in every feature pair.
+constexpr int WALK_FREE_BINS = 2, WALK_MAX_BINS = 256;
+constexpr int64_t WALK_MAX_POINT_BINS = (int64_t)13 << 19;
+constexpr int WALK_MAX_DIMS = 4;  // the walk is built for 1 to 4 dimensions (the sorted records for 2 and 3)
+constexpr int64_t WALK_MIN_POINTS = 6144, WALK_MIN_POINTS_FREE = 4096, WALK_MIN_POINTS_GENERIC = 1024;
+static bool walk_ok(int64_t n_points, const nf_hash_geom* geom, int flags) {
+  if (flags & NF_HASH_BWD_RECORDS) return false;
+  if (geom->dims < 1 || geom->dims > WALK_MAX_DIMS) return false;
+  int64_t bins = 0, most = 0;
+  for (int l = 0; l < geom->levels; ++l) {
+    const int64_t nb = (geom->rows[l] + BIN_ROWS - 1) / BIN_ROWS;
+    bins += nb;
+    most = nb > most ? nb : most;
+  }
+  const bool free = most <= WALK_FREE_BINS;
+  if (n_points < (!bwd_level_ok(geom) ? WALK_MIN_POINTS_GENERIC : free ? WALK_MIN_POINTS_FREE : WALK_MIN_POINTS * ((geom->feat + 1) / 2))) return false;
+  return free || (quick_rows(geom) && bins <= WALK_MAX_BINS && n_points * (bins - 3 * geom->levels) <= WALK_MAX_POINT_BINS);
 }
-bool bwd_direct_applies(int64_t n_points, const nf_hash_geom* geom, int flags) {
-  return direct_ok(n_points < BIN_CHUNK_POINTS ? n_points : BIN_CHUNK_POINTS, geom, flags);
+bool bwd_walk_applies(int64_t n_points, const nf_hash_geom* geom, int flags) {
+  return walk_ok(n_points < BIN_CHUNK_POINTS ? n_points : BIN_CHUNK_POINTS, geom, flags);
 }
-// gmax[32] (padded to 256 bytes) | pairs[levels][ceil(feat / 2)][n_points] of 4 (float32 gradient: 8) bytes
-static int64_t direct_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype) {
-  return 256 + (int64_t)geom->levels * ((geom->feat + 1) / 2) * n_points * (dout_dtype == NF_F32 ? 8 : 4);
+
+static int compute_units() {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0;
+    hipDeviceProp_t p;
+    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&p, dev) == hipSuccess) cus = p.multiProcessorCount;
+    if (cus <= 0) cus = 256;
+  }
+  return cus;
+}
+
+// One task at a time fits a unit (the tile is 128 KiB of LDS), so the points are sliced until there is about one task per unit; a
+// task of both features of a level costs one and a half of the others.  Slices of at least two turns of the workgroup.
+static WalkPlan walk_plan(int64_t N, const nf_hash_geom* geom) {
+  WalkPlan wp = {};
+  wp.n_levels = geom->levels;
+  wp.prep_blocks = (int)((N + WALK_PREP_THREADS - 1) / WALK_PREP_THREADS);
+  int64_t total = 0;
+  auto cost = [&](int l) { return wp.bins[l] == 1 ? 3 : 2; };
+  for (int l = 0; l < geom->levels; ++l) {
+    wp.bins[l] = (int)((geom->rows[l] + BIN_ROWS - 1) / BIN_ROWS);
+    total += wp.bins[l] * cost(l);
+  }
+  const int64_t most = N / (2 * WALK_THREADS);
+  for (int l = 0; l < geom->levels; ++l) {
+    int64_t slices = (int64_t)compute_units() * cost(l) / total;
+    slices = slices > most ? most : slices;
+    wp.slices[l] = (int)(slices < 1 ? 1 : slices);
+    wp.first[l + 1] = wp.first[l] + wp.bins[l] * wp.slices[l];
+  }
+  wp.n_tasks = wp.first[wp.n_levels];
+  return wp;
+}
+static bool walk_sliced(const WalkPlan& wp) {
+  for (int l = 0; l < wp.n_levels; ++l)
+    if (wp.slices[l] > 1) return true;
+  return false;
+}
+static int64_t walk_ws(void* workspace, const WalkPlan& wp, int64_t N, int dims, int feat, int dout_dtype, WalkWs* ws) {
+  char* p = (char*)workspace;
+  int64_t o = 0;
+  auto take = [&](int64_t bytes) {
+    char* at = p + o;
+    o += (bytes + 255) / 256 * 256;
+    return at;
+  };
+  ws->block_max = (uint32_t*)take((int64_t)wp.n_levels * ((feat + 1) / 2) * wp.prep_blocks * 4);
+  ws->points = (float*)take((int64_t)dims * N * 4);
+  ws->pairs = (uint32_t*)take((int64_t)wp.n_levels * ((feat + 1) / 2) * N * (dout_dtype == NF_F32 ? 8 : 4));
+  ws->slots = walk_sliced(wp) ? (float*)take((int64_t)wp.n_tasks * 2 * BIN_ROWS * 4) : nullptr;
+  return o;
 }
 
 int64_t bwd_bin_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags) {
   if (n_points > BIN_CHUNK_POINTS) n_points = BIN_CHUNK_POINTS;
-  if (direct_ok(n_points, geom, flags)) return direct_workspace_bytes(n_points, geom, dout_dtype);
+  if (walk_ok(n_points, geom, flags)) {
+    WalkWs ws;
+    return walk_ws(nullptr, walk_plan(n_points, geom), n_points, geom->dims, geom->feat, dout_dtype, &ws);
+  }
   auto bytes = [&](int64_t n, bool wide) -> int64_t {
     BinPlan bp;
     BinWs ws;
@@ -1346,21 +1526,21 @@ static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_
                                 void* table, int mode, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
                                 void* workspace, hipStream_t s);
 
-static int launch_bwd_direct(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
-                             float* dtable, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
-                             void* workspace, hipStream_t s);
+static int launch_bwd_walk(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
+                           void* table, int mode, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
+                           void* workspace, hipStream_t s);
 
 int launch_bwd_bin(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
                    float* dtable, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
                    void* workspace, int flags, hipStream_t s) {
   // the choice is made once, on the size the workspace was asked for: every piece then fits it
-  const bool direct = direct_ok(N < BIN_CHUNK_POINTS ? N : BIN_CHUNK_POINTS, geom, flags);
+  const bool walk = bwd_walk_applies(N, geom, flags);
   for (int64_t n0 = 0; n0 < N; n0 += BIN_CHUNK_POINTS) {
     const int64_t n = N - n0 < BIN_CHUNK_POINTS ? N - n0 : BIN_CHUNK_POINTS;
     const char* c = (const char*)coords + n0 * csn * dtype_size(cdt);
     const char* d = (const char*)dout + n0 * dout_stride * dtype_size(ddt);
-    const int rc = direct ? launch_bwd_direct(c, cdt, csn, csd, d, ddt, dout_stride, dtable, n, geom, g, primes, scale, workspace, s)
-                          : launch_bwd_bin_piece(c, cdt, csn, csd, d, ddt, dout_stride, dtable, TABLE_ADD, n, geom, g, primes, scale, workspace, s);
+    const int rc = walk ? launch_bwd_walk(c, cdt, csn, csd, d, ddt, dout_stride, dtable, TABLE_ADD, n, geom, g, primes, scale, workspace, s)
+                        : launch_bwd_bin_piece(c, cdt, csn, csd, d, ddt, dout_stride, dtable, TABLE_ADD, n, geom, g, primes, scale, workspace, s);
     if (rc) return rc;
   }
   return 0;
@@ -1368,80 +1548,60 @@ int launch_bwd_bin(const void* coords, int cdt, int64_t csn, int64_t csd, const 
 
 bool bwd_write_applies(int64_t n_points, const nf_hash_geom* geom, int flags) {
   // one pass over the points that leaves every row's whole sum in one place
-  return n_points <= BIN_CHUNK_POINTS && (geom->dims == 2 || geom->dims == 3) && !direct_ok(n_points, geom, flags);
+  if (n_points > BIN_CHUNK_POINTS) return false;
+  return walk_ok(n_points, geom, flags) || (n_points >= bwd_records_min(geom, flags) && (geom->dims == 2 || geom->dims == 3));
 }
 
 int launch_bwd_write(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride, void* table,
                      int table_dtype, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
-                     void* workspace, hipStream_t s) {
+                     void* workspace, int flags, hipStream_t s) {
   const int mode = table_dtype == NF_F32 ? TABLE_F32 : table_dtype == NF_F16 ? TABLE_F16 : TABLE_BF16;
-  return launch_bwd_bin_piece(coords, cdt, csn, csd, dout, ddt, dout_stride, table, mode, N, geom, g, primes, scale, workspace, s);
+  return walk_ok(N, geom, flags) ? launch_bwd_walk(coords, cdt, csn, csd, dout, ddt, dout_stride, table, mode, N, geom, g, primes, scale, workspace, s)
+                                 : launch_bwd_bin_piece(coords, cdt, csn, csd, dout, ddt, dout_stride, table, mode, N, geom, g, primes, scale, workspace, s);
 }
 
-static int direct_cus() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0;
-    hipDeviceProp_t p;
-    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&p, dev) == hipSuccess) cus = p.multiProcessorCount;
-    if (cus <= 0) cus = 256;
-  }
-  return cus;
-}
-
-static int launch_bwd_direct(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
-                             float* dtable, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
-                             void* workspace, hipStream_t s) {
-  NF_REQUIRE(((uintptr_t)workspace & 15u) == 0, NF_EALIGN, "workspace must be 16-byte aligned");
-  BinPlan bp = {};
-  bp.n_levels = geom->levels;
-  for (int l = 0; l < geom->levels; ++l) {
-    bp.nbins[l] = (int)((geom->rows[l] + BIN_ROWS - 1) / BIN_ROWS);
-    bp.binbase[l + 1] = bp.binbase[l] + bp.nbins[l];
-  }
-  const int NB = bp.binbase[bp.n_levels];
-  uint32_t* gmax = reinterpret_cast<uint32_t*>(workspace);
-  uint32_t* pairs = gmax + 64;
-  const bool g32 = ddt == NF_F32;
-  hipLaunchKernelGGL(hash_bwd_bin_zero_k, dim3(1), dim3(64), 0, s, gmax, 32);
-  if (int rc = check_launch("hash_bwd_bin_zero")) return rc;
-  const unsigned prep_blocks = (unsigned)((N + DIRECT_PREP_THREADS - 1) / DIRECT_PREP_THREADS);
-  if (g32)
-    hipLaunchKernelGGL(hash_bwd_direct_prep_k<true>, dim3(prep_blocks), dim3(DIRECT_PREP_THREADS), 0, s, dout, dout_stride, N,
-                       g.levels, g.feat, pairs, gmax);
-  else
-    hipLaunchKernelGGL(hash_bwd_direct_prep_k<false>, dim3(prep_blocks), dim3(DIRECT_PREP_THREADS), 0, s, dout, dout_stride, N,
-                       g.levels, g.feat, pairs, gmax);
-  if (int rc = check_launch("hash_bwd_direct_prep")) return rc;
-  // at most two workgroups per compute unit in all, so that they run as two full rounds (one fits at a time: the tile is
-  // 128 KiB of LDS; four rounds: +3 %, eight: +11 %), in slices of whole turns of the point loop and of at least 4096 points
-  const int64_t round = (int64_t)DIRECT_THREADS;
-  int64_t slices = (int64_t)2 * direct_cus() / NB;
-  if (slices < 1) slices = 1;
-  int64_t slice_points = (N + slices - 1) / slices;
-  if (slice_points < 4096) slice_points = 4096;
-  slice_points = (slice_points + round - 1) / round * round;
-  slices = (N + slice_points - 1) / slice_points;
-  const size_t lds = (size_t)2 * BIN_ROWS * sizeof(unsigned long long);
-  auto pick = [&](auto d_c) -> const void* {
-    constexpr int DD = decltype(d_c)::value;
-    return ddt == NF_F32 ? (const void*)hash_bwd_direct_k<F32, DD> : ddt == NF_BF16 ? (const void*)hash_bwd_direct_k<BF16, DD> : (const void*)hash_bwd_direct_k<F16, DD>;
-  };
-  const void* kern = g.dims == 3   ? pick(std::integral_constant<int, 3>{})
-                     : g.dims == 2 ? pick(std::integral_constant<int, 2>{})
-                     : g.dims == 1 ? pick(std::integral_constant<int, 1>{})
-                                   : pick(std::integral_constant<int, 4>{});
-  hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+static int launch_large(const char* what, const void* kern, dim3 grid, int threads, void** args, size_t lds, hipStream_t s) {
+  hipError_t e = hipSuccess;
+  if (lds > 64 * 1024) e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return fail((int)e, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-  const uint32_t* cpairs = pairs;
-  const uint32_t* cgmax = gmax;
-  const int feat = geom->feat;
+  e = hipLaunchKernel(kern, grid, dim3((unsigned)threads), args, lds, s);
+  if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(%s): %s", what, hipGetErrorString(e));
+  return check_launch(what);
+}
+
+static int launch_bwd_walk(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
+                           void* table, int mode, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
+                           void* workspace, hipStream_t s) {
+  NF_REQUIRE(((uintptr_t)workspace & 15u) == 0, NF_EALIGN, "workspace must be 16-byte aligned");
+  WalkPlan wp = walk_plan(N, geom);
+  WalkWs ws;
+  walk_ws(workspace, wp, N, geom->dims, geom->feat, ddt, &ws);
+  int levels = geom->levels, feat = geom->feat;
+  const void *prep, *walk;
+  auto pick = [&](auto d_c) {
+    constexpr int DD = decltype(d_c)::value;
+    prep = ddt == NF_F32 ? (const void*)hash_bwd_walk_prep_k<true, DD> : (const void*)hash_bwd_walk_prep_k<false, DD>;
+    walk = ddt == NF_F32 ? (const void*)hash_bwd_walk_k<F32, DD> : ddt == NF_BF16 ? (const void*)hash_bwd_walk_k<BF16, DD> : (const void*)hash_bwd_walk_k<F16, DD>;
+  };
+  if (g.dims == 3) pick(std::integral_constant<int, 3>{});
+  else if (g.dims == 2) pick(std::integral_constant<int, 2>{});
+  else if (g.dims == 1) pick(std::integral_constant<int, 1>{});
+  else pick(std::integral_constant<int, 4>{});
+  void* prep_args[] = {(void*)&coords, (void*)&cdt, (void*)&csn, (void*)&csd, (void*)&scale, (void*)&dout, (void*)&dout_stride, (void*)&N, (void*)&levels, (void*)&feat, (void*)&ws};
+  if (int rc = launch_large("hash_bwd_walk_prep", prep, dim3((unsigned)wp.prep_blocks), WALK_PREP_THREADS, prep_args, (size_t)levels * ((feat + 1) / 2) * 4, s)) return rc;
+  const void* reduce = with_mode(mode, [](auto mode_c) { return (const void*)hash_bwd_walk_reduce_k<decltype(mode_c)::value>; });
+  const unsigned units = (unsigned)compute_units(), groups = (unsigned)wp.n_tasks < units ? (unsigned)wp.n_tasks : units;
+  int64_t most_rows = 0;
+  for (int l = 0; l < levels; ++l) most_rows = geom->rows[l] > most_rows ? geom->rows[l] : most_rows;
+  DevGeom gg = g;
   for (int p = 0; p < (feat + 1) / 2; ++p) {
-    void* args[] = {(void*)&coords, (void*)&cdt, (void*)&csn, (void*)&csd, (void*)&cpairs, (void*)&N, (void*)&g, (void*)&bp,
-                    (void*)&primes, (void*)&scale, (void*)&cgmax, (void*)&dtable, (void*)&feat, (void*)&p, (void*)&slice_points};
-    e = hipLaunchKernel(kern, dim3((unsigned)NB, (unsigned)slices), dim3(DIRECT_THREADS), args, lds, s);
-    if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(hash_bwd_direct): %s", hipGetErrorString(e));
-    if (int rc = check_launch("hash_bwd_direct")) return rc;
+    int f0 = 2 * p;
+    void* args[] = {(void*)&ws, (void*)&N, (void*)&gg, (void*)&wp, (void*)&primes, (void*)&table, (void*)&mode, (void*)&feat, (void*)&p};
+    if (int rc = launch_large("hash_bwd_walk", walk, dim3(groups), WALK_THREADS, args, (size_t)2 * BIN_ROWS * 8, s)) return rc;
+    if (ws.slots == nullptr) continue;
+    void* reduce_args[] = {(void*)&ws, (void*)&table, (void*)&gg, (void*)&wp, (void*)&feat, (void*)&f0};
+    const dim3 grid((unsigned)((most_rows + REDUCE_THREADS * 4 - 1) / (REDUCE_THREADS * 4)), (unsigned)levels);
+    if (int rc = launch_large("hash_bwd_walk_reduce", reduce, grid, REDUCE_THREADS, reduce_args, 0, s)) return rc;
   }
   return 0;
 }
@@ -1465,10 +1625,6 @@ static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_
     bin_pieces += (bp.nbins[l] + 63) / 64;
   }
   const int feat = geom->feat, D = g.dims == 2 ? 2 : 3;
-  auto large_lds = [](const void* kern, size_t lds) -> int {
-    const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    return e == hipSuccess ? 0 : fail((int)e, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-  };
   auto pick_fill = [&](auto wide_c, auto g32_c) -> const void* {
     constexpr bool W = decltype(wide_c)::value, G = decltype(g32_c)::value;
     return g.dims == 6   ? (const void*)hash_bwd_bin_fill_k<W, G, 3, 3>
@@ -1477,30 +1633,17 @@ static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_
            : g.dims == 3 ? (const void*)hash_bwd_bin_fill_k<W, G, 3>
                          : (const void*)hash_bwd_bin_fill_k<W, G, 2>;
   };
-  auto pick_accum = [&](auto mode_c) -> const void* {
-    constexpr int M = decltype(mode_c)::value;
-    return ddt == NF_F16 ? (const void*)hash_bwd_bin_accum_k<F16, M> : ddt == NF_BF16 ? (const void*)hash_bwd_bin_accum_k<BF16, M> : (const void*)hash_bwd_bin_accum_k<F32, M>;
-  };
   const void* fill = wide ? (g32 ? pick_fill(std::true_type{}, std::true_type{}) : pick_fill(std::true_type{}, std::false_type{}))
                           : (g32 ? pick_fill(std::false_type{}, std::true_type{}) : pick_fill(std::false_type{}, std::false_type{}));
-  const void* accum = mode == TABLE_ADD   ? pick_accum(std::integral_constant<int, TABLE_ADD>{})
-                      : mode == TABLE_F32 ? pick_accum(std::integral_constant<int, TABLE_F32>{})
-                      : mode == TABLE_F16 ? pick_accum(std::integral_constant<int, TABLE_F16>{})
-                                          : pick_accum(std::integral_constant<int, TABLE_BF16>{});
-  const void* reduce = mode == TABLE_ADD   ? (const void*)hash_bwd_bin_reduce_k<TABLE_ADD>
-                       : mode == TABLE_F32 ? (const void*)hash_bwd_bin_reduce_k<TABLE_F32>
-                       : mode == TABLE_F16 ? (const void*)hash_bwd_bin_reduce_k<TABLE_F16>
-                                           : (const void*)hash_bwd_bin_reduce_k<TABLE_BF16>;
+  const void* accum = with_mode(mode, [&](auto mode_c) -> const void* {
+    constexpr int M = decltype(mode_c)::value;
+    return ddt == NF_F16 ? (const void*)hash_bwd_bin_accum_k<F16, M> : ddt == NF_BF16 ? (const void*)hash_bwd_bin_accum_k<BF16, M> : (const void*)hash_bwd_bin_accum_k<F32, M>;
+  });
+  const void* reduce = with_mode(mode, [](auto mode_c) { return (const void*)hash_bwd_bin_reduce_k<decltype(mode_c)::value>; });
   const size_t fill_lds = ((size_t)stage_records(D, wide) * (g32 ? 4 : 3) + 3 * (size_t)max_nb + 1 + NF_MAX_LEVELS) * 4;
   const size_t acc_lds = (size_t)BIN_ROWS * 2 * sizeof(unsigned long long) + ((size_t)LIST + LIST_PAD + (NB < SPLIT_MAX_BINS ? NB : SPLIT_MAX_BINS) + 1) * 4;
-  if (int rc = large_lds(fill, fill_lds)) return rc;
-  if (int rc = large_lds(accum, acc_lds)) return rc;
-  auto launch = [&](const char* what, const void* kern, dim3 grid, int threads, void** args, size_t lds) -> int {
-    const hipError_t e = hipLaunchKernel(kern, grid, dim3((unsigned)threads), args, lds, s);
-    if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(%s): %s", what, hipGetErrorString(e));
-    return check_launch(what);
-  };
-  const unsigned units = (unsigned)direct_cus();
+  auto launch = [&](const char* what, const void* kern, dim3 grid, int threads, void** args, size_t lds) { return launch_large(what, kern, grid, threads, args, lds, s); };
+  const unsigned units = (unsigned)compute_units();
   // more than three dimensions: the whole pipeline once per corner of the extra coordinates (`hi`), see ExtraDims
   const int passes = g.dims > 3 ? 1 << (g.dims - 3) : 1;
   for (int hi = 0; hi < passes; ++hi)

@@ -252,6 +252,14 @@ int nf_revmlp_bwd(const void* y, int64_t y_stride, const void* dy, int64_t dy_st
                   float* dw1, float* db1, float* dw2, float* db2, int64_t rows, int half, int blocks, int act,
                   int dtype, void* stream);
 
+/* The same with the weight gradients written instead of added, in grad_dtype (`dtype` or NF_F32), summed over the workgroups in a fixed
+ * order: the same inputs give the same bits on every run.  rows > 0; workspace: 16-byte aligned, nf_revmlp_bwd_workspace_bytes() bytes. */
+int nf_revmlp_bwd_summed(const void* y, int64_t y_stride, const void* dy, int64_t dy_stride, void* dx, int64_t dx_stride,
+                         void* x_rec, int64_t x_rec_stride, const void* w1, const void* b1, const void* w2, const void* b2,
+                         void* dw1, void* db1, void* dw2, void* db2, int64_t rows, int half, int blocks, int act,
+                         int dtype, int grad_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+int64_t nf_revmlp_bwd_workspace_bytes(int64_t rows, int half, int blocks);
+
 #ifdef __cplusplus
 }
 #endif

@@ -206,3 +206,37 @@ def _check_table_gradient(N, dims, F, T, L, hi, dtype, layout, same_bits):
     ulp = {torch.float16: 2**-10, torch.bfloat16: 2**-7, torch.float32: 1e-5}[dtype]
     torch.testing.assert_close(grads[0].double(), want, rtol=ulp, atol=atol)
     assert not grads[0][count == 0].any()
+
+
+@pytest.mark.parametrize("rows,H,blocks,act,dtype", [
+    (1, 64, 4, "gelu", torch.bfloat16), (31, 32, 1, "silu", torch.float16), (32, 64, 5, "relu", torch.bfloat16), (128 * 3, 48, 2, "gelu", torch.float16),
+    (4096 + 17, 64, 2, "gelu", torch.bfloat16), (256 * 128 + 32, 64, 1, "silu", torch.float16), (3 * 12 * 256 * 32, 32, 4, "gelu", torch.bfloat16),
+])
+def test_reversible_gradients_of_few_and_many_workgroups(rows, H, blocks, act, dtype):
+    """The weights' gradients are summed over one slot per workgroup, the last rows' launch included: against float32 autograd of
+    the plain composition, and the same bits in a second run."""
+    from triton_helpers_amd.layers.reversible_mlp import reversible_mlp
+
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    u = lambda *s: (torch.rand(*s, generator=g, device=DEV) * 2 - 1).mul(H**-0.5).to(dtype)  # noqa: E731
+    w = [u(blocks * 2 * H, H), u(blocks * 2, H), u(blocks * 2 * H, H), u(blocks * 2, H)]
+    x, dy = torch.randn(rows, 2 * H, generator=g, device=DEV).to(dtype), torch.randn(rows, 2 * H, generator=g, device=DEV).to(dtype)
+    got = []
+    for _ in range(2):
+        leaves = [t.clone().requires_grad_() for t in (x, *w)]
+        y = reversible_mlp(*leaves, activation=act)
+        y.backward(dy)
+        got.append([y.detach(), *_grads(leaves)])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    f = {"gelu": torch.nn.functional.gelu, "silu": torch.nn.functional.silu, "relu": torch.relu}[act]
+    leaves = [t.float().requires_grad_() for t in (x, *w)]
+    a, b = leaves[0][:, :H], leaves[0][:, H:]
+    for k in range(2 * blocks):
+        w1, b1, w2, b2 = (t[k * (t.shape[0] // (2 * blocks)) : (k + 1) * (t.shape[0] // (2 * blocks))] for t in leaves[1:])
+        s = f((b if k % 2 == 0 else a) @ w1.t() + b1) @ w2.t() + b2
+        a, b = (a + s, b) if k % 2 == 0 else (a, b + s)
+    ref = torch.cat([a, b], 1)
+    ref.backward(dy.float())
+    for p, q in zip(got[0], [ref.detach(), *_grads(leaves)]):
+        # (a ReLU takes its gates from rebuilt inputs: some open or close)
+        assert float((p.float() - q).norm()) <= (6e-2 if act == "relu" else 2e-2) * float(q.norm())

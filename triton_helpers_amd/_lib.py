@@ -52,6 +52,8 @@ EXPORTS = (
     "nf_cast_pieces_f16",
     "nf_revmlp_fwd",
     "nf_revmlp_bwd",
+    "nf_revmlp_bwd_summed",
+    "nf_revmlp_bwd_workspace_bytes",
 )
 
 
@@ -128,6 +130,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.nf_revmlp_fwd.argtypes = [P, I64, P, I64, P, P, P, P, I64, I, I, I, I, P]
     lib.nf_revmlp_bwd.restype = c_int
     lib.nf_revmlp_bwd.argtypes = [P, I64, P, I64, P, I64, P, I64, P, P, P, P, P, P, P, P, I64, I, I, I, I, P]
+    lib.nf_revmlp_bwd_summed.restype = c_int
+    lib.nf_revmlp_bwd_summed.argtypes = [P, I64, P, I64, P, I64, P, I64, P, P, P, P, P, P, P, P, I64, I, I, I, I, I, P, I64, P]
+    lib.nf_revmlp_bwd_workspace_bytes.restype = I64
+    lib.nf_revmlp_bwd_workspace_bytes.argtypes = [I64, I, I]
 
 
 def load() -> ctypes.CDLL:

@@ -369,13 +369,18 @@ variable_list reversible_backward(const Tensor& y, Tensor dy, std::array<Tensor,
   const int64_t width = y.size(-1), H = width / 2;
   const Rows ry(y, width), rd(dy, width);
   const Tensor dx = at::empty(y.sizes(), y.options()), x_rec = at::empty(y.sizes(), y.options());
-  const Pieces at(w, 4);
-  const Tensor flat = at::zeros({at.total}, y.options().dtype(at::kFloat));
-  check(nf_revmlp_bwd(ry.p, ry.stride, rd.p, rd.stride, dx.data_ptr(), width, x_rec.data_ptr(), width, ptr(w[0]), ptr(w[1]), ptr(w[2]), ptr(w[3]),
-                      (float*)at.at(flat, w[0], 0), (float*)at.at(flat, w[1], 1), (float*)at.at(flat, w[2], 2), (float*)at.at(flat, w[3], 3), ry.n,
-                      (int)H, (int)(w[0].size(0) / (2 * H)), act, code_of(y.scalar_type()), stream_of(y)),
-        "nf_revmlp_bwd");
-  const Tensor f = float_grads ? flat : flat.to(y.scalar_type());
+  const Pieces at(w, 8);
+  const int dt = code_of(y.scalar_type()), blocks = (int)(w[0].size(0) / (2 * H));
+  const auto options = float_grads ? y.options().dtype(at::kFloat) : y.options();
+  const Tensor f = ry.n > 0 ? at::empty({at.total}, options) : at::zeros({at.total}, options);
+  if (ry.n > 0) {
+    const int64_t bytes = nf_revmlp_bwd_workspace_bytes(ry.n, (int)H, blocks);
+    const Tensor ws = scratch(bytes, y);
+    check(nf_revmlp_bwd_summed(ry.p, ry.stride, rd.p, rd.stride, dx.data_ptr(), width, x_rec.data_ptr(), width, ptr(w[0]), ptr(w[1]), ptr(w[2]), ptr(w[3]),
+                               at.at(f, w[0], 0), at.at(f, w[1], 1), at.at(f, w[2], 2), at.at(f, w[3], 3), ry.n, (int)H, blocks, act, dt,
+                               float_grads ? NF_F32 : dt, ptr(ws), bytes, stream_of(y)),
+          "nf_revmlp_bwd_summed");
+  }
   return {dx, at.view(f, w[0], 0), at.view(f, w[1], 1), at.view(f, w[2], 2), at.view(f, w[3], 3)};
 }
 

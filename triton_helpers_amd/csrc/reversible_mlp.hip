@@ -15,6 +15,9 @@
 // in mlp_tile.h), which lets a lane reach the eight features of two accumulator tiles with one
 // 16-byte access; the staged weights and the flushed gradients absorb the permutation.
 //
+// Backward of four 64-wide GELU couplings (us; before: sixteen rounds of weight loads and 65536 float atomics per workgroup and coupling):
+// 1600 rows 97 -> 90, 32768 157 -> 108, 100000 220 -> 196, 2^20 unchanged (1.14 ms: the serial issue of one wave per SIMD).
+//
 // There is no counterpart in the reference; the layer math is that of its fused MLP
 // (triton_helpers/layers/fully_fused_mlp/kernel.py:17-74).
 #include "mlp_tile.h"
@@ -33,8 +36,10 @@ struct RevArgs {
   int64_t dy_stride;
   uint16_t* dx;
   int64_t dx_stride;
-  const uint16_t *w1, *b1, *w2, *b2;  // first coupling of this launch
-  float *dw1, *db1, *dw2, *db2;       // first coupling of this launch (backward)
+  const uint16_t *w1, *b1, *w2, *b2;  // forward: first coupling of this launch
+  const char* packed;                 // backward: the LDS images of the weights, first coupling of this launch
+  float* slots;                       // backward: [workgroup][blocks] sums of the weight gradients, first coupling of this launch
+  int64_t slot_stride;                // floats between the slots of two workgroups
   int64_t rows;
   int half, nblocks, act;
   int vec_in, vec_out, vec_dy, vec_dx;
@@ -177,18 +182,42 @@ __global__ __launch_bounds__(768) void rev_fwd_k(RevArgs a) {
   uint16_t* frags = reinterpret_cast<uint16_t*>(smem);  // [nblocks][F.w1, F.w2, G.w1, G.w2][LAYER]
   float* bias = reinterpret_cast<float*>(frags + (size_t)a.nblocks * 4 * LAYER);  // [nblocks][4][HP]
   const int H = FAST ? HP : a.half;
+  if constexpr (FAST) {
+    // All layers as one list of 8-element pieces, several in flight per thread: layer by layer, sixteen rounds of loads waited for one
+    // another (1600 rows of four couplings: 32 us, now 21).
+    constexpr int PIECES = MT * KC * 64, AT_ONCE = 4;
+    const int all = a.nblocks * 4 * PIECES;
+    for (int u0 = tid; u0 < all; u0 += AT_ONCE * nthreads) {
+      uint2 lo[AT_ONCE], hi[AT_ONCE];
+#pragma unroll
+      for (int i = 0; i < AT_ONCE; ++i) {
+        const int u = u0 + i * nthreads < all ? u0 + i * nthreads : u0;
+        const int layer = u / PIECES, piece = u % PIECES, mt = (piece >> 6) / KC, kc = (piece >> 6) % KC, g = (piece & 63) >> 4;
+        const uint16_t* w = (layer & 1 ? a.w2 : a.w1) + (size_t)(layer >> 1) * HP * HP + (16 * mt + (piece & 15)) * HP;
+        lo[i] = *reinterpret_cast<const uint2*>(w + k_chain(kc, g, 0));
+        hi[i] = *reinterpret_cast<const uint2*>(w + k_chain(kc, g, 4));
+      }
+#pragma unroll
+      for (int i = 0; i < AT_ONCE; ++i)
+        if (u0 + i * nthreads < all) *reinterpret_cast<uint4*>(frags + (size_t)(u0 + i * nthreads) * 8) = make_uint4(lo[i].x, lo[i].y, hi[i].x, hi[i].y);
+    }
+  }
   for (int k = 0; k < a.nblocks; ++k)
     for (int s = 0; s < 2; ++s) {
       const size_t sub = (size_t)(2 * k + s);
-      stage_weight_frags<true, false>(frags + ((size_t)k * 4 + 2 * s) * LAYER, a.w1 + sub * H * H, H, H, MT, KC, tid, nthreads);
-      stage_weight_frags<true, false>(frags + ((size_t)k * 4 + 2 * s + 1) * LAYER, a.w2 + sub * H * H, H, H, MT, KC, tid, nthreads);
+      if constexpr (!FAST) {
+        stage_weight_frags<true, false>(frags + ((size_t)k * 4 + 2 * s) * LAYER, a.w1 + sub * H * H, H, H, MT, KC, tid, nthreads);
+        stage_weight_frags<true, false>(frags + ((size_t)k * 4 + 2 * s + 1) * LAYER, a.w2 + sub * H * H, H, H, MT, KC, tid, nthreads);
+      }
       stage_bias_row<T>(bias + ((size_t)k * 4 + 2 * s) * HP, a.b1 ? a.b1 + sub * H : nullptr, H, HP, tid, nthreads);
       stage_bias_row<T>(bias + ((size_t)k * 4 + 2 * s + 1) * HP, a.b2 ? a.b2 + sub * H : nullptr, H, HP, tid, nthreads);
     }
   __syncthreads();
 
   const int64_t n_chunks = (a.rows + 31) / 32;
-  for (int64_t chunk = (int64_t)blockIdx.x * nwaves + wave; chunk < n_chunks; chunk += (int64_t)gridDim.x * nwaves) {
+  // Chunks to workgroups in turn, then to their waves: every unit has as many (262144 rows of four couplings, a workgroup's waves side by
+  // side: 87 us, so 76), and few chunks spread over the units, where a wave has a SIMD to itself.
+  for (int64_t chunk = (int64_t)wave * gridDim.x + blockIdx.x; chunk < n_chunks; chunk += (int64_t)gridDim.x * nwaves) {
     const int64_t row0 = chunk * 32;
     f32x4_t s1[2][4], s2[2][4];  // the two halves of the residual stream, float32
 #pragma unroll
@@ -366,25 +395,113 @@ __device__ __forceinline__ void sub_backward(const uint2 (&u)[2][4], const uint2
   rev_layer<T, MT, KC>(du, dzf, tw1, nullptr, lane);
 }
 
-// Bias gradient of feature 16*mt + n: the four lane groups hold partial sums over disjoint rows.
-// WIDE: the tile's features are in wide order (wide_feature())
-template <bool WIDE = false>
-__device__ __forceinline__ void flush_db_rev(float* db, int dim, int mt, int lane, float v) {
-  v += __shfl_xor(v, 16);
-  v += __shfl_xor(v, 32);
-  const int f = WIDE ? wide_feature(mt, lane & 15) : 16 * mt + lane;
-  if (db != nullptr && lane < 16 && f < dim) unsafeAtomicAdd(db + f, v);
+// What the backward keeps of a coupling in LDS, as one piece of memory: the weights as fragments, [F.w1, F.w2, G.w1, G.w2] in forward form and
+// the same transposed, then the biases in that order.  rev_pack_k lays it out once per call; a workgroup then copies it straight from
+// memory to LDS, all of it in flight at once and through no register.
+template <int HP>
+struct RevImage {
+  static constexpr int MT = HP / 16, KC = HP / 32, LAYER = MT * KC * RFRAG;
+  static constexpr int BYTES = ((8 * LAYER * 2 + 4 * HP * 4) + 1023) / 1024 * 1024;  // whole copies of a wave
+};
+constexpr int PACK_THREADS = 256;
+template <typename T, int HP>
+__global__ __launch_bounds__(PACK_THREADS) void rev_pack_k(const uint16_t* w1, const uint16_t* b1, const uint16_t* w2, const uint16_t* b2, int H, char* packed) {
+  typedef RevImage<HP> I;
+  constexpr bool WIDE = true;
+  // a workgroup per coupling and sub-MLP, and form of one of its layers
+  const int k = blockIdx.x >> 1, s = blockIdx.x & 1, tid = threadIdx.x;
+  const size_t sub = blockIdx.x;
+  uint16_t* fw = reinterpret_cast<uint16_t*>(packed + (size_t)k * I::BYTES);
+  uint16_t* tw = fw + 4 * I::LAYER;
+  float* bias = reinterpret_cast<float*>(tw + 4 * I::LAYER);
+  w1 += sub * H * H;
+  w2 += sub * H * H;
+  // the stream's features are contracted in natural order and produced in wide order (the hidden ones as ever)
+  switch (blockIdx.y) {
+    case 0:
+      stage_weight_frags<!WIDE, false, PACK_THREADS>(fw + (2 * s) * I::LAYER, w1, H, H, I::MT, I::KC, tid, PACK_THREADS);
+      stage_bias_row<T>(bias + (2 * s) * HP, b1 ? b1 + sub * H : nullptr, H, HP, tid, PACK_THREADS);
+      break;
+    case 1:
+      stage_weight_frags<true, false, PACK_THREADS, WIDE>(fw + (2 * s + 1) * I::LAYER, w2, H, H, I::MT, I::KC, tid, PACK_THREADS);
+      stage_bias_row<T, WIDE>(bias + (2 * s + 1) * HP, b2 ? b2 + sub * H : nullptr, H, HP, tid, PACK_THREADS);
+      break;
+    case 2: stage_weight_frags<true, true, PACK_THREADS, WIDE>(tw + (2 * s) * I::LAYER, w1, H, H, I::MT, I::KC, tid, PACK_THREADS); break;
+    default: stage_weight_frags<!WIDE, true, PACK_THREADS>(tw + (2 * s + 1) * I::LAYER, w2, H, H, I::MT, I::KC, tid, PACK_THREADS); break;
+  }
 }
 
-// WIDE_ROWS / WIDE_COLS: the tile's rows (mt) / columns (nt) are features in wide order
-template <bool WIDE_ROWS = false, bool WIDE_COLS = false>
-__device__ __forceinline__ void flush_tile(float* dw, int dim, int mt, int nt, int lane, f32x4_t v) {
-  const int c = WIDE_COLS ? wide_feature(nt, lane & 15) : 16 * nt + (lane & 15);
-  const int r0 = WIDE_ROWS ? wide_feature(mt, 4 * (lane >> 4)) : 16 * mt + 4 * (lane >> 4);
-  if (c >= dim) return;
+// A workgroup's sums of a coupling's weight gradients: accumulator tiles [MT][MT][F.w1, F.w2, G.w1, G.w2] of 64 lanes x 4, then bias
+// gradients [MT][F.b1, F.b2, G.b1, G.b2] of 16.
+template <int HP>
+struct RevSlot {
+  static constexpr int MT = HP / 16, TILES = MT * MT * 4, FLOATS = TILES * 256 + 4 * HP;
+};
+// Bias gradient of feature 16*mt + n: the four lane groups hold partial sums over disjoint rows.
+__device__ __forceinline__ void put_db(float* slot, int lane, float v) {
+  v += __shfl_xor(v, 16);
+  v += __shfl_xor(v, 32);
+  if (lane < 16) slot[lane] = v;
+}
+
+// The slots of all workgroups in a fixed order, to where the gradients belong: 64 pieces of four values per workgroup, sixteen
+// interleaved runs over the slots, then a fixed tree.
+struct RevGrads {
+  void *dw1, *db1, *dw2, *db2;
+  int half, n_slots, add, type;  // add: to what is there (float32)
+};
+template <int HP>
+__global__ __launch_bounds__(1024) void rev_sum_k(const float* slots, int64_t slot_stride, RevGrads o) {
+  typedef RevSlot<HP> S;
+  __shared__ f32x4_t part[16][64];
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6, H = o.half;
+  const int coupling = blockIdx.y, piece = blockIdx.x * 64 + tx;
+  const bool on = piece * 4 < S::FLOATS;
+  const float* src = slots + (int64_t)coupling * S::FLOATS + piece * 4;
+  f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (on) {
+    int sl = ty;
+    for (; sl + 48 < o.n_slots; sl += 64) {
+      f32x4_t v[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    if (r0 + r < dim) unsafeAtomicAdd(dw + (size_t)(r0 + r) * dim + c, v[r]);
+      for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const f32x4_t*>(src + (int64_t)(sl + 16 * k) * slot_stride);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) sum += v[k];
+    }
+    for (; sl < o.n_slots; sl += 16) sum += *reinterpret_cast<const f32x4_t*>(src + (int64_t)sl * slot_stride);
+  }
+  part[ty][tx] = sum;
+  __syncthreads();
+  if (ty != 0 || !on) return;
+  f32x4_t total = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int q = 0; q < 16; q += 4) total += (part[q][tx] + part[q + 1][tx]) + (part[q + 2][tx] + part[q + 3][tx]);
+  auto put = [&](void* base, int64_t at, float v) {
+    if (o.add) reinterpret_cast<float*>(base)[at] += v;
+    else if (o.type == NF_F32) reinterpret_cast<float*>(base)[at] = v;
+    else if (o.type == NF_F16) reinterpret_cast<uint16_t*>(base)[at] = F16::from_f32(v);
+    else reinterpret_cast<uint16_t*>(base)[at] = BF16::from_f32(v);
+  };
+  if (piece < S::TILES * 64) {
+    const int lane = piece & 63, tile = piece >> 6, m = tile & 3, mt = (tile >> 2) / S::MT, nt = (tile >> 2) % S::MT;
+    // first layers have their columns in wide order, second layers their rows
+    const int c = m & 1 ? 16 * nt + (lane & 15) : wide_feature(nt, lane & 15);
+    const int r0 = m & 1 ? wide_feature(mt, 4 * (lane >> 4)) : 16 * mt + 4 * (lane >> 4);
+    void* base = m & 1 ? o.dw2 : o.dw1;
+    if (c >= H) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (r0 + r < H) put(base, ((int64_t)(2 * coupling + (m >> 1)) * H + r0 + r) * H + c, total[r]);
+  } else {
+    const int at = piece * 4 - S::TILES * 256, m = (at >> 4) & 3, mt = at >> 6;
+    void* base = m & 1 ? o.db2 : o.db1;
+    if (base == nullptr) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int n = (at & 15) + r, f = m & 1 ? wide_feature(mt, n) : 16 * mt + n;
+      if (f < H) put(base, (int64_t)(2 * coupling + (m >> 1)) * H + f, total[r]);
+    }
+  }
 }
 
 template <typename T, int HP, int ACT, bool FAST>
@@ -411,8 +528,7 @@ __global__ __launch_bounds__(256) void rev_bwd_block_k(RevArgs a) {
   const int64_t n_chunks = (a.rows + 31) / 32;
 
   // The couplings of the launch, last first.  A wave owns the same rows in every coupling, so it reads (x, dx) of the
-  // coupling above from where it wrote them itself and no workgroup ever waits for another; the weight-gradient
-  // atomics of one coupling drain while the next is being computed.
+  // coupling above from where it wrote them itself and no workgroup ever waits for another.
   // (Only the variant without per-tile checks loops; the general one is launched once per coupling.)
   for (int kb = FAST ? a.nblocks - 1 : 0; kb >= 0; --kb) {
   const bool top = FAST ? kb == a.nblocks - 1 : true;
@@ -422,20 +538,13 @@ __global__ __launch_bounds__(256) void rev_bwd_block_k(RevArgs a) {
   const uint16_t* dy_p = top ? a.dy : a.dx;
   const int64_t dy_s = top ? a.dy_stride : a.dx_stride;
   const bool dy_v = top ? a.vec_dy : a.vec_dx;
-  const uint16_t* w1 = a.w1 + (size_t)2 * kb * H * H;
-  const uint16_t* w2 = a.w2 + (size_t)2 * kb * H * H;
-  const uint16_t* b1 = a.b1 ? a.b1 + (size_t)2 * kb * H : nullptr;
-  const uint16_t* b2 = a.b2 ? a.b2 + (size_t)2 * kb * H : nullptr;
   if (G2_LDS)
     for (int i = lane; i < MT * MT * 64; i += 64) g2acc[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int s = 0; s < 2; ++s) {
-    // WIDE: the stream's features are contracted in natural order and produced in wide order (the hidden ones as ever)
-    stage_weight_frags<!WIDE, false>(fw + (2 * s) * LAYER, w1 + (size_t)s * H * H, H, H, MT, KC, tid, nthreads);
-    stage_weight_frags<true, false, 0, WIDE>(fw + (2 * s + 1) * LAYER, w2 + (size_t)s * H * H, H, H, MT, KC, tid, nthreads);
-    stage_weight_frags<true, true, 0, WIDE>(tw + (2 * s) * LAYER, w1 + (size_t)s * H * H, H, H, MT, KC, tid, nthreads);
-    stage_weight_frags<!WIDE, true>(tw + (2 * s + 1) * LAYER, w2 + (size_t)s * H * H, H, H, MT, KC, tid, nthreads);
-    stage_bias_row<T>(bias + (2 * s) * HP, b1 ? b1 + (size_t)s * H : nullptr, H, HP, tid, nthreads);
-    stage_bias_row<T, WIDE>(bias + (2 * s + 1) * HP, b2 ? b2 + (size_t)s * H : nullptr, H, HP, tid, nthreads);
+  {
+    const char* image = a.packed + (size_t)kb * RevImage<HP>::BYTES + 16 * lane;
+    for (int i = __builtin_amdgcn_readfirstlane(wave) * 1024; i < RevImage<HP>::BYTES; i += 4096)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(image + i), (__attribute__((address_space(3))) void*)(smem + i), 16, 0, 0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
   __syncthreads();
 
@@ -553,8 +662,8 @@ __global__ __launch_bounds__(256) void rev_bwd_block_k(RevArgs a) {
     }
   }
 
-  // ---- weight gradients: summed over the four waves through LDS (the weight fragments are dead by now), then one
-  // pass of 64-byte coalesced atomics per workgroup ----
+  // ---- weight gradients: summed over the four waves through LDS (the weight fragments are dead by now), then to the
+  // workgroup's slot ----
   __syncthreads();
   constexpr int NREG = G2_LDS ? 3 : 4;  // accumulators that live in registers
   f32x4_t* red = reinterpret_cast<f32x4_t*>(smem) + lane;
@@ -598,31 +707,30 @@ __global__ __launch_bounds__(256) void rev_bwd_block_k(RevArgs a) {
     __syncthreads();
   }
   if (wave == 0) {
-  // layer order in dw1 / dw2: sub-MLP F is row block 0, G is row block 1 of this coupling block
-  float* gw1 = a.dw1 + (size_t)2 * kb * H * H;
-  float* gw2 = a.dw2 + (size_t)2 * kb * H * H;
-  float* gb1 = a.db1 ? a.db1 + (size_t)2 * kb * H : nullptr;
-  float* gb2 = a.db2 ? a.db2 + (size_t)2 * kb * H : nullptr;
+  float* slot = a.slots + blockIdx.x * a.slot_stride + (size_t)kb * RevSlot<HP>::FLOATS;
+  f32x4_t* tiles = reinterpret_cast<f32x4_t*>(slot) + lane;
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
-      flush_tile<false, WIDE>(gw1, H, i, j, lane, dwF1[i][j]);
-      flush_tile<WIDE, false>(gw2, H, i, j, lane, dwF2[i][j]);
-      flush_tile<false, WIDE>(gw1 + (size_t)H * H, H, i, j, lane, dwG1[i][j]);
+      const int t = (i * MT + j) * 4 * 64;
+      tiles[t] = dwF1[i][j];
+      tiles[t + 64] = dwF2[i][j];
+      tiles[t + 128] = dwG1[i][j];
       if (G2_LDS) {
         constexpr int PER_WAVE = MT * MT * 64;
         const int at = (i * MT + j) * 64 + lane;  // wave 0's g2acc is the first of the four
         dwG2[i][j] = (g2acc[at] + g2acc[PER_WAVE + at]) + (g2acc[2 * PER_WAVE + at] + g2acc[3 * PER_WAVE + at]);
       }
-      flush_tile<WIDE, false>(gw2 + (size_t)H * H, H, i, j, lane, dwG2[i][j]);
+      tiles[t + 192] = dwG2[i][j];
     }
+  float* dbs = slot + RevSlot<HP>::TILES * 256;
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
-    flush_db_rev(gb1, H, i, lane, dbF1[i]);
-    flush_db_rev(gb1 ? gb1 + H : nullptr, H, i, lane, dbG1[i]);
-    flush_db_rev<WIDE>(gb2, H, i, lane, dbF2[i]);
-    flush_db_rev<WIDE>(gb2 ? gb2 + H : nullptr, H, i, lane, dbG2[i]);
+    put_db(dbs + 64 * i, lane, dbF1[i]);
+    put_db(dbs + 64 * i + 16, lane, dbF2[i]);
+    put_db(dbs + 64 * i + 32, lane, dbG1[i]);
+    put_db(dbs + 64 * i + 48, lane, dbG2[i]);
   }
   }
   // wave 0 has read the other waves' LDS accumulators and the reduction area: both are rewritten for the next coupling
@@ -668,11 +776,12 @@ static int launch_rev_fwd(RevArgs a, hipStream_t s) {
   const int64_t chunks = (a.rows + 31) / 32;
   // weights of several blocks leave room for one workgroup per CU only: give it 12 waves to keep three per SIMD
   const int waves = lds > 80 * 1024 ? 12 : 4;
-  int64_t blocks = (chunks + waves - 1) / waves;
   const int64_t cap = (int64_t)rev_cus() * (lds > 80 * 1024 ? 1 : 2);
+  int64_t blocks = (chunks + waves - 1) / waves;
   if (blocks > cap) blocks = cap;
+  if (blocks < rev_cus()) blocks = chunks < rev_cus() ? chunks : rev_cus();
   // full-width, aligned, unragged calls of GELU, ReLU and SiLU take the variants without per-tile checks
-  const bool fast = a.half == HP && a.rows % 32 == 0 && a.vec_in && a.vec_out;
+  const bool fast = a.half == HP && a.rows % 32 == 0 && a.vec_in && a.vec_out && (uintptr_t)a.w1 % 8 == 0 && (uintptr_t)a.w2 % 8 == 0;
   const void* kern = a.act == NF_ACT_GELU   ? (fast ? (const void*)rev_fwd_k<T, HP, NF_ACT_GELU, true>
                                                     : (const void*)rev_fwd_k<T, HP, NF_ACT_GELU, false>)
                      : a.act == NF_ACT_RELU ? (fast ? (const void*)rev_fwd_k<T, HP, NF_ACT_RELU, true>
@@ -689,18 +798,19 @@ static int launch_rev_fwd(RevArgs a, hipStream_t s) {
   return check_launch("rev_fwd");
 }
 
+// workgroups of the backward: the weight-gradient accumulators take most of the register file, one wave per SIMD
+static int rev_bwd_groups(int64_t rows) {
+  const int64_t groups = ((rows + 31) / 32 + 3) / 4;
+  return (int)(groups < rev_cus() ? groups : rev_cus());
+}
+
 template <typename T, int HP>
 static int launch_rev_bwd(RevArgs a, hipStream_t s) {
-  constexpr int LAYER = (HP / 16) * (HP / 32) * RFRAG;
-  size_t lds = (size_t)8 * LAYER * 2 + (size_t)4 * HP * 4 + (HP > 32 ? (size_t)4 * (HP / 16) * (HP / 16) * 64 * 16 : 0);
+  typedef RevImage<HP> I;
+  size_t lds = I::BYTES + (HP > 32 ? (size_t)4 * I::MT * I::MT * 64 * 16 : 0);
   // the closing reduction over the waves reuses the front of LDS: the register accumulators and 4 bias sums per tile row
-  const size_t red = (size_t)(HP > 32 ? 3 : 4) * (HP / 16) * (HP / 16) * 64 * 16 + (size_t)4 * (HP / 16) * 64 * 4;
+  const size_t red = (size_t)(HP > 32 ? 3 : 4) * I::MT * I::MT * 64 * 16 + (size_t)4 * I::MT * 64 * 4;
   if (HP <= 32 && lds < red) lds = red;
-  const int64_t chunks = (a.rows + 31) / 32;
-  int64_t blocks = (chunks + 3) / 4;
-  // the weight-gradient accumulators take most of the register file: one wave per SIMD
-  const int64_t cap = (int64_t)rev_cus();
-  if (blocks > cap) blocks = cap;
   const bool fast = a.half == HP && a.rows % 32 == 0 && a.vec_in && a.vec_out && a.vec_dy && a.vec_dx && a.wide_ok;
   const void* kern = a.act == NF_ACT_GELU   ? (fast ? (const void*)rev_bwd_block_k<T, HP, NF_ACT_GELU, true>
                                                     : (const void*)rev_bwd_block_k<T, HP, NF_ACT_GELU, false>)
@@ -713,9 +823,70 @@ static int launch_rev_bwd(RevArgs a, hipStream_t s) {
     if (e != hipSuccess) return fail((int)e, "hipFuncSetAttribute: %s", hipGetErrorString(e));
   }
   void* args[] = {(void*)&a};
-  const hipError_t e = hipLaunchKernel(kern, dim3((unsigned)blocks), dim3(256), args, lds, s);
+  const hipError_t e = hipLaunchKernel(kern, dim3((unsigned)rev_bwd_groups(a.rows)), dim3(256), args, lds, s);
   if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(rev_bwd_block): %s", hipGetErrorString(e));
   return check_launch("rev_bwd_block");
+}
+
+// Rows are independent: a large batch with a ragged end runs as its multiple of 32 rows (the variants without per-tile checks, where the rest of
+// the call allows them) plus a launch for the last rows.
+static int64_t main_rows(int64_t rows) { return rows >= SPLIT_MIN_ROWS ? rows - rows % 32 : rows; }
+static int rev_bwd_slots(int64_t rows) { return rev_bwd_groups(main_rows(rows)) + (main_rows(rows) < rows ? 1 : 0); }
+
+template <typename T, int HP>
+static int rev_bwd(const char* y, int64_t y_stride, const char* dy, int64_t dy_stride, char* dx, int64_t dx_stride, char* x_rec, int64_t x_rec_stride,
+                   const void* w1, const void* b1, const void* w2, const void* b2, RevGrads grads, int64_t rows, int half, int blocks, int act,
+                   void* workspace, hipStream_t s) {
+  typedef RevImage<HP> I;
+  typedef RevSlot<HP> S;
+  char* packed = (char*)workspace;
+  float* slots = (float*)(packed + (size_t)blocks * I::BYTES);
+  const int64_t slot_stride = (int64_t)blocks * S::FLOATS;
+  hipLaunchKernelGGL((rev_pack_k<T, HP>), dim3((unsigned)(2 * blocks), 4), dim3(PACK_THREADS), 0, s, (const uint16_t*)w1, (const uint16_t*)b1, (const uint16_t*)w2,
+                     (const uint16_t*)b2, half, packed);
+  if (int rc = check_launch("rev_pack")) return rc;
+  int64_t slot = 0;
+  for (int64_t r0 = 0; r0 < rows;) {
+    const int64_t n = r0 == 0 ? main_rows(rows) : rows - r0;
+    const char *yp = y + r0 * y_stride * 2, *dyp = dy + r0 * dy_stride * 2;
+    char *dxp = dx + r0 * dx_stride * 2, *xp = x_rec + r0 * x_rec_stride * 2;
+    // Full-width, aligned, unragged calls of GELU, ReLU and SiLU take one launch that walks all couplings, last
+    // first (the first reads (y, dy), the others continue in place on (x_rec, dx)); anything else one launch per coupling.
+    const bool fused = half == HP && n % 32 == 0 && (act == NF_ACT_GELU || act == NF_ACT_RELU || act == NF_ACT_SILU) && vec16_ok(yp, y_stride) &&
+                       vec16_ok(xp, x_rec_stride) && vec16_ok(dyp, dy_stride) && vec16_ok(dxp, dx_stride);
+    for (int k = blocks - 1; k >= 0; --k) {
+      RevArgs a = {};
+      const bool first = k == blocks - 1;
+      const int kw = fused ? 0 : k;  // the fused launch offsets per coupling itself
+      a.in = (const uint16_t*)(first ? yp : xp);
+      a.in_stride = first ? y_stride : x_rec_stride;
+      a.out = (uint16_t*)xp;
+      a.out_stride = x_rec_stride;
+      a.dy = (const uint16_t*)(first ? dyp : dxp);
+      a.dy_stride = first ? dy_stride : dx_stride;
+      a.dx = (uint16_t*)dxp;
+      a.dx_stride = dx_stride;
+      a.packed = packed + (size_t)kw * I::BYTES;
+      a.slots = slots + slot * slot_stride + (int64_t)kw * S::FLOATS;
+      a.slot_stride = slot_stride;
+      a.rows = n;
+      a.half = half;
+      a.nblocks = fused ? blocks : 1;
+      a.act = act;
+      a.vec_in = vec8_ok(a.in, a.in_stride, half);
+      a.vec_out = vec8_ok(a.out, a.out_stride, half);
+      a.vec_dy = vec8_ok(a.dy, a.dy_stride, half);
+      a.vec_dx = vec8_ok(a.dx, a.dx_stride, half);
+      a.wide_ok = fused;  // the unchecked kernel is the fused launch's
+      if (int rc = launch_rev_bwd<T, HP>(a, s)) return rc;
+      if (fused) break;
+    }
+    slot += rev_bwd_groups(n);
+    r0 += n;
+  }
+  grads.n_slots = (int)slot;
+  hipLaunchKernelGGL((rev_sum_k<HP>), dim3((S::FLOATS / 4 + 63) / 64, (unsigned)blocks), dim3(1024), 0, s, slots, slot_stride, grads);
+  return check_launch("rev_sum");
 }
 
 }  // namespace nf
@@ -767,6 +938,40 @@ extern "C" int nf_revmlp_fwd(const void* x, int64_t x_stride, void* y, int64_t y
   return 0;
 }
 
+extern "C" int64_t nf_revmlp_bwd_workspace_bytes(int64_t rows, int half, int blocks) {
+  if (rows <= 0 || half < 1 || half > 64 || blocks < 1) return 0;
+  const int64_t image = half <= 32 ? RevImage<32>::BYTES : RevImage<64>::BYTES, slot = half <= 32 ? RevSlot<32>::FLOATS : RevSlot<64>::FLOATS;
+  return blocks * (image + (int64_t)rev_bwd_slots(rows) * slot * 4);
+}
+
+static int rev_bwd_call(const void* y, int64_t y_stride, const void* dy, int64_t dy_stride, void* dx, int64_t dx_stride, void* x_rec,
+                        int64_t x_rec_stride, const void* w1, const void* b1, const void* w2, const void* b2, const RevGrads& grads, int64_t rows,
+                        int half, int blocks, int act, int dtype, void* workspace, hipStream_t s) {
+  auto run = [&](auto t, auto hp) {
+    return rev_bwd<decltype(t), decltype(hp)::value>((const char*)y, y_stride, (const char*)dy, dy_stride, (char*)dx, dx_stride, (char*)x_rec, x_rec_stride,
+                                                     w1, b1, w2, b2, grads, rows, half, blocks, act, workspace, s);
+  };
+  if (half <= 32) return dtype == NF_BF16 ? run(BF16{}, std::integral_constant<int, 32>{}) : run(F16{}, std::integral_constant<int, 32>{});
+  return dtype == NF_BF16 ? run(BF16{}, std::integral_constant<int, 64>{}) : run(F16{}, std::integral_constant<int, 64>{});
+}
+
+extern "C" int nf_revmlp_bwd_summed(const void* y, int64_t y_stride, const void* dy, int64_t dy_stride, void* dx, int64_t dx_stride, void* x_rec,
+                                    int64_t x_rec_stride, const void* w1, const void* b1, const void* w2, const void* b2, void* dw1, void* db1,
+                                    void* dw2, void* db2, int64_t rows, int half, int blocks, int act, int dtype, int grad_dtype,
+                                    void* workspace, int64_t workspace_bytes, void* stream) {
+  if (int rc = rev_validate(rows, half, blocks, act, dtype)) return rc;
+  NF_REQUIRE(grad_dtype == dtype || grad_dtype == NF_F32, NF_EINVAL, "gradients come back in the storage dtype or in float32");
+  NF_REQUIRE(rows > 0, NF_EINVAL, "no rows: the gradients would be left unwritten");
+  NF_REQUIRE(y && dy && dx && x_rec && w1 && w2 && dw1 && dw2 && workspace, NF_EINVAL,
+             "NULL pointer argument (x_rec is required: it carries the reconstructed input between blocks)");
+  NF_REQUIRE(y_stride >= 2 * half && dy_stride >= 2 * half && dx_stride >= 2 * half && x_rec_stride >= 2 * half, NF_EINVAL,
+             "row stride smaller than 2*half");
+  const int64_t need = nf_revmlp_bwd_workspace_bytes(rows, half, blocks);
+  NF_REQUIRE(workspace_bytes >= need && (uintptr_t)workspace % 16 == 0, NF_EINVAL, "a 16-byte aligned workspace of %lld bytes is needed", (long long)need);
+  const RevGrads grads = {dw1, db1, dw2, db2, half, 0, 0, grad_dtype};
+  return rev_bwd_call(y, y_stride, dy, dy_stride, dx, dx_stride, x_rec, x_rec_stride, w1, b1, w2, b2, grads, rows, half, blocks, act, dtype, workspace, (hipStream_t)stream);
+}
+
 extern "C" int nf_revmlp_bwd(const void* y, int64_t y_stride, const void* dy, int64_t dy_stride, void* dx, int64_t dx_stride,
                              void* x_rec, int64_t x_rec_stride, const void* w1, const void* b1, const void* w2,
                              const void* b2, float* dw1, float* db1, float* dw2, float* db2, int64_t rows, int half,
@@ -777,58 +982,15 @@ extern "C" int nf_revmlp_bwd(const void* y, int64_t y_stride, const void* dy, in
              "NULL pointer argument (x_rec is required: it carries the reconstructed input between blocks)");
   NF_REQUIRE(y_stride >= 2 * half && dy_stride >= 2 * half && dx_stride >= 2 * half && x_rec_stride >= 2 * half, NF_EINVAL,
              "row stride smaller than 2*half");
-  // a ragged end as a call of its own (see nf_revmlp_fwd): both calls add into the same weight-gradient accumulators
-  if (rows >= SPLIT_MIN_ROWS && rows % 32 != 0) {
-    const int64_t m = rows - rows % 32;
-    if (int rc = nf_revmlp_bwd(y, y_stride, dy, dy_stride, dx, dx_stride, x_rec, x_rec_stride, w1, b1, w2, b2, dw1, db1, dw2, db2, m, half,
-                               blocks, act, dtype, stream))
-      return rc;
-    return nf_revmlp_bwd((const uint16_t*)y + m * y_stride, y_stride, (const uint16_t*)dy + m * dy_stride, dy_stride,
-                         (uint16_t*)dx + m * dx_stride, dx_stride, (uint16_t*)x_rec + m * x_rec_stride, x_rec_stride, w1, b1, w2, b2, dw1, db1,
-                         dw2, db2, rows - m, half, blocks, act, dtype, stream);
-  }
+  // the workspace from the stream's own pool: given back in stream order
   hipStream_t s = (hipStream_t)stream;
-  // Full-width, aligned, unragged calls of GELU, ReLU and SiLU take one launch that walks all couplings, last
-  // first (the first reads (y, dy), the others continue in place on (x_rec, dx)); anything else one launch per coupling.
-  const int hp = half <= 32 ? 32 : 64;
-  const bool fused = half == hp && rows % 32 == 0 && (act == NF_ACT_GELU || act == NF_ACT_RELU || act == NF_ACT_SILU) && vec8_ok(y, y_stride, half) &&
-                     vec8_ok(x_rec, x_rec_stride, half) && vec8_ok(dy, dy_stride, half) && vec8_ok(dx, dx_stride, half) &&
-                     vec16_ok(y, y_stride) && vec16_ok(x_rec, x_rec_stride) && vec16_ok(dy, dy_stride) && vec16_ok(dx, dx_stride);
-  for (int k = blocks - 1; k >= 0; --k) {
-    RevArgs a = {};
-    const bool first = k == blocks - 1;
-    const int kw = fused ? 0 : k;  // the fused launch offsets per coupling itself
-    a.in = (const uint16_t*)(first ? y : x_rec);
-    a.in_stride = first ? y_stride : x_rec_stride;
-    a.out = (uint16_t*)x_rec;
-    a.out_stride = x_rec_stride;
-    a.dy = (const uint16_t*)(first ? dy : dx);
-    a.dy_stride = first ? dy_stride : dx_stride;
-    a.dx = (uint16_t*)dx;
-    a.dx_stride = dx_stride;
-    a.w1 = (const uint16_t*)w1 + (size_t)2 * kw * half * half;
-    a.w2 = (const uint16_t*)w2 + (size_t)2 * kw * half * half;
-    a.b1 = b1 ? (const uint16_t*)b1 + (size_t)2 * kw * half : nullptr;
-    a.b2 = b2 ? (const uint16_t*)b2 + (size_t)2 * kw * half : nullptr;
-    a.dw1 = dw1 + (size_t)2 * kw * half * half;
-    a.dw2 = dw2 + (size_t)2 * kw * half * half;
-    a.db1 = db1 ? db1 + (size_t)2 * kw * half : nullptr;
-    a.db2 = db2 ? db2 + (size_t)2 * kw * half : nullptr;
-    a.rows = rows;
-    a.half = half;
-    a.nblocks = fused ? blocks : 1;
-    a.act = act;
-    a.vec_in = vec8_ok(a.in, a.in_stride, half);
-    a.vec_out = vec8_ok(a.out, a.out_stride, half);
-    a.vec_dy = vec8_ok(a.dy, a.dy_stride, half);
-    a.vec_dx = vec8_ok(a.dx, a.dx_stride, half);
-    a.wide_ok = fused;  // the unchecked kernel is the fused launch's
-    int rc;
-    if (half <= 32)
-      rc = dtype == NF_BF16 ? launch_rev_bwd<BF16, 32>(a, s) : launch_rev_bwd<F16, 32>(a, s);
-    else
-      rc = dtype == NF_BF16 ? launch_rev_bwd<BF16, 64>(a, s) : launch_rev_bwd<F16, 64>(a, s);
-    if (rc || fused) return rc;
-  }
-  return 0;
+  void* workspace = nullptr;
+  hipError_t e = hipMallocAsync(&workspace, (size_t)nf_revmlp_bwd_workspace_bytes(rows, half, blocks), s);
+  if (e != hipSuccess) return fail((int)e, "hipMallocAsync: %s", hipGetErrorString(e));
+  const RevGrads grads = {dw1, db1, dw2, db2, half, 0, 1, NF_F32};
+  const int rc = rev_bwd_call(y, y_stride, dy, dy_stride, dx, dx_stride, x_rec, x_rec_stride, w1, b1, w2, b2, grads, rows, half, blocks, act, dtype,
+                              workspace, s);
+  e = hipFreeAsync(workspace, s);
+  if (rc != 0) return rc;
+  return e == hipSuccess ? 0 : fail((int)e, "hipFreeAsync: %s", hipGetErrorString(e));
 }

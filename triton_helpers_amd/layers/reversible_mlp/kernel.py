@@ -105,13 +105,17 @@ def reversible_mlp_inverse(y: Tensor, w1: Tensor, b1: Optional[Tensor], w2: Tens
     zeros = torch.zeros_like(y2)
     dx = torch.empty_like(y2)
     x_rec = y.new_empty(y.shape)
-    dw1 = torch.zeros(w1.shape, dtype=torch.float32, device=y.device)
-    dw2 = torch.zeros_like(dw1)
+    if y2.shape[0] == 0:
+        return x_rec.float() if wide else x_rec
+    dw1, dw2 = torch.empty_like(w1), torch.empty_like(w2)
     lib = _lib.load()
-    rc = lib.nf_revmlp_bwd(
+    need = lib.nf_revmlp_bwd_workspace_bytes(y2.shape[0], H, blocks)
+    workspace = torch.empty(need, dtype=torch.uint8, device=y.device)
+    dt = _lib.dtype_code(y.dtype)
+    rc = lib.nf_revmlp_bwd_summed(
         y2.data_ptr(), y2.stride(0), zeros.data_ptr(), zeros.stride(0), dx.data_ptr(), 2 * H, x_rec.data_ptr(), 2 * H,
         w1.data_ptr(), _lib.ptr(b1), w2.data_ptr(), _lib.ptr(b2), dw1.data_ptr(), None, dw2.data_ptr(), None,
-        y2.shape[0], H, blocks, _lib.NF_ACT[activation], _lib.dtype_code(y.dtype), _lib.current_stream(y.device),
+        y2.shape[0], H, blocks, _lib.NF_ACT[activation], dt, dt, workspace.data_ptr(), need, _lib.current_stream(y.device),
     )
-    _lib.check(rc, "nf_revmlp_bwd")
+    _lib.check(rc, "nf_revmlp_bwd_summed")
     return x_rec.float() if wide else x_rec

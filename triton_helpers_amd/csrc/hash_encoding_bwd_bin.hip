@@ -977,7 +977,7 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
       const float x = (float)((double)(int)(a >> 32) * unscale_hi + (double)(uint32_t)a * unscale);
       return nonfinite && a != 0 ? qnan : x;
     };
-    constexpr int U = 8;  // rows of a thread that are under way together
+    constexpr int U = MODE == TABLE_ADD ? 4 : 8;  // rows of a thread that are under way together
     for (uint32_t r0 = tid; r0 < nrows; r0 += ACC_THREADS * U) {
       float x[U], y[U];
       float2 old[MODE == TABLE_ADD ? U : 1];

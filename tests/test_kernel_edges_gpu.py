@@ -240,3 +240,34 @@ def test_reversible_gradients_of_few_and_many_workgroups(rows, H, blocks, act, d
     for p, q in zip(got[0], [ref.detach(), *_grads(leaves)]):
         # (a ReLU takes its gates from rebuilt inputs: some open or close)
         assert float((p.float() - q).norm()) <= (6e-2 if act == "relu" else 2e-2) * float(q.norm())
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17, 2048 * 16 + 5])
+@pytest.mark.parametrize("d_in,H,d_out,hidden,act,bias", [
+    (3, 64, 1, 0, "relu", True), (32, 64, 16, 1, "silu", True), (33, 64, 16, 1, "relu2", False), (32, 32, 17, 1, "none", True), (64, 64, 64, 1, "relu", True),
+    (35, 16, 16, 0, "silu", False), (16, 64, 64, 0, "relu2", True), (64, 32, 33, 0, "relu", True),
+])
+def test_float32_mlp_gradients(rows, d_in, H, d_out, hidden, act, bias):
+    """One and two hidden layers of float32 run backward in one launch: against float64 autograd, with the same bits in a second run."""
+    from triton_helpers_amd.layers.fully_fused_mlp import fully_fused_mlp
+    from triton_helpers_amd.layers.fully_fused_mlp.kernel import _activate
+
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    u = lambda *s: torch.rand(*s, generator=g, device=DEV) * 2 - 1  # noqa: E731
+    w = [u(H, d_in), u(H) if bias else None, u(d_out, H), u(d_out) if bias else None, u(H, H) if hidden else None, u(1, H) if hidden and bias else None]
+    x, dy = u(1, rows, d_in), u(1, rows, d_out)
+    runs = []
+    for _ in range(2):
+        leaves = [None if t is None else t.clone().requires_grad_() for t in (x, *w)]
+        fully_fused_mlp(*leaves, activation=act).backward(dy)
+        runs.append(_grads(leaves))
+    assert all(a is None or torch.equal(a, b) for a, b in zip(*runs))
+    leaves = [None if t is None else t.double().requires_grad_() for t in (x, *w)]
+    lin = lambda h, m, b: h @ m.t() + (0 if b is None else b)  # noqa: E731
+    h = _activate(lin(leaves[0], leaves[1], leaves[2]), act)
+    if hidden:
+        h = _activate(lin(h, leaves[5], None if leaves[6] is None else leaves[6][0]), act)
+    lin(h, leaves[3], leaves[4]).backward(dy.double())
+    for a, b in zip(runs[0], _grads(leaves)):
+        if b is not None:
+            assert float((a.double() - b).norm()) <= 1e-5 * float(b.norm())

@@ -1,18 +1,20 @@
 // Fused MLP on float32 tensors with float32 products: v_mfma_f32_16x16x4_f32, float32 storage, operands and
 // accumulation, so values keep the float32 range and 24-bit mantissa.  (The reference multiplies float32 tensors in
 // TF32, fully_fused_mlp/kernel.py:17-47: the same range with a 10-bit mantissa.)  The 16-bit kernels are the fast
-// path; this one is bound by the float32 matrix rate (157 TFLOP/s) and by its activations' round trip in the backward.
+// path; this one is bound by the float32 matrix rate (157 TFLOP/s) and, beyond two hidden layers, by its activations'
+// round trip in the backward.
 //
 // Forward: one launch for any depth.  A wave carries 32 rows (two groups of 16) through all layers in registers.
 // The product is formed transposed, out^T = W * h^T, so that the 16x16 result tile of a layer (lane (r, g), register v:
 // feature 16*mt + 4*g + v of row r) is already the K operand of the next layer when K is walked in the order
 // 16*t + 4*g + v; the weights are read from LDS in that order (one ds_read_b128 per four products).  Weights of all
 // layers stay in LDS when they fit (up to eight layers), else each layer is staged in turn.
-// Backward: the forward is replayed keeping every hidden layer's pre-activation in the caller's workspace
-// ([depth][rows][d_hidden] float32), then one launch per layer, last to first, forms dW += dz^T h, db += sum dz and
-// overwrites the pre-activation of the layer in front with its gradient.  A workgroup sums its waves' dW in LDS and
-// stores one partial; a small second kernel adds the partials into the caller's accumulators (at most 32 adds per
-// address: thousands of waves adding into the same 16 KB of dW directly cost more than the products).
+// Backward of one or two hidden layers: one launch, see mlp32_bwd_k.  Of more: the forward is replayed keeping every hidden
+// layer's pre-activation in the caller's workspace ([depth][rows][d_hidden] float32), then one launch per layer, last to
+// first, forms dW += dz^T h, db += sum dz and overwrites the pre-activation of the layer in front with its gradient.  A
+// workgroup sums its waves' dW in LDS and stores one partial; a small second kernel adds the partials into the caller's
+// accumulators (at most 32 adds per address: thousands of waves adding into the same 16 KB of dW directly cost more than
+// the products).
 #include "fused_mlp.h"
 
 namespace nf {
@@ -69,11 +71,34 @@ __device__ __forceinline__ void store_chain(float* base, int64_t stride, int64_t
     if (col + i < width) p[i] = v[i];
 }
 
-__device__ __forceinline__ void stage_layer32(float* dst, const float* w, const float* b, int n_out, int n_in, int tid) {
-  for (int i = tid; i < 64 * 64; i += 256) {
-    const int o = i >> 6, c = i & 63;
-    dst[o * W32_STRIDE + c] = (o < n_out && c < n_in) ? w[(size_t)o * n_in + c] : 0.0f;
+// put(o, c, v): a padded 64 x 64 weight matrix, four values of a row at a time.  The loads leave together: one after the other they
+// cost a layer 4 us, a third of a launch on 10^5 rows.
+template <int THREADS = 256, typename Put>
+__device__ __forceinline__ void read_layer32(const float* w, int n_out, int n_in, int tid, Put&& put) {
+  constexpr int PER = 1024 / THREADS, ROWS = THREADS / 16;
+  f32x4_t v[PER];
+  const bool vec = n_in % 4 == 0 && (uintptr_t)w % 16 == 0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int o = (tid >> 4) + ROWS * k, c = 4 * (tid & 15);
+    v[k] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    if (o < n_out) {
+      const float* row = w + (size_t)o * n_in;
+      if (vec) {
+        if (c < n_in) v[k] = *reinterpret_cast<const f32x4_t*>(row + c);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c + e < n_in) v[k][e] = row[c + e];
+      }
+    }
   }
+#pragma unroll
+  for (int k = 0; k < PER; ++k) put((tid >> 4) + ROWS * k, 4 * (tid & 15), v[k]);
+}
+
+__device__ __forceinline__ void stage_layer32(float* dst, const float* w, const float* b, int n_out, int n_in, int tid) {
+  read_layer32(w, n_out, n_in, tid, [&](int o, int c, f32x4_t v) { *reinterpret_cast<f32x4_t*>(dst + o * W32_STRIDE + c) = v; });
   if (tid < 64) dst[64 * W32_STRIDE + tid] = (b != nullptr && tid < n_out) ? b[tid] : 0.0f;
 }
 
@@ -180,10 +205,10 @@ __global__ __launch_bounds__(256) void lin32_bwd_k(Lin32BwdArgs a) {
   const int r = lane & 15, g = lane >> 4;
   float* pdz = lds32 + 64 * W32_STRIDE + wave * (2 * 16 * T32_STRIDE);  // this wave's dz rows
   float* ph = pdz + 16 * T32_STRIDE;                                    // this wave's act(src) rows
-  for (int i = tid; i < 64 * 64; i += 256) {
-    const int o = i >> 6, c = i & 63;
-    wt[c * W32_STRIDE + o] = (o < a.n_out && c < a.n_in) ? a.w[(size_t)o * a.n_in + c] : 0.0f;
-  }
+  read_layer32(a.w, a.n_out, a.n_in, tid, [&](int o, int c, f32x4_t v) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wt[(c + e) * W32_STRIDE + o] = v[e];
+  });
   __syncthreads();
   const int mt_n = (a.n_out + 15) / 16, kt = (a.n_in + 15) / 16;
   const bool dz_vec = ((uintptr_t)a.dz % 16 == 0) && (a.dz_stride % 4 == 0);
@@ -312,14 +337,294 @@ __global__ __launch_bounds__(256) void reduce32_k(const float* part, int n_slots
   }
 }
 
+// ---------------------------------------------------------------------------------------
+// Backward of one or two hidden layers in one launch
+// ---------------------------------------------------------------------------------------
+// A wave takes sixteen rows through the hidden layers and back with everything in registers; the weights stay in LDS, as they are for the
+// way forth and transposed for the way back, and nothing but x, dy and dx passes through memory (layer by layer with the
+// pre-activations in memory, 100003 rows of 32-64-64-16: 160 us, so 63).  A product's operand with the rows along K comes from a panel
+// of the wave's own in LDS.  TI, TO: 16-column tiles of the input and the output; the hidden layers have four, narrower ones zeros.
+constexpr int fused32_tiles(int TI, int TO, int DEPTH) { return TO * 4 + (DEPTH - 1) * 16 + 4 * TI; }
+constexpr int fused32_waves(int TI, int TO, int DEPTH) { return fused32_tiles(TI, TO, DEPTH) <= 28 ? 8 : 4; }  // more gradients take the registers of two waves
+constexpr int fused32_sums(int TI, int TO, int DEPTH) { return fused32_tiles(TI, TO, DEPTH) * 256 + 3 * 64; }
+constexpr int FUSED32_MAX_SUMS = fused32_sums(4, 4, 2);
+constexpr int fused32_stride(int tiles) { return 16 * tiles + 4; }  // floats per staged row of so many tiles
+constexpr size_t fused32_lds(int TI, int TO, int DEPTH) {
+  const int weights = 64 * fused32_stride(TI) + 16 * TI * W32_STRIDE + (DEPTH - 1) * 2 * 64 * W32_STRIDE + 64 * fused32_stride(TO) + 128;
+  const int all = weights + fused32_waves(TI, TO, DEPTH) * 2 * 16 * T32_STRIDE, sums = fused32_sums(TI, TO, DEPTH);
+  return (size_t)(all > sums ? all : sums) * sizeof(float);
+}
+
+struct Fused32Args {
+  const float *x, *dy;
+  float* dx;
+  int64_t x_stride, dy_stride, dx_stride, rows;
+  const float *w_in, *b_in, *w_hid, *b_hid, *w_out;
+  float* slots;  // [workgroup][fused32_sums()]
+  int d_in, d_hidden, d_out, act;
+};
+
+// acc += W h, W's rows of S floats in LDS; the products into one tile are `MT` instructions apart
+template <int KT, int MT, int S>
+__device__ __forceinline__ void product32(f32x4_t (&acc)[4], const float* w, const f32x4_t (&h)[4], int r, int g) {
+#pragma unroll
+  for (int t = 0; t < KT; ++t) {
+    f32x4_t w4[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) w4[mt] = *reinterpret_cast<const f32x4_t*>(w + (16 * mt + r) * S + 16 * t + 4 * g);
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma4(w4[mt][v], h[t][v], acc[mt]);
+  }
+}
+
+template <int TI, int TO, int DEPTH>
+__global__ __launch_bounds__(64 * fused32_waves(TI, TO, DEPTH)) void mlp32_bwd_k(Fused32Args a) {
+  constexpr int WAVES = fused32_waves(TI, TO, DEPTH), THREADS = 64 * WAVES, SI = fused32_stride(TI), SH = W32_STRIDE, SO = fused32_stride(TO);
+  constexpr bool DEEP = DEPTH == 2;
+  extern __shared__ __align__(16) float lds32[];
+  float* w1 = lds32;               // [hidden][in]
+  float* w1t = w1 + 64 * SI;       // [in][hidden]
+  float* wot = w1t + 16 * TI * SH;  // [hidden][out]
+  float* w2 = wot + 64 * SO;       // [hidden][hidden]
+  float* w2t = w2 + (DEEP ? 64 * SH : 0);
+  float* bias = w2t + (DEEP ? 64 * SH : 0);  // two layers of 64
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4, H = a.d_hidden;
+  float* pdz = bias + 128 + wave * (2 * 16 * T32_STRIDE);  // this wave's rows of a gradient,
+  float* ph = pdz + 16 * T32_STRIDE;                       // and of the input of that layer
+  read_layer32<THREADS>(a.w_in, H, a.d_in, tid, [&](int o, int c, f32x4_t v) {
+    if (c >= 16 * TI) return;
+    *reinterpret_cast<f32x4_t*>(w1 + o * SI + c) = v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w1t[(c + e) * SH + o] = v[e];
+  });
+  if constexpr (DEEP)
+    read_layer32<THREADS>(a.w_hid, H, H, tid, [&](int o, int c, f32x4_t v) {
+      *reinterpret_cast<f32x4_t*>(w2 + o * SH + c) = v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w2t[(c + e) * SH + o] = v[e];
+    });
+  read_layer32<THREADS>(a.w_out, a.d_out, H, tid, [&](int o, int c, f32x4_t v) {
+    if (o < 16 * TO)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) wot[(c + e) * SO + o] = v[e];
+  });
+  if (tid < 64) {
+    bias[tid] = a.b_in != nullptr && tid < H ? a.b_in[tid] : 0.0f;
+    bias[64 + tid] = DEEP && a.b_hid != nullptr && tid < H ? a.b_hid[tid] : 0.0f;
+  }
+  __syncthreads();
+  const bool x_vec = ((uintptr_t)a.x % 16 == 0) && (a.x_stride % 4 == 0);
+  const bool dy_vec = ((uintptr_t)a.dy % 16 == 0) && (a.dy_stride % 4 == 0);
+  const bool dx_vec = a.dx != nullptr && ((uintptr_t)a.dx % 16 == 0) && (a.dx_stride % 4 == 0);
+  const f32x4_t zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4_t dw1[4][TI], dw2[4][DEEP ? 4 : 1], dwo[TO][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int j = 0; j < TI; ++j) dw1[i][j] = zero4;
+#pragma unroll
+    for (int j = 0; j < (DEEP ? 4 : 1); ++j) dw2[i][j] = zero4;
+#pragma unroll
+    for (int j = 0; j < TO; ++j) dwo[j][i] = zero4;
+  }
+  float db1 = 0.0f, db2 = 0.0f, dbo = 0.0f;  // of feature `lane`
+  const int64_t n_groups = (a.rows + 15) / 16, step = (int64_t)gridDim.x * WAVES;
+  f32x4_t x_next[4];
+  auto load_group = [&](int64_t grp) {
+    const int64_t row = grp * 16 + r;
+#pragma unroll
+    for (int t = 0; t < TI; ++t) x_next[t] = load_chain(a.x, a.x_stride, row, a.rows, 16 * t + 4 * g, a.d_in, x_vec);
+  };
+  auto put_panel = [&](float* panel, const f32x4_t (&v)[4], int n) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if (t < n) *reinterpret_cast<f32x4_t*>(panel + r * T32_STRIDE + 16 * t + 4 * g) = v[t];
+  };
+  auto activated = [&](const f32x4_t (&z)[4], f32x4_t (&h)[4]) {
+    with_act(a.act, [&](auto act_c) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) h[t][v] = act_fwd(z[t][v], decltype(act_c)::value);
+    });
+  };
+  auto gated = [&](f32x4_t (&d)[4], const f32x4_t (&z)[4]) {
+    with_act(a.act, [&](auto act_c) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) d[t][v] *= act_grad(z[t][v], decltype(act_c)::value);
+    });
+  };
+  // dW += dz^T h over the sixteen rows of the panels, four rows per product; lane (i, k) reads row 4*s + k, column 16*tile + i
+  auto gradient = [&](auto& dw, auto mt_c, auto nt_c) {
+    constexpr int MT = decltype(mt_c)::value, NT = decltype(nt_c)::value;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      float av[MT], bh[NT];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) av[mt] = pdz[(4 * s + g) * T32_STRIDE + 16 * mt + r];
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) bh[nt] = ph[(4 * s + g) * T32_STRIDE + 16 * nt + r];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) dw[mt][nt] = mfma4(av[mt], bh[nt], dw[mt][nt]);
+    }
+  };
+  auto column_sum = [&](int width) {
+    float sum = 0.0f;
+    if (lane < width)
+#pragma unroll
+      for (int k = 0; k < 16; ++k) sum += pdz[k * T32_STRIDE + lane];
+    return sum;
+  };
+  // groups to the workgroups in turn, then to their waves: every unit has as many
+  int64_t grp = (int64_t)wave * gridDim.x + blockIdx.x;
+  if (grp < n_groups) load_group(grp);
+  for (; grp < n_groups; grp += step) {
+    const int64_t row = grp * 16 + r;
+    f32x4_t x[4], d[4], z1[4], z2[4], h[4], acc[4];
+#pragma unroll
+    for (int t = 0; t < TI; ++t) x[t] = x_next[t];
+#pragma unroll
+    for (int t = 0; t < TO; ++t) d[t] = load_chain(a.dy, a.dy_stride, row, a.rows, 16 * t + 4 * g, a.d_out, dy_vec);  // used after the way forth
+    if (grp + step < n_groups) load_group(grp + step);
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) z1[mt] = *reinterpret_cast<const f32x4_t*>(bias + 16 * mt + 4 * g);
+    product32<TI, 4, SI>(z1, w1, x, r, g);
+    activated(z1, h);
+    if constexpr (DEEP) {
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) z2[mt] = *reinterpret_cast<const f32x4_t*>(bias + 64 + 16 * mt + 4 * g);
+      product32<4, 4, SH>(z2, w2, h, r, g);
+      activated(z2, h);
+    }
+    // output layer
+    put_panel(pdz, d, TO);
+    put_panel(ph, h, 4);
+    dbo += column_sum(16 * TO);
+    gradient(dwo, std::integral_constant<int, TO>{}, std::integral_constant<int, 4>{});
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = zero4;
+    product32<TO, 4, SO>(acc, wot, d, r, g);
+    if constexpr (DEEP) {
+      gated(acc, z2);
+      activated(z1, h);
+      put_panel(pdz, acc, 4);
+      put_panel(ph, h, 4);
+      db2 += column_sum(64);
+      gradient(dw2, std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
+#pragma unroll
+      for (int t = 0; t < 4; ++t) d[t] = zero4;
+      product32<4, 4, SH>(d, w2t, acc, r, g);
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) d[t] = acc[t];
+    }
+    gated(d, z1);
+    put_panel(pdz, d, 4);
+    put_panel(ph, x, TI);
+    db1 += column_sum(64);
+    gradient(dw1, std::integral_constant<int, 4>{}, std::integral_constant<int, TI>{});
+    if (a.dx != nullptr) {
+#pragma unroll
+      for (int t = 0; t < TI; ++t) acc[t] = zero4;
+      product32<4, TI, SH>(acc, w1t, d, r, g);
+#pragma unroll
+      for (int t = 0; t < TI; ++t) store_chain(a.dx, a.dx_stride, row, a.rows, 16 * t + 4 * g, a.d_in, dx_vec, acc[t]);
+    }
+  }
+  // the waves' sums, added in wave order (the same result on every run), to the workgroup's slot
+  __syncthreads();
+  f32x4_t* red = reinterpret_cast<f32x4_t*>(lds32) + lane;
+  float* redb = lds32 + fused32_tiles(TI, TO, DEPTH) * 256 + lane;
+  for (int w = 0; w < WAVES; ++w) {
+    if (wave == w) {
+      int at = 0;
+      auto add = [&](f32x4_t v) {
+        red[64 * at] = w == 0 ? v : red[64 * at] + v;
+        ++at;
+      };
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < TI; ++j) add(dw1[i][j]);
+      if constexpr (DEEP) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) add(dw2[i][j]);
+      }
+#pragma unroll
+      for (int i = 0; i < TO; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) add(dwo[i][j]);
+      redb[0] = w == 0 ? db1 : redb[0] + db1;
+      redb[64] = w == 0 ? db2 : redb[64] + db2;
+      redb[128] = w == 0 ? dbo : redb[128] + dbo;
+    }
+    __syncthreads();
+  }
+  constexpr int SUMS = fused32_sums(TI, TO, DEPTH);
+  f32x4_t* slot = reinterpret_cast<f32x4_t*>(a.slots + (size_t)blockIdx.x * SUMS);
+  for (int i = tid; i < SUMS / 4; i += THREADS) slot[i] = reinterpret_cast<const f32x4_t*>(lds32)[i];
+}
+
+// The slots of the workgroups in a fixed order into the caller's accumulators: sixteen interleaved runs, then a fixed tree.
+struct Fused32Sums {
+  float *dw_in, *db_in, *dw_hid, *db_hid, *dw_out, *db_out;
+  int ti, to, depth, d_in, d_hidden, d_out, n_slots, sums;
+};
+__global__ __launch_bounds__(1024) void mlp32_sum_k(const float* slots, Fused32Sums o) {
+  __shared__ float part[16][64];
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6, i = blockIdx.x * 64 + tx;
+  float sum = 0.0f;
+  if (i < o.sums) {
+#pragma unroll 4
+    for (int sl = ty; sl < o.n_slots; sl += 16) sum += slots[(size_t)sl * o.sums + i];
+  }
+  part[ty][tx] = sum;
+  __syncthreads();
+  if (ty != 0 || i >= o.sums) return;
+  float total = 0.0f;
+#pragma unroll
+  for (int q = 0; q < 16; q += 4) total += (part[q][tx] + part[q + 1][tx]) + (part[q + 2][tx] + part[q + 3][tx]);
+  const int hid = o.depth == 2 ? 16 : 0, tiles = 4 * o.ti + hid + 4 * o.to;
+  if (i >= tiles * 256) {
+    const int k = (i - tiles * 256) >> 6, f = i & 63;
+    float* db = k == 0 ? o.db_in : k == 1 ? o.db_hid : o.db_out;
+    if (db != nullptr && f < (k == 2 ? o.d_out : o.d_hidden) && (k != 1 || o.depth == 2)) db[f] += total;
+    return;
+  }
+  int tile = i >> 8;
+  float* dw = o.dw_in;
+  int nt = o.ti, n_out = o.d_hidden, n_in = o.d_in;
+  if (tile >= 4 * o.ti) {
+    tile -= 4 * o.ti;
+    nt = 4;
+    n_in = o.d_hidden;
+    dw = o.dw_hid;
+    if (tile >= hid) {
+      tile -= hid;
+      dw = o.dw_out;
+      n_out = o.d_out;
+    }
+  }
+  const int ln = (i & 255) >> 2, row = 16 * (tile / nt) + 4 * (ln >> 4) + (i & 3), col = 16 * (tile % nt) + (ln & 15);
+  if (row < n_out && col < n_in) dw[(size_t)row * n_in + col] += total;
+}
+
 template <typename Args>
-static int launch32(const void* kern, const Args& a, int64_t blocks, size_t lds, hipStream_t s, const char* what) {
+static int launch32(const void* kern, const Args& a, int64_t blocks, size_t lds, hipStream_t s, const char* what, int threads = 256) {
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return fail((int)e, "hipFuncSetAttribute: %s", hipGetErrorString(e));
   }
   void* args[] = {(void*)&a};
-  const hipError_t le = hipLaunchKernel(kern, dim3((unsigned)blocks), dim3(256), args, lds, s);
+  const hipError_t le = hipLaunchKernel(kern, dim3((unsigned)blocks), dim3((unsigned)threads), args, lds, s);
   if (le != hipSuccess) return fail((int)le, "hipLaunchKernel(%s): %s", what, hipGetErrorString(le));
   return 0;
 }
@@ -370,7 +675,25 @@ static size_t z32_bytes(int64_t rows, int d_hidden, int depth) {
   return ((size_t)depth * (size_t)rows * d_hidden * sizeof(float) + 255) / 256 * 256;
 }
 
+template <int TI, int TO, int DEPTH>
+static int bwd32_fused(const Fused32Args& a, Fused32Sums o, hipStream_t s) {
+  const int64_t groups = (a.rows + 15) / 16;
+  const int64_t blocks = groups < device_cus() ? groups : device_cus();
+  if (int rc = launch32((const void*)mlp32_bwd_k<TI, TO, DEPTH>, a, blocks, fused32_lds(TI, TO, DEPTH), s, "mlp32_bwd", 64 * fused32_waves(TI, TO, DEPTH))) return rc;
+  o.ti = TI;
+  o.to = TO;
+  o.depth = DEPTH;
+  o.n_slots = (int)blocks;
+  o.sums = fused32_sums(TI, TO, DEPTH);
+  const float* slots = a.slots;
+  void* args[] = {(void*)&slots, (void*)&o};
+  const hipError_t le = hipLaunchKernel((const void*)mlp32_sum_k, dim3((unsigned)((o.sums + 63) / 64)), dim3(1024), args, 0, s);
+  if (le != hipSuccess) return fail((int)le, "hipLaunchKernel(mlp32_sum): %s", hipGetErrorString(le));
+  return 0;
+}
+
 size_t mlp32_bwd_workspace_bytes(int64_t rows, int d_hidden, int depth) {
+  if (depth <= 2) return (size_t)device_cus() * FUSED32_MAX_SUMS * sizeof(float);
   return z32_bytes(rows, d_hidden, depth) + (size_t)SLOTS32 * PART32 * sizeof(float);
 }
 
@@ -390,9 +713,19 @@ int mlp32_bwd(const float* x, int64_t x_stride, const float* dy, int64_t dy_stri
               int d_out, int depth, int act, void* workspace, int64_t workspace_bytes, hipStream_t s) {
   const size_t need = mlp32_bwd_workspace_bytes(rows, d_hidden, depth);
   NF_REQUIRE(workspace != nullptr && workspace_bytes >= (int64_t)need, NF_EINVAL,
-             "float32 backward keeps %d pre-activations of %lld x %d float32 and partial weight gradients: it needs a "
+             "float32 backward keeps partial weight gradients and beyond two layers %d pre-activations of %lld x %d float32: it needs a "
              "workspace of %zu bytes (nf_mlp_workspace_bytes)", depth, (long long)rows, d_hidden, need);
   NF_REQUIRE((uintptr_t)workspace % 16 == 0, NF_EINVAL, "workspace must be 16-byte aligned");
+  if (depth <= 2) {
+    Fused32Args a = {x, dy, dx, x_stride, dy_stride, dx_stride, rows, w_in, b_in, w_hid, b_hid, w_out, (float*)workspace, d_in, d_hidden, d_out, act};
+    Fused32Sums o = {dw_in, db_in, dw_hid, db_hid, dw_out, db_out, 0, 0, 0, d_in, d_hidden, d_out, 0, 0};
+    const bool narrow = d_in <= 32, small = d_out <= 16;
+    if (depth == 2)
+      return narrow ? (small ? bwd32_fused<2, 1, 2>(a, o, s) : bwd32_fused<2, 4, 2>(a, o, s))
+                    : (small ? bwd32_fused<4, 1, 2>(a, o, s) : bwd32_fused<4, 4, 2>(a, o, s));
+    return narrow ? (small ? bwd32_fused<2, 1, 1>(a, o, s) : bwd32_fused<2, 4, 1>(a, o, s))
+                  : (small ? bwd32_fused<4, 1, 1>(a, o, s) : bwd32_fused<4, 4, 1>(a, o, s));
+  }
   float* z = (float*)workspace;
   float* part = (float*)((char*)workspace + z32_bytes(rows, d_hidden, depth));
   const int H = d_hidden;

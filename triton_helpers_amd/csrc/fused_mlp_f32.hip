@@ -347,7 +347,6 @@ __global__ __launch_bounds__(256) void reduce32_k(const float* part, int n_slots
 constexpr int fused32_tiles(int TI, int TO, int DEPTH) { return TO * 4 + (DEPTH - 1) * 16 + 4 * TI; }
 constexpr int fused32_waves(int TI, int TO, int DEPTH) { return fused32_tiles(TI, TO, DEPTH) <= 28 ? 8 : 4; }  // more gradients take the registers of two waves
 constexpr int fused32_sums(int TI, int TO, int DEPTH) { return fused32_tiles(TI, TO, DEPTH) * 256 + 3 * 64; }
-constexpr int FUSED32_MAX_SUMS = fused32_sums(4, 4, 2);
 constexpr int fused32_stride(int tiles) { return 16 * tiles + 4; }  // floats per staged row of so many tiles
 constexpr size_t fused32_lds(int TI, int TO, int DEPTH) {
   const int weights = 64 * fused32_stride(TI) + 16 * TI * W32_STRIDE + (DEPTH - 1) * 2 * 64 * W32_STRIDE + 64 * fused32_stride(TO) + 128;
@@ -676,24 +675,25 @@ static size_t z32_bytes(int64_t rows, int d_hidden, int depth) {
 }
 
 template <int TI, int TO, int DEPTH>
-static int bwd32_fused(const Fused32Args& a, Fused32Sums o, hipStream_t s) {
-  const int64_t groups = (a.rows + 15) / 16;
-  const int64_t blocks = groups < device_cus() ? groups : device_cus();
+static int bwd32_fused(const Fused32Args& a, Fused32Sums o, size_t slot_bytes, hipStream_t s) {
+  const int64_t groups = (a.rows + 15) / 16, slots = (int64_t)(slot_bytes / (fused32_sums(TI, TO, DEPTH) * sizeof(float)));
+  int64_t blocks = groups < device_cus() ? groups : device_cus();
+  if (blocks > slots) blocks = slots;  // (few rows of a wide network: the workspace is the layered kernels')
   if (int rc = launch32((const void*)mlp32_bwd_k<TI, TO, DEPTH>, a, blocks, fused32_lds(TI, TO, DEPTH), s, "mlp32_bwd", 64 * fused32_waves(TI, TO, DEPTH))) return rc;
   o.ti = TI;
   o.to = TO;
   o.depth = DEPTH;
   o.n_slots = (int)blocks;
   o.sums = fused32_sums(TI, TO, DEPTH);
-  const float* slots = a.slots;
-  void* args[] = {(void*)&slots, (void*)&o};
+  const float* sums = a.slots;
+  void* args[] = {(void*)&sums, (void*)&o};
   const hipError_t le = hipLaunchKernel((const void*)mlp32_sum_k, dim3((unsigned)((o.sums + 63) / 64)), dim3(1024), args, 0, s);
   if (le != hipSuccess) return fail((int)le, "hipLaunchKernel(mlp32_sum): %s", hipGetErrorString(le));
   return 0;
 }
 
+
 size_t mlp32_bwd_workspace_bytes(int64_t rows, int d_hidden, int depth) {
-  if (depth <= 2) return (size_t)device_cus() * FUSED32_MAX_SUMS * sizeof(float);
   return z32_bytes(rows, d_hidden, depth) + (size_t)SLOTS32 * PART32 * sizeof(float);
 }
 
@@ -713,7 +713,7 @@ int mlp32_bwd(const float* x, int64_t x_stride, const float* dy, int64_t dy_stri
               int d_out, int depth, int act, void* workspace, int64_t workspace_bytes, hipStream_t s) {
   const size_t need = mlp32_bwd_workspace_bytes(rows, d_hidden, depth);
   NF_REQUIRE(workspace != nullptr && workspace_bytes >= (int64_t)need, NF_EINVAL,
-             "float32 backward keeps partial weight gradients and beyond two layers %d pre-activations of %lld x %d float32: it needs a "
+             "float32 backward keeps %d pre-activations of %lld x %d float32 and partial weight gradients: it needs a "
              "workspace of %zu bytes (nf_mlp_workspace_bytes)", depth, (long long)rows, d_hidden, need);
   NF_REQUIRE((uintptr_t)workspace % 16 == 0, NF_EINVAL, "workspace must be 16-byte aligned");
   if (depth <= 2) {
@@ -721,10 +721,10 @@ int mlp32_bwd(const float* x, int64_t x_stride, const float* dy, int64_t dy_stri
     Fused32Sums o = {dw_in, db_in, dw_hid, db_hid, dw_out, db_out, 0, 0, 0, d_in, d_hidden, d_out, 0, 0};
     const bool narrow = d_in <= 32, small = d_out <= 16;
     if (depth == 2)
-      return narrow ? (small ? bwd32_fused<2, 1, 2>(a, o, s) : bwd32_fused<2, 4, 2>(a, o, s))
-                    : (small ? bwd32_fused<4, 1, 2>(a, o, s) : bwd32_fused<4, 4, 2>(a, o, s));
-    return narrow ? (small ? bwd32_fused<2, 1, 1>(a, o, s) : bwd32_fused<2, 4, 1>(a, o, s))
-                  : (small ? bwd32_fused<4, 1, 1>(a, o, s) : bwd32_fused<4, 4, 1>(a, o, s));
+      return narrow ? (small ? bwd32_fused<2, 1, 2>(a, o, need, s) : bwd32_fused<2, 4, 2>(a, o, need, s))
+                    : (small ? bwd32_fused<4, 1, 2>(a, o, need, s) : bwd32_fused<4, 4, 2>(a, o, need, s));
+    return narrow ? (small ? bwd32_fused<2, 1, 1>(a, o, need, s) : bwd32_fused<2, 4, 1>(a, o, need, s))
+                  : (small ? bwd32_fused<4, 1, 1>(a, o, need, s) : bwd32_fused<4, 4, 1>(a, o, need, s));
   }
   float* z = (float*)workspace;
   float* part = (float*)((char*)workspace + z32_bytes(rows, d_hidden, depth));

@@ -14,7 +14,7 @@ Supersets / differences:
   * float16 and bfloat16 storage (what autocast produces) runs on the 16-bit matrix instructions: the fast path.
     float32 tensors (the reference feeds them to ``tl.dot``, which multiplies in TF32: float32 range, 10-bit
     mantissa) run on the float32 matrix instruction: float32 range and mantissa, about a sixth of the 16-bit rate, and
-    beyond two hidden layers a backward scratch of ``depth * rows * d_hidden * 4`` bytes.  ``set_float32_operands("float16")`` trades the
+    a backward scratch of ``depth * rows * d_hidden * 4`` bytes.  ``set_float32_operands("float16")`` trades the
     range for speed: float32 tensors are then multiplied with float16 operands (the same 10-bit mantissa as TF32,
     float32 accumulation and results; operands beyond +-65504 overflow).
 """

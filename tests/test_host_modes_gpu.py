@@ -1,0 +1,43 @@
+"""The operators' native host path beside torch's tracer, forward-mode derivatives, saved-tensor hooks, inference mode and graph capture."""
+import pytest
+import torch
+
+from oracle import hash_encoding as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+GEO = dict(max_entries_per_level=2**10, min_res=4, max_res=32, levels=4)
+
+
+def _operator(name, seed=0):
+    """(operator, its tensor arguments): the input in front of the parameters."""
+    from triton_helpers_amd.layers.fully_fused_mlp import fully_fused_mlp
+    from triton_helpers_amd.layers.hash_encoding import hash_encoding
+    from triton_helpers_amd.layers.reversible_mlp import reversible_mlp
+
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    u = lambda *s: torch.rand(*s, generator=g, device=DEV) - 0.5  # noqa: E731
+    if name == "hash":
+        rows = O.level_row_offsets(4, 2**10, 3, 4, 32)[-1]
+        args = [u(100, 3) + 0.5, u(rows, 2).half()]
+        fn = lambda x, table: hash_encoding(x, table, **GEO)  # noqa: E731
+        fn(*args)  # the geometry's first call goes through the Python function
+        return fn, args
+    if name == "mlp":
+        return lambda x, w_in, w_hid, w_out: fully_fused_mlp(x, w_in, None, w_out, None, w_hid), [u(*s).half() for s in ((1, 70, 32), (64, 32), (64, 64), (16, 64))]
+    return lambda x, w1, w2: reversible_mlp(x, w1, None, w2, None), [u(*s).half() for s in ((70, 64), (64, 32), (64, 32))]
+
+
+OPERATORS = pytest.mark.parametrize("name", ["hash", "mlp", "reversible"])
+
+
+@OPERATORS
+@pytest.mark.parametrize("train", [False, True])
+def test_a_traced_function_runs_the_operator(name, train):
+    fn, args = _operator(name)
+    _, others = _operator(name, seed=1)
+    if train:
+        args[1:] = [t.requires_grad_() for t in args[1:]]
+    traced = torch.jit.trace(lambda *a: fn(*a) * 2, tuple(args), check_trace=False)
+    assert "PythonOp" in str(traced.graph) or "^" in str(traced.graph)
+    assert torch.equal(traced(*others), fn(*others) * 2)

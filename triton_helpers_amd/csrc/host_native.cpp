@@ -3,7 +3,7 @@
 // fused MLP at 64 rows took 66 us of interpreter, ctypes and engine time around 25 us of kernels, with the backward waiting
 // for the interpreter lock on the engine's thread.
 //
-// Each operator's function here takes the plain case (GPU tensors, no tracing or function modes) and returns None for everything
+// Each operator's function here takes the plain case (GPU tensors, no tracing or other modes) and returns None for everything
 // else, an argument error included: the Python function of the operator then takes over, which holds the full checks and
 // their messages.  Both come to the same launch functions below.
 #include <Python.h>
@@ -18,6 +18,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <array>
@@ -421,7 +422,10 @@ bool plain_or_none(PyObject* o, std::optional<Tensor>* t) {
   return true;
 }
 
-bool modes_active() { return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled(); }
+// A dispatch or function mode, or the tracer, which records an autograd Function but would see nothing of a launch made here.
+bool modes_active() {
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing();
+}
 
 bool autocast() { return at::autocast::is_autocast_enabled(at::kCUDA); }
 

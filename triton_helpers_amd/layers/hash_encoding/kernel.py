@@ -135,9 +135,10 @@ class HashEncoding(torch.autograd.Function):
         bwd_divider: Optional[int] = None,
         scale: float = 1.0,
     ) -> Tensor:
-        D_in = coords.shape[-1]
+        # (plain numbers: while a function is traced, a shape's entries are tensors)
+        D_in = int(coords.shape[-1])
         D_feature = features.shape[-1] if features is not None else 0
-        D_embed = embeddings.shape[-1]
+        D_embed = int(embeddings.shape[-1])
 
         assert coords.is_floating_point(), "Coords must be float"
 

@@ -41,3 +41,31 @@ def test_a_traced_function_runs_the_operator(name, train):
     traced = torch.jit.trace(lambda *a: fn(*a) * 2, tuple(args), check_trace=False)
     assert "PythonOp" in str(traced.graph) or "^" in str(traced.graph)
     assert torch.equal(traced(*others), fn(*others) * 2)
+
+
+@OPERATORS
+@pytest.mark.parametrize("which", ["input", "parameter"])
+@pytest.mark.parametrize("mode", ["plain", "no_grad", "train"])
+def test_forward_mode_derivatives_are_refused(name, which, mode):
+    """A tangent that no kernel carries on raises instead of getting lost."""
+    import torch.autograd.forward_ad as fw
+
+    fn, args = _operator(name)
+    if mode == "train":
+        args[-1].requires_grad_()
+    with fw.dual_level(), torch.set_grad_enabled(mode != "no_grad"):
+        i = 0 if which == "input" else 1
+        args[i] = fw.make_dual(args[i], torch.ones_like(args[i]))
+        with pytest.raises(NotImplementedError):
+            fn(*args)
+
+
+@OPERATORS
+def test_function_transforms_are_refused(name):
+    """Inside a transform the autograd Functions refuse, also where the operator's own arguments are plain tensors."""
+    fn, args = _operator(name)
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda s: fn(*args).sum() * s)(torch.ones(3, device=DEV))
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda s: (fn(*args).float() * s).sum())(torch.ones((), device=DEV))
+    fn(*args)

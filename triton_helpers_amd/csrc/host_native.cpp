@@ -3,7 +3,7 @@
 // fused MLP at 64 rows took 66 us of interpreter, ctypes and engine time around 25 us of kernels, with the backward waiting
 // for the interpreter lock on the engine's thread.
 //
-// Each operator's function here takes the plain case (GPU tensors, no tracing or other modes) and returns None for everything
+// Each operator's function here takes the plain case (GPU tensors, no tracing, tangents or other modes) and returns None for everything
 // else, an argument error included: the Python function of the operator then takes over, which holds the full checks and
 // their messages.  Both come to the same launch functions below.
 #include <Python.h>
@@ -13,6 +13,7 @@
 #include <ATen/core/LegacyTypeDispatch.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -404,14 +405,15 @@ struct ReversibleMlp : torch::autograd::Function<ReversibleMlp> {
 };
 
 // ------------------------------------------------------------------------------------------------ Python
-// A plain GPU tensor: no subclass, no wrapper of a function transform, a floating type the kernels know.
+// A plain GPU tensor: no subclass, no wrapper of a function transform, no tangent of a forward-mode derivative (the kernels have no
+// such derivative: the autograd Function refuses it), a floating type the kernels know.
 bool plain(PyObject* o, Tensor* t) {
   if (!THPVariable_CheckTypeExact(Py_TYPE(o))) return false;
   *t = THPVariable_Unpack(o);
   const auto keys = t->key_set();
   return t->is_cuda() && t->layout() == at::kStrided && !keys.has(c10::DispatchKey::FuncTorchBatched) &&
          !keys.has(c10::DispatchKey::FuncTorchGradWrapper) && !keys.has(c10::DispatchKey::Functionalize) && !keys.has(c10::DispatchKey::Python) &&
-         !t->is_conj() && !t->is_neg();
+         !t->is_conj() && !t->is_neg() && !t->_fw_grad(/*level=*/0).defined();
 }
 
 bool plain_or_none(PyObject* o, std::optional<Tensor>* t) {
@@ -422,9 +424,11 @@ bool plain_or_none(PyObject* o, std::optional<Tensor>* t) {
   return true;
 }
 
-// A dispatch or function mode, or the tracer, which records an autograd Function but would see nothing of a launch made here.
+// A dispatch or function mode, a function transform (vmap, grad, jvp: the autograd Functions refuse them), or the tracer, which records
+// an autograd Function but would see nothing of a launch made here.
 bool modes_active() {
-  return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing();
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing() ||
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
 }
 
 bool autocast() { return at::autocast::is_autocast_enabled(at::kCUDA); }

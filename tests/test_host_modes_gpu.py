@@ -69,3 +69,42 @@ def test_function_transforms_are_refused(name):
     with pytest.raises(RuntimeError):
         torch.func.grad(lambda s: (fn(*args).float() * s).sum())(torch.ones((), device=DEV))
     fn(*args)
+
+
+@OPERATORS
+def test_checkpointed_gradients(name):
+    """A saved-tensor hook that recomputes (non-reentrant checkpointing) runs with autograd on inside the operator's backward."""
+    from torch.utils.checkpoint import checkpoint
+
+    fn, args = _operator(name)
+    scale = torch.full((), 1.5, device=DEV, dtype=torch.float16)
+
+    def step(*a):  # the operator's tensors come out of a differentiable operation inside the checkpointed region
+        return fn(a[0], *(t * scale for t in a[1:])) if name == "hash" else fn(*(t * scale for t in a))
+
+    got = []
+    for through in (lambda *a: step(*a), lambda *a: checkpoint(step, *a, use_reentrant=False)):
+        leaves = [t.clone().requires_grad_(name != "hash" or i > 0) for i, t in enumerate(args)]
+        y = through(*leaves)
+        y.backward(torch.ones_like(y))
+        got.append([y.detach(), *(t.grad for t in leaves if t.requires_grad)])
+    assert all(t is not None for t in got[1])
+    for a, b in zip(*got):
+        torch.testing.assert_close(a, b, rtol=2**-10, atol=2**-10 * float(a.abs().max()))  # (atomics in two of the backwards: a rounding apart)
+
+
+@OPERATORS
+def test_saved_tensors_on_the_host(name):
+    fn, args = _operator(name)
+    got = []
+    for hooks in (False, True):
+        leaves = [t.clone().requires_grad_(i > 0) for i, t in enumerate(args)]
+        if hooks:
+            with torch.autograd.graph.save_on_cpu():
+                y = fn(*leaves)
+        else:
+            y = fn(*leaves)
+        y.backward(torch.ones_like(y))
+        got.append([t.grad for t in leaves[1:]])
+    for a, b in zip(*got):
+        torch.testing.assert_close(a, b, rtol=2**-10, atol=2**-10 * float(a.abs().max()))

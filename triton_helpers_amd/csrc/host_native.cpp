@@ -198,6 +198,8 @@ Tensor encode_table_grad(const Tensor& coords, const Tensor& grad, const Tensor&
   return de;
 }
 
+// In the nodes' backwards the saved tensors are unpacked first: that runs the user's saved-tensor hooks (checkpointing recomputes its
+// region there), which need autograd on.
 struct HashEncoding : torch::autograd::Function<HashEncoding> {
   static Tensor forward(AutogradContext* ctx, const Tensor& coords, const Tensor& table, const Tensor& pi, const Geometry* geo, double scale,
                         int64_t flags) {
@@ -209,8 +211,8 @@ struct HashEncoding : torch::autograd::Function<HashEncoding> {
     return encode_forward(coords, table, pi, *geo, scale, flags);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const at::AutoDispatchBelowADInplaceOrView below;
     const variable_list saved = ctx->get_saved_variables();
+    const at::AutoDispatchBelowADInplaceOrView below;
     const auto* geo = (const Geometry*)(uintptr_t)ctx->saved_data["geometry"].toInt();
     const Tensor de = encode_table_grad(saved[0], grads[0], saved[1], saved[2], *geo, ctx->saved_data["scale"].toDouble(), ctx->saved_data["flags"].toInt());
     return {Tensor(), de, Tensor(), Tensor(), Tensor(), Tensor()};
@@ -341,8 +343,8 @@ struct FusedMlp : torch::autograd::Function<FusedMlp> {
     return mlp_forward(std::move(m));
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const at::AutoDispatchBelowADInplaceOrView below;
     const variable_list s = ctx->get_saved_variables();
+    const at::AutoDispatchBelowADInplaceOrView below;
     variable_list r = mlp_backward(Mlp{s[0], {s[1], s[2], s[3], s[4], s[5], s[6]}, (int)ctx->saved_data["act"].toInt()}, grads[0],
                                    ctx->needs_input_grad(0), ctx->saved_data["float_grads"].toBool());
     r.resize(9);
@@ -396,8 +398,8 @@ struct ReversibleMlp : torch::autograd::Function<ReversibleMlp> {
     return y;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const at::AutoDispatchBelowADInplaceOrView below;
     const variable_list s = ctx->get_saved_variables();
+    const at::AutoDispatchBelowADInplaceOrView below;
     variable_list r = reversible_backward(s[0], grads[0], {s[1], s[2], s[3], s[4]}, (int)ctx->saved_data["act"].toInt(), false);
     r.resize(6);
     return r;

@@ -108,3 +108,84 @@ def test_saved_tensors_on_the_host(name):
         got.append([t.grad for t in leaves[1:]])
     for a, b in zip(*got):
         torch.testing.assert_close(a, b, rtol=2**-10, atol=2**-10 * float(a.abs().max()))
+
+
+_PRELUDE = """
+import torch
+from oracle import hash_encoding as O
+from triton_helpers_amd.layers.hash_encoding import hash_encoding
+geo = dict(max_entries_per_level=2**10, min_res=4, max_res=32, levels=4)
+x = torch.rand(100, 3, device="cuda")
+table = torch.rand(O.level_row_offsets(4, 2**10, 3, 4, 32)[-1], 2, device="cuda")
+"""
+_ORDERS = {
+    "ordinary call, inference, training": """
+want = hash_encoding(x, table, **geo)
+with torch.inference_mode():
+    assert torch.equal(hash_encoding(x, table, **geo), want)
+hash_encoding(x, table.requires_grad_(), **geo).sum().backward()
+assert table.grad.any()
+""",
+    "inference, training": """
+with torch.inference_mode():
+    hash_encoding(x, table, **geo)
+hash_encoding(x, table.requires_grad_(), **geo).sum().backward()
+assert table.grad.any()
+""",
+    "one call, capture": """
+want = hash_encoding(x, table, **geo)
+torch.cuda.synchronize()
+graph = torch.cuda.CUDAGraph()
+with torch.cuda.graph(graph):
+    out = hash_encoding(x, table, **geo)
+for _ in range(3):
+    out.zero_()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+""",
+}
+
+
+@pytest.mark.parametrize("order", _ORDERS)
+def test_default_primes_whatever_the_first_call_was(order):
+    """The primes are made once per process and device, so each order of first calls has a process of its own."""
+    import subprocess
+    import sys
+
+    done = subprocess.run([sys.executable, "-c", _PRELUDE + _ORDERS[order]], capture_output=True, text=True, timeout=100)
+    assert done.returncode == 0, done.stderr
+
+
+@pytest.mark.parametrize("N,dtype", [(1000, torch.float16), (8192, torch.float32), (20000, torch.float16)])
+def test_captured_training_step_of_the_encoder(N, dtype):
+    """After one ordinary step, forward and backward replay from a graph: atomics, the walk without records, sorted records."""
+    from triton_helpers_amd.layers.hash_encoding import hash_encoding
+
+    geo = dict(max_entries_per_level=2**14 if N == 8192 else 2**18, min_res=16, max_res=512, levels=4)
+    E = O.level_row_offsets(4, geo["max_entries_per_level"], 3, 16, 512)[-1]
+    x, do = torch.rand(N, 3, device=DEV), torch.randn(N, 8, device=DEV).to(dtype)
+    table = torch.randn(E, 2, device=DEV).to(dtype).requires_grad_()
+
+    def step():
+        table.grad = None
+        y = hash_encoding(x, table, **geo)
+        y.backward(do)
+        return y.detach(), table.grad
+
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        step()
+    torch.cuda.current_stream().wait_stream(stream)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for _ in range(3):
+        x.uniform_()
+        do.normal_()
+        want = [t.clone() for t in step()]
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[0], want[0])
+        torch.testing.assert_close(out[1], want[1], rtol=2**-10, atol=2**-10 * float(want[1].abs().max()))

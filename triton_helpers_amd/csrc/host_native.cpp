@@ -13,8 +13,11 @@
 #include <ATen/core/LegacyTypeDispatch.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/InferenceMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -111,15 +114,25 @@ const Geometry* find_geometry(const std::array<int64_t, 6>& key) {  // under the
   return nullptr;
 }
 
-// the paper's primes on a device, made once
-Tensor default_primes(const Tensor& like) {
+// The paper's primes on a GPU, made once per process for all callers, the Python functions among them: as an ordinary tensor, whatever
+// the mode of the first call (an inference tensor could not be saved for a backward later, a wrapper of a mode would outlive it).
+Tensor default_primes(c10::Device device) {
   static std::mutex m;
   static auto* by_device = new std::vector<Tensor>();
   std::lock_guard<std::mutex> lock(m);
-  const size_t i = like.device().index();
+  const size_t i = device.index();
   if (by_device->size() <= i) by_device->resize(i + 1);
   Tensor& t = (*by_device)[i];
-  if (!t.defined()) t = at::tensor(at::ArrayRef<int64_t>({1, 2654435761ll, 805459861ll}), at::kLong).to(like.device());
+  if (!t.defined()) {
+    const c10::DeviceGuard guard(device);
+    TORCH_CHECK(c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None,
+                "the first call of the hash encoding on a device copies its primes there: make one before capturing a graph");
+    const c10::InferenceMode ordinary(false);
+    using K = c10::DispatchKey;
+    const c10::impl::ExcludeDispatchKeyGuard no_modes(c10::DispatchKeySet(
+        {K::Python, K::PythonTLSSnapshot, K::Functionalize, K::FuncTorchVmapMode, K::FuncTorchDynamicLayerFrontMode, K::FuncTorchDynamicLayerBackMode, K::Tracer}));
+    t = at::tensor(at::ArrayRef<int64_t>({1, 2654435761ll, 805459861ll}), at::kLong).to(device);
+  }
   return t;
 }
 
@@ -524,7 +537,7 @@ PyObject* hash_encoding(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor out;
   {
     pybind11::gil_scoped_release release;
-    const Tensor primes = pi ? *pi : default_primes(coords);
+    const Tensor primes = pi ? *pi : default_primes(coords.device());
     if (at::GradMode::is_enabled() && table.requires_grad()) {
       out = HashEncoding::apply(coords, table, primes, geo, scale, flags);
     } else {
@@ -533,6 +546,21 @@ PyObject* hash_encoding(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
   }
   return wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// primes(index of a GPU): the default primes there
+PyObject* primes(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  NARGS(1);
+  int64_t index;
+  TORCH_CHECK(as_int(a[0], &index) && index >= 0 && index < c10::hip::device_count(), "index of a GPU expected");
+  Tensor t;
+  {
+    pybind11::gil_scoped_release release;
+    t = default_primes(c10::Device(c10::kCUDA, (c10::DeviceIndex)index));
+  }
+  return wrap(t);
   END_HANDLE_TH_ERRORS
 }
 
@@ -718,8 +746,8 @@ PyObject* reversible_launch_backward(PyObject*, PyObject* const* a, Py_ssize_t n
 }
 
 #define ENTRY(f) {#f, (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {ENTRY(add_geometry),       ENTRY(hash_encoding),       ENTRY(hash_table_grad),
-                         ENTRY(mlp),                ENTRY(mlp_launch_forward),  ENTRY(mlp_launch_backward),
+PyMethodDef methods[] = {ENTRY(add_geometry),       ENTRY(primes),                    ENTRY(hash_encoding), ENTRY(hash_table_grad),
+                         ENTRY(mlp),                ENTRY(mlp_launch_forward),        ENTRY(mlp_launch_backward),
                          ENTRY(reversible),         ENTRY(reversible_launch_forward), ENTRY(reversible_launch_backward),
                          {nullptr, nullptr, 0, nullptr}};
 

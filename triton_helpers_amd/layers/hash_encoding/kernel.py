@@ -52,15 +52,11 @@ _FLAGS = 0  # test hook: _lib.NF_HASH_FORCE_GENERIC / NF_HASH_FORCE_ATOMIC / NF_
 # ---------------------------------------------------------------------------
 # Launch helpers
 # ---------------------------------------------------------------------------
-_default_primes: Dict[torch.device, Tensor] = {}
-
-
 def _primes_for(device: torch.device) -> Tensor:
-    p = _default_primes.get(device)
-    if p is None:
-        p = torch.tensor([PI_1, PI_2, PI_3], dtype=torch.int64, device=device)
-        _default_primes[device] = p
-    return p
+    """The default primes on ``device``: one tensor per GPU, kept by the native host side for its own calls too."""
+    if device.type != "cuda":
+        return torch.tensor([PI_1, PI_2, PI_3], dtype=torch.int64, device=device)
+    return _lib.native().primes(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def _flat_coords(coords: Tensor) -> Tensor:

@@ -246,7 +246,7 @@ int nf_revmlp_fwd(const void* x, int64_t x_stride, void* y, int64_t y_stride, co
 /* Backward from the OUTPUT y: the inputs are recomputed block by block inside the kernel.
  * dx [rows, 2*half] in `dtype`; x_rec [rows, 2*half] in `dtype` (required: the kernel carries the stream between
  * couplings in it) receives the reconstructed input;
- * dw1, dw2, db1, db2 are float32 accumulators, NOT cleared by the call (db1, db2 may be NULL). */
+ * dw1, dw2, db1, db2 are float32 accumulators, NOT cleared by the call (db1, db2 may be NULL), added to with atomics. */
 int nf_revmlp_bwd(const void* y, int64_t y_stride, const void* dy, int64_t dy_stride, void* dx, int64_t dx_stride,
                   void* x_rec, int64_t x_rec_stride, const void* w1, const void* b1, const void* w2, const void* b2,
                   float* dw1, float* db1, float* dw2, float* db2, int64_t rows, int half, int blocks, int act,

@@ -37,6 +37,17 @@ def test_library_exports_every_declared_symbol():
     assert f"#define NF_ABI_VERSION {_lib.NF_ABI_VERSION}" in header
 
 
+def test_library_allocates_and_waits_for_nothing():
+    """The contract of every entry point: no device memory is taken or given back and no call waits, so none of these is imported."""
+    from triton_helpers_amd import _lib
+
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libnf_cdna4.so not built (run python -m triton_helpers_amd.build)")
+    names = set(re.findall(rb"hip[A-Z][A-Za-z0-9_]+", _lib.LIB_PATH.read_bytes()))
+    assert b"hipLaunchKernel" in names
+    assert not [n for n in names if re.match(rb"hip(Ext)?(Malloc|Free|HostMalloc|HostFree)|hip(Device|Stream|Event)Synchronize|hipStreamWaitEvent", n)]
+
+
 def test_argument_validation_without_gpu():
     """Entry points validate before touching the device: bad arguments come back as negative codes."""
     from triton_helpers_amd import _lib

@@ -284,3 +284,37 @@ def test_cases_that_once_missed_the_tolerance(case, rows, H, blocks, act, bias, 
     for name, leaf in zip(("dw1", "db1", "dw2", "db2"), leaves):
         if leaf is not None:
             _close(leaf.grad, want[name], name, scale_rel=True, blocks=blocks)
+
+
+@pytest.mark.parametrize("rows,H,blocks,act,bias,dtype", [
+    (1, 64, 1, "gelu", True, torch.bfloat16), (96, 64, 4, "gelu", True, torch.bfloat16), (513, 48, 2, "gelu", False, torch.float16),
+    (4096 + 17, 64, 2, "silu", True, torch.float16), (8192, 32, 4, "gelu", True, torch.bfloat16), (640, 32, 3, "relu", False, torch.float16),
+    (300, 20, 2, "none", True, torch.bfloat16), (256 * 128 * 3, 64, 4, "gelu", True, torch.float16),
+])
+def test_backward_without_a_workspace(rows, H, blocks, act, bias, dtype):
+    """``nf_revmlp_bwd`` adds float32 gradients with atomics and takes no scratch: the stream has the bits of the entry with a workspace,
+    and the gradients are its sums of at most 257 float32 parts in another order (257 * 2^-24 of the parts, which cancel a little)."""
+    from triton_helpers_amd import _lib as L_
+
+    lib = L_.load()
+    g = torch.Generator().manual_seed(rows)
+    w1, b1, w2, b2 = (None if t is None else t.to(DEV) for t in _params(blocks, H, bias, dtype, seed=rows))
+    y, dy = (torch.randn(rows, 2 * H, generator=g).to(dtype).to(DEV) for _ in range(2))
+    dt, code, stream = L_.dtype_code(dtype), L_.NF_ACT[act], L_.current_stream(y.device)
+    need = lib.nf_revmlp_bwd_workspace_bytes(rows, H, blocks)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    got = []
+    for summed in (False, True):
+        dx, x_rec = torch.empty_like(y), torch.empty_like(y)
+        grads = [None if t is None else torch.full(t.shape, 0.5, device=DEV) for t in (w1, b1, w2, b2)]
+        head = (y.data_ptr(), 2 * H, dy.data_ptr(), 2 * H, dx.data_ptr(), 2 * H, x_rec.data_ptr(), 2 * H, *(L_.ptr(t) for t in (w1, b1, w2, b2, *grads)))
+        if summed:
+            rc = lib.nf_revmlp_bwd_summed(*head, rows, H, blocks, code, dt, L_.NF_F32, ws.data_ptr(), need, stream)
+        else:
+            rc = lib.nf_revmlp_bwd(*head, rows, H, blocks, code, dt, stream)
+        assert rc == 0, lib.nf_last_error()
+        got.append((dx, x_rec, [None if t is None else t - (0.0 if summed else 0.5) for t in grads]))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    for a, b in zip(got[0][2], got[1][2]):
+        if b is not None:
+            assert float((a - b).norm()) <= 1e-4 * float(b.norm()) + 1e-5 * b.numel() ** 0.5

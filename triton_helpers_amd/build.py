@@ -8,6 +8,7 @@ operators (``csrc/host_native.cpp``) into ``triton_helpers_amd/_native.so``.
 from __future__ import annotations
 
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -40,6 +41,9 @@ NO_CONTRACT = {"hash_encoding.hip", "hash_encoding_bwd_scan.hip", "hash_encoding
 # Files whose MFMA results feed vector ALU work directly: keep them in architectural VGPRs instead of
 # bouncing every result through an accumulation register.
 MFMA_VGPR_FORM = {"fused_mlp.hip", "fused_mlp_bwd2.hip", "fused_mlp_bwdn.hip", "fused_mlp_bwd2_w8.hip", "fused_mlp_bwd2_ws.hip", "fused_mlp_fwd2.hip", "reversible_mlp.hip"}
+# Kernels at the edge of the register file that must not spill: a version of this one that spilled some was compiled wrong
+# (the high half of its 64-bit row counter was set aside in an accumulation register and never read back).
+NO_SPILL = {"reversible_mlp.hip": "rev_bwd_block_k"}
 
 
 def _hipcc() -> str:
@@ -49,7 +53,7 @@ def _hipcc() -> str:
     return exe
 
 
-def _run(cmd: List[str], verbose: bool) -> None:
+def _run(cmd: List[str], verbose: bool) -> str:
     if verbose:
         print("+", " ".join(cmd), flush=True)
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
@@ -58,6 +62,28 @@ def _run(cmd: List[str], verbose: bool) -> None:
         raise RuntimeError(f"command failed ({proc.returncode}): {' '.join(cmd)}\n{out}")
     if verbose and out.strip():
         print(out, flush=True)
+    return out
+
+
+def _check_spills(out: str, kernel: str) -> None:
+    """Refuse a build whose resource remarks show spilled registers in ``kernel``."""
+    seen = 0
+    for part in out.split("Function Name: ")[1:]:
+        name, spill = part.split()[0], re.search(r"VGPRs Spill: (\d+)", part)
+        if kernel in name:
+            seen += 1
+            if spill is None or int(spill[1]) != 0:
+                raise RuntimeError(f"{name} spills registers; its listing has to be looked through before it may run")
+    if not seen:
+        raise RuntimeError(f"no resource remarks for {kernel}")
+
+
+def _compile(cmd: List[str], src: Path, verbose: bool) -> None:
+    kernel = NO_SPILL.get(src.name)
+    if kernel is None:
+        _run(cmd, verbose)
+    else:
+        _check_spills(_run([*cmd, "-Rpass-analysis=kernel-resource-usage"], False), kernel)
 
 
 def sources() -> List[Path]:
@@ -93,10 +119,10 @@ def build(verbose: bool = True, jobs: int = 8) -> Path:
             flags.append("-ffp-contract=off")
         if src.name in MFMA_VGPR_FORM:
             flags += ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-        cmds.append([hipcc, *flags, "-c", str(src), "-o", str(obj)])
+        cmds.append(([hipcc, *flags, "-c", str(src), "-o", str(obj)], src))
         objs.append(obj)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
-        list(ex.map(lambda c: _run(c, verbose), cmds))
+        list(ex.map(lambda c: _compile(*c, verbose), cmds))
     tmp = LIB_PATH.with_suffix(".so.tmp")
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)], verbose)
     os.replace(tmp, LIB_PATH)

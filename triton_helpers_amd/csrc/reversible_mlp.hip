@@ -36,7 +36,8 @@ struct RevArgs {
   int64_t dy_stride;
   uint16_t* dx;
   int64_t dx_stride;
-  const uint16_t *w1, *b1, *w2, *b2;  // forward: first coupling of this launch
+  const uint16_t *w1, *b1, *w2, *b2;  // forward, and backward without a workspace: first coupling of this launch
+  float *dw1, *db1, *dw2, *db2;       // backward without a workspace: float32 accumulators of the weight gradients, likewise
   const char* packed;                 // backward: the LDS images of the weights, first coupling of this launch
   float* slots;                       // backward: [workgroup][blocks] sums of the weight gradients, first coupling of this launch
   int64_t slot_stride;                // floats between the slots of two workgroups
@@ -404,31 +405,35 @@ struct RevImage {
   static constexpr int BYTES = ((8 * LAYER * 2 + 4 * HP * 4) + 1023) / 1024 * 1024;  // whole copies of a wave
 };
 constexpr int PACK_THREADS = 256;
+// One of the four parts of a sub-MLP's weights (s: 0 F, 1 G): a form of one of its layers, with the bias in the forward form.  The stream's
+// features are contracted in natural order and produced in wide order (the hidden ones as ever).
 template <typename T, int HP>
-__global__ __launch_bounds__(PACK_THREADS) void rev_pack_k(const uint16_t* w1, const uint16_t* b1, const uint16_t* w2, const uint16_t* b2, int H, char* packed) {
+__device__ __forceinline__ void lay_out_part(int part, int s, uint16_t* fw, const uint16_t* w1, const uint16_t* b1, const uint16_t* w2, const uint16_t* b2,
+                                             int H, int tid) {
   typedef RevImage<HP> I;
   constexpr bool WIDE = true;
-  // a workgroup per coupling and sub-MLP, and form of one of its layers
-  const int k = blockIdx.x >> 1, s = blockIdx.x & 1, tid = threadIdx.x;
-  const size_t sub = blockIdx.x;
-  uint16_t* fw = reinterpret_cast<uint16_t*>(packed + (size_t)k * I::BYTES);
   uint16_t* tw = fw + 4 * I::LAYER;
   float* bias = reinterpret_cast<float*>(tw + 4 * I::LAYER);
-  w1 += sub * H * H;
-  w2 += sub * H * H;
-  // the stream's features are contracted in natural order and produced in wide order (the hidden ones as ever)
-  switch (blockIdx.y) {
+  switch (part) {
     case 0:
       stage_weight_frags<!WIDE, false, PACK_THREADS>(fw + (2 * s) * I::LAYER, w1, H, H, I::MT, I::KC, tid, PACK_THREADS);
-      stage_bias_row<T>(bias + (2 * s) * HP, b1 ? b1 + sub * H : nullptr, H, HP, tid, PACK_THREADS);
+      stage_bias_row<T>(bias + (2 * s) * HP, b1, H, HP, tid, PACK_THREADS);
       break;
     case 1:
       stage_weight_frags<true, false, PACK_THREADS, WIDE>(fw + (2 * s + 1) * I::LAYER, w2, H, H, I::MT, I::KC, tid, PACK_THREADS);
-      stage_bias_row<T, WIDE>(bias + (2 * s + 1) * HP, b2 ? b2 + sub * H : nullptr, H, HP, tid, PACK_THREADS);
+      stage_bias_row<T, WIDE>(bias + (2 * s + 1) * HP, b2, H, HP, tid, PACK_THREADS);
       break;
     case 2: stage_weight_frags<true, true, PACK_THREADS, WIDE>(tw + (2 * s) * I::LAYER, w1, H, H, I::MT, I::KC, tid, PACK_THREADS); break;
     default: stage_weight_frags<!WIDE, true, PACK_THREADS>(tw + (2 * s + 1) * I::LAYER, w2, H, H, I::MT, I::KC, tid, PACK_THREADS); break;
   }
+}
+template <typename T, int HP>
+__global__ __launch_bounds__(PACK_THREADS) void rev_pack_k(const uint16_t* w1, const uint16_t* b1, const uint16_t* w2, const uint16_t* b2, int H, char* packed) {
+  // a workgroup per coupling and sub-MLP, and part
+  const int k = blockIdx.x >> 1, s = blockIdx.x & 1;
+  const size_t sub = blockIdx.x;
+  lay_out_part<T, HP>((int)blockIdx.y, s, reinterpret_cast<uint16_t*>(packed + (size_t)k * RevImage<HP>::BYTES), w1 + sub * H * H,
+                      b1 ? b1 + sub * H : nullptr, w2 + sub * H * H, b2 ? b2 + sub * H : nullptr, H, threadIdx.x);
 }
 
 // A workgroup's sums of a coupling's weight gradients: accumulator tiles [MT][MT][F.w1, F.w2, G.w1, G.w2] of 64 lanes x 4, then bias
@@ -448,7 +453,7 @@ __device__ __forceinline__ void put_db(float* slot, int lane, float v) {
 // interleaved runs over the slots, then a fixed tree.
 struct RevGrads {
   void *dw1, *db1, *dw2, *db2;
-  int half, n_slots, add, type;  // add: to what is there (float32)
+  int half, n_slots, type;
 };
 template <int HP>
 __global__ __launch_bounds__(1024) void rev_sum_k(const float* slots, int64_t slot_stride, RevGrads o) {
@@ -477,8 +482,7 @@ __global__ __launch_bounds__(1024) void rev_sum_k(const float* slots, int64_t sl
 #pragma unroll
   for (int q = 0; q < 16; q += 4) total += (part[q][tx] + part[q + 1][tx]) + (part[q + 2][tx] + part[q + 3][tx]);
   auto put = [&](void* base, int64_t at, float v) {
-    if (o.add) reinterpret_cast<float*>(base)[at] += v;
-    else if (o.type == NF_F32) reinterpret_cast<float*>(base)[at] = v;
+    if (o.type == NF_F32) reinterpret_cast<float*>(base)[at] = v;
     else if (o.type == NF_F16) reinterpret_cast<uint16_t*>(base)[at] = F16::from_f32(v);
     else reinterpret_cast<uint16_t*>(base)[at] = BF16::from_f32(v);
   };
@@ -504,7 +508,41 @@ __global__ __launch_bounds__(1024) void rev_sum_k(const float* slots, int64_t sl
   }
 }
 
-template <typename T, int HP, int ACT, bool FAST>
+// A tile of a workgroup without a slot: atomics into the float32 accumulators.  WIDE_ROWS / WIDE_COLS: the tile's rows (mt) / columns (nt)
+// are features in wide order.
+template <bool WIDE_ROWS, bool WIDE_COLS>
+__device__ __forceinline__ void add_tile(float* dw, int dim, int mt, int nt, int lane, f32x4_t v) {
+  const int c = WIDE_COLS ? wide_feature(nt, lane & 15) : 16 * nt + (lane & 15);
+  const int r0 = WIDE_ROWS ? wide_feature(mt, 4 * (lane >> 4)) : 16 * mt + 4 * (lane >> 4);
+  if (c >= dim) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (r0 + r < dim) unsafeAtomicAdd(dw + (size_t)(r0 + r) * dim + c, v[r]);
+}
+template <bool WIDE>
+__device__ __forceinline__ void add_db(float* db, int dim, int mt, int lane, float v) {
+  v += __shfl_xor(v, 16);
+  v += __shfl_xor(v, 32);
+  const int f = WIDE ? wide_feature(mt, lane & 15) : 16 * mt + lane;
+  if (db != nullptr && lane < 16 && f < dim) unsafeAtomicAdd(db + f, v);
+}
+
+// The same number, but what is worked out of it does not stay in registers from one turn of a loop to the next.
+__device__ __forceinline__ int fresh(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+__device__ __forceinline__ int64_t fresh_scalar(int64_t x) {
+  asm volatile("" : "+s"(x));
+  return x;
+}
+
+// WS: with a workspace, which holds the weights as LDS images and a slot for every workgroup's sums.  Without one a workgroup lays the
+// weights out itself and adds its sums with atomics; its addresses are worked out for every coupling again and its wave's number and rows
+// are scalar, because 64-wide halves leave no register to spare (a version that spilled some was compiled wrong: half of the 64-bit
+// row counter was set aside in an accumulation register and never brought back).  Four 64-wide GELU couplings with and without a workspace:
+// 1600 rows 90 and 79 us, 32768 rows 108 and 143, 2^20 1.10 ms both.
+template <typename T, int HP, int ACT, bool FAST, bool WS>
 __global__ __launch_bounds__(256) void rev_bwd_block_k(RevArgs a) {
   constexpr int MT = HP / 16, KC = HP / 32, LAYER = MT * KC * RFRAG;
   // The backward keeps the stream's features in wide order: the unchecked variant then reaches its rows with 16-byte
@@ -513,7 +551,7 @@ __global__ __launch_bounds__(256) void rev_bwd_block_k(RevArgs a) {
   constexpr bool WIDE = true;
   const int act = ACT >= 0 ? ACT : a.act;
   extern __shared__ __align__(16) unsigned char smem[];
-  const int tid = threadIdx.x, nthreads = blockDim.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = WS ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = FAST ? HP : a.half;
   // weights: forward-form [F.w1, F.w2, G.w1, G.w2], transposed-form the same order
   uint16_t* fw = reinterpret_cast<uint16_t*>(smem);
@@ -540,7 +578,14 @@ __global__ __launch_bounds__(256) void rev_bwd_block_k(RevArgs a) {
   const bool dy_v = top ? a.vec_dy : a.vec_dx;
   if (G2_LDS)
     for (int i = lane; i < MT * MT * 64; i += 64) g2acc[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  {
+  if constexpr (!WS) {
+    const int t = fresh(tid) & (PACK_THREADS - 1);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const size_t sub = 2 * kb + (i >> 2);
+      lay_out_part<T, HP>(i & 3, i >> 2, fw, a.w1 + sub * H * H, a.b1 ? a.b1 + sub * H : nullptr, a.w2 + sub * H * H, a.b2 ? a.b2 + sub * H : nullptr, H, t);
+    }
+  } else {
     const char* image = a.packed + (size_t)kb * RevImage<HP>::BYTES + 16 * lane;
     for (int i = __builtin_amdgcn_readfirstlane(wave) * 1024; i < RevImage<HP>::BYTES; i += 4096)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(image + i), (__attribute__((address_space(3))) void*)(smem + i), 16, 0, 0);
@@ -557,7 +602,7 @@ __global__ __launch_bounds__(256) void rev_bwd_block_k(RevArgs a) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) dwF1[i][j] = dwF2[i][j] = dwG1[i][j] = dwG2[i][j] = zero4;
 
-  for (int64_t chunk = (int64_t)blockIdx.x * 4 + wave; chunk < n_chunks; chunk += (int64_t)gridDim.x * 4) {
+  for (int64_t chunk = WS ? (int64_t)blockIdx.x * 4 + wave : fresh_scalar((int64_t)blockIdx.x * 4 + wave); chunk < n_chunks; chunk += (int64_t)gridDim.x * 4) {
     const int64_t row0 = chunk * 32;
     // The halves of y and dy that a sub-MLP's residual adds need are requested before that sub-MLP runs, so their
     // latency hides behind its products; nothing is held across both sub-MLPs (registers are the scarce resource).
@@ -707,6 +752,32 @@ __global__ __launch_bounds__(256) void rev_bwd_block_k(RevArgs a) {
     __syncthreads();
   }
   if (wave == 0) {
+  if constexpr (!WS) {
+    // layer order in dw1 / dw2: sub-MLP F is row block 0, G is row block 1 of the coupling
+    const int t = fresh(lane) & 63;
+    const size_t at = (size_t)2 * kb * H * H, HH = (size_t)H * H;
+    float *db1 = a.db1 ? a.db1 + (size_t)2 * kb * H : nullptr, *db2 = a.db2 ? a.db2 + (size_t)2 * kb * H : nullptr;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        add_tile<false, WIDE>(a.dw1 + at, H, i, j, t, dwF1[i][j]);
+        add_tile<WIDE, false>(a.dw2 + at, H, i, j, t, dwF2[i][j]);
+        add_tile<false, WIDE>(a.dw1 + at + HH, H, i, j, t, dwG1[i][j]);
+        if constexpr (G2_LDS) {
+          constexpr int PER_WAVE = MT * MT * 64;
+          const int q = (i * MT + j) * 64 + t;  // wave 0's g2acc is the first of the four
+          add_tile<WIDE, false>(a.dw2 + at + HH, H, i, j, t, (g2acc[q] + g2acc[PER_WAVE + q]) + (g2acc[2 * PER_WAVE + q] + g2acc[3 * PER_WAVE + q]));
+        } else {
+          add_tile<WIDE, false>(a.dw2 + at + HH, H, i, j, t, dwG2[i][j]);
+        }
+      }
+      add_db<false>(db1, H, i, t, dbF1[i]);
+      add_db<WIDE>(db2, H, i, t, dbF2[i]);
+      add_db<false>(db1 ? db1 + H : nullptr, H, i, t, dbG1[i]);
+      add_db<WIDE>(db2 ? db2 + H : nullptr, H, i, t, dbG2[i]);
+    }
+  } else {
   float* slot = a.slots + blockIdx.x * a.slot_stride + (size_t)kb * RevSlot<HP>::FLOATS;
   f32x4_t* tiles = reinterpret_cast<f32x4_t*>(slot) + lane;
 #pragma unroll
@@ -731,6 +802,7 @@ __global__ __launch_bounds__(256) void rev_bwd_block_k(RevArgs a) {
     put_db(dbs + 64 * i + 16, lane, dbF2[i]);
     put_db(dbs + 64 * i + 32, lane, dbG1[i]);
     put_db(dbs + 64 * i + 48, lane, dbG2[i]);
+  }
   }
   }
   // wave 0 has read the other waves' LDS accumulators and the reduction area: both are rewritten for the next coupling
@@ -804,7 +876,7 @@ static int rev_bwd_groups(int64_t rows) {
   return (int)(groups < rev_cus() ? groups : rev_cus());
 }
 
-template <typename T, int HP>
+template <typename T, int HP, bool WS>
 static int launch_rev_bwd(RevArgs a, hipStream_t s) {
   typedef RevImage<HP> I;
   size_t lds = I::BYTES + (HP > 32 ? (size_t)4 * I::MT * I::MT * 64 * 16 : 0);
@@ -812,12 +884,12 @@ static int launch_rev_bwd(RevArgs a, hipStream_t s) {
   const size_t red = (size_t)(HP > 32 ? 3 : 4) * I::MT * I::MT * 64 * 16 + (size_t)4 * I::MT * 64 * 4;
   if (HP <= 32 && lds < red) lds = red;
   const bool fast = a.half == HP && a.rows % 32 == 0 && a.vec_in && a.vec_out && a.vec_dy && a.vec_dx && a.wide_ok;
-  const void* kern = a.act == NF_ACT_GELU   ? (fast ? (const void*)rev_bwd_block_k<T, HP, NF_ACT_GELU, true>
-                                                    : (const void*)rev_bwd_block_k<T, HP, NF_ACT_GELU, false>)
-                     : a.act == NF_ACT_RELU ? (fast ? (const void*)rev_bwd_block_k<T, HP, NF_ACT_RELU, true>
-                                                    : (const void*)rev_bwd_block_k<T, HP, NF_ACT_RELU, false>)
-                     : (a.act == NF_ACT_SILU && fast) ? (const void*)rev_bwd_block_k<T, HP, NF_ACT_SILU, true>
-                                            : (const void*)rev_bwd_block_k<T, HP, -1, false>;
+  const void* kern = a.act == NF_ACT_GELU   ? (fast ? (const void*)rev_bwd_block_k<T, HP, NF_ACT_GELU, true, WS>
+                                                    : (const void*)rev_bwd_block_k<T, HP, NF_ACT_GELU, false, WS>)
+                     : a.act == NF_ACT_RELU ? (fast ? (const void*)rev_bwd_block_k<T, HP, NF_ACT_RELU, true, WS>
+                                                    : (const void*)rev_bwd_block_k<T, HP, NF_ACT_RELU, false, WS>)
+                     : (a.act == NF_ACT_SILU && fast) ? (const void*)rev_bwd_block_k<T, HP, NF_ACT_SILU, true, WS>
+                                            : (const void*)rev_bwd_block_k<T, HP, -1, false, WS>;
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return fail((int)e, "hipFuncSetAttribute: %s", hipGetErrorString(e));
@@ -833,6 +905,7 @@ static int launch_rev_bwd(RevArgs a, hipStream_t s) {
 static int64_t main_rows(int64_t rows) { return rows >= SPLIT_MIN_ROWS ? rows - rows % 32 : rows; }
 static int rev_bwd_slots(int64_t rows) { return rev_bwd_groups(main_rows(rows)) + (main_rows(rows) < rows ? 1 : 0); }
 
+// workspace NULL: without one, adding into the float32 accumulators of `grads`
 template <typename T, int HP>
 static int rev_bwd(const char* y, int64_t y_stride, const char* dy, int64_t dy_stride, char* dx, int64_t dx_stride, char* x_rec, int64_t x_rec_stride,
                    const void* w1, const void* b1, const void* w2, const void* b2, RevGrads grads, int64_t rows, int half, int blocks, int act,
@@ -842,9 +915,11 @@ static int rev_bwd(const char* y, int64_t y_stride, const char* dy, int64_t dy_s
   char* packed = (char*)workspace;
   float* slots = (float*)(packed + (size_t)blocks * I::BYTES);
   const int64_t slot_stride = (int64_t)blocks * S::FLOATS;
-  hipLaunchKernelGGL((rev_pack_k<T, HP>), dim3((unsigned)(2 * blocks), 4), dim3(PACK_THREADS), 0, s, (const uint16_t*)w1, (const uint16_t*)b1, (const uint16_t*)w2,
-                     (const uint16_t*)b2, half, packed);
-  if (int rc = check_launch("rev_pack")) return rc;
+  if (workspace != nullptr) {
+    hipLaunchKernelGGL((rev_pack_k<T, HP>), dim3((unsigned)(2 * blocks), 4), dim3(PACK_THREADS), 0, s, (const uint16_t*)w1, (const uint16_t*)b1, (const uint16_t*)w2,
+                       (const uint16_t*)b2, half, packed);
+    if (int rc = check_launch("rev_pack")) return rc;
+  }
   int64_t slot = 0;
   for (int64_t r0 = 0; r0 < rows;) {
     const int64_t n = r0 == 0 ? main_rows(rows) : rows - r0;
@@ -866,9 +941,21 @@ static int rev_bwd(const char* y, int64_t y_stride, const char* dy, int64_t dy_s
       a.dy_stride = first ? dy_stride : dx_stride;
       a.dx = (uint16_t*)dxp;
       a.dx_stride = dx_stride;
-      a.packed = packed + (size_t)kw * I::BYTES;
-      a.slots = slots + slot * slot_stride + (int64_t)kw * S::FLOATS;
-      a.slot_stride = slot_stride;
+      if (workspace != nullptr) {
+        a.packed = packed + (size_t)kw * I::BYTES;
+        a.slots = slots + slot * slot_stride + (int64_t)kw * S::FLOATS;
+        a.slot_stride = slot_stride;
+      } else {
+        const size_t w_at = (size_t)2 * kw * half * half, b_at = (size_t)2 * kw * half;
+        a.w1 = (const uint16_t*)w1 + w_at;
+        a.w2 = (const uint16_t*)w2 + w_at;
+        a.b1 = b1 ? (const uint16_t*)b1 + b_at : nullptr;
+        a.b2 = b2 ? (const uint16_t*)b2 + b_at : nullptr;
+        a.dw1 = (float*)grads.dw1 + w_at;
+        a.dw2 = (float*)grads.dw2 + w_at;
+        a.db1 = grads.db1 ? (float*)grads.db1 + b_at : nullptr;
+        a.db2 = grads.db2 ? (float*)grads.db2 + b_at : nullptr;
+      }
       a.rows = n;
       a.half = half;
       a.nblocks = fused ? blocks : 1;
@@ -878,12 +965,13 @@ static int rev_bwd(const char* y, int64_t y_stride, const char* dy, int64_t dy_s
       a.vec_dy = vec8_ok(a.dy, a.dy_stride, half);
       a.vec_dx = vec8_ok(a.dx, a.dx_stride, half);
       a.wide_ok = fused;  // the unchecked kernel is the fused launch's
-      if (int rc = launch_rev_bwd<T, HP>(a, s)) return rc;
+      if (int rc = workspace != nullptr ? launch_rev_bwd<T, HP, true>(a, s) : launch_rev_bwd<T, HP, false>(a, s)) return rc;
       if (fused) break;
     }
     slot += rev_bwd_groups(n);
     r0 += n;
   }
+  if (workspace == nullptr) return 0;
   grads.n_slots = (int)slot;
   hipLaunchKernelGGL((rev_sum_k<HP>), dim3((S::FLOATS / 4 + 63) / 64, (unsigned)blocks), dim3(1024), 0, s, slots, slot_stride, grads);
   return check_launch("rev_sum");
@@ -968,7 +1056,7 @@ extern "C" int nf_revmlp_bwd_summed(const void* y, int64_t y_stride, const void*
              "row stride smaller than 2*half");
   const int64_t need = nf_revmlp_bwd_workspace_bytes(rows, half, blocks);
   NF_REQUIRE(workspace_bytes >= need && (uintptr_t)workspace % 16 == 0, NF_EINVAL, "a 16-byte aligned workspace of %lld bytes is needed", (long long)need);
-  const RevGrads grads = {dw1, db1, dw2, db2, half, 0, 0, grad_dtype};
+  const RevGrads grads = {dw1, db1, dw2, db2, half, 0, grad_dtype};
   return rev_bwd_call(y, y_stride, dy, dy_stride, dx, dx_stride, x_rec, x_rec_stride, w1, b1, w2, b2, grads, rows, half, blocks, act, dtype, workspace, (hipStream_t)stream);
 }
 
@@ -982,15 +1070,7 @@ extern "C" int nf_revmlp_bwd(const void* y, int64_t y_stride, const void* dy, in
              "NULL pointer argument (x_rec is required: it carries the reconstructed input between blocks)");
   NF_REQUIRE(y_stride >= 2 * half && dy_stride >= 2 * half && dx_stride >= 2 * half && x_rec_stride >= 2 * half, NF_EINVAL,
              "row stride smaller than 2*half");
-  // the workspace from the stream's own pool: given back in stream order
-  hipStream_t s = (hipStream_t)stream;
-  void* workspace = nullptr;
-  hipError_t e = hipMallocAsync(&workspace, (size_t)nf_revmlp_bwd_workspace_bytes(rows, half, blocks), s);
-  if (e != hipSuccess) return fail((int)e, "hipMallocAsync: %s", hipGetErrorString(e));
-  const RevGrads grads = {dw1, db1, dw2, db2, half, 0, 1, NF_F32};
-  const int rc = rev_bwd_call(y, y_stride, dy, dy_stride, dx, dx_stride, x_rec, x_rec_stride, w1, b1, w2, b2, grads, rows, half, blocks, act, dtype,
-                              workspace, s);
-  e = hipFreeAsync(workspace, s);
-  if (rc != 0) return rc;
-  return e == hipSuccess ? 0 : fail((int)e, "hipFreeAsync: %s", hipGetErrorString(e));
+  const RevGrads grads = {dw1, db1, dw2, db2, half, 0, NF_F32};
+  return rev_bwd_call(y, y_stride, dy, dy_stride, dx, dx_stride, x_rec, x_rec_stride, w1, b1, w2, b2, grads, rows, half, blocks, act, dtype, nullptr,
+                      (hipStream_t)stream);
 }

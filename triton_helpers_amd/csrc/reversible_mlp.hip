@@ -15,8 +15,11 @@
 // in mlp_tile.h), which lets a lane reach the eight features of two accumulator tiles with one
 // 16-byte access; the staged weights and the flushed gradients absorb the permutation.
 //
-// Backward of four 64-wide GELU couplings (us; before: sixteen rounds of weight loads and 65536 float atomics per workgroup and coupling):
-// 1600 rows 97 -> 90, 32768 157 -> 108, 100000 220 -> 196, 2^20 unchanged (1.14 ms: the serial issue of one wave per SIMD).
+// Backward of four GELU couplings with slots and laid-out weights (us; before: sixteen rounds of weight loads and 65536 float atomics per
+// workgroup and coupling).  64-wide: 1600 rows 97 -> 90, 32768 157 -> 108, 100000 220 -> 196, 2^20 unchanged (1.1 ms: the serial issue of
+// one wave per SIMD).  32-wide: 32768 rows 89 -> 49, 2^18 172 -> 122, and 2^20, where the atomics had drained behind other work, 488 -> 495
+// (bfloat16) and 494 -> 490 to 513 (float16): the slots' sum and the weights' layout are launches of their own there, in exchange for
+// gradients with the same bits in every run.
 //
 // There is no counterpart in the reference; the layer math is that of its fused MLP
 // (triton_helpers/layers/fully_fused_mlp/kernel.py:17-74).
@@ -449,38 +452,48 @@ __device__ __forceinline__ void put_db(float* slot, int lane, float v) {
   if (lane < 16) slot[lane] = v;
 }
 
-// The slots of all workgroups in a fixed order, to where the gradients belong: 64 pieces of four values per workgroup, sixteen
-// interleaved runs over the slots, then a fixed tree.
+// The slots of all workgroups in a fixed order, to where the gradients belong: SUM_PIECES pieces of four values per workgroup, SUM_RUNS
+// interleaved runs over the slots, then a fixed tree.  With 64 pieces and 16 runs the 32-wide gradients were 17 workgroups per coupling;
+// this is four times as many (four couplings of 256 slots: 32-wide, 17 MB, 9.2 -> 7.1 us; 64-wide, 68 MB, 13.3 -> 12.3 us).
 struct RevGrads {
   void *dw1, *db1, *dw2, *db2;
   int half, n_slots, type;
 };
+constexpr int SUM_PIECES = 16, SUM_RUNS = 64;
 template <int HP>
-__global__ __launch_bounds__(1024) void rev_sum_k(const float* slots, int64_t slot_stride, RevGrads o) {
+__global__ __launch_bounds__(SUM_PIECES* SUM_RUNS) void rev_sum_k(const float* slots, int64_t slot_stride, RevGrads o) {
   typedef RevSlot<HP> S;
-  __shared__ f32x4_t part[16][64];
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6, H = o.half;
-  const int coupling = blockIdx.y, piece = blockIdx.x * 64 + tx;
-  const bool on = piece * 4 < S::FLOATS;
+  static_assert(S::FLOATS % (4 * SUM_PIECES) == 0, "whole workgroups");
+  __shared__ f32x4_t part[SUM_RUNS][SUM_PIECES];
+  const int tx = threadIdx.x % SUM_PIECES, ty = threadIdx.x / SUM_PIECES, H = o.half;
+  const int coupling = blockIdx.y, piece = blockIdx.x * SUM_PIECES + tx;
   const float* src = slots + (int64_t)coupling * S::FLOATS + piece * 4;
   f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (on) {
-    int sl = ty;
-    for (; sl + 48 < o.n_slots; sl += 64) {
-      f32x4_t v[4];
+  int sl = ty;
+  for (; sl + 3 * SUM_RUNS < o.n_slots; sl += 4 * SUM_RUNS) {
+    f32x4_t v[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const f32x4_t*>(src + (int64_t)(sl + 16 * k) * slot_stride);
+    for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const f32x4_t*>(src + (int64_t)(sl + SUM_RUNS * k) * slot_stride);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) sum += v[k];
-    }
-    for (; sl < o.n_slots; sl += 16) sum += *reinterpret_cast<const f32x4_t*>(src + (int64_t)sl * slot_stride);
+    for (int k = 0; k < 4; ++k) sum += v[k];
   }
+  for (; sl < o.n_slots; sl += SUM_RUNS) sum += *reinterpret_cast<const f32x4_t*>(src + (int64_t)sl * slot_stride);
   part[ty][tx] = sum;
   __syncthreads();
-  if (ty != 0 || !on) return;
+  if (threadIdx.x >= 64) return;
+  // the first wave: four lanes of a piece take sixteen runs each
   f32x4_t total = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int q = 0; q < 16; q += 4) total += (part[q][tx] + part[q + 1][tx]) + (part[q + 2][tx] + part[q + 3][tx]);
+  for (int q = 0; q < SUM_RUNS / 4; q += 4) {
+    const int r = ty * (SUM_RUNS / 4) + q;
+    total += (part[r][tx] + part[r + 1][tx]) + (part[r + 2][tx] + part[r + 3][tx]);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    total[r] += __shfl_xor(total[r], 16);
+    total[r] += __shfl_xor(total[r], 32);
+  }
+  if (ty != 0) return;
   auto put = [&](void* base, int64_t at, float v) {
     if (o.type == NF_F32) reinterpret_cast<float*>(base)[at] = v;
     else if (o.type == NF_F16) reinterpret_cast<uint16_t*>(base)[at] = F16::from_f32(v);
@@ -973,7 +986,7 @@ static int rev_bwd(const char* y, int64_t y_stride, const char* dy, int64_t dy_s
   }
   if (workspace == nullptr) return 0;
   grads.n_slots = (int)slot;
-  hipLaunchKernelGGL((rev_sum_k<HP>), dim3((S::FLOATS / 4 + 63) / 64, (unsigned)blocks), dim3(1024), 0, s, slots, slot_stride, grads);
+  hipLaunchKernelGGL((rev_sum_k<HP>), dim3(S::FLOATS / 4 / SUM_PIECES, (unsigned)blocks), dim3(SUM_PIECES * SUM_RUNS), 0, s, slots, slot_stride, grads);
   return check_launch("rev_sum");
 }
 

@@ -118,9 +118,11 @@ int64_t nf_hash_encode_bwd_workspace_bytes(int64_t n_points, const nf_hash_geom*
 /* nf_hash_encode_bwd without the workspace argument, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  The
  * scratch of the sort-and-accumulate kernels is a device array inside the library, NF_HASH_BWD_STATIC_BYTES per GPU,
- * held until the process ends; the call allocates and frees nothing.  Batches whose scratch does not fit take the
- * smaller bit-plane variant where that applies (3-D points, 16-bit gradients: up to about 1.1 M points at L = 16) and
- * are refused with NF_EINVAL beyond that.  All calls on one GPU share the array: calls that overlap in time on one
+ * held until the process ends; the call allocates and frees nothing.  A batch whose scratch does not fit runs as its
+ * largest part that does and a rest, or takes the smaller bit-plane variant where that applies (3-D points, 16-bit
+ * gradients: up to about 1.1 M points at L = 16), and is refused with NF_EINVAL beyond that: with sixteen levels of
+ * 2^19 rows from about 125 000 points with float32 gradients, of 2^14 rows from 1.67 M points with float32 and 3.08 M
+ * with 16-bit ones. All calls on one GPU share the array: calls that overlap in time on one
  * GPU race on it.  The first call on a device resolves the array's address and sets the kernels' LDS attribute (it
  * may load the library's code object): make one warm-up call per device before recording calls into a HIP graph or
  * entering a region that may not touch the runtime's memory management.  Same arguments and results as

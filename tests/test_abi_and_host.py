@@ -48,6 +48,29 @@ def test_library_allocates_and_waits_for_nothing():
     assert not [n for n in names if re.match(rb"hip(Ext)?(Malloc|Free|HostMalloc|HostFree)|hip(Device|Stream|Event)Synchronize|hipStreamWaitEvent", n)]
 
 
+@pytest.mark.parametrize("log2_rows,hi,dtype,n", [(14, 512, 0, 1_048_574), (14, 512, 1, 2_097_148), (19, 7006, 0, 65_424), (19, 7006, 1, 107_256), (21, 7006, 0, 74_478),
+                                                  (21, 7006, 1, 135_063), (16, 1024, 0, 111_733)])
+def test_batches_that_the_static_scratch_serves(log2_rows, hi, dtype, n):
+    """Sixteen levels: batches that the entry point without a workspace has always taken, whole or in two parts, are not refused for
+    want of scratch (the NULL pointers are, behind that), and float32 gradients of four times as many points are."""
+    from triton_helpers_amd import _lib
+    from triton_helpers_amd.layers.hash_encoding.helpers import level_geometry
+
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libnf_cdna4.so not built")
+    lib = _lib.load()
+    geom = level_geometry(2**log2_rows, 16, 3, 2, 16, hi)
+
+    def refused(points):
+        rc = lib.nf_hash_encode_bwd_static(None, 0, 3, 1, None, dtype, 32, None, points, geom, None, 1.0, 0, None)
+        assert rc != 0
+        return b"static scratch holds" in lib.nf_last_error()
+
+    assert not refused(n) and not refused(n - 1) and not refused(n // 2)
+    if dtype == 0:
+        assert refused(4 * n)
+
+
 def test_argument_validation_without_gpu():
     """Entry points validate before touching the device: bad arguments come back as negative codes."""
     from triton_helpers_amd import _lib

@@ -82,3 +82,31 @@ def test_static_scratch_backward_matches_the_workspace_backward():
     # float32 gradients have no bit-plane variant: refused as soon as the records do not fit
     rc, de = _call(lib, L_, True, x[: 2**18], do[: 2**18].float(), E, geom, pi)
     assert rc == L_.NF_EINVAL and not bool(de.any())
+
+
+@pytest.mark.parametrize("n,log2_rows,hi,dtype", [(107_001, 19, 7006, torch.float16), (65_423, 19, 7006, torch.float32), (135_063, 21, 7006, torch.bfloat16),
+                                                  (1_048_573, 14, 512, torch.float32)])
+def test_a_batch_beyond_the_scratch_runs_in_two_parts(n, log2_rows, hi, dtype):
+    from triton_helpers_amd import _lib as L_
+    from triton_helpers_amd.layers.hash_encoding.helpers import level_geometry
+
+    lib = L_.load()
+    geom = level_geometry(2**log2_rows, L, D, F, LO, hi)
+    offs = O.level_row_offsets(L, 2**log2_rows, D, LO, hi)
+    pi = torch.tensor(O.PRIMES, dtype=torch.int64, device=DEV)
+    g = torch.Generator().manual_seed(n)
+    x = torch.rand(n, D, generator=g).to(DEV)
+    do = torch.randn(n, L * F, generator=g).to(dtype).to(DEV)
+    assert lib.nf_hash_encode_bwd_workspace_bytes(n, geom, L_.dtype_code(dtype), 0) > lib.nf_hash_encode_bwd_static_bytes()
+    got = []
+    for static in (True, False):
+        rc, de = _call(lib, L_, static, x, do, offs[-1], geom, pi)
+        assert rc == 0, lib.nf_last_error()
+        got.append(de)
+    # The rest of a batch may go to the atomics, whose weights are exact floats; a record's are off by up to 2^-17 of the gradient, and a row
+    # of the coarsest level has some ten contributions of the rest: 10 * 2^-17 = 8e-5 of gradients about 1, against a level's RMS above 1
+    # there (finer levels: fewer contributions).  Otherwise the same fixed-point sums, rounded to float32 once per part.
+    for l in range(L):
+        a, b = got[0][offs[l]:offs[l + 1]], got[1][offs[l]:offs[l + 1]]
+        rms = float(b.pow(2).mean().sqrt())
+        assert float(((a - b).abs() - 1e-4 * b.abs()).max()) <= 1e-4 * rms, l

@@ -44,22 +44,47 @@ extern "C" int nf_hash_encode_bwd_static(const void* coords, int coords_dtype, i
                                          const nf_hash_geom* geom, const int64_t* primes, float scale, int flags, void* stream) {
   NF_REQUIRE(geom != nullptr, NF_EINVAL, "geom is NULL");
   NF_REQUIRE(n_points >= 0, NF_EINVAL, "n_points negative");
-  // Which variant's scratch fits: the sorted records (fastest, ~1.5 KB per point), else the bit-planes (~110 B per
-  // point, 16-bit gradients of 3-D points only).  A call that would need neither (small batches and shapes that
-  // scatter with atomics) needs no scratch at all.
+  // Which variant's scratch fits: the sorted records (~1.3 KB per point; float32 ~2.1) or the walk without them (~0.1 to 0.2 KB) of the
+  // whole batch; else of its largest part that fits, the rest being a call of its own; else the bit-planes (~110 B per point, 16-bit
+  // gradients of 3-D points only), which also run where the rest would need a second pass of records: 16 levels of 2^19 rows, float16,
+  // 107000 points as 100864 and a rest for the atomics 146 us, with the bit-planes 180; 107000 as two halves 228; 2^14 rows, 2^21 points
+  // 370 us in two parts, with the bit-planes 1620.  A call that would need none of these (small batches and shapes that scatter with
+  // atomics) needs no scratch at all.
   const int64_t limit = (int64_t)NF_HASH_BWD_STATIC_BYTES;
-  const int64_t need_bin = nf_hash_encode_bwd_workspace_bytes(n_points, geom, dout_dtype, flags & ~NF_HASH_FORCE_PLANES);
-  const int64_t need_planes = nf_hash_encode_bwd_workspace_bytes(n_points, geom, dout_dtype, flags | NF_HASH_FORCE_PLANES);
+  auto need_of = [&](int64_t n, int f) { return nf_hash_encode_bwd_workspace_bytes(n, geom, dout_dtype, f); };
+  const int64_t need_bin = need_of(n_points, flags & ~NF_HASH_FORCE_PLANES), need_planes = need_of(n_points, flags | NF_HASH_FORCE_PLANES);
+  int64_t piece = n_points;
   int use_flags = flags;
   if (need_bin > limit || (flags & NF_HASH_FORCE_PLANES)) {
-    NF_REQUIRE(need_planes > 0 && need_planes <= limit, NF_EINVAL,
-               "n_points=%lld needs %lld bytes of scratch (%lld with the bit-plane variant, 0 = not applicable to this call); "
-               "the static scratch holds %lld: split the batch or call nf_hash_encode_bwd with a workspace",
-               (long long)n_points, (long long)need_bin, (long long)need_planes, (long long)limit);
-    use_flags |= NF_HASH_FORCE_PLANES;
+    const bool planes = need_planes > 0 && need_planes <= limit;
+    int64_t part = (n_points + 1) / 2, beyond = n_points;  // part fits, beyond does not
+    bool parts = !(flags & NF_HASH_FORCE_PLANES) && need_of(part, flags) <= limit;
+    while (parts && beyond - part > 1) {
+      const int64_t mid = part + (beyond - part) / 2;
+      (need_of(mid, flags) <= limit ? part : beyond) = mid;
+    }
+    const int64_t rest = n_points - part;
+    parts = parts && need_of(rest, flags) <= limit;
+    if (parts && (!planes || bwd_walk_applies(part, geom, flags) || rest < bwd_records_min(geom, flags))) {
+      piece = part;
+    } else {
+      NF_REQUIRE(planes, NF_EINVAL,
+                 "n_points=%lld needs %lld bytes of scratch (%lld with the bit-plane variant, 0 = not applicable to this call); "
+                 "the static scratch holds %lld: split the batch or call nf_hash_encode_bwd with a workspace",
+                 (long long)n_points, (long long)need_bin, (long long)need_planes, (long long)limit);
+      use_flags |= NF_HASH_FORCE_PLANES;
+    }
   }
   void* ws = nullptr;
   if (int rc = static_scratch(&ws)) return rc;
-  return nf_hash_encode_bwd(coords, coords_dtype, csn, csd, dout, dout_dtype, dout_stride_n, dtable, n_points, geom, primes, scale, ws,
-                            limit, use_flags, stream);
+  int64_t n0 = 0;
+  do {  // (an empty batch too: its arguments are checked)
+    const int64_t n = n_points - n0 < piece ? n_points - n0 : piece;
+    const char* c = (const char*)coords + n0 * csn * (dtype_ok(coords_dtype) ? dtype_size(coords_dtype) : 0);
+    const char* d = (const char*)dout + n0 * dout_stride_n * (dtype_ok(dout_dtype) ? dtype_size(dout_dtype) : 0);
+    if (int rc = nf_hash_encode_bwd(c, coords_dtype, csn, csd, d, dout_dtype, dout_stride_n, dtable, n, geom, primes, scale, ws, limit, use_flags, stream))
+      return rc;
+    n0 += n;
+  } while (n0 < n_points);
+  return 0;
 }

@@ -137,7 +137,11 @@ def test_hash_node_hands_unusual_calls_to_the_python_function(case):
     (2**18, 3, 2, 2**21, 8, 7006, torch.float16, "uniform"),        # wide blocks, ragged and not
     (2**18 + 2049, 3, 2, 2**21, 8, 7006, torch.float32, "corner"),
     (2**18 + 1, 2, 2, 2**21, 8, 7006, torch.bfloat16, "uniform"),
-    (2**18 + 1, 3, 2, 2**21, 16, 7006, torch.float16, "corner"),    # more bins than can be split
+    (2**18 + 1, 3, 2, 2**21, 16, 7006, torch.float16, "corner"),    # more bins than the table of tasks holds
+    (2**18 + 1, 3, 2, 2**21, 16, 7006, torch.float16, "cell"),      # heavy bins behind it, and fewer slots than shares
+    (20001, 3, 1, 2**21, 16, 7006, torch.bfloat16, "cell"),
+    (2**19, 2, 2, 2**22, 16, 30000, torch.float32, "cell"),
+    (150001, 3, 2, 2**23, 8, 4096, torch.float16, "cell"),
 ])
 def test_sorted_backward_writes_the_table(N, dims, F, T, L, hi, dtype, layout, monkeypatch):
     """The backward of the sorted records, added to a float32 table and written in the table's own type: every row against
@@ -181,6 +185,8 @@ def _check_table_gradient(N, dims, F, T, L, hi, dtype, layout, same_bits):
     x = torch.rand(N, dims, generator=g, device=DEV)
     if layout == "corner":
         x[: N // 2] *= 0.05
+    if layout == "cell":
+        x[: N // 2] = 0.4 + 1e-6 * x[: N // 2]
     *first, E = O.level_row_offsets(L, T, dims, 16, hi)
     first = torch.tensor(first, device=DEV).view(1, L, 1)
     do = torch.randn(N, L * F, generator=g, device=DEV).to(dtype)

@@ -63,10 +63,16 @@ constexpr int64_t FILL_WIDE_POINTS = (int64_t)1 << 18;
 constexpr int ACC_THREADS = 1024;
 constexpr int ACC_INFLIGHT = 2;               // records in flight per thread
 constexpr int GROUP = 16;                     // records named by one entry of a task's list
-constexpr int LIST = 6144;                    // entries of the list that LDS holds at a time
+constexpr int LIST = 5824;                    // entries of the list that LDS holds at a time
 constexpr int LIST_PAD = 2 * ACC_THREADS * ACC_INFLIGHT / GROUP;  // empty entries behind it
-constexpr int SPLIT_MAX_BINS = 1536;          // bins that can be split: those of the coarse levels, where points meet
+constexpr int SPLIT_MAX_BINS = 1536;          // bins whose tasks LDS has a table for: those of the coarse levels, where points meet
 constexpr uint32_t SPLIT_MIN_COST = 32768;    // least cost (x-pair records) of a share of a split bin
+// Of the bins behind them only those of LATE_SHARES shares and more are split, listed one by one: all levels together come to 768 shares, and
+// of sixteen levels at most nine are behind, so LATE_MAX takes them (beyond it the shares grow).
+// Points in one cell and in a cube of 0.003, 16 levels of 2^21 rows, fp16 (us; these bins unsplit, this): 2^18 points 1690 and 1110, 800 and 575;
+// 2^20 points 5960 and 1720, 1710 and 1245; uniform points 311 -> 317 and 506 -> 508.
+constexpr uint32_t LATE_SHARES = 2;
+constexpr int LATE_MAX = 256;
 constexpr uint32_t CELL_COST = 4;             // a cell record is sixteen LDS adds against an x-pair record's four
 constexpr int MAX_BINS_PER_LEVEL = 2048;        // 2^24 rows
 struct BinPlan {
@@ -704,9 +710,9 @@ __host__ __device__ __forceinline__ auto with_mode(int mode, Body&& body) {
   }
 }
 
-// TWO: rows of two features, added: a kernel of its own, which the addresses of other rows cost nine registers and 3 us at 2^18 points
-template <typename GT, int MODE, bool TWO = false>
-__global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, void* table, DevGeom g, BinPlan bp, int feat, int f0) {
+// TWO: rows of two features have kernels of their own, which the addresses of other rows cost nine registers and 3 us at 2^18 points
+template <typename GT, int MODE, bool TWO>
+__global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, void* table, DevGeom g, BinPlan bp, int row_feat, int f0) {
   typedef typename BinRec<GT>::type Rec;
   // Fixed-point sums, one plane of BIN_ROWS 64-bit cells per feature: the 64 lanes of an add go to random rows of one
   // feature, and with 8-byte cells those spread over all 64 banks (interleaved features would leave them half).
@@ -715,39 +721,75 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
   uint32_t* first_task = list + LIST + LIST_PAD;                          // [SB + 1] first task of a bin | its first slot << 16
   __shared__ uint32_t next_task[2], wave_sums[ACC_THREADS / 64];
   __shared__ int level_base[NF_MAX_LEVELS];
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, feat = TWO ? 2 : row_feat;
   const int NB = bp.binbase[bp.n_levels];
-  int SB = 0;  // bins of the leading levels, which may be split
+  int SB = 0;  // bins of the leading levels
   for (int l = 0; l < bp.n_levels && bp.binbase[l + 1] <= SPLIT_MAX_BINS; ++l) SB = bp.binbase[l + 1];
+  uint32_t* late = first_task + SB + 1;  // [n_late + 1] heavy bins behind those: bin, its first further share | its first slot << 16
   for (uint32_t i = tid; i < 2u * BIN_ROWS; i += ACC_THREADS) acc_tile[i] = 0ull;
   if (tid < bp.n_levels) level_base[tid] = bp.binbase[tid];
   __syncthreads();
-  // The tasks, worked out by every workgroup for itself: one per bin, several for a bin of more than one and a half shares.
-  uint32_t split_tasks = 0;
-  {
-    uint32_t slots = 0;
+  // The tasks, worked out by every workgroup for itself: one per bin of the leading levels, several for a bin of more than one and a half
+  // shares; the further shares of heavy bins behind those; and one per bin behind them, which takes a heavy bin's first share.  Where
+  // the slots (or the list of heavy bins) do not reach, larger shares.
+  uint32_t split_tasks, late_tasks, n_late;
+  const auto cost_of = [&](int b, int& l) {  // l: a level at or in front of the bin's
+    while (l + 1 < bp.n_levels && b >= level_base[l + 1]) ++l;
+    return ws.totals[b] * (bp.cell[l] ? CELL_COST : 1u);
+  };
+  for (uint32_t share = ws.split_cost;; share += share / 4u) {
+    const auto parts_of = [&](uint32_t cost) { return min((cost + share - 1u) / share, (uint32_t)ws.blocks); };
+    uint32_t slots = 0, total;
+    split_tasks = 0;
     for (int b0 = 0; b0 < SB; b0 += ACC_THREADS) {
       const int b = b0 + tid;
-      uint32_t n = 0, cost = 0;
+      uint32_t n = 0;
       if (b < SB) {
         int l = 0;
-        while (l + 1 < bp.n_levels && b >= level_base[l + 1]) ++l;
-        cost = ws.totals[b] * (bp.cell[l] ? CELL_COST : 1u);
-        n = cost <= ws.split_cost + ws.split_cost / 2 ? 1u : min((cost + ws.split_cost - 1u) / ws.split_cost, (uint32_t)ws.blocks);
+        const uint32_t cost = cost_of(b, l);
+        n = cost <= share + share / 2 ? 1u : parts_of(cost);
         if (cost == 0u && MODE == TABLE_ADD) n = 0u;  // nothing to add (a table that is written gets its zeros)
       }
-      uint32_t total;
       const uint32_t slot = slots + block_exclusive_scan(n > 1u ? n : 0u, wave_sums, &total);
-      if (n > 1u && slot + n > ws.max_slots) n = 1u;  // out of slots: the bin stays one task
       slots += total;
       const uint32_t first = split_tasks + block_exclusive_scan(n, wave_sums, &total);
       split_tasks += total;
       if (b < SB) first_task[b] = first | slot << 16;
-      if (blockIdx.x == 0 && n > 1u) ws.splits[atomicAdd(&ws.header->n_splits, 1u)] = BinSplit{(uint32_t)b, slot, n, 0u};
     }
-    if (tid == 0) first_task[SB] = split_tasks;
+    n_late = late_tasks = 0u;
+    if (SB < NB) {
+      uint32_t heavy = 0, parts = 0;
+      const auto each_heavy = [&](auto&& body) {
+        int l = 0;
+        for (int b = SB + tid; b < NB; b += ACC_THREADS) {
+          const uint32_t cost = cost_of(b, l);
+          if (cost >= LATE_SHARES * ws.split_cost && cost > share + share / 2 && ws.blocks > 1) body(b, parts_of(cost));
+        }
+      };
+      each_heavy([&](int, uint32_t n) {
+        ++heavy;
+        parts += n;
+      });
+      uint32_t at = block_exclusive_scan(heavy, wave_sums, &n_late);
+      uint32_t slot = slots + block_exclusive_scan(parts, wave_sums, &total), first = slot - slots - at;
+      slots += total;
+      late_tasks = total - n_late;
+      if (heavy && n_late <= (uint32_t)LATE_MAX)
+        each_heavy([&](int b, uint32_t n) {
+          late[2u * at] = (uint32_t)b;
+          late[2u * at + 1u] = first | slot << 16;
+          ++at;
+          first += n - 1u;
+          slot += n;
+        });
+    }
+    if (slots <= ws.max_slots && n_late <= (uint32_t)LATE_MAX) break;
   }
-  const uint32_t n_tasks = split_tasks + (uint32_t)(NB - SB);
+  if (tid == 0) {
+    first_task[SB] = split_tasks;
+    late[2u * n_late + 1u] = late_tasks;
+  }
+  const uint32_t n_tasks = split_tasks + late_tasks + (uint32_t)(NB - SB);
   // What a task needs, the same for all threads.
   struct Task {
     int bin, level, block0, block1;
@@ -755,7 +797,14 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
   };
   const int lane = tid & 63;
   auto task_of = [&](uint32_t t) {
-    Task k = {SB + (int)(t - split_tasks), 0, 0, ws.blocks, ~0u};
+    Task k = {SB + (int)(t - split_tasks - late_tasks), 0, 0, ws.blocks, ~0u};
+    // share `which` of n: its blocks, and its slot
+    auto share = [&](uint32_t which, uint32_t n, uint32_t slot) {
+      if (n <= 1u) return;
+      k.slot = slot + which;
+      k.block0 = (int)((int64_t)ws.blocks * which / n);
+      k.block1 = (int)((int64_t)ws.blocks * (which + 1u) / n);
+    };
     if (t < split_tasks) {
       // the bin whose first task is the last one not behind t (a bin without tasks shares it with the one behind it), found
       // in two looks of 64 lanes each
@@ -763,11 +812,21 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
       auto not_behind = [&](int b) { return __builtin_popcountll(__ballot(b < SB && (first_task[b] & 0xffffu) <= t)); };
       const int seg = (not_behind(lane * step) - 1) * step;
       k.bin = seg + not_behind(lane < step ? seg + lane : SB) - 1;
-      const uint32_t at = first_task[k.bin], t0 = at & 0xffffu, n = (first_task[k.bin + 1] & 0xffffu) - t0;
-      if (n > 1u) {
-        k.slot = (at >> 16) + t - t0;
-        k.block0 = (int)((int64_t)ws.blocks * (t - t0) / n);
-        k.block1 = (int)((int64_t)ws.blocks * (t - t0 + 1u) / n);
+      const uint32_t at = first_task[k.bin], t0 = at & 0xffffu;
+      share(t - t0, (first_task[k.bin + 1] & 0xffffu) - t0, at >> 16);
+    } else if (n_late > 0u) {
+      // the heavy bin that a further share belongs to, or the one that the bin of this place is
+      const bool further = t < split_tasks + late_tasks;
+      uint32_t found = 0;
+      for (uint32_t i0 = 0; i0 < n_late; i0 += 64u) {
+        const uint32_t i = i0 + (uint32_t)lane;
+        const uint64_t m = __ballot(i < n_late && (further ? (late[2u * i + 1u] & 0xffffu) <= t - split_tasks : late[2u * i] == (uint32_t)k.bin));
+        found += further ? (uint32_t)__builtin_popcountll(m) : m ? i0 + (uint32_t)__builtin_ctzll(m) + 1u : 0u;
+      }
+      if (found > 0u) {
+        const uint32_t i = found - 1u, at = late[2u * i + 1u], e0 = at & 0xffffu;
+        k.bin = (int)late[2u * i];
+        share(further ? t - split_tasks - e0 + 1u : 0u, (late[2u * i + 3u] & 0xffffu) - e0 + 1u, at >> 16);
       }
     }
     k.level = __builtin_popcountll(__ballot(lane < bp.n_levels && level_base[lane] <= k.bin)) - 1;
@@ -788,7 +847,7 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
     return r;
   };
   // an odd feature count leaves the last pass with one feature: plane 1 then has no column in the table
-  const bool has_pair = f0 + 1 < feat;
+  const bool has_pair = TWO || f0 + 1 < feat;
   // Task numbers come from a counter, fetched a task ahead, and so are the places of the next task's records: neither is waited
   // for.  Every workgroup leaves as soon as the counter has passed the last task.
   if (tid == 0) {
@@ -796,6 +855,13 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
     next_task[1] = atomicAdd(&ws.header->next_task, 1u);
   }
   __syncthreads();
+  if (blockIdx.x == 0) {  // for the kernel behind this one
+    const auto split = [&](uint32_t b, uint32_t slot, uint32_t n) {
+      if (n > 1u) ws.splits[atomicAdd(&ws.header->n_splits, 1u)] = BinSplit{b, slot, n, 0u};
+    };
+    for (int b = tid; b < SB; b += ACC_THREADS) split((uint32_t)b, first_task[b] >> 16, (first_task[b + 1] & 0xffffu) - (first_task[b] & 0xffffu));
+    for (uint32_t i = tid; i < n_late; i += ACC_THREADS) split(late[2u * i], late[2u * i + 1u] >> 16, (late[2u * i + 3u] & 0xffffu) - (late[2u * i + 1u] & 0xffffu) + 1u);
+  }
   uint32_t t = next_task[0], t_next = next_task[1];
   if (t >= n_tasks) return;
   Task task = task_of(t);
@@ -1038,7 +1104,7 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
 #pragma unroll
           for (int u = 0; u < U; ++u) {
             const uint32_t r = r0 + u * ACC_THREADS;
-            if (r < nrows) store_pair<MODE>(table, first + (int64_t)r * feat, x[u], y[u], feat == 2, has_pair);
+            if (r < nrows) store_pair<MODE>(table, first + (int64_t)r * feat, x[u], y[u], TWO, has_pair);
           }
         }
       }
@@ -1664,11 +1730,11 @@ static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_
              : ddt == NF_BF16 ? (const void*)hash_bwd_bin_accum_k<BF16, M, TWO>
                               : (const void*)hash_bwd_bin_accum_k<F32, M, TWO>;
     };
-    return M == TABLE_ADD && feat == 2 ? kernel(std::integral_constant<bool, M == TABLE_ADD>{}) : kernel(std::false_type{});
+    return feat == 2 ? kernel(std::true_type{}) : kernel(std::false_type{});
   });
   const void* reduce = with_mode(mode, [](auto mode_c) { return (const void*)hash_bwd_bin_reduce_k<decltype(mode_c)::value>; });
   const size_t fill_lds = ((size_t)stage_records(D, wide) * (g32 ? 4 : 3) + 3 * (size_t)max_nb + 1 + NF_MAX_LEVELS) * 4;
-  const size_t acc_lds = (size_t)BIN_ROWS * 2 * sizeof(unsigned long long) + ((size_t)LIST + LIST_PAD + (NB < SPLIT_MAX_BINS ? NB : SPLIT_MAX_BINS) + 1) * 4;
+  const size_t acc_lds = (size_t)BIN_ROWS * 2 * sizeof(unsigned long long) + ((size_t)LIST + LIST_PAD + (NB < SPLIT_MAX_BINS ? NB : SPLIT_MAX_BINS) + 1 + (NB > SPLIT_MAX_BINS ? 2 * LATE_MAX : 0) + 2) * 4;
   auto launch = [&](const char* what, const void* kern, dim3 grid, int threads, void** args, size_t lds) { return launch_large(what, kern, grid, threads, args, lds, s); };
   const unsigned units = (unsigned)compute_units();
   // more than three dimensions: the whole pipeline once per corner of the extra coordinates (`hi`), see ExtraDims

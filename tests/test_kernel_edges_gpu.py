@@ -178,6 +178,29 @@ def test_backward_of_small_batches(N, dims, F, dtype):
     _check_table_gradient(N, dims, F, 2**19, 4, 4096, dtype, "uniform", same_bits=False)
 
 
+def test_backward_atomics_of_a_batch_beyond_one_launch():
+    """2^27 + 3 points of four features without a workspace are more threads than a launch has: no point is left out.  Every point's
+    weights sum to one, so a gradient of ones sums to the points; 8 * 2^27 / 2^19 = 2048 adds of about 1/8 per row are off by at most
+    2048 * 2^-24 of a row's 256."""
+    from triton_helpers_amd import _lib as L_
+    from triton_helpers_amd.layers.hash_encoding.helpers import level_geometry
+
+    lib, n, T = L_.load(), 2**27 + 3, 2**19
+    geom = level_geometry(T, 2, 3, 4, 1000, 2000)
+    x = torch.rand(n, 3, device=DEV)
+    do = torch.ones(n, 8, device=DEV, dtype=torch.float16)
+    do[:, 4:] = 0
+    do[-1, :4] = 4096.0
+    x[-1] = 0.0  # the last point's weights are all on its first corner
+    de = torch.zeros(2 * T, 4, device=DEV)
+    pi = torch.tensor(O.PRIMES, dtype=torch.int64, device=DEV)
+    rc = lib.nf_hash_encode_bwd(x.data_ptr(), 0, 3, 1, do.data_ptr(), L_.NF_F16, 8, de.data_ptr(), n, geom, pi.data_ptr(), 1.0, None, 0, 0, L_.current_stream(x.device))
+    assert rc == 0, lib.nf_last_error()
+    total = de[:T].double().sum(0)
+    assert not de[T:].any() and float((total - (n - 1 + 4096)).abs().max()) <= 2048 * 2**-24 * n
+    assert float(de[0].min()) > 4096.0
+
+
 def _check_table_gradient(N, dims, F, T, L, hi, dtype, layout, same_bits):
     from triton_helpers_amd.layers.hash_encoding import kernel as hk
 

@@ -1048,11 +1048,18 @@ extern "C" int nf_hash_encode_bwd(const void* coords, int coords_dtype, int64_t 
                          : (g.dims == 3 ? (const void*)hash_bwd_level_k<GT, 3, 4> : (const void*)hash_bwd_level_k<GT, 2, 4>);
     };
     const void* kern = dout_dtype == NF_F32 ? pick(F32{}) : dout_dtype == NF_F16 ? pick(F16{}) : pick(BF16{});
-    const int64_t lanes = n_points * (g.feat << g.dims);
-    dim3 grid((unsigned)((lanes + TILE_THREADS - 1) / TILE_THREADS), (unsigned)g.levels);
-    void* args[] = {&coords, &coords_dtype, &csn, &csd, &dout, &dout_stride_n, &dtable, &n_points, &g, &primes, &scale};
-    const hipError_t e = hipLaunchKernel(kern, grid, dim3(TILE_THREADS), args, 0, s);
-    if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(hash_bwd_level): %s", hipGetErrorString(e));
+    // a launch has less than 2^32 threads: parts of 2^26 points, which with 32 lanes each are 2^31
+    constexpr int64_t part = (int64_t)1 << 26;
+    for (int64_t n0 = 0; n0 < n_points; n0 += part) {
+      int64_t n = n_points - n0 < part ? n_points - n0 : part;
+      const void* c = (const char*)coords + n0 * csn * dtype_size(coords_dtype);
+      const void* d = (const char*)dout + n0 * dout_stride_n * dtype_size(dout_dtype);
+      const int64_t lanes = n * (g.feat << g.dims);
+      dim3 grid((unsigned)((lanes + TILE_THREADS - 1) / TILE_THREADS), (unsigned)g.levels);
+      void* args[] = {&c, &coords_dtype, &csn, &csd, &d, &dout_stride_n, &dtable, &n, &g, &primes, &scale};
+      const hipError_t e = hipLaunchKernel(kern, grid, dim3(TILE_THREADS), args, 0, s);
+      if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(hash_bwd_level): %s", hipGetErrorString(e));
+    }
     return check_launch("hash_bwd_level");
   }
   dim3 grid((unsigned)((n_points + 255) / 256), (unsigned)g.levels);

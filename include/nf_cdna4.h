@@ -98,19 +98,23 @@ int nf_hash_encode_bwd(const void* coords, int coords_dtype, int64_t coords_stri
 
 /* The gradient of the whole table in one go: every row of the geometry's levels is WRITTEN, in table_dtype, with the sum over
  * all points (rounded once from float32; rows that no point touches get zero) -- nothing to clear before the call and
- * nothing to cast after it.  The sums are added in a fixed order: the same inputs give the same bits.  Runs on the sorted-record
- * kernels only (D = 2 or 3, batches of 8192 to 2^21 points, rows that they take) and needs the workspace of
- * nf_hash_encode_bwd_workspace_bytes(); NF_EUNSUPPORTED otherwise, before anything is launched.  (The reference clears and adds
+ * nothing to cast after it.  The sums are added in a fixed order: the same inputs give the same bits.  Runs where one pass over the
+ * points leaves every row's sum in one place: the sorted records (D = 2 or 3, from 8192 points, 16384 where the atomics take smaller
+ * batches) and the walk without records (D = 1 to 4; levels of at most 2^14 rows from 4096 points, other small tables from 6144 per
+ * feature pair, shapes outside the atomics from 1024), up to 2^21 points, rows that start on 4-byte (float32: 8-byte) boundaries; needs the
+ * workspace of nf_hash_encode_bwd_workspace_bytes(), 16-byte aligned; NF_EUNSUPPORTED otherwise, before anything is launched. (The reference clears and adds
  * in the table's type, triton_helpers/layers/hash_encoding/kernel.py:636.) */
 int nf_hash_encode_bwd_write(const void* coords, int coords_dtype, int64_t coords_stride_n, int64_t coords_stride_d,
                              const void* dout, int dout_dtype, int64_t dout_stride_n, void* dtable, int table_dtype,
                              int64_t n_points, const nf_hash_geom* geom, const int64_t* primes, float scale, void* workspace,
                              int64_t workspace_bytes, int flags, void* stream);
 
-/* Scratch bytes nf_hash_encode_bwd can use for this call shape and these flags (NF_HASH_FORCE_PLANES gives the
- * size of the smaller variant; tables of at most 2^14 rows per level take a walk without records and ask for
- * 4 bytes -- 8 with a float32 gradient -- per point, level and feature pair unless NF_HASH_BWD_RECORDS is set);
- * 0 when the workspace would not be used.
+/* Scratch bytes nf_hash_encode_bwd can use for this call shape and these flags; 0 when the workspace would not be used.
+ * Sorted records: room for two records of 12 bytes (float32 gradients: 16) per point, level and corner pair (cells of dense 3-D levels: two
+ * per point and level), 2 bytes per bin and block of 512 or 2048 points, and a 64 KiB slot per 1024 points for bins cut into tasks: 1.38 GB for 2^20
+ * points on 16 levels of 2^19 rows (float32: 2.22 GB).  The walk without records (NF_HASH_BWD_RECORDS switches it off): 4 bytes -- 8 with a
+ * float32 gradient -- per point, level and feature pair, 4 per coordinate, and 128 KiB per task where the points are cut into slices.
+ * NF_HASH_FORCE_PLANES gives the size of the smaller bit-plane variant.
  * (No counterpart in the reference: its backward allocates nothing besides the gradient table,
  * triton_helpers/layers/hash_encoding/kernel.py:636.) */
 int64_t nf_hash_encode_bwd_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags);

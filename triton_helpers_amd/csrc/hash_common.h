@@ -200,7 +200,6 @@ int launch_bwd_scan(const void* coords, int cdt, int64_t csn, int64_t csd, const
 
 // backward by binning the contributions per table stretch (hash_encoding_bwd_bin.hip)
 int64_t bwd_bin_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags);
-// whether launch_bwd_bin would walk the points without records (small tables; also for batches too small for the records)
 // two or three dimensions, hashed levels of a power of two of rows: a corner's row takes a few 32-bit instructions
 inline bool quick_rows(const nf_hash_geom* g) {
   for (int l = g->first_hash_level < 0 ? 0 : g->first_hash_level; l < g->levels; ++l)
@@ -212,6 +211,7 @@ inline bool bwd_level_ok(const nf_hash_geom* g) { return quick_rows(g) && (g->fe
 // Batches from which the sorted records run: their fixed cost is about 90 us, the atomics' 5 ns per point (and 20 us for the table's
 // zeros and rounding) or, where no kernel but the generic one has them, 13 ns.
 inline int64_t bwd_records_min(const nf_hash_geom* g, int flags) { return bwd_level_ok(g) && !(flags & NF_HASH_BWD_RECORDS) ? 16384 : 8192; }
+// whether launch_bwd_bin would walk the points without records (small tables; also for batches too small for the records)
 bool bwd_walk_applies(int64_t n_points, const nf_hash_geom* geom, int flags);
 int launch_bwd_bin(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
                    float* dtable, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,

@@ -1036,7 +1036,7 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
     // the tile to the table (or the task's slot), and back to zero for the next task
     const float qnan = __uint_as_float(0x7fc00000u);
     const int64_t first = (g.row_offset[l] + (int64_t)row0) * feat + f0;  // features f0, f0 + 1 of the bin's rows
-    // |a| < 2^48 and its quotient by 2^se are exact in double: one rounding, to float, at the end
+    // |a| <= 2^30 * 2^21 points < 2^53, exact in double, and so is its quotient by 2^se: one rounding, to float, at the end
     const double unscale = ldexp(1.0, -se), unscale_hi = ldexp(1.0, 32 - se);
     auto value = [&](uint32_t i) {
       const long long a = (long long)acc_tile[i];

@@ -14,7 +14,7 @@
 namespace nf {
 
 // ---------------------------------------------------------------------------
-// Generic path: one thread per (point, level); any D <= 4, any F, any dtype mix.
+// Generic path: one thread per (point, level); any D <= 6, any F, any dtype mix.
 // ---------------------------------------------------------------------------
 template <int D>
 __device__ __forceinline__ Cell<D> locate(const void* coords, int cdt, int64_t sn, int64_t sd, int64_t n, float scale,

@@ -1,4 +1,5 @@
-// Hash-encoding backward by binning (D = 2 or 3; features taken two at a time, the last one alone when their number is odd).
+// Hash-encoding backward by binning (D = 2 or 3, and 4 to 6 as passes of the 3-D pipeline; features taken two at a time, the last
+// one alone when their number is odd), and the walk without records for small tables and batches.
 //
 // Every (point, level, corner) contributes  w * dout[n, 2l .. 2l+1]  to one table row.  Scattering these with
 // global atomics is bound by the chip's atomic request rate; accumulating them in LDS needs the contributions to
@@ -1504,7 +1505,7 @@ static int64_t bin_ws(void* workspace, const BinPlan& bp, int64_t N, int points,
 }
 
 // Batches above this many points go through the pipeline in pieces of this size, one after the other on the stream:
-// the scratch stays at ~3 GiB (4 GiB with a float32 upstream gradient) whatever the batch, and record positions stay
+// the scratch stays at 2.8 GB (4.4 GB with a float32 upstream gradient) whatever the batch, and record positions stay
 // inside 32 bits.  The gradient table accumulates across the pieces.  (Pieces of 2^20 points would halve the scratch
 // and cost 2.5 % of a 2^21-point training step: every piece pays the fixed part of the pipeline again.)
 constexpr int64_t BIN_CHUNK_POINTS = (int64_t)1 << 21;
@@ -1518,7 +1519,7 @@ constexpr int64_t BIN_CHUNK_POINTS = (int64_t)1 << 21;
 // quicker, where they apply: 2^16 rows 4096 points 19 and 31, 8192 points 38 and 35, in every feature pair.
 constexpr int WALK_FREE_BINS = 2, WALK_MAX_BINS = 256;
 constexpr int64_t WALK_MAX_POINT_BINS = (int64_t)13 << 19;
-constexpr int WALK_MAX_DIMS = 4;  // the walk is built for 1 to 4 dimensions (the sorted records for 2 and 3)
+constexpr int WALK_MAX_DIMS = 4;  // the walk is built for 1 to 4 dimensions (the sorted records for 2 to 6)
 constexpr int64_t WALK_MIN_POINTS = 6144, WALK_MIN_POINTS_FREE = 4096, WALK_MIN_POINTS_GENERIC = 1024;
 static bool walk_ok(int64_t n_points, const nf_hash_geom* geom, int flags) {
   if (flags & NF_HASH_BWD_RECORDS) return false;

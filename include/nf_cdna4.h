@@ -238,6 +238,18 @@ int nf_mlp_bwd_summed(const void* x, int64_t x_stride, const void* dy, int64_t d
                       void* db_out, int64_t rows, int d_in, int d_hidden, int d_out, int depth, int act, int dtype,
                       int x_dtype, int grad_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The backward of a whole network of one to nine hidden layers (depth 1 .. 9) in one launch: any activation, every width of
+ * nf_mlp_fwd, rows of any alignment, x stored in either 16-bit type (dx comes back in x_dtype).  The dw_ / db_ buffers are
+ * written as nf_mlp_bwd_summed writes them, in grad_dtype (`dtype` or NF_F32): the workgroups' sums added in a fixed order.
+ * NF_EUNSUPPORTED, before anything is launched: float32 tensors, deeper networks, no rows.  workspace: 16-byte aligned,
+ * nf_mlp_bwd_whole_workspace_bytes() bytes of scratch (0: not covered). */
+int nf_mlp_bwd_whole(const void* x, int64_t x_stride, const void* dy, int64_t dy_stride, void* dx, int64_t dx_stride,
+                     const void* w_in, const void* b_in, const void* w_hid, const void* b_hid, const void* w_out,
+                     const void* b_out, void* dw_in, void* db_in, void* dw_hid, void* db_hid, void* dw_out,
+                     void* db_out, int64_t rows, int d_in, int d_hidden, int d_out, int depth, int act, int dtype,
+                     int x_dtype, int grad_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+int64_t nf_mlp_bwd_whole_workspace_bytes(int64_t rows, int d_hidden, int depth, int act, int dtype);
+
 /* n (<= 8) float32 arrays of count[k] values cast to float16 in one launch: piece k starts at dst plus the counts before it,
  * each rounded up to a multiple of 8. src and count are host arrays. */
 int nf_cast_pieces_f16(const float* const* src, const int64_t* count, int n, void* dst, void* stream);

@@ -49,6 +49,8 @@ EXPORTS = (
     "nf_mlp_bwd_rounded",
     "nf_mlp_bwd_rounded_workspace_bytes",
     "nf_mlp_bwd_summed",
+    "nf_mlp_bwd_whole",
+    "nf_mlp_bwd_whole_workspace_bytes",
     "nf_cast_pieces_f16",
     "nf_revmlp_fwd",
     "nf_revmlp_bwd",
@@ -118,6 +120,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.nf_mlp_bwd_rounded.argtypes = [P, I64, P, I64, P, I64, P, P, P, P, P, P, P, P, P, P, P, P, I64, I, I, I, I, I, I, I, P, I64, P]
     lib.nf_mlp_bwd_summed.restype = c_int
     lib.nf_mlp_bwd_summed.argtypes = [P, I64, P, I64, P, I64, P, P, P, P, P, P, P, P, P, P, P, P, I64, I, I, I, I, I, I, I, I, P, I64, P]
+    lib.nf_mlp_bwd_whole.restype = c_int
+    lib.nf_mlp_bwd_whole.argtypes = lib.nf_mlp_bwd_summed.argtypes
+    lib.nf_mlp_bwd_whole_workspace_bytes.restype = I64
+    lib.nf_mlp_bwd_whole_workspace_bytes.argtypes = [I64, I, I, I, I]
     lib.nf_mlp_bwd_rounded_workspace_bytes.restype = I64
     lib.nf_mlp_bwd_rounded_workspace_bytes.argtypes = [I, I, I]
     lib.nf_mlp_workspace_bytes.restype = I64

@@ -40,7 +40,7 @@ COMMON_FLAGS = [
 NO_CONTRACT = {"hash_encoding.hip", "hash_encoding_bwd_scan.hip", "hash_encoding_bwd_bin.hip", "hash_encoding_bwd_static.hip", "hash_check_host.hip"}
 # Files whose MFMA results feed vector ALU work directly: keep them in architectural VGPRs instead of
 # bouncing every result through an accumulation register.
-MFMA_VGPR_FORM = {"fused_mlp.hip", "fused_mlp_bwd2.hip", "fused_mlp_bwdn.hip", "fused_mlp_bwd2_w8.hip", "fused_mlp_bwd2_ws.hip", "fused_mlp_fwd2.hip", "reversible_mlp.hip"}
+MFMA_VGPR_FORM = {"fused_mlp.hip", "fused_mlp_bwd2.hip", "fused_mlp_bwdn.hip", "fused_mlp_bwd2_w8.hip", "fused_mlp_bwd2_ws.hip", "fused_mlp_bwd_roles.hip", "fused_mlp_fwd2.hip", "reversible_mlp.hip"}
 # Kernels at the edge of the register file that must not spill: a version of this one that spilled some was compiled wrong
 # (the high half of its 64-bit row counter was set aside in an accumulation register and never read back).
 NO_SPILL = {"reversible_mlp.hip": "rev_bwd_block_k"}

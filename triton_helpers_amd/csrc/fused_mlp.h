@@ -26,6 +26,9 @@ struct MlpArgs {
   // ([dw_in | dw_hid | dw_out | db_in | db_hid | db_out], float32) instead of adding them to dw_* / db_*
   float* partials;
   int64_t partial_stride;
+  // whole-network backward only: bit l set = the pre-activations that linear layer l gives are rounded to 16 bit, as where
+  // nf_mlp_bwd hands them from one launch to the next
+  uint32_t handover;
 };
 
 constexpr int FRAG_ELEMS = 64 * 8;  // 16-bit elements per fragment (1 KiB)
@@ -148,6 +151,12 @@ int launch_mlp_bwd2_w8_rounded(const MlpArgs& a, int dtype, int grad_dtype, void
 // One hidden layer, width 64, ReLU, with d_in > 32 or d_out > 16 (aligned rows, extents below 2^31 bytes): chain and
 // gradient waves (fused_mlp_bwd2_ws.hip).  *handled = false: not such a call, nothing was launched.
 int launch_mlp_bwd2_ws(const MlpArgs& a, int dtype, hipStream_t s, bool* handled, int* blocks_out = nullptr);
+
+// A whole network of up to nine hidden layers in one launch, any activation, widths and row alignment (fused_mlp_bwd_roles.hip);
+// gradients written to out[6] (dw_in, db_in, dw_hid, db_hid, dw_out, db_out; NULL entries skipped) in grad_dtype.  The workspace
+// holds mlp_bwd_roles_bytes() (0: too deep).
+size_t mlp_bwd_roles_bytes(int64_t rows, int d_hidden, int depth, int act);
+int launch_mlp_bwd_roles(const MlpArgs& a, int dtype, int grad_dtype, void* const out[6], void* workspace, hipStream_t s);
 
 // The forward of one-hidden-layer ReLU networks of width 64 with aligned rows (fused_mlp_fwd2.hip).  *handled = false: not that shape, nothing was launched.
 int launch_mlp_fwd2(const MlpArgs& a, int dtype, hipStream_t s, bool* handled);

@@ -957,3 +957,36 @@ extern "C" int nf_mlp_bwd_rounded(const void* x, int64_t x_stride, const void* d
   return nf_mlp_bwd_summed(x, x_stride, dy, dy_stride, dx, dx_stride, w_in, b_in, w_hid, b_hid, w_out, b_out, dw_in, db_in, dw_hid, db_hid, dw_out,
                            db_out, rows, d_in, d_hidden, d_out, depth, act, dtype, x_dtype, dtype, workspace, workspace_bytes, stream);
 }
+
+extern "C" int64_t nf_mlp_bwd_whole_workspace_bytes(int64_t rows, int d_hidden, int depth, int act, int dtype) {
+  if (d_hidden < 16 || d_hidden > 64 || (dtype != NF_F16 && dtype != NF_BF16)) return 0;
+  return (int64_t)mlp_bwd_roles_bytes(rows, d_hidden, depth, act);
+}
+
+extern "C" int nf_mlp_bwd_whole(const void* x, int64_t x_stride, const void* dy, int64_t dy_stride, void* dx, int64_t dx_stride, const void* w_in,
+                                const void* b_in, const void* w_hid, const void* b_hid, const void* w_out, const void* b_out, void* dw_in,
+                                void* db_in, void* dw_hid, void* db_hid, void* dw_out, void* db_out, int64_t rows, int d_in, int d_hidden,
+                                int d_out, int depth, int act, int dtype, int x_dtype, int grad_dtype, void* workspace,
+                                int64_t workspace_bytes, void* stream) {
+  if (int rc = validate(rows, d_in, d_hidden, d_out, depth, act, dtype)) return rc;
+  NF_REQUIRE(dtype != NF_F32 && (x_dtype == NF_F16 || x_dtype == NF_BF16), NF_EUNSUPPORTED, "whole backward: 16-bit tensors only (dtype code %d, x_dtype code %d)",
+             dtype, x_dtype);
+  NF_REQUIRE(grad_dtype == dtype || grad_dtype == NF_F32, NF_EINVAL, "grad_dtype code %d: the parameters' (%d) or float32", grad_dtype, dtype);
+  const int64_t need = nf_mlp_bwd_whole_workspace_bytes(rows, d_hidden, depth, act, dtype);
+  NF_REQUIRE(need > 0, NF_EUNSUPPORTED, "whole backward: one to nine hidden layers and at least one row (depth %d, %lld rows)", depth, (long long)rows);
+  NF_REQUIRE(x && dy && w_in && w_out && dw_in && dw_out && (depth == 1 || (w_hid && dw_hid)), NF_EINVAL, "NULL pointer argument");
+  NF_REQUIRE(x_stride >= d_in && dy_stride >= d_out && (dx == nullptr || dx_stride >= d_in), NF_EINVAL, "row stride smaller than row width");
+  NF_REQUIRE(workspace != nullptr && workspace_bytes >= need && (uintptr_t)workspace % 16 == 0, NF_EINVAL,
+             "whole backward needs a 16-byte aligned workspace of %lld bytes (nf_mlp_bwd_whole_workspace_bytes)", (long long)need);
+  MlpArgs a = {};
+  a.w_in = (const uint16_t*)w_in; a.b_in = (const uint16_t*)b_in; a.w_hid = (const uint16_t*)w_hid;
+  a.b_hid = (const uint16_t*)b_hid; a.w_out = (const uint16_t*)w_out; a.b_out = (const uint16_t*)b_out;
+  a.rows = rows; a.d_in = d_in; a.d_hidden = d_hidden; a.d_out = d_out; a.depth = depth; a.act = act;
+  a.in_act = NF_ACT_NONE;
+  a.x_conv = x_dtype == dtype ? 0 : (x_dtype == NF_F16 ? 1 : 2);
+  set_rows(a, (const uint16_t*)x, x_stride, nullptr, 0, (const uint16_t*)dy, dy_stride, (uint16_t*)dx, dx_stride);
+  const std::vector<int> first = plan_launches(depth + 1, bwd_max_linear(d_hidden, act));
+  for (size_t k = 1; k + 1 < first.size(); ++k) a.handover |= 1u << (first[k] - 1);
+  void* const out[6] = {dw_in, db_in, depth > 1 ? dw_hid : nullptr, depth > 1 ? db_hid : nullptr, dw_out, db_out};
+  return launch_mlp_bwd_roles(a, dtype, grad_dtype, out, workspace, (hipStream_t)stream);
+}

@@ -309,6 +309,38 @@ __device__ __forceinline__ Frag load_rows_frag(const uint16_t* base, int64_t str
   return f;
 }
 
+// A lane's eight consecutive features 32 kc + 8 g .. + 7 (natural order: one 16-byte access of a row) <-> its two runs of four
+// 32 kc + 4 g .. and 32 kc + 16 + 4 g .. (chain order), by swapping register halves between the lane groups: with a_g, b_g
+// the halves that group g holds, natural (a0 a1 a2 a3 | b0 b1 b2 b3) -> chain (a0 b0 a1 b1 | a2 b2 a3 b3).  Four instructions;
+// what a product sums stays in chain order bit for bit, and rows move 16 bytes per lane: a tile access has no two
+// neighbouring lanes on one line, so the L1 takes every lane as an access of its own, whatever its width.
+__device__ __forceinline__ void swap_groups16(uint32_t& x, uint32_t& y) {  // odd groups of x <-> even groups of y
+  const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+  x = r[0];
+  y = r[1];
+}
+__device__ __forceinline__ void swap_groups32(uint32_t& x, uint32_t& y) {  // groups 2, 3 of x <-> groups 0, 1 of y
+  const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+  x = r[0];
+  y = r[1];
+}
+__device__ __forceinline__ Frag nat_to_chain(Frag f) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    swap_groups16(f.w[i], f.w[2 + i]);
+    swap_groups32(f.w[i], f.w[2 + i]);
+  }
+  return f;
+}
+__device__ __forceinline__ Frag chain_to_nat(Frag f) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    swap_groups32(f.w[i], f.w[2 + i]);
+    swap_groups16(f.w[i], f.w[2 + i]);
+  }
+  return f;
+}
+
 // Store accumulator tile mt (lane (n,g): features 16*mt + 4*g + r) of 16 rows as 16-bit values.
 template <typename T>
 __device__ __forceinline__ void store_rows_tile(uint16_t* base, int64_t stride, int64_t row0, int64_t rows, int width,

@@ -120,6 +120,7 @@ __device__ __forceinline__ Frag load_chain(const uint16_t* base, int64_t stride,
 // the hardware answers reads past the tensor's end with zero and drops such stores, so ragged last chunks need no
 // predicates.  Pieces that lie beyond the row's width get an offset that stays past the end (OUT_OF_RANGE).
 typedef unsigned int buf_v2u __attribute__((ext_vector_type(2)));
+typedef unsigned int buf_v4u __attribute__((ext_vector_type(4)));
 constexpr uint32_t OUT_OF_RANGE = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* base, int64_t rows, int64_t stride) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)(rows * stride * 2), 0x00020000);

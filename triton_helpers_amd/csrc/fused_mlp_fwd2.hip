@@ -22,7 +22,12 @@ namespace nf {
 // eight for the 64-wide inputs / outputs.
 constexpr int fwd2_waves(int kin, int outp) { return (kin == 32 && outp == 16) ? NF_FWD2_WAVES : 8; }
 
-template <typename T, int XC, int KIN = 32, int OUTP = 16>
+// XW / YW: rows of x / y move in whole 16-byte pieces (16-byte aligned rows of a multiple of eight values) that are exchanged
+// between the lane groups, instead of 8-byte pieces.  A tile access has no two neighbouring lanes on one line and the L1 takes
+// a lane a clock, so 8-byte pieces are 64 clocks per 512 bytes: 30 of the 34 us that 64 -> 64 -> 64 -> 64 took at 2^19 rows, 25 now
+// (2^20 rows 59 -> 47, 32 -> 64 -> 64 -> 64 41 -> 36, 64 -> 64 -> 64 -> 16 36 -> 30).  The decoder shape moves a third of that and is
+// held by memory (2^20 rows 21 us either way): 8-byte pieces there.
+template <typename T, int XC, int KIN, int OUTP, bool XW, bool YW>
 __global__ __launch_bounds__(64 * fwd2_waves(KIN, OUTP)) void mlp_fwd2_k(MlpArgs a) {
   constexpr int HP = 64, NT = 2, WAVES = fwd2_waves(KIN, OUTP);
   constexpr int KC_IN = KIN / 32, KC_H = HP / 32, MT_H = HP / 16, MT_O = OUTP / 16;
@@ -38,12 +43,20 @@ __global__ __launch_bounds__(64 * fwd2_waves(KIN, OUTP)) void mlp_fwd2_k(MlpArgs
 #pragma unroll
   for (int kc = 0; kc < KC_IN; ++kc)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) off_x[kc][h] = piece_offset(lane & 15, 32 * kc + 16 * h + 4 * (lane >> 4), a.d_in, a.x_stride);
+    for (int h = 0; h < 2; ++h) off_x[kc][h] = piece_offset(lane & 15, XW ? 32 * kc + 8 * (lane >> 4) : 32 * kc + 16 * h + 4 * (lane >> 4), a.d_in, a.x_stride);
   uint32_t off_y[MT_O];
 #pragma unroll
-  for (int mt = 0; mt < MT_O; ++mt) off_y[mt] = piece_offset(lane & 15, 16 * mt + 4 * (lane >> 4), a.d_out, a.y_stride);
-  auto load_x = [&](int64_t chunk, int nt, int kc) {
+  for (int mt = 0; mt < MT_O; ++mt) {
+    if (YW && MT_O > 1) off_y[mt] = piece_offset(lane & 15, 32 * (mt >> 1) + 8 * (lane >> 4), a.d_out, a.y_stride);
+    else off_y[mt] = piece_offset(lane & 15, 16 * mt + 4 * (lane >> 4), a.d_out, a.y_stride);
+  }
+  auto load_x = [&](int64_t chunk, int nt, int kc) {  // XW: in natural order until it is used
     const uint32_t at = (uint32_t)((chunk * ROWS + 16 * nt) * a.x_stride * 2);
+    if constexpr (XW) {
+      Frag f;
+      f.u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs_x, off_x[kc][0] + at, 0, 0));
+      return f;
+    }
     const buf_v2u lo = __builtin_amdgcn_raw_buffer_load_b64(rs_x, off_x[kc][0] + at, 0, 0);
     const buf_v2u hi = __builtin_amdgcn_raw_buffer_load_b64(rs_x, off_x[kc][1] + at, 0, 0);
     Frag f;
@@ -83,6 +96,7 @@ __global__ __launch_bounds__(64 * fwd2_waves(KIN, OUTP)) void mlp_fwd2_k(MlpArgs
 #pragma unroll
       for (int kc = 0; kc < KC_IN; ++kc) {
         in[nt][kc] = XC == 0 ? nx[nt][kc] : convert_frag(nx[nt][kc], XC);
+        if constexpr (XW) in[nt][kc] = nat_to_chain(in[nt][kc]);
         if constexpr (DEEP) {
           nx[nt][kc] = nnx[nt][kc];
           nnx[nt][kc] = load_x(chunk + 2 * wave_stride, nt, kc);
@@ -107,15 +121,35 @@ __global__ __launch_bounds__(64 * fwd2_waves(KIN, OUTP)) void mlp_fwd2_k(MlpArgs
         h[nt][mt >> 1].w[2 * (mt & 1) + 1] = relu_pk(pack2<T>(acc[nt][mt][2], acc[nt][mt][3]));
       }
     layer_nt<T, NT, MT_O, KC_H, 1>(acc, h, f_out, bias_out, lane);
+    uint32_t out[NT][MT_O][2];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int mt = 0; mt < MT_O; ++mt) {
-        buf_v2u o;
-        o[0] = pack2<T>(acc[nt][mt][0], acc[nt][mt][1]);
-        o[1] = pack2<T>(acc[nt][mt][2], acc[nt][mt][3]);
-        __builtin_amdgcn_raw_buffer_store_b64(o, rs_y, off_y[mt] + (uint32_t)((chunk * ROWS + 16 * nt) * a.y_stride * 2), 0, 0);
+        out[nt][mt][0] = pack2<T>(acc[nt][mt][0], acc[nt][mt][1]);
+        out[nt][mt][1] = pack2<T>(acc[nt][mt][2], acc[nt][mt][3]);
       }
+    auto at = [&](int nt) { return (uint32_t)((chunk * ROWS + 16 * nt) * a.y_stride * 2); };
+    if constexpr (YW && MT_O > 1) {
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT_O; mt += 2) {
+          Frag f;
+          f.w[0] = out[nt][mt][0]; f.w[1] = out[nt][mt][1]; f.w[2] = out[nt][mt + 1][0]; f.w[3] = out[nt][mt + 1][1];
+          f = chain_to_nat(f);
+          const buf_v4u o = {f.w[0], f.w[1], f.w[2], f.w[3]};
+          __builtin_amdgcn_raw_buffer_store_b128(o, rs_y, off_y[mt] + at(nt), 0, 0);
+        }
+    } else {
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT_O; ++mt) {
+          const buf_v2u o = {out[nt][mt][0], out[nt][mt][1]};
+          __builtin_amdgcn_raw_buffer_store_b64(o, rs_y, off_y[mt] + at(nt), 0, 0);
+        }
+    }
   }
 }
 
@@ -130,7 +164,13 @@ static int launch_fwd2(const MlpArgs& a0, hipStream_t s) {
   const int64_t cap = (int64_t)device_cus() * NF_FWD2_WG_PER_CU;
   if (blocks > cap) blocks = cap;
   constexpr int XC_OTHER = T::code == NF_BF16 ? 1 : 2;
-  const void* kern = a.x_conv == 0 ? (const void*)mlp_fwd2_k<T, 0, KIN, OUTP> : (const void*)mlp_fwd2_k<T, XC_OTHER, KIN, OUTP>;
+  const bool same = a.x_conv == 0;
+  const void* kern = same ? (const void*)mlp_fwd2_k<T, 0, KIN, OUTP, false, false> : (const void*)mlp_fwd2_k<T, XC_OTHER, KIN, OUTP, false, false>;
+  if constexpr (KIN > 32 || OUTP > 16) {
+    const bool xw = vec_load_ok(a.x, a.x_stride, a.d_in), yw = xw && OUTP > 16 && vec_load_ok(a.y, a.y_stride, a.d_out);
+    if (yw) kern = same ? (const void*)mlp_fwd2_k<T, 0, KIN, OUTP, true, OUTP != 16> : (const void*)mlp_fwd2_k<T, XC_OTHER, KIN, OUTP, true, OUTP != 16>;
+    else if (xw) kern = same ? (const void*)mlp_fwd2_k<T, 0, KIN, OUTP, true, false> : (const void*)mlp_fwd2_k<T, XC_OTHER, KIN, OUTP, true, false>;
+  }
   void* args[] = {(void*)&a};
   const hipError_t e = hipLaunchKernel(kern, dim3((unsigned)blocks), dim3(64 * WAVES), args, LDS, s);
   if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(mlp_fwd2): %s", hipGetErrorString(e));

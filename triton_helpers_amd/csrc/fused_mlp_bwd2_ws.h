@@ -86,7 +86,10 @@ struct WsShape {
 
 // XC: how x / dx are stored (MlpArgs::x_conv, 0 or the other 16-bit type); B: the network has biases or bias
 // gradients are wanted (false: accumulators start at zero and no row sums are kept).
-template <typename T, int KIN, int OUTP, int XC, bool B, int CH = WS_CHAIN_WAVES>
+// W: rows move in whole 16-byte pieces (16-byte aligned rows of a multiple of eight values; a 16-wide dy in 8-byte ones as
+// before) that are exchanged between the lane groups.  The L1 takes a lane a clock of a tile access whatever its width
+// (with the sum of the slots, 2^20 rows, us: 64 -> 64 -> 64 -> 64 125 -> 118, 64 -> 64 -> 64 -> 16 103 -> 91; 2^16 rows 26.8 -> 24.6).
+template <typename T, int KIN, int OUTP, int XC, bool B, bool W, int CH = WS_CHAIN_WAVES>
 __global__ __launch_bounds__(64 * (CH + WS_GRAD), 1) void mlp_bwd2_ws_k(MlpArgs a) {
   using SH = WsShape<KIN, OUTP>;
   // CH chain waves share the WS_CHAIN panels of a round: four own a 32-row panel each, eight a 16-row half each
@@ -98,6 +101,7 @@ __global__ __launch_bounds__(64 * (CH + WS_GRAD), 1) void mlp_bwd2_ws_k(MlpArgs 
   constexpr int TILES = SH::TILES, NBIAS = SH::NBIAS;
   constexpr int S_H = ws_stride(64), S_X = ws_stride(KIN), S_Y = ws_stride(OUTP), P_H = ws_panel(64);
   constexpr int DY_HALVES = OUTP > 16 ? 2 : 1;
+  constexpr bool DW = W && OUTP > 16;
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x;
   constexpr int nthreads = 64 * WAVES;
@@ -126,18 +130,23 @@ __global__ __launch_bounds__(64 * (CH + WS_GRAD), 1) void mlp_bwd2_ws_k(MlpArgs 
 #pragma unroll
   for (int kc = 0; kc < KC_IN; ++kc)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) off_x[kc][h] = piece_offset(lane & 15, 32 * kc + 16 * h + 4 * (lane >> 4), a.d_in, a.x_stride);
+    for (int h = 0; h < 2; ++h) off_x[kc][h] = piece_offset(lane & 15, W ? 32 * kc + 8 * (lane >> 4) : 32 * kc + 16 * h + 4 * (lane >> 4), a.d_in, a.x_stride);
 #pragma unroll
   for (int kc = 0; kc < KC_O; ++kc)
 #pragma unroll
-    for (int h = 0; h < DY_HALVES; ++h) off_dy[kc][h] = piece_offset(lane & 15, 32 * kc + 16 * h + 4 * (lane >> 4), a.d_out, a.dy_stride);
+    for (int h = 0; h < DY_HALVES; ++h) off_dy[kc][h] = piece_offset(lane & 15, DW ? 32 * kc + 8 * (lane >> 4) : 32 * kc + 16 * h + 4 * (lane >> 4), a.d_out, a.dy_stride);
 #pragma unroll
-  for (int mt = 0; mt < MT_I; ++mt) off_dx[mt] = piece_offset(lane & 15, 16 * mt + 4 * (lane >> 4), a.d_in, a.dx_stride);
+  for (int mt = 0; mt < MT_I; ++mt) off_dx[mt] = piece_offset(lane & 15, W ? 32 * (mt >> 1) + 8 * (lane >> 4) : 16 * mt + 4 * (lane >> 4), a.d_in, a.dx_stride);
   // a chunk past the end (a wave without work in the last round) reads zeros and stores nothing
   auto at = [&](int64_t chunk, int nt, int64_t stride, uint32_t off) {
     return chunk < n_chunks ? off + (uint32_t)((chunk * 32 + 16 * nt) * stride * 2) : OUT_OF_RANGE;
   };
-  auto load_x = [&](int64_t chunk, int nt, int kc) {
+  auto load_x = [&](int64_t chunk, int nt, int kc) {  // W: in natural order until it is used, and so dy
+    if constexpr (W) {
+      Frag f;
+      f.u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs_x, at(chunk, nt, a.x_stride, off_x[kc][0]), 0, 0));
+      return f;
+    }
     const buf_v2u lo = __builtin_amdgcn_raw_buffer_load_b64(rs_x, at(chunk, nt, a.x_stride, off_x[kc][0]), 0, 0);
     const buf_v2u hi = __builtin_amdgcn_raw_buffer_load_b64(rs_x, at(chunk, nt, a.x_stride, off_x[kc][1]), 0, 0);
     Frag f;
@@ -145,6 +154,11 @@ __global__ __launch_bounds__(64 * (CH + WS_GRAD), 1) void mlp_bwd2_ws_k(MlpArgs 
     return f;
   };
   auto load_dy = [&](int64_t chunk, int nt, int kc) {
+    if constexpr (DW) {
+      Frag f;
+      f.u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs_dy, at(chunk, nt, a.dy_stride, off_dy[kc][0]), 0, 0));
+      return f;
+    }
     const buf_v2u lo = __builtin_amdgcn_raw_buffer_load_b64(rs_dy, at(chunk, nt, a.dy_stride, off_dy[kc][0]), 0, 0);
     Frag f;
     f.w[0] = lo[0]; f.w[1] = lo[1]; f.w[2] = 0u; f.w[3] = 0u;
@@ -194,11 +208,12 @@ __global__ __launch_bounds__(64 * (CH + WS_GRAD), 1) void mlp_bwd2_ws_k(MlpArgs 
 #pragma unroll
         for (int kc = 0; kc < KC_IN; ++kc) {
           in[nt][kc] = XC == 0 ? nx[nt][kc] : convert_frag(nx[nt][kc], XC);
+          if constexpr (W) in[nt][kc] = nat_to_chain(in[nt][kc]);
           nx[nt][kc] = load_x(chunk + per_round, pt0 + nt, kc);
         }
 #pragma unroll
         for (int kc = 0; kc < KC_O; ++kc) {
-          dz[nt][kc] = ndy[nt][kc];
+          dz[nt][kc] = DW ? nat_to_chain(ndy[nt][kc]) : ndy[nt][kc];
           ndy[nt][kc] = load_dy(chunk + per_round, pt0 + nt, kc);
         }
       }
@@ -261,15 +276,28 @@ __global__ __launch_bounds__(64 * (CH + WS_GRAD), 1) void mlp_bwd2_ws_k(MlpArgs 
       }
       if (a.dx != nullptr) {
         layer_nt<T, NT, MT_I, 2, 0>(acc, dz, t_in, nullptr, lane);  // dx = W_in^T dz1
+        typedef typename std::conditional<XC == 0, T, typename std::conditional<XC == 1, F16, BF16>::type>::type XT;  // what x is stored in
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-          for (int mt = 0; mt < MT_I; ++mt) {
-            buf_v2u o;
-            if (XC == 1) { o[0] = pack2<F16>(acc[nt][mt][0], acc[nt][mt][1]); o[1] = pack2<F16>(acc[nt][mt][2], acc[nt][mt][3]); }
-            else if (XC == 2) { o[0] = pack2<BF16>(acc[nt][mt][0], acc[nt][mt][1]); o[1] = pack2<BF16>(acc[nt][mt][2], acc[nt][mt][3]); }
-            else { o[0] = pack2<T>(acc[nt][mt][0], acc[nt][mt][1]); o[1] = pack2<T>(acc[nt][mt][2], acc[nt][mt][3]); }
-            __builtin_amdgcn_raw_buffer_store_b64(o, rs_dx, at(chunk, pt0 + nt, a.dx_stride, off_dx[mt]), 0, 0);
+          for (int mt = 0; mt < MT_I; mt += 2) {
+            Frag f;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              f.w[2 * h] = pack2<XT>(acc[nt][mt + h][0], acc[nt][mt + h][1]);
+              f.w[2 * h + 1] = pack2<XT>(acc[nt][mt + h][2], acc[nt][mt + h][3]);
+            }
+            if constexpr (W) {
+              f = chain_to_nat(f);
+              const buf_v4u o = {f.w[0], f.w[1], f.w[2], f.w[3]};
+              __builtin_amdgcn_raw_buffer_store_b128(o, rs_dx, at(chunk, pt0 + nt, a.dx_stride, off_dx[mt]), 0, 0);
+            } else {
+#pragma unroll
+              for (int h = 0; h < 2; ++h) {
+                const buf_v2u o = {f.w[2 * h], f.w[2 * h + 1]};
+                __builtin_amdgcn_raw_buffer_store_b64(o, rs_dx, at(chunk, pt0 + nt, a.dx_stride, off_dx[mt + h]), 0, 0);
+              }
+            }
           }
       }
     }

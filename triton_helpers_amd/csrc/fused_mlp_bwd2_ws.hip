@@ -17,7 +17,10 @@ static int launch_ws(const MlpArgs& a0, hipStream_t s, int* blocks_out) {
   if (blocks > cap) blocks = cap;
   if (blocks_out != nullptr) *blocks_out = (int)blocks;
   const bool b = a.db_in != nullptr || a.db_hid != nullptr || a.db_out != nullptr || a.b_in != nullptr || a.b_hid != nullptr;
-  const void* kern = b ? (const void*)mlp_bwd2_ws_k<T, KIN, OUTP, 0, true, CH> : (const void*)mlp_bwd2_ws_k<T, KIN, OUTP, 0, false, CH>;
+  const bool wide = vec_load_ok(a.x, a.x_stride, a.d_in) && (OUTP == 16 || vec_load_ok(a.dy, a.dy_stride, a.d_out)) &&
+                    (a.dx == nullptr || vec_load_ok(a.dx, a.dx_stride, a.d_in));
+  const void* kern = wide ? (b ? (const void*)mlp_bwd2_ws_k<T, KIN, OUTP, 0, true, true, CH> : (const void*)mlp_bwd2_ws_k<T, KIN, OUTP, 0, false, true, CH>)
+                          : (b ? (const void*)mlp_bwd2_ws_k<T, KIN, OUTP, 0, true, false, CH> : (const void*)mlp_bwd2_ws_k<T, KIN, OUTP, 0, false, false, CH>);
   const hipError_t ea = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS);
   if (ea != hipSuccess) return fail((int)ea, "hipFuncSetAttribute: %s", hipGetErrorString(ea));
   void* args[] = {(void*)&a};

@@ -282,8 +282,13 @@ variable_list mlp_backward(Mlp m, Tensor dy, bool need_dx, bool float_grads) {
                          at.view(f, m.w[5], 5)};
   };
   const bool decoder = in <= 32 && out <= 16;  // the wider shapes need x in the parameters' dtype
-  if (wt != at::kFloat && depth <= 2 && H == 64 && in <= 64 && out <= 64 && (decoder || m.x.scalar_type() == wt) && in % 4 == 0 && out % 4 == 0 &&
-      relu && g.n > 0) {
+  // ReLU at 64 wide has kernels of its own for one and two hidden layers, which lay their weights out in both forms, sum eight waves
+  // and (one hidden layer) go through an identity layer: quicker than the whole backward from about 2^15 rows, 2^17 at one
+  // (2^12 / 2^15 / 2^16 rows, us own / whole: 32 -> 64 -> 64 -> 16 15.4 / 10.6, 17.2 / 16.6, 19.9 / 20.3; 2^17 / 2^18 rows:
+  // 64 -> 64 -> 64 30 / 27, 41 / 41)
+  const bool many = g.n > (depth == 2 ? 1 << 15 : 1 << 17);
+  if (many && wt != at::kFloat && depth <= 2 && H == 64 && in <= 64 && out <= 64 && (decoder || m.x.scalar_type() == wt) && in % 4 == 0 && out % 4 == 0 &&
+      relu) {
     // The weight gradients come back summed in a fixed order, in one uninitialised buffer (no clearing, no cast
     // kernel).  The buffer is the call's own: its pieces become the .grad tensors.
     const Pieces at(m.w, 8);

@@ -14,9 +14,7 @@
 //
 // LDS holds one copy of the weights, row-major in rows of 128 bytes: a product with W reads its fragments as rows, a
 // product with W^T reads the same bytes through the transposing reads, so ten 64-wide layers and the operand areas fit
-// 150 KB and the staging is a plain copy.  The 8-byte pieces of a row are exchanged by an xor with bits of the row number
-// (swizzle()): sixteen rows at one column, and four consecutive rows at four consecutive pieces, then fall on 64
-// different banks.
+// 150 KB and the staging is a plain copy (role_split.h).
 //
 // What it replaces for most calls is up to five layers per launch, a replayed forward between launches, dW through LDS
 // transposes of 2-byte stores or matrix-core transposes, and atomics of all workgroups into cleared sums that a cast kernel
@@ -30,13 +28,13 @@
 #pragma once
 
 #include "fused_mlp_bwd2_kernels.h"
+#include "role_split.h"
 
 namespace nf {
 
 constexpr int ROLES_MAX_DEPTH = 9;               // hidden layers (MlpArgs::depth) of one launch
 // hidden layers of the kernels that leave registers for more waves (but for ReLU a layer's derivatives take as much room as its activations)
 constexpr int roles_shallow(int act) { return act == NF_ACT_RELU ? 4 : 3; }
-constexpr int ROLES_PITCH = 128;                 // bytes of a row in LDS
 constexpr int ROLES_TILES = 16;                  // 16 x 16 tiles of a layer's dW in a slot (4 x 4, whether it has them all or not)
 constexpr int ROLES_LAYER = (ROLES_TILES + 1) * 256;  // floats of a layer in a slot: its tiles, its bias sums
 constexpr int roles_slot_floats(int depth) { return (depth + 1) * ROLES_LAYER; }
@@ -44,34 +42,6 @@ constexpr size_t roles_lds(int hp, int depth, int rows) {
   return (size_t)(depth * hp + 64) * ROLES_PITCH + (size_t)depth * 64 * 4 + (size_t)4 * rows * ROLES_PITCH;
 }
 static_assert(roles_lds(64, ROLES_MAX_DEPTH, 64) <= 160 * 1024, "LDS budget");
-
-// xor on the number of an 8-byte piece of row r
-__device__ __forceinline__ int swizzle(int r) { return (((r >> 1) & 1) << 2) | ((r >> 2) & 3); }
-
-// Eight 16-bit values of row r from column c0 on, zero beyond `width` and `rows`.  vec: rows of whole 16-byte aligned pieces.
-// Otherwise a row's last piece is read as the eight values that end with the row and shifted, so that no access leaves the row.
-__device__ __forceinline__ Frag load_row8(const uint16_t* base, int64_t stride, int64_t r, int64_t rows, int width, int c0, bool vec) {
-  Frag f;
-  f.u = make_uint4(0u, 0u, 0u, 0u);
-  if (r >= rows || c0 >= width) return f;
-  const uint16_t* p = base + r * stride;
-  if (vec) {
-    f.u = *reinterpret_cast<const uint4*>(p + c0);
-  } else if (width >= 8) {
-    const int start = c0 < width - 8 ? c0 : width - 8, skip = c0 - start;  // values of the window in front of c0
-    uint4 v;
-    __builtin_memcpy(&v, p + start, 16);
-    if (skip & 4) v = make_uint4(v.z, v.w, 0u, 0u);
-    if (skip & 2) v = make_uint4(v.y, v.z, v.w, 0u);
-    if (skip & 1) v = make_uint4((v.x >> 16) | (v.y << 16), (v.y >> 16) | (v.z << 16), (v.z >> 16) | (v.w << 16), v.w >> 16);
-    f.u = v;
-  } else {  // a row of less than eight values: c0 == 0
-#pragma unroll
-    for (int j = 0; j < 7; ++j)
-      if (j < width) f.w[j >> 1] |= (uint32_t)p[j] << (16 * (j & 1));
-  }
-  return f;
-}
 
 // rows of `w` [layers * nr][nc] (row-contiguous) -> LDS rows of 128 bytes, swizzled; layer l's rows start at LDS row l * pad, rows
 // nr .. pad - 1 and columns nc .. 63 are zero
@@ -106,59 +76,6 @@ __device__ __forceinline__ void stage_rows(char* dst, const uint16_t* w, int lay
       if (u < units) *reinterpret_cast<uint2*>(dst + row * ROLES_PITCH + (((u & 15) ^ swizzle(row)) << 3)) = v[i];
     }
   }
-}
-
-// two 8-byte pieces -> fragment
-__device__ __forceinline__ Frag read_pieces(const char* p0, const char* p1) {
-  const uint2 a = *reinterpret_cast<const uint2*>(p0), b = *reinterpret_cast<const uint2*>(p1);
-  Frag f;
-  f.w[0] = a.x; f.w[1] = a.y; f.w[2] = b.x; f.w[3] = b.y;
-  return f;
-}
-__device__ __forceinline__ Frag read_pieces_tr(const char* p0, const char* p1) {
-  typedef tr_v4i16 __attribute__((address_space(3))) * lds_ptr;
-  const uint2 a = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)p0));
-  const uint2 b = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)p1));
-  Frag f;
-  f.w[0] = a.x; f.w[1] = a.y; f.w[2] = b.x; f.w[3] = b.y;
-  return f;
-}
-__device__ __forceinline__ void write_pieces(char* p0, char* p1, const Frag& f) {
-  *reinterpret_cast<uint2*>(p0) = make_uint2(f.w[0], f.w[1]);
-  *reinterpret_cast<uint2*>(p1) = make_uint2(f.w[2], f.w[3]);
-}
-
-// Workgroup barrier that waits for this wave's LDS traffic only: global loads and the dx stores stay in flight across it.
-__device__ __forceinline__ void roles_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// The same eight values back.
-__device__ __forceinline__ void store_row8(uint16_t* base, int64_t stride, int64_t r, int64_t rows, int width, int c0, const Frag& f, bool vec) {
-  if (r >= rows || c0 >= width) return;
-  uint16_t* p = base + r * stride + c0;
-  if (vec) {
-    *reinterpret_cast<uint4*>(p) = f.u;
-  } else if (c0 + 8 <= width) {
-    __builtin_memcpy(p, &f.u, 16);
-  } else {
-#pragma unroll
-    for (int j = 0; j < 7; ++j)
-      if (c0 + j < width) p[j] = (uint16_t)(f.w[j >> 1] >> (16 * (j & 1)));
-  }
-}
-
-// body(integral_constant<0 .. N - 1>): a loop over layers whose register arrays are indexed by constants whatever its size
-template <int N, int I = 0, typename Body>
-__device__ __forceinline__ void each_layer(Body&& body) {
-  if constexpr (I < N) {
-    body(std::integral_constant<int, I>{});
-    each_layer<N, I + 1>(body);
-  }
-}
-// A uniform value the optimiser knows nothing about: what is derived from it is worked out where it is used instead of being
-// kept for all layers at once (the comparisons and addresses of nine layers do not fit the scalar registers).
-__device__ __forceinline__ int opaque(int v) {
-  asm volatile("" : "+s"(v));
-  return v;
 }
 
 // The launch's arguments, read again where they are used (see opaque()).
@@ -213,12 +130,7 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
   }
   __syncthreads();
 
-  // byte offsets of this lane's pieces; a tile row (16 rows) is 2048 bytes further, a K-chunk of 32 columns 64 bytes
-  const int sw = swizzle(n);
-  const int chain0 = n * ROLES_PITCH + ((g ^ sw) << 3);      // columns 4g .. of row n (chain order); + 16 columns: ^ 32
-  const int nat0 = n * ROLES_PITCH + (((2 * g) ^ sw) << 3);  // columns 8g .. of row n (natural order); + 4 columns: ^ 8
-  // transposing reads: this lane supplies row 4g + n / 4, columns 4 (n % 4) ..; tile column t: ^ 32 (t & 1) + 64 (t / 2); rows + 16: 2048
-  const int tr0 = (4 * g + (n >> 2)) * ROLES_PITCH + ((((n & 3) ^ g) | ((n >> 3) << 2)) << 3);
+  const int chain0 = chain_offset(n, g), nat0 = natural_offset(n, g), tr0 = tr_offset(n, g);
   const f32x4_t zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
   int area = 0;
 
@@ -230,7 +142,7 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
       char* p = mine + area * AREA + panel * PANEL;
       const int o0 = natural ? nat0 : chain0, o1 = natural ? nat0 ^ 8 : chain0 ^ 32;
       write_pieces(p + o0, p + o1, f[0]);
-      if (two) write_pieces(p + 64 + o0, p + 64 + o1, f[1]);
+      if (two) write_pieces(p + (o0 ^ 64), p + (o1 ^ 64), f[1]);
     };
     for (int64_t round = 0; round < rounds; ++round) {
       const int64_t r = row0 + round * gridDim.x * ROWS;
@@ -247,14 +159,13 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
       // acc = b + W cur of linear layer l
       auto layer = [&](int l, bool natural) {
         const char* w = l == 0 ? w_in : w_hid + (l - 1) * HP * ROLES_PITCH;
-        const char* w0 = w + (natural ? nat0 : chain0);
-        const char* w1 = w + (natural ? nat0 ^ 8 : chain0 ^ 32);
+        const int o0 = natural ? nat0 : chain0, o1 = natural ? nat0 ^ 8 : chain0 ^ 32;
         const float* b = bias + l * 64 + 4 * g;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[mt] = *reinterpret_cast<const f32x4_t*>(b + 16 * mt);
         auto chunk = [&](int kc) {
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma16<T>(read_pieces(w0 + mt * 2048 + kc * 64, w1 + mt * 2048 + kc * 64), cur[kc], acc[mt]);
+          for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma16<T>(read_pieces(w + mt * 2048 + (o0 ^ 64 * kc), w + mt * 2048 + (o1 ^ 64 * kc)), cur[kc], acc[mt]);
         };
         chunk(0);
         if (KC == 2 || (l == 0 && two_in)) chunk(1);
@@ -324,7 +235,7 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
       auto out_chunk = [&](int kc) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          const char* p = w_out + kc * 32 * ROLES_PITCH + (mt >> 1) * 64 + (tr0 ^ ((mt & 1) << 5));
+          const char* p = w_out + kc * 32 * ROLES_PITCH + (tr0 ^ 32 * mt);
           acc[mt] = mfma16<T>(read_pieces_tr(p, p + 2048), dz[kc], acc[mt]);
         }
       };
@@ -367,7 +278,7 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
           for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
-              const char* p = w + kc * 32 * ROLES_PITCH + (mt >> 1) * 64 + (tr0 ^ ((mt & 1) << 5));
+              const char* p = w + kc * 32 * ROLES_PITCH + (tr0 ^ 32 * mt);
               acc[mt] = mfma16<T>(read_pieces_tr(p, p + 2048), dz[kc], acc[mt]);
             }
         }
@@ -389,7 +300,7 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
             f32x4_t v = zero4;
 #pragma unroll
             for (int c = 0; c < KC; ++c) {
-              const char* p = w_in + c * 32 * ROLES_PITCH + kc * 64 + (tr0 ^ (t << 5));
+              const char* p = w_in + c * 32 * ROLES_PITCH + (tr0 ^ 64 * kc ^ 32 * t);
               v = mfma16<T>(read_pieces_tr(p, p + 2048), dz[c], v);
             }
             typedef typename std::conditional<T::code == NF_BF16, F16, BF16>::type Other;
@@ -426,17 +337,17 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
     // ---- output layer ----
     roles_barrier();
     if (16 * qm < a.d_out) {
-      const char* pd = areas + area * AREA + trm;
-      const char* ph = areas + area * AREA + PANEL + trk;
+      const char* pd = areas + area * AREA;
+      const char* ph = areas + area * AREA + PANEL;
 #pragma unroll
       for (int s = 0; s < ROWS / 32; ++s) {
         Frag hb[TW];
 #pragma unroll
-        for (int k = 0; k < TW; ++k) hb[k] = operand(ph + s * 4096 + k * 64);
+        for (int k = 0; k < TW; ++k) hb[k] = operand(ph + s * 4096 + (trk ^ 64 * k));
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           if (i == 1 && !two_out) continue;
-          const Frag da = operand(pd + s * 4096 + i * 64);
+          const Frag da = operand(pd + s * 4096 + (trm ^ 64 * i));
 #pragma unroll
           for (int k = 0; k < TW; ++k) dw_out[i][k] = mfma16<T>(da, hb[k], dw_out[i][k]);
 #pragma unroll
@@ -451,8 +362,8 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
       const int depth = opaque(a.depth);
       if (j >= depth) return;
       roles_barrier();
-      const char* pd = areas + area * AREA + trm;
-      const char* ph = areas + area * AREA + PANEL + trk;
+      const char* pd = areas + area * AREA;
+      const char* ph = areas + area * AREA + PANEL;
       // COLS: tile columns of this layer's dW that this wave owns
       auto section = [&](auto cols_c) {
         constexpr int COLS = decltype(cols_c)::value;
@@ -460,9 +371,9 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
         for (int s = 0; s < ROWS / 32; ++s) {
           Frag hb[COLS], da[TW];
 #pragma unroll
-          for (int k = 0; k < COLS; ++k) hb[k] = operand(ph + s * 4096 + k * 64);
+          for (int k = 0; k < COLS; ++k) hb[k] = operand(ph + s * 4096 + (trk ^ 64 * k));
 #pragma unroll
-          for (int i = 0; i < TW; ++i) da[i] = operand(pd + s * 4096 + i * 64);
+          for (int i = 0; i < TW; ++i) da[i] = operand(pd + s * 4096 + (trm ^ 64 * i));
 #pragma unroll
           for (int i = 0; i < TW; ++i) {
 #pragma unroll

@@ -39,7 +39,7 @@ constexpr int ROLES_TILES = 16;                  // 16 x 16 tiles of a layer's d
 constexpr int ROLES_LAYER = (ROLES_TILES + 1) * 256;  // floats of a layer in a slot: its tiles, its bias sums
 constexpr int roles_slot_floats(int depth) { return (depth + 1) * ROLES_LAYER; }
 constexpr size_t roles_lds(int hp, int depth, int rows) {
-  return (size_t)(depth * hp + 64) * ROLES_PITCH + (size_t)depth * 64 * 4 + (size_t)4 * rows * ROLES_PITCH;
+  return (size_t)(depth * hp + 64) * ROLES_PITCH + (size_t)depth * 64 * 4 + (size_t)4 * rows * ROLES_PITCH + 32 * 4;
 }
 static_assert(roles_lds(64, ROLES_MAX_DEPTH, 64) <= 160 * 1024, "LDS budget");
 
@@ -103,6 +103,8 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
   float* bias = reinterpret_cast<float*>(w_out + 64 * ROLES_PITCH);  // [depth][64]
   char* areas = reinterpret_cast<char*>(bias + depth * 64);    // [2][dz rows | input rows][ROWS][128]
   constexpr int PANEL = ROWS * ROLES_PITCH, AREA = 2 * PANEL;
+  Sections<CW> sections = {reinterpret_cast<int*>(areas + 2 * AREA), 0};
+  if (tid < 32) sections.flags[tid] = 0;
 
   const int64_t rounds = (a.rows + (int64_t)gridDim.x * ROWS - 1) / ((int64_t)gridDim.x * ROWS);
   const bool chain = wave < CW;
@@ -143,6 +145,11 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
       const int o0 = natural ? nat0 : chain0, o1 = natural ? nat0 ^ 8 : chain0 ^ 32;
       write_pieces(p + o0, p + o1, f[0]);
       if (two) write_pieces(p + (o0 ^ 64), p + (o1 ^ 64), f[1]);
+    };
+    auto room = [&] { sections.room(lane); };
+    auto announce = [&] {
+      sections.parked(wave);
+      area ^= 1;
     };
     for (int64_t round = 0; round < rounds; ++round) {
       const int64_t r = row0 + round * gridDim.x * ROWS;
@@ -226,10 +233,10 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
         }
       }
       // ---- output layer: dW_out = dy^T h, dh = W_out^T dy ----
+      room();
       park(dz, 0, false, two_out);
       park(h[0], 1, false, KC == 2);
-      roles_barrier();
-      area ^= 1;
+      announce();
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) acc[mt] = zero4;
       auto out_chunk = [&](int kc) {
@@ -267,10 +274,10 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
         }
         if constexpr (j + 1 < MAXD) {
           if (j == depth - 1) return;  // the input layer follows below
+          room();
           park(dz, 0, false, KC == 2);
           park(h[j + 1], 1, false, KC == 2);
-          roles_barrier();
-          area ^= 1;
+          announce();
           const char* w = w_hid + (depth - 2 - j) * HP * ROLES_PITCH;
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) acc[mt] = zero4;
@@ -284,11 +291,11 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
         }
       });
       // ---- input layer: dW_in = dz^T x, dx = W_in^T dz ----
+      room();
       park(dz, 0, false, KC == 2);
       park(x, 1, HP == 32, two_in);
       load_rows(r + (int64_t)gridDim.x * ROWS);
-      roles_barrier();
-      area ^= 1;
+      announce();
       const ArgsPtr k = fresh_args();
       if (k->dx != nullptr) {
 #pragma unroll
@@ -333,9 +340,13 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
     }
   const int trm = tr0 ^ (qm << 5), trk = tr0 ^ (qn << 5);
   auto operand = [&](const char* p) { return read_pieces_tr(p, p + 2048); };
+  auto done = [&] {
+    sections.done(wave);
+    area ^= 1;
+  };
   for (int64_t round = 0; round < rounds; ++round) {
     // ---- output layer ----
-    roles_barrier();
+    sections.begin(lane);
     if (16 * qm < a.d_out) {
       const char* pd = areas + area * AREA;
       const char* ph = areas + area * AREA + PANEL;
@@ -355,13 +366,13 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
         }
       }
     }
-    area ^= 1;
+    done();
     // ---- hidden layers and the input layer (j = depth - 1) ----
     each_layer<MAXD>([&](auto step) {
       constexpr int j = decltype(step)::value;
       const int depth = opaque(a.depth);
       if (j >= depth) return;
-      roles_barrier();
+      sections.begin(lane);
       const char* pd = areas + area * AREA;
       const char* ph = areas + area * AREA + PANEL;
       // COLS: tile columns of this layer's dW that this wave owns
@@ -392,7 +403,7 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
       };
       if (HP == 32 && j == depth - 1 && two_in) section(std::integral_constant<int, 2>{});  // the input layer, wider than the others
       else section(std::integral_constant<int, TW>{});
-      area ^= 1;
+      done();
     });
   }
 

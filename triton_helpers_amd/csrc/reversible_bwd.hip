@@ -18,9 +18,6 @@
 // 324 -> 251, 2^20 1110 -> 915; 48-wide (each coupling was a launch) 96 -> 34, 174 -> 87, 461 -> 233, 1712 -> 849; 32-wide 48 -> 20, 54 -> 44,
 // 129 -> 104, 500 -> 367.  What bounds it now: the chain's vector instructions (half of the time, a third of them the activation's) and what a
 // chain wave waits for between its products, with two of them on a SIMD.
-//
-// The waves hand over through flags: with barriers, which keep them in step, the 64-wide 2^20 rows took 1060 us (flags 990; single reads of
-// LDS and a swizzle over all banks 957; the gradient waves first 903).
 #include "reversible.h"
 #include "role_split.h"
 
@@ -143,9 +140,8 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void rev_bwd_k(RevBwdArgs a) {
   char* weights = rev_smem;                                        // [CPL][F.w1, F.w2, G.w1, G.w2][HP][128]
   float* bias = reinterpret_cast<float*>(weights + CPL * 4 * MATRIX);  // [CPL][4][64]
   char* areas = reinterpret_cast<char*>(bias + CPL * 4 * 64);      // [2][gradient rows | input rows][ROWS][128]
-  int* flags = reinterpret_cast<int*>(areas + 2 * AREA);           // sections parked by each chain wave, + 16: read by each gradient wave
-  int section = 0;                                                 // this wave's sections so far
-  if (threadIdx.x < 32) flags[threadIdx.x] = 0;
+  Sections<CW> sections = {reinterpret_cast<int*>(areas + 2 * AREA), 0};
+  if (threadIdx.x < 32) sections.flags[threadIdx.x] = 0;
   const int64_t per_round = (int64_t)gridDim.x * ROWS, rounds = (a.rows + per_round - 1) / per_round;
   const f32x4_t zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
 
@@ -167,10 +163,6 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void rev_bwd_k(RevBwdArgs a) {
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc) write_pieces(p + (chain0 ^ 64 * kc), p + (chain0 ^ 64 * kc ^ 32), f[kc]);
       };
-      // An area is free when the gradient waves have read the section before the last.  No barrier: waves in step would all want the
-      // same unit at a time, the matrix cores, the vector units and LDS in turn.
-      auto room = [&] { await<4>(flags + 16, lane, section - 1); };
-      auto announce = [&] { post(flags + wave, ++section); };
       const bool first = opaque(top) == a.nblocks;
       Frag y1[KC], y2[KC], d1[KC], d2[KC];  // the stream and its gradient, lane group g: features 32 kc + 8 g ..
       // The pieces p of a half of the stream and q of the other half's gradient.  Rows of whole pieces: of a
@@ -259,10 +251,10 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void rev_bwd_k(RevBwdArgs a) {
           gate[mt >> 1].w[2 * (mt & 1)] = pack2<T>(gv[0], gv[1]);
           gate[mt >> 1].w[2 * (mt & 1) + 1] = pack2<T>(gv[2], gv[3]);
         }
-        room();
+        sections.room(lane);
         park(d, 0, 0);
         park(t, 0, 1);
-        announce();
+        sections.parked(wave);
         between(0);
         product(w + MATRIX, b + 64, t);
 #pragma unroll
@@ -277,10 +269,10 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void rev_bwd_k(RevBwdArgs a) {
         for (int mt = 0; mt < MT; ++mt)
           gate_apply<T, false>(acc[mt], gate[mt >> 1].w[2 * (mt & 1)], gate[mt >> 1].w[2 * (mt & 1) + 1], dz[mt >> 1].w[2 * (mt & 1)],
                                dz[mt >> 1].w[2 * (mt & 1) + 1]);
-        room();
+        sections.room(lane);
         park(dz, 1, 0);
         park(u, 1, 1);
-        announce();
+        sections.parked(wave);
         between(1);
         product_tr(w, dz);
 #pragma unroll
@@ -364,8 +356,7 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void rev_bwd_k(RevBwdArgs a) {
           if (j >= opaque(count)) return;
 #pragma unroll
           for (int s = 0; s < 4; ++s) {
-            await<CW>(flags, lane, ++section);
-            __builtin_amdgcn_s_setprio(3);  // what the chain waves wait for goes first (2^20 rows of four 64-wide couplings: 957 -> 903 us)
+            sections.begin(lane);
             const int o = (s & 1) * AREA;
 #pragma unroll
             for (int q = 0; q < ROWS / 32; ++q) {
@@ -382,8 +373,7 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void rev_bwd_k(RevBwdArgs a) {
 #pragma unroll
               for (int p = 0; p < 4; ++p) db[j][s] = dot2_ones<T>(da[0].w[p], db[j][s]);
             }
-            post(flags + 16 + wave - CW, section);
-            __builtin_amdgcn_s_setprio(0);
+            sections.done(wave);
           }
         });
       // to this workgroup's slot, or into the accumulators

@@ -108,9 +108,9 @@ __device__ __forceinline__ void post(int* flag, int count) {
                : "v"(p), "v"(count)
                : "memory");
 }
-template <int N>  // waits until all of flags[0 .. N) have reached count (N a power of two)
+template <int N>  // waits until all of flags[0 .. N) have reached count
 __device__ __forceinline__ void await(const int* flags, int lane, int count) {
-  auto p = (const __attribute__((address_space(3))) int*)flags + (lane & (N - 1));
+  auto p = (const __attribute__((address_space(3))) int*)flags + (lane < N ? lane : N - 1);
   int v;  // (one statement: a loop the compiler sees would cut its register allocation in two)
   asm volatile(
       "0:\n\tds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)\n\tv_cmp_gt_i32_e32 vcc, %2, %0\n\ts_cbranch_vccz 1f\n\ts_sleep 1\n\ts_branch 0b\n1:"
@@ -118,6 +118,43 @@ __device__ __forceinline__ void await(const int* flags, int lane, int count) {
       : "v"(p), "s"(count)
       : "vcc", "memory");
 }
+// How the roles of a workgroup of CW chain waves pass a section's panels on; `section` counts a wave's sections, areas alternate.  Several
+// chain waves on a SIMD go by flags: with barriers they would be in step and all want the same unit at a time (64 -> 64 with three hidden
+// SiLU layers, 2^21 rows, us: 518, so 465; 64-wide reversible couplings 6 %).  A chain wave that has its SIMD to itself is better off with
+// barriers, which are quicker (64 -> 64 with nine hidden ReLU layers, 2^19 rows: 268, with flags 286).
+template <int CW>
+struct Sections {
+  static constexpr bool FLAGS = CW > 4;
+  int* flags;  // LDS, 32 zeros: sections parked by each chain wave, + 16: read by each gradient wave
+  int section;
+
+  // chain waves: an area is free when the gradient waves have read the section before the last
+  __device__ __forceinline__ void room(int lane) const {
+    if constexpr (FLAGS) await<4>(flags + 16, lane, section - 1);
+  }
+  __device__ __forceinline__ void parked(int wave) {
+    ++section;
+    if constexpr (FLAGS) post(flags + wave, section);
+    else roles_barrier();
+  }
+  // gradient waves
+  __device__ __forceinline__ void begin(int lane) {
+    ++section;
+    if constexpr (FLAGS) {
+      await<CW>(flags, lane, section);
+      __builtin_amdgcn_s_setprio(3);  // what the chain waves wait for goes first (four 64-wide couplings, 2^20 rows: 957 -> 903 us)
+    } else {
+      roles_barrier();
+    }
+  }
+  __device__ __forceinline__ void done(int wave) const {
+    if constexpr (FLAGS) {
+      post(flags + 16 + wave - CW, section);
+      __builtin_amdgcn_s_setprio(0);
+    }
+  }
+};
+
 // A uniform value the optimiser knows nothing about: what is derived from it is worked out where it is used instead of being
 // kept for all layers at once (the comparisons and addresses of nine layers do not fit the scalar registers).
 __device__ __forceinline__ int opaque(int v) {

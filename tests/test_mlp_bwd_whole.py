@@ -59,6 +59,9 @@ CASES = [
     (16385, 32, 64, 16, 4, "relu", True, "f16", False, 0, 0),
     (40003, 48, 64, 33, 3, "silu", True, "bf16", False, 0, 0),
     (40003, 64, 64, 64, 9, "relu", False, "bf16", False, 0, 0),
+    (40003, 64, 64, 64, 5, "relu", True, "f16", False, 0, 0),
+    (80003, 32, 64, 16, 6, "relu", True, "bf16", False, 0, 0),
+    (40003, 35, 64, 3, 6, "relu", True, "bf16", False, 1, 1),
     (100003, 33, 32, 16, 4, "relu", True, "f16", False, 0, 0),
     (40003, 32, 16, 33, 6, "relu2", True, "bf16", False, 0, 0),
 ]

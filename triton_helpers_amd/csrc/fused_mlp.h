@@ -159,6 +159,7 @@ size_t mlp_bwd_roles_bytes(int64_t rows, int d_hidden, int depth, int act);
 int launch_mlp_bwd_roles(const MlpArgs& a, int dtype, int grad_dtype, void* const out[6], void* workspace, hipStream_t s);
 
 // The forward of one-hidden-layer ReLU networks of width 64 with aligned rows (fused_mlp_fwd2.hip).  *handled = false: not that shape, nothing was launched.
+bool mlp_fwd2_takes(const MlpArgs& a, int dtype);  // whether launch_mlp_fwd2 would handle it
 int launch_mlp_fwd2(const MlpArgs& a, int dtype, hipStream_t s, bool* handled);
 
 // float32 storage and float32 products (fused_mlp_f32.hip).  The backward needs mlp32_bwd_workspace_bytes of scratch.

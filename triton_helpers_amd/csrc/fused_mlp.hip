@@ -987,6 +987,13 @@ extern "C" int nf_mlp_bwd_whole(const void* x, int64_t x_stride, const void* dy,
   set_rows(a, (const uint16_t*)x, x_stride, nullptr, 0, (const uint16_t*)dy, dy_stride, (uint16_t*)dx, dx_stride);
   const std::vector<int> first = plan_launches(depth + 1, bwd_max_linear(d_hidden, act));
   for (size_t k = 1; k + 1 < first.size(); ++k) a.handover |= 1u << (first[k] - 1);
+  if (act == NF_ACT_RELU && a.handover != 0) {
+    // (ReLU: where the forward that nf_mlp_bwd replays sums as the kernel does anyway, one run is enough: five layers of 32 -> 16, 2^19 rows, 160
+    // us with a second run)
+    MlpArgs replay = launch_args(a, first[0], first[1]);
+    set_rows(replay, a.x, a.x_stride, nullptr, d_hidden, nullptr, 0, nullptr, 0);
+    if (mlp_fwd2_takes(replay, dtype)) a.handover = 0;
+  }
   void* const out[6] = {dw_in, db_in, depth > 1 ? dw_hid : nullptr, depth > 1 ? db_hid : nullptr, dw_out, db_out};
   return launch_mlp_bwd_roles(a, dtype, grad_dtype, out, workspace, (hipStream_t)stream);
 }

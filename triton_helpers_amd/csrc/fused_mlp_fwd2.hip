@@ -177,16 +177,19 @@ static int launch_fwd2(const MlpArgs& a0, hipStream_t s) {
   return check_launch("mlp_fwd2");
 }
 
-int launch_mlp_fwd2(const MlpArgs& a, int dtype, hipStream_t s, bool* handled) {
-  *handled = false;
+bool mlp_fwd2_takes(const MlpArgs& a, int dtype) {
   const int xc_other = dtype == NF_BF16 ? 1 : 2;
   const auto rows8 = [](const void* p, int64_t stride) { return (uintptr_t)p % 8 == 0 && stride % 4 == 0; };
   const bool shape = a.depth == 2 && a.d_hidden == 64 && a.d_in <= 64 && a.d_out <= 64 && a.act == NF_ACT_RELU && a.in_act == NF_ACT_NONE &&
                      (a.x_conv == 0 || a.x_conv == xc_other);
   const bool aligned = a.d_in % 4 == 0 && a.d_out % 4 == 0 && rows8(a.x, a.x_stride) && rows8(a.y, a.y_stride);
   const bool in_reach = rows_in_reach(a.rows, a.x_stride) && rows_in_reach(a.rows, a.y_stride);
-  if (!shape || !aligned || !in_reach) return 0;
-  *handled = true;
+  return shape && aligned && in_reach;
+}
+
+int launch_mlp_fwd2(const MlpArgs& a, int dtype, hipStream_t s, bool* handled) {
+  *handled = mlp_fwd2_takes(a, dtype);
+  if (!*handled) return 0;
   const bool wide_in = a.d_in > 32, wide_out = a.d_out > 16;
 #define NF_FWD2_DISPATCH(T)                                          \
   (wide_in ? (wide_out ? launch_fwd2<T, 64, 64>(a, s) : launch_fwd2<T, 64, 16>(a, s)) \

@@ -267,11 +267,14 @@ variable_list mlp_backward(Mlp m, Tensor dy, bool need_dx, bool float_grads) {
   const bool relu = m.act == NF_ACT_RELU;
   if (dy.scalar_type() != wt) dy = dy.to(wt);
   const Rows g(dy, out);
-  // Up to nine hidden layers: one launch for the whole backward, but where the kernels that nf_mlp_bwd chains stream many rows
-  // faster than its LDS does (64 wide, 2^20 rows against 2^18, us whole / chained: narrow depth 2 SiLU 153 / 132 against
-  // 48 / 51, ReLU depth 3 162 / 130 against 51 / 62, depth 9 623 / 600 against 171 / 269).
-  const bool narrow = in <= 32 && in % 4 == 0 && out <= 16;
-  const bool streams = H == 64 && m.x.scalar_type() == wt && ((depth == 2 && narrow && g.n > (3 << 17)) || (relu && depth >= 3 && g.n > (1 << 19)));
+  // Up to nine hidden layers: one launch for the whole backward, but where the kernels that nf_mlp_bwd chains stream many rows faster than
+  // its LDS does.  64 wide, us whole / chained: 32 -> 16 with two SiLU layers 2^19 rows 76 / 79, 2^20 140 / 132 (32 -> 3, whose rows are not
+  // whole 8-byte pieces, 154 / 167); ReLU, 32 -> 16, 2^20 and 1.5M rows: three layers 135 / 136 and 185 / 167, four 166 / 196 and 230 / 255,
+  // five 264 / 281 and 377 / 369, six 301 / 346 and 428 / 452, seven 394 / 436 and 560 / 587, nine 479 / 532 and 684 / 704.
+  const bool narrow = in <= 32 && in % 4 == 0 && out <= 16 && out % 4 == 0;
+  const bool streams = H == 64 && m.x.scalar_type() == wt &&
+                       (depth == 2 ? narrow && g.n > (3 << 18)
+                                   : relu && (depth == 3 || depth == 5) && g.n > (5 << 18));
   const int64_t whole_bytes = streams ? 0 : nf_mlp_bwd_whole_workspace_bytes(g.n, H, depth, m.act, dt);
   // deeper: only the ReLU backward of a 64-wide network whose first launch has three linear layers converts x on the fly
   const bool converts = whole_bytes > 0 || (depth == 1 && relu && H == 64);
@@ -283,10 +286,10 @@ variable_list mlp_backward(Mlp m, Tensor dy, bool need_dx, bool float_grads) {
   };
   const bool decoder = in <= 32 && out <= 16;  // the wider shapes need x in the parameters' dtype
   // ReLU at 64 wide has kernels of its own for one and two hidden layers, which lay their weights out in both forms, sum eight waves
-  // and (one hidden layer) go through an identity layer: quicker than the whole backward from about 2^15 rows, 2^17 at one
-  // (2^12 / 2^15 / 2^16 rows, us own / whole: 32 -> 64 -> 64 -> 16 15.4 / 10.6, 17.2 / 16.6, 19.9 / 20.3; 2^17 / 2^18 rows:
-  // 64 -> 64 -> 64 30 / 27, 41 / 41)
-  const bool many = g.n > (depth == 2 ? 1 << 15 : 1 << 17);
+  // and (one hidden layer) go through an identity layer: quicker than the whole backward from about 2^16 rows, at one layer from 2^19 where
+  // the output is narrow (us own / whole: 32 -> 64 -> 64 -> 16 2^12 rows 15.4 / 10.6, 2^16 21 / 20, 2^17 24 / 26, 2^20 64 / 101; 64 -> 64 -> 64
+  // -> 64 2^16 25 / 24, 2^17 28 / 32; 32 -> 64 -> 16 2^18 31 / 27, 2^19 42 / 41, 2^20 64 / 70; 64 -> 64 -> 64 2^18 41 / 36, 2^20 119 / 115)
+  const bool many = depth == 2 ? g.n > 1 << 16 : out <= 16 && g.n > 1 << 19;
   if (many && wt != at::kFloat && depth <= 2 && H == 64 && in <= 64 && out <= 64 && (decoder || m.x.scalar_type() == wt) && in % 4 == 0 && out % 4 == 0 &&
       relu) {
     // The weight gradients come back summed in a fixed order, in one uninitialised buffer (no clearing, no cast

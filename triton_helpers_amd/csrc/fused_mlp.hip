@@ -53,18 +53,6 @@ __global__ __launch_bounds__(512) void mlp_fwd_k(MlpArgs a) {
   float* bias_hid = bias_in + HP;
   float* bias_out = bias_hid + (size_t)n_hid * HP;
 
-  stage_weight_frags<false, false>(f_in, a.w_in, a.d_hidden, a.d_in, MT_H, KC_IN, tid, nthreads);
-  for (int k = 0; k < n_hid; ++k)
-    stage_weight_frags<true, false>(f_hid + (size_t)k * MT_H * KC_H * FRAG_ELEMS,
-                                    a.w_hid + (size_t)k * a.d_hidden * a.d_hidden, a.d_hidden, a.d_hidden, MT_H, KC_H,
-                                    tid, nthreads);
-  stage_weight_frags<true, false>(f_out, a.w_out, a.d_out, a.d_hidden, MT_O, KC_H, tid, nthreads);
-  stage_bias<T>(bias_in, a.b_in, a.d_hidden, HP, tid, nthreads);
-  for (int k = 0; k < n_hid; ++k)
-    stage_bias<T>(bias_hid + k * HP, a.b_hid ? a.b_hid + (size_t)k * a.d_hidden : nullptr, a.d_hidden, HP, tid, nthreads);
-  stage_bias<T>(bias_out, a.b_out, a.d_out, OUTP, tid, nthreads);
-  __syncthreads();
-
   const bool relu = a.act == NF_ACT_RELU;
   const int64_t n_chunks = (a.rows + 31) / 32;
   const int64_t wave_stride = (int64_t)gridDim.x * a.waves;
@@ -76,6 +64,40 @@ __global__ __launch_bounds__(512) void mlp_fwd_k(MlpArgs a) {
 #pragma unroll
     for (int kc = 0; kc < KC_IN; ++kc)
       nxt[nt][kc] = load_rows_frag(a.x, a.x_stride, first_chunk * 32 + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
+  stage_weight_frags<false, false>(f_in, a.w_in, a.d_hidden, a.d_in, MT_H, KC_IN, tid, nthreads);
+  if (n_hid > 1 && a.d_hidden == HP && (uintptr_t)a.w_hid % 8 == 0) {
+    // The hidden layers are one array: their pieces of eight values as one list, several under way per thread, and their biases.  Layer by
+    // layer, loads and biases of a deep network waited for one another twenty times (64 -> 64 x 9 -> 64, 1000 / 65536 / 2^18 rows, us: 16.0 / 18.7 / 43.6,
+    // so 14.5 / 16.4 / 37.7; 32 -> 64 x 3 -> 16 6.8 / 8.6 / 15.2, so 6.3 / 7.9 / 14.4).  A single one has nothing to wait for (8.1, so 8.6).
+    constexpr int LAYER = MT_H * KC_H * 64, AT_ONCE = 4;
+    const int all = n_hid * LAYER;
+    for (int u0 = tid; u0 < all; u0 += AT_ONCE * nthreads) {
+      uint2 lo[AT_ONCE], hi[AT_ONCE];
+#pragma unroll
+      for (int i = 0; i < AT_ONCE; ++i) {
+        const int u = u0 + i * nthreads < all ? u0 + i * nthreads : u0;
+        const int layer = u / LAYER, frag = u % LAYER >> 6, g = (u & 63) >> 4;
+        const uint16_t* w = a.w_hid + (size_t)(layer * HP + 16 * (frag / KC_H) + (u & 15)) * HP;
+        lo[i] = *reinterpret_cast<const uint2*>(w + k_chain(frag % KC_H, g, 0));
+        hi[i] = *reinterpret_cast<const uint2*>(w + k_chain(frag % KC_H, g, 4));
+      }
+#pragma unroll
+      for (int i = 0; i < AT_ONCE; ++i)
+        if (u0 + i * nthreads < all) *reinterpret_cast<uint4*>(f_hid + (size_t)(u0 + i * nthreads) * 8) = make_uint4(lo[i].x, lo[i].y, hi[i].x, hi[i].y);
+    }
+    stage_bias<T>(bias_hid, a.b_hid, n_hid * HP, n_hid * HP, tid, nthreads);
+  } else {
+    for (int k = 0; k < n_hid; ++k) {
+      stage_weight_frags<true, false>(f_hid + (size_t)k * MT_H * KC_H * FRAG_ELEMS, a.w_hid + (size_t)k * a.d_hidden * a.d_hidden, a.d_hidden,
+                                      a.d_hidden, MT_H, KC_H, tid, nthreads);
+      stage_bias<T>(bias_hid + k * HP, a.b_hid ? a.b_hid + (size_t)k * a.d_hidden : nullptr, a.d_hidden, HP, tid, nthreads);
+    }
+  }
+  stage_weight_frags<true, false>(f_out, a.w_out, a.d_out, a.d_hidden, MT_O, KC_H, tid, nthreads);
+  stage_bias<T>(bias_in, a.b_in, a.d_hidden, HP, tid, nthreads);
+  stage_bias<T>(bias_out, a.b_out, a.d_out, OUTP, tid, nthreads);
+  __syncthreads();
+
   for (int64_t chunk = first_chunk; chunk < n_chunks; chunk += wave_stride) {
     const int64_t row0 = chunk * 32;
     Frag in[2][2];

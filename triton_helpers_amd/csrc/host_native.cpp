@@ -271,11 +271,11 @@ variable_list mlp_backward(Mlp m, Tensor dy, bool need_dx, bool float_grads) {
   // its LDS does.  64 wide, us whole / chained: 32 -> 16 with two SiLU layers 2^19 rows 76 / 79, 2^20 140 / 132 (32 -> 3, whose rows are not
   // whole 8-byte pieces, 154 / 167); ReLU, 32 -> 16, 2^20 and 1.5M rows: three layers 132 to 142 / 132 and 185 / 167 (600k rows 92 / 96; 64 -> 64
   // 192 / 202 and 266 / 267), four 166 / 196 and 230 / 255, five 264 / 281 and 377 / 369, six 301 / 346 and 428 / 452, seven 394 / 436 and
-  // 560 / 587, nine 479 / 532 and 684 / 704.
+  // 560 / 587, nine 479 / 532 and 684 / 704 (float16 64 -> 64: seven 477 / 518 and 676 / 680, nine 562 / 601 and 799 / 771).
   const bool narrow = in <= 32 && in % 4 == 0 && out <= 16 && out % 4 == 0;
   const bool streams = H == 64 && m.x.scalar_type() == wt &&
                        (depth == 2 ? narrow && g.n > (3 << 18)
-                                   : relu && (depth == 3 || depth == 5) && g.n > (narrow && depth == 3 ? 3 << 18 : 5 << 18));
+                                   : relu && (depth == 3 || depth == 5 || (depth >= 7 && !narrow)) && g.n > (narrow && depth == 3 ? 3 << 18 : 5 << 18));
   const int64_t whole_bytes = streams ? 0 : nf_mlp_bwd_whole_workspace_bytes(g.n, H, depth, m.act, dt);
   // deeper: only the ReLU backward of a 64-wide network whose first launch has three linear layers converts x on the fly
   const bool converts = whole_bytes > 0 || (depth == 1 && relu && H == 64);

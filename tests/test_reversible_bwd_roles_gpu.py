@@ -4,6 +4,7 @@ stream's bits, and the batch's weight gradients are the sum of the parts'."""
 import pytest
 import torch
 
+from oracle import mlp as O
 from triton_helpers_amd import _lib
 
 pytestmark = pytest.mark.gpu
@@ -49,3 +50,41 @@ def test_a_batch_is_its_parts(cuts, pad, act, dtype, H, blocks):
         off = (a - b - c).abs()
         i = int(off.argmax())
         assert float(off.max()) <= 1.5e-4 * scale, (tuple(a.shape), i, *(float(t.flatten()[i]) for t in (a, b, c)))
+
+
+@pytest.mark.parametrize("act", ["gelu", "silu", "relu2"])
+@pytest.mark.parametrize("rows,full,H,blocks", [(33, 64, 64, 1), (1, 64, 64, 3), (50, 64, 32, 5), (70, 128, 40, 1), (16400, 16512, 64, 2), (16400, 16512, 32, 1)])
+def test_rows_that_are_not_there(rows, full, H, blocks, act):
+    """The biases take out a mean of the stream, so every row of the batch stays small, while on a row of zeros they alone drive a
+    coupling beyond float16's range.  The kernel rounds a batch up to 16 rows per chain wave: with those rows there (copies of the first with a zero
+    gradient, which add nothing) every gradient has the same bits, whatever a kernel makes of rows that are not there."""
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(rows + H + blocks)
+    mean, step, scale = (2048.0, 1.0, 64.0) if act == "relu2" else (8192.0, 8.0, 4.0)
+    w1, w2 = torch.randint(-2, 3, (blocks, 2 * H, H), generator=gen) / 16.0, torch.randint(1, 3, (blocks, 2 * H, H), generator=gen) / scale
+    w1[..., 0] = -1.0
+    w1 = torch.where(w1.sum(-1, keepdim=True) < 0, w1, -w1)
+    k = rows % blocks  # the coupling that overflows; the others change the stream by little
+    quiet = torch.arange(blocks) != k
+    w1[quiet] /= 64
+    w2[quiet] /= 64
+    params = [w1.view(-1, H), (-mean * w1.sum(-1)).view(blocks * 2, H), w2.view(-1, H), torch.zeros(blocks * 2, H)]
+    t = O.activation(params[1][2 * k + 1].half().float(), act).half().float()  # the hidden layer of a row of zeros
+    assert not torch.isfinite((w2[k, H:] @ t).half()).all(), "the case does not overflow on a row of zeros"
+    params = [p.half().cuda() for p in params]
+    y, dy = mean + step * torch.randint(-2, 3, (full, 2 * H), generator=gen), torch.randn(full, 2 * H, generator=gen)
+    y[rows:], dy[rows:] = y[0], 0.0
+    y, dy = y.half().cuda(), dy.half().cuda()
+    results = []
+    for n in (rows, full):
+        dx, x_rec = torch.empty_like(y), torch.empty_like(y)
+        g = [torch.full(p.shape, 7.0, device="cuda") for p in params]
+        need = lib.nf_revmlp_bwd_workspace_bytes(n, H, blocks)
+        ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        ptrs = [v for t in (y, dy, dx, x_rec) for v in (t.data_ptr(), t.stride(0))]
+        _lib.check(lib.nf_revmlp_bwd_summed(*ptrs, *(_lib.ptr(t) for t in (*params, *g)), n, H, blocks, _lib.NF_ACT[act], _lib.NF_F16, _lib.NF_F32,
+                                            ws.data_ptr(), need, _lib.current_stream(y.device)), "nf_revmlp_bwd_summed")
+        results.append([dx[:rows], x_rec[:rows], *g])
+    for a, b in zip(*results):
+        assert torch.isfinite(b).all(), "a row of the batch overflows: the case shows nothing"
+        assert torch.equal(a, b)

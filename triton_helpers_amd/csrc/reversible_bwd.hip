@@ -85,7 +85,7 @@ struct RevSlot {
 };
 constexpr int rev_couplings(int hp) { return hp == 64 ? 2 : 4; }  // couplings of a pass
 constexpr size_t rev_bwd_lds(int hp, int cw) {
-  return (size_t)rev_couplings(hp) * 4 * (hp * ROLES_PITCH + 64 * 4) + (size_t)4 * 16 * cw * ROLES_PITCH + 64 * 4;
+  return (size_t)rev_couplings(hp) * 4 * (hp * ROLES_PITCH + 64 * 4) + 4 * 64 * 4 + (size_t)4 * 16 * cw * ROLES_PITCH + 64 * 4;
 }
 
 // The weights of couplings k0 .. k0 + n - 1 as LDS matrices of HP rows, [coupling][F.w1, F.w2, G.w1, G.w2]: 8-byte piece 8kc + 4e + g of a row
@@ -139,9 +139,13 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void rev_bwd_k(RevBwdArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   char* weights = rev_smem;                                        // [CPL][F.w1, F.w2, G.w1, G.w2][HP][128]
   float* bias = reinterpret_cast<float*>(weights + CPL * 4 * MATRIX);  // [CPL][4][64]
-  char* areas = reinterpret_cast<char*>(bias + CPL * 4 * 64);      // [2][gradient rows | input rows][ROWS][128]
+  // Rows past the batch's end run the couplings too.  Their gradient is zero, but what the biases alone drive beyond the 16-bit range
+  // would reach dW as 0 * inf, within one coupling already.  They read zeros as biases: nothing but zeros goes through them then.
+  float* no_bias = bias + CPL * 4 * 64;                            // [4][64] zeros
+  char* areas = reinterpret_cast<char*>(no_bias + 4 * 64);         // [2][gradient rows | input rows][ROWS][128]
   Sections<CW> sections = {reinterpret_cast<int*>(areas + 2 * AREA), 0};
   if (threadIdx.x < 32) sections.flags[threadIdx.x] = 0;
+  if (threadIdx.x < 4 * 64) no_bias[threadIdx.x] = 0.0f;
   const int64_t per_round = (int64_t)gridDim.x * ROWS, rounds = (a.rows + per_round - 1) / per_round;
   const f32x4_t zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
 
@@ -288,13 +292,14 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void rev_bwd_k(RevBwdArgs a) {
       load_half(n2, e1, true, row0);
       for (int64_t round = 0; round < rounds; ++round) {
         const int64_t r = row0 + round * per_round;
+        const bool there = r < fresh_rev_args()->rows;
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc) {
           y1[kc] = n1[kc];
           y2[kc] = n2[kc];
           d1[kc] = e1[kc];
           d2[kc] = e2[kc];
-          if (r >= fresh_rev_args()->rows || 32 * kc + 8 * g >= fresh_rev_args()->half)
+          if (!there || 32 * kc + 8 * g >= fresh_rev_args()->half)
             y1[kc].u = y2[kc].u = d1[kc].u = d2[kc].u = make_uint4(0u, 0u, 0u, 0u);
         }
         // A wave's sixteen accesses to its rows keep the CU's address unit busy for 1000 clocks, and issued together the waves stand still for
@@ -302,7 +307,7 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void rev_bwd_k(RevBwdArgs a) {
 #pragma unroll 1
         for (int c = count - 1; c >= 0; --c) {
           const char* w = weights + c * 4 * MATRIX;
-          const float* b = bias + c * 4 * 64;
+          const float* b = there ? bias + c * 4 * 64 : no_bias;
           // G: y2 becomes x2, d1 the gradient of x1
           sub(w + 2 * MATRIX, b + 2 * 64, y1, d2, y2, d1, [&](int s) {
             if (c != count - 1) return;
@@ -313,10 +318,6 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void rev_bwd_k(RevBwdArgs a) {
           sub(w, b, y2, d1, y1, d2, [&](int s) {
             if (c == 0 && s == 0) store_half(y2, d1, true, r);
           });
-          if (r >= fresh_rev_args()->rows) {  // rows that are not there begin every coupling with zeros: what grows without bound here would reach dW as 0 * inf
-#pragma unroll
-            for (int kc = 0; kc < KC; ++kc) y1[kc].u = y2[kc].u = make_uint4(0u, 0u, 0u, 0u);
-          }
         }
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc) {

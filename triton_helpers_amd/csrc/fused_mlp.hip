@@ -236,7 +236,7 @@ __global__ __launch_bounds__(256) void mlp_bwd_k(MlpArgs a) {
   for (int nt = 0; nt < 2; ++nt) {
 #pragma unroll
     for (int kc = 0; kc < KC_IN; ++kc)
-      nx[nt][kc] = load_rows_frag(a.x, a.x_stride, first_chunk * 32 + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
+      nx[nt][kc] = load_rows_frag<true>(a.x, a.x_stride, first_chunk * 32 + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
 #pragma unroll
     for (int kc = 0; kc < KC_O; ++kc)
       ndy[nt][kc] = load_rows_frag(a.dy, a.dy_stride, first_chunk * 32 + 16 * nt, a.rows, a.d_out, kc, lane, a.dy_vec);
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(256) void mlp_bwd_k(MlpArgs a) {
       for (int kc = 0; kc < KC_IN; ++kc) {
         in[nt][kc] = nx[nt][kc];
         if (a.in_act != NF_ACT_NONE) in[nt][kc] = act_frag<T>(in[nt][kc], a.in_act);
-        nx[nt][kc] = load_rows_frag(a.x, a.x_stride, (chunk + wave_stride) * 32 + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
+        nx[nt][kc] = load_rows_frag<true>(a.x, a.x_stride, (chunk + wave_stride) * 32 + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
         park_frag_T(xT, kc, nt, lane, in[nt][kc]);
       }
 #pragma unroll

@@ -49,13 +49,17 @@ __device__ __forceinline__ uint32_t relu_gate_pk(uint32_t dh, uint32_t h) {
 }
 
 // B fragment in chain order straight from global memory: lane (n, g) gets features
-// 32*kc + 4*g .. +3 and 32*kc + 16 + 4*g .. +3 of row row0 + n; zero beyond `rows` / `width`.
+// 32*kc + 4*g .. +3 and 32*kc + 16 + 4*g .. +3 of row row0 + n; zero beyond `rows` / `width` (REPEAT as in load_rows_frag()).
+template <bool REPEAT>
 __device__ __forceinline__ Frag load_rows_frag_chain(const uint16_t* base, int64_t stride, int64_t row0, int64_t rows,
                                                      int width, int kc, int lane, bool vec_ok) {
   Frag f;
   f.u = make_uint4(0u, 0u, 0u, 0u);
-  const int64_t r = row0 + (lane & 15);
-  if (r >= rows) return f;
+  int64_t r = row0 + (lane & 15);
+  if (r >= rows) {
+    if (!REPEAT) return f;
+    r = rows - 1;
+  }
   const int c0 = 32 * kc + 4 * (lane >> 4);
   const uint16_t* p = base + r * stride + c0;
 #pragma unroll
@@ -77,14 +81,15 @@ __device__ __forceinline__ Frag load_rows_frag_chain(const uint16_t* base, int64
 }
 
 // Same fragment for the aligned case (8-byte aligned rows, width a multiple of 4): no branches, addresses of
-// lanes past the end of the batch or of the row are clamped in range and their data replaced by zero.
+// lanes past the end of the batch or of the row are clamped in range and their data (REPEAT: past the end of the row) replaced by zero.
+template <bool REPEAT>
 __device__ __forceinline__ Frag load_rows_frag_chain_fast(const uint16_t* base, int64_t stride, int64_t row0, int64_t rows,
                                                           int width, int kc, int lane) {
   const int64_t r = row0 + (lane & 15);
   const int c0 = 32 * kc + 4 * (lane >> 4);
-  const bool row_ok = r < rows;
+  const bool there = r < rows, row_ok = REPEAT || there;
   const bool lo_ok = row_ok && c0 < width, hi_ok = row_ok && c0 + 16 < width;
-  const uint16_t* p = base + (row_ok ? r : 0) * stride;
+  const uint16_t* p = base + (there ? r : REPEAT ? rows - 1 : 0) * stride;
   const uint2 lo = *reinterpret_cast<const uint2*>(p + (lo_ok ? c0 : 0));
   const uint2 hi = *reinterpret_cast<const uint2*>(p + (hi_ok ? c0 + 16 : 0));
   Frag f;
@@ -107,11 +112,11 @@ __device__ __forceinline__ void store_rows_tile_fast(uint16_t* base, int64_t str
   if (r < rows && c0 < width) *reinterpret_cast<uint2*>(base + r * stride + c0) = o;
 }
 
-template <bool FAST>
+template <bool FAST, bool REPEAT = false>
 __device__ __forceinline__ Frag load_chain(const uint16_t* base, int64_t stride, int64_t row0, int64_t rows, int width,
                                            int kc, int lane, bool vec_ok) {
-  if (FAST) return load_rows_frag_chain_fast(base, stride, row0, rows, width, kc, lane);
-  return load_rows_frag_chain(base, stride, row0, rows, width, kc, lane, vec_ok);
+  if (FAST) return load_rows_frag_chain_fast<REPEAT>(base, stride, row0, rows, width, kc, lane);
+  return load_rows_frag_chain<REPEAT>(base, stride, row0, rows, width, kc, lane, vec_ok);
 }
 
 // ---- rows behind a buffer descriptor -------------------------------------------------------
@@ -124,6 +129,13 @@ typedef unsigned int buf_v4u __attribute__((ext_vector_type(4)));
 constexpr uint32_t OUT_OF_RANGE = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* base, int64_t rows, int64_t stride) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)(rows * stride * 2), 0x00020000);
+}
+// Byte offset of the 16 rows from row0 on, to be added to piece_offset()s: for a lane whose row is past the end, of those that end with the
+// last row (REPEAT of load_rows_frag()).  In elements the offsets of rows_in_reach() fit 31 bits; with fewer than 16 rows the offset of the
+// first ones is negative and wraps, which a piece beyond the row's width, at 2^31 less a few rows, is still past the end with.
+__device__ __forceinline__ uint32_t repeated_rows(int64_t row0, int64_t rows, int64_t stride, int lane) {
+  const int last = ((int)rows - 1 - (lane & 15)) * (int)stride, at = (int)(row0 * stride);
+  return (uint32_t)(at < last ? at : last) << 1;
 }
 // What a launch needs of a tensor's extent for these 32-bit offsets to be safe: the tensor itself below 2^31 bytes
 // (the descriptor's range check then catches every row past the end), and the furthest row any lane ever addresses
@@ -223,14 +235,14 @@ __global__ __launch_bounds__(64 * WAVES, 1) void mlp_bwd2_k(MlpArgs a) {
   // rows of a chunk: tile nt starts (chunk * ROWS + 16 nt) rows into the tensor (a uniform value)
   auto load_x = [&](int64_t chunk, int nt, int kc) {
     if constexpr (BUF) {
-      const uint32_t at = (uint32_t)((chunk * ROWS + 16 * nt) * a.x_stride * 2);
+      const uint32_t at = repeated_rows(chunk * ROWS + 16 * nt, a.rows, a.x_stride, lane);
       const buf_v2u lo = __builtin_amdgcn_raw_buffer_load_b64(rs_x, off_x[kc][0] + at, 0, 0);
       const buf_v2u hi = __builtin_amdgcn_raw_buffer_load_b64(rs_x, off_x[kc][1] + at, 0, 0);
       Frag f;
       f.w[0] = lo[0]; f.w[1] = lo[1]; f.w[2] = hi[0]; f.w[3] = hi[1];
       return f;
     } else {
-      return load_chain<FAST>(a.x, a.x_stride, chunk * ROWS + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
+      return load_chain<FAST, true>(a.x, a.x_stride, chunk * ROWS + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
     }
   };
   auto load_dy = [&](int64_t chunk, int nt, int kc) {
@@ -853,7 +865,7 @@ __global__ __launch_bounds__(256) void mlp_bwdn_k(MlpArgs a) {
   for (int nt = 0; nt < NT; ++nt) {
 #pragma unroll
     for (int kc = 0; kc < KC_IN; ++kc)
-      nx[nt][kc] = load_chain<FAST>(a.x, a.x_stride, first_chunk * ROWS + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
+      nx[nt][kc] = load_chain<FAST, true>(a.x, a.x_stride, first_chunk * ROWS + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
 #pragma unroll
     for (int kc = 0; kc < KC_O; ++kc)
       ndy[nt][kc] = load_chain<FAST>(a.dy, a.dy_stride, first_chunk * ROWS + 16 * nt, a.rows, a.d_out, kc, lane, a.dy_vec);
@@ -872,7 +884,7 @@ __global__ __launch_bounds__(256) void mlp_bwdn_k(MlpArgs a) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) in[nt][kc].w[q] = relu_pk(in[nt][kc].w[q]);
         }
-        nx[nt][kc] = load_chain<FAST>(a.x, a.x_stride, (chunk + wave_stride) * ROWS + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
+        nx[nt][kc] = load_chain<FAST, true>(a.x, a.x_stride, (chunk + wave_stride) * ROWS + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
       }
 #pragma unroll
       for (int kc = 0; kc < KC_O; ++kc) {

@@ -137,18 +137,19 @@ __global__ __launch_bounds__(64 * (CH + WS_GRAD), 1) void mlp_bwd2_ws_k(MlpArgs 
     for (int h = 0; h < DY_HALVES; ++h) off_dy[kc][h] = piece_offset(lane & 15, DW ? 32 * kc + 8 * (lane >> 4) : 32 * kc + 16 * h + 4 * (lane >> 4), a.d_out, a.dy_stride);
 #pragma unroll
   for (int mt = 0; mt < MT_I; ++mt) off_dx[mt] = piece_offset(lane & 15, W ? 32 * (mt >> 1) + 8 * (lane >> 4) : 16 * mt + 4 * (lane >> 4), a.d_in, a.dx_stride);
-  // a chunk past the end (a wave without work in the last round) reads zeros and stores nothing
+  // a chunk past the end (a wave without work in the last round) reads zeros of dy and the last row of x, and stores nothing
   auto at = [&](int64_t chunk, int nt, int64_t stride, uint32_t off) {
     return chunk < n_chunks ? off + (uint32_t)((chunk * 32 + 16 * nt) * stride * 2) : OUT_OF_RANGE;
   };
   auto load_x = [&](int64_t chunk, int nt, int kc) {  // W: in natural order until it is used, and so dy
+    const uint32_t at_x = repeated_rows(chunk * 32 + 16 * nt, a.rows, a.x_stride, lane);
     if constexpr (W) {
       Frag f;
-      f.u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs_x, at(chunk, nt, a.x_stride, off_x[kc][0]), 0, 0));
+      f.u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs_x, off_x[kc][0] + at_x, 0, 0));
       return f;
     }
-    const buf_v2u lo = __builtin_amdgcn_raw_buffer_load_b64(rs_x, at(chunk, nt, a.x_stride, off_x[kc][0]), 0, 0);
-    const buf_v2u hi = __builtin_amdgcn_raw_buffer_load_b64(rs_x, at(chunk, nt, a.x_stride, off_x[kc][1]), 0, 0);
+    const buf_v2u lo = __builtin_amdgcn_raw_buffer_load_b64(rs_x, off_x[kc][0] + at_x, 0, 0);
+    const buf_v2u hi = __builtin_amdgcn_raw_buffer_load_b64(rs_x, off_x[kc][1] + at_x, 0, 0);
     Frag f;
     f.w[0] = lo[0]; f.w[1] = lo[1]; f.w[2] = hi[0]; f.w[3] = hi[1];
     return f;

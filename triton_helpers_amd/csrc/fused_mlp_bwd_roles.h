@@ -39,7 +39,7 @@ constexpr int ROLES_TILES = 16;                  // 16 x 16 tiles of a layer's d
 constexpr int ROLES_LAYER = (ROLES_TILES + 1) * 256;  // floats of a layer in a slot: its tiles, its bias sums
 constexpr int roles_slot_floats(int depth) { return (depth + 1) * ROLES_LAYER; }
 constexpr size_t roles_lds(int hp, int depth, int rows) {
-  return (size_t)(depth * hp + 64) * ROLES_PITCH + (size_t)2 * depth * hp * 4 + (size_t)4 * rows * ROLES_PITCH + 32 * 4;
+  return (size_t)(depth * hp + 64) * ROLES_PITCH + (size_t)depth * 64 * 4 + (size_t)4 * rows * ROLES_PITCH + 32 * 4;
 }
 static_assert(roles_lds(64, ROLES_MAX_DEPTH, 64) <= 160 * 1024, "LDS budget");
 
@@ -100,10 +100,8 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
   char* w_in = roles_smem;                                     // [HP][128]
   char* w_hid = w_in + HP * ROLES_PITCH;                       // [depth - 1][HP][128]
   char* w_out = w_hid + (size_t)(depth - 1) * HP * ROLES_PITCH;  // [64][128]
-  // Rows past the batch's end run the network too.  Their dz is zero, but an activation (or derivative) that the biases alone drive
-  // beyond the 16-bit range would enter dW as 0 * inf.  They read zeros as biases: nothing but zeros goes through them then.
-  float* bias = reinterpret_cast<float*>(w_out + 64 * ROLES_PITCH);  // [depth][HP], and as many zeros
-  char* areas = reinterpret_cast<char*>(bias + 2 * depth * HP);  // [2][dz rows | input rows][ROWS][128]
+  float* bias = reinterpret_cast<float*>(w_out + 64 * ROLES_PITCH);  // [depth][64]
+  char* areas = reinterpret_cast<char*>(bias + depth * 64);    // [2][dz rows | input rows][ROWS][128]
   constexpr int PANEL = ROWS * ROLES_PITCH, AREA = 2 * PANEL;
   Sections<CW> sections = {reinterpret_cast<int*>(areas + 2 * AREA), 0};
   if (tid < 32) sections.flags[tid] = 0;
@@ -127,9 +125,9 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
   stage_rows<THREADS>(w_in, a.w_in, 1, a.d_hidden, HP, a.d_in, tid);
   if (depth > 1) stage_rows<THREADS>(w_hid, a.w_hid, depth - 1, a.d_hidden, HP, a.d_hidden, tid);
   stage_rows<THREADS>(w_out, a.w_out, 1, a.d_out, 64, a.d_hidden, tid);
-  for (int i = tid; i < 2 * depth * HP; i += THREADS) {
-    const int l = i / HP, f = i % HP;
-    const uint16_t* b = l == 0 ? a.b_in : a.b_hid != nullptr && l < depth ? a.b_hid + (size_t)(l - 1) * a.d_hidden : nullptr;
+  for (int i = tid; i < depth * 64; i += THREADS) {
+    const int l = i >> 6, f = i & 63;
+    const uint16_t* b = l == 0 ? a.b_in : a.b_hid != nullptr ? a.b_hid + (size_t)(l - 1) * a.d_hidden : nullptr;
     bias[i] = b != nullptr && f < a.d_hidden ? T::to_f32(b[f]) : 0.0f;
   }
   __syncthreads();
@@ -157,8 +155,13 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
       const int64_t r = row0 + round * gridDim.x * ROWS;
       Frag h[MAXD][2], gate[RELU ? 1 : MAXD][2], x[2], cur[2], dz[2];  // h[0]: the last hidden layer
       f32x4_t acc[4];
-      const bool convert = fresh_args()->x_conv != 0;
-      const float* lane_bias = bias + 4 * g + (r < fresh_args()->rows ? 0 : opaque(a.depth) * HP);
+      const ArgsPtr k = fresh_args();
+      if (r >= k->rows) {  // past the batch's end x's last row again (REPEAT of load_rows_frag()).  Asked for ahead like the others it cost 4 % of nine layers
+#pragma unroll
+        for (int kc = 0; kc < 2; ++kc)
+          if (kc == 0 || two_in) nx[kc] = load_row8(k->x, k->x_stride, k->rows - 1, k->rows, k->d_in, 32 * kc + 8 * g, k->x_vec != 0);
+      }
+      const bool convert = k->x_conv != 0;
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc) {
         x[kc] = convert ? convert_frag(nx[kc], T::code == NF_BF16 ? 1 : 2) : nx[kc];
@@ -170,7 +173,7 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
       auto layer = [&](int l, bool natural) {
         const char* w = l == 0 ? w_in : w_hid + (l - 1) * HP * ROLES_PITCH;
         const int o0 = natural ? nat0 : chain0, o1 = natural ? nat0 ^ 8 : chain0 ^ 32;
-        const float* b = lane_bias + l * HP;
+        const float* b = bias + l * 64 + 4 * g;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[mt] = *reinterpret_cast<const f32x4_t*>(b + 16 * mt);
         auto chunk = [&](int kc) {
@@ -299,8 +302,8 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
       park(x, 1, HP == 32, two_in);
       load_rows(r + (int64_t)gridDim.x * ROWS);
       announce();
-      const ArgsPtr k = fresh_args();
-      if (k->dx != nullptr) {
+      const ArgsPtr kx = fresh_args();
+      if (kx->dx != nullptr) {
 #pragma unroll
         for (int kc = 0; kc < 2; ++kc) {
           if (kc == 1 && !two_in) continue;
@@ -317,7 +320,7 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
             o.w[2 * t] = convert ? pack2<Other>(v[0], v[1]) : pack2<T>(v[0], v[1]);
             o.w[2 * t + 1] = convert ? pack2<Other>(v[2], v[3]) : pack2<T>(v[2], v[3]);
           }
-          store_row8(k->dx, k->dx_stride, r, k->rows, k->d_in, 32 * kc + 8 * g, chain_to_nat(o), k->dx_vec != 0);
+          store_row8(kx->dx, kx->dx_stride, r, kx->rows, kx->d_in, 32 * kc + 8 * g, chain_to_nat(o), kx->dx_vec != 0);
         }
       }
     }

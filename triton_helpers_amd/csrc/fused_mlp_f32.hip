@@ -413,7 +413,7 @@ __global__ __launch_bounds__(64 * fused32_waves(TI, TO, DEPTH)) void mlp32_bwd_k
   const int64_t n_groups = (a.rows + 15) / 16, step = (int64_t)gridDim.x * WAVES;
   f32x4_t x_next[4];
   auto load_group = [&](int64_t grp) {
-    const int64_t row = grp * 16 + r;
+    const int64_t row = grp * 16 + r < a.rows ? grp * 16 + r : a.rows - 1;  // past the end the last row again, not zeros: see load_rows_frag()
 #pragma unroll
     for (int t = 0; t < TI; ++t) x_next[t] = load_chain(a.x, a.x_stride, row, a.rows, 16 * t + 4 * g, a.d_in, x_vec);
   };

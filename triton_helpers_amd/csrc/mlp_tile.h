@@ -288,12 +288,17 @@ __device__ __forceinline__ Frag lds_frag(const uint16_t* frags, int frag_index, 
 // ---- global <-> row-per-lane fragments ---------------------------------------------------
 // B fragment of K-chunk kc for 16 rows starting at row0: lane (n, g) gets features
 // 32*kc + 8*g .. +7 of row row0 + n; zero beyond `rows` / `width`.
+// REPEAT: rows beyond `rows` are the last row again.  So a backward loads x: what a row of zeros becomes on its way through the layers,
+// biases alone may drive beyond the 16-bit range, and dW = dz^T h would add 0 * inf for it; the last row again, its dz zero, adds
+// nothing that the row itself does not.
+template <bool REPEAT = false>
 __device__ __forceinline__ Frag load_rows_frag(const uint16_t* base, int64_t stride, int64_t row0, int64_t rows,
                                                int width, int kc, int lane, bool vec_ok) {
   Frag f;
   f.u = make_uint4(0u, 0u, 0u, 0u);
-  const int64_t r = row0 + (lane & 15);
+  int64_t r = row0 + (lane & 15);
   const int c0 = 32 * kc + 8 * (lane >> 4);
+  if (REPEAT && r >= rows) r = rows - 1;
   if (r < rows && c0 < width) {
     const uint16_t* p = base + r * stride + c0;
     if (vec_ok && c0 + 8 <= width) {

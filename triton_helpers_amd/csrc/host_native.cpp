@@ -277,9 +277,7 @@ variable_list mlp_backward(Mlp m, Tensor dy, bool need_dx, bool float_grads) {
                        (depth == 2 ? narrow && g.n > (3 << 18)
                                    : relu && (depth == 3 || depth == 5 || (depth >= 7 && !narrow)) && g.n > (narrow && depth == 3 ? 3 << 18 : 5 << 18));
   const int64_t whole_bytes = streams ? 0 : nf_mlp_bwd_whole_workspace_bytes(g.n, H, depth, m.act, dt);
-  // deeper: only the ReLU backward of a 64-wide network whose first launch has three linear layers converts x on the fly
-  const bool converts = whole_bytes > 0 || (depth == 1 && relu && H == 64);
-  if (m.x.scalar_type() != wt && !converts) m.x = m.x.to(wt);
+  if (m.x.scalar_type() != wt && whole_bytes == 0) m.x = m.x.to(wt);  // deeper networks, no rows
   Tensor flat, dx;
   const auto finish = [&](const Pieces& at, const Tensor& f) {
     return variable_list{dx, at.view(f, m.w[0], 0), at.view(f, m.w[1], 1), at.view(f, m.w[2], 2), at.view(f, m.w[3], 3), at.view(f, m.w[4], 4),
@@ -327,20 +325,13 @@ variable_list mlp_backward(Mlp m, Tensor dy, bool need_dx, bool float_grads) {
   flat = at::zeros({at.total}, m.w[0].options().dtype(at::kFloat));
   const int64_t bytes = nf_mlp_workspace_bytes(g.n, H, depth, m.act, 1, dt);
   const Tensor ws = scratch(bytes, m.x);
-  for (;;) {
-    const Rows x(m.x, in);
-    dx = need_dx ? at::empty(m.x.sizes(), m.x.options()) : Tensor();
-    const int rc = nf_mlp_bwd(x.p, x.stride, g.p, g.stride, ptr(dx), in, ptr(m.w[0]), ptr(m.w[1]), ptr(m.w[4]), ptr(m.w[5]), ptr(m.w[2]), ptr(m.w[3]),
-                              (float*)at.at(flat, m.w[0], 0), (float*)at.at(flat, m.w[1], 1), (float*)at.at(flat, m.w[4], 4),
-                              (float*)at.at(flat, m.w[5], 5), (float*)at.at(flat, m.w[2], 2), (float*)at.at(flat, m.w[3], 3), x.n, in, H, out, depth,
-                              m.act, dt, code_of(m.x.scalar_type()), ptr(ws), bytes, stream_of(m.x));
-    if (rc == NF_EUNSUPPORTED && m.x.scalar_type() != wt) {
-      m.x = m.x.to(wt);  // a shape / alignment the converting backward does not cover: cast first
-      continue;
-    }
-    check(rc, "nf_mlp_bwd");
-    break;
-  }
+  const Rows x(m.x, in);
+  dx = need_dx ? at::empty(m.x.sizes(), m.x.options()) : Tensor();
+  check(nf_mlp_bwd(x.p, x.stride, g.p, g.stride, ptr(dx), in, ptr(m.w[0]), ptr(m.w[1]), ptr(m.w[4]), ptr(m.w[5]), ptr(m.w[2]), ptr(m.w[3]),
+                   (float*)at.at(flat, m.w[0], 0), (float*)at.at(flat, m.w[1], 1), (float*)at.at(flat, m.w[4], 4), (float*)at.at(flat, m.w[5], 5),
+                   (float*)at.at(flat, m.w[2], 2), (float*)at.at(flat, m.w[3], 3), x.n, in, H, out, depth, m.act, dt, code_of(m.x.scalar_type()), ptr(ws),
+                   bytes, stream_of(m.x)),
+        "nf_mlp_bwd");
   // float32 accumulators, rounded once to the parameters' dtype (one kernel for all of them)
   return finish(at, float_grads || wt == at::kFloat ? flat : flat.to(wt));
 }

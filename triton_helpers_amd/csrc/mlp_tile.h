@@ -224,11 +224,10 @@ __device__ __forceinline__ void gate_apply(const f32x4_t dh, uint32_t g01, uint3
 // ---- staging weights into LDS as A fragments ------------------------------------------
 // dst: fragment array [MT][KC][64 lanes][8 elements]; element (mt, kc, lane(m,g), j) =
 //   transposed ? W[kmap(kc,g,j)][mmap(mt,m)] : W[mmap(mt,m)][kmap(kc,g,j)]
-// where W is [w_rows][w_cols] row-major, mmap(mt, m) = 16*mt + m, or wide_feature(mt, m) with WIDE_M; out-of-range
-// entries are zero.
+// where W is [w_rows][w_cols] row-major and mmap(mt, m) = 16*mt + m; out-of-range entries are zero.
 // NTHREADS > 0: the workgroup size is that compile-time constant, the loop is unrolled and all loads of a matrix
 // are in flight together.
-template <bool CHAIN, bool TRANSPOSED, int NTHREADS = 0, bool WIDE_M = false>
+template <bool CHAIN, bool TRANSPOSED, int NTHREADS = 0>
 __device__ __forceinline__ void stage_weight_frags(uint16_t* dst, const uint16_t* w, int w_rows, int w_cols, int MT,
                                                    int KC, int tid, int nthreads) {
   // one unit = the 8 elements of one lane of one fragment; the 8 loads of a unit are independent
@@ -238,7 +237,7 @@ __device__ __forceinline__ void stage_weight_frags(uint16_t* dst, const uint16_t
     const int lane = u & 63;
     const int frag = u >> 6;
     const int kc = frag % KC, mt = frag / KC;
-    const int m = WIDE_M ? wide_feature(mt, lane & 15) : 16 * mt + (lane & 15);
+    const int m = 16 * mt + (lane & 15);
     const int g = lane >> 4;
     uint16_t v[8];
     if (vec_ok && m < w_rows) {

@@ -267,17 +267,22 @@ variable_list mlp_backward(Mlp m, Tensor dy, bool need_dx, bool float_grads) {
   const bool relu = m.act == NF_ACT_RELU;
   if (dy.scalar_type() != wt) dy = dy.to(wt);
   const Rows g(dy, out);
+  Rows x(m.x, in);
   // Up to nine hidden layers: one launch for the whole backward, but where the kernels that nf_mlp_bwd chains stream many rows faster than
-  // its LDS does.  64 wide, us whole / chained: 32 -> 16 with two SiLU layers 2^19 rows 76 / 79, 2^20 140 / 132 (32 -> 3, whose rows are not
-  // whole 8-byte pieces, 154 / 167); ReLU, 32 -> 16, 2^20 and 1.5M rows: three layers 132 to 142 / 132 and 185 / 167 (600k rows 92 / 96; 64 -> 64
-  // 192 / 202 and 266 / 267), four 166 / 196 and 230 / 255, five 264 / 281 and 377 / 369, six 301 / 346 and 428 / 452, seven 394 / 436 and
-  // 560 / 587, nine 479 / 532 and 684 / 704 (float16 64 -> 64: seven 477 / 518 and 676 / 680, nine 562 / 601 and 799 / 771).
-  const bool narrow = in <= 32 && in % 4 == 0 && out <= 16 && out % 4 == 0;
-  const bool streams = H == 64 && m.x.scalar_type() == wt &&
-                       (depth == 2 ? narrow && g.n > (3 << 18)
-                                   : relu && (depth == 3 || depth == 5 || (depth >= 7 && !narrow)) && g.n > (narrow && depth == 3 ? 3 << 18 : 5 << 18));
+  // its LDS does.  64 wide on whole 8-byte pieces, us whole / chained: 32 -> 16 with two layers of another activation than ReLU 2^19 rows 85 / 84, 0.8 M
+  // 118 / 107, 2^20 142 / 132 (64 -> 64 197 / 272); with three ReLU layers 0.8 M 113 / 108, 1.5 M 187 / 167, 2^21 260 / 220 (64 -> 64 269 / 267 and
+  // 367 / 355 at the last two); five 381 / 373 and 527 / 497 (64 -> 64 442 / 438 and 605 / 580).  Whole is faster or as fast with four (1.5 M 236 / 254),
+  // six (433 / 448) and from seven on (563 / 585, nine 685 / 699; 64 -> 64 618 / 671, 739 / 763), in either type, and on other rows: 32 -> 16
+  // off 8-byte boundaries 0.8 M 122 / 155, 35 -> 3 with three layers 1.5 M 244 / 364.
+  const auto pieces = [](const Rows& r, int width) { return width % 4 == 0 && r.stride % 4 == 0 && (uintptr_t)r.p % 8 == 0; };
+  const bool narrow = in <= 32 && out <= 16;
+  const bool streams = H == 64 && m.x.scalar_type() == wt && pieces(x, in) && pieces(g, out) &&
+                       (depth == 2 ? narrow && g.n > 3 << 18 : relu && (depth == 3 || depth == 5) && g.n > (narrow && depth == 3 ? 3 << 18 : 7 << 18));
   const int64_t whole_bytes = streams ? 0 : nf_mlp_bwd_whole_workspace_bytes(g.n, H, depth, m.act, dt);
-  if (m.x.scalar_type() != wt && whole_bytes == 0) m.x = m.x.to(wt);  // deeper networks, no rows
+  if (m.x.scalar_type() != wt && whole_bytes == 0) {  // deeper networks, no rows
+    m.x = m.x.to(wt);
+    x = Rows(m.x, in);
+  }
   Tensor flat, dx;
   const auto finish = [&](const Pieces& at, const Tensor& f) {
     return variable_list{dx, at.view(f, m.w[0], 0), at.view(f, m.w[1], 1), at.view(f, m.w[2], 2), at.view(f, m.w[3], 3), at.view(f, m.w[4], 4),
@@ -297,7 +302,6 @@ variable_list mlp_backward(Mlp m, Tensor dy, bool need_dx, bool float_grads) {
     flat = at::empty({at.total}, float_grads ? m.w[0].options().dtype(at::kFloat) : m.w[0].options());
     const int64_t bytes = nf_mlp_bwd_rounded_workspace_bytes(in, H, out);
     const Tensor ws = scratch(bytes, m.x);
-    const Rows x(m.x, in);
     if (need_dx) dx = at::empty(m.x.sizes(), m.x.options());
     const int rc = nf_mlp_bwd_summed(x.p, x.stride, g.p, g.stride, ptr(dx), in, ptr(m.w[0]), ptr(m.w[1]), ptr(m.w[4]), ptr(m.w[5]), ptr(m.w[2]),
                                       ptr(m.w[3]), at.at(flat, m.w[0], 0), at.at(flat, m.w[1], 1), at.at(flat, m.w[4], 4), at.at(flat, m.w[5], 5),
@@ -312,7 +316,6 @@ variable_list mlp_backward(Mlp m, Tensor dy, bool need_dx, bool float_grads) {
     const Pieces at(m.w, 8);
     flat = at::empty({at.total}, float_grads ? m.w[0].options().dtype(at::kFloat) : m.w[0].options());
     const Tensor ws = scratch(whole_bytes, m.x);
-    const Rows x(m.x, in);
     dx = need_dx ? at::empty(m.x.sizes(), m.x.options()) : Tensor();
     check(nf_mlp_bwd_whole(x.p, x.stride, g.p, g.stride, ptr(dx), in, ptr(m.w[0]), ptr(m.w[1]), ptr(m.w[4]), ptr(m.w[5]), ptr(m.w[2]), ptr(m.w[3]),
                            at.at(flat, m.w[0], 0), at.at(flat, m.w[1], 1), at.at(flat, m.w[4], 4), at.at(flat, m.w[5], 5), at.at(flat, m.w[2], 2),
@@ -325,7 +328,6 @@ variable_list mlp_backward(Mlp m, Tensor dy, bool need_dx, bool float_grads) {
   flat = at::zeros({at.total}, m.w[0].options().dtype(at::kFloat));
   const int64_t bytes = nf_mlp_workspace_bytes(g.n, H, depth, m.act, 1, dt);
   const Tensor ws = scratch(bytes, m.x);
-  const Rows x(m.x, in);
   dx = need_dx ? at::empty(m.x.sizes(), m.x.options()) : Tensor();
   check(nf_mlp_bwd(x.p, x.stride, g.p, g.stride, ptr(dx), in, ptr(m.w[0]), ptr(m.w[1]), ptr(m.w[4]), ptr(m.w[5]), ptr(m.w[2]), ptr(m.w[3]),
                    (float*)at.at(flat, m.w[0], 0), (float*)at.at(flat, m.w[1], 1), (float*)at.at(flat, m.w[4], 4), (float*)at.at(flat, m.w[5], 5),

@@ -37,6 +37,20 @@ def test_library_exports_every_declared_symbol():
     assert f"#define NF_ABI_VERSION {_lib.NF_ABI_VERSION}" in header
 
 
+def test_a_compiler_without_a_feature_is_refused(monkeypatch):
+    """hipcc only prints a line for a GPU feature that it does not know, and that line for its host pass alone is expected."""
+    from triton_helpers_amd import build as b
+
+    try:
+        hipcc = b._hipcc()
+    except RuntimeError:
+        pytest.skip("no hipcc")
+    b.check_features(hipcc)
+    monkeypatch.setattr(b, "NO_MERGED_LDS", "-load-stor-opt")
+    with pytest.raises(RuntimeError, match="load-stor-opt"):
+        b.check_features(hipcc, (b.NO_PACKED_FP32, b.NO_MERGED_LDS))
+
+
 def test_library_allocates_and_waits_for_nothing():
     """The contract of every entry point: no device memory is taken or given back and no call waits, so none of these is imported."""
     from triton_helpers_amd import _lib

@@ -1,7 +1,8 @@
-"""The whole-network backward (nf_mlp_bwd_whole): against nf_mlp_bwd, the general path, over the forms both accept."""
+"""The whole-network backward (nf_mlp_bwd_whole): against the oracle, and against nf_mlp_bwd, the general path, over the forms both accept."""
 import pytest
 import torch
 
+from oracle import mlp as O
 from triton_helpers_amd import _lib
 
 NAMES = ("w_in", "b_in", "w_hid", "b_hid", "w_out", "b_out")
@@ -15,6 +16,8 @@ def test_what_it_covers():
     relu = _lib.NF_ACT["relu"]
     assert lib.nf_mlp_bwd_whole_workspace_bytes(1, 64, 1, relu, _lib.NF_F16) > 0
     assert lib.nf_mlp_bwd_whole_workspace_bytes(1 << 20, 16, 9, relu, _lib.NF_BF16) > 0
+    for H, tiles in ((16, 8), (32, 8), (64, 16)):  # one workgroup: a layer's 16 x 16 tiles and its bias sums
+        assert lib.nf_mlp_bwd_whole_workspace_bytes(1, H, 9, relu, _lib.NF_F16) == 10 * (tiles + 1) * 256 * 4
     for rows, depth, dtype in ((0, 2, _lib.NF_F16), (100, 10, _lib.NF_F16), (100, 2, _lib.NF_F32)):
         assert lib.nf_mlp_bwd_whole_workspace_bytes(rows, 64, depth, relu, dtype) == 0
         rc = lib.nf_mlp_bwd_whole(1, 32, 1, 16, None, 32, 1, None, 1, None, 1, None, 1, None, 1, None, 1, None,
@@ -64,7 +67,48 @@ CASES = [
     (40003, 35, 64, 3, 6, "relu", True, "bf16", False, 1, 1),
     (100003, 33, 32, 16, 4, "relu", True, "f16", False, 0, 0),
     (40003, 32, 16, 33, 6, "relu2", True, "bf16", False, 0, 0),
+    # two workgroups per compute unit (narrow deep ReLU) and twelve chain waves of another activation, each in more than one round
+    (100003, 32, 32, 16, 6, "relu", True, "bf16", False, 0, 0),
+    (100003, 40, 16, 40, 9, "relu", False, "f16", False, 0, 0),
+    (100003, 35, 32, 5, 3, "silu", True, "bf16", False, 1, 0),
 ]
+
+
+def _params(rows, d_in, H, d_out, depth, bias, dtype, gen):
+    def u(shape, fan_in):
+        return ((torch.rand(shape, generator=gen, device="cuda") * 2 - 1) * fan_in**-0.5).to(dtype)
+
+    return {"w_in": u((H, d_in), d_in), "w_out": u((d_out, H), H), "w_hid": u(((depth - 1) * H, H), H) if depth > 1 else None,
+            "b_in": u((H,), d_in) if bias else None, "b_out": u((d_out,), H) if bias else None,
+            "b_hid": u((depth - 1, H), H) if bias and depth > 1 else None}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [c for c in CASES if c[0] <= 1000], ids=lambda c: "-".join(map(str, c)))
+def test_whole_backward_is_the_oracles(case):
+    rows, d_in, H, d_out, depth, act, bias, dt, other, pad, shift = case
+    lib = _lib.load()
+    dtype = {"f16": torch.float16, "bf16": torch.bfloat16}[dt]
+    xt = dtype if not other else (torch.bfloat16 if dtype == torch.float16 else torch.float16)
+    gen = torch.Generator(device="cuda").manual_seed(rows + depth)
+    p = _params(rows, d_in, H, d_out, depth, bias, dtype, gen)
+    x, dy = _rows(rows, d_in, pad, shift, xt, gen), _rows(rows, d_out, pad, shift, dtype, gen)
+    got = {k: None if p[k] is None else torch.empty(p[k].shape, device="cuda") for k in NAMES}
+    dx = torch.empty(rows, d_in, dtype=xt, device="cuda")
+    code, a = _lib.dtype_code(dtype), _lib.NF_ACT[act]
+    n = lib.nf_mlp_bwd_whole_workspace_bytes(rows, H, depth, a, code)
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    _lib.check(lib.nf_mlp_bwd_whole(x.data_ptr(), x.stride(0), dy.data_ptr(), dy.stride(0), dx.data_ptr(), d_in, *(_lib.ptr(p[k]) for k in NAMES),
+                                    *(_lib.ptr(got[k]) for k in NAMES), rows, d_in, H, d_out, depth, a, code, _lib.dtype_code(xt), _lib.NF_F32,
+                                    ws.data_ptr(), n, _lib.current_stream(x.device)), "nf_mlp_bwd_whole")
+    cpu = {k: None if t is None else t.cpu() for k, t in p.items()}
+    want = O.mlp_backward(x.to(dtype).cpu(), dy.cpu(), *(cpu[k] for k in ("w_in", "b_in", "w_out", "b_out", "w_hid", "b_hid")), act=act, round_to=dtype)
+    # As a whole (2-norm): each layer's activation, derivative and gradient is rounded to 16 bit, half a unit each, on its way through at most
+    # depth + 1 layers (the oracle rounds the first alone), and dx to x's type.
+    eps = 3 * (depth + 1) * EPS[dtype] + EPS[xt]
+    for k, t in {"dx": dx, **{"d" + k: v for k, v in got.items()}}.items():
+        if t is not None:
+            assert float((t.cpu().double() - want[k].double()).norm()) <= eps * float(want[k].double().norm()), k
 
 
 @pytest.mark.gpu
@@ -75,13 +119,7 @@ def test_whole_backward_is_the_general_one(case):
     dtype = {"f16": torch.float16, "bf16": torch.bfloat16}[dt]
     xt = dtype if not other else (torch.bfloat16 if dtype == torch.float16 else torch.float16)
     gen = torch.Generator(device="cuda").manual_seed(rows + depth)
-
-    def u(shape, fan_in):
-        return ((torch.rand(shape, generator=gen, device="cuda") * 2 - 1) * fan_in**-0.5).to(dtype)
-
-    p = {"w_in": u((H, d_in), d_in), "w_out": u((d_out, H), H), "w_hid": u(((depth - 1) * H, H), H) if depth > 1 else None,
-         "b_in": u((H,), d_in) if bias else None, "b_out": u((d_out,), H) if bias else None,
-         "b_hid": u((depth - 1, H), H) if bias and depth > 1 else None}
+    p = _params(rows, d_in, H, d_out, depth, bias, dtype, gen)
     x, dy = _rows(rows, d_in, pad, shift, xt, gen), _rows(rows, d_out, pad, shift, dtype, gen)
     code, a = _lib.dtype_code(dtype), _lib.NF_ACT[act]
     stream = _lib.current_stream(x.device)

@@ -35,9 +35,12 @@ namespace nf {
 constexpr int ROLES_MAX_DEPTH = 9;               // hidden layers (MlpArgs::depth) of one launch
 // hidden layers of the kernels that leave registers for more waves (but for ReLU a layer's derivatives take as much room as its activations)
 constexpr int roles_shallow(int act) { return act == NF_ACT_RELU ? 4 : 3; }
-constexpr int ROLES_TILES = 16;                  // 16 x 16 tiles of a layer's dW in a slot (4 x 4, whether it has them all or not)
-constexpr int ROLES_LAYER = (ROLES_TILES + 1) * 256;  // floats of a layer in a slot: its tiles, its bias sums
-constexpr int roles_slot_floats(int depth) { return (depth + 1) * ROLES_LAYER; }
+// A layer in a slot: the 16 x 16 tiles of its dW (hidden width 64: 4 x 4; narrower: 2 x 4, the output layer's 4 x 2; whether it has them all or not),
+// then its bias sums in the place of another tile.  Nine layers are 44 MB (256 workgroups), narrow ones 47 MB (512).
+constexpr int roles_tiles(int hp) { return hp == 64 ? 16 : 8; }
+constexpr int roles_columns_log2(int hp, bool output) { return hp == 64 || !output ? 2 : 1; }  // tiles of a tile row
+constexpr int roles_layer_floats(int hp) { return (roles_tiles(hp) + 1) * 256; }
+constexpr int roles_slot_floats(int hp, int depth) { return (depth + 1) * roles_layer_floats(hp); }
 constexpr size_t roles_lds(int hp, int depth, int rows) {
   return (size_t)(depth * hp + 64) * ROLES_PITCH + (size_t)depth * 64 * 4 + (size_t)4 * rows * ROLES_PITCH + 32 * 4;
 }
@@ -416,12 +419,13 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
   // ---- this workgroup's slot: per layer (input first) tile (mt, nt) as the registers hold it, then the bias sums ----
   float* slot = a.partials + (size_t)blockIdx.x * a.partial_stride;
   auto put = [&](int layer, int mt, int nt, f32x4_t v) {
-    *reinterpret_cast<f32x4_t*>(slot + (size_t)layer * ROLES_LAYER + ((mt * 4 + nt) * 64 + lane) * 4) = v;
+    const int tile = (mt << roles_columns_log2(HP, layer == depth)) + nt;
+    *reinterpret_cast<f32x4_t*>(slot + (size_t)layer * roles_layer_floats(HP) + (tile * 64 + lane) * 4) = v;
   };
   auto put_bias = [&](int layer, int mt, float v) {
     v += __shfl_xor(v, 16);
     v += __shfl_xor(v, 32);
-    if (qn == 0 && lane < 16) slot[(size_t)layer * ROLES_LAYER + ROLES_TILES * 256 + 16 * mt + lane] = v;
+    if (qn == 0 && lane < 16) slot[(size_t)layer * roles_layer_floats(HP) + roles_tiles(HP) * 256 + 16 * mt + lane] = v;
   };
 #pragma unroll
   for (int i = 0; i < 2; ++i) {

@@ -13,9 +13,10 @@ struct RolesGrads {
 template <typename G>
 __global__ __launch_bounds__(1024) void mlp_sum_roles_k(const float* partials, int n_slots, int64_t slot_stride, RolesGrads p) {
   __shared__ f32x4_t part[16][64];
-  const int layer = blockIdx.x / (ROLES_TILES + 1), tile = blockIdx.x % (ROLES_TILES + 1), mt = tile >> 2, nt = tile & 3;
+  const int hp = p.d_hidden <= 32 ? 32 : 64, layer = blockIdx.y, tile = blockIdx.x;
+  const int columns_log2 = roles_columns_log2(hp, layer == p.depth), mt = tile >> columns_log2, nt = tile & ((1 << columns_log2) - 1);
   const int out_dim = layer == p.depth ? p.d_out : p.d_hidden, in_dim = layer == 0 ? p.d_in : p.d_hidden;
-  const bool bias = tile == ROLES_TILES;
+  const bool bias = tile == roles_tiles(hp);
   const size_t hid = (size_t)(layer - 1) * p.d_hidden;  // rows of the hidden layers in front (layers 1 .. depth - 1)
   typedef typename G::storage S;
   S* dst;
@@ -25,7 +26,7 @@ __global__ __launch_bounds__(1024) void mlp_sum_roles_k(const float* partials, i
   const int lane = threadIdx.x & 63, ty = threadIdx.x >> 6;
   f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
   if (!bias || 4 * lane < (out_dim + 15) / 16 * 16) {  // a bias block holds whole 16-value tiles of its layer
-    const float* src = partials + (size_t)layer * ROLES_LAYER + tile * 256 + lane * 4;
+    const float* src = partials + (size_t)layer * roles_layer_floats(hp) + tile * 256 + lane * 4;
     int sl = ty;
     for (; sl + 48 < n_slots; sl += 64) {
       f32x4_t v[4];
@@ -103,7 +104,7 @@ static int dispatch_act(const MlpArgs& a, const RolesPlan& p, hipStream_t s) {
 
 size_t mlp_bwd_roles_bytes(int64_t rows, int d_hidden, int depth, int act) {
   if (rows <= 0 || depth < 1 || depth > ROLES_MAX_DEPTH) return 0;
-  return (size_t)roles_plan(rows, d_hidden, depth, act).blocks * roles_slot_floats(depth) * sizeof(float);
+  return (size_t)roles_plan(rows, d_hidden, depth, act).blocks * roles_slot_floats(d_hidden <= 32 ? 32 : 64, depth) * sizeof(float);
 }
 
 int launch_mlp_bwd_roles(const MlpArgs& a0, int dtype, int grad_dtype, void* const out[6], void* workspace, hipStream_t s) {
@@ -111,7 +112,8 @@ int launch_mlp_bwd_roles(const MlpArgs& a0, int dtype, int grad_dtype, void* con
   const RolesPlan plan = roles_plan(a.rows, a.d_hidden, a.depth, a.act);
   if (a.dx != nullptr) a.dx_vec = vec_load_ok(a.dx, a.dx_stride, a.d_in);  // stored 16 bytes at a time
   a.partials = reinterpret_cast<float*>(workspace);
-  a.partial_stride = roles_slot_floats(a.depth);
+  const int hp = a.d_hidden <= 32 ? 32 : 64;
+  a.partial_stride = roles_slot_floats(hp, a.depth);
   int rc;
   if (a.d_hidden <= 32) rc = dtype == NF_BF16 ? dispatch_act<BF16, 32>(a, plan, s) : dispatch_act<F16, 32>(a, plan, s);
   else rc = dtype == NF_BF16 ? dispatch_act<BF16, 64>(a, plan, s) : dispatch_act<F16, 64>(a, plan, s);
@@ -124,7 +126,7 @@ int launch_mlp_bwd_roles(const MlpArgs& a0, int dtype, int grad_dtype, void* con
   const void* kern = grad_dtype == NF_F32    ? (const void*)mlp_sum_roles_k<F32>
                      : grad_dtype == NF_BF16 ? (const void*)mlp_sum_roles_k<BF16>
                                              : (const void*)mlp_sum_roles_k<F16>;
-  const hipError_t e = hipLaunchKernel(kern, dim3((unsigned)((a.depth + 1) * (ROLES_TILES + 1))), dim3(1024), args, 0, s);
+  const hipError_t e = hipLaunchKernel(kern, dim3((unsigned)roles_tiles(hp) + 1, (unsigned)a.depth + 1), dim3(1024), args, 0, s);
   if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(mlp_sum_roles): %s", hipGetErrorString(e));
   return check_launch("mlp_sum_roles");
 }

@@ -74,22 +74,22 @@ SHAPES = [
     ((1, 4097), 32, 64, 4, 2),   # BASELINE configs[4] geometry, ragged rows
     ((5, 77), 64, 64, 64, 4),
     ((2, 33), 17, 32, 33, 2),
-    # one hidden-to-hidden layer with a 64-wide input and / or output (ReLU: chain and gradient waves), ragged rows,
-    # widths padded up to the tile, more rows than one round of the grid covers
+    # (Up to nine hidden layers the backward of these few rows is the whole-network kernel; test_mlp_routes_gpu.py and
+    # test_wide_one_hidden_layer_many_rows reach the others.)  A 64-wide input and / or output, ragged rows, widths padded up to the tile
     ((5, 77), 64, 64, 64, 2),    # the reference's benchmark shape (fully_fused_mlp/__main__.py:16-23)
     ((1, 4099), 64, 64, 16, 2),
     ((2, 1000), 32, 64, 64, 2),
     ((1, 200), 48, 64, 40, 2),
-    # one hidden layer of width 64: the ReLU backward runs the two-layer kernels behind an identity layer
+    # one hidden layer of width 64
     ((1, 1000), 32, 64, 16, 1),
     ((1, 4099), 64, 64, 64, 1),
     ((2, 77), 27, 64, 3, 1),
-    # two or three hidden-to-hidden layers of width 64: ReLU takes the register-resident backward for deeper nets
+    # two or three hidden-to-hidden layers of width 64
     ((1, 1000), 32, 64, 16, 4),
     ((1, 1000), 32, 64, 16, 3),
     ((3, 100), 64, 64, 64, 3),
     ((2, 77), 40, 64, 20, 3),
-    # deeper than one launch covers: a chain of launches handing pre-activations over through the workspace
+    # deeper; twelve layers and more are a chain of launches handing pre-activations over through the workspace
     ((1, 300), 32, 64, 16, 5),
     ((2, 100), 64, 64, 64, 8),
     ((1, 203), 32, 64, 3, 12),
@@ -568,7 +568,8 @@ def test_decoder_shape_kernels(rows, d_in, d_out, bias, dtype, x_other, pad):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("bias", [True, False])
 @pytest.mark.parametrize("d_in,d_out", [(32, 16), (64, 64), (64, 16), (32, 64), (48, 40)])
-def test_rounded_weight_gradients_entry_point(dtype, bias, d_in, d_out):
+@pytest.mark.parametrize("depth", [1, 2])  # one hidden layer: behind an identity layer, whose own gradient is written nowhere
+def test_rounded_weight_gradients_entry_point(dtype, bias, d_in, d_out, depth):
     """nf_mlp_bwd_rounded against nf_mlp_bwd on the same inputs: the same dx bit for bit, weight and bias gradients equal to
     the float32 accumulators rounded once (one unit in the last place for the order of the sums), written into buffers
     that held garbage, and the same bits on a second call."""
@@ -578,7 +579,7 @@ def test_rounded_weight_gradients_entry_point(dtype, bias, d_in, d_out):
     rows, H = 50000, 64
     code = _lib.dtype_code(dtype)
     relu = _lib.NF_ACT["relu"]
-    p = {k: (None if v is None else v.to(DEV)) for k, v in _params(d_in, H, d_out, 2, bias, dtype, seed=5).items()}
+    p = {k: (None if v is None else v.to(DEV)) for k, v in _params(d_in, H, d_out, depth, bias, dtype, seed=5).items()}
     torch.manual_seed(5)
     x = torch.randn(rows, d_in, device=DEV).to(dtype)
     dy = torch.randn(rows, d_out, device=DEV).to(dtype)
@@ -588,7 +589,7 @@ def test_rounded_weight_gradients_entry_point(dtype, bias, d_in, d_out):
     dx_a = torch.empty_like(x)
     rc = lib.nf_mlp_bwd(x.data_ptr(), d_in, dy.data_ptr(), d_out, dx_a.data_ptr(), d_in,
                         *(_lib.ptr(p[k]) for k in names), *(_lib.ptr(acc[k]) for k in names),
-                        rows, d_in, H, d_out, 2, relu, code, code, None, 0, stream)
+                        rows, d_in, H, d_out, depth, relu, code, code, None, 0, stream)
     _lib.check(rc, "nf_mlp_bwd")
     n = lib.nf_mlp_bwd_rounded_workspace_bytes(d_in, H, d_out)
     ws = torch.empty(n, dtype=torch.uint8, device=DEV)
@@ -598,7 +599,7 @@ def test_rounded_weight_gradients_entry_point(dtype, bias, d_in, d_out):
         dx_b = torch.empty_like(x)
         rc = lib.nf_mlp_bwd_rounded(x.data_ptr(), d_in, dy.data_ptr(), d_out, dx_b.data_ptr(), d_in,
                                     *(_lib.ptr(p[k]) for k in names), *(_lib.ptr(out[k]) for k in names),
-                                    rows, d_in, H, d_out, 2, relu, code, code, ws.data_ptr(), n, stream)
+                                    rows, d_in, H, d_out, depth, relu, code, code, ws.data_ptr(), n, stream)
         _lib.check(rc, "nf_mlp_bwd_rounded")
         torch.cuda.synchronize()
         runs.append((dx_b, out))
@@ -617,5 +618,5 @@ def test_rounded_weight_gradients_entry_point(dtype, bias, d_in, d_out):
     # shapes it is not built for are refused before anything runs
     rc = lib.nf_mlp_bwd_rounded(x.data_ptr(), d_in, dy.data_ptr(), d_out, None, d_in,
                                 *(_lib.ptr(p[k]) for k in names), *(_lib.ptr(out[k]) for k in names),
-                                rows, d_in, H, d_out, 2, _lib.NF_ACT["silu"], code, code, ws.data_ptr(), n, stream)
-    assert rc == _lib.NF_EUNSUPPORTED
+                                rows, d_in, H, d_out, depth, _lib.NF_ACT["silu"], code, code, ws.data_ptr(), n, stream)
+    assert rc == (_lib.NF_EUNSUPPORTED if depth == 2 else -1)  # (but for ReLU one hidden layer lacks the hidden weights: an invalid argument)

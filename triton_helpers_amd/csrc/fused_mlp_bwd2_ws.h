@@ -21,8 +21,8 @@
 // The roles meet at three workgroup barriers per round.  A panel has one area per section ({h2, dy},
 // {h1, dz2}, {dz1, x}); a section is announced by the barrier in front of the NEXT section's stores, by which time its
 // own stores have long landed, and it is overwritten a full round later, after the gradient wave has passed three more
-// barriers.  Rows past the end of the batch read as zero through the buffer descriptors (a zero dy row contributes
-// nothing to any gradient) and their dx stores are dropped, so every wave runs every round and reaches every barrier.
+// barriers.  Rows past the end of the batch are zeros of dy (through the buffer descriptors) and the last row of x, which
+// contribute nothing to any gradient, and their dx stores are dropped, so every wave runs every round and reaches every barrier.
 #pragma once
 
 #include "fused_mlp_bwd2_kernels.h"

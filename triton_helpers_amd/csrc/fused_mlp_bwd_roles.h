@@ -1,16 +1,16 @@
 // Backward of a whole network in one launch: 16-bit tensors, any activation, one to nine hidden layers of width 16 .. 64,
 // any input and output width up to 64, rows of any alignment.  Weight gradients leave through one slot per workgroup.
 //
-// A workgroup is eight waves, two per SIMD, split by role (a wave's vector instructions do not start while one of its own
+// A workgroup is eight, twelve or sixteen waves, split by role (a wave's vector instructions do not start while one of its own
 // matrix products is in flight, so the two units of a SIMD overlap across waves only):
-//   * four or more chain waves own 16 rows of a round each.  A chain wave recomputes the forward with every layer's activations
+//   * four, eight or twelve chain waves own 16 rows of a round each.  A chain wave recomputes the forward with every layer's activations
 //     left in its registers (and, but for ReLU, the activation's derivative beside them), carries the gradient back
 //     through the layers, and per layer parks the two operands of dW = dz^T h in LDS, row-major;
 //   * four gradient waves own every other tile row and every other tile column of every layer's dW each and keep
 //     them in registers over the whole launch (160 of a wave's 256 at nine 64-wide hidden layers).  They read the parked
 //     operands back with the rows along K (ds_read_b64_tr_b16) while the chain waves work on the layer below.
-// The roles meet at one barrier per layer; the parked operands have two areas used in turn, so an area is written again
-// one barrier after its readers have passed theirs.  No tile is owned twice, so nothing is summed across waves at the end.
+// The roles hand a layer over at one barrier (four chain waves) or by flags in LDS (more of them); the parked operands have two areas used
+// in turn, so an area is written again when its readers are a layer further.  No tile is owned twice, so nothing is summed across waves at the end.
 //
 // LDS holds one copy of the weights, row-major in rows of 128 bytes: a product with W reads its fragments as rows, a
 // product with W^T reads the same bytes through the transposing reads, so ten 64-wide layers and the operand areas fit
@@ -19,12 +19,14 @@
 // What it replaces for most calls is up to five layers per launch, a replayed forward between launches, dW through LDS
 // transposes of 2-byte stores or matrix-core transposes, and atomics of all workgroups into cleared sums that a cast kernel
 // rounds.  Backward through autograd's host side, bfloat16, us before -> now at 2^11 / 2^16 / 2^18 rows: 64 -> 64 x 9 -> 64
-// ReLU 91 -> 23 / 168 -> 60 / 269 -> 171, 32 -> 64 x 4 -> 16 SiLU 47 -> 15 / 81 -> 41 / 168 -> 112, 35 -> 64 x 2 -> 3 ReLU
-// 20 -> 11 / 48 -> 23 / 76 -> 50, 32 -> 32 x 2 -> 16 ReLU 15 -> 10 / 31 -> 15 / 42 -> 27.
-// What bounds it: up to 2^16 rows the weights' staging, one chain of dependent layers per round and the slots (160 KB a
-// workgroup at nine layers); with many rows LDS, which moves 0.5 MB per 128 rows at depth 2 (half of the round's clocks; weight
+// ReLU 91 -> 20 / 168 -> 55 / 269 -> 145, 32 -> 64 x 4 -> 16 SiLU 47 -> 14 / 81 -> 39 / 168 -> 101, 35 -> 64 x 2 -> 3 ReLU
+// 20 -> 11 / 48 -> 22 / 76 -> 45, 32 -> 32 x 2 -> 16 ReLU 15 -> 10 / 31 -> 15 / 42 -> 26.
+// What bounds it: up to 2^16 rows the weights' staging, one chain of dependent layers per round and the slots (170 KB a
+// workgroup at nine layers): there its waves wait in 54 % of their clocks, LDS is busy 31 %, vector issue 27 %, the matrix cores 16 % (64 ->
+// 64 x 9 -> 64, 2^16 rows).  With many rows LDS (48 % busy with four layers and 2^18 rows, vector issue 40 %, matrix cores 23 %; weight
 // fragments are read once per 16 rows, as two tiles a wave need more registers than are left), and the rows' accesses at
-// one lane a clock.  Measured without the gradient waves' products it is 5 - 10 % quicker.
+// one lane a clock.  Measured without the gradient waves' products it is 5 - 10 % quicker.  The nine-layer ReLU form has no register to spare:
+// its time moves by up to 5 % with what the allocation makes of any change to its source.
 #pragma once
 
 #include "fused_mlp_bwd2_kernels.h"

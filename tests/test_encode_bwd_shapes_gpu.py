@@ -1,0 +1,38 @@
+"""The sorted-record backward at the edges of its work distribution, against the scattered-atomic kernel."""
+import pytest
+import torch
+
+from oracle import hash_encoding as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _grad(x, do, E, F, T, lo, hi, L, flags=0):
+    from triton_helpers_amd.layers.hash_encoding import kernel as hk
+
+    before, hk._FLAGS = hk._FLAGS, flags
+    try:
+        return hk.hash_encoding_table_grad(x, do, E, F, None, T, lo, hi, L)
+    finally:
+        hk._FLAGS = before
+
+
+# (points, levels): fill workgroups of 1, 2 and 4 levels, the last group short or of one level, the last block of points ragged
+@pytest.mark.parametrize("N,L", [(16384, 16), (16385, 7), (33000, 5), (65537, 17), (70000, 6), (131073, 3), (262144, 9)])
+@pytest.mark.parametrize("D,F,T,dtype", [(3, 2, 2**17, torch.float16), (3, 4, 2**15, torch.bfloat16), (2, 3, 2**16, torch.float32), (3, 2, 2**21, torch.float16)])
+def test_levels_dealt_to_fill_workgroups(N, L, D, F, T, dtype):
+    """A contribution is rounded to 2^-20 of its gradient (a dense cell's to 2^-17) and to 2^-30 of the level's largest, so a row's sum of n of
+    them is off by less than 2^-16 of n largest gradients; the atomics' float32 sum by 2^-24 of its n partial sums."""
+    torch.manual_seed(N + L)
+    lo, hi = 16, 2048
+    x = torch.rand(N, D, device=DEV)
+    x[0], x[1] = 0.0, 1.0
+    E = O.level_row_offsets(L, T, D, lo, hi)[-1]
+    do = torch.randn(N, L * F, device=DEV).to(dtype)
+    got = _grad(x, do, E, F, T, lo, hi, L, flags=16)
+    want = _grad(x, do, E, F, T, lo, hi, L, flags=2)
+    torch.testing.assert_close(got, want, rtol=1e-3, atol=1e-3)
+    level_sums = lambda t: [t[a:b].double().sum(0) for a, b in zip(O.level_row_offsets(L, T, D, lo, hi)[:-1], O.level_row_offsets(L, T, D, lo, hi)[1:])]  # noqa: E731
+    for l, s in enumerate(level_sums(got)):  # the weights of a cell add up to one
+        torch.testing.assert_close(s, do[:, l * F : (l + 1) * F].double().sum(0), rtol=0, atol=2**-16 * 5 * 8 * N**0.5)  # independent errors

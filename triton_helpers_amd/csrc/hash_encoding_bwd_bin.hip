@@ -5,7 +5,7 @@
 // global atomics is bound by the chip's atomic request rate; accumulating them in LDS needs the contributions to
 // one stretch of the table together.  So the contributions are first sorted by table bin (BIN_ROWS rows):
 //
-//   fill    : every workgroup takes some hundred consecutive points and, level by level, sorts their records by bin
+//   fill    : every workgroup takes some hundred consecutive points and a few levels and, level by level, sorts their records by bin
 //             in LDS and writes them out as one contiguous block, with the place of every bin inside the block
 //   totals  : the number of records of every bin
 //   accum   : a workgroup per compute unit takes task after task, a task being a bin (or, where a bin holds many more records
@@ -309,6 +309,8 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t m) {
 // ---------------------------------------------------------------------------------------
 // fill
 // ---------------------------------------------------------------------------------------
+// A workgroup takes some of the levels (blockIdx.y): a batch that leaves a unit one workgroup pays every level's barriers in turn (44 us for
+// sixteen levels at 2^14 to 2^17 points), several groups of levels cover each other's.
 // A level goes through three barriers: ranks inside the bins (LDS adds on one counter per bin), an exclusive scan of the
 // counters by one wave, the records into the stage in sorted order, and the stage out to the block.  The copy-out of a level runs
 // beside the hashing of the next one, and two or three workgroups per unit cover each other's barriers.
@@ -324,7 +326,7 @@ template <bool WIDE, bool G32, int D, int DX = 0>
 __global__ __launch_bounds__(WIDE ? FILL_WIDE_THREADS : FILL_THREADS, WIDE || G32 || DX ? 4 : 8) void hash_bwd_bin_fill_k(const void* coords, int cdt, int64_t csn, int64_t csd,
                                                                     const void* dout_v, int64_t dout_stride, int64_t N, int points,
                                                                     DevGeom g, BinPlan bp, const int64_t* primes, float scale,
-                                                                    BinWs ws, int max_nb, int feat, int f0, int hi) {
+                                                                    BinWs ws, int max_nb, int feat, int f0, int hi, int step) {
   extern __shared__ __align__(16) uint32_t fill_smem[];
   constexpr int RW = G32 ? 4 : 3;  // words of a record
   constexpr int THREADS = WIDE ? FILL_WIDE_THREADS : FILL_THREADS, POINTS = fill_points(WIDE), PPT = POINTS / THREADS;
@@ -337,7 +339,8 @@ __global__ __launch_bounds__(WIDE ? FILL_WIDE_THREADS : FILL_THREADS, WIDE || G3
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t n0 = (int64_t)blockIdx.x * points;
   const int here = N - n0 < points ? (int)(N - n0) : points;
-  if (blockIdx.x == 0)  // the header and the totals behind it
+  const int l_first = (int)blockIdx.y * step, l_end = min(l_first + step, bp.n_levels);  // the levels of this workgroup
+  if (blockIdx.x == 0 && blockIdx.y == 0)  // the header and the totals behind it
     for (int i = tid; i < (int)(sizeof(BinHeader) / 4) + bp.binbase[bp.n_levels]; i += THREADS) reinterpret_cast<uint32_t*>(ws.header)[i] = 0u;
   for (int i = tid; i < 2 * max_nb; i += THREADS) cnt0[i] = 0u;
   if (tid < NF_MAX_LEVELS) lmax[tid] = 0u;
@@ -412,10 +415,10 @@ __global__ __launch_bounds__(WIDE ? FILL_WIDE_THREADS : FILL_THREADS, WIDE || G3
   };
   lds_barrier();
 
-  for (int l = 0; l < bp.n_levels; ++l) {
+  for (int l = l_first; l < l_end; ++l) {
     const int nb = bp.nbins[l];
     uint32_t* cnt = cnt0 + (l & 1) * max_nb;
-    if ((l & 3) == 0) load_quad(l);
+    if (l == l_first || (l & 3) == 0) load_quad(l & ~3);
     uint32_t gp[PPT][G32 ? 2 : 1], m = 0u;
 #pragma unroll
     for (int i = 0; i < PPT; ++i) {
@@ -589,7 +592,7 @@ __global__ __launch_bounds__(WIDE ? FILL_WIDE_THREADS : FILL_THREADS, WIDE || G3
     const uint32_t pieces = (min(start[nb], ROOM) * RW + 3u) / 4u;
     for (uint32_t i = tid; i < pieces; i += THREADS) __builtin_nontemporal_store(reinterpret_cast<const Words4*>(stage)[i], reinterpret_cast<Words4*>(block) + i);
   }
-  if (tid < bp.n_levels) ws.block_max[(int64_t)tid * ws.blocks + blockIdx.x] = lmax[tid];
+  if (tid >= l_first && tid < l_end) ws.block_max[(int64_t)tid * ws.blocks + blockIdx.x] = lmax[tid];
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1738,14 +1741,19 @@ static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_
   const size_t acc_lds = (size_t)BIN_ROWS * 2 * sizeof(unsigned long long) + ((size_t)LIST + LIST_PAD + (NB < SPLIT_MAX_BINS ? NB : SPLIT_MAX_BINS) + 1 + (NB > SPLIT_MAX_BINS ? 2 * LATE_MAX : 0) + 2) * 4;
   auto launch = [&](const char* what, const void* kern, dim3 grid, int threads, void** args, size_t lds) { return launch_large(what, kern, grid, threads, args, lds, s); };
   const unsigned units = (unsigned)compute_units();
+  // Levels of a fill workgroup: four, whose gradients are one 16-byte piece of a row, or fewer where that leaves less than two workgroups a
+  // unit.  16 levels of 2^19 rows, fp16, uniform points, whole backward (us) with 16 / 4 / 2 / 1 levels to a workgroup: 2^14 points 100 / 72 /
+  // 67 / 66, 2^15 104 / 76 / 72 / 73, 2^16 108 / 83 / 84 / 84, 2^17 114 / 93 / 95 / 100, 2^18 145 / 134 / 136 / 147, 2^20 378 / 374 / 418 / 530.
+  int step = 4;
+  while (step > 1 && (int64_t)ws.blocks * ((bp.n_levels + step - 1) / step) < 2 * (int64_t)units) step /= 2;
   // more than three dimensions: the whole pipeline once per corner of the extra coordinates (`hi`), see ExtraDims
   const int passes = g.dims > 3 ? 1 << (g.dims - 3) : 1;
   for (int hi = 0; hi < passes; ++hi)
     for (int f0 = 0; f0 < feat; f0 += 2) {
       DevGeom gg = g;
       void* fill_args[] = {(void*)&coords, (void*)&cdt, (void*)&csn, (void*)&csd, (void*)&dout, (void*)&dout_stride, (void*)&N, (void*)&points,
-                           (void*)&gg, (void*)&bp, (void*)&primes, (void*)&scale, (void*)&ws, (void*)&max_nb, (void*)&feat, (void*)&f0, (void*)&hi};
-      if (int rc = launch("hash_bwd_bin_fill", fill, dim3((unsigned)ws.blocks), wide ? FILL_WIDE_THREADS : FILL_THREADS, fill_args, fill_lds)) return rc;
+                           (void*)&gg, (void*)&bp, (void*)&primes, (void*)&scale, (void*)&ws, (void*)&max_nb, (void*)&feat, (void*)&f0, (void*)&hi, (void*)&step};
+      if (int rc = launch("hash_bwd_bin_fill", fill, dim3((unsigned)ws.blocks, (unsigned)((bp.n_levels + step - 1) / step)), wide ? FILL_WIDE_THREADS : FILL_THREADS, fill_args, fill_lds)) return rc;
       void* totals_args[] = {(void*)&ws, (void*)&bp};
       const unsigned pieces = (unsigned)((ws.blocks + TOTALS_BLOCKS - 1) / TOTALS_BLOCKS);
       if (int rc = launch("hash_bwd_bin_totals", (const void*)hash_bwd_bin_totals_k, dim3((unsigned)bin_pieces, pieces), 64, totals_args, 0)) return rc;

@@ -36,3 +36,20 @@ def test_levels_dealt_to_fill_workgroups(N, L, D, F, T, dtype):
     level_sums = lambda t: [t[a:b].double().sum(0) for a, b in zip(O.level_row_offsets(L, T, D, lo, hi)[:-1], O.level_row_offsets(L, T, D, lo, hi)[1:])]  # noqa: E731
     for l, s in enumerate(level_sums(got)):  # the weights of a cell add up to one
         torch.testing.assert_close(s, do[:, l * F : (l + 1) * F].double().sum(0), rtol=0, atol=2**-16 * 5 * 8 * N**0.5)  # independent errors
+
+
+# one block more than a workgroup's threads, a second chunk of blocks, lists of more records than LDS holds at a time, fewer tasks than workgroups
+@pytest.mark.parametrize("N", [512 * 1024 + 1, 2**20 + 77])
+@pytest.mark.parametrize("cube", [1.0, 0.02])
+@pytest.mark.parametrize("F,T,L,dtype", [(2, 2**19, 3, torch.float16), (2, 2**14, 2, torch.bfloat16), (3, 2**17, 2, torch.float32)])
+def test_accumulation_in_chunks_of_blocks(N, cube, F, T, L, dtype):
+    """Bounds as above; a row of the cube sums up to 2^17 contributions, of which float32 keeps 2^-24 of each partial sum."""
+    torch.manual_seed(L)
+    lo, hi = 16, 2048
+    x = torch.rand(N, 3, device=DEV) * cube
+    E = O.level_row_offsets(L, T, 3, lo, hi)[-1]
+    do = torch.randn(N, L * F, device=DEV).to(dtype)
+    got = _grad(x, do, E, F, T, lo, hi, L, flags=16)
+    want = _grad(x, do, E, F, T, lo, hi, L, flags=2)
+    torch.testing.assert_close(got, want, rtol=1e-3, atol=2e-3 if cube == 1.0 else 2**-16 * 2**8.5 * 5)
+    assert torch.equal(got, _grad(x, do, E, F, T, lo, hi, L, flags=16))

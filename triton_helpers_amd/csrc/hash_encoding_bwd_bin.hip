@@ -40,9 +40,9 @@
 // not depend on the order of its records.  The tasks of a split bin are added in their order: a gradient has the same bits in
 // every run.  A level whose gradient holds an inf or a nan gets nan in every row it touches.
 //
-// One MI355X, 16 levels of 2^19 rows, fp16, uniform points, gradient of the table in its own type (before: count, offsets, fill
-// and accumulate passes over one run per bin, into a float32 table that was then converted): 8192 points 136 -> 92 us,
-// 2^18 184 -> 143, 2^20 506 -> 374, 2^21 947 -> 676; along rays 2^20 698 -> 431.
+// One MI355X, 16 levels of 2^19 rows, fp16, uniform points, gradient of the table in its own type (us): 2^14 points 45, 2^16 60, 2^17 75, 2^18 111,
+// 2^20 349, 2^21 646; along rays 2^18 126, 2^20 402.  (Before the levels were dealt to fill workgroups and the accumulation asked for the next
+// chunk's records ahead of the finished tile's way out: 100, 108, 114, 144, 379, 680; 158, 436.)
 //
 // Arithmetic (cell, corner rows, weights) is the forward's, see hash_encoding.hip.
 #include "hash_common.h"
@@ -61,13 +61,12 @@ constexpr int FILL_THREADS = 512, FILL_WIDE_THREADS = 1024;
 constexpr int fill_points(bool wide) { return wide ? 2 * FILL_WIDE_THREADS : FILL_THREADS; }
 constexpr int FILL_WIDE_BINS = 128;
 constexpr int64_t FILL_WIDE_POINTS = (int64_t)1 << 18;
-constexpr int ACC_THREADS = 1024;
+constexpr int ACC_THREADS = 1024;             // of sixteen waves
 constexpr int ACC_INFLIGHT = 2;               // records in flight per thread
 constexpr int GROUP = 16;                     // records named by one entry of a task's list
-constexpr int LIST = 5824;                    // entries of the list that LDS holds at a time
+constexpr int LIST = 5760;                    // entries of the list that LDS holds at a time
 constexpr int LIST_PAD = 2 * ACC_THREADS * ACC_INFLIGHT / GROUP;  // empty entries behind it
 constexpr int SPLIT_MAX_BINS = 1536;          // bins whose tasks LDS has a table for: those of the coarse levels, where points meet
-constexpr uint32_t SPLIT_MIN_COST = 32768;    // least cost (x-pair records) of a share of a split bin
 // Of the bins behind them only those of LATE_SHARES shares and more are split, listed one by one: all levels together come to 768 shares, and
 // of sixteen levels at most nine are behind, so LATE_MAX takes them (beyond it the shares grow).
 // Points in one cell and in a cube of 0.003, 16 levels of 2^21 rows, fp16 (us; these bins unsplit, this): 2^18 points 1690 and 1110, 800 and 575;
@@ -80,7 +79,8 @@ struct BinPlan {
   int n_levels;
   int nbins[NF_MAX_LEVELS];
   int binbase[NF_MAX_LEVELS + 1];  // first global bin of the level
-  int cell[NF_MAX_LEVELS];         // the level's records are cells (one per point) instead of x-pairs
+  int cell_levels;                 // leading levels whose records are cells (one per point) instead of x-pairs
+  int split_bins;                  // bins of the leading levels whose tasks LDS has a table for
   int64_t record_base[NF_MAX_LEVELS];  // first record of the level's blocks
   int block_records[NF_MAX_LEVELS];    // room of one block
 };
@@ -442,7 +442,7 @@ __global__ __launch_bounds__(WIDE ? FILL_WIDE_THREADS : FILL_THREADS, WIDE || G3
     // the records, and their ranks inside the bins: {bin, rank << 12}; ~0 where a pair does not reach into a second bin
     uint32_t rx[PPT][PAIRS], ry[PPT][PAIRS], at[PAIRS * PPT], at2[PAIRS * PPT];
     bool cells = false;
-    if constexpr (D == 3 && !G32 && DX == 0) cells = bp.cell[l] != 0;
+    if constexpr (D == 3 && !G32 && DX == 0) cells = l < bp.cell_levels;
     const int per_point = cells ? 1 : PAIRS;
 #pragma unroll
     for (int i = 0; i < PPT; ++i) {
@@ -596,50 +596,76 @@ __global__ __launch_bounds__(WIDE ? FILL_WIDE_THREADS : FILL_THREADS, WIDE || G3
 }
 
 // ---------------------------------------------------------------------------------------
-// totals: a wave adds up 64 bins of 64 blocks (and takes the largest |dout| of the level)
+// totals: a workgroup adds up 64 bins of some blocks (and takes the largest |dout| of the level)
 // ---------------------------------------------------------------------------------------
-constexpr int TOTALS_BLOCKS = 64;
-__global__ __launch_bounds__(64) void hash_bwd_bin_totals_k(BinWs ws, BinPlan bp) {
+// Bound by the latency of its loads, so a wave reads few blocks; and by the atomics of the workgroups, so those take many blocks.  A wave alone
+// with 64 blocks 10 us at 2^20 points (each with 8 of them 38), this 6.
+constexpr int TOTALS_WAVES = 16, TOTALS_ROWS = 16, TOTALS_BLOCKS = TOTALS_WAVES * TOTALS_ROWS;
+typedef uint32_t TwoStarts __attribute__((aligned(2)));  // places of two neighbouring bins in a block: first | second << 16
+__global__ __launch_bounds__(64 * TOTALS_WAVES) void hash_bwd_bin_totals_k(BinWs ws, BinPlan bp) {
+  __shared__ uint32_t part[TOTALS_WAVES][64], largest[TOTALS_WAVES];
   int first = blockIdx.x, l = 0;  // blockIdx.x counts pieces of 64 bins over all levels
   for (;; ++l) {
     const int pieces = (bp.nbins[l] + 63) / 64;
     if (first < pieces) break;
     first -= pieces;
   }
-  const int w0 = blockIdx.y * TOTALS_BLOCKS, w1 = min(w0 + TOTALS_BLOCKS, ws.blocks);
-  if (first == 0) {
-    const int w = w0 + (int)threadIdx.x;
-    const uint32_t m = wave_max_u32(w < w1 ? ws.block_max[(int64_t)l * ws.blocks + w] : 0u);
-    if (threadIdx.x == 63 && m) atomicMax(ws.header->gmax + l, m);
-  }
-  const int b = first * 64 + (int)threadIdx.x;
-  if (b >= bp.nbins[l]) return;
-  const uint16_t* mine = ws.starts + (int64_t)w0 * ws.start_stride + bp.binbase[l] + l + b;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int w0 = blockIdx.y * TOTALS_BLOCKS + wave * TOTALS_ROWS, w1 = min(w0 + TOTALS_ROWS, ws.blocks);
+  const int b = first * 64 + lane;
   uint32_t sum = 0;
-#pragma unroll 8
-  for (int w = w0; w < w1; ++w, mine += ws.start_stride) sum += (uint32_t)mine[1] - (uint32_t)mine[0];
-  if (sum) atomicAdd(ws.totals + bp.binbase[l] + b, sum);
+  if (b < bp.nbins[l]) {
+    const uint16_t* mine = ws.starts + (int64_t)w0 * ws.start_stride + bp.binbase[l] + l + b;
+#pragma unroll TOTALS_ROWS
+    for (int w = w0; w < w1; ++w, mine += ws.start_stride) {
+      const uint32_t two = *reinterpret_cast<const TwoStarts*>(mine);
+      sum += (two >> 16) - (two & 0xffffu);
+    }
+  }
+  part[wave][lane] = sum;
+  if (first == 0) {
+    const uint32_t m = wave_max_u32(lane < w1 - w0 ? ws.block_max[(int64_t)l * ws.blocks + w0 + lane] : 0u);
+    if (lane == 63) largest[wave] = m;
+  }
+  lds_barrier();
+  if (wave == 0) {
+    sum = 0;
+#pragma unroll
+    for (int w = 0; w < TOTALS_WAVES; ++w) sum += part[w][lane];
+    if (sum) atomicAdd(ws.totals + bp.binbase[l] + b, sum);
+    if (first == 0) {
+      const uint32_t m = wave_max_u32(lane < TOTALS_WAVES ? largest[lane] : 0u);
+      if (lane == 63 && m) atomicMax(ws.header->gmax + l, m);
+    }
+  }
 }
 
-__device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t x, uint32_t* wave_sums, uint32_t* total) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
-  uint32_t incl = x;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t y = (uint32_t)__shfl_up((int)incl, d);
-    if (lane >= d) incl += y;
-  }
-  __syncthreads();  // wave_sums may still be read from the previous call
-  if (lane == 63) wave_sums[wave] = incl;
-  __syncthreads();
-  uint32_t before = 0, all = 0;
-  for (int w = 0; w < nw; ++w) {
-    const uint32_t s = wave_sums[w];
-    if (w < wave) before += s;
-    all += s;
-  }
-  *total = all;
-  return before + incl - x;
+// Sums of the lanes up to each one, inside rows of 16 and over the whole wave (the moves of wave_max_u32).
+__device__ __forceinline__ uint32_t row_scan_u32(uint32_t x) {
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+  return x;
+}
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t x) {
+  x = row_scan_u32(x);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);
+  return x;
+}
+
+// Sum of the threads in front of this one, of a workgroup of sixteen waves: one barrier.  `sums` alternates between two arrays from one
+// call to the next, so that a wave may still read one while another writes the other.
+constexpr int ACC_WAVES = 16;
+__device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t x, uint32_t* sums, uint32_t* total) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const uint32_t incl = wave_scan_u32(x);
+  if (lane == 63) sums[wave] = incl;
+  lds_barrier();
+  const uint32_t up_to = row_scan_u32(sums[lane & (ACC_WAVES - 1)]);
+  *total = (uint32_t)__builtin_amdgcn_readlane((int)up_to, ACC_WAVES - 1);
+  return (wave ? (uint32_t)__builtin_amdgcn_readlane((int)up_to, wave - 1) : 0u) + incl - x;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -714,6 +740,12 @@ __host__ __device__ __forceinline__ auto with_mode(int mode, Body&& body) {
   }
 }
 
+// What bounds it: 2^20 points, 64-bit adds (108 us of the LDS pipe at the 4.6 lanes a clock and unit that random rows reach) next to 800 MB of
+// records (130 us); what came on top were the phases of a task, one after the other.  A workgroup planned for 10 - 14 us before its first record (scans
+// through LDS, an answer of the task counter, a search of the levels per bin; now 6 - 8), made a task's list in 3 - 5 us and waited for
+// its first records behind that.  Now the next chunk's list is made when the last add is done and its records come while the tile leaves:
+// 2^14 points 46 -> 26 us, 2^17 57 -> 42, 2^18 along rays added to float32 104 -> 87, 2^20 212 -> 190.  (Cells and pairs mixed, as cells keep the LDS pipe busy and
+// pairs the memory: 2^20 uniform 351 instead of 356 us for the whole chain, 2^21 690 instead of 660, 2^17 along rays 109 instead of 96.)
 // TWO: rows of two features have kernels of their own, which the addresses of other rows cost nine registers and 3 us at 2^18 points
 template <typename GT, int MODE, bool TWO>
 __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, void* table, DevGeom g, BinPlan bp, int row_feat, int f0) {
@@ -723,24 +755,28 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
   extern __shared__ unsigned long long acc_tile[];
   uint32_t* list = reinterpret_cast<uint32_t*>(acc_tile + 2 * BIN_ROWS);  // [LIST + LIST_PAD] first word of up to GROUP records in the level | their number << 27
   uint32_t* first_task = list + LIST + LIST_PAD;                          // [SB + 1] first task of a bin | its first slot << 16
-  __shared__ uint32_t next_task[2], wave_sums[ACC_THREADS / 64];
-  __shared__ int level_base[NF_MAX_LEVELS];
-  const int tid = threadIdx.x, feat = TWO ? 2 : row_feat;
-  const int NB = bp.binbase[bp.n_levels];
-  int SB = 0;  // bins of the leading levels
-  for (int l = 0; l < bp.n_levels && bp.binbase[l + 1] <= SPLIT_MAX_BINS; ++l) SB = bp.binbase[l + 1];
+  __shared__ uint32_t next_task, wave_sums[2][ACC_WAVES], level_max[NF_MAX_LEVELS];
+  const int tid = threadIdx.x, lane = tid & 63, feat = TWO ? 2 : row_feat;
+  const int NB = bp.binbase[bp.n_levels], SB = bp.split_bins, cell_bins = bp.binbase[bp.cell_levels];
+  // What has to come from memory is asked for first: the number of a second task, and the bins' totals
+  // (An address that is the same in all lanes would have the compiler broadcast the counter's answer, that is, wait for it and for every load
+  // in front of it: 0.7 - 2 us a task.)
+  uint32_t lane_zero;
+  asm volatile("v_mov_b32 %0, 0" : "=v"(lane_zero));
+  uint32_t* const counter = &ws.header->next_task + lane_zero;
+  uint32_t ticket = 0u;
+  if (tid == 0) ticket = atomicAdd(counter, 1u);
+  const uint32_t first_total = ws.totals[min(tid, NB - 1)], first_max = ws.header->gmax[min(tid, NF_MAX_LEVELS - 1)];
+  const int level_base = lane < bp.n_levels ? bp.binbase[lane] : NB;  // of the lane's level
   uint32_t* late = first_task + SB + 1;  // [n_late + 1] heavy bins behind those: bin, its first further share | its first slot << 16
-  for (uint32_t i = tid; i < 2u * BIN_ROWS; i += ACC_THREADS) acc_tile[i] = 0ull;
-  if (tid < bp.n_levels) level_base[tid] = bp.binbase[tid];
-  __syncthreads();
+  for (uint32_t i = tid; i < BIN_ROWS; i += ACC_THREADS) reinterpret_cast<uint4*>(acc_tile)[i] = make_uint4(0u, 0u, 0u, 0u);
+  if (tid < NF_MAX_LEVELS) level_max[tid] = first_max;
   // The tasks, worked out by every workgroup for itself: one per bin of the leading levels, several for a bin of more than one and a half
   // shares; the further shares of heavy bins behind those; and one per bin behind them, which takes a heavy bin's first share.  Where
   // the slots (or the list of heavy bins) do not reach, larger shares.
-  uint32_t split_tasks, late_tasks, n_late;
-  const auto cost_of = [&](int b, int& l) {  // l: a level at or in front of the bin's
-    while (l + 1 < bp.n_levels && b >= level_base[l + 1]) ++l;
-    return ws.totals[b] * (bp.cell[l] ? CELL_COST : 1u);
-  };
+  uint32_t split_tasks, late_tasks, n_late, turn = 0;
+  const auto scan = [&](uint32_t x, uint32_t* total) { return block_exclusive_scan(x, wave_sums[turn++ & 1u], total); };
+  const auto cost_of = [&](int b, uint32_t total) { return total * (b < cell_bins ? CELL_COST : 1u); };
   for (uint32_t share = ws.split_cost;; share += share / 4u) {
     const auto parts_of = [&](uint32_t cost) { return min((cost + share - 1u) / share, (uint32_t)ws.blocks); };
     uint32_t slots = 0, total;
@@ -749,24 +785,22 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
       const int b = b0 + tid;
       uint32_t n = 0;
       if (b < SB) {
-        int l = 0;
-        const uint32_t cost = cost_of(b, l);
+        const uint32_t cost = cost_of(b, b0 == 0 ? first_total : ws.totals[b]);
         n = cost <= share + share / 2 ? 1u : parts_of(cost);
         if (cost == 0u && MODE == TABLE_ADD) n = 0u;  // nothing to add (a table that is written gets its zeros)
       }
-      const uint32_t slot = slots + block_exclusive_scan(n > 1u ? n : 0u, wave_sums, &total);
-      slots += total;
-      const uint32_t first = split_tasks + block_exclusive_scan(n, wave_sums, &total);
-      split_tasks += total;
-      if (b < SB) first_task[b] = first | slot << 16;
+      // tasks and slots in one scan: neither comes to 2^16 (all levels together are at most 8 * 192 shares)
+      const uint32_t before = scan(n | (n > 1u ? n : 0u) << 16, &total);
+      if (b < SB) first_task[b] = (before & 0xffffu) + split_tasks | ((before >> 16) + slots) << 16;
+      split_tasks += total & 0xffffu;
+      slots += total >> 16;
     }
     n_late = late_tasks = 0u;
     if (SB < NB) {
       uint32_t heavy = 0, parts = 0;
       const auto each_heavy = [&](auto&& body) {
-        int l = 0;
         for (int b = SB + tid; b < NB; b += ACC_THREADS) {
-          const uint32_t cost = cost_of(b, l);
+          const uint32_t cost = cost_of(b, ws.totals[b]);
           if (cost >= LATE_SHARES * ws.split_cost && cost > share + share / 2 && ws.blocks > 1) body(b, parts_of(cost));
         }
       };
@@ -774,8 +808,8 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
         ++heavy;
         parts += n;
       });
-      uint32_t at = block_exclusive_scan(heavy, wave_sums, &n_late);
-      uint32_t slot = slots + block_exclusive_scan(parts, wave_sums, &total), first = slot - slots - at;
+      uint32_t at = scan(heavy, &n_late);
+      uint32_t slot = slots + scan(parts, &total), first = slot - slots - at;
       slots += total;
       late_tasks = total - n_late;
       if (heavy && n_late <= (uint32_t)LATE_MAX)
@@ -792,22 +826,24 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
   if (tid == 0) {
     first_task[SB] = split_tasks;
     late[2u * n_late + 1u] = late_tasks;
+    next_task = gridDim.x + ticket;
   }
+  lds_barrier();
   const uint32_t n_tasks = split_tasks + late_tasks + (uint32_t)(NB - SB);
+  if (blockIdx.x >= n_tasks) return;
   // What a task needs, the same for all threads.
   struct Task {
     int bin, level, block0, block1;
     uint32_t slot;
   };
-  const int lane = tid & 63;
   auto task_of = [&](uint32_t t) {
     Task k = {SB + (int)(t - split_tasks - late_tasks), 0, 0, ws.blocks, ~0u};
     // share `which` of n: its blocks, and its slot
     auto share = [&](uint32_t which, uint32_t n, uint32_t slot) {
       if (n <= 1u) return;
       k.slot = slot + which;
-      k.block0 = (int)((int64_t)ws.blocks * which / n);
-      k.block1 = (int)((int64_t)ws.blocks * (which + 1u) / n);
+      k.block0 = (int)((uint32_t)ws.blocks * which / n);  // (at most 4096 blocks, and no more shares than those)
+      k.block1 = (int)((uint32_t)ws.blocks * (which + 1u) / n);
     };
     if (t < split_tasks) {
       // the bin whose first task is the last one not behind t (a bin without tasks shares it with the one behind it), found
@@ -833,7 +869,7 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
         share(further ? t - split_tasks - e0 + 1u : 0u, (late[2u * i + 3u] & 0xffffu) - e0 + 1u, at >> 16);
       }
     }
-    k.level = __builtin_popcountll(__ballot(lane < bp.n_levels && level_base[lane] <= k.bin)) - 1;
+    k.level = __builtin_popcountll(__ballot(lane < bp.n_levels && level_base <= k.bin)) - 1;
     k.bin = __builtin_amdgcn_readfirstlane(k.bin);
     k.level = __builtin_amdgcn_readfirstlane(k.level);
     k.block0 = __builtin_amdgcn_readfirstlane(k.block0);
@@ -841,24 +877,85 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
     k.slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)k.slot);
     return k;
   };
-  // where this thread's block of the task's first ACC_THREADS has the bin's records: {first, end}
-  auto block_part = [&](const Task& k, int w) {
-    uint2 r = make_uint2(0u, 0u);
-    if (w < k.block1) {
-      const uint16_t* s = ws.starts + (int64_t)w * ws.start_stride + k.bin + k.level;
-      r = make_uint2(s[0], s[1]);
+  // an odd feature count leaves the last pass with one feature: plane 1 then has no column in the table
+  const bool has_pair = TWO || f0 + 1 < feat;
+  constexpr uint32_t RW = sizeof(Rec) / 4;
+  // A task's blocks, ACC_THREADS at a time, and where this thread's block has the bin's records: first | end << 16 (asked for without a
+  // branch, at the end of which they would be waited for).
+  struct Chunk {
+    Task task;
+    int w0;
+    bool valid, last;
+    uint32_t part;
+  };
+  auto chunk_of = [&](const Task& k, int w0) {
+    const int w = min(w0 + tid, k.block1 - 1);
+    const uint32_t part = *reinterpret_cast<const TwoStarts*>(ws.starts + (int64_t)w * ws.start_stride + k.bin + k.level);
+    return Chunk{k, w0, true, w0 + ACC_THREADS >= k.block1, part};
+  };
+  // Places in the sequence come from a counter, fetched a task ahead, and so are the places of the next chunk's records: neither is
+  // waited for.  Every workgroup leaves as soon as the counter has passed the last task.
+  uint32_t t_next = (uint32_t)__builtin_amdgcn_readfirstlane((int)next_task);
+  bool taken = false;  // the next place has been asked for
+  auto chunk_behind = [&](const Chunk& c) {
+    if (!c.last) return chunk_of(c.task, c.w0 + ACC_THREADS);
+    if (t_next >= n_tasks) return Chunk{c.task, c.task.block1, false, true, 0u};
+    if (tid == 0) ticket = atomicAdd(counter, 1u);
+    taken = true;
+    const Task k = task_of(t_next);
+    return chunk_of(k, k.block0);
+  };
+  // The level's records behind a buffer descriptor: a lane without a record asks for one past the end and gets zeros (zero
+  // weights), so the loop carries no bounds tests.
+  auto records_of = [&](int l) {
+    return __builtin_amdgcn_make_buffer_rsrc(ws.records + bp.record_base[l] * (int64_t)RW, 0,
+                                             (int)((uint32_t)ws.blocks * (uint32_t)bp.block_records[l] * (uint32_t)sizeof(Rec)), 0x00020000);
+  };
+  // The chunk's records as a list of groups, up to LIST of them at a time.
+  struct Groups {
+    uint32_t at, c, mine, before, all;
+  };
+  auto groups_of = [&](const Chunk& k) {  // (one barrier)
+    Groups s;
+    s.at = ((uint32_t)(k.w0 + tid) * (uint32_t)bp.block_records[k.task.level] + (k.part & 0xffffu)) * RW;
+    s.c = k.w0 + tid < k.task.block1 ? (k.part >> 16) - (k.part & 0xffffu) : 0u;
+    s.mine = (s.c + GROUP - 1u) / GROUP;
+    s.before = scan(s.mine, &s.all);
+    return s;
+  };
+  auto write_list = [&](const Groups& s, uint32_t e0) {  // entries e0 .. e0 + LIST; returns how many there are
+    for (uint32_t e = s.before < e0 ? e0 : s.before; e < s.before + s.mine && e < e0 + LIST; ++e) {
+      const uint32_t k = (e - s.before) * GROUP;
+      list[e - e0] = (s.at + k * RW) | min(s.c - k, (uint32_t)GROUP) << 27;
+    }
+    const uint32_t now = min(s.all - e0, (uint32_t)LIST);
+    for (uint32_t e = now + tid; e < now + LIST_PAD; e += ACC_THREADS) list[e] = 0u;
+    return now;
+  };
+  const uint32_t in_group = (uint32_t)tid % GROUP;
+  auto load_rec = [&](const __amdgpu_buffer_rsrc_t& rs, uint32_t entry) {
+    const uint32_t at = in_group < entry >> 27 ? (entry & 0x7ffffffu) * 4u + in_group * (uint32_t)sizeof(Rec) : 0xf0000000u;
+    Rec r;
+    if constexpr (sizeof(Rec) == 12) {
+      typedef unsigned int v3u __attribute__((ext_vector_type(3)));
+      const v3u v = __builtin_amdgcn_raw_buffer_load_b96(rs, at, 0, 0);
+      r.x = v[0]; r.y = v[1]; r.z = v[2];
+    } else {
+      typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+      const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0);
+      r.x = v[0]; r.y = v[1]; r.z = v[2]; r.w = v[3];
     }
     return r;
   };
-  // an odd feature count leaves the last pass with one feature: plane 1 then has no column in the table
-  const bool has_pair = TWO || f0 + 1 < feat;
-  // Task numbers come from a counter, fetched a task ahead, and so are the places of the next task's records: neither is waited
-  // for.  Every workgroup leaves as soon as the counter has passed the last task.
-  if (tid == 0) {
-    next_task[0] = atomicAdd(&ws.header->next_task, 1u);
-    next_task[1] = atomicAdd(&ws.header->next_task, 1u);
-  }
-  __syncthreads();
+  constexpr uint32_t ROUND = ACC_THREADS * ACC_INFLIGHT;
+  Rec q[ACC_INFLIGHT];  // the records of a round, a round ahead of their adds
+  const uint32_t* mine = list + (uint32_t)tid / GROUP;
+  auto load_round = [&](const __amdgpu_buffer_rsrc_t& rs, uint32_t e) {
+#pragma unroll
+    for (int k = 0; k < ACC_INFLIGHT; ++k) q[k] = load_rec(rs, mine[e + k * (ACC_THREADS / GROUP)]);
+  };
+  const Task first_of_all = task_of(blockIdx.x);
+  Chunk now = chunk_of(first_of_all, first_of_all.block0);
   if (blockIdx.x == 0) {  // for the kernel behind this one
     const auto split = [&](uint32_t b, uint32_t slot, uint32_t n) {
       if (n > 1u) ws.splits[atomicAdd(&ws.header->n_splits, 1u)] = BinSplit{b, slot, n, 0u};
@@ -866,17 +963,16 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
     for (int b = tid; b < SB; b += ACC_THREADS) split((uint32_t)b, first_task[b] >> 16, (first_task[b + 1] & 0xffffu) - (first_task[b] & 0xffffu));
     for (uint32_t i = tid; i < n_late; i += ACC_THREADS) split(late[2u * i], late[2u * i + 1u] >> 16, (late[2u * i + 3u] & 0xffffu) - (late[2u * i + 1u] & 0xffffu) + 1u);
   }
-  uint32_t t = next_task[0], t_next = next_task[1];
-  if (t >= n_tasks) return;
-  Task task = task_of(t);
-  uint2 part = block_part(task, task.block0 + tid);
+  Groups groups = groups_of(now);
+  uint32_t entries = write_list(groups, 0);
+  lds_barrier();
+  load_round(records_of(now.task.level), 0);
+  Chunk next = chunk_behind(now);
   for (;;) {
+    const Task& task = now.task;
     const int l = task.level;
-    const uint32_t row0 = (uint32_t)(task.bin - bp.binbase[l]) << BIN_ROWS_LOG2;
-    const uint32_t left = g.rows[l] - row0;
-    const uint32_t nrows = left < (uint32_t)BIN_ROWS ? left : (uint32_t)BIN_ROWS;
     // fixed-point scale 2^se of the level:  |w * g| * 2^se < 2^30
-    const float gm = BinRec<GT>::level_max(ws.header->gmax[l]);
+    const float gm = BinRec<GT>::level_max(level_max[l]);
     const bool nonfinite = !(gm <= 3.0e38f);
     int se = 0;
     if (!nonfinite && gm > 0.0f) {
@@ -887,48 +983,17 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
     }
     const float scale = nonfinite ? 0.0f : ldexpf(1.0f, se);  // |g| * 2^se < 2^30, and |se| stays inside float's exponents
     const float scale_w = scale * (1.0f / (float)W_MAX);      // with the decoding of the pair records' weights
-    // The level's records behind a buffer descriptor: a lane without a record asks for one past the end and gets zeros (zero
-    // weights), so the loop carries no bounds tests.
-    constexpr uint32_t RW = sizeof(Rec) / 4;
-    const uint32_t room = (uint32_t)bp.block_records[l];
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(ws.records + bp.record_base[l] * (int64_t)RW, 0,
-                                                                        (int)((uint32_t)ws.blocks * room * (uint32_t)sizeof(Rec)), 0x00020000);
-    const uint32_t in_group = (uint32_t)tid % GROUP;
-    auto load_rec = [&](uint32_t entry) {
-      const uint32_t at = in_group < entry >> 27 ? (entry & 0x7ffffffu) * 4u + in_group * (uint32_t)sizeof(Rec) : 0xf0000000u;
-      Rec r;
-      if constexpr (sizeof(Rec) == 12) {
-        typedef unsigned int v3u __attribute__((ext_vector_type(3)));
-        const v3u v = __builtin_amdgcn_raw_buffer_load_b96(rs, at, 0, 0);
-        r.x = v[0]; r.y = v[1]; r.z = v[2];
-      } else {
-        typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-        const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0);
-        r.x = v[0]; r.y = v[1]; r.z = v[2]; r.w = v[3];
-      }
-      return r;
-    };
+    const __amdgpu_buffer_rsrc_t rs = records_of(l);
     // a lane without a record, and a record without a gradient, add nothing
     auto live = [](const Rec& r) {
       if constexpr (sizeof(Rec) == 12) return (r.z & 0x7fff7fffu) != 0u;
       else return ((r.z | r.w) & 0x7fffffffu) != 0u;
     };
     auto add_to = [&](uint32_t at, int32_t v) { atomicAdd(acc_tile + at, (unsigned long long)(long long)v); };
-    constexpr uint32_t ROUND = ACC_THREADS * ACC_INFLIGHT;
-    // The next round's records are loaded before this round's adds; a level with an inf or a nan in its gradient only marks the
-    // rows it touches (its own copy of the loop, so that the usual one has no test per record).
-    auto rounds = [&](uint32_t entries, auto add) {
-      const uint32_t* mine = list + (uint32_t)tid / GROUP;  // (the list goes on with empty entries for two rounds)
-      Rec q[ACC_INFLIGHT];
-#pragma unroll
-      for (int k = 0; k < ACC_INFLIGHT; ++k) q[k] = load_rec(mine[k * (ACC_THREADS / GROUP)]);
-      for (uint32_t e = 0; e < entries; e += ROUND / GROUP) {
-        mine += ROUND / GROUP;
-        add(q, [&] {
-#pragma unroll
-          for (int k = 0; k < ACC_INFLIGHT; ++k) q[k] = load_rec(mine[k * (ACC_THREADS / GROUP)]);
-        });
-      }
+    // The next round's records are loaded before this round's adds (the list goes on with empty entries for two rounds); a level with an inf
+    // or a nan in its gradient only marks the rows it touches (its own copy of the loop, so that the usual one has no test per record).
+    auto rounds = [&](auto add) {
+      for (uint32_t e = 0; e < entries; e += ROUND / GROUP) add(q, [&] { load_round(rs, e + ROUND / GROUP); });
     };
     auto add_pairs = [&](auto nonfinite_c) {
       constexpr bool NONFINITE = decltype(nonfinite_c)::value;
@@ -1001,42 +1066,44 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
       };
     };
     bool cells = false;
-    if constexpr (sizeof(Rec) == 12) cells = bp.cell[l] != 0;
-    // the task's records, listed for up to ACC_THREADS blocks and LIST entries at a time
-    Task task_next = {};
-    uint2 part_next = make_uint2(0u, 0u);
-    uint32_t t_later = 0u;
-    bool ahead = false;
-    for (int w0 = task.block0; w0 < task.block1; w0 += ACC_THREADS) {
-      if (w0 != task.block0) part = block_part(task, w0 + tid);
-      const uint32_t at = ((uint32_t)(w0 + tid) * room + part.x) * RW, c = part.y - part.x, mine = (c + GROUP - 1u) / GROUP;
-      uint32_t entries;
-      const uint32_t before = block_exclusive_scan(mine, wave_sums, &entries);
-      for (uint32_t e0 = 0; e0 == 0 || e0 < entries; e0 += LIST) {
-        for (uint32_t e = before < e0 ? e0 : before; e < before + mine && e < e0 + LIST; ++e) {
-          const uint32_t k = (e - before) * GROUP;
-          list[e - e0] = (at + k * RW) | min(c - k, (uint32_t)GROUP) << 27;
-        }
-        const uint32_t now = min(entries - e0, (uint32_t)LIST);
-        for (uint32_t e = now + tid; e < now + LIST_PAD; e += ACC_THREADS) list[e] = 0u;
-        if (!ahead) {
-          ahead = true;
-          if (t_next < n_tasks) {
-            task_next = task_of(t_next);
-            part_next = block_part(task_next, task_next.block0 + tid);
-          }
-          if (tid == 0) t_later = atomicAdd(&ws.header->next_task, 1u);
-        }
-        lds_barrier();
-        if (cells) {
-          if (nonfinite) rounds(now, add_cells(std::true_type{}));
-          else rounds(now, add_cells(std::false_type{}));
-        } else if (nonfinite) rounds(now, add_pairs(std::true_type{}));
-        else rounds(now, add_pairs(std::false_type{}));
-        if (tid == 0) next_task[0] = t_later;
-        lds_barrier();
-      }
+    if constexpr (sizeof(Rec) == 12) cells = l < bp.cell_levels;
+    auto add_list = [&] {
+      if (cells) {
+        if (nonfinite) rounds(add_cells(std::true_type{}));
+        else rounds(add_cells(std::false_type{}));
+      } else if (nonfinite) rounds(add_pairs(std::true_type{}));
+      else rounds(add_pairs(std::false_type{}));
+    };
+    add_list();
+    for (uint32_t e0 = LIST; e0 < groups.all; e0 += LIST) {  // (a bin of very many records)
+      lds_barrier();
+      entries = write_list(groups, e0);
+      lds_barrier();
+      load_round(rs, 0);
+      add_list();
     }
+    // The next chunk's list takes the place of this one's and its first records are asked for; then, under way with those, the
+    // finished tile leaves.
+    if (tid == 0 && taken) next_task = gridDim.x + ticket;
+    groups = groups_of(next);
+    if (taken) t_next = (uint32_t)__builtin_amdgcn_readfirstlane((int)next_task);
+    taken = false;
+    const bool done = now.last;
+    Chunk behind = next;
+    if (next.valid) {
+      entries = write_list(groups, 0);
+      lds_barrier();
+      load_round(records_of(next.task.level), 0);
+      behind = chunk_behind(next);
+    }
+    if (!done) {
+      now = next;
+      next = behind;
+      continue;
+    }
+    const uint32_t row0 = (uint32_t)(task.bin - bp.binbase[l]) << BIN_ROWS_LOG2;
+    const uint32_t left = g.rows[l] - row0;
+    const uint32_t nrows = left < (uint32_t)BIN_ROWS ? left : (uint32_t)BIN_ROWS;
     // the tile to the table (or the task's slot), and back to zero for the next task
     const float qnan = __uint_as_float(0x7fc00000u);
     const int64_t first = (g.row_offset[l] + (int64_t)row0) * feat + f0;  // features f0, f0 + 1 of the bin's rows
@@ -1113,11 +1180,10 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
         }
       }
     }
-    if (t_next >= n_tasks) return;
-    t_next = next_task[0];
-    task = task_next;
-    part = part_next;
-    // (the scan of the next task's parts has barriers between this task's last use of the tile and the next adds)
+    if (!next.valid) return;
+    lds_barrier();  // the tile is clear
+    now = next;
+    next = behind;
   }
 }
 
@@ -1450,6 +1516,7 @@ static bool bin_plan(int64_t N, int points, const nf_hash_geom* geom, BinPlan* b
   // features are taken two at a time (one pass of fill + accumulate per pair; the last feature of an odd count alone)
   if (geom->dims < 2 || geom->dims > NF_MAX_DIMS || geom->feat < 1 || N <= 0) return false;
   bp->n_levels = geom->levels;
+  bp->cell_levels = bp->split_bins = 0;
   const int64_t blocks = (N + points - 1) / points;
   int nb_total = 0;
   int64_t R = 0;
@@ -1460,13 +1527,15 @@ static bool bin_plan(int64_t N, int points, const nf_hash_geom* geom, BinPlan* b
     bp->nbins[l] = (int)nb;
     bp->binbase[l] = nb_total;
     const int64_t res = geom->res[l];
-    bp->cell[l] = cells && geom->dims == 3 && l < geom->first_hash_level && res * res + res + 1 < BIN_ROWS;
+    const bool cell = cells && geom->dims == 3 && l < geom->first_hash_level && res * res + res + 1 < BIN_ROWS && bp->cell_levels == l;
+    if (cell) bp->cell_levels = l + 1;
     // a cell level leaves at most two records per point; an x-pair level has room for every pair to be split in two
     // (normally half of it is used); more than three dimensions run as passes of the 3-D pipeline
-    bp->block_records[l] = points * (bp->cell[l] ? 2 : geom->dims >= 3 ? 8 : 4);
+    bp->block_records[l] = points * (cell ? 2 : geom->dims >= 3 ? 8 : 4);
     bp->record_base[l] = R;
     R += blocks * bp->block_records[l];
     nb_total += (int)nb;
+    if (nb_total <= SPLIT_MAX_BINS) bp->split_bins = nb_total;
   }
   bp->binbase[geom->levels] = nb_total;
   *records = R;
@@ -1481,6 +1550,15 @@ static bool wide_blocks(int64_t n_points, const nf_hash_geom* geom) {
   return false;
 }
 
+// Cost (x-pair records) of a share of a split bin: a third of what a compute unit gets of them on every level, and no less than pays for the
+// slot that the share is summed in.  16 levels of 2^19 rows, fp16, whole backward (us), least share 8192 / 16384 / 32768: along rays 2^14 points
+// 52 / 60 / 73, 2^16 76 / 73 / 88, 2^17 91 / 87 / 97; uniform 2^18 115 / 115 / 111, added to float32 129 / 128 / 124.
+static int64_t split_cost(int64_t N, int levels) {
+  const int64_t third = N * levels / 192, small = N < 32768 ? 8192 : N < 65536 ? N / 4 : 16384, large = N < 262144 ? N / 8 : 32768;
+  const int64_t least = small > large ? small : large;
+  return third > least ? third : least;
+}
+
 static int64_t bin_ws(void* workspace, const BinPlan& bp, int64_t N, int points, int64_t R, int rec_words, BinWs* ws) {
   char* p = (char*)workspace;
   const int NB = bp.binbase[bp.n_levels];
@@ -1493,9 +1571,7 @@ static int64_t bin_ws(void* workspace, const BinPlan& bp, int64_t N, int points,
   };
   ws->blocks = (int)blocks;
   ws->start_stride = (NB + bp.n_levels + 1) & ~1;
-  // a share of a split bin: a third of what a compute unit gets of x-pair records on every level
-  const int64_t share = N * bp.n_levels / 192;
-  ws->split_cost = (uint32_t)(share > SPLIT_MIN_COST ? share : SPLIT_MIN_COST);
+  ws->split_cost = (uint32_t)split_cost(N, bp.n_levels);
   ws->max_slots = (uint32_t)(16 + N / 1024);
   ws->header = (BinHeader*)take(sizeof(BinHeader) + NB * 4);
   ws->totals = (uint32_t*)(ws->header + 1);
@@ -1756,7 +1832,7 @@ static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_
       if (int rc = launch("hash_bwd_bin_fill", fill, dim3((unsigned)ws.blocks, (unsigned)((bp.n_levels + step - 1) / step)), wide ? FILL_WIDE_THREADS : FILL_THREADS, fill_args, fill_lds)) return rc;
       void* totals_args[] = {(void*)&ws, (void*)&bp};
       const unsigned pieces = (unsigned)((ws.blocks + TOTALS_BLOCKS - 1) / TOTALS_BLOCKS);
-      if (int rc = launch("hash_bwd_bin_totals", (const void*)hash_bwd_bin_totals_k, dim3((unsigned)bin_pieces, pieces), 64, totals_args, 0)) return rc;
+      if (int rc = launch("hash_bwd_bin_totals", (const void*)hash_bwd_bin_totals_k, dim3((unsigned)bin_pieces, pieces), 64 * TOTALS_WAVES, totals_args, 0)) return rc;
       void* acc_args[] = {(void*)&ws, (void*)&table, (void*)&gg, (void*)&bp, (void*)&feat, (void*)&f0};
       if (int rc = launch("hash_bwd_bin_accum", accum, dim3(units), ACC_THREADS, acc_args, acc_lds)) return rc;
       const unsigned max_splits = (unsigned)NB < ws.max_slots / 2 ? (unsigned)NB : ws.max_slots / 2;

@@ -49,6 +49,29 @@ def test_forward_with_levels_in_lds(N, dims, F, T, L, dtype, monkeypatch):
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
 
 
+@pytest.mark.parametrize("N", [1, 255, 257, 16384, 40960, 40961, 65535, 65537])
+@pytest.mark.parametrize("dims,F,T,L,dtype", [
+    (3, 2, 2**19, 16, torch.float16), (3, 4, 2**19, 16, torch.bfloat16), (3, 4, 2**20, 8, torch.float16), (3, 8, 2**17, 16, torch.float16), (3, 2, 2**18, 5, torch.float32),
+    (3, 4, 2**16, 7, torch.float32), (2, 2, 2**16, 3, torch.float32), (2, 4, 2**15, 4, torch.float16), (3, 2, 2**19, 20, torch.float16),
+])
+def test_forward_per_point_and_level(N, dims, F, T, L, dtype, monkeypatch):
+    """Rows of 4, 8 and 16 bytes, units of work dealt out in turn and XCD by XCD: the bits of the generic kernel (flag 1), on the upper edge too,
+    and into rows of a wider output, which may not be aligned."""
+    from triton_helpers_amd.layers.hash_encoding import kernel as hk
+
+    torch.manual_seed(8)
+    x = torch.rand(N, dims, device=DEV)
+    x[: N // 8, 0] = 1.0
+    x[: N // 16] = 1.0
+    table = torch.randn(O.level_row_offsets(L, T, dims, 16, 4000)[-1], F, device=DEV).to(dtype)
+    tail = torch.zeros(N, 3, device=DEV, dtype=dtype)
+    outs = []
+    for flags in (0, 1):
+        monkeypatch.setattr(hk, "_FLAGS", flags)
+        outs.append([hk.hash_encoding(x, table, f, None, T, 16, 4000, L) for f in (None, tail)])
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
 def _grads(tensors):
     return [None if t is None else t.grad for t in tensors]
 

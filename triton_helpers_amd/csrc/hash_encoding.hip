@@ -596,22 +596,32 @@ __global__ __launch_bounds__(LEVELS_THREADS) void hash_fwd_levels_k(const void* 
   }
 }
 
-// Small batches: one thread per (point, level), the levels of a point side by side in blockIdx.y.  A thread per point
-// walks its levels one after the other, and a batch of a few thousand points is then a handful of workgroups that wait
-// out sixteen rounds of memory latency (forward) or queue five hundred atomics per thread behind each other (backward)
-// while most of the chip idles.  Same arithmetic, in the same order, as the kernels above.
-template <typename TT, int D>
+// Small batches: one thread per (point, level).  A thread per point walks its levels one after the other, and a batch of a few thousand
+// points is then a handful of workgroups that wait out sixteen rounds of memory latency while most of the chip idles.  Same arithmetic, in
+// the same order, as the kernels above.
+// A workgroup's 256 points of one level are a unit of work, and the units stand level by level.  BY_XCD: every XCD takes `share` of them in
+// a row (two levels of sixteen), so that a level's table is read into one L2 or two and not into all eight.
+template <typename TT, int D, int FEAT, bool BY_XCD>
 __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_level_k(const void* coords, int cdt, int64_t csn, int64_t csd,
-                                                                 const uint32_t* table, uint16_t* out, int64_t out_stride,
-                                                                 int64_t N, DevGeom g, const int64_t* primes, float scale) {
-  const int l = blockIdx.y;
-  const int64_t n = (int64_t)blockIdx.x * TILE_THREADS + threadIdx.x;
+                                                                 const uint32_t* table, typename TT::storage* out, int64_t out_stride,
+                                                                 int64_t N, uint32_t chunks, uint32_t share, DevGeom g, const int64_t* primes,
+                                                                 float scale) {
+  constexpr int RW = FEAT * (int)sizeof(typename TT::storage) / 4;  // words of a row
+  typedef uint32_t Row __attribute__((ext_vector_type(RW)));
+  int l = (int)blockIdx.y;
+  int64_t n = (int64_t)blockIdx.x * TILE_THREADS + threadIdx.x;
+  if constexpr (BY_XCD) {
+    const uint32_t unit = blockIdx.x % LEVELS_XCDS * share + blockIdx.x / LEVELS_XCDS;
+    l = (int)(unit / chunks);
+    n = (int64_t)(unit - (uint32_t)l * chunks) * TILE_THREADS + threadIdx.x;
+    if (l >= g.levels) return;
+  }
   if (n >= N) return;
   constexpr int CN = 1 << D;
   const uint32_t pi[3] = {(uint32_t)primes[0], (uint32_t)primes[1], D > 2 ? (uint32_t)primes[D > 2 ? 2 : 0] : 0u};
   const uint32_t res = (uint32_t)g.res[l];
   const float fres = (float)g.res[l];
-  const uint32_t* tab = table + g.row_offset[l];
+  const Row* tab = reinterpret_cast<const Row*>(table) + g.row_offset[l];
   uint32_t c[3];
   float fr[3];
 #pragma unroll
@@ -624,19 +634,31 @@ __global__ __launch_bounds__(TILE_THREADS) void hash_fwd_level_k(const void* coo
     fr[d] = pos - fl;
   }
   const Corner8 r = D == 3 ? rows_d3(c, l >= g.first_hash, res, g.rows[l] - 1, pi) : rows_d2(c, l >= g.first_hash, res, g.rows[l] - 1, pi);
-  uint32_t v[CN];
+  Row v[CN];
 #pragma unroll
   for (int j = 0; j < CN; ++j) v[j] = tab[r.row[j]];
   float w[8];
   if (D == 3) weights_d3(fr, w);
   else weights_d2(fr, w);
-  float a0 = 0.0f, a1 = 0.0f;
+  Row sum;
 #pragma unroll
-  for (int j = 0; j < CN; ++j) {
-    a0 = a0 + w[j] * TT::to_f32((uint16_t)(v[j] & 0xffffu));
-    a1 = a1 + w[j] * TT::to_f32((uint16_t)(v[j] >> 16));
+  for (int e = 0; e < RW; ++e) {
+    if constexpr (sizeof(typename TT::storage) == 4) {
+      float a = 0.0f;
+#pragma unroll
+      for (int j = 0; j < CN; ++j) a = a + w[j] * __uint_as_float(v[j][e]);
+      sum[e] = __float_as_uint(a);
+    } else {
+      float a0 = 0.0f, a1 = 0.0f;
+#pragma unroll
+      for (int j = 0; j < CN; ++j) {
+        a0 = a0 + w[j] * TT::to_f32((uint16_t)(v[j][e] & 0xffffu));
+        a1 = a1 + w[j] * TT::to_f32((uint16_t)(v[j][e] >> 16));
+      }
+      sum[e] = TT::pack(a0, a1);
+    }
   }
-  *reinterpret_cast<uint32_t*>(out + n * out_stride + 2 * l) = TT::pack(a0, a1);
+  *reinterpret_cast<Row*>(out + n * out_stride + FEAT * l) = sum;
 }
 
 // Backward of small batches: one lane per (point, level, corner, feature).  What it costs are the atomics' requests, one per 64 bytes
@@ -688,9 +710,30 @@ constexpr int SWEEP_PPT = 4;
 constexpr int64_t SWEEP_MIN_POINTS = ((int64_t)1 << 17) + 1;
 constexpr int64_t SWEEP_MIN_POINTS_D2 = (int64_t)1 << 16;
 constexpr int64_t SWEEP_MIN_POINTS_F32 = (int64_t)1 << 16;
-// the forward per (point, level) serves batches up to this where the staged kernel is the alternative (three
-// dimensions: 45 against 53 us at 2^16 points, 75 against 52 us at 2^17); in two dimensions up to the sweep's minimum
-constexpr int64_t LEVEL_MAX_POINTS = 65536;
+// The forward per (point, level) serves batches up to this where the staged kernel is the alternative, which takes sixteen rounds of latency for any
+// batch up to 2^17 points (us, level / staged: two features 2^16 points 35 / 51, 2^17 62 / 51; four 1000 4 / 54, 2^15 27 / 58, 2^16
+// 48 / 59, 100000 72 / 63; eight, levels of 1 MiB 2^16 33 / 35).  Rows of four and eight features in levels beyond an L2: four in 8 MiB
+// 2^15 37 / 59, 2^16 68 / 64; eight 2^15 39 / 42, 2^16 72 / 62.
+constexpr int64_t L2_BYTES = 4 << 20;
+static int64_t largest_level(const nf_hash_geom* g, int es) {
+  int64_t rows = 0;
+  for (int l = 0; l < g->levels; ++l) rows = g->rows[l] > rows ? g->rows[l] : rows;
+  return rows * g->feat * es;
+}
+static int64_t level_max_points(const nf_hash_geom* g) { return g->feat > 2 && largest_level(g, 2) > L2_BYTES ? 40960 : 65536; }
+// Units of a level on one XCD (hash_fwd_level_k): where a level fits an L2 and the table does not, in batches that every XCD would read most of
+// it for.  2^15 points on 16 levels of 2^19 rows touch most of a table's lines from every XCD, 150 MB in all (us, dealt out in turn / by XCD,
+// uniform and rays): fp16 2^15 points 26 / 21 and 21 / 20, 2^16 43 / 35 and 35 / 34; float32 60000 56 / 43 and 48 / 43; four features
+// 2^16 57 / 48 and 49 / 47; but 8192 points along rays 9.2 / 10.4, a table of 3 MB 2^16 28 / 32, levels of 8 MiB 61 / 61, two dimensions
+// (most levels dense, their rows in order) 2^16 19 / 25, 2^18 points 246 / 276; and, each XCD reading a table of 13 MB often enough to be worth
+// its misses, 2^15 points 18 / 18 along rays, 2^16 30 / 32.
+static bool level_by_xcd(const nf_hash_geom* g, int table_dt, int64_t n_points) {
+  const int es = table_dt == NF_F32 ? 4 : 2;
+  int64_t rows = 0;
+  for (int l = 0; l < g->levels; ++l) rows += g->rows[l];
+  const int64_t bytes = rows * g->feat * es;
+  return g->dims == 3 && n_points >= 16384 && n_points * 320 <= bytes && largest_level(g, es) <= L2_BYTES && bytes > 2 * L2_BYTES;
+}
 
 // How a sweep's points are dealt out.  A compute unit works its gathers off at a rate of its own (one workgroup on a unit runs
 // at the rate of three: 1024 points take 83 us either way, because the unit's L1 takes about three lanes in four clocks
@@ -700,8 +743,7 @@ constexpr int64_t LEVEL_MAX_POINTS = 65536;
 constexpr int64_t COMPUTE_UNITS = 256;
 
 // Levels in LDS: batches from which the copying pays.  Under that the per-(point, level) kernels run (16-bit pairs: 5.3 and 5.8 us
-// at 8192 points, 8.5 and 6.3 at 2^14; float32: 5.1 and 5.0 us at 4096, 6.2 and 5.5 at 8192), and for rows of four features the staged
-// kernel, which takes 20 us and more for any batch.
+// at 8192 points, 8.5 and 6.3 at 2^14; float32: 5.1 and 5.0 us at 4096, 6.2 and 5.5 at 8192).
 constexpr int64_t LEVELS_MIN_POINTS_16 = 16384, LEVELS_MIN_POINTS_F32 = 4096;
 
 // points per wave, at most `most`, four waves to a workgroup
@@ -733,16 +775,17 @@ static bool tiled_ok(const nf_hash_geom* g, int table_dt, const void* rows_ptr, 
   return true;
 }
 
-// the per-(point, level) kernels for small batches: rows of one 16-bit pair, two or three dimensions, hashed levels of
-// a power of two of rows, pairs that can be read and written as one 32-bit word
-static bool level_ok(const nf_hash_geom* g, int table_dt, const void* rows_ptr, int64_t row_stride) {
-  if ((g->dims != 2 && g->dims != 3) || g->feat != 2 || table_dt == NF_F32) return false;
+// the per-(point, level) kernel: three dimensions, or two and two features (four 65535 points 29 us, the generic kernel 28), hashed levels of a
+// power of two of rows, rows of 4, 8 or 16 bytes that can be read and written as one piece
+static bool level_ok(const nf_hash_geom* g, int table_dt, const void* table, const void* rows_ptr, int64_t row_stride) {
+  const int es = table_dt == NF_F32 ? 4 : 2, row = g->feat * es;
+  if (!(g->dims == 3 || (g->dims == 2 && g->feat == 2)) || !(g->feat == 2 || g->feat == 4 || (g->feat == 8 && es == 2))) return false;
   for (int l = g->first_hash_level; l < g->levels; ++l) {
     if (l < 0) return false;
     const int64_t r = g->rows[l];
     if ((r & (r - 1)) != 0) return false;
   }
-  return ((uintptr_t)rows_ptr & 3u) == 0 && row_stride % 2 == 0;
+  return (uintptr_t)table % row == 0 && (uintptr_t)rows_ptr % row == 0 && row_stride * es % row == 0;
 }
 
 // whether every level fits LDS and the rows can be read and written in words; pair: two levels fit together
@@ -843,6 +886,37 @@ static int dispatch_fwd_generic(int table_dt, const void* coords, int cdt, int64
     default: launch_fwd_generic<D, BF16>(coords, cdt, csn, csd, table, out, out_stride, N, g, primes, scale, vec, s); break;
   }
   return check_launch("hash_fwd_generic");
+}
+
+static int launch_fwd_level(int table_dt, const void* coords, int cdt, int64_t csn, int64_t csd, const void* table, void* out, int64_t out_stride,
+                            int64_t N, const DevGeom& g, const int64_t* primes, float scale, bool by_xcd, hipStream_t s) {
+  auto pick = [&](auto tt) -> const void* {
+    typedef decltype(tt) TT;
+    auto dims = [&](auto f_c) -> const void* {
+      constexpr int F = decltype(f_c)::value;
+      if constexpr (F == 2)
+        if (g.dims == 2) return (const void*)hash_fwd_level_k<TT, 2, F, false>;
+      return by_xcd ? (const void*)hash_fwd_level_k<TT, 3, F, true> : (const void*)hash_fwd_level_k<TT, 3, F, false>;
+    };
+    if constexpr (sizeof(typename TT::storage) == 2)
+      if (g.feat == 8) return dims(std::integral_constant<int, 8>{});
+    return g.feat == 4 ? dims(std::integral_constant<int, 4>{}) : dims(std::integral_constant<int, 2>{});
+  };
+  const void* kern = table_dt == NF_F32 ? pick(F32{}) : table_dt == NF_F16 ? pick(F16{}) : pick(BF16{});
+  // launches of at most 2^26 points: units stay inside 32 bits
+  constexpr int64_t part = (int64_t)1 << 26;
+  const int row = g.feat * (table_dt == NF_F32 ? 4 : 2);
+  for (int64_t n0 = 0; n0 < N; n0 += part) {
+    int64_t n = N - n0 < part ? N - n0 : part;
+    uint32_t chunks = (uint32_t)((n + TILE_THREADS - 1) / TILE_THREADS), share = by_xcd ? (chunks * (uint32_t)g.levels + LEVELS_XCDS - 1) / LEVELS_XCDS : 0u;
+    const void* c = (const char*)coords + n0 * csn * dtype_size(cdt);
+    void* o = (char*)out + n0 * out_stride * (row / g.feat);
+    DevGeom gg = g;
+    void* args[] = {(void*)&c, (void*)&cdt, (void*)&csn, (void*)&csd, (void*)&table, (void*)&o, (void*)&out_stride, (void*)&n, (void*)&chunks, (void*)&share, (void*)&gg, (void*)&primes, (void*)&scale};
+    const hipError_t e = hipLaunchKernel(kern, by_xcd ? dim3(share * LEVELS_XCDS) : dim3(chunks, (unsigned)g.levels), dim3(TILE_THREADS), args, 0, s);
+    if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(hash_fwd_level): %s", hipGetErrorString(e));
+  }
+  return check_launch("hash_fwd_level");
 }
 
 template <int FW>
@@ -954,19 +1028,11 @@ extern "C" int nf_hash_encode_fwd(const void* coords, int coords_dtype, int64_t 
     }
     return check_launch("hash_fwd_sweep");
   }
-  // batches below the sweep's minimum: a thread per (point, level)
-  if (!(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FWD_STAGED)) && level_ok(geom, table_dtype, out, out_stride_n) &&
-      (n_points <= LEVEL_MAX_POINTS || !tiled_ok(geom, table_dtype, out, out_stride_n))) {
-    dim3 grid((unsigned)((n_points + TILE_THREADS - 1) / TILE_THREADS), (unsigned)g.levels);
-    const void* kern = table_dtype == NF_F16 ? (g.dims == 3 ? (const void*)hash_fwd_level_k<F16, 3> : (const void*)hash_fwd_level_k<F16, 2>)
-                                             : (g.dims == 3 ? (const void*)hash_fwd_level_k<BF16, 3> : (const void*)hash_fwd_level_k<BF16, 2>);
-    const uint32_t* tab = (const uint32_t*)table;
-    uint16_t* o = (uint16_t*)out;
-    void* args[] = {&coords, &coords_dtype, &csn, &csd, &tab, &o, &out_stride_n, &n_points, &g, &primes, &scale};
-    const hipError_t e = hipLaunchKernel(kern, grid, dim3(TILE_THREADS), args, 0, s);
-    if (e != hipSuccess) return fail((int)e, "hipLaunchKernel(hash_fwd_level): %s", hipGetErrorString(e));
-    return check_launch("hash_fwd_level");
-  }
+  // batches below the sweep's minimum, and rows that neither sweep nor staged kernel takes: a thread per (point, level)
+  if (!(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FWD_STAGED)) && level_ok(geom, table_dtype, table, out, out_stride_n) &&
+      (n_points <= level_max_points(geom) || !tiled_ok(geom, table_dtype, out, out_stride_n, geom->feat)))
+    return launch_fwd_level(table_dtype, coords, coords_dtype, csn, csd, table, out, out_stride_n, n_points, g, primes, scale,
+                            level_by_xcd(geom, table_dtype, n_points), s);
   if (!(flags & NF_HASH_FORCE_GENERIC) && tiled_ok(geom, table_dtype, out, out_stride_n)) {
     constexpr int PPT = 2;
     constexpr int P = TILE_THREADS * PPT;

@@ -324,3 +324,30 @@ def test_float32_mlp_gradients(rows, d_in, H, d_out, hidden, act, bias):
     for a, b in zip(runs[0], _grads(leaves)):
         if b is not None:
             assert float((a.double() - b).norm()) <= 1e-5 * float(b.norm())
+
+
+@pytest.mark.parametrize("d_in,H,d_out,depth,act,bias", [(32, 64, 16, 2, "silu", True), (64, 64, 64, 4, "relu2", False), (35, 64, 3, 3, "relu", True), (64, 64, 33, 9, "relu", True),
+                                                         (16, 16, 1, 3, "silu", True), (48, 32, 33, 9, "silu", False), (27, 32, 64, 2, "relu", True), (32, 64, 16, 1, "relu", True)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_mlp_forward_of_every_batch_size(d_in, H, d_out, depth, act, bias, dtype):
+    """A wave takes sixteen rows of a small batch at a time and 32 of a large one, and the weights are staged as one list where their matrices are
+    16-byte aligned: a row's result has the same bits in every batch, and from matrices that are not."""
+    from triton_helpers_amd.layers.fully_fused_mlp import fully_fused_mlp
+
+    torch.manual_seed(depth)
+    n = depth - 1
+    u = lambda *s: ((torch.rand(*s, device=DEV) * 2 - 1) / s[-1] ** 0.5).to(dtype)  # noqa: E731
+    w = {"w_in": u(H, d_in), "w_out": u(d_out, H), "b_in": u(H) if bias else None, "b_out": u(d_out) if bias else None,
+         "w_hid": u(n * H, H) if n else None, "b_hid": u(n, H) if n and bias else None}
+    x = torch.randn(1, 131_090, d_in, device=DEV).to(dtype)
+    want = fully_fused_mlp(x, **w, activation=act)
+    for rows in (1, 17, 4097, 32768, 32769, 65536, 65537, 131_072, 131_073):
+        assert torch.equal(fully_fused_mlp(x[:, :rows], **w, activation=act), want[:, :rows]), rows
+    shifted = {}
+    for k, t in w.items():
+        if t is not None:
+            flat = torch.empty(t.numel() + 1, dtype=dtype, device=DEV)
+            flat[1:] = t.flatten()
+            t = flat[1:].view(t.shape)
+        shifted[k] = t
+    assert torch.equal(fully_fused_mlp(x[:, :4097], **shifted, activation=act), want[:, :4097])

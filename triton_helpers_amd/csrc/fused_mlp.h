@@ -52,23 +52,23 @@ __device__ __forceinline__ void stage_bias(float* dst, const uint16_t* b, int n_
 }
 
 // acc[nt][mt] = bias + W(frags) * in[nt][kc]; K chunks outermost, so that the products into one accumulator tile are
-// 2 * MT instructions apart
-template <typename T, int MT, int KC>
-__device__ __forceinline__ void layer_mma(f32x4_t (&acc)[2][4], const Frag (&in)[2][2], const uint16_t* frags,
+// NT * MT instructions apart
+template <typename T, int MT, int KC, int NT>
+__device__ __forceinline__ void layer_mma(f32x4_t (&acc)[NT][4], const Frag (&in)[NT][2], const uint16_t* frags,
                                           const float* bias, int lane) {
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const f32x4_t b4 = *reinterpret_cast<const f32x4_t*>(bias + 16 * mt + 4 * (lane >> 4));
-    acc[0][mt] = b4;
-    acc[1][mt] = b4;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[nt][mt] = b4;
   }
 #pragma unroll
   for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const Frag a = lds_frag(frags, mt * KC + kc, lane);
-      acc[0][mt] = mfma16<T>(a, in[0][kc], acc[0][mt]);
-      acc[1][mt] = mfma16<T>(a, in[1][kc], acc[1][mt]);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[nt][mt] = mfma16<T>(a, in[nt][kc], acc[nt][mt]);
     }
 }
 

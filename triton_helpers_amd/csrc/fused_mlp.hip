@@ -20,12 +20,12 @@
 namespace nf {
 
 // activation + rounding of a hidden layer; the packed tiles become the next layer's B fragments
-template <typename T, int KC_H, bool RELU>
-__device__ __forceinline__ void hidden_epilogue(const f32x4_t (&acc)[2][4], Frag (&in)[2][2], int act) {
+template <typename T, int KC_H, bool RELU, int NT>
+__device__ __forceinline__ void hidden_epilogue(const f32x4_t (&acc)[NT][4], Frag (&in)[NT][2], int act) {
   with_act(RELU ? NF_ACT_RELU : act, [&](auto act_c) {
     constexpr int ACT = decltype(act_c)::value;
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int kc = 0; kc < KC_H; ++kc) {
         act_pack<T, RELU>(acc[nt][2 * kc], ACT, in[nt][kc].w[0], in[nt][kc].w[1]);
@@ -37,10 +37,85 @@ __device__ __forceinline__ void hidden_epilogue(const f32x4_t (&acc)[2][4], Frag
 // ---------------------------------------------------------------------------------------
 // Forward
 // ---------------------------------------------------------------------------------------
-// XC: how x is stored (MlpArgs::x_conv), fixed at compile time.
-template <typename T, int KIN, int HP, int OUTP, int XC>
+// All weights of a network into LDS as A fragments, [w_in | w_hid | w_out], and its biases behind them.  The layers are one list of
+// fragments, several to a wave under way together, and the biases are asked for first: layer by layer, every matrix and every bias waited for the
+// one in front.  Rows move in 16-byte pieces, which are the order of the first layer's products and two halves of a fragment each in
+// that of the others (8-byte pieces keep the L1 busy twice as long, a clock per lane).  Loads carry no condition of their own
+// (addresses are held inside their matrix, what is outside is zeroed on its way to LDS), as a branch would be waited for at its end, and what a
+// fragment is, is worked out once per wave.  Two layers alone have little to wait for (32 -> 64 -> 16, 2^18 rows 6.9 us, as a list 7.6).
+template <typename T, int KIN, int HP, int OUTP, bool LIST>
+__device__ __forceinline__ void stage_network(uint16_t* frags, float* bias, const MlpArgs& a, int tid, int nthreads) {
+  constexpr int KC_IN = KIN / 32, KC_H = HP / 32, MT_H = HP / 16, MT_O = OUTP / 16, AT_ONCE = 4;
+  constexpr int F_IN = MT_H * KC_IN, F_HID = MT_H * KC_H, F_OUT = MT_O * KC_H;
+  const int H = a.d_hidden, n_hid = a.depth - 1, hidden = n_hid * F_HID;
+  if (!LIST) {
+    stage_weight_frags<false, false>(frags, a.w_in, H, a.d_in, MT_H, KC_IN, tid, nthreads);
+    for (int k = 0; k < n_hid; ++k) {
+      stage_weight_frags<true, false>(frags + (size_t)(F_IN + k * F_HID) * FRAG_ELEMS, a.w_hid + (size_t)k * H * H, H, H, MT_H, KC_H, tid, nthreads);
+      stage_bias<T>(bias + (k + 1) * HP, a.b_hid ? a.b_hid + (size_t)k * H : nullptr, H, HP, tid, nthreads);
+    }
+    stage_weight_frags<true, false>(frags + (size_t)(F_IN + hidden) * FRAG_ELEMS, a.w_out, a.d_out, H, MT_O, KC_H, tid, nthreads);
+    stage_bias<T>(bias, a.b_in, H, HP, tid, nthreads);
+    stage_bias<T>(bias + (n_hid + 1) * HP, a.b_out, a.d_out, OUTP, tid, nthreads);
+    return;
+  }
+  const int n_bias = HP + n_hid * HP + OUTP;
+  const auto bias_at = [&](int i, bool& valid) {
+    const bool out = i >= HP + n_hid * HP;
+    const int layer = i / HP, f = out ? i - (HP + n_hid * HP) : i % HP;
+    const uint16_t* b = out ? a.b_out : layer == 0 ? a.b_in : a.b_hid;
+    valid = b != nullptr && f < (out ? a.d_out : H);
+    return valid ? b + (out || layer == 0 ? f : (layer - 1) * H + f) : a.w_out;
+  };
+  bool first_valid;
+  const uint16_t first_bias = *bias_at(tid < n_bias ? tid : 0, first_valid);
+  const bool in_listed = a.d_in % 8 == 0 && (uintptr_t)a.w_in % 16 == 0;
+  const int lane = tid & 63, m = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = nthreads >> 6;
+  const int all = F_IN + hidden + F_OUT;
+  for (int f0 = (in_listed ? 0 : F_IN) + wave; f0 < all; f0 += AT_ONCE * nwaves) {
+    uint4 v[AT_ONCE];
+    bool there[AT_ONCE];
+#pragma unroll
+    for (int i = 0; i < AT_ONCE; ++i) {
+      const int f = f0 + i * nwaves;
+      if (f >= all) break;  // (the same for the whole wave)
+      const bool in = f < F_IN, out = f >= F_IN + hidden;
+      const uint32_t p = (uint32_t)(in ? f : out ? f - F_IN - hidden : f - F_IN), layer = in || out ? 0u : p / F_HID, frag = p - layer * F_HID;
+      const int mt = (int)(in ? frag / KC_IN : frag / KC_H), kc = (int)(in ? frag % KC_IN : frag % KC_H);
+      const int rows = out ? a.d_out : H, cols = in ? a.d_in : H, row = 16 * mt + m, k = 32 * kc + 8 * g;
+      const uint16_t* w = in ? a.w_in : out ? a.w_out : a.w_hid + (size_t)layer * H * H;
+      there[i] = row < rows && k < cols;
+      v[i] = *reinterpret_cast<const uint4*>(w + __umul24((uint32_t)(row < rows ? row : 0), (uint32_t)cols) + (k < cols ? k : 0));
+    }
+#pragma unroll
+    for (int i = 0; i < AT_ONCE; ++i) {
+      const int f = f0 + i * nwaves;
+      if (f >= all) break;
+      uint16_t* dst = frags + (size_t)f * FRAG_ELEMS;
+      if (!there[i]) v[i] = make_uint4(0u, 0u, 0u, 0u);
+      if (f < F_IN) {
+        *reinterpret_cast<uint4*>(dst + lane * 8) = v[i];
+      } else {  // features 8g .. 8g + 7 of 32: the half g / 2 of lane groups 2 (g % 2) and the one behind it
+        uint16_t* half = dst + (m + 32 * (g & 1)) * 8 + 4 * (g >> 1);
+        *reinterpret_cast<uint2*>(half) = make_uint2(v[i].x, v[i].y);
+        *reinterpret_cast<uint2*>(half + 16 * 8) = make_uint2(v[i].z, v[i].w);
+      }
+    }
+  }
+  if (!in_listed) stage_weight_frags<false, false>(frags, a.w_in, H, a.d_in, MT_H, KC_IN, tid, nthreads);
+  if (tid < n_bias) bias[tid] = first_valid ? T::to_f32(first_bias) : 0.0f;
+  for (int i = tid + nthreads; i < n_bias; i += nthreads) {
+    bool valid;
+    const uint16_t b = *bias_at(i, valid);
+    bias[i] = valid ? T::to_f32(b) : 0.0f;
+  }
+}
+
+// XC: how x is stored (MlpArgs::x_conv), fixed at compile time.  NT: 16-row groups that a wave carries at once, two or, in a batch that
+// leaves SIMDs without a wave, one.  LIST: see stage_network().
+template <typename T, int KIN, int HP, int OUTP, int XC, int NT, bool LIST>
 __global__ __launch_bounds__(512) void mlp_fwd_k(MlpArgs a) {
-  constexpr int KC_IN = KIN / 32, KC_H = HP / 32, MT_H = HP / 16, MT_O = OUTP / 16;
+  constexpr int KC_IN = KIN / 32, KC_H = HP / 32, MT_H = HP / 16, MT_O = OUTP / 16, ROWS = 16 * NT;
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x, nthreads = blockDim.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -54,61 +129,31 @@ __global__ __launch_bounds__(512) void mlp_fwd_k(MlpArgs a) {
   float* bias_out = bias_hid + (size_t)n_hid * HP;
 
   const bool relu = a.act == NF_ACT_RELU;
-  const int64_t n_chunks = (a.rows + 31) / 32;
+  const int64_t n_chunks = (a.rows + ROWS - 1) / ROWS;
   const int64_t wave_stride = (int64_t)gridDim.x * a.waves;
   // the next chunk's rows are requested before the current chunk is computed (loads past the end return zeros)
-  Frag nxt[2][2];
-  const int64_t first_chunk = (int64_t)blockIdx.x * a.waves + wave;
+  Frag nxt[NT][2];
+  // a small batch's chunks go to the workgroups in turn, then to their waves; a large one's stay together
+  const int64_t first_chunk = NT == 1 ? (int64_t)wave * gridDim.x + blockIdx.x : (int64_t)blockIdx.x * a.waves + wave;
 #pragma unroll
-  for (int nt = 0; nt < 2; ++nt)
+  for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int kc = 0; kc < KC_IN; ++kc)
-      nxt[nt][kc] = load_rows_frag(a.x, a.x_stride, first_chunk * 32 + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
-  stage_weight_frags<false, false>(f_in, a.w_in, a.d_hidden, a.d_in, MT_H, KC_IN, tid, nthreads);
-  if (n_hid > 1 && a.d_hidden == HP && (uintptr_t)a.w_hid % 8 == 0) {
-    // The hidden layers are one array: their pieces of eight values as one list, several under way per thread, and their biases.  Layer by
-    // layer, loads and biases of a deep network waited for one another twenty times (64 -> 64 x 9 -> 64, 1000 / 65536 / 2^18 rows, us: 16.0 / 18.7 / 43.6,
-    // so 14.5 / 16.4 / 37.7; 32 -> 64 x 3 -> 16 6.8 / 8.6 / 15.2, so 6.3 / 7.9 / 14.4).  A single one has nothing to wait for (8.1, so 8.6).
-    constexpr int LAYER = MT_H * KC_H * 64, AT_ONCE = 4;
-    const int all = n_hid * LAYER;
-    for (int u0 = tid; u0 < all; u0 += AT_ONCE * nthreads) {
-      uint2 lo[AT_ONCE], hi[AT_ONCE];
-#pragma unroll
-      for (int i = 0; i < AT_ONCE; ++i) {
-        const int u = u0 + i * nthreads < all ? u0 + i * nthreads : u0;
-        const int layer = u / LAYER, frag = u % LAYER >> 6, g = (u & 63) >> 4;
-        const uint16_t* w = a.w_hid + (size_t)(layer * HP + 16 * (frag / KC_H) + (u & 15)) * HP;
-        lo[i] = *reinterpret_cast<const uint2*>(w + k_chain(frag % KC_H, g, 0));
-        hi[i] = *reinterpret_cast<const uint2*>(w + k_chain(frag % KC_H, g, 4));
-      }
-#pragma unroll
-      for (int i = 0; i < AT_ONCE; ++i)
-        if (u0 + i * nthreads < all) *reinterpret_cast<uint4*>(f_hid + (size_t)(u0 + i * nthreads) * 8) = make_uint4(lo[i].x, lo[i].y, hi[i].x, hi[i].y);
-    }
-    stage_bias<T>(bias_hid, a.b_hid, n_hid * HP, n_hid * HP, tid, nthreads);
-  } else {
-    for (int k = 0; k < n_hid; ++k) {
-      stage_weight_frags<true, false>(f_hid + (size_t)k * MT_H * KC_H * FRAG_ELEMS, a.w_hid + (size_t)k * a.d_hidden * a.d_hidden, a.d_hidden,
-                                      a.d_hidden, MT_H, KC_H, tid, nthreads);
-      stage_bias<T>(bias_hid + k * HP, a.b_hid ? a.b_hid + (size_t)k * a.d_hidden : nullptr, a.d_hidden, HP, tid, nthreads);
-    }
-  }
-  stage_weight_frags<true, false>(f_out, a.w_out, a.d_out, a.d_hidden, MT_O, KC_H, tid, nthreads);
-  stage_bias<T>(bias_in, a.b_in, a.d_hidden, HP, tid, nthreads);
-  stage_bias<T>(bias_out, a.b_out, a.d_out, OUTP, tid, nthreads);
+      nxt[nt][kc] = load_rows_frag(a.x, a.x_stride, first_chunk * ROWS + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
+  stage_network<T, KIN, HP, OUTP, LIST>(f_in, bias_in, a, tid, nthreads);
   __syncthreads();
 
   for (int64_t chunk = first_chunk; chunk < n_chunks; chunk += wave_stride) {
-    const int64_t row0 = chunk * 32;
-    Frag in[2][2];
-    f32x4_t acc[2][4];
+    const int64_t row0 = chunk * ROWS;
+    Frag in[NT][2];
+    f32x4_t acc[NT][4];
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int kc = 0; kc < KC_IN; ++kc) {
         in[nt][kc] = XC == 0 ? nxt[nt][kc] : convert_frag(nxt[nt][kc], XC);
         if (a.in_act != NF_ACT_NONE) in[nt][kc] = act_frag<T>(in[nt][kc], a.in_act);
-        nxt[nt][kc] = load_rows_frag(a.x, a.x_stride, (chunk + wave_stride) * 32 + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
+        nxt[nt][kc] = load_rows_frag(a.x, a.x_stride, (chunk + wave_stride) * ROWS + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
       }
 
     layer_mma<T, MT_H, KC_IN>(acc, in, f_in, bias_in, lane);
@@ -125,7 +170,7 @@ __global__ __launch_bounds__(512) void mlp_fwd_k(MlpArgs a) {
     }
     layer_mma<T, MT_O, KC_H>(acc, in, f_out, bias_out, lane);
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int mt = 0; mt < MT_O; ++mt)
         store_rows_tile<T>(a.y, a.y_stride, row0 + 16 * nt, a.rows, a.d_out, mt, lane, acc[nt][mt], a.y_vec);
@@ -570,14 +615,26 @@ static int launch_fwd(const MlpArgs& a0, hipStream_t s) {
   const size_t lds = ((size_t)(HP / 16) * (KIN / 32) + (size_t)n_hid * (HP / 16) * (HP / 32) + (size_t)(OUTP / 16) * (HP / 32)) * 1024 +
                      ((size_t)HP + (size_t)n_hid * HP + OUTP) * 4;
   NF_REQUIRE(lds <= LDS_LIMIT, NF_EUNSUPPORTED, "weights of depth %d need %zu B of LDS (limit %zu)", a.depth, lds, LDS_LIMIT);
+  const int units = device_cus();
+  // One group of sixteen rows to a wave, the workgroups of eight waves spread over the units, where two would leave SIMDs without a wave or, with
+  // long chains of layers, with one (us, layers staged in turn and two groups / two groups / one: 32 -> 64 x 4 -> 16 SiLU 1000 rows 8.5 / 8.3 / 6.0, 65536 12.3 / 11.7 /
+  // 10.3, 10^5 18.0 / 17.0 / 13.7, 2^17 18.2 / 17.3 / 15.9; 64 x 10 ReLU 1000 14.3 / 15.3 / 10.6, 2^17 23.8 / 24.3 / 23.3; one hidden layer SiLU
+  // 1000 6.6 / 5.6 / 5.2, 65536 7.7 / 7.4 / 7.6).
+  const bool list = n_hid > 0 && ((uintptr_t)a.w_hid | (uintptr_t)a.w_out) % 16 == 0;
+  const bool small = list && a.rows <= (n_hid == 1 ? 32768 : HP == 32 ? 65536 : 131072);
   // weights beyond half of LDS leave room for one workgroup per CU: give it eight waves to keep two per SIMD
-  a.waves = lds > 76 * 1024 ? 8 : 4;
-  const int64_t chunks = (a.rows + 31) / 32;
+  a.waves = lds > 76 * 1024 || small ? 8 : 4;
+  const int64_t chunks = (a.rows + (small ? 15 : 31)) / (small ? 16 : 32);
   int64_t blocks = (chunks + a.waves - 1) / a.waves;
-  const int64_t cap = (int64_t)device_cus() * (lds > 76 * 1024 ? 1 : (lds > 40 * 1024 ? 2 : 3));
+  const int64_t cap = (int64_t)units * (lds > 76 * 1024 ? 1 : (lds > 40 * 1024 ? 2 : 3));
   if (blocks > cap) blocks = cap;
+  if (small) blocks = chunks < units ? chunks : units;
   constexpr int XC_OTHER = T::code == NF_BF16 ? 1 : 2;
-  const void* kern = a.x_conv == 0 ? (const void*)mlp_fwd_k<T, KIN, HP, OUTP, 0> : (const void*)mlp_fwd_k<T, KIN, HP, OUTP, XC_OTHER>;
+  const auto pick = [&](auto xc_c) -> const void* {
+    constexpr int XC = decltype(xc_c)::value;
+    return small ? (const void*)mlp_fwd_k<T, KIN, HP, OUTP, XC, 1, true> : list ? (const void*)mlp_fwd_k<T, KIN, HP, OUTP, XC, 2, true> : (const void*)mlp_fwd_k<T, KIN, HP, OUTP, XC, 2, false>;
+  };
+  const void* kern = a.x_conv == 0 ? pick(std::integral_constant<int, 0>{}) : pick(std::integral_constant<int, XC_OTHER>{});
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return fail((int)e, "hipFuncSetAttribute: %s", hipGetErrorString(e));

@@ -51,6 +51,85 @@ __device__ __forceinline__ void stage_bias(float* dst, const uint16_t* b, int n_
   for (int i = tid; i < n_pad; i += nthreads) dst[i] = (b != nullptr && i < n_valid) ? T::to_f32(b[i]) : 0.0f;
 }
 
+// Features 8q .. 8q + 7 of a 32-feature chunk of row m into a fragment in chain order: the half q / 2 of lane groups 2 (q % 2) and the one behind it.
+__device__ __forceinline__ void put_chain(uint16_t* frag, int m, int q, uint4 v) {
+  uint16_t* half = frag + (m + 32 * (q & 1)) * 8 + 4 * (q >> 1);
+  *reinterpret_cast<uint2*>(half) = make_uint2(v.x, v.y);
+  *reinterpret_cast<uint2*>(half + 16 * 8) = make_uint2(v.z, v.w);
+}
+
+// All weights of a network into LDS as A fragments, [w_in | w_hid | w_out], and its biases behind them.  The layers are one list of
+// fragments, several to a wave under way together, and the biases are asked for first: layer by layer, every matrix and every bias waited for the
+// one in front.  Rows move in 16-byte pieces, which are the order of the first layer's products and two halves of a fragment each in
+// that of the others (8-byte pieces keep the L1 busy twice as long, a clock per lane).  Loads carry no condition of their own
+// (addresses are held inside their matrix, what is outside is zeroed on its way to LDS), as a branch would be waited for at its end, and what a
+// fragment is, is worked out once per wave.  Two layers alone have little to wait for (32 -> 64 -> 16, 2^18 rows 6.9 us, as a list 7.6).  IN_CHAIN: the first layer's products are in chain order, too.
+template <typename T, int KIN, int HP, int OUTP, bool LIST, bool IN_CHAIN>
+__device__ __forceinline__ void stage_network(uint16_t* frags, float* bias, const MlpArgs& a, int tid, int nthreads) {
+  constexpr int KC_IN = KIN / 32, KC_H = HP / 32, MT_H = HP / 16, MT_O = OUTP / 16, AT_ONCE = 4;
+  constexpr int F_IN = MT_H * KC_IN, F_HID = MT_H * KC_H, F_OUT = MT_O * KC_H;
+  const int H = a.d_hidden, n_hid = a.depth - 1, hidden = n_hid * F_HID;
+  if (!LIST) {
+    stage_weight_frags<IN_CHAIN, false>(frags, a.w_in, H, a.d_in, MT_H, KC_IN, tid, nthreads);
+    for (int k = 0; k < n_hid; ++k) {
+      stage_weight_frags<true, false>(frags + (size_t)(F_IN + k * F_HID) * FRAG_ELEMS, a.w_hid + (size_t)k * H * H, H, H, MT_H, KC_H, tid, nthreads);
+      stage_bias<T>(bias + (k + 1) * HP, a.b_hid ? a.b_hid + (size_t)k * H : nullptr, H, HP, tid, nthreads);
+    }
+    stage_weight_frags<true, false>(frags + (size_t)(F_IN + hidden) * FRAG_ELEMS, a.w_out, a.d_out, H, MT_O, KC_H, tid, nthreads);
+    stage_bias<T>(bias, a.b_in, H, HP, tid, nthreads);
+    stage_bias<T>(bias + (n_hid + 1) * HP, a.b_out, a.d_out, OUTP, tid, nthreads);
+    return;
+  }
+  const int n_bias = HP + n_hid * HP + OUTP;
+  const auto bias_at = [&](int i, bool& valid) {
+    const bool out = i >= HP + n_hid * HP;
+    const int layer = i / HP, f = out ? i - (HP + n_hid * HP) : i % HP;
+    const uint16_t* b = out ? a.b_out : layer == 0 ? a.b_in : a.b_hid;
+    valid = b != nullptr && f < (out ? a.d_out : H);
+    return valid ? b + (out || layer == 0 ? f : (layer - 1) * H + f) : a.w_out;
+  };
+  bool first_valid;
+  const uint16_t first_bias = *bias_at(tid < n_bias ? tid : 0, first_valid);
+  const bool in_listed = a.d_in % 8 == 0 && (uintptr_t)a.w_in % 16 == 0;
+  const int lane = tid & 63, m = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = nthreads >> 6;
+  const int all = F_IN + hidden + F_OUT;
+  for (int f0 = (in_listed ? 0 : F_IN) + wave; f0 < all; f0 += AT_ONCE * nwaves) {
+    uint4 v[AT_ONCE];
+    bool there[AT_ONCE];
+#pragma unroll
+    for (int i = 0; i < AT_ONCE; ++i) {
+      const int f = f0 + i * nwaves;
+      if (f >= all) break;  // (the same for the whole wave)
+      const bool in = f < F_IN, out = f >= F_IN + hidden;
+      const uint32_t p = (uint32_t)(in ? f : out ? f - F_IN - hidden : f - F_IN), layer = in || out ? 0u : p / F_HID, frag = p - layer * F_HID;
+      const int mt = (int)(in ? frag / KC_IN : frag / KC_H), kc = (int)(in ? frag % KC_IN : frag % KC_H);
+      const int rows = out ? a.d_out : H, cols = in ? a.d_in : H, row = 16 * mt + m, k = 32 * kc + 8 * g;
+      const uint16_t* w = in ? a.w_in : out ? a.w_out : a.w_hid + (size_t)layer * H * H;
+      there[i] = row < rows && k < cols;
+      v[i] = *reinterpret_cast<const uint4*>(w + __umul24((uint32_t)(row < rows ? row : 0), (uint32_t)cols) + (k < cols ? k : 0));
+    }
+#pragma unroll
+    for (int i = 0; i < AT_ONCE; ++i) {
+      const int f = f0 + i * nwaves;
+      if (f >= all) break;
+      uint16_t* dst = frags + (size_t)f * FRAG_ELEMS;
+      if (!there[i]) v[i] = make_uint4(0u, 0u, 0u, 0u);
+      if (!IN_CHAIN && f < F_IN) {
+        *reinterpret_cast<uint4*>(dst + lane * 8) = v[i];
+      } else {
+        put_chain(dst, m, g, v[i]);
+      }
+    }
+  }
+  if (!in_listed) stage_weight_frags<IN_CHAIN, false>(frags, a.w_in, H, a.d_in, MT_H, KC_IN, tid, nthreads);
+  if (tid < n_bias) bias[tid] = first_valid ? T::to_f32(first_bias) : 0.0f;
+  for (int i = tid + nthreads; i < n_bias; i += nthreads) {
+    bool valid;
+    const uint16_t b = *bias_at(i, valid);
+    bias[i] = valid ? T::to_f32(b) : 0.0f;
+  }
+}
+
 // acc[nt][mt] = bias + W(frags) * in[nt][kc]; K chunks outermost, so that the products into one accumulator tile are
 // NT * MT instructions apart
 template <typename T, int MT, int KC, int NT>

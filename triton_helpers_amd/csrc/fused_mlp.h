@@ -64,12 +64,16 @@ __device__ __forceinline__ void put_chain(uint16_t* frag, int m, int q, uint4 v)
 // that of the others (8-byte pieces keep the L1 busy twice as long, a clock per lane).  Loads carry no condition of their own
 // (addresses are held inside their matrix, what is outside is zeroed on its way to LDS), as a branch would be waited for at its end, and what a
 // fragment is, is worked out once per wave.  Two layers alone have little to wait for (32 -> 64 -> 16, 2^18 rows 6.9 us, as a list 7.6).  IN_CHAIN: the first layer's products are in chain order, too.
-template <typename T, int KIN, int HP, int OUTP, bool LIST, bool IN_CHAIN>
-__device__ __forceinline__ void stage_network(uint16_t* frags, float* bias, const MlpArgs& a, int tid, int nthreads) {
+// first_rows asks for the wave's first rows, behind the first weights: loads come back in order, and rows from HBM in front of the weights held up the
+// barrier (one-hidden-layer ReLU networks over inputs that no cache holds, rows first / weights first: 32 -> 64 -> 64 -> 16, 2^20 rows 23.9 / 19.4 us,
+// 64 -> 64 -> 64 -> 64, 2^18 14.6 / 13.8; eight hidden layers, 2^18 rows 35.3 / 34.5).
+template <typename T, int KIN, int HP, int OUTP, bool LIST, bool IN_CHAIN, typename FirstRows>
+__device__ __forceinline__ void stage_network(uint16_t* frags, float* bias, const MlpArgs& a, int tid, int nthreads, FirstRows first_rows) {
   constexpr int KC_IN = KIN / 32, KC_H = HP / 32, MT_H = HP / 16, MT_O = OUTP / 16, AT_ONCE = 4;
   constexpr int F_IN = MT_H * KC_IN, F_HID = MT_H * KC_H, F_OUT = MT_O * KC_H;
   const int H = a.d_hidden, n_hid = a.depth - 1, hidden = n_hid * F_HID;
   if (!LIST) {
+    first_rows();
     stage_weight_frags<IN_CHAIN, false>(frags, a.w_in, H, a.d_in, MT_H, KC_IN, tid, nthreads);
     for (int k = 0; k < n_hid; ++k) {
       stage_weight_frags<true, false>(frags + (size_t)(F_IN + k * F_HID) * FRAG_ELEMS, a.w_hid + (size_t)k * H * H, H, H, MT_H, KC_H, tid, nthreads);
@@ -93,7 +97,7 @@ __device__ __forceinline__ void stage_network(uint16_t* frags, float* bias, cons
   const bool in_listed = a.d_in % 8 == 0 && (uintptr_t)a.w_in % 16 == 0;
   const int lane = tid & 63, m = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = nthreads >> 6;
   const int all = F_IN + hidden + F_OUT;
-  for (int f0 = (in_listed ? 0 : F_IN) + wave; f0 < all; f0 += AT_ONCE * nwaves) {
+  for (int f0 = (in_listed ? 0 : F_IN) + wave, round = 0; f0 < all || round == 0; f0 += AT_ONCE * nwaves, ++round) {
     uint4 v[AT_ONCE];
     bool there[AT_ONCE];
 #pragma unroll
@@ -108,6 +112,7 @@ __device__ __forceinline__ void stage_network(uint16_t* frags, float* bias, cons
       there[i] = row < rows && k < cols;
       v[i] = *reinterpret_cast<const uint4*>(w + __umul24((uint32_t)(row < rows ? row : 0), (uint32_t)cols) + (k < cols ? k : 0));
     }
+    if (round == 0) first_rows();
 #pragma unroll
     for (int i = 0; i < AT_ONCE; ++i) {
       const int f = f0 + i * nwaves;

@@ -61,12 +61,14 @@ __global__ __launch_bounds__(512) void mlp_fwd_k(MlpArgs a) {
   Frag nxt[NT][2];
   // a small batch's chunks go to the workgroups in turn, then to their waves; a large one's stay together
   const int64_t first_chunk = NT == 1 ? (int64_t)wave * gridDim.x + blockIdx.x : (int64_t)blockIdx.x * a.waves + wave;
+  auto first_rows = [&] {
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-    for (int kc = 0; kc < KC_IN; ++kc)
-      nxt[nt][kc] = load_rows_frag(a.x, a.x_stride, first_chunk * ROWS + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
-  stage_network<T, KIN, HP, OUTP, LIST, false>(f_in, bias_in, a, tid, nthreads);
+      for (int kc = 0; kc < KC_IN; ++kc)
+        nxt[nt][kc] = load_rows_frag(a.x, a.x_stride, first_chunk * ROWS + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
+  };
+  stage_network<T, KIN, HP, OUTP, LIST, false>(f_in, bias_in, a, tid, nthreads, first_rows);
   __syncthreads();
 
   for (int64_t chunk = first_chunk; chunk < n_chunks; chunk += wave_stride) {

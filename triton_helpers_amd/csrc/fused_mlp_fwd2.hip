@@ -66,13 +66,15 @@ __global__ __launch_bounds__(64 * fwd2_waves(KIN, OUTP)) void mlp_fwd2_k(MlpArgs
   // rows in flight per wave: the next chunk, and for 64-wide inputs (eight waves, 4 KB per chunk) the one behind it too (64 -> 64 -> 16: 45.8 -> 40.9 us per 2^20 rows)
   constexpr bool DEEP = KIN > 32;
   Frag nx[NT][KC_IN], nnx[NT][KC_IN];
+  auto first_rows = [&] {
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-    for (int kc = 0; kc < KC_IN; ++kc) {
-      nx[nt][kc] = load_x(first_chunk, nt, kc);
-      if constexpr (DEEP) nnx[nt][kc] = load_x(first_chunk + wave_stride, nt, kc);
-    }
+      for (int kc = 0; kc < KC_IN; ++kc) {
+        nx[nt][kc] = load_x(first_chunk, nt, kc);
+        if constexpr (DEEP) nnx[nt][kc] = load_x(first_chunk + wave_stride, nt, kc);
+      }
+  };
 
   uint16_t* f_in = reinterpret_cast<uint16_t*>(smem);   // W_in  [MT_H][KC_IN]
   uint16_t* f_hid = f_in + MT_H * KC_IN * FRAG_ELEMS;   // W_hid [MT_H][KC_H]
@@ -80,10 +82,10 @@ __global__ __launch_bounds__(64 * fwd2_waves(KIN, OUTP)) void mlp_fwd2_k(MlpArgs
   float* bias_in = reinterpret_cast<float*>(f_out + MT_O * KC_H * FRAG_ELEMS);
   float* bias_hid = bias_in + HP;
   float* bias_out = bias_hid + HP;
-  // (us, matrix by matrix in 8-byte pieces / this: 32 -> 64 -> 64 -> 16 2^19 rows 13.7 / 11.9, 2^20 19.9 / 19.0; 64 -> 64 -> 64 -> 64 2^18 16.0 / 14.4,
-  // 2^19 24.8 / 23.0, 2^21 106 / 102)
-  if (((uintptr_t)a.w_hid | (uintptr_t)a.w_out) % 16 == 0) stage_network<T, KIN, HP, OUTP, true, true>(f_in, bias_in, a, tid, nthreads);
-  else stage_network<T, KIN, HP, OUTP, false, true>(f_in, bias_in, a, tid, nthreads);
+  // (us over inputs that no cache holds, matrix by matrix in 8-byte pieces / this: 32 -> 64 -> 64 -> 16 2^18 rows 9.3 / 7.5, 2^20 22.5 / 19.4;
+  // 64 -> 64 -> 64 -> 64 2^18 15.6 / 13.8, 2^19 30.0 / 28.3)
+  if (((uintptr_t)a.w_hid | (uintptr_t)a.w_out) % 16 == 0) stage_network<T, KIN, HP, OUTP, true, true>(f_in, bias_in, a, tid, nthreads, first_rows);
+  else stage_network<T, KIN, HP, OUTP, false, true>(f_in, bias_in, a, tid, nthreads, first_rows);
   __syncthreads();
 
   for (int64_t chunk = first_chunk; chunk < n_chunks; chunk += wave_stride) {

@@ -1,0 +1,32 @@
+"""The backward kernels stage their weights in both forms from one read of every matrix where those are 16-byte aligned."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("d_in,d_out", [(32, 16), (8, 4), (24, 12), (16, 16), (64, 64), (40, 36), (48, 16), (32, 64)])
+@pytest.mark.parametrize("dtype,bias", [(torch.bfloat16, False), (torch.float16, True)])
+def test_matrices_off_their_alignment_give_the_same_bits(d_in, d_out, dtype, bias):
+    """2^16 + 3 rows of one hidden-to-hidden ReLU layer: the decoder's and the role-split kernel.  Views one element into a buffer are staged form by form."""
+    from triton_helpers_amd.layers.fully_fused_mlp import fully_fused_mlp
+
+    torch.manual_seed(d_in + d_out)
+    u = lambda *s: ((torch.rand(*s, device=DEV) * 2 - 1) / s[-1] ** 0.5).to(dtype)  # noqa: E731
+    w = {"w_in": u(64, d_in), "w_hid": u(64, 64), "w_out": u(d_out, 64)}
+    if bias:
+        w.update(b_in=u(64), b_hid=u(1, 64), b_out=u(d_out))
+    x, dy = torch.randn(1, 2**16 + 3, d_in, device=DEV).to(dtype), torch.randn(1, 2**16 + 3, d_out, device=DEV).to(dtype)
+
+    def grads(shift):
+        leaves = {"x": x.clone().requires_grad_()}
+        for k, t in w.items():
+            flat = torch.empty(t.numel() + 8, dtype=dtype, device=DEV)
+            leaves[k] = flat[shift : shift + t.numel()].view(t.shape).copy_(t).detach().requires_grad_()
+        y = fully_fused_mlp(activation="relu", **{"b_in": None, "b_out": None, "b_hid": None, **leaves})
+        y.backward(dy)
+        return [t.grad for t in leaves.values()]
+
+    for a, b in zip(grads(0), grads(1)):
+        assert torch.equal(a, b)

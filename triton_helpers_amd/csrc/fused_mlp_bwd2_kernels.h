@@ -194,6 +194,67 @@ __device__ __forceinline__ void layer_nt(f32x4_t (&acc)[NT][4], const Frag (&in)
 // Four parked copies of every gradient tile and bias row must fit LDS for the one-step sum of the waves.
 constexpr bool bwd2_parallel_sum(int tiles, int nbias) { return 4 * (tiles * 1024 + nbias * 256) <= 160 * 1024; }
 
+// The weights of a two-layer network in both forms, each matrix read once: a unit of four rows of eight values is 16 bytes of each
+// row, which are the forward fragments' halves as they are and, turned in registers, eight columns of the transposed ones.  (Form by form, the
+// transposed ones a value at a time, the L1 had 152 loads of 64 lanes to answer for a decoder, a clock per lane; these are 16.  32 -> 64 -> 64 -> 16, kernel and
+// its sum: 1000 rows 15.2 -> 14.6 us, 2^18 27.5 -> 26.6, 2^20 60.9 -> 59.4.)  The output matrix
+// has the transposed form only; OUTP its rows rounded up to 32.  first_rows asks for the wave's first rows behind the weights, as loads come back in order.
+template <int KIN, int HP, int OUTP, int NTHREADS, typename FirstRows>
+__device__ __forceinline__ void stage_both_forms(uint16_t* f_in, uint16_t* f_hid, uint16_t* t_in, uint16_t* t_hid, uint16_t* t_out, const MlpArgs& a, int tid, FirstRows first_rows) {
+  constexpr int U_IN = HP / 4 * (KIN / 8), U_HID = HP / 4 * (HP / 8), U_OUT = OUTP / 4 * (HP / 8), ALL = U_IN + U_HID + U_OUT;
+  constexpr int PER = (ALL + NTHREADS - 1) / NTHREADS;
+  static_assert(U_IN % 64 == 0 && U_HID % 64 == 0 && U_OUT % 64 == 0, "a wave's units are of one matrix");
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  struct Unit {
+    int rg, cg;  // four rows, eight columns
+    uint4 v[4];
+  } unit[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int u = 64 * wave + i * NTHREADS;  // the wave's first
+    if (u >= ALL) break;
+    const bool in = u < U_IN, out = u >= U_IN + U_HID;
+    const int p = (in ? u : out ? u - U_IN - U_HID : u - U_IN) + lane, groups = in ? KIN / 8 : HP / 8;
+    const int rows = out ? a.d_out : HP, cols = in ? a.d_in : HP;
+    const uint16_t* w = in ? a.w_in : out ? a.w_out : a.w_hid;
+    unit[i].rg = p / groups;
+    unit[i].cg = p % groups;
+    const int c = 8 * unit[i].cg;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 4 * unit[i].rg + e;
+      const bool there = r < rows && c < cols;
+      unit[i].v[e] = *reinterpret_cast<const uint4*>(w + (there ? r * cols + c : 0));
+    }
+  }
+  first_rows();
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int u = 64 * wave + i * NTHREADS;
+    if (u >= ALL) break;
+    const bool in = u < U_IN, out = u >= U_IN + U_HID;
+    const int rg = unit[i].rg, cg = unit[i].cg, rows = out ? a.d_out : HP, cols = in ? a.d_in : HP;
+    uint4(&v)[4] = unit[i].v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (4 * rg + e >= rows || 8 * cg >= cols) v[e] = make_uint4(0u, 0u, 0u, 0u);
+    if (!out) {
+      uint16_t* f = (in ? f_in : f_hid) + (size_t)((rg >> 2) * (in ? KIN / 32 : HP / 32) + (cg >> 2)) * FRAG_ELEMS;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) put_chain(f, 4 * (rg & 3) + e, cg & 3, v[e]);
+    }
+    // columns 8 cg .. of the rows 4 rg ..: element 4 ((rg / 4) % 2) .. of lane group rg % 4
+    uint16_t* t = (in ? t_in : out ? t_out : t_hid) + (size_t)((cg >> 1) * (out ? OUTP / 32 : HP / 32) + (rg >> 3)) * FRAG_ELEMS +
+                  ((rg & 3) * 16 + 8 * (cg & 1)) * 8 + 4 * ((rg >> 2) & 1);
+    const uint32_t(&d)[4][4] = reinterpret_cast<const uint32_t(&)[4][4]>(v);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      *reinterpret_cast<uint2*>(t + 16 * c) = make_uint2(__builtin_amdgcn_perm(d[1][c], d[0][c], 0x05040100u), __builtin_amdgcn_perm(d[3][c], d[2][c], 0x05040100u));
+      *reinterpret_cast<uint2*>(t + 16 * c + 8) = make_uint2(__builtin_amdgcn_perm(d[1][c], d[0][c], 0x07060302u), __builtin_amdgcn_perm(d[3][c], d[2][c], 0x07060302u));
+    }
+  }
+}
+
 // NT: 16-row tiles per chunk (2 or 4).  Four give the scheduler two independent 32-row groups to interleave.
 // XC: how x / dx are stored (MlpArgs::x_conv), fixed at compile time so that the usual case pays nothing for it;
 // XC == 3: stored like the weights, and the network's activation is applied to x as it is loaded (MlpArgs::in_act).
@@ -279,11 +340,15 @@ __global__ __launch_bounds__(64 * WAVES, 1) void mlp_bwd2_k(MlpArgs a) {
   uint32_t* trA = reinterpret_cast<uint32_t*>(bias_hid + HP) + (size_t)wave * NT * TR_PANEL_DWORDS;  // NT / 2 groups x 2 panels
   uint32_t* trD = trA + TR_PANEL_DWORDS;
 
-  stage_weight_frags<true, false, nthreads>(f_in, a.w_in, a.d_hidden, a.d_in, MT_H, KC_IN, tid, nthreads);
-  stage_weight_frags<true, false, nthreads>(f_hid, a.w_hid, a.d_hidden, a.d_hidden, MT_H, KC_H, tid, nthreads);
-  stage_weight_frags<true, true, nthreads>(t_in, a.w_in, a.d_hidden, a.d_in, MT_I, KC_H, tid, nthreads);
-  stage_weight_frags<true, true, nthreads>(t_hid, a.w_hid, a.d_hidden, a.d_hidden, MT_H, KC_H, tid, nthreads);
-  stage_weight_frags<true, true, nthreads>(t_out, a.w_out, a.d_out, a.d_hidden, MT_H, KC_O, tid, nthreads);
+  if (a.d_hidden == HP && a.d_in % 8 == 0 && ((uintptr_t)a.w_in | (uintptr_t)a.w_hid | (uintptr_t)a.w_out) % 16 == 0) {
+    stage_both_forms<KIN, HP, 32 * KC_O, nthreads>(f_in, f_hid, t_in, t_hid, t_out, a, tid, [] {});
+  } else {
+    stage_weight_frags<true, false, nthreads>(f_in, a.w_in, a.d_hidden, a.d_in, MT_H, KC_IN, tid, nthreads);
+    stage_weight_frags<true, false, nthreads>(f_hid, a.w_hid, a.d_hidden, a.d_hidden, MT_H, KC_H, tid, nthreads);
+    stage_weight_frags<true, true, nthreads>(t_in, a.w_in, a.d_hidden, a.d_in, MT_I, KC_H, tid, nthreads);
+    stage_weight_frags<true, true, nthreads>(t_hid, a.w_hid, a.d_hidden, a.d_hidden, MT_H, KC_H, tid, nthreads);
+    stage_weight_frags<true, true, nthreads>(t_out, a.w_out, a.d_out, a.d_hidden, MT_H, KC_O, tid, nthreads);
+  }
   stage_bias<T>(bias_in, a.b_in, a.d_hidden, HP, tid, nthreads);
   stage_bias<T>(bias_hid, a.b_hid, a.d_hidden, HP, tid, nthreads);
   __syncthreads();

@@ -53,3 +53,21 @@ def test_accumulation_in_chunks_of_blocks(N, cube, F, T, L, dtype):
     want = _grad(x, do, E, F, T, lo, hi, L, flags=2)
     torch.testing.assert_close(got, want, rtol=1e-3, atol=2e-3 if cube == 1.0 else 2**-16 * 2**8.5 * 5)
     assert torch.equal(got, _grad(x, do, E, F, T, lo, hi, L, flags=16))
+
+
+# rows of one piece of 16 bytes, of four, of eight, of numbers between them and of more; blocks of points and chunks that are short, whole and one over
+@pytest.mark.parametrize("N", [8192, 8193, 8447, 8449, 9215, 9216, 9999])
+@pytest.mark.parametrize("L,F,dtype", [(4, 2, torch.float16), (16, 2, torch.bfloat16), (10, 4, torch.float16), (6, 8, torch.float16), (9, 8, torch.bfloat16),
+                                       (2, 2, torch.float32), (16, 2, torch.float32), (7, 4, torch.float32), (13, 4, torch.float32)])  # fmt: skip
+def test_gradient_rows_turned_for_the_walk(N, L, F, dtype):
+    """Rows that are not 16-byte aligned are read a value at a time and give the same bits.  Bounds against the atomics as above."""
+    torch.manual_seed(N + L)
+    T, lo, hi = 2**14, 8, 512
+    x = torch.rand(N, 3, device=DEV)
+    E = O.level_row_offsets(L, T, 3, lo, hi)[-1]
+    do = torch.randn(N, L * F, device=DEV).to(dtype)
+    do[N // 2, -1] = 40.0  # the largest of the last plane
+    shifted = torch.empty(N * L * F + 1, device=DEV, dtype=dtype)[1:].view(N, L * F).copy_(do)
+    got = _grad(x, do, E, F, T, lo, hi, L)
+    assert torch.equal(got, _grad(x, shifted, E, F, T, lo, hi, L))
+    torch.testing.assert_close(got, _grad(x, do, E, F, T, lo, hi, L, flags=2), rtol=1e-3, atol=1e-3)

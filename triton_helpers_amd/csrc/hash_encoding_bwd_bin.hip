@@ -1225,10 +1225,11 @@ __global__ __launch_bounds__(REDUCE_THREADS) void hash_bwd_bin_reduce_k(BinWs ws
 // set the fixed-point scales.  A bin of one slice goes from the tile to the table; slices leave their sums in slots, which a last
 // pass adds in their order: a gradient has the same bits in every run.
 // Before (two rounds of workgroups that waited for each point, scattered adds of the tiles, zeros and rounding of the table as passes of
-// their own) -> now: 2^14 rows float32, 2^18 points 145 -> 68 us, of which the walk 91 -> 42; fp16 2^16 rows, 8192 points 80 -> 35 (was: records).
+// their own) -> now: 2^14 rows float32, 2^18 points 145 -> 63 us, of which the walk 91 -> 42; fp16 2^16 rows, 8192 points 80 -> 28 (was: records).
 constexpr int WALK_THREADS = 1024;
 constexpr int WALK_PREP_THREADS = 256;
 constexpr int WALK_STRIDE = 16;  // points between neighbouring lanes of a walk
+constexpr int PREP_PITCH = 9;    // 16-byte pieces between the rows that hash_bwd_walk_prep_k turns in LDS
 
 struct WalkPlan {
   int n_levels, n_tasks, prep_blocks;
@@ -1249,13 +1250,16 @@ struct WalkWs {
 
 // Gradient pairs level by level and coordinates dimension by dimension, both in the order of the walk: neighbouring lanes of a walk take
 // points WALK_STRIDE apart, because along a ray neighbouring points share cells and their adds to one row would wait for each other
-// (T = 2^14, 2^18 points along rays: 258 us without, 85 with).  The pass is bound by its loads, a row per lane: they are all
-// asked for before any is used (a loop over the levels that waited for each pair took 45 us for 2^18 rows of 16 float32 pairs, this 18).
+// (T = 2^14, 2^18 points along rays: 258 us without, 85 with).  Rows of whole 16-byte pieces (`vec`) come in as they lie, 512 bytes of four
+// neighbouring points to 32 lanes, up to 128 bytes of a row at once, and are turned to a row per lane in LDS: read a row per lane from memory,
+// the lines of a unit's lanes are ten times its L1 and every piece fetched its line again.  A thread's pieces are all of the same planes, so the
+// maxima are taken before the turn (one per plane and row behind it: 72.9 us).  The chain of a float32 table of 2^14 rows, 2^18 points 66.0 -> 63.3 us
+// (this kernel 20.0 -> 16.6, 67 MB), 4096 points 21.8 -> 19.9; fp16 2^18 61.6 -> 59.3, rows of four features 2^17 77.5 -> 73.3.
 template <bool G32, int D>
 __global__ __launch_bounds__(WALK_PREP_THREADS) void hash_bwd_walk_prep_k(const void* coords, int cdt, int64_t csn, int64_t csd, float scale,
                                                                           const void* dout_v, int64_t dout_stride, int64_t N, int levels, int feat,
-                                                                          WalkWs ws) {
-  extern __shared__ uint32_t plane_max[];
+                                                                          int vec, WalkWs ws) {
+  extern __shared__ __align__(16) uint32_t plane_max[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int np = (feat + 1) / 2, planes = levels * np;
   for (int i = tid; i < planes; i += WALK_PREP_THREADS) plane_max[i] = 0u;
@@ -1265,57 +1269,95 @@ __global__ __launch_bounds__(WALK_PREP_THREADS) void hash_bwd_walk_prep_k(const 
   constexpr int CHUNK = 64 * WALK_STRIDE;
   const int64_t chunk = at / CHUNK * CHUNK;
   const int in_chunk = (int)(at - chunk);
-  const int64_t n = !valid ? 0 : chunk + CHUNK <= N ? chunk + (in_chunk & 63) * WALK_STRIDE + (in_chunk >> 6) : at;
+  const bool whole = chunk + CHUNK <= N;  // (the same for the workgroup)
+  const int64_t n = !valid ? 0 : whole ? chunk + (in_chunk & 63) * WALK_STRIDE + (in_chunk >> 6) : at;
   float v[D];
   load_point_d<D>(coords, cdt, csn, csd, n, scale, v);
-#pragma unroll
-  for (int d = 0; d < D; ++d)
-    if (valid) ws.points[d * N + at] = v[d];
   const uint16_t* row16 = reinterpret_cast<const uint16_t*>(dout_v) + n * dout_stride;
   const float* row32 = reinterpret_cast<const float*>(dout_v) + n * dout_stride;
+  static_assert(WALK_PREP_THREADS == 4 * 64, "a workgroup's positions are four points of each of a chunk's groups");
   auto put = [&](int plane, uint32_t x, uint32_t y) {
-    if (valid) {
-      if (G32) reinterpret_cast<uint2*>(ws.pairs)[(int64_t)plane * N + at] = make_uint2(x, y);
-      else ws.pairs[(int64_t)plane * N + at] = x;
-    }
-    uint32_t m = G32 ? max(x & 0x7fffffffu, y & 0x7fffffffu) : max(x & 0x7fffu, (x >> 16) & 0x7fffu);
-    m = wave_max_u32(valid ? m : 0u);
-    if (lane == 63 && m) atomicMax(plane_max + plane, m);
+    if (!valid) return;
+    if (G32) reinterpret_cast<uint2*>(ws.pairs)[(int64_t)plane * N + at] = make_uint2(x, y);
+    else ws.pairs[(int64_t)plane * N + at] = x;
   };
-  // rows of whole 16-byte pieces, each four planes (float32: two); pieces of a row that ends between them read zeros
-  constexpr int PER = G32 ? 2 : 4;
-  const bool row_vec = (feat & 1) == 0 && planes % PER == 0 && ((uintptr_t)dout_v & 15u) == 0 && dout_stride % (G32 ? 4 : 8) == 0;
-  if (row_vec) {
-    constexpr int AT_ONCE = 8;
-    const uint4* row = G32 ? reinterpret_cast<const uint4*>(row32) : reinterpret_cast<const uint4*>(row16);
-    for (int q0 = 0; q0 < planes / PER; q0 += AT_ONCE) {
-      uint4 q[AT_ONCE];
+  auto pair_max = [&](uint32_t x, uint32_t y) { return G32 ? max(x & 0x7fffffffu, y & 0x7fffffffu) : max(x & 0x7fffu, (x >> 16) & 0x7fffu); };
+  if (vec) {
+    constexpr int PER = G32 ? 2 : 4;  // planes of a piece
+    uint4* tile = reinterpret_cast<uint4*>(plane_max + (planes + 3) / 4 * 4);  // [position][PREP_PITCH]
+    const int pieces = planes / PER;
+    auto block = [&](int q0, auto width_c) {  // pieces q0 .. of the rows
+      constexpr int W = decltype(width_c)::value;
+      uint4 v[W];
 #pragma unroll
-      for (int i = 0; i < AT_ONCE; ++i)
-        if (q0 + i < planes / PER) q[i] = row[q0 + i];
+      for (int i = 0; i < W; ++i) {
+        const int u = tid + i * WALK_PREP_THREADS, row = u / W, q = q0 + u % W;
+        const int64_t first = chunk + in_chunk / WALK_PREP_THREADS * (WALK_PREP_THREADS / 64);
+        int64_t r = whole ? first + row / 4 * WALK_STRIDE + row % 4 : (int64_t)blockIdx.x * WALK_PREP_THREADS + row;
+        r = r < N ? r : N - 1;
+        const char* p = reinterpret_cast<const char*>(dout_v) + r * dout_stride * (G32 ? 4 : 2);
+        v[i] = reinterpret_cast<const uint4*>(p)[q < pieces ? q : pieces - 1];
+      }
 #pragma unroll
-      for (int i = 0; i < AT_ONCE; ++i)
-        if (q0 + i < planes / PER) {
+      for (int i = 0; i < W; ++i) {
+        const int u = tid + i * WALK_PREP_THREADS, row = u / W, slot = whole ? row % 4 * 64 + row / 4 : row;
+        tile[slot * PREP_PITCH + u % W] = v[i];
+      }
+      // a thread's pieces are of the same planes, and so are those of every W-th lane
+      uint32_t m[PER] = {};
+#pragma unroll
+      for (int i = 0; i < W; ++i) {
+        if constexpr (G32) {
+          m[0] = max(m[0], pair_max(v[i].x, v[i].y));
+          m[1] = max(m[1], pair_max(v[i].z, v[i].w));
+        } else {
+          m[0] = max(m[0], pair_max(v[i].x, 0u));
+          m[1] = max(m[1], pair_max(v[i].y, 0u));
+          m[2] = max(m[2], pair_max(v[i].z, 0u));
+          m[3] = max(m[3], pair_max(v[i].w, 0u));
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+#pragma unroll
+        for (int d = W; d < 64; d *= 2) m[k] = max(m[k], (uint32_t)__shfl_xor((int)m[k], d));
+        if (lane < W && q0 + lane < pieces) atomicMax(plane_max + (q0 + lane) * PER + k, m[k]);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < W; ++i)
+        if (q0 + i < pieces) {
+          const uint4 q = tile[tid * PREP_PITCH + i];
           const int plane = (q0 + i) * PER;
           if constexpr (G32) {
-            put(plane, q[i].x, q[i].y);
-            put(plane + 1, q[i].z, q[i].w);
+            put(plane, q.x, q.y);
+            put(plane + 1, q.z, q.w);
           } else {
-            put(plane, q[i].x, 0u);
-            put(plane + 1, q[i].y, 0u);
-            put(plane + 2, q[i].z, 0u);
-            put(plane + 3, q[i].w, 0u);
+            put(plane, q.x, 0u);
+            put(plane + 1, q.y, 0u);
+            put(plane + 2, q.z, 0u);
+            put(plane + 3, q.w, 0u);
           }
         }
-    }
+      __syncthreads();
+    };
+    int q0 = 0;
+    for (; pieces - q0 > 4; q0 += 8) block(q0, std::integral_constant<int, 8>{});
+    if (q0 < pieces) block(q0, std::integral_constant<int, 4>{});
   } else {
     for (int plane = 0; plane < planes; ++plane) {
       const int e0 = plane / np * feat + 2 * (plane % np);
       const bool two = 2 * (plane % np) + 1 < feat;
-      if (G32) put(plane, __float_as_uint(row32[e0]), two ? __float_as_uint(row32[e0 + 1]) : 0u);
-      else put(plane, (uint32_t)row16[e0] | (two ? (uint32_t)row16[e0 + 1] << 16 : 0u), 0u);
+      const uint32_t x = G32 ? __float_as_uint(row32[e0]) : (uint32_t)row16[e0] | (two ? (uint32_t)row16[e0 + 1] << 16 : 0u);
+      const uint32_t y = G32 && two ? __float_as_uint(row32[e0 + 1]) : 0u;
+      put(plane, x, y);
+      const uint32_t m = wave_max_u32(valid ? pair_max(x, y) : 0u);
+      if (lane == 63 && m) atomicMax(plane_max + plane, m);
     }
   }
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (valid) ws.points[d * N + at] = v[d];
   __syncthreads();
   for (int i = tid; i < planes; i += WALK_PREP_THREADS) ws.block_max[(int64_t)i * gridDim.x + blockIdx.x] = plane_max[i];
 }
@@ -1754,8 +1796,11 @@ static int launch_bwd_walk(const void* coords, int cdt, int64_t csn, int64_t csd
   else if (g.dims == 2) pick(std::integral_constant<int, 2>{});
   else if (g.dims == 1) pick(std::integral_constant<int, 1>{});
   else pick(std::integral_constant<int, 4>{});
-  void* prep_args[] = {(void*)&coords, (void*)&cdt, (void*)&csn, (void*)&csd, (void*)&scale, (void*)&dout, (void*)&dout_stride, (void*)&N, (void*)&levels, (void*)&feat, (void*)&ws};
-  if (int rc = launch_large("hash_bwd_walk_prep", prep, dim3((unsigned)wp.prep_blocks), WALK_PREP_THREADS, prep_args, (size_t)levels * ((feat + 1) / 2) * 4, s)) return rc;
+  const int planes = levels * ((feat + 1) / 2);
+  int vec = feat % 2 == 0 && planes % (ddt == NF_F32 ? 2 : 4) == 0 && (uintptr_t)dout % 16 == 0 && dout_stride % (ddt == NF_F32 ? 4 : 8) == 0;
+  void* prep_args[] = {(void*)&coords, (void*)&cdt, (void*)&csn, (void*)&csd, (void*)&scale, (void*)&dout, (void*)&dout_stride, (void*)&N, (void*)&levels, (void*)&feat, (void*)&vec, (void*)&ws};
+  const size_t prep_lds = (size_t)(planes + 3) / 4 * 16 + (vec ? (size_t)WALK_PREP_THREADS * PREP_PITCH * 16 : 0);
+  if (int rc = launch_large("hash_bwd_walk_prep", prep, dim3((unsigned)wp.prep_blocks), WALK_PREP_THREADS, prep_args, prep_lds, s)) return rc;
   const void* reduce = with_mode(mode, [](auto mode_c) { return (const void*)hash_bwd_walk_reduce_k<decltype(mode_c)::value>; });
   const unsigned units = (unsigned)compute_units(), groups = (unsigned)wp.n_tasks < units ? (unsigned)wp.n_tasks : units;
   int64_t most_rows = 0;

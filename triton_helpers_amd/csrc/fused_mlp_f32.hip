@@ -4,7 +4,7 @@
 // path; this one is bound by the float32 matrix rate (157 TFLOP/s) and, beyond two hidden layers, by its activations'
 // round trip in the backward.
 //
-// Forward: one launch for any depth.  A wave carries 32 rows (two groups of 16) through all layers in registers.
+// Forward: one launch for any depth.  A wave carries 32 rows (two groups of 16), in small batches 16, through all layers in registers.
 // The product is formed transposed, out^T = W * h^T, so that the 16x16 result tile of a layer (lane (r, g), register v:
 // feature 16*mt + 4*g + v of row r) is already the K operand of the next layer when K is walked in the order
 // 16*t + 4*g + v; the weights are read from LDS in that order (one ds_read_b128 per four products).  Weights of all
@@ -25,8 +25,6 @@ constexpr int W32_RESIDENT_MAX = 8;                      // layers kept in LDS a
 constexpr int T32_STRIDE = 80;                           // floats per row of a wave's 16-row transposing panel
 constexpr int PART32 = 64 * 64 + 64;                     // floats of one workgroup's partial dW (64 x 64) and db (64)
 constexpr int SLOTS32 = 512;                             // most workgroups of a backward launch
-constexpr int NT32 = 2;                                  // 16-row groups a wave of the forward carries at once
-constexpr int CHUNK32 = 4 * NT32 * 16;                   // rows per workgroup and pass of the forward
 
 struct Mlp32Args {
   const float* x;
@@ -115,10 +113,15 @@ __device__ __forceinline__ void stage_layer32(float* dst, const float* w, const 
   if (tid < 64) dst[64 * W32_STRIDE + tid] = (b != nullptr && tid < n_out) ? b[tid] : 0.0f;
 }
 
-template <int ACT>
+// Forward.  NT: 16-row groups that a wave carries at once (fwd32()).  PIECES: rows of x and y are whole 16-byte aligned pieces, which are read and
+// written without a test per value.  Bound by the float32 products (157 TFLOP/s) from about 2^18 rows; below by what a workgroup waits for before
+// its first one.  Layers staged one after the other, rows asked for when the chunk in front was done, 128 rows to a workgroup -> this, us: 32 -> 64 ->
+// 64 -> 16, 4096 rows 11.4 -> 7.4, 100003 28.7 -> 23.6 (1.4 GFLOP), 2^18 47.9 -> 46.0; eight hidden layers of 64, 2^15 42.9 -> 35.4; 64 -> 64 -> 64 ->
+// 64, 2^20 265 -> 249.
+template <int ACT, int NT, bool PIECES>
 __global__ __launch_bounds__(256, 2) void mlp32_fwd_k(Mlp32Args a) {
   extern __shared__ float lds32[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int H = a.d_hidden, last = a.depth;
   auto layer_w = [&](int l) { return l == 0 ? a.w_in : l == last ? a.w_out : a.w_hid + (size_t)(l - 1) * H * H; };
@@ -127,23 +130,90 @@ __global__ __launch_bounds__(256, 2) void mlp32_fwd_k(Mlp32Args a) {
   };
   auto n_in = [&](int l) { return l == 0 ? a.d_in : H; };
   auto n_out = [&](int l) { return l == last ? a.d_out : H; };
-  if (a.resident) {
-    for (int l = 0; l < a.n_layers; ++l) stage_layer32(lds32 + l * W32_LAYER, layer_w(l), layer_b(l), n_out(l), n_in(l), tid);
-    __syncthreads();
-  }
   const bool x_vec = ((uintptr_t)a.x % 16 == 0) && (a.x_stride % 4 == 0);
   const bool y_vec = a.y != nullptr && ((uintptr_t)a.y % 16 == 0) && (a.y_stride % 4 == 0);
-  const int64_t n_chunks = (a.rows + CHUNK32 - 1) / CHUNK32;
-  for (int64_t chunk = blockIdx.x; chunk < n_chunks; chunk += gridDim.x) {
-    const int64_t row0 = chunk * CHUNK32 + wave * (NT32 * 16) + r;
-    f32x4_t h[NT32][4];
-    const int kt_in = (a.d_in + 15) / 16;
+  const int kt_in = (a.d_in + 15) / 16;
+  // a chunk's rows go to the workgroups in turn, then to their waves; the next chunk's are requested before this one's products
+  const int64_t n_chunks = (a.rows + 16 * NT - 1) / (16 * NT), per_round = (int64_t)gridDim.x * 4;
+  f32x4_t nx[NT][4];
+  auto load_rows = [&](int64_t chunk) {
 #pragma unroll
-    for (int nt = 0; nt < NT32; ++nt)
+    for (int nt = 0; nt < NT; ++nt) {
+      const int64_t row = chunk * (16 * NT) + 16 * nt + r;
+      const float* p = a.x + (row < a.rows ? row : a.rows - 1) * a.x_stride;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        h[nt][t] = t < kt_in ? load_chain(a.x, a.x_stride, row0 + 16 * nt, a.rows, 16 * t + 4 * g, a.d_in, x_vec)
-                             : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int t = 0; t < 4; ++t) {
+        if (t >= kt_in) break;
+        const int col = 16 * t + 4 * g;
+        if constexpr (PIECES) nx[nt][t] = *reinterpret_cast<const f32x4_t*>(p + (col < a.d_in ? col : 0));
+        else nx[nt][t] = load_chain(a.x, a.x_stride, row, a.rows, col, a.d_in, x_vec);
+      }
+    }
+  };
+  const int64_t first_chunk = (int64_t)wave * gridDim.x + blockIdx.x;
+  if (a.resident) {
+    // The layers are staged LAYERS at a time, their loads under way together and the first rows' behind them; layer by layer each waited
+    // for the one in front.
+    constexpr int LAYERS = 3, PER = 1024 / 256;
+    for (int l0 = 0; l0 < a.n_layers; l0 += LAYERS) {
+      f32x4_t v[LAYERS][PER];
+      // a wave takes the bias of a layer
+      const int bl = l0 + wave;
+      const float* b = wave < LAYERS && bl < a.n_layers ? layer_b(bl) : nullptr;
+      const bool has_bias = b != nullptr && lane < n_out(bl);
+      const float bias = *(has_bias ? b + lane : a.w_in);
+#pragma unroll
+      for (int k = 0; k < LAYERS; ++k) {
+        const int l = l0 + k;
+        if (l >= a.n_layers) break;
+        const float* w = layer_w(l);
+        const int rows = n_out(l), cols = n_in(l);
+        if (cols % 4 != 0 || (uintptr_t)w % 16 != 0) continue;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+          const int o = (tid >> 4) + 16 * i, c = 4 * (tid & 15);
+          v[k][i] = *reinterpret_cast<const f32x4_t*>(w + (o < rows ? o : 0) * cols + (c < cols ? c : 0));
+        }
+      }
+      if (PIECES && l0 == 0) load_rows(first_chunk);
+#pragma unroll
+      for (int k = 0; k < LAYERS; ++k) {
+        const int l = l0 + k;
+        if (l >= a.n_layers) break;
+        float* dst = lds32 + l * W32_LAYER;
+        const float* w = layer_w(l);
+        const int rows = n_out(l), cols = n_in(l);
+        if (cols % 4 != 0 || (uintptr_t)w % 16 != 0) {
+          read_layer32(w, rows, cols, tid, [&](int o, int c, f32x4_t x) { *reinterpret_cast<f32x4_t*>(dst + o * W32_STRIDE + c) = x; });
+          continue;
+        }
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+          const int o = (tid >> 4) + 16 * i, c = 4 * (tid & 15);
+          *reinterpret_cast<f32x4_t*>(dst + o * W32_STRIDE + c) = o < rows && c < cols ? v[k][i] : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+      }
+      if (wave < LAYERS && bl < a.n_layers) lds32[bl * W32_LAYER + 64 * W32_STRIDE + lane] = has_bias ? bias : 0.0f;
+    }
+    __syncthreads();
+  } else if (PIECES) {
+    load_rows(first_chunk);
+  }
+  const int64_t rounds = (n_chunks + per_round - 1) / per_round;
+  for (int64_t round = 0; round < rounds; ++round) {
+    const int64_t chunk = first_chunk + round * per_round;
+    if (a.resident && chunk >= n_chunks) break;
+    const int64_t row0 = chunk * (16 * NT) + r;
+    f32x4_t h[NT][4];
+    if (!PIECES) load_rows(chunk);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if (t >= kt_in) break;
+        h[nt][t] = PIECES && 16 * t + 4 * g >= a.d_in ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : nx[nt][t];
+      }
+    if (PIECES) load_rows(chunk + per_round);
     for (int l = 0; l < a.n_layers; ++l) {
       const float* wl = lds32;
       if (a.resident) {
@@ -154,12 +224,12 @@ __global__ __launch_bounds__(256, 2) void mlp32_fwd_k(Mlp32Args a) {
         __syncthreads();
       }
       const int kt = (n_in(l) + 15) / 16, mt_n = (n_out(l) + 15) / 16;
-      f32x4_t acc[NT32][4];
+      f32x4_t acc[NT][4];
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt) {
         const f32x4_t b4 = *reinterpret_cast<const f32x4_t*>(wl + 64 * W32_STRIDE + 16 * mt + 4 * g);
 #pragma unroll
-        for (int nt = 0; nt < NT32; ++nt) acc[nt][mt] = b4;
+        for (int nt = 0; nt < NT; ++nt) acc[nt][mt] = b4;
       }
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
@@ -171,18 +241,23 @@ __global__ __launch_bounds__(256, 2) void mlp32_fwd_k(Mlp32Args a) {
 #pragma unroll
           for (int v = 0; v < 4; ++v)
 #pragma unroll
-            for (int nt = 0; nt < NT32; ++nt) acc[nt][mt] = mfma4(w4[v], h[nt][t][v], acc[nt][mt]);
+            for (int nt = 0; nt < NT; ++nt) acc[nt][mt] = mfma4(w4[v], h[nt][t][v], acc[nt][mt]);
         }
       }
       if (l == last) {
 #pragma unroll
-        for (int nt = 0; nt < NT32; ++nt)
+        for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
           for (int mt = 0; mt < 4; ++mt)
-            if (mt < mt_n) store_chain(a.y, a.y_stride, row0 + 16 * nt, a.rows, 16 * mt + 4 * g, a.d_out, y_vec, acc[nt][mt]);
+            if (mt < mt_n) {
+              const int64_t row = row0 + 16 * nt;
+              const int col = 16 * mt + 4 * g;
+              if constexpr (!PIECES) store_chain(a.y, a.y_stride, row, a.rows, col, a.d_out, y_vec, acc[nt][mt]);
+              else if (row < a.rows && col < a.d_out) *reinterpret_cast<f32x4_t*>(a.y + row * a.y_stride + col) = acc[nt][mt];
+            }
       } else {
 #pragma unroll
-        for (int nt = 0; nt < NT32; ++nt)
+        for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
           for (int mt = 0; mt < 4; ++mt) {
             if (a.z != nullptr && mt < mt_n)
@@ -657,17 +732,32 @@ static int fwd32(Mlp32Args a, hipStream_t s) {
   a.n_layers = a.y != nullptr ? a.depth + 1 : a.depth;
   a.resident = a.n_layers <= W32_RESIDENT_MAX;
   const size_t lds = (size_t)(a.resident ? a.n_layers : 1) * W32_LAYER * sizeof(float);
-  const int64_t chunks = (a.rows + CHUNK32 - 1) / CHUNK32;
   const int64_t cap = (int64_t)device_cus() * (lds > 76 * 1024 ? 1 : 2);
-  const int64_t blocks = chunks < cap ? chunks : cap;
-  const void* kern = nullptr;
-  switch (a.act) {
-    case NF_ACT_RELU: kern = (const void*)mlp32_fwd_k<NF_ACT_RELU>; break;
-    case NF_ACT_SILU: kern = (const void*)mlp32_fwd_k<NF_ACT_SILU>; break;
-    case NF_ACT_RELU2: kern = (const void*)mlp32_fwd_k<NF_ACT_RELU2>; break;
-    case NF_ACT_GELU: kern = (const void*)mlp32_fwd_k<NF_ACT_GELU>; break;
-    default: kern = (const void*)mlp32_fwd_k<NF_ACT_NONE>; break;
-  }
+  // One group of sixteen rows to a wave where a SIMD's share of them is a tenth less than that of pairs, or there is no pair for every SIMD.  us, one /
+  // two: 32 -> 64 -> 64 -> 16, 4096 rows 7.4 / 10.2, 40000 14.0 / 15.1, 100003 23.6 / 25.9, 2^18 47.5 / 46.0; eight hidden layers of 64, 2^15 35.4 /
+  // 43.7; 16 -> 32 -> 32 -> 4, 2^16 10.0 / 9.7; 64 -> 64 -> 64 -> 64, 2^20 259 / 249.
+  const int64_t simds = (int64_t)device_cus() * 4, ones = (a.rows + 15) / 16, twos = (a.rows + 31) / 32;
+  const auto share = [&](int64_t units) { return (units + simds - 1) / simds; };
+  const bool single = twos <= simds || 10 * share(ones) < 9 * 2 * share(twos);
+  const int64_t chunks = single ? ones : twos, full = (chunks + 3) / 4;
+  int64_t blocks = full < cap ? full : cap;
+  if (blocks < device_cus()) blocks = chunks < device_cus() ? chunks : device_cus();
+  const auto pieces = [](const float* p, int64_t stride, int width) { return (uintptr_t)p % 16 == 0 && stride % 4 == 0 && width % 4 == 0; };
+  const bool whole = pieces(a.x, a.x_stride, a.d_in) && (a.y == nullptr || pieces(a.y, a.y_stride, a.d_out));
+  auto pick = [&](auto nt_c, auto whole_c) -> const void* {
+    constexpr int NT = decltype(nt_c)::value;
+    constexpr bool PIECES = decltype(whole_c)::value;
+    switch (a.act) {
+      case NF_ACT_RELU: return (const void*)mlp32_fwd_k<NF_ACT_RELU, NT, PIECES>;
+      case NF_ACT_SILU: return (const void*)mlp32_fwd_k<NF_ACT_SILU, NT, PIECES>;
+      case NF_ACT_RELU2: return (const void*)mlp32_fwd_k<NF_ACT_RELU2, NT, PIECES>;
+      case NF_ACT_GELU: return (const void*)mlp32_fwd_k<NF_ACT_GELU, NT, PIECES>;
+      default: return (const void*)mlp32_fwd_k<NF_ACT_NONE, NT, PIECES>;
+    }
+  };
+  const std::integral_constant<int, 1> one;
+  const std::integral_constant<int, 2> two;
+  const void* kern = whole ? (single ? pick(one, std::true_type{}) : pick(two, std::true_type{})) : single ? pick(one, std::false_type{}) : pick(two, std::false_type{});
   return launch32(kern, a, blocks, lds, s, "mlp32_fwd");
 }
 

@@ -250,6 +250,14 @@ int nf_mlp_bwd_whole(const void* x, int64_t x_stride, const void* dy, int64_t dy
                      int x_dtype, int grad_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 int64_t nf_mlp_bwd_whole_workspace_bytes(int64_t rows, int d_hidden, int depth, int act, int dtype);
 
+/* nf_mlp_bwd of a float32 network of one or two hidden layers with the dw_ / db_ buffers WRITTEN, so that nothing has to be cleared in front: the
+ * same sums.  NF_EUNSUPPORTED, before anything is launched: deeper networks, no rows.  workspace: as for nf_mlp_bwd. */
+int nf_mlp_bwd_f32(const float* x, int64_t x_stride, const float* dy, int64_t dy_stride, float* dx, int64_t dx_stride,
+                   const float* w_in, const float* b_in, const float* w_hid, const float* b_hid, const float* w_out,
+                   const float* b_out, float* dw_in, float* db_in, float* dw_hid, float* db_hid, float* dw_out,
+                   float* db_out, int64_t rows, int d_in, int d_hidden, int d_out, int depth, int act, void* workspace,
+                   int64_t workspace_bytes, void* stream);
+
 /* n (<= 8) float32 arrays of count[k] values cast to float16 in one launch: piece k starts at dst plus the counts before it,
  * each rounded up to a multiple of 8. src and count are host arrays. */
 int nf_cast_pieces_f16(const float* const* src, const int64_t* count, int n, void* dst, void* stream);

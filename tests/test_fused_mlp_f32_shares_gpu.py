@@ -30,3 +30,37 @@ def test_every_share_gives_the_same_rows(rows, d_in, hidden, d_out, depth, shift
         if k < depth:
             h = h.relu()
     assert ((y.double() - h).abs() <= a * (66 * (depth + 1) * 2.0**-24)).all()
+
+
+@pytest.mark.parametrize("d_in,hidden,d_out,depth,bias", [(32, 64, 16, 2, True), (64, 64, 64, 2, False), (35, 32, 3, 1, True), (33, 16, 17, 2, True), (16, 64, 64, 1, False)])
+@pytest.mark.parametrize("rows", [1, 1000, 4097])
+def test_written_gradients_are_the_added_ones(rows, d_in, hidden, d_out, depth, bias):
+    """nf_mlp_bwd_f32 over buffers of NaN against nf_mlp_bwd over zeros: the same bits, and nothing beside the gradients is touched."""
+    from triton_helpers_amd import _lib
+
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(rows + d_in)
+    u = lambda *s: (torch.rand(*s, generator=g, device="cuda") * 2 - 1) * s[-1] ** -0.5  # noqa: E731
+    x, dy = u(rows, d_in), u(rows, d_out)
+    w = [u(hidden, d_in), u(hidden) if bias else None, u(hidden, hidden) if depth == 2 else None, u(1, hidden) if depth == 2 and bias else None,
+         u(d_out, hidden), u(d_out) if bias else None]  # fmt: skip
+    n = lib.nf_mlp_workspace_bytes(rows, hidden, depth, _lib.NF_ACT["relu"], 1, _lib.NF_F32)
+    ws, got = torch.empty(n, dtype=torch.uint8, device="cuda"), []
+    for fill in (0.0, float("nan")):
+        grads = [None if t is None else torch.full((t.numel() + 64,), fill, device="cuda") for t in w]
+        dx = torch.empty_like(x)
+        args = [x.data_ptr(), d_in, dy.data_ptr(), d_out, dx.data_ptr(), d_in, *map(_lib.ptr, w), *map(_lib.ptr, grads), rows, d_in, hidden, d_out, depth, _lib.NF_ACT["relu"]]
+        types, call = ([_lib.NF_F32, _lib.NF_F32], lib.nf_mlp_bwd) if fill == 0.0 else ([], lib.nf_mlp_bwd_f32)
+        _lib.check(call(*args, *types, ws.data_ptr(), n, _lib.current_stream(x.device)), "backward")
+        got.append([dx] + [t[:-64] for t in grads if t is not None])
+        rest = torch.cat([t[-64:] for t in grads if t is not None])
+        assert rest.isnan().all() if fill != fill else (rest == 0).all()
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+def test_written_gradients_need_rows_and_at_most_two_hidden_layers():
+    from triton_helpers_amd import _lib
+
+    lib = _lib.load()
+    for rows, depth in ((0, 2), (8, 3)):
+        assert lib.nf_mlp_bwd_f32(1, 32, 1, 16, None, 32, 1, None, 1, None, 1, None, 1, None, 1, None, 1, None, rows, 32, 64, 16, depth, 1, None, 0, None) == -2

@@ -51,6 +51,7 @@ EXPORTS = (
     "nf_mlp_bwd_summed",
     "nf_mlp_bwd_whole",
     "nf_mlp_bwd_whole_workspace_bytes",
+    "nf_mlp_bwd_f32",
     "nf_cast_pieces_f16",
     "nf_revmlp_fwd",
     "nf_revmlp_bwd",
@@ -122,6 +123,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.nf_mlp_bwd_summed.argtypes = [P, I64, P, I64, P, I64, P, P, P, P, P, P, P, P, P, P, P, P, I64, I, I, I, I, I, I, I, I, P, I64, P]
     lib.nf_mlp_bwd_whole.restype = c_int
     lib.nf_mlp_bwd_whole.argtypes = lib.nf_mlp_bwd_summed.argtypes
+    lib.nf_mlp_bwd_f32.restype = c_int
+    lib.nf_mlp_bwd_f32.argtypes = [P, I64, P, I64, P, I64, P, P, P, P, P, P, P, P, P, P, P, P, I64, I, I, I, I, I, P, I64, P]
     lib.nf_mlp_bwd_whole_workspace_bytes.restype = I64
     lib.nf_mlp_bwd_whole_workspace_bytes.argtypes = [I64, I, I, I, I]
     lib.nf_mlp_bwd_rounded_workspace_bytes.restype = I64

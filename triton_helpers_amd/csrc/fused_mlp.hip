@@ -836,6 +836,20 @@ extern "C" int nf_mlp_fwd(const void* x, int64_t x_stride, void* y, int64_t y_st
   return 0;
 }
 
+extern "C" int nf_mlp_bwd_f32(const float* x, int64_t x_stride, const float* dy, int64_t dy_stride, float* dx, int64_t dx_stride, const float* w_in,
+                              const float* b_in, const float* w_hid, const float* b_hid, const float* w_out, const float* b_out, float* dw_in,
+                              float* db_in, float* dw_hid, float* db_hid, float* dw_out, float* db_out, int64_t rows, int d_in, int d_hidden,
+                              int d_out, int depth, int act, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (int rc = validate(rows, d_in, d_hidden, d_out, depth, act, NF_F32)) return rc;
+  (void)b_out;
+  NF_REQUIRE(rows > 0, NF_EUNSUPPORTED, "written weight gradients: no rows (the buffers would stay unwritten)");
+  NF_REQUIRE(x && dy && w_in && w_out && dw_in && dw_out, NF_EINVAL, "NULL pointer argument");
+  NF_REQUIRE(depth == 1 || (w_hid && dw_hid), NF_EINVAL, "w_hid / dw_hid is NULL but depth=%d", depth);
+  NF_REQUIRE(x_stride >= d_in && dy_stride >= d_out && (dx == nullptr || dx_stride >= d_in), NF_EINVAL, "row stride smaller than row width");
+  return mlp32_bwd(x, x_stride, dy, dy_stride, dx, dx_stride, w_in, b_in, w_hid, b_hid, w_out, dw_in, db_in, dw_hid, db_hid, dw_out, db_out, rows,
+                   d_in, d_hidden, d_out, depth, act, true, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
 extern "C" int nf_mlp_bwd(const void* x, int64_t x_stride, const void* dy, int64_t dy_stride, void* dx, int64_t dx_stride,
                           const void* w_in, const void* b_in, const void* w_hid, const void* b_hid, const void* w_out,
                           const void* b_out, float* dw_in, float* db_in, float* dw_hid, float* db_hid, float* dw_out,
@@ -852,7 +866,7 @@ extern "C" int nf_mlp_bwd(const void* x, int64_t x_stride, const void* dy, int64
   if (dtype == NF_F32)
     return mlp32_bwd((const float*)x, x_stride, (const float*)dy, dy_stride, (float*)dx, dx_stride, (const float*)w_in,
                      (const float*)b_in, (const float*)w_hid, (const float*)b_hid, (const float*)w_out, dw_in, db_in, dw_hid,
-                     db_hid, dw_out, db_out, rows, d_in, d_hidden, d_out, depth, act, workspace, workspace_bytes,
+                     db_hid, dw_out, db_out, rows, d_in, d_hidden, d_out, depth, act, false, workspace, workspace_bytes,
                      (hipStream_t)stream);
   MlpArgs a = {};
   a.w_in = (const uint16_t*)w_in; a.b_in = (const uint16_t*)b_in; a.w_hid = (const uint16_t*)w_hid;

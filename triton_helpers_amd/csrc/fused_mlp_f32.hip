@@ -676,6 +676,7 @@ __global__ __launch_bounds__(64 * fused32_waves(TI, TO, DEPTH)) void mlp32_bwd_k
 struct Fused32Sums {
   float *dw_in, *db_in, *dw_hid, *db_hid, *dw_out, *db_out;
   int ti, to, depth, d_in, d_hidden, d_out, n_slots, sums;
+  int write;  // the sums replace what is there instead of being added to it
 };
 __global__ __launch_bounds__(1024) void mlp32_sum_k(const float* slots, Fused32Sums o) {
   __shared__ float part[16][64];
@@ -695,7 +696,7 @@ __global__ __launch_bounds__(1024) void mlp32_sum_k(const float* slots, Fused32S
   if (i >= tiles * 256) {
     const int k = (i - tiles * 256) >> 6, f = i & 63;
     float* db = k == 0 ? o.db_in : k == 1 ? o.db_hid : o.db_out;
-    if (db != nullptr && f < (k == 2 ? o.d_out : o.d_hidden) && (k != 1 || o.depth == 2)) db[f] += total;
+    if (db != nullptr && f < (k == 2 ? o.d_out : o.d_hidden) && (k != 1 || o.depth == 2)) db[f] = (o.write ? 0.0f : db[f]) + total;
     return;
   }
   int tile = i >> 8;
@@ -713,7 +714,10 @@ __global__ __launch_bounds__(1024) void mlp32_sum_k(const float* slots, Fused32S
     }
   }
   const int ln = (i & 255) >> 2, row = 16 * (tile / nt) + 4 * (ln >> 4) + (i & 3), col = 16 * (tile % nt) + (ln & 15);
-  if (row < n_out && col < n_in) dw[(size_t)row * n_in + col] += total;
+  if (row < n_out && col < n_in) {
+    float* p = dw + (size_t)row * n_in + col;
+    *p = (o.write ? 0.0f : *p) + total;
+  }
 }
 
 template <typename Args>
@@ -825,7 +829,8 @@ int mlp32_fwd(const float* x, int64_t x_stride, float* y, int64_t y_stride, cons
 int mlp32_bwd(const float* x, int64_t x_stride, const float* dy, int64_t dy_stride, float* dx, int64_t dx_stride,
               const float* w_in, const float* b_in, const float* w_hid, const float* b_hid, const float* w_out, float* dw_in,
               float* db_in, float* dw_hid, float* db_hid, float* dw_out, float* db_out, int64_t rows, int d_in, int d_hidden,
-              int d_out, int depth, int act, void* workspace, int64_t workspace_bytes, hipStream_t s) {
+              int d_out, int depth, int act, bool write, void* workspace, int64_t workspace_bytes, hipStream_t s) {
+  NF_REQUIRE(!write || depth <= 2, NF_EUNSUPPORTED, "float32 gradients are written for one and two hidden layers (depth=%d)", depth);
   const size_t need = mlp32_bwd_workspace_bytes(rows, d_hidden, depth);
   NF_REQUIRE(workspace != nullptr && workspace_bytes >= (int64_t)need, NF_EINVAL,
              "float32 backward keeps %d pre-activations of %lld x %d float32 and partial weight gradients: it needs a "
@@ -833,7 +838,7 @@ int mlp32_bwd(const float* x, int64_t x_stride, const float* dy, int64_t dy_stri
   NF_REQUIRE((uintptr_t)workspace % 16 == 0, NF_EINVAL, "workspace must be 16-byte aligned");
   if (depth <= 2) {
     Fused32Args a = {x, dy, dx, x_stride, dy_stride, dx_stride, rows, w_in, b_in, w_hid, b_hid, w_out, (float*)workspace, d_in, d_hidden, d_out, act};
-    Fused32Sums o = {dw_in, db_in, dw_hid, db_hid, dw_out, db_out, 0, 0, 0, d_in, d_hidden, d_out, 0, 0};
+    Fused32Sums o = {dw_in, db_in, dw_hid, db_hid, dw_out, db_out, 0, 0, 0, d_in, d_hidden, d_out, 0, 0, write};
     const bool narrow = d_in <= 32, small = d_out <= 16;
     if (depth == 2)
       return narrow ? (small ? bwd32_fused<2, 1, 2>(a, o, need, s) : bwd32_fused<2, 4, 2>(a, o, need, s))

@@ -325,14 +325,24 @@ variable_list mlp_backward(Mlp m, Tensor dy, bool need_dx, bool float_grads) {
     return finish(at, flat);
   }
   const Pieces at(m.w, 4);
-  flat = at::zeros({at.total}, m.w[0].options().dtype(at::kFloat));
   const int64_t bytes = nf_mlp_workspace_bytes(g.n, H, depth, m.act, 1, dt);
+  // float32 networks of one and two hidden layers: the gradients are written, with no fill in front (32 -> 64 -> 64 -> 16, 100003 rows: forward and backward 84 -> 78 us)
+  const bool written = wt == at::kFloat && depth <= 2 && g.n > 0;
+  flat = written ? at::empty({at.total}, m.w[0].options()) : at::zeros({at.total}, m.w[0].options().dtype(at::kFloat));
   const Tensor ws = scratch(bytes, m.x);
   dx = need_dx ? at::empty(m.x.sizes(), m.x.options()) : Tensor();
-  check(nf_mlp_bwd(x.p, x.stride, g.p, g.stride, ptr(dx), in, ptr(m.w[0]), ptr(m.w[1]), ptr(m.w[4]), ptr(m.w[5]), ptr(m.w[2]), ptr(m.w[3]),
-                   (float*)at.at(flat, m.w[0], 0), (float*)at.at(flat, m.w[1], 1), (float*)at.at(flat, m.w[4], 4), (float*)at.at(flat, m.w[5], 5),
-                   (float*)at.at(flat, m.w[2], 2), (float*)at.at(flat, m.w[3], 3), x.n, in, H, out, depth, m.act, dt, code_of(m.x.scalar_type()), ptr(ws),
-                   bytes, stream_of(m.x)),
+  const auto grad = [&](int i) { return (float*)at.at(flat, m.w[i], i); };
+  if (written) {
+    const auto f = [](const void* p) { return (const float*)p; };
+    check(nf_mlp_bwd_f32(f(x.p), x.stride, f(g.p), g.stride, (float*)ptr(dx), in, f(ptr(m.w[0])), f(ptr(m.w[1])), f(ptr(m.w[4])), f(ptr(m.w[5])),
+                         f(ptr(m.w[2])), f(ptr(m.w[3])), grad(0), grad(1), grad(4), grad(5), grad(2), grad(3), x.n, in, H, out, depth, m.act, ptr(ws),
+                         bytes, stream_of(m.x)),
+          "nf_mlp_bwd_f32");
+    return finish(at, flat);
+  }
+  check(nf_mlp_bwd(x.p, x.stride, g.p, g.stride, ptr(dx), in, ptr(m.w[0]), ptr(m.w[1]), ptr(m.w[4]), ptr(m.w[5]), ptr(m.w[2]), ptr(m.w[3]), grad(0),
+                   grad(1), grad(4), grad(5), grad(2), grad(3), x.n, in, H, out, depth, m.act, dt, code_of(m.x.scalar_type()), ptr(ws), bytes,
+                   stream_of(m.x)),
         "nf_mlp_bwd");
   // float32 accumulators, rounded once to the parameters' dtype (one kernel for all of them)
   return finish(at, float_grads || wt == at::kFloat ? flat : flat.to(wt));

@@ -30,3 +30,26 @@ def test_matrices_off_their_alignment_give_the_same_bits(d_in, d_out, dtype, bia
 
     for a, b in zip(grads(0), grads(1)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("half,blocks,rows", [(64, 1, 33), (64, 3, 64), (64, 5, 4096), (32, 4, 96), (32, 7, 4100), (16, 2, 64)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_couplings_off_their_alignment_give_the_same_bits(half, blocks, rows, bias):
+    """Reversible weights on 16-byte, 8-byte and odd addresses, full and padded widths, a last group and a last pass of fewer couplings."""
+    from triton_helpers_amd.layers.reversible_mlp import reversible_mlp
+
+    torch.manual_seed(half + blocks)
+    u = lambda *s: ((torch.rand(*s, device=DEV) * 2 - 1) / half**0.5).bfloat16()  # noqa: E731
+    w = [u(2 * blocks * half, half), u(2 * blocks, half) if bias else None, u(2 * blocks * half, half), u(2 * blocks, half) if bias else None]
+    x, dy = torch.randn(rows, 2 * half, device=DEV).bfloat16(), torch.randn(rows, 2 * half, device=DEV).bfloat16()
+
+    def run(shift):
+        leaves = [x.clone().requires_grad_()] + [None if t is None else torch.empty(t.numel() + 8, dtype=t.dtype, device=DEV)[shift : shift + t.numel()].view(t.shape).copy_(t).detach().requires_grad_() for t in w]
+        y = reversible_mlp(*leaves, activation="gelu")
+        y.backward(dy)
+        return [y.detach()] + [t.grad for t in leaves if t is not None]
+
+    want = run(0)
+    for shift in (1, 4):
+        for a, b in zip(want, run(shift)):
+            assert torch.equal(a, b)

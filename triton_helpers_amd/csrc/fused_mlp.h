@@ -51,13 +51,6 @@ __device__ __forceinline__ void stage_bias(float* dst, const uint16_t* b, int n_
   for (int i = tid; i < n_pad; i += nthreads) dst[i] = (b != nullptr && i < n_valid) ? T::to_f32(b[i]) : 0.0f;
 }
 
-// Features 8q .. 8q + 7 of a 32-feature chunk of row m into a fragment in chain order: the half q / 2 of lane groups 2 (q % 2) and the one behind it.
-__device__ __forceinline__ void put_chain(uint16_t* frag, int m, int q, uint4 v) {
-  uint16_t* half = frag + (m + 32 * (q & 1)) * 8 + 4 * (q >> 1);
-  *reinterpret_cast<uint2*>(half) = make_uint2(v.x, v.y);
-  *reinterpret_cast<uint2*>(half + 16 * 8) = make_uint2(v.z, v.w);
-}
-
 // All weights of a network into LDS as A fragments, [w_in | w_hid | w_out], and its biases behind them.  The layers are one list of
 // fragments, several to a wave under way together, and the biases are asked for first: layer by layer, every matrix and every bias waited for the
 // one in front.  Rows move in 16-byte pieces, which are the order of the first layer's products and two halves of a fragment each in

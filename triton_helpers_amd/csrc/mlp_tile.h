@@ -469,4 +469,11 @@ inline bool vec_store_ok(const void* p, int64_t stride_elems, int width) {
   return ((uintptr_t)p % 8 == 0) && (stride_elems % 4 == 0) && (width % 4 == 0);
 }
 
+// Features 8q .. 8q + 7 of a 32-feature chunk of row m into a fragment in chain order: the half q / 2 of lane groups 2 (q % 2) and the one behind it.
+__device__ __forceinline__ void put_chain(uint16_t* frag, int m, int q, uint4 v) {
+  uint16_t* half = frag + (m + 32 * (q & 1)) * 8 + 4 * (q >> 1);
+  *reinterpret_cast<uint2*>(half) = make_uint2(v.x, v.y);
+  *reinterpret_cast<uint2*>(half + 16 * 8) = make_uint2(v.z, v.w);
+}
+
 }  // namespace nf

@@ -146,35 +146,59 @@ __global__ __launch_bounds__(768) void rev_fwd_k(RevArgs a) {
   float* bias = reinterpret_cast<float*>(frags + (size_t)a.nblocks * 4 * LAYER);  // [nblocks][4][HP]
   const int H = FAST ? HP : a.half;
   if constexpr (FAST) {
-    // All layers as one list of 8-element pieces, several in flight per thread: layer by layer, sixteen rounds of loads waited for one
-    // another (1600 rows of four couplings: 32 us, now 21).
-    constexpr int PIECES = MT * KC * 64, AT_ONCE = 4;
+    // The biases are asked for first, then all layers as one list of 16-byte pieces, several in flight per thread: half as many
+    // accesses as 8-byte ones, a clock each.  (Layer by layer sixteen rounds of loads waited for one another, and so did the biases, row by row.
+    // Four GELU couplings, us, layer by layer / 8-byte pieces and bias rows / this: 1600 rows 32 / 21 / 16; 4096 rows 21.5 / 16.6 for the last two, 2^16
+    // 35.5 / 26.5, 2^18 77 / 68.5; 32-wide 4096 rows 10.4 / 8.2.)
+    const int n_bias = a.nblocks * 4 * HP;
+    const auto bias_at = [&](int i) {  // [coupling][F.b1, F.b2, G.b1, G.b2][HP]
+      const uint16_t* b = i / HP & 1 ? a.b2 : a.b1;
+      return b != nullptr ? b + (size_t)(i / (2 * HP)) * HP + i % HP : a.w1;
+    };
+    const auto has_bias = [&](int i) { return (i / HP & 1 ? a.b2 : a.b1) != nullptr; };
+    const int second = tid + nthreads;
+    const uint16_t b0 = *bias_at(tid < n_bias ? tid : 0), b1 = *bias_at(second < n_bias ? second : 0);
+    constexpr int PIECES = MT * KC * 64, AT_ONCE = 6;
     const int all = a.nblocks * 4 * PIECES;
-    for (int u0 = tid; u0 < all; u0 += AT_ONCE * nthreads) {
-      uint2 lo[AT_ONCE], hi[AT_ONCE];
+    auto stage = [&](auto wide_c) {
+      for (int u0 = tid; u0 < all; u0 += AT_ONCE * nthreads) {
+        uint4 v[AT_ONCE];
 #pragma unroll
-      for (int i = 0; i < AT_ONCE; ++i) {
-        const int u = u0 + i * nthreads < all ? u0 + i * nthreads : u0;
-        const int layer = u / PIECES, piece = u % PIECES, mt = (piece >> 6) / KC, kc = (piece >> 6) % KC, g = (piece & 63) >> 4;
-        const uint16_t* w = (layer & 1 ? a.w2 : a.w1) + (size_t)(layer >> 1) * HP * HP + (16 * mt + (piece & 15)) * HP;
-        lo[i] = *reinterpret_cast<const uint2*>(w + k_chain(kc, g, 0));
-        hi[i] = *reinterpret_cast<const uint2*>(w + k_chain(kc, g, 4));
+        for (int i = 0; i < AT_ONCE; ++i) {
+          const int u = u0 + i * nthreads;
+          if (u - lane >= all) break;  // (the same for the whole wave: a matrix is whole waves' pieces)
+          const int layer = u / PIECES, piece = u % PIECES, mt = (piece >> 6) / KC, kc = (piece >> 6) % KC;
+          const uint16_t* w = (layer & 1 ? a.w2 : a.w1) + (size_t)(layer >> 1) * HP * HP + (16 * mt + (lane & 15)) * HP + 32 * kc + 8 * (lane >> 4);
+          if constexpr (decltype(wide_c)::value) {
+            v[i] = *reinterpret_cast<const uint4*>(w);
+          } else {
+            const uint2 lo = *reinterpret_cast<const uint2*>(w), hi = *reinterpret_cast<const uint2*>(w + 4);
+            v[i] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i) {
+          const int u = u0 + i * nthreads;
+          if (u - lane >= all) break;
+          put_chain(frags + (size_t)(u - lane) * 8, lane & 15, lane >> 4, v[i]);
+        }
       }
-#pragma unroll
-      for (int i = 0; i < AT_ONCE; ++i)
-        if (u0 + i * nthreads < all) *reinterpret_cast<uint4*>(frags + (size_t)(u0 + i * nthreads) * 8) = make_uint4(lo[i].x, lo[i].y, hi[i].x, hi[i].y);
-    }
-  }
-  for (int k = 0; k < a.nblocks; ++k)
-    for (int s = 0; s < 2; ++s) {
-      const size_t sub = (size_t)(2 * k + s);
-      if constexpr (!FAST) {
+    };
+    if (((uintptr_t)a.w1 | (uintptr_t)a.w2) % 16 == 0) stage(std::true_type{});
+    else stage(std::false_type{});
+    if (tid < n_bias) bias[tid] = has_bias(tid) ? T::to_f32(b0) : 0.0f;
+    if (second < n_bias) bias[second] = has_bias(second) ? T::to_f32(b1) : 0.0f;
+    for (int i = second + nthreads; i < n_bias; i += nthreads) bias[i] = has_bias(i) ? T::to_f32(*bias_at(i)) : 0.0f;
+  } else {
+    for (int k = 0; k < a.nblocks; ++k)
+      for (int s = 0; s < 2; ++s) {
+        const size_t sub = (size_t)(2 * k + s);
         stage_weight_frags<true, false>(frags + ((size_t)k * 4 + 2 * s) * LAYER, a.w1 + sub * H * H, H, H, MT, KC, tid, nthreads);
         stage_weight_frags<true, false>(frags + ((size_t)k * 4 + 2 * s + 1) * LAYER, a.w2 + sub * H * H, H, H, MT, KC, tid, nthreads);
+        stage_bias_row<T>(bias + ((size_t)k * 4 + 2 * s) * HP, a.b1 ? a.b1 + sub * H : nullptr, H, HP, tid, nthreads);
+        stage_bias_row<T>(bias + ((size_t)k * 4 + 2 * s + 1) * HP, a.b2 ? a.b2 + sub * H : nullptr, H, HP, tid, nthreads);
       }
-      stage_bias_row<T>(bias + ((size_t)k * 4 + 2 * s) * HP, a.b1 ? a.b1 + sub * H : nullptr, H, HP, tid, nthreads);
-      stage_bias_row<T>(bias + ((size_t)k * 4 + 2 * s + 1) * HP, a.b2 ? a.b2 + sub * H : nullptr, H, HP, tid, nthreads);
-    }
+  }
   __syncthreads();
 
   const int64_t n_chunks = (a.rows + 31) / 32;

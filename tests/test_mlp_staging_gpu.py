@@ -53,3 +53,27 @@ def test_couplings_off_their_alignment_give_the_same_bits(half, blocks, rows, bi
     for shift in (1, 4):
         for a, b in zip(want, run(shift)):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("rows", [1, 1000, 40001])
+@pytest.mark.parametrize("d_in,hidden,d_out,depth,act", [(32, 64, 16, 2, "relu"), (64, 64, 64, 9, "relu"), (8, 32, 33, 5, "relu"), (24, 16, 3, 1, "silu"), (40, 64, 64, 3, "silu"), (56, 32, 64, 9, "relu2")])
+def test_whole_backward_off_its_alignment_gives_the_same_bits(rows, d_in, hidden, d_out, depth, act):
+    """The list of 16-byte pieces against the matrices one by one: padded rows and columns of every matrix, the fewest and the most layers."""
+    from triton_helpers_amd.layers.fully_fused_mlp import fully_fused_mlp
+
+    torch.manual_seed(rows + d_in)
+    u = lambda *s: ((torch.rand(*s, device=DEV) * 2 - 1) / s[-1] ** 0.5).half()  # noqa: E731
+    w = {"w_in": u(hidden, d_in), "b_in": u(hidden), "w_out": u(d_out, hidden), "b_out": u(d_out)}
+    if depth > 1:
+        w.update(w_hid=u((depth - 1) * hidden, hidden), b_hid=u(depth - 1, hidden))
+    x, dy = torch.randn(1, rows, d_in, device=DEV).half(), torch.randn(1, rows, d_out, device=DEV).half()
+
+    def grads(shift):
+        leaves = {"x": x.clone().requires_grad_()}
+        for k, t in w.items():
+            leaves[k] = torch.empty(t.numel() + 8, dtype=t.dtype, device=DEV)[shift : shift + t.numel()].view(t.shape).copy_(t).detach().requires_grad_()
+        fully_fused_mlp(activation=act, **{"w_hid": None, "b_hid": None, **leaves}).backward(dy)
+        return [t.grad for t in leaves.values()]
+
+    for a, b in zip(grads(0), grads(4)):
+        assert torch.equal(a, b)

@@ -83,6 +83,55 @@ __device__ __forceinline__ void stage_rows(char* dst, const uint16_t* w, int lay
   }
 }
 
+// All matrices and hidden biases of a network as one list of 16-byte pieces, laid out as stage_rows() does, with several of a thread's under way
+// together and first_rows(), which asks for the wave's first rows, behind them.  The biases are asked for first.  Matrix by matrix in 8-byte pieces, a
+// clock each for the L1, each waited for the one in front and all for the rows (us with the sum of the gradients, before / this: 32 -> 64 -> 64 -> 16
+// 1000 rows 9.8 / 9.2, 2^16 19.5 / 18.7; 64 -> 64 x 8 -> 64, 2^16 51 / 47.6; three layers of SiLU, 2^18 69.2 / 67.1).
+template <typename T, int HP, int N, typename FirstRows>
+__device__ __forceinline__ void stage_pieces(char* dst, float* bias, const MlpArgs& a, int tid, FirstRows first_rows) {
+  constexpr int AT_ONCE = 6, HP_LOG2 = HP == 32 ? 5 : 6;
+  const int lane = tid & 63, first = __builtin_amdgcn_readfirstlane(tid - lane), H = a.d_hidden, units = (a.depth * HP + 64) * 8;
+  const auto bias_at = [&](int i, bool& there) {
+    const int l = i >> 6, f = i & 63;
+    const uint16_t* b = l == 0 ? a.b_in : a.b_hid != nullptr ? a.b_hid + (size_t)(l - 1) * H : nullptr;
+    there = b != nullptr && f < H;
+    return there ? b + f : a.w_in;
+  };
+  bool there;
+  const uint16_t b0 = *bias_at(tid < a.depth * 64 ? tid : 0, there);
+  for (int u0 = first; u0 < units || u0 == first; u0 += N * AT_ONCE) {  // (a wave's pieces are eight rows of one matrix)
+    uint4 v[AT_ONCE];
+    bool inside[AT_ONCE];
+#pragma unroll
+    for (int i = 0; i < AT_ONCE; ++i) {
+      const int u = u0 + i * N;
+      if (u >= units) break;
+      const int row = (u >> 3) + (lane >> 3), c = 8 * (lane & 7), l = u >> (3 + HP_LOG2);  // l == depth and on: the output's 64 rows
+      const bool out = l >= a.depth;
+      const int r = out ? row - a.depth * HP : row & (HP - 1), nr = out ? a.d_out : H, nc = l == 0 ? a.d_in : H;
+      const uint16_t* w = out ? a.w_out : l == 0 ? a.w_in : a.w_hid + (size_t)(l - 1) * H * H;
+      inside[i] = r < nr && c < nc;
+      v[i] = *reinterpret_cast<const uint4*>(w + (r < nr ? r : 0) * nc + (c < nc ? c : 0));
+    }
+    if (u0 == first) first_rows();
+#pragma unroll
+    for (int i = 0; i < AT_ONCE; ++i) {
+      const int u = u0 + i * N;
+      if (u >= units) break;
+      const int row = (u >> 3) + (lane >> 3);
+      if (!inside[i]) v[i] = make_uint4(0u, 0u, 0u, 0u);
+      char* d = dst + row * ROLES_PITCH;
+      *reinterpret_cast<uint2*>(d + (((2 * (lane & 7)) ^ swizzle(row)) << 3)) = make_uint2(v[i].x, v[i].y);
+      *reinterpret_cast<uint2*>(d + (((2 * (lane & 7) + 1) ^ swizzle(row)) << 3)) = make_uint2(v[i].z, v[i].w);
+    }
+  }
+  if (tid < a.depth * 64) bias[tid] = there ? T::to_f32(b0) : 0.0f;
+  for (int i = tid + N; i < a.depth * 64; i += N) {
+    const uint16_t b = *bias_at(i, there);
+    bias[i] = there ? T::to_f32(b) : 0.0f;
+  }
+}
+
 // The launch's arguments, read again where they are used (see opaque()).
 typedef const MlpArgs __attribute__((address_space(4))) * ArgsPtr;
 __device__ __forceinline__ ArgsPtr fresh_args() {
@@ -126,14 +175,21 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
       if (kc == 0 || two_out) ndy[kc] = load_row8(k->dy, k->dy_stride, r, k->rows, k->d_out, 32 * kc + 8 * g, k->dy_vec != 0);
     }
   };
-  if (chain) load_rows(row0);
-  stage_rows<THREADS>(w_in, a.w_in, 1, a.d_hidden, HP, a.d_in, tid);
-  if (depth > 1) stage_rows<THREADS>(w_hid, a.w_hid, depth - 1, a.d_hidden, HP, a.d_hidden, tid);
-  stage_rows<THREADS>(w_out, a.w_out, 1, a.d_out, 64, a.d_hidden, tid);
-  for (int i = tid; i < depth * 64; i += THREADS) {
-    const int l = i >> 6, f = i & 63;
-    const uint16_t* b = l == 0 ? a.b_in : a.b_hid != nullptr ? a.b_hid + (size_t)(l - 1) * a.d_hidden : nullptr;
-    bias[i] = b != nullptr && f < a.d_hidden ? T::to_f32(b[f]) : 0.0f;
+  auto first_rows = [&] {
+    if (chain) load_rows(row0);
+  };
+  if (a.d_in % 8 == 0 && a.d_hidden % 8 == 0 && ((uintptr_t)a.w_in | (uintptr_t)a.w_hid | (uintptr_t)a.w_out) % 16 == 0) {
+    stage_pieces<T, HP, THREADS>(w_in, bias, a, tid, first_rows);
+  } else {
+    first_rows();
+    stage_rows<THREADS>(w_in, a.w_in, 1, a.d_hidden, HP, a.d_in, tid);
+    if (depth > 1) stage_rows<THREADS>(w_hid, a.w_hid, depth - 1, a.d_hidden, HP, a.d_hidden, tid);
+    stage_rows<THREADS>(w_out, a.w_out, 1, a.d_out, 64, a.d_hidden, tid);
+    for (int i = tid; i < depth * 64; i += THREADS) {
+      const int l = i >> 6, f = i & 63;
+      const uint16_t* b = l == 0 ? a.b_in : a.b_hid != nullptr ? a.b_hid + (size_t)(l - 1) * a.d_hidden : nullptr;
+      bias[i] = b != nullptr && f < a.d_hidden ? T::to_f32(b[f]) : 0.0f;
+    }
   }
   __syncthreads();
 

@@ -14,9 +14,9 @@
 //
 // What it replaces: one wave per SIMD held a coupling's four gradients next to the chain (512 registers, matrix-core transposes for
 // their operands, both forms of the weights in LDS), issued vector and matrix instructions in turn and moved (y, dy) -> (x, dx) once per
-// coupling: 4.4 GB of 2^20 rows and four couplings.  Four GELU couplings in bfloat16, us: 64-wide, 1000 rows 112 -> 37, 2^16 141 -> 94, 2^18
-// 324 -> 243, 2^20 1110 -> 884; 48-wide (each coupling was a launch) 96 -> 35, 174 -> 88, 461 -> 231, 1712 -> 836; 32-wide 48 -> 19, 54 -> 43,
-// 129 -> 101, 500 -> 365.  What bounds it now: the chain's vector instructions (half of the time, a third of them the activation's) and what a
+// coupling: 4.4 GB of 2^20 rows and four couplings.  Four GELU couplings in bfloat16, us: 64-wide, 1000 rows 112 -> 35, 2^16 141 -> 84, 2^18
+// 324 -> 237, 2^20 1110 -> 865; 48-wide (each coupling was a launch) 96 -> 35, 174 -> 88, 461 -> 231, 1712 -> 836; 32-wide 48 -> 18, 54 -> 43,
+// 129 -> 98, 500 -> 362.  What bounds it now: the chain's vector instructions (half of the time, a third of them the activation's) and what a
 // chain wave waits for between its products, with two of them on a SIMD.
 #include "reversible.h"
 #include "role_split.h"

@@ -752,7 +752,7 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
   typedef typename BinRec<GT>::type Rec;
   // Fixed-point sums, one plane of BIN_ROWS 64-bit cells per feature: the 64 lanes of an add go to random rows of one
   // feature, and with 8-byte cells those spread over all 64 banks (interleaved features would leave them half).
-  extern __shared__ unsigned long long acc_tile[];
+  extern __shared__ __align__(16) unsigned long long acc_tile[];
   uint32_t* list = reinterpret_cast<uint32_t*>(acc_tile + 2 * BIN_ROWS);  // [LIST + LIST_PAD] first word of up to GROUP records in the level | their number << 27
   uint32_t* first_task = list + LIST + LIST_PAD;                          // [SB + 1] first task of a bin | its first slot << 16
   __shared__ uint32_t next_task, wave_sums[2][ACC_WAVES], level_max[NF_MAX_LEVELS];
@@ -769,6 +769,7 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
   const uint32_t first_total = ws.totals[min(tid, NB - 1)], first_max = ws.header->gmax[min(tid, NF_MAX_LEVELS - 1)];
   const int level_base = lane < bp.n_levels ? bp.binbase[lane] : NB;  // of the lane's level
   uint32_t* late = first_task + SB + 1;  // [n_late + 1] heavy bins behind those: bin, its first further share | its first slot << 16
+  static_assert(__alignof__(acc_tile) >= alignof(uint4), "the tile is cleared in 16-byte pieces");
   for (uint32_t i = tid; i < BIN_ROWS; i += ACC_THREADS) reinterpret_cast<uint4*>(acc_tile)[i] = make_uint4(0u, 0u, 0u, 0u);
   if (tid < NF_MAX_LEVELS) level_max[tid] = first_max;
   // The tasks, worked out by every workgroup for itself: one per bin of the leading levels, several for a bin of more than one and a half
@@ -1367,7 +1368,7 @@ __global__ __launch_bounds__(WALK_THREADS) void hash_bwd_walk_k(WalkWs ws, int64
                                                                 int feat, int p) {
   constexpr bool G32 = sizeof(typename BinRec<GT>::type) == 16;
   constexpr int CN = 1 << D, VD = D > 3 ? D : 3;
-  extern __shared__ unsigned long long acc_tile[];  // 2 * BIN_ROWS sums
+  extern __shared__ __align__(16) unsigned long long acc_tile[];  // 2 * BIN_ROWS sums
   __shared__ uint32_t level_max, hit;
   const int tid = threadIdx.x, lane = tid & 63;
   const int np = (feat + 1) / 2, f0 = 2 * p;

@@ -60,19 +60,24 @@ __device__ __forceinline__ void stage_bias(float* dst, const uint16_t* b, int n_
 // first_rows asks for the wave's first rows, behind the first weights: loads come back in order, and rows from HBM in front of the weights held up the
 // barrier (one-hidden-layer ReLU networks over inputs that no cache holds, rows first / weights first: 32 -> 64 -> 64 -> 16, 2^20 rows 23.9 / 19.4 us,
 // 64 -> 64 -> 64 -> 64, 2^18 14.6 / 13.8; eight hidden layers, 2^18 rows 35.3 / 34.5).
-template <typename T, int KIN, int HP, int OUTP, bool LIST, bool IN_CHAIN, typename FirstRows>
+// PIECE: bytes that w_hid and w_out lie on.  16, or 8 (views into a flat buffer): the same list in two pieces of 8 bytes each; a first or, of 8 bytes, a last matrix
+// off those is staged by itself behind the list.  0 (w_hid off 8 bytes, no hidden matrix): layer by layer.  Matrices 8 bytes off, us, layer by layer / as a list: 64 x 10 ReLU
+// 1000 rows 17.1 / 8.7, 2^18 42.6 / 36.6; 32 -> 64 x 3 -> 16 SiLU 1000 7.7 / 5.2, 2^16 9.9 / 8.1; 32 -> 64 -> 64 -> 16 2^18 8.6 / 7.6.  The two lists are
+// chosen between in front of this function: as a choice inside it the loops' wave-uniform branches became masks (32 -> 64 -> 64 -> 16, 2^18 rows 9.2 -> 10.3).
+// NTHREADS: as for stage_weight_frags().
+template <typename T, int KIN, int HP, int OUTP, int PIECE, bool IN_CHAIN, int NTHREADS = 0, typename FirstRows>
 __device__ __forceinline__ void stage_network(uint16_t* frags, float* bias, const MlpArgs& a, int tid, int nthreads, FirstRows first_rows) {
   constexpr int KC_IN = KIN / 32, KC_H = HP / 32, MT_H = HP / 16, MT_O = OUTP / 16, AT_ONCE = 4;
   constexpr int F_IN = MT_H * KC_IN, F_HID = MT_H * KC_H, F_OUT = MT_O * KC_H;
   const int H = a.d_hidden, n_hid = a.depth - 1, hidden = n_hid * F_HID;
-  if (!LIST) {
+  if constexpr (PIECE == 0) {
     first_rows();
-    stage_weight_frags<IN_CHAIN, false>(frags, a.w_in, H, a.d_in, MT_H, KC_IN, tid, nthreads);
+    stage_weight_frags<IN_CHAIN, false, NTHREADS>(frags, a.w_in, H, a.d_in, MT_H, KC_IN, tid, nthreads);
     for (int k = 0; k < n_hid; ++k) {
-      stage_weight_frags<true, false>(frags + (size_t)(F_IN + k * F_HID) * FRAG_ELEMS, a.w_hid + (size_t)k * H * H, H, H, MT_H, KC_H, tid, nthreads);
+      stage_weight_frags<true, false, NTHREADS>(frags + (size_t)(F_IN + k * F_HID) * FRAG_ELEMS, a.w_hid + (size_t)k * H * H, H, H, MT_H, KC_H, tid, nthreads);
       stage_bias<T>(bias + (k + 1) * HP, a.b_hid ? a.b_hid + (size_t)k * H : nullptr, H, HP, tid, nthreads);
     }
-    stage_weight_frags<true, false>(frags + (size_t)(F_IN + hidden) * FRAG_ELEMS, a.w_out, a.d_out, H, MT_O, KC_H, tid, nthreads);
+    stage_weight_frags<true, false, NTHREADS>(frags + (size_t)(F_IN + hidden) * FRAG_ELEMS, a.w_out, a.d_out, H, MT_O, KC_H, tid, nthreads);
     stage_bias<T>(bias, a.b_in, H, HP, tid, nthreads);
     stage_bias<T>(bias + (n_hid + 1) * HP, a.b_out, a.d_out, OUTP, tid, nthreads);
     return;
@@ -87,9 +92,9 @@ __device__ __forceinline__ void stage_network(uint16_t* frags, float* bias, cons
   };
   bool first_valid;
   const uint16_t first_bias = *bias_at(tid < n_bias ? tid : 0, first_valid);
-  const bool in_listed = a.d_in % 8 == 0 && (uintptr_t)a.w_in % 16 == 0;
+  const bool in_listed = a.d_in % 8 == 0 && (uintptr_t)a.w_in % (PIECE == 16 ? 16 : 8) == 0, out_listed = PIECE == 16 || (uintptr_t)a.w_out % 8 == 0;
   const int lane = tid & 63, m = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = nthreads >> 6;
-  const int all = F_IN + hidden + F_OUT;
+  const int all = F_IN + hidden + (out_listed ? F_OUT : 0);
   for (int f0 = (in_listed ? 0 : F_IN) + wave, round = 0; f0 < all || round == 0; f0 += AT_ONCE * nwaves, ++round) {
     uint4 v[AT_ONCE];
     bool there[AT_ONCE];
@@ -103,7 +108,13 @@ __device__ __forceinline__ void stage_network(uint16_t* frags, float* bias, cons
       const int rows = out ? a.d_out : H, cols = in ? a.d_in : H, row = 16 * mt + m, k = 32 * kc + 8 * g;
       const uint16_t* w = in ? a.w_in : out ? a.w_out : a.w_hid + (size_t)layer * H * H;
       there[i] = row < rows && k < cols;
-      v[i] = *reinterpret_cast<const uint4*>(w + __umul24((uint32_t)(row < rows ? row : 0), (uint32_t)cols) + (k < cols ? k : 0));
+      w += __umul24((uint32_t)(row < rows ? row : 0), (uint32_t)cols) + (k < cols ? k : 0);
+      if constexpr (PIECE == 16) {
+        v[i] = *reinterpret_cast<const uint4*>(w);
+      } else {
+        const uint2 lo = *reinterpret_cast<const uint2*>(w), hi = *reinterpret_cast<const uint2*>(w + 4);
+        v[i] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+      }
     }
     if (round == 0) first_rows();
 #pragma unroll
@@ -119,7 +130,8 @@ __device__ __forceinline__ void stage_network(uint16_t* frags, float* bias, cons
       }
     }
   }
-  if (!in_listed) stage_weight_frags<IN_CHAIN, false>(frags, a.w_in, H, a.d_in, MT_H, KC_IN, tid, nthreads);
+  if (!in_listed) stage_weight_frags<IN_CHAIN, false, NTHREADS>(frags, a.w_in, H, a.d_in, MT_H, KC_IN, tid, nthreads);
+  if (!out_listed) stage_weight_frags<true, false, NTHREADS>(frags + (size_t)(F_IN + hidden) * FRAG_ELEMS, a.w_out, a.d_out, H, MT_O, KC_H, tid, nthreads);
   if (tid < n_bias) bias[tid] = first_valid ? T::to_f32(first_bias) : 0.0f;
   for (int i = tid + nthreads; i < n_bias; i += nthreads) {
     bool valid;

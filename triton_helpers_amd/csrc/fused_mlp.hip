@@ -68,7 +68,9 @@ __global__ __launch_bounds__(512) void mlp_fwd_k(MlpArgs a) {
       for (int kc = 0; kc < KC_IN; ++kc)
         nxt[nt][kc] = load_rows_frag(a.x, a.x_stride, first_chunk * ROWS + 16 * nt, a.rows, a.d_in, kc, lane, a.x_vec);
   };
-  stage_network<T, KIN, HP, OUTP, LIST, false>(f_in, bias_in, a, tid, nthreads, first_rows);
+  if constexpr (!LIST) stage_network<T, KIN, HP, OUTP, 0, false>(f_in, bias_in, a, tid, nthreads, first_rows);
+  else if (((uintptr_t)a.w_hid | (uintptr_t)a.w_out) % 16 == 0) stage_network<T, KIN, HP, OUTP, 16, false>(f_in, bias_in, a, tid, nthreads, first_rows);
+  else stage_network<T, KIN, HP, OUTP, 8, false>(f_in, bias_in, a, tid, nthreads, first_rows);
   __syncthreads();
 
   for (int64_t chunk = first_chunk; chunk < n_chunks; chunk += wave_stride) {
@@ -548,7 +550,7 @@ static int launch_fwd(const MlpArgs& a0, hipStream_t s) {
   // long chains of layers, with one (us, layers staged in turn and two groups / two groups / one: 32 -> 64 x 4 -> 16 SiLU 1000 rows 8.5 / 8.3 / 6.0, 65536 12.3 / 11.7 /
   // 10.3, 10^5 18.0 / 17.0 / 13.7, 2^17 18.2 / 17.3 / 15.9; 64 x 10 ReLU 1000 14.3 / 15.3 / 10.6, 2^17 23.8 / 24.3 / 23.3; one hidden layer SiLU
   // 1000 6.6 / 5.6 / 5.2, 65536 7.7 / 7.4 / 7.6).
-  const bool list = n_hid > 0 && ((uintptr_t)a.w_hid | (uintptr_t)a.w_out) % 16 == 0;
+  const bool list = n_hid > 0 && (uintptr_t)a.w_hid % 8 == 0;
   const bool small = list && a.rows <= (n_hid == 1 ? 32768 : HP == 32 ? 65536 : 131072);
   // weights beyond half of LDS leave room for one workgroup per CU: give it eight waves to keep two per SIMD
   a.waves = lds > 76 * 1024 || small ? 8 : 4;

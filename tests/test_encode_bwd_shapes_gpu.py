@@ -55,6 +55,26 @@ def test_accumulation_in_chunks_of_blocks(N, cube, F, T, L, dtype):
     assert torch.equal(got, _grad(x, do, E, F, T, lo, hi, L, flags=16))
 
 
+@pytest.mark.parametrize("N", [16384, 40000, 131071, 262143])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("F", [2, 3])
+def test_shares_of_a_bin_are_rounded_once(N, dtype, F):
+    """Points on 64 corners of the cells of two dense levels: a point's weights are one and zeros, and its gradient a multiple of 2^-18 below 2^8, which the
+    fixed point keeps whole.  Each of the rows gets hundreds of them, in bins that are cut into many shares: its gradient is their exact
+    sum, rounded to float32 once."""
+    torch.manual_seed(N)
+    T, lo, hi, L = 2**19, 16, 64, 2
+    cells = torch.randint(0, 16, (64, 3), device=DEV)[torch.randint(0, 64, (N,), device=DEV)]
+    x = cells / 16.0
+    offsets = O.level_row_offsets(L, T, 3, lo, hi)
+    do = (torch.randint(-127, 128, (N, L * F), device=DEV) * torch.exp2(torch.randint(-18, 2, (N, L * F), device=DEV).float())).to(dtype)
+    rows = O.encode_indices(x.cpu(), None, T, L, lo, hi)[:, :, 0].to(DEV)  # of the corner with all the weight
+    want = torch.zeros(offsets[-1], F, dtype=torch.float64, device=DEV)
+    for l in range(L):
+        want.index_add_(0, offsets[l] + rows[:, l], do[:, l * F : (l + 1) * F].double())
+    assert torch.equal(_grad(x, do, offsets[-1], F, T, lo, hi, L, flags=16), want.float())
+
+
 # rows of one piece of 16 bytes, of four, of eight, of numbers between them and of more; blocks of points and chunks that are short, whole and one over
 @pytest.mark.parametrize("N", [8192, 8193, 8447, 8449, 9215, 9216, 9999])
 @pytest.mark.parametrize("L,F,dtype", [(4, 2, torch.float16), (16, 2, torch.bfloat16), (10, 4, torch.float16), (6, 8, torch.float16), (9, 8, torch.bfloat16),

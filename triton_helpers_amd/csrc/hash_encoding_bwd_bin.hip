@@ -98,7 +98,7 @@ struct BinHeader {  // cleared by the fill kernel's first workgroup for the kern
   uint32_t gmax[NF_MAX_LEVELS];  // largest |dout| bit pattern of every level
 };
 
-// A bin cut into several tasks, each summing into a slot (of BIN_ROWS rows of two floats) of its own.
+// A bin cut into several tasks, each leaving its sums in a slot (of BIN_ROWS rows of two) of its own.
 struct BinSplit {
   uint32_t bin, slot, n, pad;
 };
@@ -109,10 +109,10 @@ struct BinWs {
   uint32_t* block_max;  // [levels][blocks] largest |dout| bit pattern
   BinSplit* splits;
   uint16_t* starts;     // [blocks][start_stride]: place of every bin inside the block, one more per level for its end
-  float* slots;
+  void* slots;          // of 64-bit fixed point (`whole_slots`) or of floats
   uint32_t* records;    // 3 words per record (16-bit gradient) or 4 (float32 gradient)
   uint32_t max_slots, split_cost;
-  int start_stride, blocks;
+  int start_stride, blocks, whole_slots;
 };
 
 // record = {row0 | row1 << 13 | w1[18:13] << 26,  w0 | w1[12:0] << 19,  packed gradient pair}
@@ -696,6 +696,29 @@ __device__ __forceinline__ int32_t round_to_int(float x) {
   return r;
 }
 
+// Fixed-point scale 2^se of a level whose largest |gradient| is gm:  |w * g| * 2^se < 2^30.  A level with an inf or a nan has none.
+struct FixedPoint {
+  int se;
+  bool nonfinite;
+  __device__ __forceinline__ explicit FixedPoint(float gm) : se(0), nonfinite(!(gm <= 3.0e38f)) {
+    if (nonfinite || !(gm > 0.0f)) return;
+    int ex;
+    frexpf(gm, &ex);
+    se = 30 - ex;
+    se = se > 120 ? 120 : se;
+  }
+  // A sum a of these: |a| <= 2^30 * 2^21 points < 2^53, exact in double, and so is its quotient by 2^se: one rounding, to float, at the end
+  struct ToFloat {
+    double lo, hi;
+    bool nonfinite;
+    __device__ __forceinline__ float operator()(long long a) const {
+      const float x = (float)((double)(int)(a >> 32) * hi + (double)(uint32_t)a * lo);
+      return nonfinite && a != 0 ? __uint_as_float(0x7fc00000u) : x;
+    }
+  };
+  __device__ __forceinline__ ToFloat to_float() const { return {ldexp(1.0, -se), ldexp(1.0, 32 - se), nonfinite}; }
+};
+
 // How a sum reaches the gradient table.
 enum TableMode { TABLE_ADD = 0, TABLE_F32 = 1, TABLE_F16 = 2, TABLE_BF16 = 3 };  // added to float32, or written in a type of its own
 template <int MODE>
@@ -972,17 +995,9 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
   for (;;) {
     const Task& task = now.task;
     const int l = task.level;
-    // fixed-point scale 2^se of the level:  |w * g| * 2^se < 2^30
-    const float gm = BinRec<GT>::level_max(level_max[l]);
-    const bool nonfinite = !(gm <= 3.0e38f);
-    int se = 0;
-    if (!nonfinite && gm > 0.0f) {
-      int ex;
-      frexpf(gm, &ex);  // gm = f * 2^ex, f in [0.5, 1)
-      se = 30 - ex;
-      se = se > 120 ? 120 : se < -120 ? -120 : se;
-    }
-    const float scale = nonfinite ? 0.0f : ldexpf(1.0f, se);  // |g| * 2^se < 2^30, and |se| stays inside float's exponents
+    const FixedPoint fixed(BinRec<GT>::level_max(level_max[l]));
+    const bool nonfinite = fixed.nonfinite;
+    const float scale = nonfinite ? 0.0f : ldexpf(1.0f, fixed.se);  // |g| * 2^se < 2^30, and |se| stays inside float's exponents
     const float scale_w = scale * (1.0f / (float)W_MAX);      // with the decoding of the pair records' weights
     const __amdgpu_buffer_rsrc_t rs = records_of(l);
     // a lane without a record, and a record without a gradient, add nothing
@@ -1106,78 +1121,83 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
     const uint32_t left = g.rows[l] - row0;
     const uint32_t nrows = left < (uint32_t)BIN_ROWS ? left : (uint32_t)BIN_ROWS;
     // the tile to the table (or the task's slot), and back to zero for the next task
-    const float qnan = __uint_as_float(0x7fc00000u);
     const int64_t first = (g.row_offset[l] + (int64_t)row0) * feat + f0;  // features f0, f0 + 1 of the bin's rows
-    // |a| <= 2^30 * 2^21 points < 2^53, exact in double, and so is its quotient by 2^se: one rounding, to float, at the end
-    const double unscale = ldexp(1.0, -se), unscale_hi = ldexp(1.0, 32 - se);
-    auto value = [&](uint32_t i) {
+    const FixedPoint::ToFloat to_float = fixed.to_float();
+    auto take = [&](uint32_t i) {
       const long long a = (long long)acc_tile[i];
       acc_tile[i] = 0ull;
-      const float x = (float)((double)(int)(a >> 32) * unscale_hi + (double)(uint32_t)a * unscale);
-      return nonfinite && a != 0 ? qnan : x;
+      return a;
     };
     constexpr int U = MODE == TABLE_ADD ? 4 : 8;  // rows of a thread that are under way together
-    for (uint32_t r0 = tid; r0 < nrows; r0 += ACC_THREADS * U) {
+    if (task.slot != ~0u) {
+      if (ws.whole_slots) {
+        longlong2* dst = reinterpret_cast<longlong2*>(ws.slots) + (int64_t)task.slot * BIN_ROWS;
+#pragma unroll 4
+        for (uint32_t r = tid; r < nrows; r += ACC_THREADS) {
+          const long long x = take(r), y = take(BIN_ROWS + r);
+          dst[r] = make_longlong2(x, y);
+        }
+      } else {
+        float2* dst = reinterpret_cast<float2*>(ws.slots) + (int64_t)task.slot * BIN_ROWS;
+#pragma unroll 4
+        for (uint32_t r = tid; r < nrows; r += ACC_THREADS) {
+          const float x = to_float(take(r)), y = to_float(take(BIN_ROWS + r));
+          dst[r] = make_float2(x, y);
+        }
+      }
+    } else for (uint32_t r0 = tid; r0 < nrows; r0 += ACC_THREADS * U) {
       float x[U], y[U];
       float2 old[MODE == TABLE_ADD ? U : 1];
       // Added: the old values of all these rows are asked for before any is needed (rows of an even number of features pair by pair).  One
       // read and write after another for rows of other than two features: F = 4, 10^5 points 285 us, this 266; F = 8 774 and 715.  (With
       // one, two or eight rows under way the same within 1 %; asked for in front of the records' adds slower, 300 us: what is left
       // is the traffic of rows half used per pass, all units writing back at once.)
-      if constexpr (MODE == TABLE_ADD)
-        if (task.slot == ~0u) {
-          const float* src = reinterpret_cast<const float*>(table) + first;
-          if constexpr (TWO) {
+      if constexpr (MODE == TABLE_ADD) {
+        const float* src = reinterpret_cast<const float*>(table) + first;
+        if constexpr (TWO) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) old[u] = reinterpret_cast<const float2*>(src)[min(r0 + u * ACC_THREADS, nrows - 1u)];
-          } else if ((feat & 1) == 0) {
+          for (int u = 0; u < U; ++u) old[u] = reinterpret_cast<const float2*>(src)[min(r0 + u * ACC_THREADS, nrows - 1u)];
+        } else if ((feat & 1) == 0) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) old[u] = *reinterpret_cast<const float2*>(src + (int64_t)min(r0 + u * ACC_THREADS, nrows - 1u) * feat);
-          } else {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-              const float* cell = src + (int64_t)min(r0 + u * ACC_THREADS, nrows - 1u) * feat;
-              old[u] = make_float2(cell[0], has_pair ? cell[1] : 0.0f);
-            }
-          }
-        }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint32_t r = r0 + u * ACC_THREADS;
-        x[u] = r < nrows ? value(r) : 0.0f;
-        y[u] = r < nrows ? value(BIN_ROWS + r) : 0.0f;
-      }
-      if (task.slot != ~0u) {
-        float2* dst = reinterpret_cast<float2*>(ws.slots + (int64_t)task.slot * (2 * BIN_ROWS));
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          if (r0 + u * ACC_THREADS < nrows) dst[r0 + u * ACC_THREADS] = make_float2(x[u], y[u]);
-      } else {
-        if constexpr (MODE == TABLE_ADD) {
-          float* dst = reinterpret_cast<float*>(table) + first;
-          if constexpr (TWO) {
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-              if (x[u] != 0.0f || y[u] != 0.0f) reinterpret_cast<float2*>(dst)[r0 + u * ACC_THREADS] = make_float2(old[u].x + x[u], old[u].y + y[u]);
-          } else if ((feat & 1) == 0) {
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-              if (x[u] != 0.0f || y[u] != 0.0f)
-                *reinterpret_cast<float2*>(dst + (int64_t)(r0 + u * ACC_THREADS) * feat) = make_float2(old[u].x + x[u], old[u].y + y[u]);
-          } else {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-              float* cell = dst + (int64_t)(r0 + u * ACC_THREADS) * feat;
-              if (x[u] != 0.0f) cell[0] = old[u].x + x[u];
-              if (has_pair && y[u] != 0.0f) cell[1] = old[u].y + y[u];
-            }
-          }
+          for (int u = 0; u < U; ++u) old[u] = *reinterpret_cast<const float2*>(src + (int64_t)min(r0 + u * ACC_THREADS, nrows - 1u) * feat);
         } else {
 #pragma unroll
           for (int u = 0; u < U; ++u) {
-            const uint32_t r = r0 + u * ACC_THREADS;
-            if (r < nrows) store_pair<MODE>(table, first + (int64_t)r * feat, x[u], y[u], TWO, has_pair);
+            const float* cell = src + (int64_t)min(r0 + u * ACC_THREADS, nrows - 1u) * feat;
+            old[u] = make_float2(cell[0], has_pair ? cell[1] : 0.0f);
           }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t r = r0 + u * ACC_THREADS;
+        x[u] = r < nrows ? to_float(take(r)) : 0.0f;
+        y[u] = r < nrows ? to_float(take(BIN_ROWS + r)) : 0.0f;
+      }
+      if constexpr (MODE == TABLE_ADD) {
+        float* dst = reinterpret_cast<float*>(table) + first;
+        if constexpr (TWO) {
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            if (x[u] != 0.0f || y[u] != 0.0f) reinterpret_cast<float2*>(dst)[r0 + u * ACC_THREADS] = make_float2(old[u].x + x[u], old[u].y + y[u]);
+        } else if ((feat & 1) == 0) {
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            if (x[u] != 0.0f || y[u] != 0.0f)
+              *reinterpret_cast<float2*>(dst + (int64_t)(r0 + u * ACC_THREADS) * feat) = make_float2(old[u].x + x[u], old[u].y + y[u]);
+        } else {
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            float* cell = dst + (int64_t)(r0 + u * ACC_THREADS) * feat;
+            if (x[u] != 0.0f) cell[0] = old[u].x + x[u];
+            if (has_pair && y[u] != 0.0f) cell[1] = old[u].y + y[u];
+          }
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const uint32_t r = r0 + u * ACC_THREADS;
+          if (r < nrows) store_pair<MODE>(table, first + (int64_t)r * feat, x[u], y[u], TWO, has_pair);
         }
       }
     }
@@ -1189,11 +1209,11 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
 }
 
 // ---------------------------------------------------------------------------------------
-// reduce: the slots of a bin with several tasks, in the order of the tasks
+// reduce: the slots of a bin with several tasks
 // ---------------------------------------------------------------------------------------
 constexpr int REDUCE_THREADS = 256, REDUCE_VALUES = 256;
 template <int MODE>
-__global__ __launch_bounds__(REDUCE_THREADS) void hash_bwd_bin_reduce_k(BinWs ws, void* table, DevGeom g, BinPlan bp, int feat, int f0) {
+__global__ __launch_bounds__(REDUCE_THREADS) void hash_bwd_bin_reduce_k(BinWs ws, void* table, DevGeom g, BinPlan bp, int feat, int f0, int ddt) {
   if (blockIdx.y >= ws.header->n_splits) return;
   const BinSplit sp = ws.splits[blockIdx.y];
   int l = 0;
@@ -1201,11 +1221,17 @@ __global__ __launch_bounds__(REDUCE_THREADS) void hash_bwd_bin_reduce_k(BinWs ws
   const uint32_t row0 = (sp.bin - (uint32_t)bp.binbase[l]) << BIN_ROWS_LOG2;
   const uint32_t left = g.rows[l] - row0, nvals = 2u * (left < (uint32_t)BIN_ROWS ? left : (uint32_t)BIN_ROWS);
   const int64_t first = (g.row_offset[l] + (int64_t)row0) * feat + f0;
-  const float* src = ws.slots + (int64_t)sp.slot * (2 * BIN_ROWS);
-  for (uint32_t i = blockIdx.x * REDUCE_VALUES + threadIdx.x; i < min(nvals, (blockIdx.x + 1u) * REDUCE_VALUES); i += REDUCE_THREADS) {
-    float x = 0.0f;
+  const uint32_t pattern = ws.header->gmax[l];
+  const FixedPoint::ToFloat to_float = FixedPoint(ddt == NF_F32 ? BinRec<F32>::level_max(pattern) : ddt == NF_F16 ? BinRec<F16>::level_max(pattern) : BinRec<BF16>::level_max(pattern)).to_float();
+  const auto total = [&](auto* slots, uint32_t i) {
+    const auto* src = slots + (int64_t)sp.slot * (2 * BIN_ROWS) + i;
+    std::remove_reference_t<decltype(*slots)> sum = 0;
 #pragma unroll 8
-    for (uint32_t k = 0; k < sp.n; ++k) x += src[(int64_t)k * (2 * BIN_ROWS) + i];
+    for (uint32_t k = 0; k < sp.n; ++k) sum += src[(int64_t)k * (2 * BIN_ROWS)];
+    return sum;
+  };
+  for (uint32_t i = blockIdx.x * REDUCE_VALUES + threadIdx.x; i < min(nvals, (blockIdx.x + 1u) * REDUCE_VALUES); i += REDUCE_THREADS) {
+    const float x = ws.whole_slots ? to_float(total(reinterpret_cast<long long*>(ws.slots), i)) : total(reinterpret_cast<float*>(ws.slots), i);
     if ((i & 1u) && f0 + 1 >= feat) continue;
     const int64_t to = first + (int64_t)(i >> 1) * feat + (i & 1u);
     if constexpr (MODE == TABLE_ADD) {
@@ -1596,8 +1622,12 @@ static bool wide_blocks(int64_t n_points, const nf_hash_geom* geom) {
 // Cost (x-pair records) of a share of a split bin: a third of what a compute unit gets of them on every level, and no less than pays for the
 // slot that the share is summed in.  16 levels of 2^19 rows, fp16, whole backward (us), least share 8192 / 16384 / 32768: along rays 2^14 points
 // 52 / 60 / 73, 2^16 76 / 73 / 88, 2^17 91 / 87 / 97; uniform 2^18 115 / 115 / 111, added to float32 129 / 128 / 124.
+// Shares of fewer than SPLIT_FLOAT_COST records leave their sums as they are, in 64-bit fixed point: a bin of that many records that was one task,
+// rounded once, is several then, and float sums of their floats would be rounded for each (2.5e-8 -> 5e-8 of a row at four shares).  The slots
+// are twice as large, 1 us of the chain at 2^17 points along rays; in the larger batches, cut no finer, it would be 3 to 7 us.
+constexpr int64_t SPLIT_FLOAT_COST = 32768;
 static int64_t split_cost(int64_t N, int levels) {
-  const int64_t third = N * levels / 192, small = N < 32768 ? 8192 : N < 65536 ? N / 4 : 16384, large = N < 262144 ? N / 8 : 32768;
+  const int64_t third = N * levels / 192, small = N < 32768 ? 8192 : N < 65536 ? N / 4 : 16384, large = N < 262144 ? N / 8 : SPLIT_FLOAT_COST;
   const int64_t least = small > large ? small : large;
   return third > least ? third : least;
 }
@@ -1616,12 +1646,13 @@ static int64_t bin_ws(void* workspace, const BinPlan& bp, int64_t N, int points,
   ws->start_stride = (NB + bp.n_levels + 1) & ~1;
   ws->split_cost = (uint32_t)split_cost(N, bp.n_levels);
   ws->max_slots = (uint32_t)(16 + N / 1024);
+  ws->whole_slots = ws->split_cost < SPLIT_FLOAT_COST;
   ws->header = (BinHeader*)take(sizeof(BinHeader) + NB * 4);
   ws->totals = (uint32_t*)(ws->header + 1);
   ws->block_max = (uint32_t*)take(blocks * NF_MAX_LEVELS * 4);
   ws->splits = (BinSplit*)take((int64_t)ws->max_slots * sizeof(BinSplit));
   ws->starts = (uint16_t*)take(blocks * ws->start_stride * 2);
-  ws->slots = (float*)take((int64_t)ws->max_slots * 2 * BIN_ROWS * 4);
+  ws->slots = take((int64_t)ws->max_slots * 2 * BIN_ROWS * (ws->whole_slots ? 8 : 4));
   ws->records = (uint32_t*)take((int64_t)rec_words * R * 4);
   return o;
 }
@@ -1881,8 +1912,9 @@ static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_
       if (int rc = launch("hash_bwd_bin_totals", (const void*)hash_bwd_bin_totals_k, dim3((unsigned)bin_pieces, pieces), 64 * TOTALS_WAVES, totals_args, 0)) return rc;
       void* acc_args[] = {(void*)&ws, (void*)&table, (void*)&gg, (void*)&bp, (void*)&feat, (void*)&f0};
       if (int rc = launch("hash_bwd_bin_accum", accum, dim3(units), ACC_THREADS, acc_args, acc_lds)) return rc;
+      void* reduce_args[] = {(void*)&ws, (void*)&table, (void*)&gg, (void*)&bp, (void*)&feat, (void*)&f0, (void*)&ddt};
       const unsigned max_splits = (unsigned)NB < ws.max_slots / 2 ? (unsigned)NB : ws.max_slots / 2;
-      if (int rc = launch("hash_bwd_bin_reduce", reduce, dim3(2 * BIN_ROWS / REDUCE_VALUES, max_splits), REDUCE_THREADS, acc_args, 0)) return rc;
+      if (int rc = launch("hash_bwd_bin_reduce", reduce, dim3(2 * BIN_ROWS / REDUCE_VALUES, max_splits), REDUCE_THREADS, reduce_args, 0)) return rc;
     }
   return 0;
 }

@@ -1129,75 +1129,76 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
       return a;
     };
     constexpr int U = MODE == TABLE_ADD ? 4 : 8;  // rows of a thread that are under way together
-    if (task.slot != ~0u) {
-      if (ws.whole_slots) {
-        longlong2* dst = reinterpret_cast<longlong2*>(ws.slots) + (int64_t)task.slot * BIN_ROWS;
+    const bool whole_slot = task.slot != ~0u && ws.whole_slots;
+    if (whole_slot) {
+      longlong2* dst = reinterpret_cast<longlong2*>(ws.slots) + (int64_t)task.slot * BIN_ROWS;
 #pragma unroll 4
-        for (uint32_t r = tid; r < nrows; r += ACC_THREADS) {
-          const long long x = take(r), y = take(BIN_ROWS + r);
-          dst[r] = make_longlong2(x, y);
-        }
-      } else {
-        float2* dst = reinterpret_cast<float2*>(ws.slots) + (int64_t)task.slot * BIN_ROWS;
-#pragma unroll 4
-        for (uint32_t r = tid; r < nrows; r += ACC_THREADS) {
-          const float x = to_float(take(r)), y = to_float(take(BIN_ROWS + r));
-          dst[r] = make_float2(x, y);
-        }
+      for (uint32_t r = tid; r < nrows; r += ACC_THREADS) {
+        const long long x = take(r), y = take(BIN_ROWS + r);
+        dst[r] = make_longlong2(x, y);
       }
-    } else for (uint32_t r0 = tid; r0 < nrows; r0 += ACC_THREADS * U) {
+    }
+    for (uint32_t r0 = whole_slot ? nrows : tid; r0 < nrows; r0 += ACC_THREADS * U) {
       float x[U], y[U];
       float2 old[MODE == TABLE_ADD ? U : 1];
       // Added: the old values of all these rows are asked for before any is needed (rows of an even number of features pair by pair).  One
       // read and write after another for rows of other than two features: F = 4, 10^5 points 285 us, this 266; F = 8 774 and 715.  (With
       // one, two or eight rows under way the same within 1 %; asked for in front of the records' adds slower, 300 us: what is left
       // is the traffic of rows half used per pass, all units writing back at once.)
-      if constexpr (MODE == TABLE_ADD) {
-        const float* src = reinterpret_cast<const float*>(table) + first;
-        if constexpr (TWO) {
+      if constexpr (MODE == TABLE_ADD)
+        if (task.slot == ~0u) {
+          const float* src = reinterpret_cast<const float*>(table) + first;
+          if constexpr (TWO) {
 #pragma unroll
-          for (int u = 0; u < U; ++u) old[u] = reinterpret_cast<const float2*>(src)[min(r0 + u * ACC_THREADS, nrows - 1u)];
-        } else if ((feat & 1) == 0) {
+            for (int u = 0; u < U; ++u) old[u] = reinterpret_cast<const float2*>(src)[min(r0 + u * ACC_THREADS, nrows - 1u)];
+          } else if ((feat & 1) == 0) {
 #pragma unroll
-          for (int u = 0; u < U; ++u) old[u] = *reinterpret_cast<const float2*>(src + (int64_t)min(r0 + u * ACC_THREADS, nrows - 1u) * feat);
-        } else {
+            for (int u = 0; u < U; ++u) old[u] = *reinterpret_cast<const float2*>(src + (int64_t)min(r0 + u * ACC_THREADS, nrows - 1u) * feat);
+          } else {
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const float* cell = src + (int64_t)min(r0 + u * ACC_THREADS, nrows - 1u) * feat;
-            old[u] = make_float2(cell[0], has_pair ? cell[1] : 0.0f);
+            for (int u = 0; u < U; ++u) {
+              const float* cell = src + (int64_t)min(r0 + u * ACC_THREADS, nrows - 1u) * feat;
+              old[u] = make_float2(cell[0], has_pair ? cell[1] : 0.0f);
+            }
           }
         }
-      }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const uint32_t r = r0 + u * ACC_THREADS;
         x[u] = r < nrows ? to_float(take(r)) : 0.0f;
         y[u] = r < nrows ? to_float(take(BIN_ROWS + r)) : 0.0f;
       }
-      if constexpr (MODE == TABLE_ADD) {
-        float* dst = reinterpret_cast<float*>(table) + first;
-        if constexpr (TWO) {
+      if (task.slot != ~0u) {
+        float2* dst = reinterpret_cast<float2*>(ws.slots) + (int64_t)task.slot * BIN_ROWS;
 #pragma unroll
-          for (int u = 0; u < U; ++u)
-            if (x[u] != 0.0f || y[u] != 0.0f) reinterpret_cast<float2*>(dst)[r0 + u * ACC_THREADS] = make_float2(old[u].x + x[u], old[u].y + y[u]);
-        } else if ((feat & 1) == 0) {
+        for (int u = 0; u < U; ++u)
+          if (r0 + u * ACC_THREADS < nrows) dst[r0 + u * ACC_THREADS] = make_float2(x[u], y[u]);
+      } else {
+        if constexpr (MODE == TABLE_ADD) {
+          float* dst = reinterpret_cast<float*>(table) + first;
+          if constexpr (TWO) {
 #pragma unroll
-          for (int u = 0; u < U; ++u)
-            if (x[u] != 0.0f || y[u] != 0.0f)
-              *reinterpret_cast<float2*>(dst + (int64_t)(r0 + u * ACC_THREADS) * feat) = make_float2(old[u].x + x[u], old[u].y + y[u]);
+            for (int u = 0; u < U; ++u)
+              if (x[u] != 0.0f || y[u] != 0.0f) reinterpret_cast<float2*>(dst)[r0 + u * ACC_THREADS] = make_float2(old[u].x + x[u], old[u].y + y[u]);
+          } else if ((feat & 1) == 0) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (x[u] != 0.0f || y[u] != 0.0f)
+                *reinterpret_cast<float2*>(dst + (int64_t)(r0 + u * ACC_THREADS) * feat) = make_float2(old[u].x + x[u], old[u].y + y[u]);
+          } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              float* cell = dst + (int64_t)(r0 + u * ACC_THREADS) * feat;
+              if (x[u] != 0.0f) cell[0] = old[u].x + x[u];
+              if (has_pair && y[u] != 0.0f) cell[1] = old[u].y + y[u];
+            }
+          }
         } else {
 #pragma unroll
           for (int u = 0; u < U; ++u) {
-            float* cell = dst + (int64_t)(r0 + u * ACC_THREADS) * feat;
-            if (x[u] != 0.0f) cell[0] = old[u].x + x[u];
-            if (has_pair && y[u] != 0.0f) cell[1] = old[u].y + y[u];
+            const uint32_t r = r0 + u * ACC_THREADS;
+            if (r < nrows) store_pair<MODE>(table, first + (int64_t)r * feat, x[u], y[u], TWO, has_pair);
           }
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const uint32_t r = r0 + u * ACC_THREADS;
-          if (r < nrows) store_pair<MODE>(table, first + (int64_t)r * feat, x[u], y[u], TWO, has_pair);
         }
       }
     }

@@ -38,6 +38,18 @@ def test_levels_dealt_to_fill_workgroups(N, L, D, F, T, dtype):
         torch.testing.assert_close(s, do[:, l * F : (l + 1) * F].double().sum(0), rtol=0, atol=2**-16 * 5 * 8 * N**0.5)  # independent errors
 
 
+@pytest.mark.parametrize("N,L,F,dtype", [(470_000, 16, 8, torch.float32), (1_000_001, 15, 4, torch.float32), (1_000_001, 15, 8, torch.float16)])
+def test_all_levels_to_a_fill_workgroup(N, L, F, dtype):
+    """Gradients of more than 224 MiB.  Bounds as above."""
+    assert N * L * F * dtype.itemsize > 224 * 2**20
+    torch.manual_seed(N + L)
+    T, lo, hi = 2**17, 16, 2048
+    x = torch.rand(N, 3, device=DEV)
+    E = O.level_row_offsets(L, T, 3, lo, hi)[-1]
+    do = torch.randn(N, L * F, device=DEV).to(dtype)
+    torch.testing.assert_close(_grad(x, do, E, F, T, lo, hi, L, flags=16), _grad(x, do, E, F, T, lo, hi, L, flags=2), rtol=1e-3, atol=2e-3)
+
+
 # one block more than a workgroup's threads, a second chunk of blocks, lists of more records than LDS holds at a time, fewer tasks than workgroups
 @pytest.mark.parametrize("N", [512 * 1024 + 1, 2**20 + 77])
 @pytest.mark.parametrize("cube", [1.0, 0.02])

@@ -5,7 +5,7 @@
 // global atomics is bound by the chip's atomic request rate; accumulating them in LDS needs the contributions to
 // one stretch of the table together.  So the contributions are first sorted by table bin (BIN_ROWS rows):
 //
-//   fill    : every workgroup takes some hundred consecutive points and a few levels and, level by level, sorts their records by bin
+//   fill    : every workgroup takes some hundred consecutive points and a few levels (in the largest batches all) and, level by level, sorts their records by bin
 //             in LDS and writes them out as one contiguous block, with the place of every bin inside the block
 //   totals  : the number of records of every bin
 //   accum   : a workgroup per compute unit takes task after task, a task being a bin (or, where a bin holds many more records
@@ -61,6 +61,7 @@ constexpr int FILL_THREADS = 512, FILL_WIDE_THREADS = 1024;
 constexpr int fill_points(bool wide) { return wide ? 2 * FILL_WIDE_THREADS : FILL_THREADS; }
 constexpr int FILL_WIDE_BINS = 128;
 constexpr int64_t FILL_WIDE_POINTS = (int64_t)1 << 18;
+constexpr int64_t FILL_ROWS_BYTES = (int64_t)224 << 20;
 constexpr int ACC_THREADS = 1024;             // of sixteen waves
 constexpr int ACC_INFLIGHT = 2;               // records in flight per thread
 constexpr int GROUP = 16;                     // records named by one entry of a task's list
@@ -309,7 +310,7 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t m) {
 // ---------------------------------------------------------------------------------------
 // fill
 // ---------------------------------------------------------------------------------------
-// A workgroup takes some of the levels (blockIdx.y): a batch that leaves a unit one workgroup pays every level's barriers in turn (44 us for
+// A workgroup takes some of the levels (blockIdx.y), or all of them: a batch that leaves a unit one workgroup pays every level's barriers in turn (44 us for
 // sixteen levels at 2^14 to 2^17 points), several groups of levels cover each other's.
 // A level goes through three barriers: ranks inside the bins (LDS adds on one counter per bin), an exclusive scan of the
 // counters by one wave, the records into the stage in sorted order, and the stage out to the block.  The copy-out of a level runs
@@ -1898,7 +1899,10 @@ static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_
   // Levels of a fill workgroup: four, whose gradients are one 16-byte piece of a row, or fewer where that leaves less than two workgroups a
   // unit.  16 levels of 2^19 rows, fp16, uniform points, whole backward (us) with 16 / 4 / 2 / 1 levels to a workgroup: 2^14 points 100 / 72 /
   // 67 / 66, 2^15 104 / 76 / 72 / 73, 2^16 108 / 83 / 84 / 84, 2^17 114 / 93 / 95 / 100, 2^18 145 / 134 / 136 / 147, 2^20 378 / 374 / 418 / 530.
-  int step = 4;
+  // All levels where the gradient rows do not stay in the memory-side cache (256 MB) from one workgroup's four levels to the next's: fill of one
+  // pass (us), several workgroups / one to a row: 134 MB, fp16 2^21 points 352 / 356; 190 MB, float32 390 / 398, fp16 rows of four 290 / 297; 268 MB, float32 2^21
+  // 630 / 538, fp16 rows of four 487 / 417, of eight 240 / 234.  (The workgroups of a row next to each other on one XCD: 574 and 438 there, but 173 -> 216 at fp16 2^20.)
+  int step = N * bp.n_levels * feat * (g32 ? 4 : 2) > FILL_ROWS_BYTES ? bp.n_levels : 4;
   while (step > 1 && (int64_t)ws.blocks * ((bp.n_levels + step - 1) / step) < 2 * (int64_t)units) step /= 2;
   // more than three dimensions: the whole pipeline once per corner of the extra coordinates (`hi`), see ExtraDims
   const int passes = g.dims > 3 ? 1 << (g.dims - 3) : 1;

@@ -5,8 +5,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# single rows, one group of sixteen more or less than the waves or the SIMDs take at once, a share that favours one group, ragged ends
-@pytest.mark.parametrize("rows", [1, 17, 4096, 16385, 32768, 32769, 40003, 65537, 100003])
+# single rows, one group of sixteen more or less than the waves or the SIMDs take at once, a share that favours one group, a last round of a few
+# chunks, of most and of all, ragged ends
+@pytest.mark.parametrize("rows", [1, 17, 4096, 16320, 16384, 16385, 32768, 32769, 40003, 65536, 65537, 88000, 100003, 131089])
 @pytest.mark.parametrize("d_in,hidden,d_out,depth,shift", [(32, 64, 16, 2, 0), (64, 64, 64, 8, 0), (36, 32, 4, 7, 0), (35, 64, 3, 2, 0), (32, 64, 16, 1, 1), (64, 16, 64, 9, 0)])
 def test_every_share_gives_the_same_rows(rows, d_in, hidden, d_out, depth, shift):
     """A row's result does not depend on its batch.  Against 64 bits: a layer rounds each of its up to 66 additions to 2^-24 of the sum of the

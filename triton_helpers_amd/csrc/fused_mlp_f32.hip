@@ -37,6 +37,7 @@ struct Mlp32Args {
   int d_in, d_hidden, d_out, depth, act;
   int resident;  // 1: every layer's weights staged once per workgroup
   int n_layers;  // linear layers computed: depth + 1, or depth when only the pre-activations are wanted
+  int block_step, wave_step;  // chunks of the forward between neighbouring workgroups, and between the waves of one
 };
 
 __device__ __forceinline__ f32x4_t mfma4(float a, float b, f32x4_t c) {
@@ -133,8 +134,9 @@ __global__ __launch_bounds__(256, 2) void mlp32_fwd_k(Mlp32Args a) {
   const bool x_vec = ((uintptr_t)a.x % 16 == 0) && (a.x_stride % 4 == 0);
   const bool y_vec = a.y != nullptr && ((uintptr_t)a.y % 16 == 0) && (a.y_stride % 4 == 0);
   const int kt_in = (a.d_in + 15) / 16;
-  // a chunk's rows go to the workgroups in turn, then to their waves; the next chunk's are requested before this one's products
+  // The next chunk's rows are requested before this one's products.
   const int64_t n_chunks = (a.rows + 16 * NT - 1) / (16 * NT), per_round = (int64_t)gridDim.x * 4;
+  const int64_t first_of_workgroup = (int64_t)blockIdx.x * a.block_step, first_chunk = first_of_workgroup + (int64_t)wave * a.wave_step;
   f32x4_t nx[NT][4];
   auto load_rows = [&](int64_t chunk) {
 #pragma unroll
@@ -150,7 +152,6 @@ __global__ __launch_bounds__(256, 2) void mlp32_fwd_k(Mlp32Args a) {
       }
     }
   };
-  const int64_t first_chunk = (int64_t)wave * gridDim.x + blockIdx.x;
   if (a.resident) {
     // The layers are staged LAYERS at a time, their loads under way together and the first rows' behind them; layer by layer each waited
     // for the one in front.
@@ -199,9 +200,8 @@ __global__ __launch_bounds__(256, 2) void mlp32_fwd_k(Mlp32Args a) {
   } else if (PIECES) {
     load_rows(first_chunk);
   }
-  const int64_t rounds = (n_chunks + per_round - 1) / per_round;
-  for (int64_t round = 0; round < rounds; ++round) {
-    const int64_t chunk = first_chunk + round * per_round;
+  for (int64_t done = 0; first_of_workgroup + done < n_chunks; done += per_round) {  // (the same for the workgroup)
+    const int64_t chunk = first_chunk + done;
     if (a.resident && chunk >= n_chunks) break;
     const int64_t row0 = chunk * (16 * NT) + r;
     f32x4_t h[NT][4];
@@ -737,15 +737,22 @@ static int fwd32(Mlp32Args a, hipStream_t s) {
   a.resident = a.n_layers <= W32_RESIDENT_MAX;
   const size_t lds = (size_t)(a.resident ? a.n_layers : 1) * W32_LAYER * sizeof(float);
   const int64_t cap = (int64_t)device_cus() * (lds > 76 * 1024 ? 1 : 2);
-  // One group of sixteen rows to a wave where a SIMD's share of them is a tenth less than that of pairs, or there is no pair for every SIMD.  us, one /
-  // two: 32 -> 64 -> 64 -> 16, 4096 rows 7.4 / 10.2, 40000 14.0 / 15.1, 100003 23.6 / 25.9, 2^18 47.5 / 46.0; eight hidden layers of 64, 2^15 35.4 /
-  // 43.7; 16 -> 32 -> 32 -> 4, 2^16 10.0 / 9.7; 64 -> 64 -> 64 -> 64, 2^20 259 / 249.
+  // One group of sixteen rows to a wave where there is a wave for every group, or, with the layers in LDS, where a SIMD's share of groups is a tenth less than
+  // that of pairs.  Layers that pass through LDS are staged once more for every round of chunks, and half as many rows to a round are up to twice the rounds.
+  // us, one / two: 32 -> 64 -> 64 -> 16, 4096 rows 7.6 / 10.4, 40000 13.0 / 15.3, 100003 22.9 / 25.3, 2^18 47.0 / 45.5; 64 -> 64 -> 64 -> 64, 2^20 259 / 249;
+  // 32 -> 64 x 6 -> 16 (a workgroup to a unit), 16384 rows 16.1 / 23.9, 20000 26.0 / 24.2; 32 -> 64 x 9 -> 16 (in turn), 2^15 31.4 / 37.8, 36000 53.3 / 51.0, 100003 110 / 98.7.
   const int64_t simds = (int64_t)device_cus() * 4, ones = (a.rows + 15) / 16, twos = (a.rows + 31) / 32;
   const auto share = [&](int64_t units) { return (units + simds - 1) / simds; };
-  const bool single = twos <= simds || 10 * share(ones) < 9 * 2 * share(twos);
+  const bool single = ones <= 4 * cap || (a.resident && 10 * share(ones) < 9 * 2 * share(twos));
   const int64_t chunks = single ? ones : twos, full = (chunks + 3) / 4;
   int64_t blocks = full < cap ? full : cap;
   if (blocks < device_cus()) blocks = chunks < device_cus() ? chunks : device_cus();
+  // The chunks of a batch that leaves waves without one go to the workgroups in turn, then to their waves; of a larger one, four at a time to a workgroup:
+  // what the last round has left is then a chunk for every SIMD of some units.  A wave of every workgroup came down on one SIMD of every unit, and
+  // where the layers do not stay in LDS all workgroups went through that round (us, so / this: 32 -> 64 x 3 -> 16, 88000 rows 34.9 / 28.2; 64 x 11, 216000 256 / 236).
+  const bool spread = chunks <= 4 * blocks - 4;
+  a.block_step = spread ? 1 : 4;
+  a.wave_step = spread ? (int)blocks : 1;
   const auto pieces = [](const float* p, int64_t stride, int width) { return (uintptr_t)p % 16 == 0 && stride % 4 == 0 && width % 4 == 0; };
   const bool whole = pieces(a.x, a.x_stride, a.d_in) && (a.y == nullptr || pieces(a.y, a.y_stride, a.d_out));
   auto pick = [&](auto nt_c, auto whole_c) -> const void* {

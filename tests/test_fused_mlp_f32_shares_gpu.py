@@ -33,6 +33,22 @@ def test_every_share_gives_the_same_rows(rows, d_in, hidden, d_out, depth, shift
     assert ((y.double() - h).abs() <= a * (66 * (depth + 1) * 2.0**-24)).all()
 
 
+@pytest.mark.parametrize("rows", [16385, 33000, 70001])
+@pytest.mark.parametrize("d_in,hidden,d_out,depth", [(32, 16, 16, 1), (64, 64, 64, 3), (35, 32, 1, 4), (16, 32, 4, 9)])
+@pytest.mark.parametrize("act", ["silu", "relu2", "none"])
+def test_pairs_of_groups_give_the_rows_of_single_ones(rows, d_in, hidden, d_out, depth, act):
+    from triton_helpers_amd.layers.fully_fused_mlp import fully_fused_mlp
+
+    g = torch.Generator(device="cuda").manual_seed(rows + depth)
+    u = lambda *s: (torch.rand(*s, generator=g, device="cuda") * 2 - 1) * s[-1] ** -0.5  # noqa: E731
+    x, w = torch.randn(1, rows, d_in, generator=g, device="cuda"), [u(hidden, d_in), u(hidden), u(d_out, hidden), u(d_out)]
+    w += [u((depth - 1) * hidden, hidden), u(depth - 1, hidden)] if depth > 1 else [None, None]
+    with torch.no_grad():
+        y = fully_fused_mlp(x, *w, activation=act)
+        assert torch.equal(y, torch.cat([fully_fused_mlp(p, *w, activation=act) for p in x.split(4096, dim=1)], dim=1))
+    assert y.isfinite().all()
+
+
 @pytest.mark.parametrize("d_in,hidden,d_out,depth,bias", [(32, 64, 16, 2, True), (64, 64, 64, 2, False), (35, 32, 3, 1, True), (33, 16, 17, 2, True), (16, 64, 64, 1, False)])
 @pytest.mark.parametrize("rows", [1, 1000, 4097])
 def test_written_gradients_are_the_added_ones(rows, d_in, hidden, d_out, depth, bias):

@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256, 2) void mlp32_fwd_k(Mlp32Args a) {
   // The next chunk's rows are requested before this one's products.
   const int64_t n_chunks = (a.rows + 16 * NT - 1) / (16 * NT), per_round = (int64_t)gridDim.x * 4;
   const int64_t first_of_workgroup = (int64_t)blockIdx.x * a.block_step, first_chunk = first_of_workgroup + (int64_t)wave * a.wave_step;
-  f32x4_t nx[NT][4];
+  f32x4_t nx[NT][4];  // (PIECES)
   auto load_rows = [&](int64_t chunk) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
@@ -147,8 +147,7 @@ __global__ __launch_bounds__(256, 2) void mlp32_fwd_k(Mlp32Args a) {
       for (int t = 0; t < 4; ++t) {
         if (t >= kt_in) break;
         const int col = 16 * t + 4 * g;
-        if constexpr (PIECES) nx[nt][t] = *reinterpret_cast<const f32x4_t*>(p + (col < a.d_in ? col : 0));
-        else nx[nt][t] = load_chain(a.x, a.x_stride, row, a.rows, col, a.d_in, x_vec);
+        nx[nt][t] = *reinterpret_cast<const f32x4_t*>(p + (col < a.d_in ? col : 0));
       }
     }
   };
@@ -172,6 +171,7 @@ __global__ __launch_bounds__(256, 2) void mlp32_fwd_k(Mlp32Args a) {
         if (cols % 4 != 0 || (uintptr_t)w % 16 != 0) continue;
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
+          if (16 * i >= rows) break;  // no tile reads these (32 -> 32 x 4 -> 1, 56000 rows, with them 13.9 us, without 13.0)
           const int o = (tid >> 4) + 16 * i, c = 4 * (tid & 15);
           v[k][i] = *reinterpret_cast<const f32x4_t*>(w + (o < rows ? o : 0) * cols + (c < cols ? c : 0));
         }
@@ -190,6 +190,7 @@ __global__ __launch_bounds__(256, 2) void mlp32_fwd_k(Mlp32Args a) {
         }
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
+          if (16 * i >= rows) break;
           const int o = (tid >> 4) + 16 * i, c = 4 * (tid & 15);
           *reinterpret_cast<f32x4_t*>(dst + o * W32_STRIDE + c) = o < rows && c < cols ? v[k][i] : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
         }
@@ -205,13 +206,16 @@ __global__ __launch_bounds__(256, 2) void mlp32_fwd_k(Mlp32Args a) {
     if (a.resident && chunk >= n_chunks) break;
     const int64_t row0 = chunk * (16 * NT) + r;
     f32x4_t h[NT][4];
-    if (!PIECES) load_rows(chunk);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        if (t >= kt_in) break;
-        h[nt][t] = PIECES && 16 * t + 4 * g >= a.d_in ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : nx[nt][t];
+        if constexpr (PIECES) {
+          if (t >= kt_in) break;
+          h[nt][t] = 16 * t + 4 * g >= a.d_in ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : nx[nt][t];
+        } else {
+          h[nt][t] = t < kt_in ? load_chain(a.x, a.x_stride, row0 + 16 * nt, a.rows, 16 * t + 4 * g, a.d_in, x_vec) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
       }
     if (PIECES) load_rows(chunk + per_round);
     for (int l = 0; l < a.n_layers; ++l) {
@@ -768,7 +772,12 @@ static int fwd32(Mlp32Args a, hipStream_t s) {
   };
   const std::integral_constant<int, 1> one;
   const std::integral_constant<int, 2> two;
-  const void* kern = whole ? (single ? pick(one, std::true_type{}) : pick(two, std::true_type{})) : single ? pick(one, std::false_type{}) : pick(two, std::false_type{});
+  // Pairs of groups in whole pieces for ReLU alone: with the next rows in its registers, the kernel of another activation has 186 of them and is slower than
+  // with rows read value by value where they are needed (135), the more so the narrower the network (50200 rows, us, pieces / values: 32 -> 16 -> 16
+  // ReLU2 8.4 / 6.7, 32 -> 64 x 3 -> 4 SiLU 23.0 / 21.4, 64 -> 64 -> 64 ReLU2 18.3 / 16.0; ReLU, 149 registers value by value: 16 -> 32 -> 4 7.1 / 7.8, 32 -> 64 x 3 -> 4 20.3 / 20.5).
+  const void* kern = single ? (whole ? pick(one, std::true_type{}) : pick(one, std::false_type{}))
+                     : whole && a.act == NF_ACT_RELU ? (const void*)mlp32_fwd_k<NF_ACT_RELU, 2, true>
+                                                     : pick(two, std::false_type{});
   return launch32(kern, a, blocks, lds, s, "mlp32_fwd");
 }
 

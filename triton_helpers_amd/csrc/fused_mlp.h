@@ -67,7 +67,7 @@ __device__ __forceinline__ void stage_bias(float* dst, const uint16_t* b, int n_
 // NTHREADS: as for stage_weight_frags().
 template <typename T, int KIN, int HP, int OUTP, int PIECE, bool IN_CHAIN, int NTHREADS = 0, typename FirstRows>
 __device__ __forceinline__ void stage_network(uint16_t* frags, float* bias, const MlpArgs& a, int tid, int nthreads, FirstRows first_rows) {
-  constexpr int KC_IN = KIN / 32, KC_H = HP / 32, MT_H = HP / 16, MT_O = OUTP / 16, AT_ONCE = 4;
+  constexpr int KC_IN = KIN / 32, KC_H = HP / 32, MT_H = HP / 16, MT_O = OUTP / 16, AT_ONCE = NTHREADS > 0 ? 4 : 6;
   constexpr int F_IN = MT_H * KC_IN, F_HID = MT_H * KC_H, F_OUT = MT_O * KC_H;
   const int H = a.d_hidden, n_hid = a.depth - 1, hidden = n_hid * F_HID;
   if constexpr (PIECE == 0) {

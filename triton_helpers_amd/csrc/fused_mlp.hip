@@ -549,9 +549,10 @@ static int launch_fwd(const MlpArgs& a0, hipStream_t s) {
   // One group of sixteen rows to a wave, the workgroups of eight waves spread over the units, where two would leave SIMDs without a wave or, with
   // long chains of layers, with one (us, layers staged in turn and two groups / two groups / one: 32 -> 64 x 4 -> 16 SiLU 1000 rows 8.5 / 8.3 / 6.0, 65536 12.3 / 11.7 /
   // 10.3, 10^5 18.0 / 17.0 / 13.7, 2^17 18.2 / 17.3 / 15.9; 64 x 10 ReLU 1000 14.3 / 15.3 / 10.6, 2^17 23.8 / 24.3 / 23.3; one hidden layer SiLU
-  // 1000 6.6 / 5.6 / 5.2, 65536 7.7 / 7.4 / 7.6).
+  // 1000 6.6 / 5.6 / 5.2, 65536 7.7 / 7.4 / 7.6).  Rows that are read value by value wait longer than a single group's chain takes: where one workgroup
+  // fits a unit, two from 32768 on (35 -> 64 x 9 -> 16 ReLU, one / two: 33000 rows 13.7 / 13.7, 65536 15.8 / 14.5, 2^17 25.2 / 21.6).
   const bool list = n_hid > 0 && (uintptr_t)a.w_hid % 8 == 0;
-  const bool small = list && a.rows <= (n_hid == 1 ? 32768 : HP == 32 ? 65536 : 131072);
+  const bool small = list && a.rows <= (n_hid == 1 || (!a.x_vec && lds > 76 * 1024) ? 32768 : HP == 32 ? 65536 : 131072);
   // weights beyond half of LDS leave room for one workgroup per CU: give it eight waves to keep two per SIMD
   a.waves = lds > 76 * 1024 || small ? 8 : 4;
   const int64_t chunks = (a.rows + (small ? 15 : 31)) / (small ? 16 : 32);

@@ -49,7 +49,7 @@ def test_forward_with_levels_in_lds(N, dims, F, T, L, dtype, monkeypatch):
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
 
 
-@pytest.mark.parametrize("N", [1, 255, 257, 16384, 40960, 40961, 65535, 65537])
+@pytest.mark.parametrize("N", [1, 255, 257, 16384, 40960, 40961, 53248, 53249, 65535, 65537])
 @pytest.mark.parametrize("dims,F,T,L,dtype", [
     (3, 2, 2**19, 16, torch.float16), (3, 4, 2**19, 16, torch.bfloat16), (3, 4, 2**20, 8, torch.float16), (3, 8, 2**17, 16, torch.float16), (3, 2, 2**18, 4, torch.float32),
     (3, 4, 2**16, 8, torch.float32), (2, 2, 2**16, 2, torch.float32), (2, 4, 2**15, 4, torch.float16), (3, 2, 2**19, 32, torch.float16),

@@ -711,29 +711,37 @@ constexpr int SWEEP_PPT = 4;
 constexpr int64_t SWEEP_MIN_POINTS = ((int64_t)1 << 17) + 1;
 constexpr int64_t SWEEP_MIN_POINTS_D2 = (int64_t)1 << 16;
 constexpr int64_t SWEEP_MIN_POINTS_F32 = (int64_t)1 << 16;
-// The forward per (point, level) serves batches up to this where the staged kernel is the alternative, which takes sixteen rounds of latency for any
-// batch up to 2^17 points (us, level / staged: two features 2^16 points 35 / 51, 2^17 62 / 51; four 1000 4 / 54, 2^15 27 / 58, 2^16
-// 48 / 59, 100000 72 / 63; eight, levels of 1 MiB 2^16 33 / 35).  Rows of four and eight features in levels beyond an L2: four in 8 MiB
-// 2^15 37 / 59, 2^16 68 / 64; eight 2^15 39 / 42, 2^16 72 / 62.
 constexpr int64_t L2_BYTES = 4 << 20;
 static int64_t largest_level(const nf_hash_geom* g, int es) {
   int64_t rows = 0;
   for (int l = 0; l < g->levels; ++l) rows = g->rows[l] > rows ? g->rows[l] : rows;
   return rows * g->feat * es;
 }
-static int64_t level_max_points(const nf_hash_geom* g) { return g->feat > 2 && largest_level(g, 2) > L2_BYTES ? 40960 : 65536; }
 // Units of a level on one XCD (hash_fwd_level_k): where a level fits an L2 and the table does not, in batches that every XCD would read most of
 // it for.  2^15 points on 16 levels of 2^19 rows touch most of a table's lines from every XCD, 150 MB in all (us, dealt out in turn / by XCD,
 // uniform and rays): fp16 2^15 points 26 / 21 and 21 / 20, 2^16 43 / 35 and 35 / 34; float32 60000 56 / 43 and 48 / 43; four features
 // 2^16 57 / 48 and 49 / 47; but 8192 points along rays 9.2 / 10.4, a table of 3 MB 2^16 28 / 32, levels of 8 MiB 61 / 61, two dimensions
 // (most levels dense, their rows in order) 2^16 19 / 25, 2^18 points 246 / 276; and, each XCD reading a table of 13 MB often enough to be worth
-// its misses, 2^15 points 18 / 18 along rays, 2^16 30 / 32.
+// its misses, 2^15 points 18 / 18 along rays, 2^16 30 / 32.  Two thirds of the levels have to be hashed: dense ones take a fraction of the time, above all along
+// rays, and the XCDs that have those wait for the others (hashed levels of all, 2^15 points along rays, uniform): 2 of 16 (2^20 rows, 8 .. 128) 8.6 / 14 and
+// 17 / 21; 8 of 16 (2^19 rows, 16 .. 400) 15.0 / 17.8 and 21 / 20; 10 of 16 (.. 1500) 19.2 / 19.6; 12 of 16 (.. 7006) 21 / 20.  With 11 or more of 16 1.1 times as
+// fast along rays and 1.3 times uniform, on average over 29 tables at 16384 to 50000 points; the worst, a table of 50 MB at 16384 points along rays, 14.7 / 15.6.
 static bool level_by_xcd(const nf_hash_geom* g, int table_dt, int64_t n_points) {
   const int es = table_dt == NF_F32 ? 4 : 2;
   int64_t rows = 0;
   for (int l = 0; l < g->levels; ++l) rows += g->rows[l];
   const int64_t bytes = rows * g->feat * es;
-  return g->dims == 3 && n_points >= 16384 && n_points * 320 <= bytes && largest_level(g, es) <= L2_BYTES && bytes > 2 * L2_BYTES;
+  return g->dims == 3 && n_points >= 16384 && n_points * 320 <= bytes && largest_level(g, es) <= L2_BYTES && bytes > 2 * L2_BYTES &&
+         3 * (g->levels - g->first_hash_level) >= 2 * g->levels;
+}
+// The forward per (point, level) serves batches up to this where the staged kernel is the alternative, which takes sixteen rounds of latency for any
+// batch up to 2^17 points (us, level / staged: two features 2^16 points 35 / 51, 2^17 62 / 51; four 1000 4 / 54, 2^15 27 / 58, 2^16
+// 48 / 59, 100000 72 / 63).  Rows of four features in levels beyond an L2: 8 MiB 2^15 37 / 59, 2^16 68 / 64.  Rows of eight in any: levels of 1 MiB 50000 points
+// 28.4 / 28.2 along rays, 2^16 uniform 40 / 35, of 4 MiB 50000 51 / 46, of 8 MiB 2^15 39 / 42, 2^16 72 / 62; but by XCD 50000 points of 2 MiB 30 / 38 and, rays,
+// 29 / 32, 2^16 36 / 41 and 35 / 34.
+static int64_t level_max_points(const nf_hash_geom* g, int table_dt, int64_t n_points) {
+  if (g->feat == 8) return level_by_xcd(g, table_dt, n_points) ? 53248 : 40960;
+  return g->feat > 2 && largest_level(g, 2) > L2_BYTES ? 40960 : 65536;
 }
 
 // How a sweep's points are dealt out.  A compute unit works its gathers off at a rate of its own (one workgroup on a unit runs
@@ -1032,7 +1040,7 @@ extern "C" int nf_hash_encode_fwd(const void* coords, int coords_dtype, int64_t 
   }
   // batches below the sweep's minimum, and rows that neither sweep nor staged kernel takes: a thread per (point, level)
   if (!(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FWD_STAGED)) && level_ok(geom, table_dtype, table, out, out_stride_n) &&
-      (n_points <= level_max_points(geom) || !tiled_ok(geom, table_dtype, out, out_stride_n, geom->feat)))
+      (n_points <= level_max_points(geom, table_dtype, n_points) || !tiled_ok(geom, table_dtype, out, out_stride_n, geom->feat)))
     return launch_fwd_level(table_dtype, coords, coords_dtype, csn, csd, table, out, out_stride_n, n_points, g, primes, scale,
                             level_by_xcd(geom, table_dtype, n_points), s);
   if (!(flags & NF_HASH_FORCE_GENERIC) && tiled_ok(geom, table_dtype, out, out_stride_n)) {

@@ -727,21 +727,23 @@ static int64_t largest_level(const nf_hash_geom* g, int es) {
 // 17 / 21; 8 of 16 (2^19 rows, 16 .. 400) 15.0 / 17.8 and 21 / 20; 10 of 16 (.. 1500) 19.2 / 19.6; 12 of 16 (.. 7006) 21 / 20.  With 11 or more of 16 1.1 times as
 // fast along rays and 1.3 times uniform, on average over 29 tables at 16384 to 50000 points; the worst, a table of 50 MB at 16384 points along rays, 14.7 / 15.6.
 static bool level_by_xcd(const nf_hash_geom* g, int table_dt, int64_t n_points) {
+  if (g->dims != 3 || n_points < 16384 || 3 * (g->levels - g->first_hash_level) < 2 * g->levels) return false;
   const int es = table_dt == NF_F32 ? 4 : 2;
   int64_t rows = 0;
   for (int l = 0; l < g->levels; ++l) rows += g->rows[l];
   const int64_t bytes = rows * g->feat * es;
-  return g->dims == 3 && n_points >= 16384 && n_points * 320 <= bytes && largest_level(g, es) <= L2_BYTES && bytes > 2 * L2_BYTES &&
-         3 * (g->levels - g->first_hash_level) >= 2 * g->levels;
+  return n_points * 320 <= bytes && largest_level(g, es) <= L2_BYTES && bytes > 2 * L2_BYTES;
 }
 // The forward per (point, level) serves batches up to this where the staged kernel is the alternative, which takes sixteen rounds of latency for any
 // batch up to 2^17 points (us, level / staged: two features 2^16 points 35 / 51, 2^17 62 / 51; four 1000 4 / 54, 2^15 27 / 58, 2^16
 // 48 / 59, 100000 72 / 63).  Rows of four features in levels beyond an L2: 8 MiB 2^15 37 / 59, 2^16 68 / 64.  Rows of eight in any: levels of 1 MiB 50000 points
 // 28.4 / 28.2 along rays, 2^16 uniform 40 / 35, of 4 MiB 50000 51 / 46, of 8 MiB 2^15 39 / 42, 2^16 72 / 62; but by XCD 50000 points of 2 MiB 30 / 38 and, rays,
 // 29 / 32, 2^16 36 / 41 and 35 / 34.
+constexpr int64_t LEVEL_POINTS = 40960;  // taken whatever the rows
 static int64_t level_max_points(const nf_hash_geom* g, int table_dt, int64_t n_points) {
-  if (g->feat == 8) return level_by_xcd(g, table_dt, n_points) ? 53248 : 40960;
-  return g->feat > 2 && largest_level(g, 2) > L2_BYTES ? 40960 : 65536;
+  if (n_points <= LEVEL_POINTS) return LEVEL_POINTS;  // (the loops over the levels are 0.05 us of a call of 5.4)
+  if (g->feat == 8) return level_by_xcd(g, table_dt, n_points) ? 53248 : LEVEL_POINTS;
+  return g->feat > 2 && largest_level(g, 2) > L2_BYTES ? LEVEL_POINTS : 65536;
 }
 
 // How a sweep's points are dealt out.  A compute unit works its gathers off at a rate of its own (one workgroup on a unit runs

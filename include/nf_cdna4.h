@@ -111,7 +111,8 @@ int nf_hash_encode_bwd_write(const void* coords, int coords_dtype, int64_t coord
 
 /* Scratch bytes nf_hash_encode_bwd can use for this call shape and these flags; 0 when the workspace would not be used.
  * Sorted records: room for two records of 12 bytes (float32 gradients: 16) per point, level and corner pair (cells of dense 3-D levels: two
- * per point and level), 2 bytes per bin and block of 512 or 2048 points, and a 64 KiB slot per 1024 points for bins cut into tasks: 1.38 GB for 2^20
+ * per point and level), 2 bytes per bin and block of 512 or 2048 points, and a 64 KiB slot (128 KiB below 2^18 points; a workspace with room for 64 KiB
+ * runs too, with larger tasks) per 1024 points for bins cut into tasks: 1.38 GB for 2^20
  * points on 16 levels of 2^19 rows (float32: 2.22 GB).  The walk without records (NF_HASH_BWD_RECORDS switches it off): 4 bytes -- 8 with a
  * float32 gradient -- per point, level and feature pair, 4 per coordinate, and 128 KiB per task where the points are cut into slices.
  * NF_HASH_FORCE_PLANES gives the size of the smaller bit-plane variant.

@@ -63,7 +63,8 @@ def test_library_allocates_and_waits_for_nothing():
 
 
 @pytest.mark.parametrize("log2_rows,hi,dtype,n", [(14, 512, 0, 1_048_574), (14, 512, 1, 2_097_148), (19, 7006, 0, 65_424), (19, 7006, 1, 107_256), (21, 7006, 0, 74_478),
-                                                  (21, 7006, 1, 135_063), (16, 1024, 0, 111_733)])
+                                                  (21, 7006, 1, 135_063), (16, 1024, 0, 111_733),
+                                                  (19, 7006, 0, 124_928), (22, 7006, 0, 123_904)])
 def test_batches_that_the_static_scratch_serves(log2_rows, hi, dtype, n):
     """Sixteen levels: batches that the entry point without a workspace has always taken, whole or in two parts, are not refused for
     want of scratch (the NULL pointers are, behind that), and float32 gradients of four times as many points are."""

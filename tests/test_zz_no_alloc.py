@@ -85,7 +85,7 @@ def test_static_scratch_backward_matches_the_workspace_backward():
 
 
 @pytest.mark.parametrize("n,log2_rows,hi,dtype", [(107_001, 19, 7006, torch.float16), (65_423, 19, 7006, torch.float32), (135_063, 21, 7006, torch.bfloat16),
-                                                  (1_048_573, 14, 512, torch.float32)])
+                                                  (1_048_573, 14, 512, torch.float32), (124_001, 19, 7006, torch.float32)])
 def test_a_batch_beyond_the_scratch_runs_in_two_parts(n, log2_rows, hi, dtype):
     from triton_helpers_amd import _lib as L_
     from triton_helpers_amd.layers.hash_encoding.helpers import level_geometry

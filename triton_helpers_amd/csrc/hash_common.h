@@ -199,7 +199,10 @@ int launch_bwd_scan(const void* coords, int cdt, int64_t csn, int64_t csd, const
 
 
 // backward by binning the contributions per table stretch (hash_encoding_bwd_bin.hip)
-int64_t bwd_bin_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags);
+// (`whole` false: the least it runs in, with shares of bins that are larger and summed in floats)
+int64_t bwd_bin_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags, bool whole);
+// scratch of the variant that these flags choose: what it asks for, or the least it runs in (hash_encoding.hip)
+int64_t bwd_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags, bool whole);
 // two or three dimensions, hashed levels of a power of two of rows: a corner's row takes a few 32-bit instructions
 inline bool quick_rows(const nf_hash_geom* g) {
   for (int l = g->first_hash_level < 0 ? 0 : g->first_hash_level; l < g->levels; ++l)
@@ -215,11 +218,11 @@ inline int64_t bwd_records_min(const nf_hash_geom* g, int flags) { return bwd_le
 bool bwd_walk_applies(int64_t n_points, const nf_hash_geom* geom, int flags);
 int launch_bwd_bin(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
                    float* dtable, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
-                   void* workspace, int flags, hipStream_t s);
+                   void* workspace, int64_t workspace_bytes, int flags, hipStream_t s);
 // the same with every row of the table's gradient written, in a type of its own, instead of added to float32
 bool bwd_write_applies(int64_t n_points, const nf_hash_geom* geom, int flags);
 int launch_bwd_write(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride, void* table,
                      int table_dtype, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
-                     void* workspace, int flags, hipStream_t s);
+                     void* workspace, int64_t workspace_bytes, int flags, hipStream_t s);
 
 }  // namespace nf

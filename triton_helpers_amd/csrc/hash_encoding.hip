@@ -1081,13 +1081,17 @@ static bool bwd_tiles_apply(int64_t n_points, const nf_hash_geom* geom, int flag
   return n_points >= bwd_records_min(geom, flags) || bwd_walk_applies(n_points, geom, flags);
 }
 
-extern "C" int64_t nf_hash_encode_bwd_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags) {
+int64_t nf::bwd_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags, bool whole) {
   if (geom == nullptr || (flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FORCE_ATOMIC))) return 0;
   if (!bwd_tiles_apply(n_points, geom, flags)) return 0;
   const int64_t scan = n_points >= SCAN_MIN_POINTS ? bwd_scan_workspace_bytes(n_points, geom, dout_dtype) : 0;
   if (flags & NF_HASH_FORCE_PLANES) return scan;
-  const int64_t bin = bwd_bin_workspace_bytes(n_points, geom, dout_dtype, flags);
+  const int64_t bin = bwd_bin_workspace_bytes(n_points, geom, dout_dtype, flags, whole);
   return bin > 0 ? bin : scan;  // the bit-planes are what runs where the other kernels do not cover the geometry
+}
+
+extern "C" int64_t nf_hash_encode_bwd_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags) {
+  return bwd_workspace_bytes(n_points, geom, dout_dtype, flags, true);
 }
 
 extern "C" int nf_hash_encode_bwd(const void* coords, int coords_dtype, int64_t csn, int64_t csd, const void* dout,
@@ -1110,10 +1114,10 @@ extern "C" int nf_hash_encode_bwd(const void* coords, int coords_dtype, int64_t 
   if (!(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FORCE_ATOMIC)) && workspace != nullptr &&
       bwd_tiles_apply(n_points, geom, flags) &&
       ((uintptr_t)dout % (dout_dtype == NF_F32 ? 8 : 4) == 0) && (dout_stride_n % 2 == 0) && ((uintptr_t)workspace % 4 == 0)) {
-    const int64_t need_bin = bwd_bin_workspace_bytes(n_points, geom, dout_dtype, flags);
+    const int64_t need_bin = bwd_bin_workspace_bytes(n_points, geom, dout_dtype, flags, false);
     if (!(flags & NF_HASH_FORCE_PLANES) && need_bin > 0 && workspace_bytes >= need_bin && ((uintptr_t)workspace % 16 == 0))
       return launch_bwd_bin(coords, coords_dtype, csn, csd, dout, dout_dtype, dout_stride_n, dtable, n_points, geom, g, primes,
-                            scale, workspace, flags, s);
+                            scale, workspace, workspace_bytes, flags, s);
     const int64_t need = n_points >= SCAN_MIN_POINTS ? bwd_scan_workspace_bytes(n_points, geom, dout_dtype) : 0;
     if (need > 0 && workspace_bytes >= need)
       return launch_bwd_scan(coords, coords_dtype, csn, csd, dout, dout_dtype, dout_stride_n, dtable, n_points, geom, g,
@@ -1165,12 +1169,12 @@ extern "C" int nf_hash_encode_bwd_write(const void* coords, int coords_dtype, in
                  !(flags & (NF_HASH_FORCE_GENERIC | NF_HASH_FORCE_ATOMIC | NF_HASH_FORCE_PLANES)),
              NF_EUNSUPPORTED, "no kernel that writes this gradient in one go (nothing was launched; use nf_hash_encode_bwd)");
   NF_REQUIRE(coords && dout && dtable && primes && workspace, NF_EINVAL, "NULL pointer argument");
-  const int64_t need = bwd_bin_workspace_bytes(n_points, geom, dout_dtype, flags);
+  const int64_t need = bwd_bin_workspace_bytes(n_points, geom, dout_dtype, flags, false);
   NF_REQUIRE(need > 0 && (uintptr_t)dout % (dout_dtype == NF_F32 ? 8 : 4) == 0 && dout_stride_n % 2 == 0, NF_EUNSUPPORTED,
              "shape or alignment outside the sorted-record kernels (nothing was launched; use nf_hash_encode_bwd)");
   NF_REQUIRE(workspace_bytes >= need && (uintptr_t)workspace % 16 == 0, NF_EINVAL, "a 16-byte aligned workspace of %lld bytes is needed", (long long)need);
   return launch_bwd_write(coords, coords_dtype, csn, csd, dout, dout_dtype, dout_stride_n, dtable, table_dtype, n_points, geom, g, primes, scale,
-                          workspace, flags, (hipStream_t)stream);
+                          workspace, workspace_bytes, flags, (hipStream_t)stream);
 }
 
 extern "C" int nf_hash_encode_indices_fast(const void* coords, int coords_dtype, int64_t csn, int64_t csd,

@@ -1627,14 +1627,15 @@ static bool wide_blocks(int64_t n_points, const nf_hash_geom* geom) {
 // Shares of fewer than SPLIT_FLOAT_COST records leave their sums as they are, in 64-bit fixed point: a bin of that many records that was one task,
 // rounded once, is several then, and float sums of their floats would be rounded for each (2.5e-8 -> 5e-8 of a row at four shares).  The slots
 // are twice as large, 1 us of the chain at 2^17 points along rays; in the larger batches, cut no finer, it would be 3 to 7 us.
+// A workspace without room for them (`whole` false) gets shares of SPLIT_FLOAT_COST records and slots of floats, whatever the batch.
 constexpr int64_t SPLIT_FLOAT_COST = 32768;
-static int64_t split_cost(int64_t N, int levels) {
+static int64_t split_cost(int64_t N, int levels, bool whole) {
   const int64_t third = N * levels / 192, small = N < 32768 ? 8192 : N < 65536 ? N / 4 : 16384, large = N < 262144 ? N / 8 : SPLIT_FLOAT_COST;
-  const int64_t least = small > large ? small : large;
+  const int64_t least = !whole ? SPLIT_FLOAT_COST : small > large ? small : large;
   return third > least ? third : least;
 }
 
-static int64_t bin_ws(void* workspace, const BinPlan& bp, int64_t N, int points, int64_t R, int rec_words, BinWs* ws) {
+static int64_t bin_ws(void* workspace, const BinPlan& bp, int64_t N, int points, int64_t R, int rec_words, bool whole, BinWs* ws) {
   char* p = (char*)workspace;
   const int NB = bp.binbase[bp.n_levels];
   const int64_t blocks = (N + points - 1) / points;
@@ -1646,7 +1647,7 @@ static int64_t bin_ws(void* workspace, const BinPlan& bp, int64_t N, int points,
   };
   ws->blocks = (int)blocks;
   ws->start_stride = (NB + bp.n_levels + 1) & ~1;
-  ws->split_cost = (uint32_t)split_cost(N, bp.n_levels);
+  ws->split_cost = (uint32_t)split_cost(N, bp.n_levels, whole);
   ws->max_slots = (uint32_t)(16 + N / 1024);
   ws->whole_slots = ws->split_cost < SPLIT_FLOAT_COST;
   ws->header = (BinHeader*)take(sizeof(BinHeader) + NB * 4);
@@ -1746,7 +1747,7 @@ static int64_t walk_ws(void* workspace, const WalkPlan& wp, int64_t N, int dims,
   return o;
 }
 
-int64_t bwd_bin_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags) {
+int64_t bwd_bin_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int dout_dtype, int flags, bool whole) {
   if (n_points > BIN_CHUNK_POINTS) n_points = BIN_CHUNK_POINTS;
   if (walk_ok(n_points, geom, flags)) {
     WalkWs ws;
@@ -1757,7 +1758,7 @@ int64_t bwd_bin_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int 
     BinWs ws;
     int64_t R;
     const int points = fill_points(wide);
-    return bin_plan(n, points, geom, &bp, &R, dout_dtype != NF_F32) ? bin_ws(nullptr, bp, n, points, R, dout_dtype == NF_F32 ? 4 : 3, &ws) : 0;
+    return bin_plan(n, points, geom, &bp, &R, dout_dtype != NF_F32) ? bin_ws(nullptr, bp, n, points, R, dout_dtype == NF_F32 ? 4 : 3, whole, &ws) : 0;
   };
   if (!wide_blocks(n_points, geom)) return bytes(n_points, false);
   // room for every smaller batch too: many small blocks have more starts than fewer wide ones
@@ -1767,7 +1768,7 @@ int64_t bwd_bin_workspace_bytes(int64_t n_points, const nf_hash_geom* geom, int 
 
 static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
                                 void* table, int mode, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
-                                void* workspace, hipStream_t s);
+                                void* workspace, int64_t workspace_bytes, hipStream_t s);
 
 static int launch_bwd_walk(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
                            void* table, int mode, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
@@ -1775,7 +1776,7 @@ static int launch_bwd_walk(const void* coords, int cdt, int64_t csn, int64_t csd
 
 int launch_bwd_bin(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
                    float* dtable, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
-                   void* workspace, int flags, hipStream_t s) {
+                   void* workspace, int64_t workspace_bytes, int flags, hipStream_t s) {
   // the choice is made once, on the size the workspace was asked for: every piece then fits it
   const bool walk = bwd_walk_applies(N, geom, flags);
   for (int64_t n0 = 0; n0 < N; n0 += BIN_CHUNK_POINTS) {
@@ -1783,7 +1784,7 @@ int launch_bwd_bin(const void* coords, int cdt, int64_t csn, int64_t csd, const 
     const char* c = (const char*)coords + n0 * csn * dtype_size(cdt);
     const char* d = (const char*)dout + n0 * dout_stride * dtype_size(ddt);
     const int rc = walk ? launch_bwd_walk(c, cdt, csn, csd, d, ddt, dout_stride, dtable, TABLE_ADD, n, geom, g, primes, scale, workspace, s)
-                        : launch_bwd_bin_piece(c, cdt, csn, csd, d, ddt, dout_stride, dtable, TABLE_ADD, n, geom, g, primes, scale, workspace, s);
+                        : launch_bwd_bin_piece(c, cdt, csn, csd, d, ddt, dout_stride, dtable, TABLE_ADD, n, geom, g, primes, scale, workspace, workspace_bytes, s);
     if (rc) return rc;
   }
   return 0;
@@ -1797,10 +1798,10 @@ bool bwd_write_applies(int64_t n_points, const nf_hash_geom* geom, int flags) {
 
 int launch_bwd_write(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride, void* table,
                      int table_dtype, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
-                     void* workspace, int flags, hipStream_t s) {
+                     void* workspace, int64_t workspace_bytes, int flags, hipStream_t s) {
   const int mode = table_dtype == NF_F32 ? TABLE_F32 : table_dtype == NF_F16 ? TABLE_F16 : TABLE_BF16;
   return walk_ok(N, geom, flags) ? launch_bwd_walk(coords, cdt, csn, csd, dout, ddt, dout_stride, table, mode, N, geom, g, primes, scale, workspace, s)
-                                 : launch_bwd_bin_piece(coords, cdt, csn, csd, dout, ddt, dout_stride, table, mode, N, geom, g, primes, scale, workspace, s);
+                                 : launch_bwd_bin_piece(coords, cdt, csn, csd, dout, ddt, dout_stride, table, mode, N, geom, g, primes, scale, workspace, workspace_bytes, s);
 }
 
 static int launch_large(const char* what, const void* kern, dim3 grid, int threads, void** args, size_t lds, hipStream_t s) {
@@ -1854,7 +1855,7 @@ static int launch_bwd_walk(const void* coords, int cdt, int64_t csn, int64_t csd
 
 static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_t csd, const void* dout, int ddt, int64_t dout_stride,
                                 void* table, int mode, int64_t N, const nf_hash_geom* geom, const DevGeom& g, const int64_t* primes, float scale,
-                                void* workspace, hipStream_t s) {
+                                void* workspace, int64_t workspace_bytes, hipStream_t s) {
   const bool g32 = ddt == NF_F32;
   BinPlan bp;
   int64_t R;
@@ -1863,7 +1864,7 @@ static int launch_bwd_bin_piece(const void* coords, int cdt, int64_t csn, int64_
   NF_REQUIRE(bin_plan(N, points, geom, &bp, &R, !g32), NF_EUNSUPPORTED, "binned backward does not cover this geometry");
   NF_REQUIRE(((uintptr_t)workspace & 15u) == 0, NF_EALIGN, "workspace must be 16-byte aligned");
   BinWs ws;
-  bin_ws(workspace, bp, N, points, R, g32 ? 4 : 3, &ws);
+  if (bin_ws(workspace, bp, N, points, R, g32 ? 4 : 3, true, &ws) > workspace_bytes) bin_ws(workspace, bp, N, points, R, g32 ? 4 : 3, false, &ws);
   const int NB = bp.binbase[bp.n_levels];
   int max_nb = 1, bin_pieces = 0;
   for (int l = 0; l < bp.n_levels; ++l) {

@@ -44,14 +44,14 @@ extern "C" int nf_hash_encode_bwd_static(const void* coords, int coords_dtype, i
                                          const nf_hash_geom* geom, const int64_t* primes, float scale, int flags, void* stream) {
   NF_REQUIRE(geom != nullptr, NF_EINVAL, "geom is NULL");
   NF_REQUIRE(n_points >= 0, NF_EINVAL, "n_points negative");
-  // Which variant's scratch fits: the sorted records (~1.3 KB per point; float32 ~2.1) or the walk without them (~0.1 to 0.2 KB) of the
+  // Which variant's least scratch fits: the sorted records (~1.3 KB per point; float32 ~2.1) or the walk without them (~0.1 to 0.2 KB) of the
   // whole batch; else of its largest part that fits, the rest being a call of its own; else the bit-planes (~110 B per point, 16-bit
   // gradients of 3-D points only), which also run where the rest would need a second pass of records: 16 levels of 2^19 rows, float16,
   // 107000 points as 100864 and a rest for the atomics 146 us, with the bit-planes 180; 107000 as two halves 228; 2^14 rows, 2^21 points
   // 370 us in two parts, with the bit-planes 1620.  A call that would need none of these (small batches and shapes that scatter with
   // atomics) needs no scratch at all.
   const int64_t limit = (int64_t)NF_HASH_BWD_STATIC_BYTES;
-  auto need_of = [&](int64_t n, int f) { return nf_hash_encode_bwd_workspace_bytes(n, geom, dout_dtype, f); };
+  auto need_of = [&](int64_t n, int f) { return bwd_workspace_bytes(n, geom, dout_dtype, f, false); };
   const int64_t need_bin = need_of(n_points, flags & ~NF_HASH_FORCE_PLANES), need_planes = need_of(n_points, flags | NF_HASH_FORCE_PLANES);
   int64_t piece = n_points;
   int use_flags = flags;

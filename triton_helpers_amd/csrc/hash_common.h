@@ -211,8 +211,10 @@ inline bool quick_rows(const nf_hash_geom* g) {
 }
 // whether the atomics per (point, level, corner, feature) take a small batch
 inline bool bwd_level_ok(const nf_hash_geom* g) { return quick_rows(g) && (g->feat == 2 || g->feat == 4); }
-// Batches from which the sorted records run: their fixed cost is about 90 us, the atomics' 5 ns per point (and 20 us for the table's
-// zeros and rounding) or, where no kernel but the generic one has them, 13 ns.
+// Batches from which the sorted records run where the atomics per (point, level) take smaller ones.  Not where the times meet (16 levels of 2^19
+// rows, us: 2^13 points by atomics 35 added, 64 with the table's zeros and rounding; 2^14 by records 51 added, 47 written): a record's weight is 19
+// bits and its sum fixed point at the scale of the level's largest gradient, a level with an inf gives nan, and batches of fewer points keep the
+// atomics' float sums.  The other shapes' atomics, 13 ns per point, leave at 8192.
 inline int64_t bwd_records_min(const nf_hash_geom* g, int flags) { return bwd_level_ok(g) && !(flags & NF_HASH_BWD_RECORDS) ? 16384 : 8192; }
 // whether launch_bwd_bin would walk the points without records (small tables; also for batches too small for the records)
 bool bwd_walk_applies(int64_t n_points, const nf_hash_geom* geom, int flags);

@@ -40,8 +40,8 @@
 // not depend on the order of its records.  The tasks of a split bin are added in their order: a gradient has the same bits in
 // every run.  A level whose gradient holds an inf or a nan gets nan in every row it touches.
 //
-// One MI355X, 16 levels of 2^19 rows, fp16, uniform points, gradient of the table in its own type (us): 2^14 points 45, 2^16 60, 2^17 75, 2^18 111,
-// 2^20 349, 2^21 646; along rays 2^18 126, 2^20 402.  (Before the levels were dealt to fill workgroups and the accumulation asked for the next
+// One MI355X, 16 levels of 2^19 rows, fp16, uniform points, gradient of the table in its own type (us): 2^14 points 47, 2^16 62, 2^17 79, 2^18 112,
+// 2^20 350, 2^21 648; along rays 2^18 127, 2^20 402.  (Before the levels were dealt to fill workgroups and the accumulation asked for the next
 // chunk's records ahead of the finished tile's way out: 100, 108, 114, 144, 379, 680; 158, 436.)
 //
 // Arithmetic (cell, corner rows, weights) is the forward's, see hash_encoding.hip.
@@ -1142,10 +1142,10 @@ __global__ __launch_bounds__(ACC_THREADS) void hash_bwd_bin_accum_k(BinWs ws, vo
     for (uint32_t r0 = whole_slot ? nrows : tid; r0 < nrows; r0 += ACC_THREADS * U) {
       float x[U], y[U];
       float2 old[MODE == TABLE_ADD ? U : 1];
-      // Added: the old values of all these rows are asked for before any is needed (rows of an even number of features pair by pair).  One
-      // read and write after another for rows of other than two features: F = 4, 10^5 points 285 us, this 266; F = 8 774 and 715.  (With
-      // one, two or eight rows under way the same within 1 %; asked for in front of the records' adds slower, 300 us: what is left
-      // is the traffic of rows half used per pass, all units writing back at once.)
+      // Added: the old values of all these rows are asked for before any is needed (rows of an even number of features pair by pair).  Rows
+      // of other than two features, 16 levels of 2^19 rows, one / four / eight rows of a thread under way (us): 10^5 points F = 1 81 / 79 / 77,
+      // F = 3 195 / 189 / 188, F = 4 204 / 201 / 200, F = 8 567 / 580 / 566; 5 * 10^5 points 198 / 192 / 188, 483 / 468 / 467, 503 / 492 / 492,
+      // 1181 / 1191 / 1179: what takes the time is the traffic of rows half used per pass.
       if constexpr (MODE == TABLE_ADD)
         if (task.slot == ~0u) {
           const float* src = reinterpret_cast<const float*>(table) + first;

@@ -1279,15 +1279,16 @@ struct WalkWs {
 
 // Gradient pairs level by level and coordinates dimension by dimension, both in the order of the walk: neighbouring lanes of a walk take
 // points WALK_STRIDE apart, because along a ray neighbouring points share cells and their adds to one row would wait for each other
-// (T = 2^14, 2^18 points along rays: 258 us without, 85 with).  Rows of whole 16-byte pieces (`vec`) come in as they lie, 512 bytes of four
+// (T = 2^14, 2^18 points along rays: 258 us without, 85 with).  Rows of whole 16-byte pieces (VEC) come in as they lie, 512 bytes of four
 // neighbouring points to 32 lanes, up to 128 bytes of a row at once, and are turned to a row per lane in LDS: read a row per lane from memory,
 // the lines of a unit's lanes are ten times its L1 and every piece fetched its line again.  A thread's pieces are all of the same planes, so the
 // maxima are taken before the turn (one per plane and row behind it: 72.9 us).  The chain of a float32 table of 2^14 rows, 2^18 points 66.0 -> 63.3 us
-// (this kernel 20.0 -> 16.6, 67 MB), 4096 points 21.8 -> 19.9; fp16 2^18 61.6 -> 59.3, rows of four features 2^17 77.5 -> 73.3.
-template <bool G32, int D>
+// (this kernel 20.0 -> 16.6, 67 MB), 4096 points 21.8 -> 19.9; fp16 2^18 61.6 -> 59.3, rows of four features 2^17 77.5 -> 73.3.  Other rows
+// have a kernel of their own, as one for both needs the registers of eight pieces (one feature, 8 levels of 2^15 rows, 425718 points 18.4 -> 16.7).
+template <bool G32, int D, bool VEC>
 __global__ __launch_bounds__(WALK_PREP_THREADS) void hash_bwd_walk_prep_k(const void* coords, int cdt, int64_t csn, int64_t csd, float scale,
                                                                           const void* dout_v, int64_t dout_stride, int64_t N, int levels, int feat,
-                                                                          int vec, WalkWs ws) {
+                                                                          WalkWs ws) {
   extern __shared__ __align__(16) uint32_t plane_max[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int np = (feat + 1) / 2, planes = levels * np;
@@ -1311,7 +1312,7 @@ __global__ __launch_bounds__(WALK_PREP_THREADS) void hash_bwd_walk_prep_k(const 
     else ws.pairs[(int64_t)plane * N + at] = x;
   };
   auto pair_max = [&](uint32_t x, uint32_t y) { return G32 ? max(x & 0x7fffffffu, y & 0x7fffffffu) : max(x & 0x7fffu, (x >> 16) & 0x7fffu); };
-  if (vec) {
+  if constexpr (VEC) {
     constexpr int PER = G32 ? 2 : 4;  // planes of a piece
     uint4* tile = reinterpret_cast<uint4*>(plane_max + (planes + 3) / 4 * 4);  // [position][PREP_PITCH]
     const int pieces = planes / PER;
@@ -1822,18 +1823,19 @@ static int launch_bwd_walk(const void* coords, int cdt, int64_t csn, int64_t csd
   walk_ws(workspace, wp, N, geom->dims, geom->feat, ddt, &ws);
   int levels = geom->levels, feat = geom->feat;
   const void *prep, *walk;
+  const int planes = levels * ((feat + 1) / 2);
+  const bool vec = feat % 2 == 0 && planes % (ddt == NF_F32 ? 2 : 4) == 0 && (uintptr_t)dout % 16 == 0 && dout_stride % (ddt == NF_F32 ? 4 : 8) == 0;
   auto pick = [&](auto d_c) {
     constexpr int DD = decltype(d_c)::value;
-    prep = ddt == NF_F32 ? (const void*)hash_bwd_walk_prep_k<true, DD> : (const void*)hash_bwd_walk_prep_k<false, DD>;
+    prep = ddt == NF_F32 ? (vec ? (const void*)hash_bwd_walk_prep_k<true, DD, true> : (const void*)hash_bwd_walk_prep_k<true, DD, false>)
+                         : (vec ? (const void*)hash_bwd_walk_prep_k<false, DD, true> : (const void*)hash_bwd_walk_prep_k<false, DD, false>);
     walk = ddt == NF_F32 ? (const void*)hash_bwd_walk_k<F32, DD> : ddt == NF_BF16 ? (const void*)hash_bwd_walk_k<BF16, DD> : (const void*)hash_bwd_walk_k<F16, DD>;
   };
   if (g.dims == 3) pick(std::integral_constant<int, 3>{});
   else if (g.dims == 2) pick(std::integral_constant<int, 2>{});
   else if (g.dims == 1) pick(std::integral_constant<int, 1>{});
   else pick(std::integral_constant<int, 4>{});
-  const int planes = levels * ((feat + 1) / 2);
-  int vec = feat % 2 == 0 && planes % (ddt == NF_F32 ? 2 : 4) == 0 && (uintptr_t)dout % 16 == 0 && dout_stride % (ddt == NF_F32 ? 4 : 8) == 0;
-  void* prep_args[] = {(void*)&coords, (void*)&cdt, (void*)&csn, (void*)&csd, (void*)&scale, (void*)&dout, (void*)&dout_stride, (void*)&N, (void*)&levels, (void*)&feat, (void*)&vec, (void*)&ws};
+  void* prep_args[] = {(void*)&coords, (void*)&cdt, (void*)&csn, (void*)&csd, (void*)&scale, (void*)&dout, (void*)&dout_stride, (void*)&N, (void*)&levels, (void*)&feat, (void*)&ws};
   const size_t prep_lds = (size_t)(planes + 3) / 4 * 16 + (vec ? (size_t)WALK_PREP_THREADS * PREP_PITCH * 16 : 0);
   if (int rc = launch_large("hash_bwd_walk_prep", prep, dim3((unsigned)wp.prep_blocks), WALK_PREP_THREADS, prep_args, prep_lds, s)) return rc;
   const void* reduce = with_mode(mode, [](auto mode_c) { return (const void*)hash_bwd_walk_reduce_k<decltype(mode_c)::value>; });

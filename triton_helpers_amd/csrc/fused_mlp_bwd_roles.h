@@ -83,14 +83,24 @@ __device__ __forceinline__ void stage_rows(char* dst, const uint16_t* w, int lay
   }
 }
 
+// Whether the matrices come in 16-byte pieces.  64-wide kernels are compiled for either, narrow ones for both: with the other way of staging in it a 64-wide
+// kernel takes longer over its rows, and a narrow one is allocated the better for it (us, forward and backward, 2^20 rows, both ways in one / one each: 16 -> 64
+// -> 20 ReLU 104.9 / 101.3, 32 -> 64 -> 20 107.2 / 103.3, 32 -> 64 x 4 -> 16 205.6 / 201.9; 64 -> 64 x 9 -> 64, 2^16 off 16 bytes 69.2 / 68.0; but 32 -> 32 -> 33 121.7 / 126.8).
+enum class WholePieces { NO, YES, ANY };
+__host__ __device__ __forceinline__ bool whole_pieces(const MlpArgs& a) {
+  return a.d_in % 8 == 0 && a.d_hidden % 8 == 0 && ((uintptr_t)a.w_in | (uintptr_t)a.w_hid | (uintptr_t)a.w_out) % 16 == 0;
+}
+
 // All matrices and hidden biases of a network as one list of 16-byte pieces, laid out as stage_rows() does, with several of a thread's under way
 // together and first_rows(), which asks for the wave's first rows, behind them.  The biases are asked for first.  Matrix by matrix in 8-byte pieces, a
 // clock each for the L1, each waited for the one in front and all for the rows (us with the sum of the gradients, before / this: 32 -> 64 -> 64 -> 16
 // 1000 rows 9.8 / 9.2, 2^16 19.5 / 18.7; 64 -> 64 x 8 -> 64, 2^16 51 / 47.6; three layers of SiLU, 2^18 69.2 / 67.1).
-template <typename T, int HP, int N, typename FirstRows>
+// WHOLE: whether the matrices are such pieces (else they are staged one by one behind the rows), or ANY for both ways in one kernel.
+template <typename T, int HP, int N, WholePieces WHOLE, typename FirstRows>
 __device__ __forceinline__ void stage_pieces(char* dst, float* bias, const MlpArgs& a, int tid, FirstRows first_rows) {
   constexpr int AT_ONCE = 6, HP_LOG2 = HP == 32 ? 5 : 6;
-  const int lane = tid & 63, first = __builtin_amdgcn_readfirstlane(tid - lane), H = a.d_hidden, units = (a.depth * HP + 64) * 8;
+  const bool pieces = WHOLE == WholePieces::ANY ? whole_pieces(a) : WHOLE == WholePieces::YES;
+  const int lane = tid & 63, first = __builtin_amdgcn_readfirstlane(tid - lane), H = a.d_hidden, units = pieces ? (a.depth * HP + 64) * 8 : 0;
   const auto bias_at = [&](int i, bool& there) {
     const int l = i >> 6, f = i & 63;
     const uint16_t* b = l == 0 ? a.b_in : a.b_hid != nullptr ? a.b_hid + (size_t)(l - 1) * H : nullptr;
@@ -130,6 +140,10 @@ __device__ __forceinline__ void stage_pieces(char* dst, float* bias, const MlpAr
     const uint16_t b = *bias_at(i, there);
     bias[i] = there ? T::to_f32(b) : 0.0f;
   }
+  if (pieces) return;
+  stage_rows<N>(dst, a.w_in, 1, H, HP, a.d_in, tid);
+  if (a.depth > 1) stage_rows<N>(dst + HP * ROLES_PITCH, a.w_hid, a.depth - 1, H, HP, H, tid);
+  stage_rows<N>(dst + a.depth * HP * ROLES_PITCH, a.w_out, 1, a.d_out, 64, H, tid);
 }
 
 // The launch's arguments, read again where they are used (see opaque()).
@@ -140,8 +154,8 @@ __device__ __forceinline__ ArgsPtr fresh_args() {
   return p;
 }
 
-// MAXD: most hidden layers (fewer leave registers for more waves); CW: chain waves; OCC: waves per SIMD the kernel is compiled for.
-template <typename T, int HP, int ACT, int MAXD, int CW, int OCC>
+// MAXD: most hidden layers (fewer leave registers for more waves); CW: chain waves; OCC: waves per SIMD the kernel is compiled for; WHOLE: see stage_pieces().
+template <typename T, int HP, int ACT, int MAXD, int CW, int OCC, WholePieces WHOLE>
 __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a) {
   constexpr int MT = HP / 16, KC = HP / 32, ROWS = 16 * CW, THREADS = 64 * (CW + 4);  // rows of a round
   constexpr bool RELU = ACT == NF_ACT_RELU;
@@ -175,22 +189,9 @@ __global__ __launch_bounds__(64 * (CW + 4), OCC) void mlp_bwd_roles_k(MlpArgs a)
       if (kc == 0 || two_out) ndy[kc] = load_row8(k->dy, k->dy_stride, r, k->rows, k->d_out, 32 * kc + 8 * g, k->dy_vec != 0);
     }
   };
-  auto first_rows = [&] {
+  stage_pieces<T, HP, THREADS, WHOLE>(w_in, bias, a, tid, [&] {
     if (chain) load_rows(row0);
-  };
-  if (a.d_in % 8 == 0 && a.d_hidden % 8 == 0 && ((uintptr_t)a.w_in | (uintptr_t)a.w_hid | (uintptr_t)a.w_out) % 16 == 0) {
-    stage_pieces<T, HP, THREADS>(w_in, bias, a, tid, first_rows);
-  } else {
-    first_rows();
-    stage_rows<THREADS>(w_in, a.w_in, 1, a.d_hidden, HP, a.d_in, tid);
-    if (depth > 1) stage_rows<THREADS>(w_hid, a.w_hid, depth - 1, a.d_hidden, HP, a.d_hidden, tid);
-    stage_rows<THREADS>(w_out, a.w_out, 1, a.d_out, 64, a.d_hidden, tid);
-    for (int i = tid; i < depth * 64; i += THREADS) {
-      const int l = i >> 6, f = i & 63;
-      const uint16_t* b = l == 0 ? a.b_in : a.b_hid != nullptr ? a.b_hid + (size_t)(l - 1) * a.d_hidden : nullptr;
-      bias[i] = b != nullptr && f < a.d_hidden ? T::to_f32(b[f]) : 0.0f;
-    }
-  }
+  });
   __syncthreads();
 
   const int chain0 = chain_offset(n, g), nat0 = natural_offset(n, g), tr0 = tr_offset(n, g);

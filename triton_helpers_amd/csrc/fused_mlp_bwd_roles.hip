@@ -80,9 +80,15 @@ template <typename T, int HP, int ACT>
 static int launch_roles(const MlpArgs& a, const RolesPlan& p, hipStream_t s) {
   constexpr int SH = roles_shallow(ACT), MANY = HP == 64 ? 8 : 12;
   const size_t lds = roles_lds(HP, a.depth, 16 * p.cw);
-  const void* kern = a.depth > SH   ? (const void*)mlp_bwd_roles_k<T, HP, ACT, ROLES_MAX_DEPTH, 4, HP == 32 && ACT == NF_ACT_RELU ? 4 : 2>
-                     : p.cw == MANY ? (const void*)mlp_bwd_roles_k<T, HP, ACT, SH, MANY, MANY / 4 + 1>
-                                    : (const void*)mlp_bwd_roles_k<T, HP, ACT, SH, 4, 2>;
+  const auto pick = [&](auto whole_c) -> const void* {
+    constexpr WholePieces WHOLE = decltype(whole_c)::value;
+    return a.depth > SH   ? (const void*)mlp_bwd_roles_k<T, HP, ACT, ROLES_MAX_DEPTH, 4, HP == 32 && ACT == NF_ACT_RELU ? 4 : 2, WHOLE>
+           : p.cw == MANY ? (const void*)mlp_bwd_roles_k<T, HP, ACT, SH, MANY, MANY / 4 + 1, WHOLE>
+                          : (const void*)mlp_bwd_roles_k<T, HP, ACT, SH, 4, 2, WHOLE>;
+  };
+  const void* kern;
+  if constexpr (HP == 32) kern = pick(std::integral_constant<WholePieces, WholePieces::ANY>{});
+  else kern = whole_pieces(a) ? pick(std::integral_constant<WholePieces, WholePieces::YES>{}) : pick(std::integral_constant<WholePieces, WholePieces::NO>{});
   const hipError_t ea = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (ea != hipSuccess) return fail((int)ea, "hipFuncSetAttribute: %s", hipGetErrorString(ea));
   void* args[] = {(void*)&a};

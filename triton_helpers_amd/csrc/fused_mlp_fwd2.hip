@@ -27,8 +27,9 @@ constexpr int fwd2_waves(int kin, int outp) { return (kin == 32 && outp == 16) ?
 // a lane a clock, so 8-byte pieces are 64 clocks per 512 bytes: 30 of the 34 us that 64 -> 64 -> 64 -> 64 took at 2^19 rows, 25 now
 // (2^20 rows 59 -> 47, 32 -> 64 -> 64 -> 64 41 -> 36, 64 -> 64 -> 64 -> 16 36 -> 30).  The decoder shape moves a third of that and is
 // held by memory (2^20 rows 21 us either way): 8-byte pieces there.
-// W16: the hidden and the output matrix lie on 16 bytes (with the other ways of staging in the same kernel 2^18 rows of the decoder shape take 9.4 us, so 9.0).
-template <typename T, int XC, int KIN, int OUTP, bool XW, bool YW, bool W16>
+// LIST8: the hidden matrix lies on 8 bytes and it or the output matrix not on 16.  With all ways of staging in one kernel 2^18 rows of the decoder shape take 9.4 us, with
+// those of 16 bytes alone in one 8.75 (2^16 5.66; 64 -> 64 -> 64 -> 64, 2^19 rows 27.4), so 8.6 (5.5; 27.1).
+template <typename T, int XC, int KIN, int OUTP, bool XW, bool YW, bool LIST8>
 __global__ __launch_bounds__(64 * fwd2_waves(KIN, OUTP)) void mlp_fwd2_k(MlpArgs a) {
   constexpr int HP = 64, NT = 2, WAVES = fwd2_waves(KIN, OUTP);
   constexpr int KC_IN = KIN / 32, KC_H = HP / 32, MT_H = HP / 16, MT_O = OUTP / 16;
@@ -85,8 +86,8 @@ __global__ __launch_bounds__(64 * fwd2_waves(KIN, OUTP)) void mlp_fwd2_k(MlpArgs
   float* bias_out = bias_hid + HP;
   // (us over inputs that no cache holds, matrix by matrix in 8-byte pieces / this: 32 -> 64 -> 64 -> 16 2^18 rows 9.3 / 7.5, 2^20 22.5 / 19.4;
   // 64 -> 64 -> 64 -> 64 2^18 15.6 / 13.8, 2^19 30.0 / 28.3)
-  if constexpr (W16) stage_network<T, KIN, HP, OUTP, 16, true, nthreads>(f_in, bias_in, a, tid, nthreads, first_rows);
-  else if ((uintptr_t)a.w_hid % 8 == 0) stage_network<T, KIN, HP, OUTP, 8, true, nthreads>(f_in, bias_in, a, tid, nthreads, first_rows);
+  if constexpr (LIST8) stage_network<T, KIN, HP, OUTP, 8, true, nthreads>(f_in, bias_in, a, tid, nthreads, first_rows);
+  else if (((uintptr_t)a.w_hid | (uintptr_t)a.w_out) % 16 == 0) stage_network<T, KIN, HP, OUTP, 16, true, nthreads>(f_in, bias_in, a, tid, nthreads, first_rows);
   else stage_network<T, KIN, HP, OUTP, 0, true, nthreads>(f_in, bias_in, a, tid, nthreads, first_rows);
   __syncthreads();
 
@@ -166,10 +167,10 @@ static int launch_fwd2(const MlpArgs& a0, hipStream_t s) {
   const int64_t cap = (int64_t)device_cus() * NF_FWD2_WG_PER_CU;
   if (blocks > cap) blocks = cap;
   constexpr int XC_OTHER = T::code == NF_BF16 ? 1 : 2;
-  const bool w16 = ((uintptr_t)a.w_hid | (uintptr_t)a.w_out) % 16 == 0;
+  const bool list8 = (uintptr_t)a.w_hid % 8 == 0 && ((uintptr_t)a.w_hid | (uintptr_t)a.w_out) % 16 != 0;
   const auto pick = [&](auto xw_c, auto yw_c) -> const void* {
     constexpr bool XW = decltype(xw_c)::value, YW = decltype(yw_c)::value;
-    if (w16) return a.x_conv == 0 ? (const void*)mlp_fwd2_k<T, 0, KIN, OUTP, XW, YW, true> : (const void*)mlp_fwd2_k<T, XC_OTHER, KIN, OUTP, XW, YW, true>;
+    if (list8) return a.x_conv == 0 ? (const void*)mlp_fwd2_k<T, 0, KIN, OUTP, XW, YW, true> : (const void*)mlp_fwd2_k<T, XC_OTHER, KIN, OUTP, XW, YW, true>;
     return a.x_conv == 0 ? (const void*)mlp_fwd2_k<T, 0, KIN, OUTP, XW, YW, false> : (const void*)mlp_fwd2_k<T, XC_OTHER, KIN, OUTP, XW, YW, false>;
   };
   const void* kern = pick(std::false_type{}, std::false_type{});

@@ -292,10 +292,10 @@ variable_list mlp_backward(Mlp m, Tensor dy, bool need_dx, bool float_grads) {
   // ReLU at 64 wide has kernels of its own for one and two hidden layers, which lay their weights out in both forms, sum eight waves
   // and (one hidden layer) go through an identity layer: quicker than the whole backward from about 2^16 rows, at one layer from 2^19 where
   // the output is narrow (us own / whole: 32 -> 64 -> 64 -> 16 2^12 rows 14.9 / 9.8, 2^16 19.4 / 18.6, 2^17 22 / 24, 2^20 60 / 102; 64 -> 64 -> 64
-  // -> 64 2^16 22.2 / 22.3, 2^17 25.5 / 29.7; 32 -> 64 -> 16 2^18 29.4 / 26.2, 2^19 39.2 / 40.9, 2^20 61 / 70).  One layer with a wide output takes the whole
-  // backward in every batch: it is the quicker one for most widths (2^20 rows, inputs in caches or not: 16 -> 64 -> 32 86 / 75, 32 -> 64 -> 32 83 / 79, 48 -> 64 -> 32
-  // 104 / 103, 32 -> 64 -> 64 87 / 89; 64 -> 64 -> 64 2^18 41 / 40), but not from 2^19 rows on where both are wide or the output is off 16 bytes (64 -> 64 -> 64 2^19 61 / 66,
-  // 2^20 104 / 116; 32 -> 64 -> 20 85 / 102).
+  // -> 64 2^16 22.2 / 22.3, 2^17 25.5 / 29.7; 32 -> 64 -> 16 2^18 27.8 / 25.1, 2^19 38.2 / 39.1, 2^20 61 / 70).  One layer with a wide output takes the whole
+  // backward in every batch: it is the quicker one of narrow inputs and below 2^19 rows (2^20 rows 16 -> 64 -> 32 72 / 65, 32 -> 64 -> 32 73 / 66; 64 -> 64 -> 64 2^18
+  // 35.2 / 33.9), but not in the largest ones where both are wide or the output is off 16 bytes (2^20 rows 48 -> 64 -> 32 90 / 93, 32 -> 64 -> 64 76 / 78,
+  // 64 -> 64 -> 64 102 / 112, 2^19 53 / 56; 32 -> 64 -> 20 76 / 79, 2^19 44.0 / 44.6).
   const bool many = depth == 2 ? g.n > 1 << 16 : out <= 16 && g.n > 1 << 19;
   if (many && wt != at::kFloat && depth <= 2 && H == 64 && in <= 64 && out <= 64 && (decoder || m.x.scalar_type() == wt) && in % 4 == 0 && out % 4 == 0 &&
       relu) {
